@@ -153,7 +153,7 @@ __device__ __forceinline__ void compute_tile4(const Tile4& t, u16x8 q, int valid
     ps += pr;
     const f32x2 p2 = {pr, pr};
 #pragma unroll
-    for (int e = 0; e < 4; ++e)   // <2 x float> FMAs: v_pk_fma_f32
+    for (int e = 0; e < 4; ++e)
       o2[e] = __builtin_elementwise_fma(p2, f32x2{T::to_float(t.v[r][2 * e]), T::to_float(t.v[r][2 * e + 1])}, o2[e]);
   }
 #pragma unroll
