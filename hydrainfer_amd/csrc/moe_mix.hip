@@ -333,82 +333,203 @@ __global__ __launch_bounds__(256) void grouped_linear_kernel(typename A::storage
   }
 }
 
-// MFMA form (bfloat16, K a multiple of 8, rows 16-byte aligned): a workgroup of four waves takes TM rows of one expert and
-// TN output columns; the rows' inputs (gathered through src) and the expert's weight rows go through LDS in slices of 64
-// k — the next slice is on its way into registers while the current one is multiplied — and every wave multiplies its
-// (TM / WGM) x (TN / WGN) part with 16x16x32 MFMAs: lane l holds k 8 (l / 16) .. + 7 of row (A) or column (B) l % 16, the
-// accumulator's lane l column l % 16 of rows 4 (l / 16) .. + 3.  Rows of LDS are padded to 72 elements (144 bytes): the
-// sixteen rows a 16-byte read touches fall into different banks.
-constexpr int kKS = 64, kLDK = 72;
-template <int TM, int TN, int WGM, int WGN>
-__global__ __launch_bounds__(256) void grouped_linear_tiled_kernel(u16* __restrict__ y, const u16* __restrict__ x, int64_t x_stride,
-                                                                   const int32_t* __restrict__ src, const u16* __restrict__ w,
-                                                                   const int32_t* __restrict__ seg, int E, int64_t N, int64_t K,
-                                                                   int act, Glu glu) {
-  constexpr int FM = TM / WGM / 16, FN = TN / WGN / 16;
-  constexpr int PA = TM * 8 / 256, PB = TN * 8 / 256;      // 16-byte pieces of a slice a thread moves
-  __shared__ __attribute__((aligned(16))) u16 As[TM * kLDK];
-  __shared__ __attribute__((aligned(16))) u16 Bs[TN * kLDK];
-  int e, row0, row1;
-  if (!find_tile(seg, E, TM, blockIdx.y, e, row0, row1)) return;      // (the whole workgroup: no barrier is left waiting)
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+// MFMA form (bfloat16, K a multiple of 8, rows 16-byte aligned).  A workgroup of WGM x WGN waves takes TM rows of one expert
+// and TN output columns.  The rows' inputs (gathered through src) and the expert's weight rows go straight from memory to LDS
+// (no registers, no writes by the waves) in slices of 64 k and NS slots; every wave multiplies its (TM / WGM) x (TN / WGN)
+// part with 16x16x32 MFMAs: lane l holds k 8 (l / 16) .. + 7 of row (A) or column (B) l % 16, the accumulator's lane l
+// column l % 16 of rows 4 (l / 16) .. + 3.  Half a slice is multiplied while the other half's operands are read from LDS, one
+// read between four products; the one workgroup barrier of a slice stands between its halves, so that a wave always has
+// products to issue behind it.
+// With many rows an expert it is bound by the matrix cores and LDS bandwidth (256 x 256: a byte read from LDS feeds 43
+// multiply-adds, 128 x 128 over four waves 32), with few by the weights: those of an expert with one row tile are read past
+// the caches.  Measured with 16 experts, 2 x 2752 outputs of 4096 and back: 15956 rows 866 + 444 us through registers in
+// tiles of 128 x 128 and padded LDS rows, 671 + 383 us here (1.07 and 0.94 PFLOP/s); 128 rows 162 + 75 us before, 123 + 61 us here (5.9 TB/s).
+// A slice's row is 128 bytes, unpadded (64 lanes land 16 bytes each one after the other): its 16-byte chunk c sits at position
+// c ^ (row / 2 % 8), so that the 16 lanes that one pass of a 16-byte LDS read serves — rows 0-3, 12-15 of one k group and
+// 4-11 of the next — fall into different banks.
+// Workgroups are numbered so that the eight XCDs (dealt round robin) work on eight runs of tiles, the row tiles of an expert
+// next to each other: they share the weight columns in the XCD's L2.
+constexpr int kKS = 64;
+template <int N>
+__device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+
+template <int TM, int TN, int WGM, int WGN, int NS, bool FAR>
+__global__ __launch_bounds__(64 * WGM * WGN) void grouped_linear_mfma_kernel(u16* __restrict__ y, const u16* __restrict__ x, int64_t x_stride,
+                                                                             const int32_t* __restrict__ src, const u16* __restrict__ w,
+                                                                             const int32_t* __restrict__ seg, int E, int64_t N, int64_t K,
+                                                                             int act, Glu glu) {
+  constexpr int NW = WGM * WGN, FM = TM / WGM / 16, FN = TN / WGN / 16;
+  constexpr int GA = TM / 8 / NW, GB = TN / 8 / NW;        // load instructions of a wave and slice: eight rows each
+  constexpr int kSlice = (TM + TN) * 2 * kKS;              // bytes
+  static_assert(GA * NW * 8 == TM && GB * NW * 8 == TN && FN % 2 == 0, "whole groups of eight rows a wave, columns in pairs");
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int n_col = (int)((N + TN - 1) / TN);
+  int e = 0, row0 = 0, row1 = 0;
+  int64_t col0 = 0;
+  bool once = false;                                       // the expert has one row tile: nobody reads its weights again
+  {
+    int m_tiles = 0;
+    for (int i = 0; i < E; ++i) m_tiles += (seg[i + 1] - seg[i] + TM - 1) / TM;
+    const int total = m_tiles * n_col, per = (total + 7) >> 3;
+    const int at = (int)(blockIdx.x >> 3);
+    int tile = (int)(blockIdx.x & 7) * per + at;
+    if (at >= per || tile >= total) return;                // (the whole workgroup: no barrier is left waiting)
+    for (; e < E; ++e) {
+      row0 = seg[e];
+      row1 = seg[e + 1];
+      const int nt = (row1 - row0 + TM - 1) / TM;
+      if (tile < nt * n_col) {
+        const int c = tile / nt;
+        row0 += (tile - c * nt) * TM;
+        col0 = (int64_t)c * TN;
+        once = nt == 1;
+        break;
+      }
+      tile -= nt * n_col;
+    }
+    row1 = min(row1, row0 + TM);
+  }
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int wm0 = (wave / WGN) * (TM / WGM), wn0 = (wave % WGN) * (TN / WGN);
-  const int64_t col0 = (int64_t)blockIdx.x * TN;
-  const u16* we = w + (int64_t)e * N * K;
-  const u16x8 zero8 = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-  const u16* pa[PA];
-  const u16* pb[PB];
-  int ka[PA], kb[PB];
+  const u16* wt = w + ((int64_t)e * N + col0) * K;         // the tile's first weight row
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+  // where a lane's 16 bytes of every load come from (a row or column past the last one repeats it; never stored)
+  uint32_t oa[GA], ob[GB];
+  const u16* pa[GA];
 #pragma unroll
-  for (int p = 0; p < PA; ++p) {
-    const int idx = threadIdx.x + 256 * p, r = idx >> 3;
-    ka[p] = (idx & 7) * 8;
-    pa[p] = nullptr;
-    if (row0 + r < row1) pa[p] = x + (src ? (int64_t)src[row0 + r] : (int64_t)(row0 + r)) * x_stride + ka[p];
+  for (int j = 0; j < GA; ++j) {
+    const int grp = wave * GA + j, r = min(row0 + 8 * grp + (lane >> 3), row1 - 1);
+    const int64_t at = (src ? (int64_t)src[r] : (int64_t)r) * x_stride + 8 * ((lane & 7) ^ (((grp & 1) << 2) + (lane >> 4)));
+    if constexpr (FAR) pa[j] = x + at;
+    else oa[j] = (uint32_t)(2 * at);
   }
 #pragma unroll
-  for (int p = 0; p < PB; ++p) {
-    const int idx = threadIdx.x + 256 * p, c = idx >> 3;
-    kb[p] = (idx & 7) * 8;
-    pb[p] = col0 + c < N ? we + (col0 + c) * K + kb[p] : nullptr;
+  for (int j = 0; j < GB; ++j) {
+    const int grp = wave * GB + j;
+    const int64_t left = N - 1 - col0;
+    const int64_t c = 8 * grp + (lane >> 3) < left ? 8 * grp + (lane >> 3) : left;
+    ob[j] = (uint32_t)(2 * (c * K + 8 * ((lane & 7) ^ (((grp & 1) << 2) + (lane >> 4)))));
   }
-  u16x8 ra[PA], rb[PB];
-  auto fetch = [&](int64_t k0) __attribute__((always_inline)) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+  // (m0, the LDS address of the transfer, is a reserved register: nothing else in this kernel uses it)
+  auto bring = [&](int64_t k0, int slot) __attribute__((always_inline)) {
+    const uint32_t to = lds0 + (uint32_t)(slot * kSlice);
 #pragma unroll
-    for (int p = 0; p < PA; ++p) ra[p] = (pa[p] && k0 + ka[p] < K) ? *reinterpret_cast<const u16x8*>(pa[p] + k0) : zero8;
+    for (int j = 0; j < GA; ++j) {
+      const uint32_t at = __builtin_amdgcn_readfirstlane(to + (uint32_t)(wave * GA + j) * 1024u);
+      if constexpr (FAR) asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(pa[j] + k0), "s"(at) : "memory", "m0");
+      else asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(oa[j]), "s"(x + k0), "s"(at) : "memory", "m0");
+    }
+    const uint32_t tb = to + (uint32_t)(2 * kKS * TM + wave * GB * 1024);
+    if (TM < 256 && once) {
 #pragma unroll
-    for (int p = 0; p < PB; ++p) rb[p] = (pb[p] && k0 + kb[p] < K) ? *reinterpret_cast<const u16x8*>(pb[p] + k0) : zero8;
+      for (int j = 0; j < GB; ++j)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(ob[j]), "s"(wt + k0), "s"(__builtin_amdgcn_readfirstlane(tb + 1024u * j)) : "memory", "m0");
+    } else {
+#pragma unroll
+      for (int j = 0; j < GB; ++j)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(ob[j]), "s"(wt + k0), "s"(__builtin_amdgcn_readfirstlane(tb + 1024u * j)) : "memory", "m0");
+    }
   };
+#pragma clang diagnostic pop
+  const int l16 = lane & 15, kq = lane >> 4;
   f32x4 acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int l16 = lane & 15, kq = lane >> 4;
-  fetch(0);
-  for (int64_t k0 = 0; k0 < K; k0 += kKS) {
+  const bool live = row0 + wm0 < row1;                     // a wave past the expert's rows only helps to bring the slices in
+  // a half slice's operands and its products
+  struct Frags {
+    u16x8 a[FM], b[FN];
+  };
+  auto read = [&](Frags& f, int slot, int half) __attribute__((always_inline)) {
+    const int chunk = ((4 * half + kq) ^ ((l16 >> 1) & 7)) * 16;
+    const char* A = smem + slot * kSlice + (wm0 + l16) * 128 + chunk;
+    const char* B = smem + slot * kSlice + (TM + wn0 + l16) * 128 + chunk;
 #pragma unroll
-    for (int p = 0; p < PA; ++p) *reinterpret_cast<u16x8*>(As + ((threadIdx.x + 256 * p) >> 3) * kLDK + ka[p]) = ra[p];
+    for (int j = 0; j < FN; ++j) f.b[j] = *reinterpret_cast<const u16x8*>(B + j * 2048);
 #pragma unroll
-    for (int p = 0; p < PB; ++p) *reinterpret_cast<u16x8*>(Bs + ((threadIdx.x + 256 * p) >> 3) * kLDK + kb[p]) = rb[p];
-    lds_barrier();      // (LDS only: the next slice's loads stay in flight)
-    if (k0 + kKS < K) fetch(k0 + kKS);
+    for (int i = 0; i < FM; ++i) f.a[i] = *reinterpret_cast<const u16x8*>(A + i * 2048);
+  };
+  auto multiply = [&](const Frags& f) __attribute__((always_inline)) {
 #pragma unroll
-    for (int ks = 0; ks < kKS / 32; ++ks) {
-      u16x8 af[FM], bf[FN];
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int i = 0; i < FM; ++i) af[i] = *reinterpret_cast<const u16x8*>(As + (wm0 + 16 * i + l16) * kLDK + 32 * ks + 8 * kq);
+      for (int j = 0; j < FN; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, f.a[i]), __builtin_bit_cast(bf16x8, f.b[j]),
+                                                            acc[i][j], 0, 0, 0);
+  };
+  // the reads of one half slice dealt between the products of the other
+  auto interleave = [&]() __attribute__((always_inline)) {
 #pragma unroll
-      for (int j = 0; j < FN; ++j) bf[j] = *reinterpret_cast<const u16x8*>(Bs + (wn0 + 16 * j + l16) * kLDK + 32 * ks + 8 * kq);
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, af[i]), __builtin_bit_cast(bf16x8, bf[j]),
-                                                              acc[i][j], 0, 0, 0);
+    for (int i = 0; i < FM + FN; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, FM * FN / (FM + FN), 0);
     }
-    lds_barrier();      // (LDS only: the next slice's loads stay in flight)
+  };
+  const int n_whole = (int)(K / kKS);
+#pragma unroll
+  for (int p = 0; p < NS; ++p)
+    if (p < n_whole) bring((int64_t)p * kKS, p);
+  if (n_whole >= NS) wait_loads<(NS - 1) * (GA + GB)>();
+  else wait_loads<0>();
+  lds_barrier();
+  Frags f0, f1;
+  if (n_whole && live) read(f0, 0, 0);
+  int slot = 0;
+  for (int t = 0; t < n_whole; ++t) {
+    const int next = slot == NS - 1 ? 0 : slot + 1;
+    if (live) {
+      read(f1, slot, 1);
+      multiply(f0);
+      interleave();
+    }
+    if (t + 1 < n_whole) {
+      // slice t + 1 is there when at most the NS - 2 slices behind it are on their way; past the barrier every wave's part of
+      // it is, and every wave has read all of slice t: its slot can be filled again
+      if (n_whole - 2 - t >= NS - 2) wait_loads<(NS - 2) * (GA + GB)>();
+      else wait_loads<0>();
+      lds_barrier();
+      if (t + NS < n_whole) bring((int64_t)(t + NS) * kKS, slot);
+    }
+    if (live) {
+      read(f0, next, 0);                                   // (behind the last slice: whatever the slot holds, never used)
+      multiply(f1);
+      interleave();
+    }
+    slot = next;
   }
+  if (K % kKS) {                                           // the last slice, part of it past K: through registers, zeros there
+    const int64_t k0 = (int64_t)n_whole * kKS;
+    const u16x8 zero8 = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    __syncthreads();                                       // every wave is done with the slices
+#pragma unroll
+    for (int j = 0; j < GA; ++j) {
+      const int grp = wave * GA + j;
+      const bool in = k0 + 8 * ((lane & 7) ^ (((grp & 1) << 2) + (lane >> 4))) < K;
+      const char* from;
+      if constexpr (FAR) from = reinterpret_cast<const char*>(pa[j] + k0);
+      else from = reinterpret_cast<const char*>(x + k0) + oa[j];
+      *reinterpret_cast<u16x8*>(smem + grp * 1024 + lane * 16) = in ? *reinterpret_cast<const u16x8*>(from) : zero8;
+    }
+#pragma unroll
+    for (int j = 0; j < GB; ++j) {
+      const int grp = wave * GB + j;
+      const bool in = k0 + 8 * ((lane & 7) ^ (((grp & 1) << 2) + (lane >> 4))) < K;
+      *reinterpret_cast<u16x8*>(smem + 2 * kKS * TM + grp * 1024 + lane * 16) =
+          in ? *reinterpret_cast<const u16x8*>(reinterpret_cast<const char*>(wt + k0) + ob[j]) : zero8;
+    }
+    __syncthreads();
+    if (live) {
+      read(f0, 0, 0);
+      read(f1, 0, 1);
+      multiply(f0);
+      multiply(f1);
+    }
+  }
+  if (!live) return;
   if (act == 2) {      // columns in turns of 16 gates and 16 ups: a lane holds both numbers of a pair
 #pragma unroll
     for (int i = 0; i < FM; ++i)
@@ -436,6 +557,20 @@ __global__ __launch_bounds__(256) void grouped_linear_tiled_kernel(u16* __restri
         if (rr < row1) y[(int64_t)rr * N + c] = BF16::from_float(act_apply(acc[i][j][r], act));
       }
     }
+}
+
+template <int TM, int TN, int WGM, int WGN, int NS>
+int launch_grouped(u16* y, const u16* x, int64_t x_stride, const int32_t* src, const u16* w, const int32_t* seg, int64_t max_rows, int E,
+                   int64_t N, int64_t K, int act, const Glu& glu, hipStream_t s) {
+  // every expert's rows start a tile of their own
+  const int64_t grid = ((max_rows + TM - 1) / TM + E) * ((N + TN - 1) / TN) + 7;
+  if (grid > 0x7fffffff) return HX_ERR_SHAPE;
+  constexpr size_t lds = (size_t)NS * (TM + TN) * 2 * kKS;
+  const bool far = max_rows * x_stride > 0x3fffffff;       // (a token brings a row at least: no input row lies further on)
+  auto kernel = far ? grouped_linear_mfma_kernel<TM, TN, WGM, WGN, NS, true> : grouped_linear_mfma_kernel<TM, TN, WGM, WGN, NS, false>;
+  if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  kernel<<<dim3((unsigned)grid), dim3(64 * WGM * WGN), lds, s>>>(y, x, x_stride, src, w, seg, E, N, K, act, glu);
+  return hxm::check_launch();
 }
 
 // The same, four elements a lane: width, row strides and pointers are multiples of four elements.  Rows and weights of the
@@ -576,20 +711,16 @@ extern "C" int hxm_grouped_linear(void* y, const void* x, int64_t x_stride, cons
   if (x_stride < k_dim) return HX_ERR_STRIDE;
   const Glu glu{glu_limit, glu_alpha, glu_up_shift};
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == HX_BF16 && k_dim % 8 == 0 && x_stride % 8 == 0 && aligned16(x) && aligned16(w)) {
-    // few rows an expert (decode steps): tiles of 32 rows, the four waves side by side over 128 columns; else 128 x 128
-    const bool small = max_rows <= (int64_t)32 * n_experts;
-    const int tm = small ? 32 : 128;
-    const int64_t tiles = (max_rows + tm - 1) / tm + n_experts;      // every expert's rows start a tile of their own
-    if (tiles > 65535) return HX_ERR_SHAPE;
-    const dim3 grid((unsigned)((n_dim + 127) / 128), (unsigned)tiles);
-    if (small)
-      grouped_linear_tiled_kernel<32, 128, 1, 4><<<grid, dim3(256), 0, s>>>((u16*)y, (const u16*)x, x_stride, src, (const u16*)w, seg,
-                                                                            n_experts, n_dim, k_dim, act, glu);
-    else
-      grouped_linear_tiled_kernel<128, 128, 2, 2><<<grid, dim3(256), 0, s>>>((u16*)y, (const u16*)x, x_stride, src, (const u16*)w, seg,
-                                                                             n_experts, n_dim, k_dim, act, glu);
-    return hxm::check_launch();
+  if (dtype == HX_BF16 && k_dim % 8 == 0 && k_dim < (1 << 22) && x_stride % 8 == 0 && aligned16(x) && aligned16(w)) {      // (offsets inside a weight tile: 32 bits)
+    u16* yy = (u16*)y;
+    const u16 *xx = (const u16*)x, *ww = (const u16*)w;
+    // Rows an expert on average: up to 32 the weights are all there is to read (tiles of 32 rows: 123 us with 128 rows and 16
+    // experts of 5504 x 4096, like 128 x 128, at a quarter of its LDS).  A mean of 120 is where most experts need a second
+    // tile of 128 rows: 400 tokens of 4 choices and 16 experts take 181 + 82 us in tiles of 128, 206 + 94 us in tiles of 256;
+    // 512 tokens 252 + 105 and 223 + 96 us.
+    if (max_rows <= (int64_t)32 * n_experts) return launch_grouped<32, 128, 1, 4, 3>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
+    if (max_rows < (int64_t)120 * n_experts) return launch_grouped<128, 128, 2, 2, 3>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
+    return launch_grouped<256, 256, 2, 4, 2>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
   }
   const int64_t tiles = (max_rows + kGM - 1) / kGM + n_experts;
   if (tiles > 65535) return HX_ERR_SHAPE;

@@ -1,0 +1,66 @@
+"""The grouped product of the experts' rows (csrc/moe_mix.hip, the matrix-core form) at the edges of its tiles: one row, a tile
+and one row more, columns and k that no tile divides, experts without rows, rows gathered and rows as they come, and inputs
+whose rows lie further apart than 32-bit offsets reach."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+LIMIT, ALPHA, SHIFT = 7.0, 1.702, 1.0
+
+
+def _reference(x, w, act):
+    """(result, bound of its float sum's error) of one expert's rows in 64 bits"""
+    z = x @ w.t()
+    dz = w.shape[1] * 2.0 ** -24 * (x.abs() @ w.abs().t())
+    if act == "relu2":
+        return z.clamp(min=0) ** 2, 2 * (z.abs() + dz) * dz
+    if act == "glu":
+        n = z.shape[1] // 32
+        g, u = z.view(-1, n, 2, 16).unbind(2)
+        dg, du = dz.view(-1, n, 2, 16).unbind(2)
+        g, u = g.clamp(max=LIMIT), u.clamp(-LIMIT, LIMIT)
+        # |d/dg g sigmoid(alpha g)| < 1.1, and a few units in the last place of the hardware's exponential and reciprocal
+        silu = g * torch.sigmoid(ALPHA * g)
+        y = silu * (u + SHIFT)
+        return y.reshape(-1, 16 * n), (1.1 * dg * (u + SHIFT).abs() + silu.abs() * du + 2.0 ** -19 * y.abs()).reshape(-1, 16 * n)
+    return z, dz
+
+
+@pytest.mark.parametrize("rows", [[1], [0, 33, 0, 31], [129, 0, 127], [128, 200], [256, 257], [1, 511, 128, 130], [0, 700]])
+@pytest.mark.parametrize("n, k", [(32, 8), (160, 72), (288, 64), (544, 200)])
+@pytest.mark.parametrize("act", ["none", "relu2", "glu"])
+def test_grouped_linear_edges(rows, n, k, act):
+    _check(rows, n, k, act, False)
+
+
+@pytest.mark.parametrize("rows", [[1, 30], [129, 0, 127], [256, 257]])
+def test_grouped_linear_of_rows_far_apart(rows):
+    _check(rows, 160, 200, "none", True)
+
+
+def _check(rows, n, k, act, far):
+    from hydrainfer_amd._C.kernel.moe_mix import grouped_linear
+    g = torch.Generator().manual_seed(len(rows) * 1000 + sum(rows) + n + k)
+    E, total = len(rows), sum(rows)
+    x = torch.randn((total, k), generator=g).bfloat16()
+    w = (torch.randn((E, n, k), generator=g) * k ** -0.5).bfloat16()
+    src = torch.randperm(total, generator=g).int()
+    seg = [0]
+    for r in rows:
+        seg.append(seg[-1] + r)
+    xd = x.cuda()
+    if far:                      # the same rows, (2^30 / rows) elements apart and more
+        stride = (2 ** 30 // total + 8) // 8 * 8 + 8
+        wide = torch.empty(total * stride, dtype=torch.bfloat16, device="cuda").view(total, stride)
+        wide[:, :k] = xd
+        xd = wide[:, :k]
+    segd = torch.tensor(seg, dtype=torch.int32, device="cuda")
+    for gather in (None, src):
+        got = grouped_linear(xd, w.cuda(), segd, total, src=None if gather is None else gather.cuda(), act=act, limit=LIMIT, alpha=ALPHA,
+                             up_shift=SHIFT).double().cpu()
+        xs = x.double() if gather is None else x.double()[gather.long()]
+        for e in range(E):
+            want, bound = _reference(xs[seg[e]:seg[e + 1]], w[e].double(), act)
+            off = (got[seg[e]:seg[e + 1]] - want).abs()
+            assert bool((off <= 2.0 ** -8 * want.abs() + 1.01 * bound + 1e-30).all()), (e, float(off.max()))      # one rounding to bfloat16
