@@ -10,10 +10,11 @@
 // a few DPP steps: nothing leaves the wave and no barrier stands in the serial chain.  Tokens go by in chunks of TC: the
 // chunk's q, k (and per-channel decays) come once per workgroup as float into LDS, zero-padded to PARTS * KR channels, and
 // are read back 16 bytes at a time; the next chunk is on its way into registers while the current one is scanned (two LDS
-// images, one barrier a chunk), so the serial chain waits for no global load.  The state comes from the sequence's slot
+// images, one barrier a chunk), so the serial chain waits for no global load.  Batches of single tokens, short portions and
+// keys of more than 128 channels (longer portions: chunk_scan.hip).  The state comes from the sequence's slot
 // (zeros for a portion that starts at position 0) and goes back.  KR x PARTS follows the key size (8 x 4 ... 16 x 16); a
-// launch of prompts with few workgroups takes more lanes a column, a batch of single tokens two columns a lane.
-#include "hx_common.h"
+// batch of single tokens takes two columns a lane.
+#include "chunk_scan.h"
 #include "mix_rows.h"
 #include "../../include/hydra_mix.h"
 
@@ -345,21 +346,24 @@ extern "C" int hxm_state_scan(const hxm_state_scan_args* args, void* stream) {
   if (a.q_stride < (int64_t)a.qk_heads * a.dim || a.k_stride < (int64_t)a.qk_heads * a.dim || a.v_stride < (int64_t)a.heads * a.vdim)
     return HX_ERR_STRIDE;
   hipStream_t s = (hipStream_t)stream;
-  // key channels a lane x lanes a column: 8 x 4, 8 x 8, 16 x 8, 16 x 16 (chunks of 16 tokens; 8 at the widest).  Portions of
-  // prompts in a launch that would leave compute units without a workgroup take twice the lanes a column and half the key
-  // channels a lane: twice the waves, each with half the serial work per token (measured at 4 x 1024 tokens, states of
-  // 128 x 128: 338 -> 290 us with 256 workgroups, 394 -> 435 us with 512; decode steps 26 -> 43 us: their state rows get
-  // too short).
-  static int n_cu = 0;
-  if (n_cu == 0) {
-    int dev = 0, v = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v < 1) v = 256;
-    n_cu = v;
+  // Portions of prompts go sixteen tokens at a time (chunk_scan.hip) where the sizes allow it, short ones one at a time here: a
+  // chunk costs its sixteen however few tokens it holds.  Measured with 32 heads of 128 x 128 under the delta rule: 32 portions of
+  // two tokens 48 us here, 61 us in chunks; 16 of four 30 and 33; 8 of sixteen 26 and 22; 32 of 64 217 and 139.
+  if (a.n_tokens >= 6 * (int64_t)a.n_seq) {
+    hxm::ChunkScanArgs c{};
+    c.out = a.out; c.q = a.q; c.k = a.k; c.v = a.v;
+    c.q_stride = a.q_stride; c.k_stride = a.k_stride; c.v_stride = a.v_stride;
+    c.q_dtype = a.q_dtype; c.k_dtype = a.k_dtype; c.v_dtype = a.v_dtype;
+    c.form = a.mode == HXM_SCAN_DECAY ? hxm::kChunkDecay : a.mode == HXM_SCAN_BONUS ? hxm::kChunkBonus : hxm::kChunkDelta;
+    c.per_channel = a.decay_per_channel;
+    c.decay = a.decay; c.vscale = a.vscale; c.beta = a.beta; c.bonus = a.bonus;
+    c.state = a.state; c.slot_stride = a.slot_stride; c.slots = a.slots; c.q_cu = a.q_cu; c.positions = a.positions;
+    c.n_seq = a.n_seq; c.heads = a.heads; c.qk_heads = a.qk_heads; c.K = a.dim; c.V = a.vdim;
+    if (hxm::chunk_scan_fits(c)) return hxm::chunk_scan(c, s);
   }
-  const bool prompt = a.n_tokens > a.n_seq;
-  auto few = [&](int cols) { return prompt && (int64_t)a.n_seq * a.heads * ((a.vdim + cols - 1) / cols) <= n_cu; };
+  // key channels a lane x lanes a column: 8 x 4, 8 x 8, 16 x 8, 16 x 16 (chunks of 16 tokens; 8 at the widest)
   if (a.dim <= 32) return launch_rows<8, 4, 16>(a, s);
-  if (a.dim <= 64) return few(32) ? launch_rows<4, 16, 16>(a, s) : launch_rows<8, 8, 16>(a, s);
-  if (a.dim <= 128) return few(32) ? launch_rows<8, 16, 16>(a, s) : launch_rows<16, 8, 16>(a, s);
+  if (a.dim <= 64) return launch_rows<8, 8, 16>(a, s);
+  if (a.dim <= 128) return launch_rows<16, 8, 16>(a, s);
   return launch_rows<16, 16, 8>(a, s);
 }

@@ -1,0 +1,122 @@
+"""Portions of prompts through the recurrences with a matrix state (csrc/chunk_scan.hip) against a token at a time in 64 bits:
+portions around the sixteen tokens of a chunk, single tokens beside them, keys and values that fill no tile, every operand
+type, rows that cannot be read four elements at a time, decays that vanish."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# 2-norm of the error over that of the result: sums of up to 128 + 16 products and products of up to 16 decays, a unit in the last
+# place (2^-24) each at worst a few of them in a row
+TOL = 32 * 2.0 ** -24
+
+
+def _scan(form, q, k, v, decay, vscale, beta, bonus, S, cu, fresh):
+    """One token at a time; q, k [T, H, K], v [T, H, V], decay [T, H, K], S [n, H, K, V], all double."""
+    out = torch.empty_like(v)
+    for s in range(len(cu) - 1):
+        X = torch.zeros_like(S[s]) if fresh[s] else S[s]
+        for t in range(cu[s], cu[s + 1]):
+            kv = lambda w: k[t][:, :, None] * w[:, None, :]
+            if form == "bonus":
+                out[t] = (q[t][:, None, :] @ (X + bonus[:, :, None] * kv(v[t])))[:, 0]
+                X = decay[t][:, :, None] * X + kv(v[t])
+            else:
+                X = decay[t][:, :, None] * X
+                w = v[t] * vscale[t][:, None]
+                if form == "delta":
+                    w = beta[t][:, None] * (v[t] - (k[t][:, None, :] @ X)[:, 0])
+                X = X + kv(w)
+                out[t] = (q[t][:, None, :] @ X)[:, 0]
+        S[s] = X
+    return out, S
+
+
+def _check(name, got, want, tol=TOL):
+    off = (got.double().cpu() - want).norm() / want.norm()
+    assert float(off) <= tol, (name, float(off))
+
+
+LENS = [[17], [16, 1, 33], [1, 15, 31, 2], [48, 5]]
+
+
+@pytest.mark.parametrize("lens", LENS)
+@pytest.mark.parametrize("K, V", [(64, 64), (128, 128), (12, 20), (100, 130), (65, 7)])
+@pytest.mark.parametrize("form, per_channel", [("decay", False), ("decay", True), ("delta", False), ("bonus", True)])
+@pytest.mark.parametrize("types", ["bf16", "f32", "mixed"])
+def test_portions_through_a_scan(lens, K, V, form, per_channel, types):
+    from hydrainfer_amd._C.kernel.seq_mix import state_scan
+    from hydrainfer_amd._C.kernel.stream_ops import SequenceState
+    g = torch.Generator().manual_seed(sum(lens) * 1000 + K + V)
+    n, T, H = len(lens), sum(lens), 4
+    G = H if form == "bonus" else 2
+    qk_t, v_t = (torch.bfloat16 if types == "bf16" else torch.float32), (torch.float32 if types == "f32" else torch.bfloat16)
+    unit = lambda x: torch.nn.functional.normalize(x, dim=-1)
+    proj = torch.cat([unit(torch.randn((T, G, K), generator=g)).reshape(T, G * K), unit(torch.randn((T, G, K), generator=g)).reshape(T, G * K),
+                      torch.zeros((T, 1))], dim=1).to(qk_t)       # (an odd row length: views that do not start on multiples of four)
+    q, k = proj[:, :G * K], proj[:, G * K:2 * G * K]
+    v = torch.randn((T, H * V), generator=g).to(v_t)
+    decay = torch.rand((T, H * K if per_channel else H), generator=g) ** 0.2
+    decay[T // 3] = 0.0                                            # forgets everything, and nothing divides by it
+    decay[T // 2, 0] = 1e-30
+    vscale, beta, bonus = torch.rand((T, H), generator=g), torch.rand((T, H), generator=g), torch.randn(H * K, generator=g)
+    state = torch.randn((n + 1, 1, H * K * V + 3), generator=g)
+    slots = torch.randperm(n + 1, generator=g)[:n].int()
+    cu = [0]
+    for x in lens:
+        cu.append(cu[-1] + x)
+    starts = [0 if s % 2 == 0 else 40 + s for s in range(n)]
+    pos = torch.tensor([starts[s] + i for s in range(n) for i in range(lens[s])], dtype=torch.int32)
+    tok_seq = torch.tensor([s for s in range(n) for _ in range(lens[s])], dtype=torch.int32)
+    heads = lambda x: x.double().view(T, G, K).repeat_interleave(H // G, dim=1)
+    want, S = _scan(form, heads(q), heads(k), v.double().view(T, H, V), (decay.double().view(T, H, -1)).expand(T, H, K),
+                    vscale.double() if form == "decay" else torch.ones((T, H), dtype=torch.float64), beta.double(), bonus.double().view(H, K),
+                    state[slots.long(), 0, 3:].double().view(n, H, K, V), cu, [p == 0 for p in starts])
+    d = lambda x: x.cuda()
+    st = d(state)
+    before = st.clone()
+    seq = SequenceState(st, d(slots), d(tok_seq))
+    pd = d(proj)
+    got = state_scan(form, pd[:, :G * K], pd[:, G * K:2 * G * K], d(v), d(decay), seq, 3, d(torch.tensor(cu, dtype=torch.int32)), d(pos), H, G, K, V,
+                     vscale=d(vscale) if form == "decay" else None, beta=d(beta) if form == "delta" else None, bonus=d(bonus) if form == "bonus" else None)
+    _check("out", got, want.reshape(T, H * V))
+    _check("state", st[slots.long().cuda(), 0, 3:].view(n, H, K, V), S)
+    other = [s for s in range(n + 1) if s not in slots.tolist()]
+    assert torch.equal(st[other], before[other]) and torch.equal(st[:, 0, :3], before[:, 0, :3])
+
+
+@pytest.mark.parametrize("lens", LENS)
+@pytest.mark.parametrize("K, V", [(64, 64), (128, 128), (12, 20), (100, 130), (65, 7)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_portions_through_the_gated_recurrence(lens, K, V, dtype):
+    from hydrainfer_amd._C.kernel.recurrence import gated_recurrence
+    from hydrainfer_amd._C.kernel.stream_ops import SequenceState
+    g = torch.Generator().manual_seed(sum(lens) * 1000 + K + V)
+    n, T, H, eps = len(lens), sum(lens), 3, 1e-5
+    proj = (2 * torch.randn((T, H * (2 * K + V) + 1), generator=g)).to(dtype)
+    proj[0, :4] = torch.tensor([300.0, -300.0, 90.0, -90.0])      # where a plain exponential leaves the range of a float
+    proj[1 % T, H * K:H * K + 4] = torch.tensor([300.0, -300.0, 90.0, -90.0])
+    f_bias, low, norm_w = torch.randn(H * K, generator=g), torch.rand(H * K, generator=g) ** 2, 1 + 0.1 * torch.randn(V, generator=g)
+    low[0] = 0.0
+    state = torch.randn((n, 2, H * K * V), generator=g)
+    cu = [0]
+    for x in lens:
+        cu.append(cu[-1] + x)
+    starts = [0 if s % 2 == 0 else 40 + s for s in range(n)]
+    pos = torch.tensor([starts[s] + i for s in range(n) for i in range(lens[s])], dtype=torch.int32)
+    tok_seq = torch.tensor([s for s in range(n) for _ in range(lens[s])], dtype=torch.int32)
+    x = proj.double()
+    f = low.double() + (1 - low.double()) * torch.sigmoid(x[:, H * K:2 * H * K] + f_bias.double())
+    q = torch.nn.functional.silu(x[:, :H * K])
+    ones = torch.ones((T, H), dtype=torch.float64)
+    o, S = _scan("decay", q.view(T, H, K), (1 - f).view(T, H, K), x[:, 2 * H * K:-1].reshape(T, H, V), f.view(T, H, K), ones, ones, None,
+                 state[:, 1].double().view(n, H, K, V), cu, [p == 0 for p in starts])
+    want = o / torch.sqrt((o * o).mean(-1, keepdim=True) + eps) * norm_w.double()
+    st, pd = state.cuda(), proj.cuda()
+    seq = SequenceState(st, torch.arange(n, dtype=torch.int32, device="cuda"), tok_seq.cuda())
+    got = gated_recurrence(pd[:, :H * K], pd[:, H * K:2 * H * K], pd[:, 2 * H * K:-1], f_bias.cuda(), low.cuda(), norm_w.cuda(), eps, seq, 1,
+                           torch.tensor(cu, dtype=torch.int32).cuda(), pos.cuda(), H, K, V, max_q_len=max(lens))
+    # (1 - f) is taken from a float f: an absolute 2^-24, the larger part of a small gate
+    _check("state", st[:, 1].view(n, H, K, V), S, 2 * TOL)
+    _check("out", got, want.reshape(T, H * V), 2 * TOL if dtype == torch.float32 else 2.0 ** -8)
+    assert torch.equal(st[:, 0].cpu(), state[:, 0])
