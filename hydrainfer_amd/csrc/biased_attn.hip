@@ -107,6 +107,11 @@ __device__ __forceinline__ void wave_lds_sync() {
 // a score under a soft cap: cap * tanh(s / cap); cap 0: the score itself
 __device__ __forceinline__ float capped(float s, float cap) { return cap > 0.f ? cap * tanhf(s / cap) : s; }
 
+// D[32 x 32] += A[32 x 16] B[16 x 32]; lane (c = l % 32, h = l / 32): A[c][8 h + j], B[8 h + j][c], D[(e & 3) + 8 (e / 4) + 4 h][c]
+__device__ __forceinline__ f32x16 mma32(u16x8 a, u16x8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
 // the first key a query at position i sees
 __device__ __forceinline__ int first_visible(int i, int kind, int size) {
   if (kind == HXM_MASK_WINDOW) return i - size + 1 > 0 ? i - size + 1 : 0;
@@ -585,6 +590,315 @@ __global__ __launch_bounds__(256) void biased_attn_group_kernel(hxm_biased_attn_
   }
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// Wide form (bfloat16, portions of prompts, key and value heads of 64 or 128, pages of whole 16-row groups): a workgroup of four
+// waves takes 128 rows, 32 a wave, of ONE (sequence, key head) and goes over the keys in tiles of 64.  The group form is bound by
+// LDS reads (a 16-byte read feeds one 16 x 16 x 32 product) and by the vector work of its softmax; here
+//   * the products are 32 x 32 x 16 and swapped, S^T = K Q^T and O^T += V^T P^T: a row of the softmax is one lane (its mask,
+//     slope, temperature are scalars of the lane, its maximum and sum one exchange with lane + 32), and P goes into the second
+//     product from the registers it was made in;
+//   * a tile's key and value rows go straight from the paged cache to LDS (1 KiB an instruction, whole rows), the next tile's
+//     while this one is worked on: two images, one barrier a tile.  Rows cannot be padded this way; their 16-byte chunks are
+//     swizzled by the lane that asks for them (keys: chunk ^ row, values: 64-byte quarter ^ row);
+//   * a row keeps the maximum it refers its weights to until a score exceeds it by 2^8: the accumulators are rarely rescaled.
+// The order of the row tiles: the XCDs (workgroups are dealt round robin) take key heads of their own where there are enough of
+// them, and of every sequence the tiles with the most keys come first.
+// Measured, 4 portions of 797 - 1151 tokens, 32 heads of 128 on 8 key heads, sinks: 221 us in the group form, 57 us
+// here (550 TFLOP/s of the pairs that a mask leaves); window of 512 and soft cap 223 and 61 us; chunks of 512 and slopes 163 and
+// 48 us.  Down to 64 rows of a key head it is the faster one (16 tokens behind 500 keys: 30 and 21 us).
+// ---------------------------------------------------------------------------------------------------------------
+template <int D, int V, bool MODS>      // MODS: slopes or a soft cap
+__global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_attn_args a, int tile_slots) {
+  constexpr int KT = 64, TQ = 128, KS = D / 16, NDB = V / 32;
+  constexpr int RSK = 2 * D, RSV = 2 * V, LK = D / 8, LV = V / 8;        // bytes and 16-byte chunks of a row
+  constexpr int KTILE = KT * RSK, IMG = KTILE + KT * RSV;
+  extern __shared__ __attribute__((aligned(16))) char smem_w[];        // [2][K tile | V tile]
+  auto kswz = [](int row) { return LK == 16 ? (row & 15) : ((row >> 1) & 7); };
+  auto vswz = [](int row) { return LV == 16 ? ((row & 3) << 2) : (((row >> 1) & 1) << 2); };
+  typedef __attribute__((address_space(4))) const int32_t c_i32;       // (uniform indices: through the scalar cache)
+  c_i32 *q_cu = (c_i32*)a.q_cu, *positions = (c_i32*)a.positions;
+  const int G = a.kv_heads, R = a.n_heads / a.kv_heads;
+
+  // workgroup -> (sequence, row tile, key head): within a sequence the last tiles, which see the most keys, first
+  int kvh, slot;
+  {
+    const int wg = blockIdx.x, total = tile_slots * G;
+    if (G % 8 == 0) {                        // XCD x: key heads x G / 8 ..
+      const int hp = G / 8, i = wg >> 3;
+      kvh = (wg & 7) * hp + i % hp;
+      slot = i / hp;
+    } else {
+      kvh = wg / tile_slots;
+      slot = wg - kvh * tile_slots;
+    }
+    if (wg >= total) return;
+  }
+  // (sequences in groups of four: the longest tile of each, then the second of each, ...)
+  int b = -1, tile = 0, q0 = 0, n_rows = 0;
+  for (int g0 = 0; g0 < a.n_seq && b < 0; g0 += 4) {
+    int cq[5], tl[4], group_tiles = 0, max_tiles = 0;
+#pragma unroll
+    for (int i = 0; i < 5; ++i) cq[i] = q_cu[min(g0 + i, a.n_seq)];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      tl[i] = ((cq[i + 1] - cq[i]) * R + TQ - 1) / TQ;
+      group_tiles += tl[i];
+      max_tiles = max(max_tiles, tl[i]);
+    }
+    if (slot >= group_tiles) { slot -= group_tiles; continue; }
+    for (int rank = 0; rank < max_tiles && b < 0; ++rank) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (b < 0 && tl[i] > rank) {
+          if (slot == 0) { b = g0 + i; tile = tl[i] - 1 - rank; q0 = cq[i]; n_rows = (cq[i + 1] - cq[i]) * R; }
+          --slot;
+        }
+      }
+    }
+  }
+  if (b < 0) return;                         // spare slot (the grid is an upper bound)
+  b = __builtin_amdgcn_readfirstlane(b);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int c = lane & 31, hi = lane >> 5;
+  // row tiles end with the portion: a partial one is the first, with the fewest keys.  Rows below 0 do not exist.
+  const int row0_wg = n_rows - ((n_rows + TQ - 1) / TQ - tile) * TQ, row0 = row0_wg + 32 * wave;
+  const int r = max(row0 + c, 0), tok = r / R, head = kvh * R + r % R;
+  const int pos = a.positions[q0 + tok];
+  const int lo = first_visible(pos, a.mask_kind, a.mask_size);
+  // what any row of the workgroup, of the wave sees (positions rise within a portion)
+  const int k_first = first_visible(positions[q0 + max(row0_wg, 0) / R], a.mask_kind, a.mask_size);
+  const int k_last = positions[q0 + (row0_wg + TQ - 1) / R];
+  const int wpos0 = positions[q0 + max(row0, 0) / R], wpos1 = positions[q0 + max(row0 + 31, 0) / R];
+  const int wlo0 = first_visible(wpos0, a.mask_kind, a.mask_size), wlo1 = first_visible(wpos1, a.mask_kind, a.mask_size);
+  const bool live = row0 + 31 >= 0;
+  const int t_first = k_first / KT, t_last = k_last / KT;
+
+  const u16* kc = (const u16*)a.key_cache + (int64_t)kvh * a.head_stride;
+  const u16* vc = (const u16*)a.value_cache + (int64_t)kvh * a.head_stride;
+  c_i32* table = (c_i32*)(a.block_table + ((c_i32*)a.cu_block_lens)[b]);
+  const int bs = a.block_size, bshift = (bs & (bs - 1)) == 0 ? __ffs(bs) - 1 : -1;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem_w;
+  // Wave w brings keys 16 w .. of a tile (one page): RPK / RPV rows an instruction, LK / LV lanes a row.
+  constexpr int RPK = 64 / LK, RPV = 64 / LV;
+  const int rk = lane / LK, ck = lane % LK, rv = lane / LV, cv = lane % LV;
+  auto bring = [&](int t, int img) __attribute__((always_inline)) {
+    const int key0 = min(t * KT + 16 * wave, k_last), r_max = k_last - key0;      // (rows past the last key repeat it; masked)
+    const int page = bshift >= 0 ? key0 >> bshift : key0 / bs;
+    const int64_t off = (int64_t)table[page] * a.cache_block_stride + (int64_t)(key0 - page * bs) * a.cache_row_stride;
+    const uint32_t kd = lds0 + (uint32_t)(img * IMG + 16 * wave * RSK), vd = lds0 + (uint32_t)(img * IMG + KTILE + 16 * wave * RSV);
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+    // (m0, the LDS address of the transfer, is a reserved register: nothing else in this kernel uses it)
+#pragma unroll
+    for (int j = 0; j < 16 / RPK; ++j) {
+      const int rr = RPK * j + rk;
+      const u16* from = kc + off + (int64_t)min(rr, r_max) * a.cache_row_stride + 8 * (ck ^ kswz(rr));
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(__builtin_amdgcn_readfirstlane(kd + 1024u * j)) : "memory", "m0");
+    }
+#pragma unroll
+    for (int j = 0; j < 16 / RPV; ++j) {
+      const int rr = RPV * j + rv;
+      const u16* from = vc + off + (int64_t)min(rr, r_max) * a.cache_row_stride + 8 * (cv ^ vswz(rr));
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(__builtin_amdgcn_readfirstlane(vd + 1024u * j)) : "memory", "m0");
+    }
+#pragma clang diagnostic pop
+  };
+  bring(t_first, 0);
+  // the queries (B operand): row c, columns 16 ks + 8 hi ..
+  u16x8 qf[KS];
+  {
+    const u16* qg = (const u16*)a.q + ((int64_t)(q0 + tok) * a.n_heads + head) * D + 8 * hi;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const u16x8*>(qg + 16 * ks);
+  }
+  // scores in units of log2: z = scale2 s - slope2 (pos - key), or under a cap cap2 tanh(s hsc / cap) in its place
+  constexpr float kLog2e = 1.4426950408889634f;
+  const float hsc = a.head_scale ? a.scale * a.head_scale[head] : a.scale;
+  const float slope2 = MODS && a.slopes ? a.slopes[head] * kLog2e : 0.f;
+  const bool cap = MODS && a.softcap > 0.f;
+  const float cap2 = cap ? a.softcap * kLog2e : 0.f;
+  float scale2 = cap ? 2.f * kLog2e * hsc / a.softcap : hsc * kLog2e;
+  if (!MODS) {             // (a maximum of scores is one of scaled scores where the scale is positive; -inf times it stays -inf)
+    if (scale2 < 0.f) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) qf[ks] ^= (u16)0x8000;
+    }
+    scale2 = fmaxf(fabsf(scale2), 1e-30f);
+  }
+
+  f32x16 acc[NDB];
+#pragma unroll
+  for (int i = 0; i < NDB; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[i][e] = 0.f;
+  float m = HX_NEG_BIG, l = 0.f;
+  // the transposing reads of V: lane 4 q + p of every 16 lanes brings row q, columns 16 half + 4 p ..
+  const int tr_q = (lane & 15) >> 2, tr_x = vswz(tr_q) >> 2;
+  const int tr_off = (4 * hi + tr_q) * RSV + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
+  auto tile_step = [&](int t, int img) __attribute__((always_inline)) {
+    const char* kt = smem_w + img * IMG;
+    const char* vt = kt + KTILE;
+    f32x16 s[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s[u][e] = 0.f;
+    {
+      // the keys' fragments of the first half before its products, those of the second under them
+      const char* krd = kt + c * RSK;
+      const int kz = kswz(c);
+      u16x8 ka[KS], kb[KS];
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) ka[ks] = *reinterpret_cast<const u16x8*>(krd + 16 * ((2 * ks + hi) ^ kz));
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        kb[ks] = *reinterpret_cast<const u16x8*>(krd + 32 * RSK + 16 * ((2 * ks + hi) ^ kz));
+        s[0] = mma32(ka[ks], qf[ks], s[0]);
+      }
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) s[1] = mma32(kb[ks], qf[ks], s[1]);
+      __builtin_amdgcn_sched_group_barrier(0x100, KS, 0);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, KS, 0);
+    }
+    // element e of half u: key t KT + 32 u + (e & 3) + 8 (e >> 2) + 4 hi
+    const int key_l = t * KT + 4 * hi;
+    float unit = scale2;                     // what a score still has to be multiplied by
+    if (MODS) {
+      unit = 1.f;
+      if (cap) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int e = 0; e < 16; ++e)       // cap2 tanh(y) = cap2 - 2 cap2 / (1 + e^(2 y))
+            s[u][e] = __builtin_fmaf(-2.f * cap2, __builtin_amdgcn_rcpf(1.f + fast_exp2(s[u][e] * scale2)), cap2);
+      } else {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) s[u][e] *= scale2;
+      }
+      if (a.slopes) {
+        const float base = slope2 * (float)(key_l - pos);
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) s[u][e] += __builtin_fmaf(slope2, (float)(32 * u + (e & 3) + 8 * (e >> 2)), base);
+      }
+    }
+    float mx = HX_NEG_BIG;
+    if (t * KT + KT - 1 <= wpos0 && t * KT >= wlo1) {      // every row of the wave sees the whole tile
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[u][e]);
+    } else {
+      const int last = pos - key_l, first = lo - key_l;
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int k = 32 * u + (e & 3) + 8 * (e >> 2);
+          if (k > last || k < first) s[u][e] = -INFINITY;
+          mx = fmaxf(mx, s[u][e]);
+        }
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float m_cand = fmaxf(m, mx * unit);
+    const bool grow = m_cand > m + 8.0f;
+    if (__builtin_amdgcn_ballot_w64(grow)) {
+      const float m_new = grow ? m_cand : m, alpha = fast_exp2(m - m_new);
+      l *= alpha;
+#pragma unroll
+      for (int i = 0; i < NDB; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][e] *= alpha;
+      m = m_new;
+    }
+    u16x8 pf[2][2];
+    float pa = 0.f, pb = 0.f;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int e = 0; e < 16; e += 2) {
+        const float e0 = fast_exp2(__builtin_fmaf(s[u][e], unit, -m)), e1 = fast_exp2(__builtin_fmaf(s[u][e + 1], unit, -m));
+        pa += e0;
+        pb += e1;
+        pf[u][e >> 3][e & 7] = BF16::from_float(e0);
+        pf[u][e >> 3][(e & 7) + 1] = BF16::from_float(e1);
+      }
+    l += pa + pb;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int k2 = 0; k2 < 2; ++k2) {
+        const char* vrd = vt + (32 * u + 16 * k2) * RSV + tr_off;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) {
+          const u16x4 x0 = lds_tr_read(vrd + 64 * (db ^ tr_x)), x1 = lds_tr_read(vrd + 8 * RSV + 64 * (db ^ tr_x));
+          acc[db] = mma32(u16x8{x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]}, pf[u][k2], acc[db]);
+        }
+      }
+  };
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  for (int t = t_first; t <= t_last; ++t) {
+    const int img = (t - t_first) & 1;
+    if (t < t_last) bring(t + 1, img ^ 1);
+    if (live && t * KT <= wpos1 && t * KT + KT - 1 >= wlo0) tile_step(t, img);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this wave's part of the next tile is there
+    __syncthreads();                                       // everybody's is, and this one has been read
+  }
+  if (!live) return;
+  // out, through LDS (the images are free): whole rows a store.  O[row c][column 32 db + 8 (e >> 2) + 4 hi + (e & 3)]
+  float total = l + __shfl_xor(l, 32, 64);
+  if (a.sinks) total += fast_exp2(a.sinks[head] * kLog2e - m);      // the sink: one more term, without a value
+  const float inv = 1.0f / total;
+  char* ob = smem_w + wave * 32 * RSV;
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+#pragma unroll
+    for (int e4 = 0; e4 < 4; ++e4) {
+      u16x4 o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = BF16::from_float(acc[db][4 * e4 + i] * inv);
+      *reinterpret_cast<u16x4*>(ob + c * RSV + (((8 * db + 2 * e4 + hi) ^ (c & (LV - 1))) << 3)) = o;
+    }
+  wave_lds_sync();
+#pragma unroll
+  for (int j = 0; j < 32 / RPV; ++j) {
+    const int rl = RPV * j + rv, ro = row0 + rl;
+    // 8-byte slots 2 ch, 2 ch + 1 of row rl sit in chunk ch ^ (rl' >> 1), in turned order when rl' is odd (rl' = rl mod V / 8)
+    u16x8 v = *reinterpret_cast<const u16x8*>(ob + rl * RSV + 16 * (cv ^ ((rl & (LV - 1)) >> 1)));
+    if (rl & 1) v = u16x8{v[4], v[5], v[6], v[7], v[0], v[1], v[2], v[3]};
+    if (ro >= 0) *reinterpret_cast<u16x8*>((u16*)a.out + ((int64_t)(q0 + ro / R) * a.n_heads + kvh * R + ro % R) * V + 8 * cv) = v;
+  }
+}
+
+template <int D, int V>
+int launch_wide(const hxm_biased_attn_args& a, hipStream_t s) {
+  // row tiles of all sequences, at most
+  const int R = a.n_heads / a.kv_heads;
+  const int64_t slots = ((int64_t)a.n_tokens * R + 127) / 128 + a.n_seq, grid = (slots * a.kv_heads + 7) / 8 * 8;
+  if (grid > 0x7fffffff) return HX_ERR_SHAPE;
+  const bool mods = a.slopes || a.softcap > 0.f;
+  auto kernel = mods ? biased_attn_wide_kernel<D, V, true> : biased_attn_wide_kernel<D, V, false>;
+  constexpr size_t lds = 2 * 64 * (2 * D + 2 * V);
+  if (lds > 48 * 1024) {
+    const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) {
+      hxm::last_hip_error() = (int)e;
+      return HX_ERR_HIP;
+    }
+  }
+  kernel<<<dim3((unsigned)grid), dim3(256), lds, s>>>(a, (int)slots);
+  return hxm::check_launch();
+}
+
 // the splits of a (sequence, kv head, row tile) merged: out = sum_s O_s e^(m_s - M) / sum_s l_s e^(m_s - M)
 __global__ __launch_bounds__(256) void biased_attn_combine_kernel(hxm_biased_attn_args a, int tiles_per_seq) {
   const int64_t item = blockIdx.x;
@@ -701,6 +1015,12 @@ extern "C" int hxm_biased_attention(const hxm_biased_attn_args* args, void* stre
   hipStream_t s = (hipStream_t)stream;
   if (a.n_splits > 1 && (a.n_splits > 64 || !a.ws_o || !a.ws_ml || !tile_form_serves(a))) return HX_ERR_WORKSPACE;
   if (tile_form_serves(a)) {
+    // portions of prompts with heads of 64 or 128 over pages of whole 16-row groups: from half a row tile of 128 on
+    const bool wide = (a.dim == 64 || a.dim == 128) && (a.vdim == 64 || a.vdim == 128);
+    if (wide && a.form != 2 && a.block_size % 16 == 0 && aligned16(a.out) && (int64_t)a.max_q_len * (a.n_heads / a.kv_heads) >= 64) {
+      if (a.dim == 64) return a.vdim == 64 ? launch_wide<64, 64>(a, s) : launch_wide<64, 128>(a, s);
+      return a.vdim == 64 ? launch_wide<128, 64>(a, s) : launch_wide<128, 128>(a, s);
+    }
     const int kk = ((a.dim > a.vdim ? a.dim : a.vdim) + 31) / 32;
     if (kk <= 1) return launch_tile<1>(a, s);
     if (kk <= 2) return launch_tile<2>(a, s);

@@ -1,0 +1,81 @@
+"""Biased attention over portions of prompts with heads of 64 and 128 (csrc/biased_attn.hip, the wide form) at the edges of its
+tiles — 128 rows of a key head, 64 keys — under every mask, with slopes, soft caps, temperatures of either sign and of zero,
+sinks, and other key than value sizes."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+BLOCK = 16
+
+
+def _first(mask, size, p):
+    return max(0, p - size + 1) if mask == "window" else p // size * size if mask == "chunk" else 0
+
+
+def _reference(q, k, v, pos, scale, slopes, mask, size, cap, sinks):
+    """(result, bound) for one sequence: q [n, H, D], k [keys, H, D], v [keys, H, V] in double"""
+    s = torch.einsum("nhd,khd->hnk", q, k) * scale[:, None, None]
+    if cap:
+        s = cap * torch.tanh(s / cap)
+    j = torch.arange(k.shape[0])
+    far = (torch.tensor(pos)[:, None] - j[None, :]).double()
+    if slopes is not None:
+        s = s - slopes[:, None, None] * far
+    seen = (far >= 0) & (j[None, :] >= torch.tensor([_first(mask, size, p) for p in pos])[:, None])
+    s = s.masked_fill(~seen[None], -math.inf)
+    if sinks is not None:
+        s = torch.cat([s, sinks[:, None, None].expand(-1, s.shape[1], 1)], dim=2)
+    p = torch.softmax(s, dim=2)[:, :, :k.shape[0]]
+    out = torch.einsum("hnk,khv->nhv", p, v)
+    # the weights and the result are rounded to bfloat16 once each: eight significant bits, so by up to 2^-8 of themselves (half of the
+    # last place, 2^-7, of a number just above a power of two); 1e-6 of what is summed for the float arithmetic
+    return out, 2.0 ** -8 * out.abs() + (2.0 ** -8 + 1e-6) * torch.einsum("hnk,khv->nhv", p, v.abs()) + 1e-6
+
+
+# (tokens brought, tokens held) of every sequence
+BATCHES = [[(16, 16)], [(31, 31), (33, 100)], [(64, 65), (1, 200), (32, 32)], [(129, 129)], [(127, 400), (5, 5), (16, 64), (40, 63), (17, 17)]]
+
+
+@pytest.mark.parametrize("batch", BATCHES)
+@pytest.mark.parametrize("H, G, D, V", [(4, 1, 128, 128), (32, 8, 64, 64), (6, 2, 128, 64), (16, 16, 64, 128)])
+@pytest.mark.parametrize("mask, size", [("causal", 0), ("window", 1), ("window", 63), ("chunk", 48)])
+@pytest.mark.parametrize("extra", ["plain", "slopes", "cap", "temperatures and sinks"])
+def test_wide_form(batch, H, G, D, V, mask, size, extra):
+    from hydrainfer_amd._C.kernel.biased_attn import biased_attention
+    g = torch.Generator().manual_seed(H * D + V + size + sum(a + b for a, b in batch))
+    new, kv = [a for a, _ in batch], [b for _, b in batch]
+    if max(new) * (H // G) < 64:
+        new[0], kv[0] = 64, max(64, kv[0])
+    nb = [(n + BLOCK - 1) // BLOCK for n in kv]
+    perm = torch.randperm(sum(nb) + 1, generator=g)
+    r = lambda *s: torch.randn(s, generator=g).bfloat16()
+    hs = max(D, V)
+    T, kc, vc = sum(new), r(sum(nb) + 1, BLOCK, G, hs), r(sum(nb) + 1, BLOCK, G, hs)
+    q = r(T, H, D)
+    q[0] *= 20                    # a row whose weights sit on one key
+    slopes = torch.tensor([2.0 ** (-8.0 * (h + 1) / H) for h in range(H)]) if extra == "slopes" else None
+    cap = 4.0 if extra == "cap" else 0.0
+    temps = sinks = None
+    if extra == "temperatures and sinks":
+        temps, sinks = torch.randn(H, generator=g), 2 * torch.randn(H, generator=g)
+        temps[0], sinks[1] = 0.0, -math.inf
+    cu_b = torch.tensor([0] + nb).cumsum(0).int()
+    cu_q = torch.tensor([0] + new).cumsum(0).int()
+    pos = [p for a, b in zip(new, kv) for p in range(b - a, b)]
+    seq = torch.tensor([s for s, a in enumerate(new) for _ in range(a)], dtype=torch.int32)
+    table = perm[:sum(nb)].int()
+    c = lambda t: None if t is None else t.cuda()
+    got = biased_attention(c(q), c(kc), c(vc), V, c(seq), c(torch.tensor(pos, dtype=torch.int32)), c(cu_q), c(table), c(cu_b), D ** -0.5, c(slopes), mask,
+                           size, max_q_len=max(new), max_kv_len=max(kv), softcap=cap, head_scale=c(temps), sinks=c(sinks)).double().cpu()
+    for s in range(len(new)):
+        lo, hi = int(cu_q[s]), int(cu_q[s + 1])
+        pages = table[int(cu_b[s]):int(cu_b[s + 1])].long()
+        k, v = (x[pages].reshape(-1, G, hs)[:kv[s]].double().repeat_interleave(H // G, dim=1) for x in (kc, vc))
+        scale = torch.full((H,), D ** -0.5, dtype=torch.float64) * (temps.double() if temps is not None else 1.0)
+        want, bound = _reference(q[lo:hi].double(), k[..., :D], v[..., :V], pos[lo:hi], scale, None if slopes is None else slopes.double(), mask, size, cap,
+                                 None if sinks is None else sinks.double())
+        off = (got[lo:hi] - want).abs()
+        assert bool((off <= bound).all()), (s, float((off - bound).max()))
