@@ -43,6 +43,68 @@ __device__ __forceinline__ int page_row(int key, int block_size, int block_shift
   return block_shift >= 0 ? key & (block_size - 1) : key % block_size;
 }
 
+// The least value over the wave, uniform (the vector ALU alone: four DPP steps and two swaps)
+template <int CTRL>
+__device__ __forceinline__ int dpp_int(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true); }
+__device__ __forceinline__ int wave_min_int(int v) {
+  v = min(v, dpp_int<0xB1>(v));       // lane ^ 1
+  v = min(v, dpp_int<0x4E>(v));       // lane ^ 2
+  v = min(v, dpp_int<0x141>(v));      // the half row's mirror image
+  v = min(v, dpp_int<0x140>(v));      // the row's
+  const auto a = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+  v = min((int)a[0], (int)a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+  return __builtin_amdgcn_readfirstlane(min((int)b[0], (int)b[1]));
+}
+__device__ __forceinline__ int wave_max_int(int v) { return -wave_min_int(-v); }
+
+// The slot-th (sequence, tile of TQ rows) pair of a batch whose sequences bring (cu[i + 1] - cu[i]) * per rows: sequences in groups of
+// four, of every group the last tile of each — it sees the most keys —, then the one before it of each, ...; row tiles end with
+// the portion, so that a partial tile is the first.  false: a spare slot.  cu: a uniform pointer (scalar loads).
+template <int TQ, typename P>
+__device__ __forceinline__ bool find_row_tile(P cu, int n_seq, int per, int slot, int& b, int& tile, int& q0, int& n_rows) {
+  for (int g0 = 0; g0 < n_seq; g0 += 4) {
+    int cq[5], tl[4], all = 0, most = 0;
+#pragma unroll
+    for (int i = 0; i < 5; ++i) cq[i] = cu[min(g0 + i, n_seq)];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      tl[i] = ((cq[i + 1] - cq[i]) * per + TQ - 1) / TQ;      // (0 past the last sequence: its offsets repeat)
+      all += tl[i];
+      most = max(most, tl[i]);
+    }
+    if (slot >= all) { slot -= all; continue; }
+    // the last rank with at most `slot` tiles in front of it (walked rank by rank a prompt's hundreds took microseconds)
+    auto before = [&](int rank) { return (min(tl[0], rank) + min(tl[1], rank)) + (min(tl[2], rank) + min(tl[3], rank)); };
+    int lo = 0, hi = most;
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (before(mid) <= slot) lo = mid;
+      else hi = mid;
+    }
+    // (turned from rank to rank: dealt round robin, the eight XCDs would else keep a sequence each, long or short)
+    const int there = (tl[0] > lo) + (tl[1] > lo) + (tl[2] > lo) + (tl[3] > lo);
+    slot = (slot - before(lo) + (lo >> 1)) % there;
+    b = -1;
+    tile = q0 = n_rows = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (b < 0 && tl[i] > lo) {
+        if (slot == 0) {
+          b = g0 + i;
+          tile = tl[i] - 1 - lo;
+          q0 = cq[i];
+          n_rows = (cq[i + 1] - cq[i]) * per;
+        }
+        --slot;
+      }
+    }
+    b = __builtin_amdgcn_readfirstlane(b);
+    return true;
+  }
+  return false;
+}
+
 struct AttnParams {
   void* out;
   const void* q;

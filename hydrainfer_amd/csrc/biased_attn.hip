@@ -603,9 +603,9 @@ __global__ __launch_bounds__(256) void biased_attn_group_kernel(hxm_biased_attn_
 //   * a row keeps the maximum it refers its weights to until a score exceeds it by 2^8: the accumulators are rarely rescaled.
 // The order of the row tiles: the XCDs (workgroups are dealt round robin) take key heads of their own where there are enough of
 // them, and of every sequence the tiles with the most keys come first.
-// Measured, 4 portions of 797 - 1151 tokens, 32 heads of 128 on 8 key heads, sinks: 221 us in the group form, 57 us
-// here (550 TFLOP/s of the pairs that a mask leaves); window of 512 and soft cap 223 and 61 us; chunks of 512 and slopes 163 and
-// 48 us.  Down to 64 rows of a key head it is the faster one (16 tokens behind 500 keys: 30 and 21 us).
+// Measured, 4 portions of 797 - 1151 tokens, 32 heads of 128 on 8 key heads, sinks: 221 us in the group form, 51 us
+// here (630 TFLOP/s of the pairs that a mask leaves); window of 512 and soft cap 223 and 58 us; chunks of 512 and slopes 163 and
+// 45 us.  Down to 64 rows of a key head it is the faster one (16 tokens behind 500 keys: 30 and 21 us).
 // ---------------------------------------------------------------------------------------------------------------
 template <int D, int V, bool MODS>      // MODS: slopes or a soft cap
 __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_attn_args a, int tile_slots) {
@@ -616,7 +616,7 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
   auto kswz = [](int row) { return LK == 16 ? (row & 15) : ((row >> 1) & 7); };
   auto vswz = [](int row) { return LV == 16 ? ((row & 3) << 2) : (((row >> 1) & 1) << 2); };
   typedef __attribute__((address_space(4))) const int32_t c_i32;       // (uniform indices: through the scalar cache)
-  c_i32 *q_cu = (c_i32*)a.q_cu, *positions = (c_i32*)a.positions;
+  c_i32* q_cu = (c_i32*)a.q_cu;
   const int G = a.kv_heads, R = a.n_heads / a.kv_heads;
 
   // workgroup -> (sequence, row tile, key head): within a sequence the last tiles, which see the most keys, first
@@ -633,31 +633,8 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
     }
     if (wg >= total) return;
   }
-  // (sequences in groups of four: the longest tile of each, then the second of each, ...)
-  int b = -1, tile = 0, q0 = 0, n_rows = 0;
-  for (int g0 = 0; g0 < a.n_seq && b < 0; g0 += 4) {
-    int cq[5], tl[4], group_tiles = 0, max_tiles = 0;
-#pragma unroll
-    for (int i = 0; i < 5; ++i) cq[i] = q_cu[min(g0 + i, a.n_seq)];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      tl[i] = ((cq[i + 1] - cq[i]) * R + TQ - 1) / TQ;
-      group_tiles += tl[i];
-      max_tiles = max(max_tiles, tl[i]);
-    }
-    if (slot >= group_tiles) { slot -= group_tiles; continue; }
-    for (int rank = 0; rank < max_tiles && b < 0; ++rank) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (b < 0 && tl[i] > rank) {
-          if (slot == 0) { b = g0 + i; tile = tl[i] - 1 - rank; q0 = cq[i]; n_rows = (cq[i + 1] - cq[i]) * R; }
-          --slot;
-        }
-      }
-    }
-  }
-  if (b < 0) return;                         // spare slot (the grid is an upper bound)
-  b = __builtin_amdgcn_readfirstlane(b);
+  int b, tile, q0, n_rows;
+  if (!find_row_tile<TQ>(q_cu, a.n_seq, R, slot, b, tile, q0, n_rows)) return;      // spare slot (the grid is an upper bound)
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int c = lane & 31, hi = lane >> 5;
   // row tiles end with the portion: a partial one is the first, with the fewest keys.  Rows below 0 do not exist.
@@ -665,11 +642,14 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
   const int r = max(row0 + c, 0), tok = r / R, head = kvh * R + r % R;
   const int pos = a.positions[q0 + tok];
   const int lo = first_visible(pos, a.mask_kind, a.mask_size);
-  // what any row of the workgroup, of the wave sees (positions rise within a portion)
-  const int k_first = first_visible(positions[q0 + max(row0_wg, 0) / R], a.mask_kind, a.mask_size);
-  const int k_last = positions[q0 + (row0_wg + TQ - 1) / R];
-  const int wpos0 = positions[q0 + max(row0, 0) / R], wpos1 = positions[q0 + max(row0 + 31, 0) / R];
-  const int wlo0 = first_visible(wpos0, a.mask_kind, a.mask_size), wlo1 = first_visible(wpos1, a.mask_kind, a.mask_size);
+  // what the rows of the wave see, and any row of the workgroup (every wave looks at all of them: no order of the positions is assumed)
+  const int wpos0 = wave_min_int(pos), wpos1 = wave_max_int(pos), wlo0 = wave_min_int(lo), wlo1 = wave_max_int(lo);
+  int k_first, k_last;
+  {
+    const int p0 = a.positions[q0 + max(row0_wg + lane, 0) / R], p1 = a.positions[q0 + max(row0_wg + 64 + lane, 0) / R];
+    k_first = wave_min_int(min(first_visible(p0, a.mask_kind, a.mask_size), first_visible(p1, a.mask_kind, a.mask_size)));
+    k_last = wave_max_int(max(p0, p1));
+  }
   const bool live = row0 + 31 >= 0;
   const int t_first = k_first / KT, t_last = k_last / KT;
 
@@ -710,6 +690,9 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
     const u16* qg = (const u16*)a.q + ((int64_t)(q0 + tok) * a.n_heads + head) * D + 8 * hi;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const u16x8*>(qg + 16 * ks);
+    // (they are there before the loop: a wait for them inside it would be one for the tile on its way)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[ks]));
   }
   // scores in units of log2: z = scale2 s - slope2 (pos - key), or under a cap cap2 tanh(s hsc / cap) in its place
   constexpr float kLog2e = 1.4426950408889634f;

@@ -64,7 +64,7 @@ def test_wide_form(batch, H, G, D, V, mask, size, extra):
         temps[0], sinks[1] = 0.0, -math.inf
     cu_b = torch.tensor([0] + nb).cumsum(0).int()
     cu_q = torch.tensor([0] + new).cumsum(0).int()
-    pos = [p for a, b in zip(new, kv) for p in range(b - a, b)]
+    pos = [p for a, b in zip(new, kv) for p in (range(b - a, b) if a % 2 else torch.randint(0, b, (a,), generator=g).tolist())]      # (even portions: in no order)
     seq = torch.tensor([s for s, a in enumerate(new) for _ in range(a)], dtype=torch.int32)
     table = perm[:sum(nb)].int()
     c = lambda t: None if t is None else t.cuda()
