@@ -7,6 +7,7 @@
 #include "../../include/hydra_mix.h"
 
 namespace hxm {
+int& last_hip_error();
 int check_launch();
 int& tile_form();      // 0: row form only (A/B measurements), 1: tile form where it applies
 }
@@ -779,6 +780,460 @@ __global__ __launch_bounds__(256) void latent_attn_group_kernel(hxm_latent_attn_
   }
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// Wide form (bfloat16, portions of prompts, latents of 64 KK columns, pages of whole 16-row groups): a workgroup of four waves takes
+// 128 rows, 32 a wave, and goes over the keys in tiles of 64 whose rows go straight from the paged cache to LDS, the next tile's
+// while this one is worked on.  The products are 32 x 32 x 16 and swapped, S^T = C Q^T and O^T += C^T P^T: a row of the softmax is a
+// lane, its weights go into the second product from the registers they were made in.  Both products read the one image: 16-byte
+// chunk x of row r sits at x ^ swz(r), with the row's two low bits above its next two, so that the 16 rows of one pass of a
+// 16-byte read as well as the four rows of a transposing read fall into different banks.
+// The tile and group forms read a row from LDS (or memory) once per 16 x 16 x 32 product; here a byte feeds twice the products.  A
+// lane holds 24 KK registers of queries and accumulators: two waves a SIMD up to 256 columns, one at 320; wider latents take the
+// form below.  (No register may spill here: the waits for scratch would be waits for the tile on its way.)
+// Measured, 4 portions of 1000 tokens: 256 columns, 16 heads 282 us in the tile form, 62 us here; 64 columns, 32 heads 141 and
+// 35 us; 320 columns under a window of 512, 16 heads 315 (group form) and 92 us.
+// ---------------------------------------------------------------------------------------------------------------
+__device__ __forceinline__ f32x16 mma32(u16x8 a, u16x8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+template <int KK>
+__global__ __launch_bounds__(256, KK <= 4 ? 2 : 1) void latent_attn_wide_kernel(hxm_latent_attn_args a) {
+  constexpr int R = 64 * KK, KT = 64, TQ = 128, KS = R / 16, NDB = R / 32, RS = 2 * R, L = R / 8, IMG = KT * RS;
+  constexpr bool FULL = RS % 256 == 0;       // a row is whole bank rows (256 bytes): 16 rows need 16 places, else 8 of each parity
+  extern __shared__ __attribute__((aligned(256))) char smem_w[];       // [2][64 rows]
+  auto swz = [](int row) { return FULL ? ((row & 3) << 2 | (row >> 2 & 3)) : ((row >> 1 & 1) << 2 | (row >> 2 & 3)); };
+  typedef __attribute__((address_space(4))) const int32_t c_i32;       // (uniform indices: through the scalar cache)
+  c_i32* q_cu = (c_i32*)a.q_cu;
+  const int H = a.n_heads;
+  int b, tile, q0, n_rows;
+  if (!find_row_tile<TQ>(q_cu, a.n_seq, H, blockIdx.x, b, tile, q0, n_rows)) return;      // spare slot (the grid is an upper bound)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int c = lane & 31, hi = lane >> 5;
+  // row tiles end with the portion: a partial one is the first, with the fewest keys.  Rows below 0 do not exist.
+  const int row0_wg = n_rows - ((n_rows + TQ - 1) / TQ - tile) * TQ, row0 = row0_wg + 32 * wave;
+  const int r = max(row0 + c, 0), tok = r / H, head = r % H;
+  auto first_key = [&](int p) { return a.window > 0 ? max(0, p - a.window + 1) : 0; };
+  const int pos = a.positions[q0 + tok], lo = first_key(pos);
+  // what the rows of the wave see, and any row of the workgroup (every wave looks at all of them: no order of the positions is assumed)
+  const int wpos0 = wave_min_int(pos), wpos1 = wave_max_int(pos), wlo0 = wave_min_int(lo), wlo1 = wave_max_int(lo);
+  int k_first, k_last;
+  {
+    const int p0 = a.positions[q0 + max(row0_wg + lane, 0) / H], p1 = a.positions[q0 + max(row0_wg + 64 + lane, 0) / H];
+    k_first = wave_min_int(min(first_key(p0), first_key(p1)));
+    k_last = wave_max_int(max(p0, p1));
+  }
+  const bool live = row0 + 31 >= 0;
+  const int t_first = k_first / KT, t_last = k_last / KT;
+
+  const u16* cache = (const u16*)a.cache;
+  c_i32* table = (c_i32*)(a.block_table + ((c_i32*)a.cu_block_lens)[b]);
+  const int bs = a.block_size, bshift = (bs & (bs - 1)) == 0 ? __ffs(bs) - 1 : -1;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem_w;
+  // Wave w brings keys 16 w .. of a tile (one page): 16 L chunks, 64 an instruction.
+  constexpr int NL = 16 * L / 64;
+  auto bring = [&](int t, int img) __attribute__((always_inline)) {
+    const int key0 = min(t * KT + 16 * wave, k_last), r_max = k_last - key0;      // (rows past the last key repeat it; masked)
+    const int page = bshift >= 0 ? key0 >> bshift : key0 / bs;
+    const u16* base = cache + (int64_t)table[page] * a.cache_block_stride + (int64_t)(key0 - page * bs) * a.cache_row_stride;
+    const uint32_t to = lds0 + (uint32_t)(img * IMG + 16 * wave * RS);
+    int ln = lane;
+    asm volatile("" : "+v"(ln));             // (worked out anew every time: kept, the addresses would push the queries out of registers)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+    // (m0, the LDS address of the transfer, is a reserved register: nothing else in this kernel uses it)
+#pragma unroll
+    for (int j = 0; j < NL; ++j) {
+      const int rr = (64 * j + ln) / L, ch = (64 * j + ln) % L;
+      const uint32_t off = (uint32_t)min(rr, r_max) * (uint32_t)(2 * a.cache_row_stride) + 16u * (uint32_t)(ch ^ swz(rr));
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(__builtin_amdgcn_readfirstlane(to + 1024u * j)) : "memory", "m0");
+    }
+#pragma clang diagnostic pop
+  };
+  bring(t_first, 0);
+  u16x8 qf[KS];                              // the queries (B operand): row c, columns 16 ks + 8 hi ..
+  {
+    const u16* qg = (const u16*)a.q + (int64_t)(q0 + tok) * a.q_token_stride + (int64_t)head * a.q_head_stride + 8 * hi;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const u16x8*>(qg + 16 * ks);
+    // (they are there before the loop: a wait for them inside it would be one for the tile on its way)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[ks]));
+  }
+  constexpr float kLog2e = 1.4426950408889634f;
+  float scale2 = a.scale * kLog2e;
+  if (scale2 < 0.f) {                        // (a maximum of scores is one of scaled scores where the scale is positive)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] ^= (u16)0x8000;
+  }
+  scale2 = fmaxf(fabsf(scale2), 1e-30f);
+
+  f32x16 acc[NDB];
+#pragma unroll
+  for (int i = 0; i < NDB; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[i][e] = 0.f;
+  float m = HX_NEG_BIG, l = 0.f;
+  // Reads of rows: chunk 2 ks + hi of row c.  The swizzle touches the low four bits of a chunk (three where rows are not whole
+  // bank rows): ks = NP x + y sits at x rows' worth of these and y bit by bit beside the place of ks = 0.
+  constexpr int NP = FULL ? 8 : 4;
+  const uint32_t kp0 = lds0 + (uint32_t)(c * RS + 16 * (hi ^ swz(c)));
+  // Transposing reads: lane 4 q + p of every 16 lanes brings row 4 hi + q (and the row 8 below it), columns 16 half + 4 p .. of a
+  // block of 32: chunks 4 db .. + 3, db = NB x + y the same way.
+  constexpr int NB = FULL ? 4 : 2;
+  uint32_t vp0, vp1;
+  {
+    const int q = (lane & 15) >> 2, p = lane & 3, x = 2 * ((lane >> 4) & 1) + (p >> 1);
+    vp0 = lds0 + (uint32_t)((4 * hi + q) * RS + 16 * (x ^ swz(4 * hi + q)) + 8 * (p & 1));
+    vp1 = lds0 + (uint32_t)((4 * hi + q + 8) * RS + 16 * (x ^ swz(4 * hi + q + 8)) + 8 * (p & 1));
+  }
+  auto row_read = [](uint32_t at) __attribute__((always_inline)) {
+    return *reinterpret_cast<__attribute__((address_space(3))) const u16x8*>((uintptr_t)at);
+  };
+  auto tr_read = [](uint32_t at) __attribute__((always_inline)) {
+    typedef __attribute__((address_space(3))) hx_s16x4_t lds_s4;
+    return __builtin_bit_cast(u16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(uintptr_t)at));
+  };
+  // 32 keys from key0 on, rows kt of the image (all 64 of a tile at once would not leave the registers for 512 columns)
+  auto step = [&](int key0, uint32_t kt) __attribute__((always_inline)) {
+    uint32_t kp = kp0, va = vp0, vb = vp1;
+    asm volatile("" : "+v"(kp), "+v"(va), "+v"(vb));      // (their sums are made where they are read, not kept in registers)
+    f32x16 s;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) s[e] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) s = mma32(row_read((kp ^ (32u * (ks % NP))) + kt + 32u * NP * (ks / NP)), qf[ks], s);
+    // (reads stay a few products ahead)
+    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+    for (int i = 0; i < KS - 4; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+    const int key_l = key0 + 4 * hi;         // element e: key key_l + (e & 3) + 8 (e >> 2)
+    float mx = HX_NEG_BIG;
+    if (key0 + 31 <= wpos0 && key0 >= wlo1) {              // every row of the wave sees all of them
+#pragma unroll
+      for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[e]);
+    } else {
+      const int last = pos - key_l, first = lo - key_l;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int k = (e & 3) + 8 * (e >> 2);
+        if (k > last || k < first) s[e] = -INFINITY;
+        mx = fmaxf(mx, s[e]);
+      }
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    // a row keeps the maximum its weights refer to until a score exceeds it by 2^8
+    const float m_cand = fmaxf(m, mx * scale2);
+    const bool grow = m_cand > m + 8.0f;
+    if (__builtin_amdgcn_ballot_w64(grow)) {
+      const float m_new = grow ? m_cand : m, alpha = fast_exp2(m - m_new);
+      l *= alpha;
+#pragma unroll
+      for (int i = 0; i < NDB; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][e] *= alpha;
+      m = m_new;
+    }
+    u16x8 pf[2];
+    float pa = 0.f, pb = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; e += 2) {
+      const float e0 = fast_exp2(__builtin_fmaf(s[e], scale2, -m)), e1 = fast_exp2(__builtin_fmaf(s[e + 1], scale2, -m));
+      pa += e0;
+      pb += e1;
+      pf[e >> 3][e & 7] = BF16::from_float(e0);
+      pf[e >> 3][(e & 7) + 1] = BF16::from_float(e1);
+    }
+    l += pa + pb;
+#pragma unroll
+    for (int k2 = 0; k2 < 2; ++k2) {
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) {
+        const uint32_t at = kt + 16u * k2 * RS + 64u * NB * (db / NB);
+        const u16x4 x0 = tr_read((va ^ (64u * (db % NB))) + at), x1 = tr_read((vb ^ (64u * (db % NB))) + at);
+        acc[db] = mma32(u16x8{x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]}, pf[k2], acc[db]);
+      }
+    }
+    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+    for (int i = 0; i < 2 * NDB - 2; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+  };
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  for (int t = t_first; t <= t_last; ++t) {
+    const int img = (t - t_first) & 1;
+    if (t < t_last) bring(t + 1, img ^ 1);
+#pragma unroll 1
+    for (int key0 = t * KT; key0 < t * KT + KT; key0 += 32)
+      if (live && key0 <= wpos1 && key0 + 31 >= wlo0) step(key0, (uint32_t)(img * IMG + (key0 - t * KT) * RS));
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this wave's part of the next tile is there
+    __syncthreads();                                       // everybody's is, and this one has been read
+  }
+  if (!live) return;
+  // out, through LDS (the images are free): whole rows a store.  O[row c][column 32 db + 8 (e >> 2) + 4 hi + (e & 3)]
+  float total = l + __shfl_xor(l, 32, 64);
+  if (a.sinks) total += fast_exp2(a.sinks[head] * kLog2e - m);      // the sink: one more term, without a value
+  float gsc = 1.0f / total;
+  if (a.gate_pre) {
+    const float z = BF16::to_float(((const u16*)a.gate_pre)[(int64_t)(q0 + tok) * a.gate_stride + head]);
+    gsc = gsc / (1.0f + __expf(-z));
+  }
+  char* ob = smem_w + wave * 32 * RS;
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+#pragma unroll
+    for (int e4 = 0; e4 < 4; ++e4) {         // 8-byte slot 8 db + 2 e4 + hi of row c, turned by the row within its 128 bytes
+      u16x4 o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = BF16::from_float(acc[db][4 * e4 + i] * gsc);
+      *reinterpret_cast<u16x4*>(ob + c * RS + (((8 * db + 2 * e4 + hi) ^ (c & 15)) << 3)) = o;
+    }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+  for (int j = 0; j < 2 * NL; ++j) {
+    const int rl = (64 * j + lane) / L, ch = (64 * j + lane) % L, ro = row0 + rl;
+    // slots 2 ch, 2 ch + 1 of row rl sit in chunk ch ^ (rl' >> 1), in turned order when rl' is odd (rl' = rl mod 16)
+    u16x8 v = *reinterpret_cast<const u16x8*>(ob + rl * RS + 16 * (ch ^ ((rl & 15) >> 1)));
+    if (rl & 1) v = u16x8{v[4], v[5], v[6], v[7], v[0], v[1], v[2], v[3]};
+    if (ro >= 0) *reinterpret_cast<u16x8*>((u16*)a.out + (int64_t)(q0 + ro / H) * a.out_token_stride + (int64_t)(ro % H) * a.out_head_stride + 8 * ch) = v;
+  }
+}
+
+// The same for wider latents (64 KK columns, KK even): four waves of 16 rows, 16 x 16 x 32 products — a row's queries and
+// accumulators are 192 registers a lane at 512 columns, two waves a SIMD.  A byte from LDS feeds half the products of the form
+// above; it is bound by the latency and number of its LDS reads (without those of the keys the same launch takes three quarters of
+// the time).  Tiles of 32 keys and 64 rows: two workgroups a CU, one working while the other brings queries in or results out.
+// Measured, 4 portions of 797 - 1151 tokens, 32 heads, 512 columns: 861 us in the group form, 226 us here (560 TFLOP/s; 780
+// behind long contexts, where less of the time goes to queries and results).  Row r of sixteen has its chunks at x ^ swz(r): rows r and 15 - r share a 32-byte place (their
+// chunks turned), so that a pass of a 16-byte read (rows 0-3 and 12-15 of one chunk, 4-11 of the next) and a transposing read
+// (eight rows, 32 bytes each) both reach every bank once.
+__device__ __forceinline__ float groups_max(float v) {      // over the four lanes with the same lane % 16
+  const auto a = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
+  const unsigned a0 = a[0], a1 = a[1];
+  v = fmaxf(__builtin_bit_cast(float, a0), __builtin_bit_cast(float, a1));
+  const auto b = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
+  const unsigned b0 = b[0], b1 = b[1];
+  return fmaxf(__builtin_bit_cast(float, b0), __builtin_bit_cast(float, b1));
+}
+
+template <int KK>
+__global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_attn_args a) {
+  constexpr int R = 64 * KK, KT = 32, TQ = 64, KS = R / 32, NDB = R / 16, RS = 2 * R, L = R / 8, IMG = KT * RS;
+  static_assert(RS % 256 == 0, "rows of whole bank rows");
+  extern __shared__ __attribute__((aligned(256))) char smem_w[];       // [2][32 rows]
+  auto swz = [](int row) { return (row & 15) < 8 ? 2 * (row & 7) : 31 - 2 * (row & 15); };
+  typedef __attribute__((address_space(4))) const int32_t c_i32;       // (uniform indices: through the scalar cache)
+  c_i32* q_cu = (c_i32*)a.q_cu;
+  const int H = a.n_heads;
+  int b, tile, q0, n_rows;
+  if (!find_row_tile<TQ>(q_cu, a.n_seq, H, blockIdx.x, b, tile, q0, n_rows)) return;      // spare slot (the grid is an upper bound)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int c = lane & 15, g = lane >> 4;
+  const int row0_wg = n_rows - ((n_rows + TQ - 1) / TQ - tile) * TQ, row0 = row0_wg + 16 * wave;
+  const int r = max(row0 + c, 0), tok = r / H, head = r % H;
+  auto first_key = [&](int p) { return a.window > 0 ? max(0, p - a.window + 1) : 0; };
+  const int pos = a.positions[q0 + tok], lo = first_key(pos);
+  const int wpos0 = wave_min_int(pos), wpos1 = wave_max_int(pos), wlo0 = wave_min_int(lo), wlo1 = wave_max_int(lo);
+  static_assert(TQ == 64, "a lane looks at one row of the workgroup");
+  const int p_wg = a.positions[q0 + max(row0_wg + lane, 0) / H];
+  const int k_first = wave_min_int(first_key(p_wg)), k_last = wave_max_int(p_wg);
+  const bool live = row0 + 15 >= 0;
+  const int t_first = k_first / KT, t_last = k_last / KT;
+
+  const u16* cache = (const u16*)a.cache;
+  c_i32* table = (c_i32*)(a.block_table + ((c_i32*)a.cu_block_lens)[b]);
+  const int bs = a.block_size, bshift = (bs & (bs - 1)) == 0 ? __ffs(bs) - 1 : -1;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem_w;
+  // Wave w brings keys 8 w .. of a tile (one page): 8 L chunks, 64 an instruction.
+  constexpr int NL = 8 * L / 64;
+  auto bring = [&](int t, int img) __attribute__((always_inline)) {
+    const int key0 = min(t * KT + 8 * wave, k_last), r_max = k_last - key0;       // (rows past the last key repeat it; masked)
+    const int page = bshift >= 0 ? key0 >> bshift : key0 / bs;
+    const u16* base = cache + (int64_t)table[page] * a.cache_block_stride + (int64_t)(key0 - page * bs) * a.cache_row_stride;
+    const uint32_t to = lds0 + (uint32_t)(img * IMG + 8 * wave * RS);
+    int ln = lane;
+    asm volatile("" : "+v"(ln));             // (worked out anew every time: kept, the addresses would push the queries out of registers)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+    // (m0, the LDS address of the transfer, is a reserved register: nothing else in this kernel uses it)
+#pragma unroll
+    for (int j = 0; j < NL; ++j) {
+      const int rr = (64 * j + ln) / L, ch = (64 * j + ln) % L;
+      const uint32_t off = (uint32_t)min(rr, r_max) * (uint32_t)(2 * a.cache_row_stride) + 16u * (uint32_t)(ch ^ swz(8 * (wave & 1) + rr));
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(__builtin_amdgcn_readfirstlane(to + 1024u * j)) : "memory", "m0");
+    }
+#pragma clang diagnostic pop
+  };
+  bring(t_first, 0);
+  u16x8 qf[KS];                              // the queries (B operand): row c, columns 32 ks + 8 g ..
+  {
+    const u16* qg = (const u16*)a.q + (int64_t)(q0 + tok) * a.q_token_stride + (int64_t)head * a.q_head_stride + 8 * g;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const u16x8*>(qg + 32 * ks);
+    // (they are there before the loop: a wait for them inside it would be one for the tile on its way)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[ks]));
+  }
+  constexpr float kLog2e = 1.4426950408889634f;
+  float scale2 = a.scale * kLog2e;
+  if (scale2 < 0.f) {                        // (a maximum of scores is one of scaled scores where the scale is positive)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] ^= (u16)0x8000;
+  }
+  scale2 = fmaxf(fabsf(scale2), 1e-30f);
+  f32x4 acc[NDB];
+#pragma unroll
+  for (int i = 0; i < NDB; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = HX_NEG_BIG, l = 0.f;
+  // Reads of rows: chunk 4 ks + g of row c; the swizzle touches the low four bits of a chunk, ks = 4 x + y.  Transposing reads:
+  // lane 4 q + p of a group of 16 brings row 4 g + q (and the row 16 below it: the same place), columns 16 db + 4 p ..: chunk
+  // 2 db + p / 2, db = 8 x + y.
+  const uint32_t kp0 = lds0 + (uint32_t)(c * RS + 16 * (g ^ swz(c)));
+  const uint32_t vp0 = lds0 + (uint32_t)((4 * g + (c >> 2)) * RS + 16 * (((c & 3) >> 1) ^ swz(4 * g + (c >> 2))) + 8 * (c & 1));
+  auto row_read = [](uint32_t at) __attribute__((always_inline)) {
+    return *reinterpret_cast<__attribute__((address_space(3))) const u16x8*>((uintptr_t)at);
+  };
+  auto tr_read = [](uint32_t at) __attribute__((always_inline)) {
+    typedef __attribute__((address_space(3))) hx_s16x4_t lds_s4;
+    return __builtin_bit_cast(u16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(uintptr_t)at));
+  };
+  // 32 keys from key0 on, rows kt of the image
+  auto step = [&](int key0, uint32_t kt) __attribute__((always_inline)) {
+    uint32_t kp = kp0 + kt, va = vp0 + kt;
+    asm volatile("" : "+v"(kp), "+v"(va));   // (their sums are made where they are read, not kept in registers)
+    f32x4 s[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) s[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) s[u] = Mfma<BF16>::mma(row_read((kp ^ (64u * (ks % 4))) + 16u * u * RS + 256u * (ks / 4)), qf[ks], s[u]);
+    // (reads stay a few products ahead)
+    __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+#pragma unroll
+    for (int i = 0; i < 2 * KS - 8; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+    const int key_l = key0 + 4 * g;          // element e of half u: key key_l + 16 u + e
+    float mx = HX_NEG_BIG;
+    if (key0 + 31 <= wpos0 && key0 >= wlo1) {              // every row of the wave sees all of them
+#pragma unroll
+      for (int e = 0; e < 8; ++e) mx = fmaxf(mx, s[e >> 2][e & 3]);
+    } else {
+      const int last = pos - key_l, first = lo - key_l;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int k = 16 * (e >> 2) + (e & 3);
+        if (k > last || k < first) s[e >> 2][e & 3] = -INFINITY;
+        mx = fmaxf(mx, s[e >> 2][e & 3]);
+      }
+    }
+    mx = groups_max(mx);
+    // a row keeps the maximum its weights refer to until a score exceeds it by 2^8
+    const float m_cand = fmaxf(m, mx * scale2);
+    const bool grow = m_cand > m + 8.0f;
+    if (__builtin_amdgcn_ballot_w64(grow)) {
+      const float m_new = grow ? m_cand : m, alpha = fast_exp2(m - m_new);
+      l *= alpha;
+#pragma unroll
+      for (int i = 0; i < NDB; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][e] *= alpha;
+      m = m_new;
+    }
+    u16x8 pf;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float p = fast_exp2(__builtin_fmaf(s[e >> 2][e & 3], scale2, -m));
+      l += p;
+      pf[e] = BF16::from_float(p);
+    }
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) {
+      const uint32_t at = (va ^ (32u * (db % 8))) + 256u * (db / 8);
+      const u16x4 x0 = tr_read(at), x1 = tr_read(at + 16u * RS);
+      acc[db] = Mfma<BF16>::mma(u16x8{x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]}, pf, acc[db]);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x100, 12, 0);
+#pragma unroll
+    for (int i = 0; i < NDB - 6; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
+  };
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  for (int t = t_first; t <= t_last; ++t) {
+    const int img = (t - t_first) & 1;
+    if (t < t_last) bring(t + 1, img ^ 1);
+    if (live && t * KT <= wpos1 && t * KT + KT - 1 >= wlo0) step(t * KT, (uint32_t)(img * IMG));
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this wave's part of the next tile is there
+    __syncthreads();                                       // everybody's is, and this one has been read
+  }
+  if (!live) return;
+  // out, through LDS (the images are free): whole rows a store.  O[row c][column 16 db + 4 g + e]
+  float total = l + __shfl_xor(l, 16, 64);
+  total += __shfl_xor(total, 32, 64);
+  if (a.sinks) total += fast_exp2(a.sinks[head] * kLog2e - m);      // the sink: one more term, without a value
+  float gsc = 1.0f / total;
+  if (a.gate_pre) {
+    const float z = BF16::to_float(((const u16*)a.gate_pre)[(int64_t)(q0 + tok) * a.gate_stride + head]);
+    gsc = gsc / (1.0f + __expf(-z));
+  }
+  char* ob = smem_w + wave * 16 * RS;
+#pragma unroll
+  for (int db = 0; db < NDB; ++db) {         // 8-byte slot 4 db + g of row c, turned by the row within its 128 bytes
+    u16x4 o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = BF16::from_float(acc[db][i] * gsc);
+    *reinterpret_cast<u16x4*>(ob + c * RS + (((4 * db + g) ^ c) << 3)) = o;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+  for (int j = 0; j < 2 * NL; ++j) {
+    const int rl = (64 * j + lane) / L, ch = (64 * j + lane) % L, ro = row0 + rl;
+    // slots 2 ch, 2 ch + 1 of row rl sit in chunk ch ^ (rl >> 1), in turned order when rl is odd
+    u16x8 v = *reinterpret_cast<const u16x8*>(ob + rl * RS + 16 * (ch ^ (rl >> 1)));
+    if (rl & 1) v = u16x8{v[4], v[5], v[6], v[7], v[0], v[1], v[2], v[3]};
+    if (ro >= 0) *reinterpret_cast<u16x8*>((u16*)a.out + (int64_t)(q0 + ro / H) * a.out_token_stride + (int64_t)(ro % H) * a.out_head_stride + 8 * ch) = v;
+  }
+}
+
+template <int KK>
+int launch_wide(const hxm_latent_attn_args& a, hipStream_t s) {
+  constexpr int rows = KK <= 5 ? 128 : 64, keys = KK <= 5 ? 64 : 32;
+  const int64_t grid = ((int64_t)a.n_tokens * a.n_heads + rows - 1) / rows + a.n_seq;      // row tiles of all sequences, at most
+  if (grid > 0x7fffffff) return HX_ERR_SHAPE;
+  constexpr size_t lds = 2 * keys * 2 * 64 * KK;
+  void (*kernel)(hxm_latent_attn_args);
+  if constexpr (KK <= 5) kernel = latent_attn_wide_kernel<KK>;
+  else kernel = latent_attn_wide16_kernel<KK>;
+  if (lds > 48 * 1024) {
+    const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) {
+      hxm::last_hip_error() = (int)e;
+      return HX_ERR_HIP;
+    }
+  }
+  kernel<<<dim3((unsigned)grid), dim3(256), lds, s>>>(a);
+  return hxm::check_launch();
+}
+
 // the splits of a (sequence, row tile) merged: out = sum_s O_s e^(m_s - M) / sum_s l_s e^(m_s - M), times the head gate
 __global__ __launch_bounds__(256) void latent_attn_combine_kernel(hxm_latent_attn_args a, int tiles_per_seq) {
   const int64_t item = blockIdx.x;
@@ -917,6 +1372,18 @@ extern "C" int hxm_latent_attention(const hxm_latent_attn_args* args, void* stre
   hipStream_t s = (hipStream_t)stream;
   if (a.max_q_len < 1) return HX_ERR_SHAPE;
   if (tile_form_serves(a)) {
+    if (a.kv_rank % 64 == 0 && a.kv_rank != 448 && a.block_size % 16 == 0 && a.out_token_stride % 8 == 0 && a.out_head_stride % 8 == 0 && aligned16(a.out) &&
+        (int64_t)a.max_q_len * a.n_heads >= 64 && a.max_q_len > 1 && a.cache_row_stride < (1 << 26) && hxm::tile_form() == 1) {
+      switch (a.kv_rank / 64) {
+        case 1: return launch_wide<1>(a, s);
+        case 2: return launch_wide<2>(a, s);
+        case 3: return launch_wide<3>(a, s);
+        case 4: return launch_wide<4>(a, s);
+        case 5: return launch_wide<5>(a, s);
+        case 6: return launch_wide<6>(a, s);
+        default: return launch_wide<8>(a, s);
+      }
+    }
     switch ((a.kv_rank + 31) / 32) {
       case 1: return launch_tile<1>(a, s);
       case 2: return launch_tile<2>(a, s);

@@ -1,0 +1,58 @@
+"""Latent attention over portions of prompts (csrc/latent_attn.hip, the wide forms: 64 to 320 columns, 384 and 512) at the edges of
+their tiles — 128 or 64 rows of token and head, 64 or 32 keys — with windows, sinks, gates, a negative scale, queries and results
+as views of other layouts."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+BLOCK = 16
+# (tokens brought, tokens held) of every sequence
+BATCHES = [[(2, 2)], [(33, 33), (2, 100)], [(5, 70), (1, 200), (32, 32)], [(129, 129)], [(40, 400), (5, 5), (16, 64), (31, 63), (17, 17)]]
+
+
+@pytest.mark.parametrize("batch", BATCHES)
+@pytest.mark.parametrize("R", [64, 128, 192, 256, 320, 384, 512])
+@pytest.mark.parametrize("H", [3, 32])
+@pytest.mark.parametrize("window, extra", [(0, "plain"), (1, "plain"), (31, "sinks"), (50, "gate"), (0, "negative"), (64, "sinks and gate")])
+def test_wide_forms(batch, R, H, window, extra):
+    from hydrainfer_amd._C.kernel.latent_attn import latent_attention
+    g = torch.Generator().manual_seed(R * 100 + H + window + sum(a + b for a, b in batch))
+    new, kv = [a for a, _ in batch], [b for _, b in batch]
+    if max(new) * H < 64:
+        new[0], kv[0] = 22, max(22, kv[0])
+    nb = [(n + BLOCK - 1) // BLOCK for n in kv]
+    T, perm = sum(new), torch.randperm(sum(nb) + 1, generator=g)
+    cache = torch.randn((sum(nb) + 1, BLOCK, 1, R + 8), generator=g).bfloat16()      # rows wider than the latent
+    q = torch.randn((H, T, R), generator=g).bfloat16()
+    q[0, 0] *= 20                 # a row whose weights sit on one key
+    scale = (-1.0 if extra == "negative" else 1.0) * R ** -0.5
+    sinks = 2 * torch.randn(H, generator=g) if "sinks" in extra else None
+    gate = torch.randn((T, H + 5), generator=g).bfloat16() if "gate" in extra else None
+    cu_b, cu_q = torch.tensor([0] + nb).cumsum(0).int(), torch.tensor([0] + new).cumsum(0).int()
+    pos = [p for a, b in zip(new, kv) for p in (range(b - a, b) if a % 2 else torch.randint(0, b, (a,), generator=g).tolist())]      # (even portions: in no order)
+    seq = torch.tensor([s for s, a in enumerate(new) for _ in range(a)], dtype=torch.int32)
+    table = perm[:sum(nb)].int()
+    c = lambda t: None if t is None else t.cuda()
+    out = torch.full((H, T, R), 7.0, dtype=torch.bfloat16, device="cuda")
+    latent_attention(c(q).transpose(0, 1), c(cache), c(seq), c(torch.tensor(pos, dtype=torch.int32)), c(cu_q), c(table), c(cu_b), scale, window or None,
+                     max(new), gate_pre=c(gate), out=out.transpose(0, 1), max_kv_len=max(kv), sinks=c(sinks))
+    got = out.double().cpu()
+    for s in range(len(new)):
+        lo, hi = int(cu_q[s]), int(cu_q[s + 1])
+        k = cache[table[int(cu_b[s]):int(cu_b[s + 1])].long()].reshape(-1, R + 8)[:kv[s], :R].double()
+        z = torch.matmul(q[:, lo:hi].double(), k.t()) * scale
+        far = torch.tensor(pos[lo:hi])[:, None] - torch.arange(kv[s])[None, :]
+        z = z.masked_fill(((far < 0) | (far >= window if window else far < 0))[None], -math.inf)
+        if sinks is not None:
+            z = torch.cat([z, sinks.double()[:, None, None].expand(-1, hi - lo, 1)], dim=2)
+        p = torch.softmax(z, dim=2)[:, :, :kv[s]]
+        f = torch.sigmoid(gate[lo:hi, :H].double()).t()[:, :, None] if gate is not None else 1.0
+        want, size = torch.matmul(p, k) * f, torch.matmul(p, k.abs()) * f
+        # the weights and the result are rounded to bfloat16 once each: eight significant bits, so by up to 2^-8 of themselves; 1e-6 of what
+        # is summed for the float arithmetic
+        bound = 2.0 ** -8 * want.abs() + (2.0 ** -8 + 1e-6) * size + 1e-6
+        off = (got[:, lo:hi] - want).abs()
+        assert bool((off <= bound).all()), (s, float((off - bound).max()))
