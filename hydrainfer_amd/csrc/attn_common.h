@@ -60,20 +60,33 @@ __device__ __forceinline__ int wave_max_int(int v) { return -wave_min_int(-v); }
 
 // The slot-th (sequence, tile of TQ rows) pair of a batch whose sequences bring (cu[i + 1] - cu[i]) * per rows: sequences in groups of
 // four, of every group the last tile of each — it sees the most keys —, then the one before it of each, ...; row tiles end with
-// the portion, so that a partial tile is the first.  false: a spare slot.  cu: a uniform pointer (scalar loads).
+// the portion, so that a partial tile is the first.  false: a spare slot.  Every lane counts one group's tiles: one round of loads
+// for 256 sequences (walked a group at a time, a decode of 32 waited for eight).
 template <int TQ, typename P>
 __device__ __forceinline__ bool find_row_tile(P cu, int n_seq, int per, int slot, int& b, int& tile, int& q0, int& n_rows) {
-  for (int g0 = 0; g0 < n_seq; g0 += 4) {
-    int cq[5], tl[4], all = 0, most = 0;
+  const int lane = threadIdx.x & 63;
+  for (int base = 0; base < n_seq; base += 256) {
+    int cq[5], tl[4], upto = 0, most = 0;
 #pragma unroll
-    for (int i = 0; i < 5; ++i) cq[i] = cu[min(g0 + i, n_seq)];
+    for (int i = 0; i < 5; ++i) cq[i] = cu[min(base + 4 * lane + i, n_seq)];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) upto += ((cq[i + 1] - cq[i]) * per + TQ - 1) / TQ;      // (0 past the last sequence: its offsets repeat)
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int v = __shfl_up(upto, off, 64);
+      if (lane >= off) upto += v;
+    }
+    const uint64_t past = __builtin_amdgcn_ballot_w64(upto > slot);
+    if (!past) { slot -= __builtin_amdgcn_readlane(upto, 63); continue; }
+    const int at = __builtin_ctzll(past), g0 = base + 4 * at;
+    if (at > 0) slot -= __builtin_amdgcn_readlane(upto, at - 1);
+#pragma unroll
+    for (int i = 0; i < 5; ++i) cq[i] = __builtin_amdgcn_readlane(cq[i], at);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      tl[i] = ((cq[i + 1] - cq[i]) * per + TQ - 1) / TQ;      // (0 past the last sequence: its offsets repeat)
-      all += tl[i];
+      tl[i] = ((cq[i + 1] - cq[i]) * per + TQ - 1) / TQ;
       most = max(most, tl[i]);
     }
-    if (slot >= all) { slot -= all; continue; }
     // the last rank with at most `slot` tiles in front of it (walked rank by rank a prompt's hundreds took microseconds)
     auto before = [&](int rank) { return (min(tl[0], rank) + min(tl[1], rank)) + (min(tl[2], rank) + min(tl[3], rank)); };
     int lo = 0, hi = most;

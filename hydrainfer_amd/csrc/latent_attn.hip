@@ -1012,9 +1012,13 @@ __global__ __launch_bounds__(256, KK <= 4 ? 2 : 1) void latent_attn_wide_kernel(
 // The same for wider latents (64 KK columns, KK even): four waves of 16 rows, 16 x 16 x 32 products — a row's queries and
 // accumulators are 192 registers a lane at 512 columns, two waves a SIMD.  A byte from LDS feeds half the products of the form
 // above; it is bound by the latency and number of its LDS reads (without those of the keys the same launch takes three quarters of
-// the time).  Tiles of 32 keys and 64 rows: two workgroups a CU, one working while the other brings queries in or results out.
+// the time).  Tiles of 32 keys and 64 rows: two workgroups a CU, one working while the other brings queries in or results out.  Also
+// the form for few rows, decode steps first: the keys of a row tile are then dealt to several workgroups (wide_plan), each writes
+// its rows' sums, maximum and weight, and the kernel below merges them.
 // Measured, 4 portions of 797 - 1151 tokens, 32 heads, 512 columns: 861 us in the group form, 226 us here (560 TFLOP/s; 780
-// behind long contexts, where less of the time goes to queries and results).  Row r of sixteen has its chunks at x ^ swz(r): rows r and 15 - r share a 32-byte place (their
+// behind long contexts, where less of the time goes to queries and results).  32 tokens of 301 - 1747 keys, 32 heads, 512 columns
+// under a window of 512: 31 us and 30 to merge in the tile form, 18 and 4.5 here, of which 6 pass before the first product and
+// about 5 are the splits' sums going out (8 MB); 1 token behind 1000 keys 70 us and 24, most of it the host's.  Row r of sixteen has its chunks at x ^ swz(r): rows r and 15 - r share a 32-byte place (their
 // chunks turned), so that a pass of a 16-byte read (rows 0-3 and 12-15 of one chunk, 4-11 of the next) and a transposing read
 // (eight rows, 32 bytes each) both reach every bank once.
 __device__ __forceinline__ float groups_max(float v) {      // over the four lanes with the same lane % 16
@@ -1027,16 +1031,21 @@ __device__ __forceinline__ float groups_max(float v) {      // over the four lan
 }
 
 template <int KK>
-__global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_attn_args a) {
-  constexpr int R = 64 * KK, KT = 32, TQ = 64, KS = R / 32, NDB = R / 16, RS = 2 * R, L = R / 8, IMG = KT * RS;
-  static_assert(RS % 256 == 0, "rows of whole bank rows");
+__global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_attn_args a, int tiles_per_seq) {
+  constexpr int R = 64 * KK, KT = 32, TQ = 64, KPW = 8, KS = R / 32, NDB = R / 16, RS = 2 * R, L = R / 8, IMG = KT * RS;
+  constexpr bool FULL = RS % 256 == 0;       // rows of whole bank rows: 16 places of a chunk, else 8 for each parity of the row
   extern __shared__ __attribute__((aligned(256))) char smem_w[];       // [2][32 rows]
-  auto swz = [](int row) { return (row & 15) < 8 ? 2 * (row & 7) : 31 - 2 * (row & 15); };
+  auto swz = [](int row) {
+    if (FULL) return (row & 15) < 8 ? 2 * (row & 7) : 31 - 2 * (row & 15);
+    const int h = (row & 15) >> 1;
+    return h < 4 ? 2 * h : 15 - 2 * h;
+  };
   typedef __attribute__((address_space(4))) const int32_t c_i32;       // (uniform indices: through the scalar cache)
   c_i32* q_cu = (c_i32*)a.q_cu;
   const int H = a.n_heads;
+  const int n_splits = a.n_splits > 1 ? a.n_splits : 1, split = n_splits > 1 ? (int)(blockIdx.x % n_splits) : 0;
   int b, tile, q0, n_rows;
-  if (!find_row_tile<TQ>(q_cu, a.n_seq, H, blockIdx.x, b, tile, q0, n_rows)) return;      // spare slot (the grid is an upper bound)
+  if (!find_row_tile<TQ>(q_cu, a.n_seq, H, (int)(n_splits > 1 ? blockIdx.x / n_splits : blockIdx.x), b, tile, q0, n_rows)) return;      // spare slot (the grid is an upper bound)
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int c = lane & 15, g = lane >> 4;
   const int row0_wg = n_rows - ((n_rows + TQ - 1) / TQ - tile) * TQ, row0 = row0_wg + 16 * wave;
@@ -1048,19 +1057,24 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
   const int p_wg = a.positions[q0 + max(row0_wg + lane, 0) / H];
   const int k_first = wave_min_int(first_key(p_wg)), k_last = wave_max_int(p_wg);
   const bool live = row0 + 15 >= 0;
-  const int t_first = k_first / KT, t_last = k_last / KT;
+  int t_first = k_first / KT, t_last = k_last / KT;
+  if (n_splits > 1) {                        // this split's run of tiles (the last splits may get none)
+    const int per = (t_last - t_first + n_splits) / n_splits;
+    t_first += split * per;
+    t_last = min(t_last, t_first + per - 1);
+  }
 
   const u16* cache = (const u16*)a.cache;
   c_i32* table = (c_i32*)(a.block_table + ((c_i32*)a.cu_block_lens)[b]);
   const int bs = a.block_size, bshift = (bs & (bs - 1)) == 0 ? __ffs(bs) - 1 : -1;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem_w;
   // Wave w brings keys 8 w .. of a tile (one page): 8 L chunks, 64 an instruction.
-  constexpr int NL = 8 * L / 64;
+  constexpr int NL = KPW * L / 64;
   auto bring = [&](int t, int img) __attribute__((always_inline)) {
-    const int key0 = min(t * KT + 8 * wave, k_last), r_max = k_last - key0;       // (rows past the last key repeat it; masked)
+    const int key0 = min(t * KT + KPW * wave, k_last), r_max = k_last - key0;       // (rows past the last key repeat it; masked)
     const int page = bshift >= 0 ? key0 >> bshift : key0 / bs;
     const u16* base = cache + (int64_t)table[page] * a.cache_block_stride + (int64_t)(key0 - page * bs) * a.cache_row_stride;
-    const uint32_t to = lds0 + (uint32_t)(img * IMG + 8 * wave * RS);
+    const uint32_t to = lds0 + (uint32_t)(img * IMG + KPW * wave * RS);
     int ln = lane;
     asm volatile("" : "+v"(ln));             // (worked out anew every time: kept, the addresses would push the queries out of registers)
 #pragma clang diagnostic push
@@ -1069,12 +1083,12 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
 #pragma unroll
     for (int j = 0; j < NL; ++j) {
       const int rr = (64 * j + ln) / L, ch = (64 * j + ln) % L;
-      const uint32_t off = (uint32_t)min(rr, r_max) * (uint32_t)(2 * a.cache_row_stride) + 16u * (uint32_t)(ch ^ swz(8 * (wave & 1) + rr));
+      const uint32_t off = (uint32_t)min(rr, r_max) * (uint32_t)(2 * a.cache_row_stride) + 16u * (uint32_t)(ch ^ swz(KPW * wave + rr));
       asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(__builtin_amdgcn_readfirstlane(to + 1024u * j)) : "memory", "m0");
     }
 #pragma clang diagnostic pop
   };
-  bring(t_first, 0);
+  if (t_first <= t_last) bring(t_first, 0);
   u16x8 qf[KS];                              // the queries (B operand): row c, columns 32 ks + 8 g ..
   {
     const u16* qg = (const u16*)a.q + (int64_t)(q0 + tok) * a.q_token_stride + (int64_t)head * a.q_head_stride + 8 * g;
@@ -1095,9 +1109,10 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
 #pragma unroll
   for (int i = 0; i < NDB; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m = HX_NEG_BIG, l = 0.f;
-  // Reads of rows: chunk 4 ks + g of row c; the swizzle touches the low four bits of a chunk, ks = 4 x + y.  Transposing reads:
-  // lane 4 q + p of a group of 16 brings row 4 g + q (and the row 16 below it: the same place), columns 16 db + 4 p ..: chunk
-  // 2 db + p / 2, db = 8 x + y.
+  // Reads of rows: chunk 4 ks + g of row c; the swizzle touches the low four (three) bits of a chunk, ks = NP x + y.  Transposing
+  // reads: lane 4 q + p of a group of 16 brings row 4 g + q (and the row 16 below it: the same place), columns 16 db + 4 p ..:
+  // chunk 2 db + p / 2, db = 2 NP x + y.
+  constexpr int NP = FULL ? 4 : 2;
   const uint32_t kp0 = lds0 + (uint32_t)(c * RS + 16 * (g ^ swz(c)));
   const uint32_t vp0 = lds0 + (uint32_t)((4 * g + (c >> 2)) * RS + 16 * (((c & 3) >> 1) ^ swz(4 * g + (c >> 2))) + 8 * (c & 1));
   auto row_read = [](uint32_t at) __attribute__((always_inline)) {
@@ -1117,15 +1132,16 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-      for (int u = 0; u < 2; ++u) s[u] = Mfma<BF16>::mma(row_read((kp ^ (64u * (ks % 4))) + 16u * u * RS + 256u * (ks / 4)), qf[ks], s[u]);
+      for (int u = 0; u < 2; ++u) s[u] = Mfma<BF16>::mma(row_read((kp ^ (64u * (ks % NP))) + 16u * u * RS + 64u * NP * (ks / NP)), qf[ks], s[u]);
     // (reads stay a few products ahead)
-    __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+    constexpr int kAhead = 2 * KS < 8 ? 2 * KS : 8;
+    __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);
 #pragma unroll
-    for (int i = 0; i < 2 * KS - 8; ++i) {
+    for (int i = 0; i < 2 * KS - kAhead; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, kAhead, 0);
     const int key_l = key0 + 4 * g;          // element e of half u: key key_l + 16 u + e
     float mx = HX_NEG_BIG;
     if (key0 + 31 <= wpos0 && key0 >= wlo1) {              // every row of the wave sees all of them
@@ -1162,17 +1178,18 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
     }
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
-      const uint32_t at = (va ^ (32u * (db % 8))) + 256u * (db / 8);
+      const uint32_t at = (va ^ (32u * (db % (2 * NP)))) + 64u * NP * (db / (2 * NP));
       const u16x4 x0 = tr_read(at), x1 = tr_read(at + 16u * RS);
       acc[db] = Mfma<BF16>::mma(u16x8{x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]}, pf, acc[db]);
     }
-    __builtin_amdgcn_sched_group_barrier(0x100, 12, 0);
+    constexpr int kAheadV = NDB < 6 ? NDB : 6;
+    __builtin_amdgcn_sched_group_barrier(0x100, 2 * kAheadV, 0);
 #pragma unroll
-    for (int i = 0; i < NDB - 6; ++i) {
+    for (int i = 0; i < NDB - kAheadV; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, kAheadV, 0);
   };
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
@@ -1187,6 +1204,20 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
   // out, through LDS (the images are free): whole rows a store.  O[row c][column 16 db + 4 g + e]
   float total = l + __shfl_xor(l, 16, 64);
   total += __shfl_xor(total, 32, 64);
+  if (n_splits > 1) {
+    // what this split adds to a row, not normalised: ws_o [sequence][row][split][R], ws_ml [..][split][maximum (log2), sum]
+    if (row0 + c >= 0) {
+      const size_t at = ((size_t)b * tiles_per_seq * 16 + (row0 + c)) * n_splits + split;
+      float* wo = a.ws_o + at * R + 4 * g;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) *reinterpret_cast<f32x4*>(wo + 16 * db) = acc[db];
+      if (g == 0) {
+        a.ws_ml[2 * at] = m;
+        a.ws_ml[2 * at + 1] = total;
+      }
+    }
+    return;
+  }
   if (a.sinks) total += fast_exp2(a.sinks[head] * kLog2e - m);      // the sink: one more term, without a value
   float gsc = 1.0f / total;
   if (a.gate_pre) {
@@ -1205,7 +1236,7 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-  for (int j = 0; j < 2 * NL; ++j) {
+  for (int j = 0; j < 16 * L / 64; ++j) {
     const int rl = (64 * j + lane) / L, ch = (64 * j + lane) % L, ro = row0 + rl;
     // slots 2 ch, 2 ch + 1 of row rl sit in chunk ch ^ (rl >> 1), in turned order when rl is odd
     u16x8 v = *reinterpret_cast<const u16x8*>(ob + rl * RS + 16 * (ch ^ (rl >> 1)));
@@ -1214,24 +1245,124 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
   }
 }
 
+// The splits of a row merged: out = sum_s O_s 2^(m_s - M) / sum_s l_s 2^(m_s - M), times the head gate.  A row to R / 4 lanes (a power
+// of two of them); one pass over the splits, four at a time, their loads all in flight together.
+__global__ __launch_bounds__(256) void latent_attn_merge_kernel(hxm_latent_attn_args a, int tiles_per_seq, int lanes_log2) {
+  const int R = a.kv_rank, H = a.n_heads, NS = a.n_splits, lanes = 1 << lanes_log2;
+  const int64_t item = (((int64_t)blockIdx.x * 256 + threadIdx.x) >> lanes_log2);
+  const int b = (int)(item / (tiles_per_seq * 16)), r = (int)(item % (tiles_per_seq * 16));
+  if (b >= a.n_seq) return;
+  const int q0 = a.q_cu[b];
+  if (r >= (a.q_cu[b + 1] - q0) * H) return;
+  const int t = q0 + r / H, h = r % H;
+  const float* ml = a.ws_ml + 2 * (size_t)item * NS;
+  float gate = 1.f;
+  if (a.gate_pre) gate = 1.0f / (1.0f + __expf(-BF16::to_float(((const u16*)a.gate_pre)[(int64_t)t * a.gate_stride + h])));
+  u16* og = (u16*)a.out + (int64_t)t * a.out_token_stride + (int64_t)h * a.out_head_stride;
+  for (int c = 4 * ((int)threadIdx.x & (lanes - 1)); c < R; c += 4 * lanes) {
+    const float* wo = a.ws_o + (size_t)item * NS * R + c;
+    f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
+    float M = HX_NEG_BIG, total = 0.f;
+    for (int s0 = 0; s0 < NS; s0 += 4) {
+      float mx[4], l[4];
+      f32x4 v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int s = min(s0 + i, NS - 1);
+        mx[i] = ml[2 * s];
+        l[i] = ml[2 * s + 1];
+        v[i] = *reinterpret_cast<const f32x4*>(wo + (size_t)s * R);
+      }
+      const float m_new = fmaxf(M, fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3])));
+      const float keep = fast_exp2(M - m_new);
+      total *= keep;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] *= keep;
+      M = m_new;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float w = s0 + i < NS ? fast_exp2(mx[i] - M) : 0.f;
+        total += w * l[i];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] += w * v[i][e];
+      }
+    }
+    if (a.sinks) total += fast_exp2(a.sinks[h] * 1.4426950408889634f - M);      // the sink counts once, here
+    const float gsc = gate / total;
+    *reinterpret_cast<u16x4*>(og + c) = u16x4{BF16::from_float(o[0] * gsc), BF16::from_float(o[1] * gsc), BF16::from_float(o[2] * gsc), BF16::from_float(o[3] * gsc)};
+  }
+}
+
+int prepare_lds(const void* kernel, size_t lds) {
+  if (lds <= 48 * 1024) return HX_OK;
+  const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (e == hipSuccess) return HX_OK;
+  hxm::last_hip_error() = (int)e;
+  return HX_ERR_HIP;
+}
+
+// How the wide forms lay a launch out (the tile forms below keep the latents they do not take: widths or strides that are not whole
+// 16-byte columns of 64, pages that are not whole 16-row groups).  rows32: waves of 32 rows (enough row tiles of 128 to fill the chip), else waves of 16 rows
+// and the keys of a row tile dealt to `splits` workgroups where there are few of them.
+struct WidePlan {
+  bool fits, rows32;
+  int splits;
+};
+WidePlan wide_plan(const hxm_latent_attn_args& a) {
+  WidePlan p{false, false, 1};
+  if (a.kv_rank % 64 || a.block_size % 16 || a.out_token_stride % 8 || a.out_head_stride % 8 || !aligned16(a.out) || !aligned16(a.ws_o) ||
+      a.cache_row_stride >= (1 << 26) || hxm::tile_form() != 1)
+    return p;
+  p.fits = true;
+  const int64_t rows = (int64_t)a.max_q_len * a.n_heads;
+  p.rows32 = a.kv_rank <= 320 && a.n_seq * ((rows + 127) / 128) >= 256;
+  if (p.rows32) return p;
+  int reach = a.max_kv_len;
+  if (a.window > 0 && a.window + a.max_q_len < reach) reach = a.window + a.max_q_len;
+  const int64_t tiles = a.n_seq * ((rows + 63) / 64);
+  int64_t want = (512 + tiles - 1) / tiles;
+  // (a split more shortens the walk over the keys and lengthens the writing and merging of what the splits hold, 8 bytes a row and
+  //  column: their sum is least where the square of the splits is a multiple of keys / rows.  At 18, 36 and 72 times, 512 columns
+  //  and 32 heads: 32 tokens of 301 - 1747 keys 36.4, 31.7, 30.5 us, under a window of 512 26, 25, 22.7; 16 tokens behind 4000
+  //  keys 41, 37, 33; 16 portions of 4 behind 1000 keys 49, 35, 35.)
+  while (want > 1 && want * want * a.n_seq * rows > (int64_t)72 * reach) --want;
+  if (want > reach / 64) want = reach / 64;      // (two tiles of 32 keys a split at least)
+  if (want > 64) want = 64;
+  if (want > 1) p.splits = (int)want;
+  return p;
+}
+
 template <int KK>
-int launch_wide(const hxm_latent_attn_args& a, hipStream_t s) {
-  constexpr int rows = KK <= 5 ? 128 : 64, keys = KK <= 5 ? 64 : 32;
-  const int64_t grid = ((int64_t)a.n_tokens * a.n_heads + rows - 1) / rows + a.n_seq;      // row tiles of all sequences, at most
+int launch_wide16(const hxm_latent_attn_args& a, hipStream_t s) {
+  const int n_splits = a.n_splits > 1 ? a.n_splits : 1, tiles16 = (int)(((int64_t)a.max_q_len * a.n_heads + 15) / 16);
+  const int64_t grid = (((int64_t)a.n_tokens * a.n_heads + 63) / 64 + a.n_seq) * n_splits;      // row tiles of all sequences, at most
   if (grid > 0x7fffffff) return HX_ERR_SHAPE;
-  constexpr size_t lds = 2 * keys * 2 * 64 * KK;
-  void (*kernel)(hxm_latent_attn_args);
-  if constexpr (KK <= 5) kernel = latent_attn_wide_kernel<KK>;
-  else kernel = latent_attn_wide16_kernel<KK>;
-  if (lds > 48 * 1024) {
-    const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) {
-      hxm::last_hip_error() = (int)e;
-      return HX_ERR_HIP;
+  constexpr size_t lds = 2 * 32 * 2 * 64 * KK;
+  if (const int rc = prepare_lds((const void*)latent_attn_wide16_kernel<KK>, lds)) return rc;
+  latent_attn_wide16_kernel<KK><<<dim3((unsigned)grid), dim3(256), lds, s>>>(a, tiles16);
+  if (n_splits > 1) {
+    int lanes_log2 = 4;                      // a row to R / 4 lanes, at most a power of two of them
+    while ((8 << lanes_log2) <= a.kv_rank && lanes_log2 < 7) ++lanes_log2;
+    const int64_t threads = ((int64_t)a.n_seq * tiles16 * 16) << lanes_log2;
+    latent_attn_merge_kernel<<<dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s>>>(a, tiles16, lanes_log2);
+  }
+  return hxm::check_launch();
+}
+
+template <int KK>
+int launch_wide(const hxm_latent_attn_args& a, const WidePlan& p, hipStream_t s) {
+  if (a.n_splits > 1 && (a.n_splits > 64 || !a.ws_o || !a.ws_ml)) return HX_ERR_WORKSPACE;
+  if constexpr (KK <= 5) {
+    if (p.rows32) {
+      const int64_t grid = ((int64_t)a.n_tokens * a.n_heads + 127) / 128 + a.n_seq;
+      if (grid > 0x7fffffff) return HX_ERR_SHAPE;
+      constexpr size_t lds = 2 * 64 * 2 * 64 * KK;
+      if (const int rc = prepare_lds((const void*)latent_attn_wide_kernel<KK>, lds)) return rc;
+      latent_attn_wide_kernel<KK><<<dim3((unsigned)grid), dim3(256), lds, s>>>(a);
+      return hxm::check_launch();
     }
   }
-  kernel<<<dim3((unsigned)grid), dim3(256), lds, s>>>(a);
-  return hxm::check_launch();
+  return launch_wide16<KK>(a, s);
 }
 
 // the splits of a (sequence, row tile) merged: out = sum_s O_s e^(m_s - M) / sum_s l_s e^(m_s - M), times the head gate
@@ -1351,7 +1482,8 @@ extern "C" int hxm_latent_attention_plan(const hxm_latent_attn_args* args, int32
   *n_splits = 1;
   *ws_floats = 0;
   if (args->n_tokens <= 0 || args->max_q_len < 1 || args->n_seq < 1 || !tile_form_serves(*args)) return HX_OK;
-  const int ns = tile_splits(*args);
+  const WidePlan p = wide_plan(*args);
+  const int ns = p.fits ? p.splits : tile_splits(*args);
   if (ns > 1) {
     const int64_t tiles_per_seq = ((int64_t)args->max_q_len * args->n_heads + 15) / 16;
     const int64_t R16 = (args->kv_rank + 15) / 16 * 16;
@@ -1372,16 +1504,17 @@ extern "C" int hxm_latent_attention(const hxm_latent_attn_args* args, void* stre
   hipStream_t s = (hipStream_t)stream;
   if (a.max_q_len < 1) return HX_ERR_SHAPE;
   if (tile_form_serves(a)) {
-    if (a.kv_rank % 64 == 0 && a.kv_rank != 448 && a.block_size % 16 == 0 && a.out_token_stride % 8 == 0 && a.out_head_stride % 8 == 0 && aligned16(a.out) &&
-        (int64_t)a.max_q_len * a.n_heads >= 64 && a.max_q_len > 1 && a.cache_row_stride < (1 << 26) && hxm::tile_form() == 1) {
+    const WidePlan p = wide_plan(a);
+    if (p.fits) {
       switch (a.kv_rank / 64) {
-        case 1: return launch_wide<1>(a, s);
-        case 2: return launch_wide<2>(a, s);
-        case 3: return launch_wide<3>(a, s);
-        case 4: return launch_wide<4>(a, s);
-        case 5: return launch_wide<5>(a, s);
-        case 6: return launch_wide<6>(a, s);
-        default: return launch_wide<8>(a, s);
+        case 1: return launch_wide<1>(a, p, s);
+        case 2: return launch_wide<2>(a, p, s);
+        case 3: return launch_wide<3>(a, p, s);
+        case 4: return launch_wide<4>(a, p, s);
+        case 5: return launch_wide<5>(a, p, s);
+        case 6: return launch_wide<6>(a, p, s);
+        case 7: return launch_wide<7>(a, p, s);
+        default: return launch_wide<8>(a, p, s);
       }
     }
     switch ((a.kv_rank + 31) / 32) {

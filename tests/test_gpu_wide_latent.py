@@ -1,6 +1,6 @@
 """Latent attention over portions of prompts (csrc/latent_attn.hip, the wide forms: 64 to 320 columns, 384 and 512) at the edges of
 their tiles — 128 or 64 rows of token and head, 64 or 32 keys — with windows, sinks, gates, a negative scale, queries and results
-as views of other layouts."""
+as views of other layouts; and over single tokens, whose keys are dealt to several workgroups."""
 import math
 
 import pytest
@@ -18,11 +18,28 @@ BATCHES = [[(2, 2)], [(33, 33), (2, 100)], [(5, 70), (1, 200), (32, 32)], [(129,
 @pytest.mark.parametrize("H", [3, 32])
 @pytest.mark.parametrize("window, extra", [(0, "plain"), (1, "plain"), (31, "sinks"), (50, "gate"), (0, "negative"), (64, "sinks and gate")])
 def test_wide_forms(batch, R, H, window, extra):
-    from hydrainfer_amd._C.kernel.latent_attn import latent_attention
-    g = torch.Generator().manual_seed(R * 100 + H + window + sum(a + b for a, b in batch))
     new, kv = [a for a, _ in batch], [b for _, b in batch]
     if max(new) * H < 64:
         new[0], kv[0] = 22, max(22, kv[0])
+    check(new, kv, R, H, window, extra)
+
+
+# single tokens: one tile and a split's edge, splits that get no tile (one sequence far shorter than another), more sequences than a
+# round of the row tiles' search holds
+STEPS = [[64], [129, 1, 32, 33], [2000, 3], [700] * 5, [40] * 260 + [130]]
+
+
+@pytest.mark.parametrize("kv", STEPS, ids=lambda v: f"{len(v)}x{max(v)}")
+@pytest.mark.parametrize("R", [64, 448, 512])
+@pytest.mark.parametrize("H", [1, 16, 65])
+@pytest.mark.parametrize("window, extra", [(0, "plain"), (300, "sinks and gate"), (0, "negative")])
+def test_single_tokens(kv, R, H, window, extra):
+    check([1] * len(kv), kv, R, H, window, extra)
+
+
+def check(new, kv, R, H, window, extra):
+    from hydrainfer_amd._C.kernel.latent_attn import latent_attention
+    g = torch.Generator().manual_seed(R * 100 + H + window + sum(new) + sum(kv))
     nb = [(n + BLOCK - 1) // BLOCK for n in kv]
     T, perm = sum(new), torch.randperm(sum(nb) + 1, generator=g)
     cache = torch.randn((sum(nb) + 1, BLOCK, 1, R + 8), generator=g).bfloat16()      # rows wider than the latent
