@@ -112,11 +112,19 @@ def biased_attention(q: Tensor, key_cache: Tensor, value_cache: Tensor, vdim: in
     if form in ("auto", "tile") and q.dtype == torch.bfloat16 and max_q_len > 0 and max_kv_len > 0 and D % 8 == 0 and vdim % 8 == 0 \
             and D <= 256 and vdim <= 256:
         # key splits: enough waves to fill the chip when the launch has few row tiles, at least two 32-key chunks a split
-        tiles = n_seq * G * ((max_q_len * (H // G) + 15) // 16)
+        rows = max_q_len * (H // G)
+        tiles = n_seq * G * ((rows + 15) // 16)
         reach = max_kv_len
         if mask != "causal":
             reach = min(reach, mask_size + (max_q_len if mask == "window" else 0))
-        ns = min((2048 + tiles - 1) // tiles, ((reach + 31) // 32) // 2, 64)
+        # heads of 64 and 128: five waves of the step form fill a CU (1024 and 2048 waves: 32 tokens of 1025 - 2047 keys 39.5 and
+        # 41.9 us, 128 of 500 - 1500 109 and 116); portions of 64 rows and more go undivided to the wide form unless they are few
+        # and their keys many (one portion behind keys, 32 heads on 8 key heads, wide and split: 32 tokens behind 2000 44.8 and
+        # 24.9 us, 100 behind 2000 46.4 and 36.4, 100 behind none 21 and 23.5, 8 times 16 behind 500 21.4 and 23.9)
+        whole = form == "auto" and D in (64, 128) and vdim in (64, 128) and bs % 16 == 0
+        ns = min(((1024 if whole else 2048) + tiles - 1) // tiles, ((reach + 31) // 32) // 2, 64)
+        if whole and rows >= 64 and (tiles > 256 or reach < 1024):
+            ns = 1
         if ns > 1:
             v16 = (vdim + 15) // 16 * 16
             ws = torch.empty(tiles * ns * 16 * (v16 + 2), dtype=torch.float32, device=q.device)

@@ -58,6 +58,15 @@ __device__ __forceinline__ int wave_min_int(int v) {
 }
 __device__ __forceinline__ int wave_max_int(int v) { return -wave_min_int(-v); }
 
+__device__ __forceinline__ float groups_max(float v) {      // over the four lanes with the same lane % 16
+  const auto a = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
+  const unsigned a0 = a[0], a1 = a[1];
+  v = fmaxf(__builtin_bit_cast(float, a0), __builtin_bit_cast(float, a1));
+  const auto b = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
+  const unsigned b0 = b[0], b1 = b[1];
+  return fmaxf(__builtin_bit_cast(float, b0), __builtin_bit_cast(float, b1));
+}
+
 // The slot-th (sequence, tile of TQ rows) pair of a batch whose sequences bring (cu[i + 1] - cu[i]) * per rows: sequences in groups of
 // four, of every group the last tile of each — it sees the most keys —, then the one before it of each, ...; row tiles end with
 // the portion, so that a partial tile is the first.  false: a spare slot.  Every lane counts one group's tiles: one round of loads

@@ -882,6 +882,289 @@ int launch_wide(const hxm_biased_attn_args& a, hipStream_t s) {
   return hxm::check_launch();
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// Step form (bfloat16, fewer than 64 rows of a key head or few row tiles behind many keys, key and value heads of 64 or 128,
+// pages of whole 16-row groups): a workgroup is one wave with 16 rows of ONE (sequence, key head) and one run of its keys, in tiles of 32.  Bound by memory: the
+// tile form asks for a key's row in 64-byte pieces, sixteen rows an instruction, and has one chunk in flight; here rows go whole
+// from the paged cache to LDS, the next tile's while this one's are awaited — no register holds them and no barrier is needed.
+// 32 KB of LDS at heads of 128: five waves a CU, 80 to 160 KB in flight.  Products are 16 x 16 x 32 and swapped, S^T = K Q^T,
+// O^T += V^T P^T: a row of the softmax is one lane, its weights stay in their registers.  16-byte chunk x of row r sits at
+// x ^ swz(r): rows r and 15 - r share a 32-byte place (their chunks turned), so that a pass of a 16-byte read and a transposing
+// read (eight rows, 32 bytes each) both reach every bank once.
+// Measured, 32 heads of 128 on 8 key heads, kernel and merge: 32 tokens of 1025 - 2047 keys 48 + 8 us in the tile form, 36 + 4 here
+// (5.5 TB/s); 128 tokens of 500 - 1500 keys 163 us and 109; 32 tokens, 2 key heads 57 us and 24; 16 tokens behind 4000 keys
+// 93 us (tile), 79 (wide) and 29.
+// ---------------------------------------------------------------------------------------------------------------
+template <int D, int V, bool MODS>      // MODS: slopes or a soft cap
+__global__ __launch_bounds__(64) void biased_attn_step_kernel(hxm_biased_attn_args a, int tiles_per_seq) {
+  constexpr int KT = 32, KS = D / 32, NDB = V / 16, RSK = 2 * D, RSV = 2 * V, LK = D / 8, LV = V / 8;
+  constexpr int KTILE = KT * RSK, IMG = KTILE + KT * RSV, NLK = 16 * LK / 64, NLV = 16 * LV / 64;      // transfers of 16 rows
+  extern __shared__ __attribute__((aligned(256))) char smem_s[];       // [2][K rows | V rows]
+  auto swz = [](int row, bool full) {        // full: rows of whole bank rows, 16 places of a chunk, else 8 for each parity of the row
+    if (full) return (row & 15) < 8 ? 2 * (row & 7) : 31 - 2 * (row & 15);
+    const int h = (row & 15) >> 1;
+    return h < 4 ? 2 * h : 15 - 2 * h;
+  };
+  typedef __attribute__((address_space(4))) const int32_t c_i32;       // (uniform indices: through the scalar cache)
+  const int G = a.kv_heads, R = a.n_heads / a.kv_heads, n_splits = a.n_splits > 1 ? a.n_splits : 1;
+  // workgroup -> (sequence, row tile, split, key head), key heads fastest: the rows of a page are asked for at about one time
+  int at = blockIdx.x;
+  const int kvh = at % G;
+  at /= G;
+  const int split = at % n_splits;
+  at /= n_splits;
+  const int tile = at % tiles_per_seq, b = at / tiles_per_seq;
+  const int q0 = ((c_i32*)a.q_cu)[b], n_rows = (((c_i32*)a.q_cu)[b + 1] - q0) * R, n_tiles = (n_rows + 15) / 16;
+  if (tile >= n_tiles) return;
+  const int lane = threadIdx.x, c = lane & 15, g = lane >> 4;
+  const int row0 = n_rows - (n_tiles - tile) * 16;      // (row tiles end with the portion; rows below 0 do not exist)
+  const int r = max(row0 + c, 0), tok = r / R, head = kvh * R + r % R;
+  const int pos = a.positions[q0 + tok], lo = first_visible(pos, a.mask_kind, a.mask_size);
+  const int pos_min = wave_min_int(pos), k_last = wave_max_int(pos), k_first = wave_min_int(lo), lo_max = wave_max_int(lo);
+  int t_first = k_first / KT, t_last = k_last / KT;
+  if (n_splits > 1) {                        // this split's run of tiles (the last splits may get none)
+    const int per = (t_last - t_first + n_splits) / n_splits;
+    t_first += split * per;
+    t_last = min(t_last, t_first + per - 1);
+  }
+  u16x8 qf[KS];                              // the queries (B operand): row c, columns 32 ks + 8 g ..
+  {
+    const u16* qg = (const u16*)a.q + ((int64_t)(q0 + tok) * a.n_heads + head) * D + 8 * g;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const u16x8*>(qg + 32 * ks);
+  }
+  constexpr float kLog2e = 1.4426950408889634f;
+  float hsc = a.head_scale ? a.scale * a.head_scale[head] : a.scale;
+  float slope2 = MODS && a.slopes ? a.slopes[head] * kLog2e : 0.f;
+  float sink2 = a.sinks ? a.sinks[head] * kLog2e : -INFINITY;
+  const int32_t* table = a.block_table + ((c_i32*)a.cu_block_lens)[b];
+  const int bs = a.block_size, bshift = (bs & (bs - 1)) == 0 ? __ffs(bs) - 1 : -1;
+  auto page_of = [&](int key) { return bshift >= 0 ? key >> bshift : key / bs; };
+  // lane i: the page of the i-th group of 16 keys from group pages0 on
+  int pages0 = 2 * t_first, pages = table[page_of(min(16 * (pages0 + lane), k_last))];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[ks]));
+  asm volatile("" : "+v"(pages), "+v"(hsc), "+v"(slope2), "+v"(sink2));      // (all there before the transfers start: a wait for them would be one for those)
+  const u16* kc = (const u16*)a.key_cache + (int64_t)kvh * a.head_stride;
+  const u16* vc = (const u16*)a.value_cache + (int64_t)kvh * a.head_stride;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem_s;
+  const uint32_t row_bytes = (uint32_t)(2 * a.cache_row_stride);
+  auto bring = [&](int t, int img) __attribute__((always_inline)) {
+    if (2 * t + 1 - pages0 > 63) {
+      pages0 = 2 * t;
+      pages = table[page_of(min(16 * (pages0 + lane), k_last))];
+      asm volatile("" : "+v"(pages));        // (waited for here: after the branch it would be a wait in every tile)
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (the reads of the image that this replaces are done)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+    // (m0, the LDS address of the transfer, is a reserved register: nothing else in this kernel uses it)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int key0 = min(t * KT + 16 * u, k_last), r_max = k_last - key0;      // (rows past the last key repeat it; masked)
+      const int64_t off = (int64_t)__builtin_amdgcn_readlane(pages, 2 * t + u - pages0) * a.cache_block_stride +
+                          (int64_t)(key0 - page_of(key0) * bs) * a.cache_row_stride;
+      const uint32_t kd = lds0 + (uint32_t)(img * IMG + 16 * u * RSK), vd = lds0 + (uint32_t)(img * IMG + KTILE + 16 * u * RSV);
+#pragma unroll
+      for (int j = 0; j < NLK; ++j) {
+        const int rr = (64 * j + lane) / LK, ch = (64 * j + lane) % LK;
+        const uint32_t from = (uint32_t)min(rr, r_max) * row_bytes + 16u * (uint32_t)(ch ^ swz(rr, D == 128));
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(from), "s"(kc + off), "s"(__builtin_amdgcn_readfirstlane(kd + 1024u * j)) : "memory", "m0");
+      }
+#pragma unroll
+      for (int j = 0; j < NLV; ++j) {
+        const int rr = (64 * j + lane) / LV, ch = (64 * j + lane) % LV;
+        const uint32_t from = (uint32_t)min(rr, r_max) * row_bytes + 16u * (uint32_t)(ch ^ swz(rr, V == 128));
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(from), "s"(vc + off), "s"(__builtin_amdgcn_readfirstlane(vd + 1024u * j)) : "memory", "m0");
+      }
+    }
+#pragma clang diagnostic pop
+  };
+  if (t_first <= t_last) bring(t_first, 0);
+  // scores in units of log2: z = scale2 s - slope2 (pos - key), or under a cap cap2 tanh(s hsc / cap) in its place
+  const bool cap = MODS && a.softcap > 0.f;
+  const float cap2 = cap ? a.softcap * kLog2e : 0.f;
+  float scale2 = cap ? 2.f * kLog2e * hsc / a.softcap : hsc * kLog2e;
+  if (!MODS) {             // (a maximum of scores is one of scaled scores where the scale is positive; -inf times it stays -inf)
+    if (scale2 < 0.f) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) qf[ks] ^= (u16)0x8000;
+    }
+    scale2 = fmaxf(fabsf(scale2), 1e-30f);
+  }
+  f32x4 acc[NDB];
+#pragma unroll
+  for (int i = 0; i < NDB; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = HX_NEG_BIG, l = 0.f;
+  // Reads of rows: chunk 4 ks + g of row c.  Transposing reads: lane 4 q + p of a group of 16 brings row 4 g + q (and the row 16
+  // below it: the same place), columns 16 db + 4 p ..: chunk 2 db + p / 2.
+  const uint32_t kp0 = lds0 + (uint32_t)(c * RSK + 16 * (g ^ swz(c, D == 128)));
+  const uint32_t vp0 = lds0 + (uint32_t)(KTILE + (4 * g + (c >> 2)) * RSV + 16 * (((c & 3) >> 1) ^ swz(4 * g + (c >> 2), V == 128)) + 8 * (c & 1));
+  auto row_read = [](uint32_t from) __attribute__((always_inline)) {
+    return *reinterpret_cast<__attribute__((address_space(3))) const u16x8*>((uintptr_t)from);
+  };
+  auto tr_read = [](uint32_t from) __attribute__((always_inline)) {
+    typedef __attribute__((address_space(3))) hx_s16x4_t lds_s4;
+    return __builtin_bit_cast(u16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(uintptr_t)from));
+  };
+  for (int t = t_first; t <= t_last; ++t) {
+    const int img = (t - t_first) & 1, key0 = t * KT;
+    if (t < t_last) {
+      bring(t + 1, img ^ 1);
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (NLK + NLV)) : "memory");      // this tile is there, the next on its way
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    const uint32_t kp = kp0 + (uint32_t)(img * IMG), va = vp0 + (uint32_t)(img * IMG);
+    f32x4 s[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) s[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) s[u] = Mfma<BF16>::mma(row_read((kp ^ (64u * ks)) + 16u * u * RSK), qf[ks], s[u]);
+    const int key_l = key0 + 4 * g;          // element e of half u: key key_l + 16 u + e
+    float unit = scale2;                     // what a score still has to be multiplied by
+    if (MODS) {
+      unit = 1.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float z = s[e >> 2][e & 3];
+        // cap2 tanh(y) = cap2 - 2 cap2 / (1 + e^(2 y))
+        z = cap ? __builtin_fmaf(-2.f * cap2, __builtin_amdgcn_rcpf(1.f + fast_exp2(z * scale2)), cap2) : z * scale2;
+        if (a.slopes) z += slope2 * (float)(key_l + 16 * (e >> 2) + (e & 3) - pos);
+        s[e >> 2][e & 3] = z;
+      }
+    }
+    float mx = HX_NEG_BIG;
+    if (key0 + KT - 1 <= pos_min && key0 >= lo_max) {      // every row of the wave sees all of them
+#pragma unroll
+      for (int e = 0; e < 8; ++e) mx = fmaxf(mx, s[e >> 2][e & 3]);
+    } else {
+      const int last = pos - key_l, first = lo - key_l;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int k = 16 * (e >> 2) + (e & 3);
+        if (k > last || k < first) s[e >> 2][e & 3] = -INFINITY;
+        mx = fmaxf(mx, s[e >> 2][e & 3]);
+      }
+    }
+    mx = groups_max(mx);
+    // a row keeps the maximum its weights refer to until a score exceeds it by 2^8
+    const float m_cand = fmaxf(m, mx * unit);
+    const bool grow = m_cand > m + 8.0f;
+    if (__builtin_amdgcn_ballot_w64(grow)) {
+      const float m_new = grow ? m_cand : m, alpha = fast_exp2(m - m_new);
+      l *= alpha;
+#pragma unroll
+      for (int i = 0; i < NDB; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][e] *= alpha;
+      m = m_new;
+    }
+    u16x8 pf;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float p = fast_exp2(__builtin_fmaf(s[e >> 2][e & 3], unit, -m));
+      l += p;
+      pf[e] = BF16::from_float(p);
+    }
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) {
+      const u16x4 x0 = tr_read(va ^ (32u * db)), x1 = tr_read((va ^ (32u * db)) + 16u * RSV);
+      acc[db] = Mfma<BF16>::mma(u16x8{x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]}, pf, acc[db]);
+    }
+    // (reads stay a few products ahead)
+    constexpr int kAhead = NDB < 6 ? NDB : 6;
+    __builtin_amdgcn_sched_group_barrier(0x100, 2 * kAhead, 0);
+#pragma unroll
+    for (int i = 0; i < NDB - kAhead; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, kAhead, 0);
+  }
+  if (row0 + c < 0) return;
+  float total = l + __shfl_xor(l, 16, 64);      // (rows below 0 are whole columns of lanes)
+  total += __shfl_xor(total, 32, 64);
+  if (n_splits > 1) {
+    // what this split adds to a row, not normalised: ws_o [sequence, key head, tile][row][split][V], ws_ml [..][split][maximum (log2), sum]
+    const size_t slot = ((((size_t)b * G + kvh) * tiles_per_seq + tile) * 16 + c) * n_splits + split;
+    float* wo = a.ws_o + slot * V + 4 * g;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) *reinterpret_cast<f32x4*>(wo + 16 * db) = acc[db];
+    if (g == 0) {
+      a.ws_ml[2 * slot] = m;
+      a.ws_ml[2 * slot + 1] = total;
+    }
+    return;
+  }
+  const float inv = 1.0f / (total + fast_exp2(sink2 - m));      // the sink: one more term, without a value
+  u16* og = (u16*)a.out + ((int64_t)(q0 + tok) * a.n_heads + head) * V + 4 * g;
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+    *reinterpret_cast<u16x4*>(og + 16 * db) = u16x4{BF16::from_float(acc[db][0] * inv), BF16::from_float(acc[db][1] * inv), BF16::from_float(acc[db][2] * inv), BF16::from_float(acc[db][3] * inv)};
+}
+
+// The splits of a row merged: out = sum_s O_s 2^(m_s - M) / sum_s l_s 2^(m_s - M).  A row to V / 4 lanes; one pass over the splits,
+// four at a time, their loads all in flight together.
+template <int V>
+__global__ __launch_bounds__(256) void biased_attn_merge_kernel(hxm_biased_attn_args a, int tiles_per_seq) {
+  const int64_t at = (int64_t)blockIdx.x * 256 + threadIdx.x, slot = at / (V / 4);      // slot: row c of (sequence, key head, tile)
+  const int G = a.kv_heads, R = a.n_heads / a.kv_heads, NS = a.n_splits, col = 4 * (int)(at % (V / 4));
+  const int64_t item = slot / 16;
+  const int tile = (int)(item % tiles_per_seq), kvh = (int)(item / tiles_per_seq % G), b = (int)(item / tiles_per_seq / G);
+  if (b >= a.n_seq) return;
+  const int q0 = a.q_cu[b], n_rows = (a.q_cu[b + 1] - q0) * R, n_tiles = (n_rows + 15) / 16;
+  const int r = n_rows - (n_tiles - tile) * 16 + (int)(slot % 16);
+  if (tile >= n_tiles || r < 0) return;
+  const int head = kvh * R + r % R;
+  const float* ml = a.ws_ml + 2 * slot * NS;
+  const float* wo = a.ws_o + slot * NS * V + col;
+  const float sink2 = a.sinks ? a.sinks[head] * 1.4426950408889634f : -INFINITY;
+  f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
+  float M = HX_NEG_BIG, total = 0.f;
+  for (int s0 = 0; s0 < NS; s0 += 4) {
+    float mx[4], l[4];
+    f32x4 v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int s = min(s0 + i, NS - 1);
+      mx[i] = ml[2 * s];
+      l[i] = ml[2 * s + 1];
+      v[i] = *reinterpret_cast<const f32x4*>(wo + (size_t)s * V);
+    }
+    const float m_new = fmaxf(M, fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3])));
+    const float keep = fast_exp2(M - m_new);
+    total *= keep;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] *= keep;
+    M = m_new;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float w = s0 + i < NS ? fast_exp2(mx[i] - M) : 0.f;
+      total += w * l[i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] += w * v[i][e];
+    }
+  }
+  const float inv = 1.0f / (total + fast_exp2(sink2 - M));      // the sink counts once, here
+  u16* og = (u16*)a.out + ((int64_t)(q0 + r / R) * a.n_heads + head) * V + col;
+  *reinterpret_cast<u16x4*>(og) = u16x4{BF16::from_float(o[0] * inv), BF16::from_float(o[1] * inv), BF16::from_float(o[2] * inv), BF16::from_float(o[3] * inv)};
+}
+
+template <int D, int V>
+int launch_step(const hxm_biased_attn_args& a, hipStream_t s) {
+  const int R = a.n_heads / a.kv_heads, tiles_per_seq = (int)(((int64_t)a.max_q_len * R + 15) / 16), n_splits = a.n_splits > 1 ? a.n_splits : 1;
+  const int64_t items = (int64_t)a.n_seq * a.kv_heads * tiles_per_seq;
+  if (items * n_splits > 0x7fffffff) return HX_ERR_SHAPE;
+  const bool mods = a.slopes || a.softcap > 0.f;
+  auto kernel = mods ? biased_attn_step_kernel<D, V, true> : biased_attn_step_kernel<D, V, false>;
+  kernel<<<dim3((unsigned)(items * n_splits)), dim3(64), 2 * 32 * (2 * D + 2 * V), s>>>(a, tiles_per_seq);
+  if (n_splits > 1) biased_attn_merge_kernel<V><<<dim3((unsigned)((items * 16 * (V / 4) + 255) / 256)), dim3(256), 0, s>>>(a, tiles_per_seq);
+  return hxm::check_launch();
+}
+
 // the splits of a (sequence, kv head, row tile) merged: out = sum_s O_s e^(m_s - M) / sum_s l_s e^(m_s - M)
 __global__ __launch_bounds__(256) void biased_attn_combine_kernel(hxm_biased_attn_args a, int tiles_per_seq) {
   const int64_t item = blockIdx.x;
@@ -998,11 +1281,16 @@ extern "C" int hxm_biased_attention(const hxm_biased_attn_args* args, void* stre
   hipStream_t s = (hipStream_t)stream;
   if (a.n_splits > 1 && (a.n_splits > 64 || !a.ws_o || !a.ws_ml || !tile_form_serves(a))) return HX_ERR_WORKSPACE;
   if (tile_form_serves(a)) {
-    // portions of prompts with heads of 64 or 128 over pages of whole 16-row groups: from half a row tile of 128 on
-    const bool wide = (a.dim == 64 || a.dim == 128) && (a.vdim == 64 || a.vdim == 128);
-    if (wide && a.form != 2 && a.block_size % 16 == 0 && aligned16(a.out) && (int64_t)a.max_q_len * (a.n_heads / a.kv_heads) >= 64) {
+    // heads of 64 or 128 over pages of whole 16-row groups: the wide form from half a row tile of 128 on, the step form below and
+    // where the caller has the keys of a row tile dealt out (the tile form: other head and page sizes)
+    const bool whole = (a.dim == 64 || a.dim == 128) && (a.vdim == 64 || a.vdim == 128) && a.form != 2 && a.block_size % 16 == 0 && aligned16(a.out);
+    if (whole && a.n_splits <= 1 && (int64_t)a.max_q_len * (a.n_heads / a.kv_heads) >= 64) {
       if (a.dim == 64) return a.vdim == 64 ? launch_wide<64, 64>(a, s) : launch_wide<64, 128>(a, s);
       return a.vdim == 64 ? launch_wide<128, 64>(a, s) : launch_wide<128, 128>(a, s);
+    }
+    if (whole && a.cache_row_stride < (1 << 26) && aligned16(a.ws_o)) {
+      if (a.dim == 64) return a.vdim == 64 ? launch_step<64, 64>(a, s) : launch_step<64, 128>(a, s);
+      return a.vdim == 64 ? launch_step<128, 64>(a, s) : launch_step<128, 128>(a, s);
     }
     const int kk = ((a.dim > a.vdim ? a.dim : a.vdim) + 31) / 32;
     if (kk <= 1) return launch_tile<1>(a, s);

@@ -1021,15 +1021,6 @@ __global__ __launch_bounds__(256, KK <= 4 ? 2 : 1) void latent_attn_wide_kernel(
 // about 5 are the splits' sums going out (8 MB); 1 token behind 1000 keys 70 us and 24, most of it the host's.  Row r of sixteen has its chunks at x ^ swz(r): rows r and 15 - r share a 32-byte place (their
 // chunks turned), so that a pass of a 16-byte read (rows 0-3 and 12-15 of one chunk, 4-11 of the next) and a transposing read
 // (eight rows, 32 bytes each) both reach every bank once.
-__device__ __forceinline__ float groups_max(float v) {      // over the four lanes with the same lane % 16
-  const auto a = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
-  const unsigned a0 = a[0], a1 = a[1];
-  v = fmaxf(__builtin_bit_cast(float, a0), __builtin_bit_cast(float, a1));
-  const auto b = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
-  const unsigned b0 = b[0], b1 = b[1];
-  return fmaxf(__builtin_bit_cast(float, b0), __builtin_bit_cast(float, b1));
-}
-
 template <int KK>
 __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_attn_args a, int tiles_per_seq) {
   constexpr int R = 64 * KK, KT = 32, TQ = 64, KPW = 8, KS = R / 32, NDB = R / 16, RS = 2 * R, L = R / 8, IMG = KT * RS;

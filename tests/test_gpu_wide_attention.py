@@ -1,6 +1,7 @@
 """Biased attention over portions of prompts with heads of 64 and 128 (csrc/biased_attn.hip, the wide form) at the edges of its
 tiles — 128 rows of a key head, 64 keys — under every mask, with slopes, soft caps, temperatures of either sign and of zero,
-sinks, and other key than value sizes."""
+sinks, and other key than value sizes; and over single tokens and a few (the step form: 16 rows, 32 keys), their keys dealt to several
+waves or not."""
 import math
 
 import pytest
@@ -44,11 +45,28 @@ BATCHES = [[(16, 16)], [(31, 31), (33, 100)], [(64, 65), (1, 200), (32, 32)], [(
 @pytest.mark.parametrize("mask, size", [("causal", 0), ("window", 1), ("window", 63), ("chunk", 48)])
 @pytest.mark.parametrize("extra", ["plain", "slopes", "cap", "temperatures and sinks"])
 def test_wide_form(batch, H, G, D, V, mask, size, extra):
-    from hydrainfer_amd._C.kernel.biased_attn import biased_attention
-    g = torch.Generator().manual_seed(H * D + V + size + sum(a + b for a, b in batch))
     new, kv = [a for a, _ in batch], [b for _, b in batch]
     if max(new) * (H // G) < 64:
         new[0], kv[0] = 64, max(64, kv[0])
+    check(new, kv, H, G, D, V, mask, size, extra)
+
+
+# single tokens at the edges of tiles and splits, sequences far shorter than others, two row tiles, more keys in one run than a wave
+# holds pages of (1024), sixteen tokens behind many keys
+STEPS = [[(1, 1)], [(1, 32), (1, 33), (1, 200), (1, 1025)], [(3, 70), (1, 16), (7, 2300)], [(1, 100)] * 40, [(16, 1500), (2, 40)]]
+
+
+@pytest.mark.parametrize("batch", STEPS, ids=lambda b: f"{len(b)}x{max(b)}")
+@pytest.mark.parametrize("H, G, D, V", [(4, 1, 128, 128), (32, 8, 64, 64), (6, 2, 128, 64), (16, 16, 64, 128), (17, 1, 128, 128)])
+@pytest.mark.parametrize("mask, size, extra", [("causal", 0, "plain"), ("window", 63, "slopes"), ("chunk", 48, "cap"), ("causal", 0, "temperatures and sinks")])
+@pytest.mark.parametrize("divided", [True, False])
+def test_step_form(batch, H, G, D, V, mask, size, extra, divided):
+    check([a for a, _ in batch], [b for _, b in batch], H, G, D, V, mask, size, extra, divided)
+
+
+def check(new, kv, H, G, D, V, mask, size, extra, divided=True):
+    from hydrainfer_amd._C.kernel.biased_attn import biased_attention
+    g = torch.Generator().manual_seed(H * D + V + size + sum(new) + sum(kv))
     nb = [(n + BLOCK - 1) // BLOCK for n in kv]
     perm = torch.randperm(sum(nb) + 1, generator=g)
     r = lambda *s: torch.randn(s, generator=g).bfloat16()
@@ -69,7 +87,7 @@ def test_wide_form(batch, H, G, D, V, mask, size, extra):
     table = perm[:sum(nb)].int()
     c = lambda t: None if t is None else t.cuda()
     got = biased_attention(c(q), c(kc), c(vc), V, c(seq), c(torch.tensor(pos, dtype=torch.int32)), c(cu_q), c(table), c(cu_b), D ** -0.5, c(slopes), mask,
-                           size, max_q_len=max(new), max_kv_len=max(kv), softcap=cap, head_scale=c(temps), sinks=c(sinks)).double().cpu()
+                           size, max_q_len=max(new), max_kv_len=max(kv) if divided else 0, softcap=cap, head_scale=c(temps), sinks=c(sinks)).double().cpu()
     for s in range(len(new)):
         lo, hi = int(cu_q[s]), int(cu_q[s + 1])
         pages = table[int(cu_b[s]):int(cu_b[s + 1])].long()
