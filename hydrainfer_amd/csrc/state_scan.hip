@@ -12,8 +12,8 @@
 // are read back 16 bytes at a time; the next chunk is on its way into registers while the current one is scanned (two LDS
 // images, one barrier a chunk), so the serial chain waits for no global load.  Batches of single tokens, short portions and
 // keys of more than 128 channels (longer portions: chunk_scan.hip).  The state comes from the sequence's slot
-// (zeros for a portion that starts at position 0) and goes back.  KR x PARTS follows the key size (8 x 4 ... 16 x 16); a
-// batch of single tokens takes two columns a lane.
+// (zeros for a portion that starts at position 0) and goes back.  KR x PARTS follows the key size (8 x 4 ... 16 x 16).  Batches of
+// single tokens take the step form below where their rows can be moved four columns at a time, else two columns a lane.
 #include "chunk_scan.h"
 #include "mix_rows.h"
 #include "../../include/hydra_mix.h"
@@ -331,6 +331,152 @@ int launch_rows(const hxm_state_scan_args& a, hipStream_t s) {
   }
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// Step form: batches of single tokens, bound by the states that go by.  The form above reads a state 32 bytes at a time (a lane
+// owns a column); here a workgroup takes 64 columns of one (sequence, head), a lane four neighbouring ones of NR consecutive rows:
+// its loads and stores are 16 bytes, a row's 256 together.  The sums over key channels end in four exchanges of lanes and one of
+// waves through LDS (the delta rule has two).  A portion of several tokens goes by one after the other, its operands waited for
+// each time.
+// Measured, 32 tokens, 64 heads of 128 x 64, one decay a head: 49 us above (2.9 TB/s), 23 us here (5.9 TB/s); 128
+// tokens 188 and 81 us; 32 tokens, 32 heads of 128 x 128 under the delta rule 49 and 24 us; 256 tokens, 64 heads of 32 x 16, where
+// most lanes are idle, 64 and 35 us.
+// ---------------------------------------------------------------------------------------------------------------
+template <int NR, int MODE, bool VEC>      // NR: rows a lane; KP = 16 NR >= dim
+__global__ __launch_bounds__(256) void state_step_kernel(hxm_state_scan_args a) {
+  constexpr int KP = 16 * NR, OPS = VEC ? 3 : 2;
+  __shared__ __attribute__((aligned(16))) float ops[OPS][KP], us[MODE == HXM_SCAN_BONUS ? KP : 4], vs[64], red[3][4][64];
+  const int seq = blockIdx.x, head = blockIdx.y, K = a.dim, V = a.vdim, tid = threadIdx.x;
+  const int wave = tid >> 6, lane = tid & 63, at4 = 4 * (lane & 15), first = (4 * wave + (lane >> 4)) * NR;
+  const int col0 = (int)blockIdx.z * 64, col = col0 + at4, col_in = min(col, V - 4);      // (columns past the last four repeat them, and go nowhere)
+  const int t_begin = a.q_cu[seq], t_end = a.q_cu[seq + 1];
+  if (t_end <= t_begin) return;
+  char* slot = (char*)(a.state + (int64_t)a.slots[seq] * a.slot_stride + (int64_t)head * K * V);
+  const int64_t qk_first = (int64_t)(head / (a.heads / a.qk_heads)) * K;
+  // a token's operands: thread i brings channel i of each (zeros past the last) and value i
+  float f[OPS], fv, decay = 0.f, vscale = 1.f, beta = 0.f;
+  auto fetch = [&](int t) {
+    const int i = min(tid, K - 1);
+    const int64_t th = (int64_t)t * a.heads + head;
+    f[0] = load_one(a.q, a.q_dtype, (int64_t)t * a.q_stride + qk_first + i);
+    f[1] = load_one(a.k, a.k_dtype, (int64_t)t * a.k_stride + qk_first + i);
+    if (VEC) f[OPS - 1] = a.decay[th * K + i];
+    fv = load_one(a.v, a.v_dtype, (int64_t)t * a.v_stride + (int64_t)head * V + min(col0 + lane, V - 1));
+    if (!VEC) decay = a.decay[th];
+    if (MODE == HXM_SCAN_DECAY && a.vscale) vscale = a.vscale[th];
+    if (MODE == HXM_SCAN_DELTA) beta = a.beta[th];
+  };
+  if (MODE == HXM_SCAN_BONUS && tid < KP) us[tid] = tid < K ? a.bonus[(int64_t)head * K + tid] : 0.f;
+  fetch(t_begin);
+  f32x4 S[NR];
+  auto row_at = [&](int r) { return (uint32_t)(min(first + r, K - 1) * V + col_in) * 4u; };      // (bytes)
+  if (a.positions[t_begin] == 0) {
+#pragma unroll
+    for (int r = 0; r < NR; ++r) S[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+  } else {
+#pragma unroll
+    for (int r = 0; r < NR; ++r) S[r] = *reinterpret_cast<const f32x4*>(slot + row_at(r));
+  }
+  // the sum over the workgroup's rows of what a lane holds for its four columns
+  auto over_rows = [&](f32x4 x, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float y = x[e];
+      y += __shfl_xor(y, 16, 64);
+      x[e] = y + __shfl_xor(y, 32, 64);
+    }
+    if (lane < 16) *reinterpret_cast<f32x4*>(&red[buf][wave][at4]) = x;
+    __syncthreads();
+    return (*reinterpret_cast<const f32x4*>(&red[buf][0][at4]) + *reinterpret_cast<const f32x4*>(&red[buf][1][at4])) +
+           (*reinterpret_cast<const f32x4*>(&red[buf][2][at4]) + *reinterpret_cast<const f32x4*>(&red[buf][3][at4]));
+  };
+  auto rows4 = [&](int op, int r) __attribute__((always_inline)) { return *reinterpret_cast<const f32x4*>(&ops[op][first + r]); };
+  for (int t = t_begin; t < t_end; ++t) {
+    if (tid < KP) {
+#pragma unroll
+      for (int i = 0; i < OPS; ++i) ops[i][tid] = tid < K ? f[i] : 0.f;
+    }
+    if (tid < 64) vs[tid] = fv * vscale;
+    const float d1 = decay, b = beta;
+    __syncthreads();
+    if (t + 1 < t_end) fetch(t + 1);
+    const f32x4 v = *reinterpret_cast<const f32x4*>(&vs[at4]);
+    f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f}, sk = o;
+#pragma unroll
+    for (int r0 = 0; r0 < NR; r0 += 4) {
+      const f32x4 q4 = rows4(0, r0), k4 = rows4(1, r0), d4 = VEC ? rows4(OPS - 1, r0) : f32x4{d1, d1, d1, d1};
+      f32x4 u4 = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (MODE == HXM_SCAN_BONUS) u4 = *reinterpret_cast<const f32x4*>(&us[first + r0]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = r0 + i;
+        const float q = q4[i], k = k4[i], d = d4[i];
+        const float u = u4[i];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (MODE == HXM_SCAN_DECAY) {
+            S[r][e] = d * S[r][e] + k * v[e];
+            o[e] += S[r][e] * q;
+          } else if (MODE == HXM_SCAN_BONUS) {
+            const float kv = k * v[e];
+            o[e] += (S[r][e] + u * kv) * q;
+            S[r][e] = d * S[r][e] + kv;
+          } else {
+            S[r][e] *= d;
+            sk[e] += S[r][e] * k;
+          }
+        }
+      }
+    }
+    if (MODE == HXM_SCAN_DELTA) {
+      sk = over_rows(sk, 2);
+      f32x4 w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = b * (v[e] - sk[e]);
+#pragma unroll
+      for (int r0 = 0; r0 < NR; r0 += 4) {
+        const f32x4 q4 = rows4(0, r0), k4 = rows4(1, r0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            S[r0 + i][e] += k4[i] * w[e];
+            o[e] += S[r0 + i][e] * q4[i];
+          }
+      }
+    }
+    o = over_rows(o, (t - t_begin) & 1);     // (two images: a wave may still be reading the last token's)
+    if (wave == 0 && lane < 16 && col < V) *reinterpret_cast<f32x4*>(a.out + ((int64_t)t * a.heads + head) * V + col) = o;
+  }
+#pragma unroll
+  for (int r = 0; r < NR; ++r)
+    if (first + r < K && col < V) *reinterpret_cast<f32x4*>(slot + row_at(r)) = S[r];
+}
+
+template <int NR, int MODE>
+int launch_step_mode(const hxm_state_scan_args& a, hipStream_t s) {
+  const dim3 grid((unsigned)a.n_seq, (unsigned)a.heads, (unsigned)((a.vdim + 63) / 64)), block(256);
+  if (a.decay_per_channel) state_step_kernel<NR, MODE, true><<<grid, block, 0, s>>>(a);
+  else state_step_kernel<NR, MODE, false><<<grid, block, 0, s>>>(a);
+  return hxm::check_launch();
+}
+
+template <int NR>
+int launch_step(const hxm_state_scan_args& a, hipStream_t s) {
+  switch (a.mode) {
+    case HXM_SCAN_DECAY: return launch_step_mode<NR, HXM_SCAN_DECAY>(a, s);
+    case HXM_SCAN_BONUS: return launch_step_mode<NR, HXM_SCAN_BONUS>(a, s);
+    case HXM_SCAN_DELTA: return launch_step_mode<NR, HXM_SCAN_DELTA>(a, s);
+    default: return HX_ERR_UNSUPPORTED;
+  }
+}
+
+// Four columns of a row at a time: rows and slots start on multiples of four floats.  Only as many tokens as sequences: a second
+// token of a portion costs it 2 us, twice what it costs above, and a batch of a few more tokens may hold one long portion.
+bool step_serves(const hxm_state_scan_args& a) {
+  auto al = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  return a.n_tokens == a.n_seq && a.vdim % 4 == 0 && a.slot_stride % 4 == 0 && al(a.state) && al(a.out);
+}
+
 }  // namespace
 
 extern "C" int hxm_state_scan(const hxm_state_scan_args* args, void* stream) {
@@ -360,6 +506,11 @@ extern "C" int hxm_state_scan(const hxm_state_scan_args* args, void* stream) {
     c.state = a.state; c.slot_stride = a.slot_stride; c.slots = a.slots; c.q_cu = a.q_cu; c.positions = a.positions;
     c.n_seq = a.n_seq; c.heads = a.heads; c.qk_heads = a.qk_heads; c.K = a.dim; c.V = a.vdim;
     if (hxm::chunk_scan_fits(c)) return hxm::chunk_scan(c, s);
+  }
+  if (step_serves(a)) {
+    if (a.dim <= 64) return launch_step<4>(a, s);
+    if (a.dim <= 128) return launch_step<8>(a, s);
+    return launch_step<16>(a, s);
   }
   // key channels a lane x lanes a column: 8 x 4, 8 x 8, 16 x 8, 16 x 16 (chunks of 16 tokens; 8 at the widest)
   if (a.dim <= 32) return launch_rows<8, 4, 16>(a, s);

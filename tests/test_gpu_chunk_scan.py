@@ -45,6 +45,20 @@ LENS = [[17], [16, 1, 33], [1, 15, 31, 2], [48, 5]]
 @pytest.mark.parametrize("form, per_channel", [("decay", False), ("decay", True), ("delta", False), ("bonus", True)])
 @pytest.mark.parametrize("types", ["bf16", "f32", "mixed"])
 def test_portions_through_a_scan(lens, K, V, form, per_channel, types):
+    _through_a_scan(lens, K, V, form, per_channel, types, 3)
+
+
+# batches of as many tokens as sequences (csrc/state_scan.hip, the step form): columns and rows that fill no workgroup, a sequence that
+# brings two tokens and one that brings none, slots that start on a multiple of four floats and (the form with a column a lane) not
+@pytest.mark.parametrize("lens", [[1], [1, 1, 1, 1, 1], [2, 0, 1]])
+@pytest.mark.parametrize("K, V", [(64, 64), (128, 128), (12, 20), (100, 132), (65, 8), (256, 68), (3, 4)])
+@pytest.mark.parametrize("form, per_channel", [("decay", False), ("decay", True), ("delta", False), ("bonus", True)])
+@pytest.mark.parametrize("types, pad", [("bf16", 4), ("f32", 4), ("mixed", 4), ("mixed", 3)])
+def test_single_tokens_through_a_scan(lens, K, V, form, per_channel, types, pad):
+    _through_a_scan(lens, K, V, form, per_channel, types, pad)
+
+
+def _through_a_scan(lens, K, V, form, per_channel, types, pad):
     from hydrainfer_amd._C.kernel.seq_mix import state_scan
     from hydrainfer_amd._C.kernel.stream_ops import SequenceState
     g = torch.Generator().manual_seed(sum(lens) * 1000 + K + V)
@@ -60,7 +74,7 @@ def test_portions_through_a_scan(lens, K, V, form, per_channel, types):
     decay[T // 3] = 0.0                                            # forgets everything, and nothing divides by it
     decay[T // 2, 0] = 1e-30
     vscale, beta, bonus = torch.rand((T, H), generator=g), torch.rand((T, H), generator=g), torch.randn(H * K, generator=g)
-    state = torch.randn((n + 1, 1, H * K * V + 3), generator=g)
+    state = torch.randn((n + 1, 1, H * K * V + pad), generator=g)
     slots = torch.randperm(n + 1, generator=g)[:n].int()
     cu = [0]
     for x in lens:
@@ -71,18 +85,18 @@ def test_portions_through_a_scan(lens, K, V, form, per_channel, types):
     heads = lambda x: x.double().view(T, G, K).repeat_interleave(H // G, dim=1)
     want, S = _scan(form, heads(q), heads(k), v.double().view(T, H, V), (decay.double().view(T, H, -1)).expand(T, H, K),
                     vscale.double() if form == "decay" else torch.ones((T, H), dtype=torch.float64), beta.double(), bonus.double().view(H, K),
-                    state[slots.long(), 0, 3:].double().view(n, H, K, V), cu, [p == 0 for p in starts])
+                    state[slots.long(), 0, pad:].double().view(n, H, K, V), cu, [p == 0 for p in starts])
     d = lambda x: x.cuda()
     st = d(state)
     before = st.clone()
     seq = SequenceState(st, d(slots), d(tok_seq))
     pd = d(proj)
-    got = state_scan(form, pd[:, :G * K], pd[:, G * K:2 * G * K], d(v), d(decay), seq, 3, d(torch.tensor(cu, dtype=torch.int32)), d(pos), H, G, K, V,
+    got = state_scan(form, pd[:, :G * K], pd[:, G * K:2 * G * K], d(v), d(decay), seq, pad, d(torch.tensor(cu, dtype=torch.int32)), d(pos), H, G, K, V,
                      vscale=d(vscale) if form == "decay" else None, beta=d(beta) if form == "delta" else None, bonus=d(bonus) if form == "bonus" else None)
     _check("out", got, want.reshape(T, H * V))
-    _check("state", st[slots.long().cuda(), 0, 3:].view(n, H, K, V), S)
+    _check("state", st[slots.long().cuda(), 0, pad:].view(n, H, K, V), S)
     other = [s for s in range(n + 1) if s not in slots.tolist()]
-    assert torch.equal(st[other], before[other]) and torch.equal(st[:, 0, :3], before[:, 0, :3])
+    assert torch.equal(st[other], before[other]) and torch.equal(st[:, 0, :pad], before[:, 0, :pad])
 
 
 @pytest.mark.parametrize("lens", LENS)
