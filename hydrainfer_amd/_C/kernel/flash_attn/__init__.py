@@ -110,8 +110,7 @@ def mha_varlen_fwd(out: Tensor, q: Tensor, k: Tensor, v: Tensor, cu_seqlens_q: T
     if need > 0:
         ws = torch.empty(need, dtype=torch.uint8, device=q.device)
         a.workspace, a.workspace_bytes = ws.data_ptr(), need
-    with torch.cuda.device(q.device):
-        _lib.check(l.hx_mha_varlen_fwd(ctypes.byref(a), _lib.current_stream()), "mha_varlen_fwd")
+    _lib.check(l.hx_mha_varlen_fwd(ctypes.byref(a), _lib.current_stream()), "mha_varlen_fwd")
 
 
 def decode_attention_fused(out: Tensor, q: Tensor, k_new: Tensor, v_new: Tensor, key_cache: Tensor,
@@ -182,9 +181,7 @@ def decode_attention_fused(out: Tensor, q: Tensor, k_new: Tensor, v_new: Tensor,
     if need > 0:
         ws = torch.empty(need, dtype=torch.uint8, device=q.device)
         a.workspace, a.workspace_bytes = ws.data_ptr(), need
-    with torch.cuda.device(q.device):
-        _lib.check(l.hx_decode_attention_fused(ctypes.byref(a), ctypes.byref(fz), _lib.current_stream()),
-                   "decode_attention_fused")
+    _lib.check(l.hx_decode_attention_fused(ctypes.byref(a), ctypes.byref(fz), _lib.current_stream()), "decode_attention_fused")
 
 
 def decode_rank(cu_seqlens_k: Tensor, out: Optional[Tensor] = None) -> Tensor:
@@ -199,6 +196,5 @@ def decode_rank(cu_seqlens_k: Tensor, out: Optional[Tensor] = None) -> Tensor:
         out = torch.empty(batch + 1, dtype=torch.int32, device=cu_seqlens_k.device)
     elif out.dtype != torch.int32 or not out.is_contiguous() or out.numel() < batch + 1:
         raise _lib.HydraHipError("decode_rank: out must be contiguous int32 [1 + batch]")
-    with torch.cuda.device(cu_seqlens_k.device):
-        _lib.check(_lib.lib().hx_decode_rank(cu_seqlens_k.data_ptr(), batch, out.data_ptr(), _lib.current_stream()), "decode_rank")
+    _lib.check(_lib.lib().hx_decode_rank(cu_seqlens_k.data_ptr(), batch, out.data_ptr(), _lib.current_stream()), "decode_rank")
     return out
