@@ -93,11 +93,53 @@ __global__ __launch_bounds__(256) void route_softmax_topk_kernel(const float* __
   }
 }
 
+// A token's choice by one wave: z[i] is the logit of expert lane + 64 i (-inf past the last).  A choice is a maximum over the wave on
+// the vector ALU and a ballot for the lowest expert that holds it; the weights are the softmax of the chosen logits.
+template <int PER>
+__device__ __forceinline__ void choose_top(const float (&z)[PER], int lane, int E, int top, float* __restrict__ weights, int32_t* __restrict__ experts) {
+  uint64_t left[PER];         // the experts not chosen yet
+#pragma unroll
+  for (int i = 0; i < PER; ++i) left[i] = __ballot(lane + 64 * i < E);
+  float my_z = 0.f, first = 0.f;      // lane k keeps the k-th choice
+  int my_e = 0;
+  for (int k = 0; k < top; ++k) {
+    float best = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      if ((left[i] >> lane) & 1) best = fmaxf(best, z[i]);
+    best = row16_max(best);
+    const int bits = __builtin_bit_cast(int, best);
+    best = fmaxf(fmaxf(__builtin_bit_cast(float, __builtin_amdgcn_readlane(bits, 0)), __builtin_bit_cast(float, __builtin_amdgcn_readlane(bits, 16))),
+                 fmaxf(__builtin_bit_cast(float, __builtin_amdgcn_readlane(bits, 32)), __builtin_bit_cast(float, __builtin_amdgcn_readlane(bits, 48))));
+    int chosen = -1, fallback = -1;
+#pragma unroll
+    for (int i = PER - 1; i >= 0; --i) {
+      const uint64_t at = __ballot(z[i] == best) & left[i];
+      if (at) chosen = 64 * i + __builtin_ctzll(at);
+      if (left[i]) fallback = 64 * i + __builtin_ctzll(left[i]);
+    }
+    if (chosen < 0) chosen = fallback;                        // (logits that are not numbers: still distinct experts)
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      if (chosen >= 64 * i && chosen < 64 * (i + 1)) left[i] &= ~(1ull << (chosen & 63));
+    if (k == 0) first = best;
+    if (lane == k) {
+      my_z = best;
+      my_e = chosen;
+    }
+  }
+  const float ex = lane < top ? expf(my_z - first) : 0.f;
+  const float total = wave_sum(ex);
+  if (lane < top) {
+    weights[lane] = ex / total;
+    experts[lane] = my_e;
+  }
+}
+
 // Router product and choice in one kernel: a workgroup takes 16 tokens; its waves deal the sum over k among themselves, U
 // slices of 16 neighbouring k at a time, with float matrix instructions (16 tokens x 16 experts x 4 k: a lane brings four
 // neighbouring k of its token's row and of its experts' rows, element e of every lane makes one instruction), their sums meet
-// in LDS in a fixed order, and every wave chooses for the tokens whose number is its own (mod waves).  A choice is a maximum
-// over the wave on the vector ALU and a ballot for the lowest expert that holds it.
+// in LDS in a fixed order, and every wave chooses for the tokens whose number is its own (mod waves).
 template <int NT, int WAVES>      // experts in tiles of 16
 __global__ __launch_bounds__(64 * WAVES) void router_topk_kernel(const float* __restrict__ x, int64_t x_stride, const float* __restrict__ w,
                                                                  const float* __restrict__ bias, int64_t n_tokens, int64_t K, int E, int top,
@@ -163,44 +205,49 @@ __global__ __launch_bounds__(64 * WAVES) void router_topk_kernel(const float* __
         z[i] = s + (bias ? bias[e] : 0.f);
       }
     }
-    uint64_t left[PER];         // the experts not chosen yet
-#pragma unroll
-    for (int i = 0; i < PER; ++i) left[i] = __ballot(lane + 64 * i < E);
-    float my_z = 0.f, first = 0.f;      // lane k keeps the k-th choice
-    int my_e = 0;
-    for (int k = 0; k < top; ++k) {
-      float best = -INFINITY;
-#pragma unroll
-      for (int i = 0; i < PER; ++i)
-        if ((left[i] >> lane) & 1) best = fmaxf(best, z[i]);
-      best = row16_max(best);
-      const int bits = __builtin_bit_cast(int, best);
-      best = fmaxf(fmaxf(__builtin_bit_cast(float, __builtin_amdgcn_readlane(bits, 0)), __builtin_bit_cast(float, __builtin_amdgcn_readlane(bits, 16))),
-                   fmaxf(__builtin_bit_cast(float, __builtin_amdgcn_readlane(bits, 32)), __builtin_bit_cast(float, __builtin_amdgcn_readlane(bits, 48))));
-      int chosen = -1, fallback = -1;
-#pragma unroll
-      for (int i = PER - 1; i >= 0; --i) {
-        const uint64_t at = __ballot(z[i] == best) & left[i];
-        if (at) chosen = 64 * i + __builtin_ctzll(at);
-        if (left[i]) fallback = 64 * i + __builtin_ctzll(left[i]);
-      }
-      if (chosen < 0) chosen = fallback;                        // (logits that are not numbers: still distinct experts)
-#pragma unroll
-      for (int i = 0; i < PER; ++i)
-        if (chosen >= 64 * i && chosen < 64 * (i + 1)) left[i] &= ~(1ull << (chosen & 63));
-      if (k == 0) first = best;
-      if (lane == k) {
-        my_z = best;
-        my_e = chosen;
-      }
-    }
-    const float ex = lane < top ? expf(my_z - first) : 0.f;
-    const float total = wave_sum(ex);
-    if (lane < top) {
-      weights[t * top + lane] = ex / total;
-      experts[t * top + lane] = my_e;
-    }
+    choose_top<PER>(z, lane, E, top, weights + t * top, experts + t * top);
   }
+}
+
+// The same for few tokens: a workgroup of sixteen waves a token, a wave an expert after the other, its products on the vector ALU.
+// The form above puts sixteen tokens on one CU: their matrix products (float, 4 us for 16 experts of 4096) and the rows that pass
+// through its one L1 take what the chip's other CUs could share.  4 of 16 experts of 4096: 32 tokens 17.3 us above, 6.7 here; 4 of
+// 128: 67 and 33 us.
+__global__ __launch_bounds__(1024) void router_few_kernel(const float* __restrict__ x, int64_t x_stride, const float* __restrict__ w,
+                                                          const float* __restrict__ bias, int64_t K, int E, int top,
+                                                          float* __restrict__ weights, int32_t* __restrict__ experts) {
+  __shared__ float logits[128];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int64_t t = blockIdx.x;
+  const float* xr = x + t * x_stride;
+  for (int e = wave; e < E; e += 16) {
+    const float* wr = w + (int64_t)e * K;
+    constexpr int U = 8;                                   // pieces of 256 in flight
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int64_t k0 = 4 * lane; k0 < K; k0 += 256 * U) {
+      f32x4 xv[U], wv[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t k = k0 + 256 * u < K ? k0 + 256 * u : 4 * lane;      // (past the end: the lane's first, and not used)
+        xv[u] = *reinterpret_cast<const f32x4*>(xr + k);
+        wv[u] = *reinterpret_cast<const f32x4*>(wr + k);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const bool in = k0 + 256 * u < K;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = in ? __builtin_fmaf(xv[u][i], wv[u][i], acc[i]) : acc[i];
+      }
+    }
+    const float sum = wave_sum((acc[0] + acc[1]) + (acc[2] + acc[3]));
+    if (lane == 0) logits[e] = sum + (bias ? bias[e] : 0.f);
+  }
+  __syncthreads();
+  if (wave > 0) return;
+  float z[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) z[i] = lane + 64 * i < E ? logits[lane + 64 * i] : -INFINITY;
+  choose_top<2>(z, lane, E, top, weights + t * top, experts + t * top);
 }
 
 // one workgroup of 1024 threads: histogram, exclusive scan, scatter, all through LDS counters
@@ -683,6 +730,12 @@ extern "C" int hxm_router_topk(const float* x, int64_t x_stride, const float* w,
   if (x_stride < k_dim || x_stride % 4 || !aligned16(x) || !aligned16(w)) return HX_ERR_STRIDE;
   const dim3 grid((unsigned)((n_tokens + 15) / 16));
   hipStream_t s = (hipStream_t)stream;
+  // A workgroup a token while the CUs take them in one round, two where an expert's row is soon read (above / a workgroup a token:
+  // 16 experts of 4096, 256 tokens 17.4 / 7.3 us, 512 17.5 / 11.7, 1024 17.7 / 20.7; 128 of 1024, 256 21.4 / 20.2, 384 21.6 / 35.1).
+  if (n_tokens <= (n_experts <= 32 ? 512 : 256)) {
+    router_few_kernel<<<dim3((unsigned)n_tokens), dim3(1024), 0, s>>>(x, x_stride, w, bias, k_dim, n_experts, top, weights, experts);
+    return hxm::check_launch();
+  }
 #define HXM_ROUTER(NT_, WAVES_)                                                                                                  \
   router_topk_kernel<NT_, WAVES_><<<grid, dim3(64 * WAVES_), 0, s>>>(x, x_stride, w, bias, n_tokens, k_dim, n_experts, top, weights, experts)
   if (n_experts <= 16) HXM_ROUTER(1, 16);
