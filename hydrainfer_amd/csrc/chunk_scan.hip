@@ -18,10 +18,10 @@
 //   per head:    chunk_head_kernel — Q K^T and K K^T on the matrix cores, decays as factors of the accumulators' rows.
 //   per channel: chunk_channel_kernel — A by running products over the tokens on the vector ALU, a lane one or two key channels,
 //                summed over the wave by a transposing butterfly that leaves one element of A in every second lane.
-// What bounds it now: the chunks of a sequence follow each other (2.6 us each with states of 128 x 128, 1.4 us of that float
-// matrix products).  Measured against one token at a time, 4 portions of 797 - 1151 tokens: delta rule, 32 heads of 128 x 128,
-// 479 -> 206 us; decayed sum, 64 heads of 128 x 64, 432 -> 165 us; bonus form, 32 heads of 64 x 64, 207 -> 104 us; gated form,
-// 32 heads of 128 x 128, 691 -> 208 us with its norm.  Error against 64 bits (2-norm): results 1.4e-7 / 1.0e-7 / 1.0e-7 (delta
+// What bounds it now: the chunks of a sequence follow each other (2.5 us each with states of 128 x 128; 1.8 us of float matrix
+// products on the SIMDs that hold a consumer and a maker of A or M).  Measured against one token at a time, 4 portions of 797 -
+// 1151 tokens: delta rule, 32 heads of 128 x 128, 479 -> 189 us; decayed sum, 64 heads of 128 x 64, 432 -> 155 us; bonus form, 32
+// heads of 64 x 64, 207 -> 102 us; gated form, 32 heads of 128 x 128, 720 -> 213 us with its norm.  Error against 64 bits (2-norm): results 1.4e-7 / 1.0e-7 / 1.0e-7 (delta
 // / decay / bonus; 1.1e-7 / 1.1e-7 / 0.9e-7 before), states 1.0e-7 / 0.9e-7 / 0.7e-7 / 1.1e-7 (gated last; 0.8, 0.8, 0.5, 1.4).
 #include <type_traits>
 #include "chunk_scan.h"
@@ -122,6 +122,20 @@ __device__ __forceinline__ f32x4 times_rows(const float* a, int m, int g, f32x4 
   return c;
 }
 
+// (for the scheduler) FIRST reads from LDS, then a read behind every PER products, N times, then REST products: left alone it
+// asks for two rows and waits for them after every eight products (delta rule 198 -> 189 us, decayed sum 165 -> 155; the gated
+// form, bound by its producers, gains nothing)
+template <int FIRST, int N, int PER, int REST>
+__device__ __forceinline__ void products_behind_reads() {
+  __builtin_amdgcn_sched_group_barrier(0x100, FIRST, 0);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, PER, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+  }
+  __builtin_amdgcn_sched_group_barrier(0x008, REST, 0);
+}
+
 // A chunk's rows on their way to LDS: NT threads, [16][W] of them, four channels a piece; row stride in LDS W + 4.
 template <typename A, bool VEC, int W, int NT>
 struct Rows {
@@ -196,6 +210,7 @@ __global__ __launch_bounds__(512) void chunk_head_kernel(ChunkScanArgs a) {
       const f32x4 within = times_rows(A, m, g, w);
 #pragma unroll
       for (int e = 0; e < 4; ++e) o[e] = __builtin_fmaf(o[e], pre[e], within[e]);
+      products_behind_reads<14, 20, 3, 12>();
       const int n = rows_of(c);
       const int64_t t0 = t_begin + (int64_t)c * C;
 #pragma unroll
@@ -212,6 +227,7 @@ __global__ __launch_bounds__(512) void chunk_head_kernel(ChunkScanArgs a) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) st.S[kt][e] = __builtin_fmaf(st.S[kt][e], total, more[e]);
       }
+      products_behind_reads<16, 16, 2, 1>();
       lds_barrier();
     }
     st.store(slot, a.K, a.V, col, g);
@@ -422,6 +438,7 @@ __global__ __launch_bounds__(768) void chunk_channel_kernel(ChunkScanArgs a) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) w[e] = vs[e * VS];
       const f32x4 o = st.times(p + m * RS + 4 * g) + times_rows(A, m, g, w);
+      if constexpr (!GATED) products_behind_reads<10, 4, 4, 20>();
       const int n = rows_of(c);
       const int64_t t0 = t_begin + (int64_t)c * C;
 #pragma unroll
@@ -437,6 +454,7 @@ __global__ __launch_bounds__(768) void chunk_channel_kernel(ChunkScanArgs a) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) st.S[kt][e] = __builtin_fmaf(st.S[kt][e], d[e], more[e]);
       }
+      if constexpr (!GATED) products_behind_reads<6, 10, 2, 12>();
       lds_barrier();
     }
     st.store(slot, a.K, a.V, col, g);
