@@ -111,7 +111,10 @@ struct F16 {
   static __device__ __forceinline__ float to_float(u16 b) {
     return (float)__builtin_bit_cast(_Float16, b);
   }
+  // (of the float itself: left to the compiler, a product and its rounding become one v_fma_mixlo_f16 in some kernels and two
+  // instructions in others, and a fused form would differ from the plain one in a last place)
   static __device__ __forceinline__ u16 from_float(float f) {
+    asm("" : "+v"(f));
     return __builtin_bit_cast(u16, (_Float16)f);  // RNE
   }
 };
