@@ -1050,11 +1050,10 @@ __global__ __launch_bounds__(64) void biased_attn_step_kernel(hxm_biased_attn_ar
       }
     }
     mx = groups_max(mx);
-    // a row keeps the maximum its weights refer to until a score exceeds it by 2^8
-    const float m_cand = fmaxf(m, mx * unit);
-    const bool grow = m_cand > m + 8.0f;
-    if (__builtin_amdgcn_ballot_w64(grow)) {
-      const float m_new = grow ? m_cand : m, alpha = fast_exp2(m - m_new);
+    // (the weights always refer to the largest score so far: its own is then 1, which no rounding to bfloat16 touches)
+    const float m_new = fmaxf(m, mx * unit);
+    if (__builtin_amdgcn_ballot_w64(m_new > m)) {
+      const float alpha = fast_exp2(m - m_new);
       l *= alpha;
 #pragma unroll
       for (int i = 0; i < NDB; ++i)

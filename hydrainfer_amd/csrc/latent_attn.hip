@@ -1096,6 +1096,7 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
     for (int ks = 0; ks < KS; ++ks) qf[ks] ^= (u16)0x8000;
   }
   scale2 = fmaxf(fabsf(scale2), 1e-30f);
+  const float lag = n_splits > 1 ? 0.f : 8.0f;
   f32x4 acc[NDB];
 #pragma unroll
   for (int i = 0; i < NDB; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1148,9 +1149,10 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
       }
     }
     mx = groups_max(mx);
-    // a row keeps the maximum its weights refer to until a score exceeds it by 2^8
+    // a row keeps the maximum its weights refer to until a score exceeds it by 2^8 (where the keys are dealt out, and few steps
+    // are taken, by nothing: the largest weight is then 1, which no rounding to bfloat16 touches)
     const float m_cand = fmaxf(m, mx * scale2);
-    const bool grow = m_cand > m + 8.0f;
+    const bool grow = m_cand > m + lag;
     if (__builtin_amdgcn_ballot_w64(grow)) {
       const float m_new = grow ? m_cand : m, alpha = fast_exp2(m - m_new);
       l *= alpha;
