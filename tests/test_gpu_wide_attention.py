@@ -42,8 +42,8 @@ BATCHES = [[(16, 16)], [(31, 31), (33, 100)], [(64, 65), (1, 200), (32, 32)], [(
 
 @pytest.mark.parametrize("batch", BATCHES)
 @pytest.mark.parametrize("H, G, D, V", [(4, 1, 128, 128), (32, 8, 64, 64), (6, 2, 128, 64), (16, 16, 64, 128)])
-@pytest.mark.parametrize("mask, size", [("causal", 0), ("window", 1), ("window", 63), ("chunk", 48)])
-@pytest.mark.parametrize("extra", ["plain", "slopes", "cap", "temperatures and sinks"])
+@pytest.mark.parametrize("mask, size, extra", [("causal", 0, "plain"), ("window", 1, "plain"), ("window", 63, "slopes"), ("chunk", 48, "cap"),
+                                               ("causal", 0, "cap"), ("chunk", 48, "temperatures and sinks"), ("causal", 0, "temperatures and sinks")])
 def test_wide_form(batch, H, G, D, V, mask, size, extra):
     new, kv = [a for a, _ in batch], [b for _, b in batch]
     if max(new) * (H // G) < 64:

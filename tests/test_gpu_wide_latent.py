@@ -15,8 +15,7 @@ BATCHES = [[(2, 2)], [(33, 33), (2, 100)], [(5, 70), (1, 200), (32, 32)], [(129,
 
 @pytest.mark.parametrize("batch", BATCHES)
 @pytest.mark.parametrize("R", [64, 128, 192, 256, 320, 384, 512])
-@pytest.mark.parametrize("H", [3, 32])
-@pytest.mark.parametrize("window, extra", [(0, "plain"), (1, "plain"), (31, "sinks"), (50, "gate"), (0, "negative"), (64, "sinks and gate")])
+@pytest.mark.parametrize("H, window, extra", [(32, 0, "plain"), (3, 1, "plain"), (32, 31, "sinks"), (3, 0, "negative"), (32, 64, "sinks and gate")])
 def test_wide_forms(batch, R, H, window, extra):
     new, kv = [a for a, _ in batch], [b for _, b in batch]
     if max(new) * H < 64:
@@ -31,8 +30,7 @@ STEPS = [[64], [129, 1, 32, 33], [2000, 3], [700] * 5, [40] * 260 + [130]]
 
 @pytest.mark.parametrize("kv", STEPS, ids=lambda v: f"{len(v)}x{max(v)}")
 @pytest.mark.parametrize("R", [64, 448, 512])
-@pytest.mark.parametrize("H", [1, 16, 65])
-@pytest.mark.parametrize("window, extra", [(0, "plain"), (300, "sinks and gate"), (0, "negative")])
+@pytest.mark.parametrize("H, window, extra", [(1, 0, "plain"), (16, 0, "negative"), (16, 300, "sinks and gate"), (65, 300, "plain")])
 def test_single_tokens(kv, R, H, window, extra):
     check([1] * len(kv), kv, R, H, window, extra)
 
