@@ -613,7 +613,9 @@ int launch_grouped(u16* y, const u16* x, int64_t x_stride, const int32_t* src, c
   const int64_t grid = ((max_rows + TM - 1) / TM + E) * ((N + TN - 1) / TN) + 7;
   if (grid > 0x7fffffff) return HX_ERR_SHAPE;
   constexpr size_t lds = (size_t)NS * (TM + TN) * 2 * kKS;
-  const bool far = max_rows * x_stride > 0x3fffffff;       // (a token brings a row at least: no input row lies further on)
+  // Offsets of 32 bits (bytes) only for rows that come as they are, of which max_rows is the number: src may name any row of x, and how
+  // many there are is not known here.
+  const bool far = src || max_rows * x_stride > 0x3fffffff;
   auto kernel = far ? grouped_linear_mfma_kernel<TM, TN, WGM, WGN, NS, true> : grouped_linear_mfma_kernel<TM, TN, WGM, WGN, NS, false>;
   if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   kernel<<<dim3((unsigned)grid), dim3(64 * WGM * WGN), lds, s>>>(y, x, x_stride, src, w, seg, E, N, K, act, glu);

@@ -217,7 +217,7 @@ int hxm_moe_plan(const int32_t* experts, int64_t n_tokens, int32_t top, int32_t 
                  int32_t* src, void* stream);
 
 /* Y[r, :] = act(X[src ? src[r] : r, :] . W[e]^T) for the rows r of every expert e (seg as above, n_rows = seg[n_experts]
- * is NOT read by the host: max_rows bounds it).  X: dtype rows of k_dim with stride x_stride; W: dtype [n_experts, n_dim,
+ * is NOT read by the host: max_rows bounds it).  X: dtype rows of k_dim with stride x_stride, with src any number of them; W: dtype [n_experts, n_dim,
  * k_dim]; Y: dtype [max_rows, n_dim].  act: 0 none, 1 squared ReLU, 2 a gated activation: the rows of W come in turns of 16 gates
  * and 16 ups (n_dim a multiple of 32), g = min(gate, glu_limit), u = clamp(up, -glu_limit, glu_limit) (glu_limit <= 0: no clamp),
  * Y [max_rows, n_dim / 2] = g * sigmoid(glu_alpha * g) * (u + glu_up_shift).  Products accumulate in float. */

@@ -39,6 +39,28 @@ def test_grouped_linear_of_rows_far_apart(rows):
     _check(rows, 160, 200, "none", True)
 
 
+@pytest.mark.parametrize("rows", [[3, 0, 5], [60, 70], [300, 1]])
+def test_grouped_linear_of_few_rows_out_of_a_long_input(rows):
+    # rows on both sides of 4 GiB, where an offset of 32 bits would start again at x: there lie other numbers
+    from hydrainfer_amd._C.kernel.moe_mix import grouped_linear
+    E, total, n, k, stride = len(rows), sum(rows), 160, 328, 2 ** 20
+    g = torch.Generator().manual_seed(total)
+    x = torch.empty((2600, stride), dtype=torch.bfloat16, device="cuda")
+    src = torch.randperm(2600, generator=g)[:total].int()
+    src[:2] = torch.tensor([2599, 2599 - 2048])
+    x[:, :k] = torch.randn((2600, k), generator=g).bfloat16().cuda()
+    w = (torch.randn((E, n, k), generator=g) * k ** -0.5).bfloat16()
+    seg = [0]
+    for r in rows:
+        seg.append(seg[-1] + r)
+    got = grouped_linear(x[:, :k], w.cuda(), torch.tensor(seg, dtype=torch.int32, device="cuda"), total, src=src.cuda()).double().cpu()
+    xs = x[:, :k].cpu().double()[src.long()]
+    for e in range(E):
+        want, bound = _reference(xs[seg[e]:seg[e + 1]], w[e].double(), "none")
+        off = (got[seg[e]:seg[e + 1]] - want).abs()
+        assert bool((off <= 2.0 ** -8 * want.abs() + 1.01 * bound + 1e-30).all()), (e, float(off.max()))      # one rounding to bfloat16
+
+
 def _check(rows, n, k, act, far):
     from hydrainfer_amd._C.kernel.moe_mix import grouped_linear
     g = torch.Generator().manual_seed(len(rows) * 1000 + sum(rows) + n + k)
