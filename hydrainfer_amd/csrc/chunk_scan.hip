@@ -122,6 +122,28 @@ __device__ __forceinline__ f32x4 times_rows(const float* a, int m, int g, f32x4 
   return c;
 }
 
+// The same where a row of w may not be a finite number: nothing of it reaches the rows of tokens before its own (zero times infinity
+// would).  Rare, and slow: on the vector ALU, a token after the other.
+__device__ __forceinline__ f32x4 times_rows_in_order(const float* a, int m, int g, f32x4 w) {
+  f32x4 c = f32x4{0.f, 0.f, 0.f, 0.f};
+  asm volatile("" : "+v"(m), "+v"(g));                     // (nothing of this is worked out ahead of the loop over chunks)
+#pragma unroll
+  for (int f = 0; f < 4; ++f)
+#pragma unroll 1
+    for (int h = 0; h < 4; ++h) {                          // token 4 h + f
+      const float x = __shfl(w[f], 16 * h + m, 64);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (4 * h + f <= 4 * g + e) c[e] = __builtin_fmaf(a[(4 * g + e) * RA + 4 * h + f], x, c[e]);
+    }
+  return c;
+}
+// uniform: some number of some lane is infinite or none
+__device__ __forceinline__ bool some_not_finite(f32x4 w) {
+  const bool fine = __builtin_isfinite(w[0]) && __builtin_isfinite(w[1]) && __builtin_isfinite(w[2]) && __builtin_isfinite(w[3]);
+  return __builtin_amdgcn_ballot_w64(!fine) != 0;
+}
+
 // (for the scheduler) FIRST reads from LDS, then a read behind every PER products, N times, then REST products: left alone it
 // asks for two rows and waits for them after every eight products (delta rule 198 -> 189 us, decayed sum 165 -> 155; the gated
 // form, bound by its producers, gains nothing)
@@ -193,24 +215,29 @@ __global__ __launch_bounds__(512) void chunk_head_kernel(ChunkScanArgs a) {
       const float* M = A + C * RA;
       const f32x4 pre = *reinterpret_cast<const f32x4*>(M + C * RA + 4 * g), suf = *reinterpret_cast<const f32x4*>(M + C * RA + C + 4 * g);
       const float total = M[C * RA + C - 1];
-      f32x4 w;
+      f32x4 x, w;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) w[e] = vs[(4 * g + e) * VS + 16 * cw + m];
+      for (int e = 0; e < 4; ++e) x[e] = vs[(4 * g + e) * VS + 16 * cw + m];
       if constexpr (DELTA) {
         const f32x4 y = st.times(k), b = *reinterpret_cast<const f32x4*>(sc + 2 * C + 4 * g);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) w[e] = b[e] * (w[e] - pre[e] * y[e]);
-        w = times_rows(M, m, g, w);
+        for (int e = 0; e < 4; ++e) x[e] = b[e] * (x[e] - pre[e] * y[e]);
+        w = times_rows(M, m, g, x);
       } else {
         const f32x4 s = *reinterpret_cast<const f32x4*>(sc + C + 4 * g);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) w[e] *= s[e];
+        for (int e = 0; e < 4; ++e) w[e] = x[e] * s[e];
       }
-      f32x4 o = st.times(q);
-      const f32x4 within = times_rows(A, m, g, w);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = __builtin_fmaf(o[e], pre[e], within[e]);
+      const f32x4 before = st.times(q);
+      f32x4 within = times_rows(A, m, g, w);
       products_behind_reads<14, 20, 3, 12>();
+      if (some_not_finite(w)) {                            // (of x: then every row of w)
+        if constexpr (DELTA) w = times_rows_in_order(M, m, g, x);
+        within = times_rows_in_order(A, m, g, w);
+      }
+      f32x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = __builtin_fmaf(before[e], pre[e], within[e]);
       const int n = rows_of(c);
       const int64_t t0 = t_begin + (int64_t)c * C;
 #pragma unroll
@@ -437,8 +464,11 @@ __global__ __launch_bounds__(768) void chunk_channel_kernel(ChunkScanArgs a) {
       f32x4 w;
 #pragma unroll
       for (int e = 0; e < 4; ++e) w[e] = vs[e * VS];
-      const f32x4 o = st.times(p + m * RS + 4 * g) + times_rows(A, m, g, w);
+      const f32x4 before = st.times(p + m * RS + 4 * g);
+      f32x4 within = times_rows(A, m, g, w);
       if constexpr (!GATED) products_behind_reads<10, 4, 4, 20>();
+      if (some_not_finite(w)) within = times_rows_in_order(A, m, g, w);
+      const f32x4 o = before + within;
       const int n = rows_of(c);
       const int64_t t0 = t_begin + (int64_t)c * C;
 #pragma unroll

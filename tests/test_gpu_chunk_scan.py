@@ -99,6 +99,67 @@ def _through_a_scan(lens, K, V, form, per_channel, types, pad):
     assert torch.equal(st[other], before[other]) and torch.equal(st[:, 0, :pad], before[:, 0, :pad])
 
 
+# What is not a finite number in a token's operands shows from that token on, in its columns, and nowhere before: the tokens are a chunk's
+# last, one in its middle and one behind it.
+@pytest.mark.parametrize("K, V", [(64, 64), (128, 128), (12, 20)])
+@pytest.mark.parametrize("form, per_channel", [("decay", False), ("decay", True), ("delta", False), ("bonus", True)])
+@pytest.mark.parametrize("what, value", [("v", float("inf")), ("v", float("nan")), ("k", float("nan")), ("scalar", float("nan"))])
+def test_not_finite_numbers_reach_later_tokens_only(K, V, form, per_channel, what, value):
+    from hydrainfer_amd._C.kernel.seq_mix import state_scan
+    from hydrainfer_amd._C.kernel.stream_ops import SequenceState
+    g = torch.Generator().manual_seed(K + V)
+    lens, bad, H = [40, 16, 23], [25, 55, 58], 2
+    n, T = len(lens), sum(lens)
+    unit = lambda x: torch.nn.functional.normalize(x, dim=-1).reshape(T, H * K)
+    q, k, v = unit(torch.randn((T, H, K), generator=g)), unit(torch.randn((T, H, K), generator=g)), torch.randn((T, H * V), generator=g)
+    decay = 0.5 + 0.5 * torch.rand((T, H * K if per_channel else H), generator=g)
+    vscale, beta, bonus = torch.rand((T, H), generator=g), torch.rand((T, H), generator=g), torch.randn(H * K, generator=g)
+    for t in bad:
+        if what == "v":
+            v[t, V + 3] = value
+        elif what == "k":
+            k[t, K + 5] = value
+        else:
+            vscale[t, 1] = beta[t, 1] = value
+    cu = [0, 40, 56, 79]
+    state = torch.randn((n, 1, H * K * V), generator=g)
+    h = lambda x, m: x.double().view(T, H, m)
+    want, S = _scan(form, h(q, K), h(k, K), h(v, V), decay.double().view(T, H, -1).expand(T, H, K),
+                    vscale.double() if form == "decay" else torch.ones((T, H), dtype=torch.float64), beta.double(), bonus.double().view(H, K),
+                    state.double().view(n, H, K, V), cu, [True, False, False])
+    d = lambda x: x.cuda()
+    pos = torch.tensor([(0 if s == 0 else 9) + i for s in range(n) for i in range(lens[s])], dtype=torch.int32)
+    st = d(state)
+    seq = SequenceState(st, torch.arange(n, dtype=torch.int32, device="cuda"), d(torch.tensor([s for s in range(n) for _ in range(lens[s])], dtype=torch.int32)))
+    got = state_scan(form, d(q), d(k), d(v), d(decay), seq, 0, d(torch.tensor(cu, dtype=torch.int32)), d(pos), H, H, K, V,
+                     vscale=d(vscale) if form == "decay" else None, beta=d(beta) if form == "delta" else None, bonus=d(bonus) if form == "bonus" else None)
+    for got, want in ((got.double().cpu(), want.reshape(T, H * V)), (st.double().cpu().view(n, H, K, V), S)):
+        fine = torch.isfinite(want)
+        assert torch.equal(torch.isfinite(got), fine)
+        _check("finite", got[fine], want[fine])
+
+
+@pytest.mark.parametrize("what", ["v", "k"])
+def test_not_finite_numbers_in_the_gated_recurrence(what):
+    from hydrainfer_amd._C.kernel.recurrence import gated_recurrence
+    from hydrainfer_amd._C.kernel.stream_ops import SequenceState
+    g = torch.Generator().manual_seed(5)
+    T, H, K, V, bad = 37, 2, 128, 64, 30
+    proj = torch.randn((T, H * (2 * K + V)), generator=g)
+    f_bias, low, norm_w = torch.randn(H * K, generator=g), torch.rand(H * K, generator=g), 1 + 0.1 * torch.randn(V, generator=g)
+
+    def run(p):
+        seq = SequenceState(torch.zeros((1, 1, H * K * V), device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda"), torch.zeros(T, dtype=torch.int32, device="cuda"))
+        p = p.cuda()
+        return gated_recurrence(p[:, :H * K], p[:, H * K:2 * H * K], p[:, 2 * H * K:], f_bias.cuda(), low.cuda(), norm_w.cuda(), 1e-5, seq, 0,
+                                torch.tensor([0, T], dtype=torch.int32).cuda(), torch.arange(T, dtype=torch.int32).cuda(), H, K, V, max_q_len=T).cpu()
+    clean = run(proj)
+    proj[bad, H * K + K + 7 if what == "k" else 2 * H * K + V + 3] = float("nan")
+    got = run(proj)
+    assert torch.isfinite(got[:bad]).all() and torch.equal(got[:, :V], clean[:, :V]) and torch.isnan(got[bad:, V:]).all()
+    _check("before", got[:bad], clean[:bad].double(), 2 * TOL)
+
+
 @pytest.mark.parametrize("lens", LENS)
 @pytest.mark.parametrize("K, V", [(64, 64), (128, 128), (12, 20), (100, 130), (65, 7)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
