@@ -706,7 +706,7 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) qf[ks] ^= (u16)0x8000;
     }
-    scale2 = fmaxf(fabsf(scale2), 1e-30f);
+    scale2 = fabsf(scale2) < 1e-30f ? 1e-30f : fabsf(scale2);      // (not fmaxf: what is not a number stays so)
   }
 
   f32x16 acc[NDB];
@@ -990,7 +990,7 @@ __global__ __launch_bounds__(64) void biased_attn_step_kernel(hxm_biased_attn_ar
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) qf[ks] ^= (u16)0x8000;
     }
-    scale2 = fmaxf(fabsf(scale2), 1e-30f);
+    scale2 = fabsf(scale2) < 1e-30f ? 1e-30f : fabsf(scale2);      // (not fmaxf: what is not a number stays so)
   }
   f32x4 acc[NDB];
 #pragma unroll

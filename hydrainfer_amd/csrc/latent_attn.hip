@@ -866,7 +866,7 @@ __global__ __launch_bounds__(256, KK <= 4 ? 2 : 1) void latent_attn_wide_kernel(
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) qf[ks] ^= (u16)0x8000;
   }
-  scale2 = fmaxf(fabsf(scale2), 1e-30f);
+  scale2 = fabsf(scale2) < 1e-30f ? 1e-30f : fabsf(scale2);      // (not fmaxf: what is not a number stays so)
 
   f32x16 acc[NDB];
 #pragma unroll
@@ -1095,7 +1095,7 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) qf[ks] ^= (u16)0x8000;
   }
-  scale2 = fmaxf(fabsf(scale2), 1e-30f);
+  scale2 = fabsf(scale2) < 1e-30f ? 1e-30f : fabsf(scale2);      // (not fmaxf: what is not a number stays so)
   const float lag = n_splits > 1 ? 0.f : 8.0f;
   f32x4 acc[NDB];
 #pragma unroll

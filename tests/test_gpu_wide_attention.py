@@ -97,3 +97,21 @@ def check(new, kv, H, G, D, V, mask, size, extra, divided=True):
                                  None if sinks is None else sinks.double())
         off = (got[lo:hi] - want).abs()
         assert bool((off <= bound).all()), (s, float((off - bound).max()))
+
+
+@pytest.mark.parametrize("new, kv", [([40, 16], [40, 300]), ([1, 1], [40, 300])])
+@pytest.mark.parametrize("divided", [True, False])
+def test_a_temperature_that_is_no_number_shows(new, kv, divided):
+    from hydrainfer_amd._C.kernel.biased_attn import biased_attention
+    H, G, D = 8, 2, 64
+    g = torch.Generator().manual_seed(sum(new))
+    r = lambda *s: torch.randn(s, generator=g).bfloat16().cuda()
+    i = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    nb = [(n + BLOCK - 1) // BLOCK for n in kv]
+    pos = [p for a, b in zip(new, kv) for p in range(b - a, b)]
+    temps = torch.rand(H, generator=g) + 0.5
+    temps[3] = math.nan
+    out = biased_attention(r(sum(new), H, D), r(sum(nb), BLOCK, G, D), r(sum(nb), BLOCK, G, D), D, i([s for s, a in enumerate(new) for _ in range(a)]), i(pos),
+                           i([0, new[0], sum(new)]), i(list(range(sum(nb)))), i([0, nb[0], sum(nb)]), D ** -0.5, None, "causal", 0, max_q_len=max(new),
+                           max_kv_len=max(kv) if divided else 0, head_scale=temps.cuda()).view(-1, H, D)
+    assert torch.isnan(out[:, 3]).all() and torch.isfinite(out[:, [h for h in range(H) if h != 3]]).all()

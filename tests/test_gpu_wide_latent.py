@@ -71,3 +71,14 @@ def check(new, kv, R, H, window, extra):
         bound = 2.0 ** -8 * want.abs() + (2.0 ** -8 + 1e-6) * size + 1e-6
         off = (got[:, lo:hi] - want).abs()
         assert bool((off <= bound).all()), (s, float((off - bound).max()))
+
+
+@pytest.mark.parametrize("R, tokens", [(64, 1100), (512, 30), (512, 1)])
+def test_a_scale_that_is_no_number_shows(R, tokens):
+    from hydrainfer_amd._C.kernel.latent_attn import latent_attention
+    H, nb = 32, (tokens + 200 + BLOCK - 1) // BLOCK
+    g = torch.Generator().manual_seed(R)
+    i = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    out = latent_attention(torch.randn((tokens, H, R), generator=g).bfloat16().cuda(), torch.randn((nb, BLOCK, 1, R), generator=g).bfloat16().cuda(), i([0] * tokens),
+                           i(list(range(200, 200 + tokens))), i([0, tokens]), i(list(range(nb))), i([0, nb]), math.nan, None, tokens, max_kv_len=200 + tokens)
+    assert torch.isnan(out).all()
