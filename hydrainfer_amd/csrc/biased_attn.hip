@@ -658,11 +658,12 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
   c_i32* table = (c_i32*)(a.block_table + ((c_i32*)a.cu_block_lens)[b]);
   const int bs = a.block_size, bshift = (bs & (bs - 1)) == 0 ? __ffs(bs) - 1 : -1;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem_w;
-  // Wave w brings keys 16 w .. of a tile (one page): RPK / RPV rows an instruction, LK / LV lanes a row.
+  // Wave w brings keys 16 w .. of a tile (one page): RPK / RPV rows an instruction, LK / LV lanes a row.  What lies in front of the
+  // first key that some row sees, or behind the last, is not touched (its page may be gone): rows there repeat that key, masked.
   constexpr int RPK = 64 / LK, RPV = 64 / LV;
   const int rk = lane / LK, ck = lane % LK, rv = lane / LV, cv = lane % LV;
   auto bring = [&](int t, int img) __attribute__((always_inline)) {
-    const int key0 = min(t * KT + 16 * wave, k_last), r_max = k_last - key0;      // (rows past the last key repeat it; masked)
+    const int key0 = min(max(t * KT + 16 * wave, k_first & ~15), k_last), r_min = k_first - key0, r_max = k_last - key0;
     const int page = bshift >= 0 ? key0 >> bshift : key0 / bs;
     const int64_t off = (int64_t)table[page] * a.cache_block_stride + (int64_t)(key0 - page * bs) * a.cache_row_stride;
     const uint32_t kd = lds0 + (uint32_t)(img * IMG + 16 * wave * RSK), vd = lds0 + (uint32_t)(img * IMG + KTILE + 16 * wave * RSV);
@@ -672,13 +673,13 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
 #pragma unroll
     for (int j = 0; j < 16 / RPK; ++j) {
       const int rr = RPK * j + rk;
-      const u16* from = kc + off + (int64_t)min(rr, r_max) * a.cache_row_stride + 8 * (ck ^ kswz(rr));
+      const u16* from = kc + off + (int64_t)max(min(rr, r_max), r_min) * a.cache_row_stride + 8 * (ck ^ kswz(rr));
       asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(__builtin_amdgcn_readfirstlane(kd + 1024u * j)) : "memory", "m0");
     }
 #pragma unroll
     for (int j = 0; j < 16 / RPV; ++j) {
       const int rr = RPV * j + rv;
-      const u16* from = vc + off + (int64_t)min(rr, r_max) * a.cache_row_stride + 8 * (cv ^ vswz(rr));
+      const u16* from = vc + off + (int64_t)max(min(rr, r_max), r_min) * a.cache_row_stride + 8 * (cv ^ vswz(rr));
       asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(__builtin_amdgcn_readfirstlane(vd + 1024u * j)) : "memory", "m0");
     }
 #pragma clang diagnostic pop
@@ -940,8 +941,12 @@ __global__ __launch_bounds__(64) void biased_attn_step_kernel(hxm_biased_attn_ar
   const int32_t* table = a.block_table + ((c_i32*)a.cu_block_lens)[b];
   const int bs = a.block_size, bshift = (bs & (bs - 1)) == 0 ? __ffs(bs) - 1 : -1;
   auto page_of = [&](int key) { return bshift >= 0 ? key >> bshift : key / bs; };
+  // The key that a group of 16 is brought from on.  What lies in front of the first key that some row sees, or behind the last, is not
+  // touched (its page may be gone): rows there repeat that key, masked.
+  const int k_from = k_first & ~15;
+  auto group_key = [&](int group) { return min(max(16 * group, k_from), k_last); };
   // lane i: the page of the i-th group of 16 keys from group pages0 on
-  int pages0 = 2 * t_first, pages = table[page_of(min(16 * (pages0 + lane), k_last))];
+  int pages0 = 2 * t_first, pages = table[page_of(group_key(pages0 + lane))];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[ks]));
   asm volatile("" : "+v"(pages), "+v"(hsc), "+v"(slope2), "+v"(sink2));      // (all there before the transfers start: a wait for them would be one for those)
@@ -952,7 +957,7 @@ __global__ __launch_bounds__(64) void biased_attn_step_kernel(hxm_biased_attn_ar
   auto bring = [&](int t, int img) __attribute__((always_inline)) {
     if (2 * t + 1 - pages0 > 63) {
       pages0 = 2 * t;
-      pages = table[page_of(min(16 * (pages0 + lane), k_last))];
+      pages = table[page_of(group_key(pages0 + lane))];
       asm volatile("" : "+v"(pages));        // (waited for here: after the branch it would be a wait in every tile)
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (the reads of the image that this replaces are done)
@@ -961,20 +966,20 @@ __global__ __launch_bounds__(64) void biased_attn_step_kernel(hxm_biased_attn_ar
     // (m0, the LDS address of the transfer, is a reserved register: nothing else in this kernel uses it)
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const int key0 = min(t * KT + 16 * u, k_last), r_max = k_last - key0;      // (rows past the last key repeat it; masked)
+      const int key0 = group_key(2 * t + u), r_min = k_first - key0, r_max = k_last - key0;
       const int64_t off = (int64_t)__builtin_amdgcn_readlane(pages, 2 * t + u - pages0) * a.cache_block_stride +
                           (int64_t)(key0 - page_of(key0) * bs) * a.cache_row_stride;
       const uint32_t kd = lds0 + (uint32_t)(img * IMG + 16 * u * RSK), vd = lds0 + (uint32_t)(img * IMG + KTILE + 16 * u * RSV);
 #pragma unroll
       for (int j = 0; j < NLK; ++j) {
         const int rr = (64 * j + lane) / LK, ch = (64 * j + lane) % LK;
-        const uint32_t from = (uint32_t)min(rr, r_max) * row_bytes + 16u * (uint32_t)(ch ^ swz(rr, D == 128));
+        const uint32_t from = (uint32_t)max(min(rr, r_max), r_min) * row_bytes + 16u * (uint32_t)(ch ^ swz(rr, D == 128));
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(from), "s"(kc + off), "s"(__builtin_amdgcn_readfirstlane(kd + 1024u * j)) : "memory", "m0");
       }
 #pragma unroll
       for (int j = 0; j < NLV; ++j) {
         const int rr = (64 * j + lane) / LV, ch = (64 * j + lane) % LV;
-        const uint32_t from = (uint32_t)min(rr, r_max) * row_bytes + 16u * (uint32_t)(ch ^ swz(rr, V == 128));
+        const uint32_t from = (uint32_t)max(min(rr, r_max), r_min) * row_bytes + 16u * (uint32_t)(ch ^ swz(rr, V == 128));
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(from), "s"(vc + off), "s"(__builtin_amdgcn_readfirstlane(vd + 1024u * j)) : "memory", "m0");
       }
     }

@@ -830,10 +830,11 @@ __global__ __launch_bounds__(256, KK <= 4 ? 2 : 1) void latent_attn_wide_kernel(
   c_i32* table = (c_i32*)(a.block_table + ((c_i32*)a.cu_block_lens)[b]);
   const int bs = a.block_size, bshift = (bs & (bs - 1)) == 0 ? __ffs(bs) - 1 : -1;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem_w;
-  // Wave w brings keys 16 w .. of a tile (one page): 16 L chunks, 64 an instruction.
+  // Wave w brings keys 16 w .. of a tile (one page): 16 L chunks, 64 an instruction.  What lies in front of the first key that some row
+  // sees, or behind the last, is not touched (its page may be gone): rows there repeat that key, masked.
   constexpr int NL = 16 * L / 64;
   auto bring = [&](int t, int img) __attribute__((always_inline)) {
-    const int key0 = min(t * KT + 16 * wave, k_last), r_max = k_last - key0;      // (rows past the last key repeat it; masked)
+    const int key0 = min(max(t * KT + 16 * wave, k_first & ~15), k_last), r_min = k_first - key0, r_max = k_last - key0;
     const int page = bshift >= 0 ? key0 >> bshift : key0 / bs;
     const u16* base = cache + (int64_t)table[page] * a.cache_block_stride + (int64_t)(key0 - page * bs) * a.cache_row_stride;
     const uint32_t to = lds0 + (uint32_t)(img * IMG + 16 * wave * RS);
@@ -845,7 +846,7 @@ __global__ __launch_bounds__(256, KK <= 4 ? 2 : 1) void latent_attn_wide_kernel(
 #pragma unroll
     for (int j = 0; j < NL; ++j) {
       const int rr = (64 * j + ln) / L, ch = (64 * j + ln) % L;
-      const uint32_t off = (uint32_t)min(rr, r_max) * (uint32_t)(2 * a.cache_row_stride) + 16u * (uint32_t)(ch ^ swz(rr));
+      const uint32_t off = (uint32_t)max(min(rr, r_max), r_min) * (uint32_t)(2 * a.cache_row_stride) + 16u * (uint32_t)(ch ^ swz(rr));
       asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(__builtin_amdgcn_readfirstlane(to + 1024u * j)) : "memory", "m0");
     }
 #pragma clang diagnostic pop
@@ -1059,10 +1060,10 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
   c_i32* table = (c_i32*)(a.block_table + ((c_i32*)a.cu_block_lens)[b]);
   const int bs = a.block_size, bshift = (bs & (bs - 1)) == 0 ? __ffs(bs) - 1 : -1;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem_w;
-  // Wave w brings keys 8 w .. of a tile (one page): 8 L chunks, 64 an instruction.
+  // Wave w brings keys 8 w .. of a tile (one page): 8 L chunks, 64 an instruction; none in front of the first or behind the last, as above.
   constexpr int NL = KPW * L / 64;
   auto bring = [&](int t, int img) __attribute__((always_inline)) {
-    const int key0 = min(t * KT + KPW * wave, k_last), r_max = k_last - key0;       // (rows past the last key repeat it; masked)
+    const int key0 = min(max(t * KT + KPW * wave, k_first & ~(KPW - 1)), k_last), r_min = k_first - key0, r_max = k_last - key0;
     const int page = bshift >= 0 ? key0 >> bshift : key0 / bs;
     const u16* base = cache + (int64_t)table[page] * a.cache_block_stride + (int64_t)(key0 - page * bs) * a.cache_row_stride;
     const uint32_t to = lds0 + (uint32_t)(img * IMG + KPW * wave * RS);
@@ -1074,7 +1075,7 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
 #pragma unroll
     for (int j = 0; j < NL; ++j) {
       const int rr = (64 * j + ln) / L, ch = (64 * j + ln) % L;
-      const uint32_t off = (uint32_t)min(rr, r_max) * (uint32_t)(2 * a.cache_row_stride) + 16u * (uint32_t)(ch ^ swz(KPW * wave + rr));
+      const uint32_t off = (uint32_t)max(min(rr, r_max), r_min) * (uint32_t)(2 * a.cache_row_stride) + 16u * (uint32_t)(ch ^ swz(KPW * wave + rr));
       asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(__builtin_amdgcn_readfirstlane(to + 1024u * j)) : "memory", "m0");
     }
 #pragma clang diagnostic pop

@@ -64,11 +64,32 @@ def test_step_form(batch, H, G, D, V, mask, size, extra, divided):
     check([a for a, _ in batch], [b for _, b in batch], H, G, D, V, mask, size, extra, divided)
 
 
-def check(new, kv, H, G, D, V, mask, size, extra, divided=True):
+# Rows that no token of a portion sees are never read: pages left of a window or chunk may have been given back, and the rows of the last
+# page behind the last token hold anything.
+@pytest.mark.parametrize("batch", [[(64, 700), (33, 1100)], [(129, 333)], [(1, 700), (3, 1101), (1, 40)], [(16, 2005)]], ids=lambda b: f"{len(b)}x{max(b)}")
+@pytest.mark.parametrize("H, G, D, V", [(6, 2, 128, 64), (8, 8, 64, 128)])
+@pytest.mark.parametrize("mask, size", [("window", 300), ("chunk", 500), ("causal", 0)])
+@pytest.mark.parametrize("divided", [True, False])
+def test_rows_that_nobody_sees(batch, H, G, D, V, mask, size, divided):
+    check([a for a, _ in batch], [b for _, b in batch], H, G, D, V, mask, size, "plain", divided, unseen=True)
+
+
+def hide(cache, table, first, last):
+    """What lies outside of keys first .. last of a sequence becomes NaN; its pages there the last block of the cache, all NaN."""
+    cache[-1] = math.nan
+    for i, page in enumerate(table.tolist()):
+        keys = torch.arange(i * BLOCK, (i + 1) * BLOCK)
+        if i < first // BLOCK or i > last // BLOCK:
+            table[i] = cache.shape[0] - 1
+        else:
+            cache[page, (keys < first) | (keys > last)] = math.nan
+
+
+def check(new, kv, H, G, D, V, mask, size, extra, divided=True, unseen=False):
     from hydrainfer_amd._C.kernel.biased_attn import biased_attention
     g = torch.Generator().manual_seed(H * D + V + size + sum(new) + sum(kv))
     nb = [(n + BLOCK - 1) // BLOCK for n in kv]
-    perm = torch.randperm(sum(nb) + 1, generator=g)
+    perm = torch.randperm(sum(nb) + (0 if unseen else 1), generator=g)
     r = lambda *s: torch.randn(s, generator=g).bfloat16()
     hs = max(D, V)
     T, kc, vc = sum(new), r(sum(nb) + 1, BLOCK, G, hs), r(sum(nb) + 1, BLOCK, G, hs)
@@ -86,7 +107,13 @@ def check(new, kv, H, G, D, V, mask, size, extra, divided=True):
     seq = torch.tensor([s for s, a in enumerate(new) for _ in range(a)], dtype=torch.int32)
     table = perm[:sum(nb)].int()
     c = lambda t: None if t is None else t.cuda()
-    got = biased_attention(c(q), c(kc), c(vc), V, c(seq), c(torch.tensor(pos, dtype=torch.int32)), c(cu_q), c(table), c(cu_b), D ** -0.5, c(slopes), mask,
+    kg, vg, pages = kc.clone(), vc.clone(), table.clone()
+    if unseen:
+        for s in range(len(new)):
+            own, rows = slice(int(cu_b[s]), int(cu_b[s + 1])), pos[int(cu_q[s]):int(cu_q[s + 1])]
+            for x, t in ((kg, table[own].clone()), (vg, pages[own])):
+                hide(x, t, min(_first(mask, size, p) for p in rows), max(rows))
+    got = biased_attention(c(q), c(kg), c(vg), V, c(seq), c(torch.tensor(pos, dtype=torch.int32)), c(cu_q), c(pages), c(cu_b), D ** -0.5, c(slopes), mask,
                            size, max_q_len=max(new), max_kv_len=max(kv) if divided else 0, softcap=cap, head_scale=c(temps), sinks=c(sinks)).double().cpu()
     for s in range(len(new)):
         lo, hi = int(cu_q[s]), int(cu_q[s + 1])

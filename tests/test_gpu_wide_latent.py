@@ -35,11 +35,31 @@ def test_single_tokens(kv, R, H, window, extra):
     check([1] * len(kv), kv, R, H, window, extra)
 
 
-def check(new, kv, R, H, window, extra):
+# Rows that no token of a portion sees are never read: pages left of a window may have been given back, and the rows of the last page
+# behind the last token hold anything.
+@pytest.mark.parametrize("new, kv", [([1, 3, 1], [700, 1101, 40]), ([33, 20], [700, 90]), ([300, 41, 761], [700, 2005, 800])])
+@pytest.mark.parametrize("R", [64, 320, 512])
+@pytest.mark.parametrize("window", [300, 0])
+def test_rows_that_nobody_sees(new, kv, R, window):
+    check(new, kv, R, 32, window, "plain", unseen=True)
+
+
+def hide(cache, table, first, last):
+    """What lies outside of keys first .. last of a sequence becomes NaN; its pages there the last block of the cache, all NaN."""
+    cache[-1] = math.nan
+    for i, page in enumerate(table.tolist()):
+        keys = torch.arange(i * BLOCK, (i + 1) * BLOCK)
+        if i < first // BLOCK or i > last // BLOCK:
+            table[i] = cache.shape[0] - 1
+        else:
+            cache[page, (keys < first) | (keys > last)] = math.nan
+
+
+def check(new, kv, R, H, window, extra, unseen=False):
     from hydrainfer_amd._C.kernel.latent_attn import latent_attention
     g = torch.Generator().manual_seed(R * 100 + H + window + sum(new) + sum(kv))
     nb = [(n + BLOCK - 1) // BLOCK for n in kv]
-    T, perm = sum(new), torch.randperm(sum(nb) + 1, generator=g)
+    T, perm = sum(new), torch.randperm(sum(nb) + (0 if unseen else 1), generator=g)
     cache = torch.randn((sum(nb) + 1, BLOCK, 1, R + 8), generator=g).bfloat16()      # rows wider than the latent
     q = torch.randn((H, T, R), generator=g).bfloat16()
     q[0, 0] *= 20                 # a row whose weights sit on one key
@@ -51,8 +71,13 @@ def check(new, kv, R, H, window, extra):
     seq = torch.tensor([s for s, a in enumerate(new) for _ in range(a)], dtype=torch.int32)
     table = perm[:sum(nb)].int()
     c = lambda t: None if t is None else t.cuda()
+    shown, pages = cache.clone(), table.clone()
+    if unseen:
+        for s in range(len(new)):
+            rows = pos[int(cu_q[s]):int(cu_q[s + 1])]
+            hide(shown, pages[int(cu_b[s]):int(cu_b[s + 1])], max(0, min(rows) - window + 1) if window else 0, max(rows))
     out = torch.full((H, T, R), 7.0, dtype=torch.bfloat16, device="cuda")
-    latent_attention(c(q).transpose(0, 1), c(cache), c(seq), c(torch.tensor(pos, dtype=torch.int32)), c(cu_q), c(table), c(cu_b), scale, window or None,
+    latent_attention(c(q).transpose(0, 1), c(shown), c(seq), c(torch.tensor(pos, dtype=torch.int32)), c(cu_q), c(pages), c(cu_b), scale, window or None,
                      max(new), gate_pre=c(gate), out=out.transpose(0, 1), max_kv_len=max(kv), sinks=c(sinks))
     got = out.double().cpu()
     for s in range(len(new)):
