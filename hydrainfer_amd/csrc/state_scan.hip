@@ -491,6 +491,7 @@ extern "C" int hxm_state_scan(const hxm_state_scan_args* args, void* stream) {
     if (d != HX_F32 && d != HX_BF16) return HX_ERR_DTYPE;
   if (a.q_stride < (int64_t)a.qk_heads * a.dim || a.k_stride < (int64_t)a.qk_heads * a.dim || a.v_stride < (int64_t)a.heads * a.vdim)
     return HX_ERR_STRIDE;
+  if (a.mode != HXM_SCAN_DECAY && a.mode != HXM_SCAN_BONUS && a.mode != HXM_SCAN_DELTA) return HX_ERR_UNSUPPORTED;
   hipStream_t s = (hipStream_t)stream;
   // Portions of prompts go sixteen tokens at a time (chunk_scan.hip) where the sizes allow it, short ones one at a time here: a
   // chunk costs its sixteen however few tokens it holds.  Measured with 32 heads of 128 x 128 under the delta rule: 32 portions of
