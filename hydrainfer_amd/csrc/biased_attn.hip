@@ -651,7 +651,7 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
     k_last = wave_max_int(max(p0, p1));
   }
   const bool live = row0 + 31 >= 0;
-  const int t_first = k_first / KT, t_last = k_last / KT;
+  const int t_first = k_first / KT, t_last = k_last < 0 ? t_first - 1 : k_last / KT;      // (positions below 0 see nothing)
 
   const u16* kc = (const u16*)a.key_cache + (int64_t)kvh * a.head_stride;
   const u16* vc = (const u16*)a.value_cache + (int64_t)kvh * a.head_stride;
@@ -684,7 +684,7 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
     }
 #pragma clang diagnostic pop
   };
-  bring(t_first, 0);
+  if (t_first <= t_last) bring(t_first, 0);
   // the queries (B operand): row c, columns 16 ks + 8 hi ..
   u16x8 qf[KS];
   {
@@ -922,7 +922,7 @@ __global__ __launch_bounds__(64) void biased_attn_step_kernel(hxm_biased_attn_ar
   const int r = max(row0 + c, 0), tok = r / R, head = kvh * R + r % R;
   const int pos = a.positions[q0 + tok], lo = first_visible(pos, a.mask_kind, a.mask_size);
   const int pos_min = wave_min_int(pos), k_last = wave_max_int(pos), k_first = wave_min_int(lo), lo_max = wave_max_int(lo);
-  int t_first = k_first / KT, t_last = k_last / KT;
+  int t_first = k_first / KT, t_last = k_last < 0 ? t_first - 1 : k_last / KT;      // (positions below 0 see nothing)
   if (n_splits > 1) {                        // this split's run of tiles (the last splits may get none)
     const int per = (t_last - t_first + n_splits) / n_splits;
     t_first += split * per;
@@ -946,7 +946,7 @@ __global__ __launch_bounds__(64) void biased_attn_step_kernel(hxm_biased_attn_ar
   const int k_from = k_first & ~15;
   auto group_key = [&](int group) { return min(max(16 * group, k_from), k_last); };
   // lane i: the page of the i-th group of 16 keys from group pages0 on
-  int pages0 = 2 * t_first, pages = table[page_of(group_key(pages0 + lane))];
+  int pages0 = 2 * t_first, pages = k_last < 0 ? 0 : table[page_of(group_key(pages0 + lane))];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[ks]));
   asm volatile("" : "+v"(pages), "+v"(hsc), "+v"(slope2), "+v"(sink2));      // (all there before the transfers start: a wait for them would be one for those)

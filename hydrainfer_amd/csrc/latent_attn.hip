@@ -824,7 +824,7 @@ __global__ __launch_bounds__(256, KK <= 4 ? 2 : 1) void latent_attn_wide_kernel(
     k_last = wave_max_int(max(p0, p1));
   }
   const bool live = row0 + 31 >= 0;
-  const int t_first = k_first / KT, t_last = k_last / KT;
+  const int t_first = k_first / KT, t_last = k_last < 0 ? t_first - 1 : k_last / KT;      // (positions below 0 see nothing)
 
   const u16* cache = (const u16*)a.cache;
   c_i32* table = (c_i32*)(a.block_table + ((c_i32*)a.cu_block_lens)[b]);
@@ -851,7 +851,7 @@ __global__ __launch_bounds__(256, KK <= 4 ? 2 : 1) void latent_attn_wide_kernel(
     }
 #pragma clang diagnostic pop
   };
-  bring(t_first, 0);
+  if (t_first <= t_last) bring(t_first, 0);
   u16x8 qf[KS];                              // the queries (B operand): row c, columns 16 ks + 8 hi ..
   {
     const u16* qg = (const u16*)a.q + (int64_t)(q0 + tok) * a.q_token_stride + (int64_t)head * a.q_head_stride + 8 * hi;
@@ -1049,7 +1049,7 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
   const int p_wg = a.positions[q0 + max(row0_wg + lane, 0) / H];
   const int k_first = wave_min_int(first_key(p_wg)), k_last = wave_max_int(p_wg);
   const bool live = row0 + 15 >= 0;
-  int t_first = k_first / KT, t_last = k_last / KT;
+  int t_first = k_first / KT, t_last = k_last < 0 ? t_first - 1 : k_last / KT;      // (positions below 0 see nothing)
   if (n_splits > 1) {                        // this split's run of tiles (the last splits may get none)
     const int per = (t_last - t_first + n_splits) / n_splits;
     t_first += split * per;

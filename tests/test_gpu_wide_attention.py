@@ -142,3 +142,23 @@ def test_a_temperature_that_is_no_number_shows(new, kv, divided):
                            i([0, new[0], sum(new)]), i(list(range(sum(nb)))), i([0, nb[0], sum(nb)]), D ** -0.5, None, "causal", 0, max_q_len=max(new),
                            max_kv_len=max(kv) if divided else 0, head_scale=temps.cuda()).view(-1, H, D)
     assert torch.isnan(out[:, 3]).all() and torch.isfinite(out[:, [h for h in range(H) if h != 3]]).all()
+
+
+@pytest.mark.parametrize("n", [1, 40])
+@pytest.mark.parametrize("divided", [True, False])
+def test_a_sequence_without_keys(n, divided):
+    # its tokens stand in front of its first key (position -1) and it has no pages: nothing is looked up for it
+    from hydrainfer_amd._C.kernel.biased_attn import biased_attention
+    H, G, D = 8, 2, 128
+    g = torch.Generator().manual_seed(n)
+    r = lambda *s: torch.randn(s, generator=g).bfloat16().cuda()
+    i = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    q, kc, vc = r(2 * n, H, D), r(30, BLOCK, G, D), r(30, BLOCK, G, D)
+    table, sinks = i(list(range(30))), torch.randn(H, generator=g).cuda()
+    run = lambda q, pos, q_cu, blocks, seq: biased_attention(q, kc, vc, D, i(seq), i(pos), i(q_cu), table, i(blocks), D ** -0.5, None, "causal", 0, max_q_len=n,
+                                                             max_kv_len=480 if divided else 0, sinks=sinks).view(-1, H, D)
+    own = list(range(480 - n, 480))
+    got = run(q, [-1] * n + own, [0, n, 2 * n], [0, 0, 30], [0] * n + [1] * n)
+    alone = run(q[n:].contiguous(), own, [0, n], [0, 30], [0] * n)
+    assert (got[:n] == 0).all()                                   # the sink takes all the weight
+    assert float((got[n:].double() - alone.double()).norm() / alone.double().norm()) < 2.0 ** -7      # (keys may be dealt out otherwise)

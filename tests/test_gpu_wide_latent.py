@@ -107,3 +107,20 @@ def test_a_scale_that_is_no_number_shows(R, tokens):
     out = latent_attention(torch.randn((tokens, H, R), generator=g).bfloat16().cuda(), torch.randn((nb, BLOCK, 1, R), generator=g).bfloat16().cuda(), i([0] * tokens),
                            i(list(range(200, 200 + tokens))), i([0, tokens]), i(list(range(nb))), i([0, nb]), math.nan, None, tokens, max_kv_len=200 + tokens)
     assert torch.isnan(out).all()
+
+
+@pytest.mark.parametrize("R, n", [(512, 1), (64, 1100)])
+def test_a_sequence_without_keys(R, n):
+    # its tokens stand in front of its first key (position -1) and it has no pages: nothing is looked up for it
+    from hydrainfer_amd._C.kernel.latent_attn import latent_attention
+    H, nb = 32, (n + 500) // BLOCK
+    g = torch.Generator().manual_seed(n)
+    i = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    q, cache = torch.randn((2 * n, H, R), generator=g).bfloat16().cuda(), torch.randn((nb, BLOCK, 1, R), generator=g).bfloat16().cuda()
+    table, sinks = i(list(range(nb))), torch.randn(H, generator=g).cuda()
+    run = lambda q, pos, q_cu, blocks, seq: latent_attention(q, cache, i(seq), i(pos), i(q_cu), table, i(blocks), R ** -0.5, None, n, max_kv_len=n + 400, sinks=sinks)
+    own = list(range(400, 400 + n))
+    got = run(q, [-1] * n + own, [0, n, 2 * n], [0, 0, nb], [0] * n + [1] * n)
+    alone = run(q[n:], own, [0, n], [0, nb], [0] * n)
+    assert (got[:n] == 0).all()                                   # the sink takes all the weight
+    assert float((got[n:].double() - alone.double()).norm() / alone.double().norm()) < 2.0 ** -7      # (keys may be dealt out otherwise)
