@@ -1200,7 +1200,7 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
   total += __shfl_xor(total, 32, 64);
   if (n_splits > 1) {
     // what this split adds to a row, not normalised: ws_o [sequence][row][split][R], ws_ml [..][split][maximum (log2), sum]
-    if (row0 + c >= 0) {
+    if (row0 + c >= 0 && row0 + c < tiles_per_seq * 16) {      // (rows past max_q_len tokens have no place)
       const size_t at = ((size_t)b * tiles_per_seq * 16 + (row0 + c)) * n_splits + split;
       float* wo = a.ws_o + at * R + 4 * g;
 #pragma unroll

@@ -124,3 +124,27 @@ def test_a_sequence_without_keys(R, n):
     alone = run(q[n:], own, [0, n], [0, nb], [0] * n)
     assert (got[:n] == 0).all()                                   # the sink takes all the weight
     assert float((got[n:].double() - alone.double()).norm() / alone.double().norm()) < 2.0 ** -7      # (keys may be dealt out otherwise)
+
+
+def test_rows_past_max_q_len_have_no_place_in_the_workspace():
+    import ctypes
+    from hydrainfer_amd import _lib
+    H, R, new, kv = 32, 512, 3, 1000
+    nb = (kv + BLOCK - 1) // BLOCK
+    g = torch.Generator().manual_seed(1)
+    i = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    q, cache = torch.randn((new, H, R), generator=g).bfloat16().cuda(), torch.randn((nb, BLOCK, 1, R), generator=g).bfloat16().cuda()
+    out = torch.empty_like(q)
+    ints = dict(tok_seq=i([0] * new), positions=i(list(range(kv - new, kv))), q_cu=i([0, new]), block_table=i(list(range(nb))), cu_block_lens=i([0, nb]))
+    a = _lib.hxm_latent_attn_args(out=out.data_ptr(), q=q.data_ptr(), cache=cache.data_ptr(), q_token_stride=H * R, q_head_stride=R, out_token_stride=H * R,
+                                  out_head_stride=R, cache_block_stride=BLOCK * R, cache_row_stride=R, block_size=BLOCK, n_tokens=new, n_seq=1, n_heads=H, kv_rank=R,
+                                  max_q_len=1, max_kv_len=kv, scale=R ** -0.5, dtype=_lib.dtype_code(q),
+                                  **{k: v.data_ptr() for k, v in ints.items()})
+    splits, floats = ctypes.c_int32(0), ctypes.c_int64(0)
+    _lib.mix_check(_lib.mix_lib().hxm_latent_attention_plan(ctypes.byref(a), ctypes.byref(splits), ctypes.byref(floats)), "plan")
+    assert splits.value > 1
+    n_o = floats.value // (R + 2) * R
+    ws_o, ws_ml = (torch.full((4 * n,), 7.0, device="cuda") for n in (n_o, floats.value - n_o))      # three tokens would fill three quarters
+    a.n_splits, a.ws_o, a.ws_ml = splits.value, ws_o.data_ptr(), ws_ml.data_ptr()
+    _lib.mix_check(_lib.mix_lib().hxm_latent_attention(ctypes.byref(a), _lib.current_stream()), "latent_attention")
+    assert (ws_o[n_o:] == 7.0).all() and (ws_ml[floats.value - n_o:] == 7.0).all()
