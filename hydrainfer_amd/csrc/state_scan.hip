@@ -513,9 +513,19 @@ extern "C" int hxm_state_scan(const hxm_state_scan_args* args, void* stream) {
     if (a.dim <= 128) return launch_step<8>(a, s);
     return launch_step<16>(a, s);
   }
-  // key channels a lane x lanes a column: 8 x 4, 8 x 8, 16 x 8, 16 x 16 (chunks of 16 tokens; 8 at the widest)
+  // key channels a lane x lanes a column: 8 x 4, 8 x 8, 16 x 8, 16 x 16 (chunks of 16 tokens; 8 at the widest).  Portions of
+  // prompts in a launch that would leave compute units without a workgroup take twice the lanes a column and half the key
+  // channels a lane: twice the waves, each with half the serial work per token (measured, the delta rule with a decay per channel:
+  // 4 portions of 1000 tokens, 4 heads of 128 x 128 368 -> 282 us, 32 of 64 x 64 253 -> 217; one of 5 tokens 8.5 -> 7.2.  With 512
+  // workgroups and 4 x 1024 tokens 394 -> 435 us; decode steps 26 -> 43 us: their state rows get too short).
+  static const int n_cu = [] {
+    int dev = 0, v = 0;
+    return hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0 ? v : 256;
+  }();
+  const bool prompt = a.n_tokens > a.n_seq;
+  auto few = [&](int cols) { return prompt && (int64_t)a.n_seq * a.heads * ((a.vdim + cols - 1) / cols) <= n_cu; };
   if (a.dim <= 32) return launch_rows<8, 4, 16>(a, s);
-  if (a.dim <= 64) return launch_rows<8, 8, 16>(a, s);
-  if (a.dim <= 128) return launch_rows<16, 8, 16>(a, s);
+  if (a.dim <= 64) return few(32) ? launch_rows<4, 16, 16>(a, s) : launch_rows<8, 8, 16>(a, s);
+  if (a.dim <= 128) return few(32) ? launch_rows<8, 16, 16>(a, s) : launch_rows<16, 8, 16>(a, s);
   return launch_rows<16, 16, 8>(a, s);
 }

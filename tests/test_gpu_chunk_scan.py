@@ -58,13 +58,22 @@ def test_single_tokens_through_a_scan(lens, K, V, form, per_channel, types, pad)
     _through_a_scan(lens, K, V, form, per_channel, types, pad)
 
 
+# portions that go a token at a time: short ones, and the forms and types that have no chunks; with few workgroups (more lanes a column)
+# and with many
+@pytest.mark.parametrize("lens", [[5], [3, 1, 2], [17, 33], [2] * 40], ids=lambda v: f"{len(v)}x{v[0]}")
+@pytest.mark.parametrize("K, V", [(64, 64), (128, 130), (40, 20), (100, 7)])
+@pytest.mark.parametrize("form, per_channel, types", [("delta", True, "mixed"), ("bonus", False, "f32"), ("decay", False, "odd"), ("delta", False, "odd")])
+def test_portions_a_token_at_a_time(lens, K, V, form, per_channel, types):
+    _through_a_scan(lens, K, V, form, per_channel, types, 3)
+
+
 def _through_a_scan(lens, K, V, form, per_channel, types, pad):
     from hydrainfer_amd._C.kernel.seq_mix import state_scan
     from hydrainfer_amd._C.kernel.stream_ops import SequenceState
     g = torch.Generator().manual_seed(sum(lens) * 1000 + K + V)
     n, T, H = len(lens), sum(lens), 4
     G = H if form == "bonus" else 2
-    qk_t, v_t = (torch.bfloat16 if types == "bf16" else torch.float32), (torch.float32 if types == "f32" else torch.bfloat16)
+    qk_t, v_t = (torch.bfloat16 if types in ("bf16", "odd") else torch.float32), (torch.float32 if types in ("f32", "odd") else torch.bfloat16)
     unit = lambda x: torch.nn.functional.normalize(x, dim=-1)
     proj = torch.cat([unit(torch.randn((T, G, K), generator=g)).reshape(T, G * K), unit(torch.randn((T, G, K), generator=g)).reshape(T, G * K),
                       torch.zeros((T, 1))], dim=1).to(qk_t)       # (an odd row length: views that do not start on multiples of four)
