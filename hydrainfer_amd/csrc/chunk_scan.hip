@@ -1,7 +1,6 @@
 // chunk_scan.hip — a recurrence with a matrix state S [K, V] per head and sequence over portions of prompts, sixteen tokens at a
-// time, all of it in float (v_mfma_f32_16x16x4_f32: nothing is rounded to a narrower type, so a chunk differs from sixteen
-// single steps by the order of float sums alone).  With S the state before the chunk and products of decays only — never a
-// quotient, so that decays that vanish give zeros and not 0 / 0:
+// time, all of it in float (v_mfma_f32_16x16x4_f32, an ascending chain of fused multiply-adds) or wider.  With S the state before the
+// chunk and products of decays only — never a quotient, so that decays that vanish give zeros and not 0 / 0:
 //     Y = (K * prefix) S                            delta rule: what the chunk's keys read from the old state
 //     W = M (b (V - Y)), M = (I + b (K K^T) L)^-1   delta rule (strictly lower part; M by substitution); else W = s V
 //     O = (Q * prefix) S + A W                      A[t, s] = sum_d q_t[d] k_s[d] prod(s < r <= t) a_r[d] for s <= t
@@ -20,9 +19,16 @@
 //                summed over the wave by a transposing butterfly that leaves one element of A in every second lane.
 // What bounds it now: the chunks of a sequence follow each other (2.5 us each with states of 128 x 128; 1.8 us of float matrix
 // products on the SIMDs that hold a consumer and a maker of A or M).  Measured against one token at a time, 4 portions of 797 -
-// 1151 tokens: delta rule, 32 heads of 128 x 128, 479 -> 189 us; decayed sum, 64 heads of 128 x 64, 432 -> 155 us; bonus form, 32
-// heads of 64 x 64, 207 -> 102 us; gated form, 32 heads of 128 x 128, 720 -> 213 us with its norm.  Error against 64 bits (2-norm): results 1.4e-7 / 1.0e-7 / 1.0e-7 (delta
-// / decay / bonus; 1.1e-7 / 1.1e-7 / 0.9e-7 before), states 1.0e-7 / 0.9e-7 / 0.7e-7 / 1.1e-7 (gated last; 0.8, 0.8, 0.5, 1.4).
+// 1151 tokens: delta rule, 32 heads of 128 x 128, 479 -> 189 us; decayed sum, 64 heads of 128 x 64, 432 -> 143 us; bonus form, 32
+// heads of 64 x 64, 207 -> 105 us; gated form, 32 heads of 128 x 128, 720 -> 201 us with its norm.
+// What the rounding costs: a token at a time rounds a state's element once a token, and each rounding decays with the state.  Here
+// the products of decays, of keys with them and the chunk's sums are rounded besides, and four things keep that from showing: sums
+// over tokens run from the first token to the last and on top of the decayed state (row_of_token); products of decays carry what
+// their roundings leave over (Product); sums over key channels are cut in eight or sixteen chains; and the bonus form, whose
+// k v is often exact, adds up within a chunk in double and keeps the rest of its suffixed keys.  Error against 64 bits (2-norm), a
+// token at a time and here, 3 portions of 200 - 600 tokens, 16 heads of 128 x 128 (64 x 64): results delta 1.07 1.07 (1.00 1.00),
+// decay 1.04 0.84 (0.97 0.77), bonus 0.90 0.82 (0.83 0.77) e-7; states delta 0.74 0.73 (0.75 0.74), decay 0.68 0.62 (0.72
+// 0.66), bonus 0.46 0.45 (0.47 0.45), gated 1.42 1.08 (1.41 1.07) e-7.
 #include <type_traits>
 #include "chunk_scan.h"
 #include "mix_rows.h"
@@ -37,11 +43,18 @@ namespace {
 using namespace hx;
 using hxm::ChunkScanArgs;
 
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 constexpr int C = 16;             // tokens a chunk
 constexpr int RA = C + 4;         // floats per row of a token by token matrix in LDS
 constexpr int VW = 64;            // value channels a workgroup
 constexpr int VS = VW + 4;        // floats per row of a chunk's values in LDS
 constexpr int kAhead = 3;         // chunks whose rows are on their way
+
+// Where token t of a chunk stands in LDS and in the accumulators: an instruction that sums over tokens takes rows e, 4 + e, 8 + e and
+// 12 + e, one a lane group, in this order, and they are tokens 4 e .. 4 e + 3 this way.  Sums over tokens thus grow from the first
+// to the last, as they do a token at a time: what has decayed is small when it is rounded.  (Its own inverse.)
+__device__ __forceinline__ constexpr int row_of_token(int t) { return (t & 3) << 2 | t >> 2; }
 
 __device__ __forceinline__ f32x4 mma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
@@ -76,6 +89,25 @@ __device__ __forceinline__ float sigmoid_gate(float x) {
   return __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
 }
 
+// A product of decays with what its roundings left over: the value is rounded once, however many factors it has.
+struct Product {
+  float hi = 1.f, lo = 0.f;
+  __device__ __forceinline__ void by(float f) {
+    const float p = hi * f;
+    lo = __builtin_fmaf(lo, f, __builtin_fmaf(hi, f, -p));
+    hi = p;
+  }
+  __device__ __forceinline__ float value() const { return hi + lo; }
+  __device__ __forceinline__ float times(float x) const { return __builtin_fmaf(x, hi, x * lo); }
+  __device__ __forceinline__ float rest(float x, float product) const { return __builtin_fmaf(x, hi, -product) + x * lo; }
+};
+struct PlainProduct {
+  float v = 1.f;
+  __device__ __forceinline__ void by(float f) { v *= f; }
+  __device__ __forceinline__ float value() const { return v; }
+  __device__ __forceinline__ float times(float x) const { return x * v; }
+};
+
 // the consumer's state: KT tiles of 16 key channels x this lane's value channel
 template <int KT>
 struct State {
@@ -98,28 +130,36 @@ struct State {
         if (col < V && kk < K) slot[(int64_t)kk * V + col] = S[kt][e];
       }
   }
-  // rows (token m) of x times the state; four chains
+  // rows (token m) of x times the state; eight chains (shorter ones round less)
   __device__ __forceinline__ f32x4 times(const float* row) const {
-    f32x4 o[4];
+    f32x4 o[8];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int e = 0; e < 8; ++e) o[e] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) {
       const f32x4 x = *reinterpret_cast<const f32x4*>(row + 16 * kt);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = mma4(x[e], S[kt][e], o[e]);
+      for (int e = 0; e < 4; ++e) o[4 * (kt & 1) + e] = mma4(x[e], S[kt][e], o[4 * (kt & 1) + e]);
     }
-    return (o[0] + o[1]) + (o[2] + o[3]);
+    return ((o[0] + o[1]) + (o[2] + o[3])) + ((o[4] + o[5]) + (o[6] + o[7]));
   }
 };
 
-// a [16 x 16] matrix's rows (in LDS) times four accumulator rows
-__device__ __forceinline__ f32x4 times_rows(const float* a, int m, int g, f32x4 w) {
+// c plus a [16 x 16] matrix's rows (in LDS) times four accumulator rows
+__device__ __forceinline__ f32x4 times_rows(const float* a, int m, int g, f32x4 w, f32x4 c = f32x4{0.f, 0.f, 0.f, 0.f}) {
   const f32x4 x = *reinterpret_cast<const f32x4*>(a + m * RA + 4 * g);
-  f32x4 c = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int e = 0; e < 4; ++e) c = mma4(x[e], w[e], c);
   return c;
+}
+
+// The same summed in double (whose accumulator rows are 4 e + g where a float's are 4 g + e)
+__device__ __forceinline__ f32x4 times_rows_double(const float* a, int m, int g, f32x4 w, f32x4 c) {
+  const f32x4 x = *reinterpret_cast<const f32x4*>(a + row_of_token(m) * RA + 4 * g);
+  f64x4 d = f64x4{c[0], c[1], c[2], c[3]};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) d = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x[e], (double)w[e], d, 0, 0, 0);
+  return f32x4{(float)d[0], (float)d[1], (float)d[2], (float)d[3]};
 }
 
 // The same where a row of w may not be a finite number: nothing of it reaches the rows of tokens before its own (zero times infinity
@@ -130,11 +170,11 @@ __device__ __forceinline__ f32x4 times_rows_in_order(const float* a, int m, int 
 #pragma unroll
   for (int f = 0; f < 4; ++f)
 #pragma unroll 1
-    for (int h = 0; h < 4; ++h) {                          // token 4 h + f
+    for (int h = 0; h < 4; ++h) {                          // row 4 h + f, token 4 f + h
       const float x = __shfl(w[f], 16 * h + m, 64);
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if (4 * h + f <= 4 * g + e) c[e] = __builtin_fmaf(a[(4 * g + e) * RA + 4 * h + f], x, c[e]);
+        if (4 * f + h <= 4 * e + g) c[e] = __builtin_fmaf(a[(4 * g + e) * RA + 4 * h + f], x, c[e]);
     }
   return c;
 }
@@ -145,8 +185,9 @@ __device__ __forceinline__ bool some_not_finite(f32x4 w) {
 }
 
 // (for the scheduler) FIRST reads from LDS, then a read behind every PER products, N times, then REST products: left alone it
-// asks for two rows and waits for them after every eight products (delta rule 198 -> 189 us, decayed sum 165 -> 155; the gated
-// form, bound by its producers, gains nothing)
+// asks for two rows and waits for them after every eight products.  Tuned by measuring, 4 portions of 797 - 1151 tokens and 32 heads:
+// delta rule 128 x 128 207 us without, 189 here (<6, 28, 2, 12> 200, <12, 22, 3, 3> 214), 64 x 64 126 and 122; bonus form 64 x 64
+// 115 and 105.  The gated form, bound by its producers, gains nothing.
 template <int FIRST, int N, int PER, int REST>
 __device__ __forceinline__ void products_behind_reads() {
   __builtin_amdgcn_sched_group_barrier(0x100, FIRST, 0);
@@ -176,7 +217,7 @@ struct Rows {
       f32x4 f;
 #pragma unroll
       for (int j = 0; j < 4; ++j) f[j] = p[i].get(j, row_of(i, tid) < n, c0 + col_of(i, tid), n_ch) * scale;
-      *reinterpret_cast<f32x4*>(lds + row_of(i, tid) * (W + 4) + col_of(i, tid)) = f;
+      *reinterpret_cast<f32x4*>(lds + row_of_token(row_of(i, tid)) * (W + 4) + col_of(i, tid)) = f;
     }
   }
 };
@@ -188,7 +229,7 @@ template <int KP, bool DELTA, typename QK, typename VT, bool VEC>
 __global__ __launch_bounds__(512) void chunk_head_kernel(ChunkScanArgs a) {
   constexpr int KT = KP / 16, RS = KP + 4;
   constexpr int kRaw = 2 * C * RS + C * VS + 3 * C;       // q | k | v | decay, value scale, write strength
-  constexpr int kMade = 2 * C * RA + 2 * C;               // A | M (T while it is made) | prefix, suffix
+  constexpr int kMade = 2 * C * RA + 3 * C;               // A | M (T while it is made) | prefix, suffix, what the prefix's rounding left over
   extern __shared__ __attribute__((aligned(16))) float lds[];      // raw[3] | made[2]
   const int seq = blockIdx.z, head = blockIdx.x, col0 = (int)blockIdx.y * VW;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -214,6 +255,7 @@ __global__ __launch_bounds__(512) void chunk_head_kernel(ChunkScanArgs a) {
       const float* A = made(c);
       const float* M = A + C * RA;
       const f32x4 pre = *reinterpret_cast<const f32x4*>(M + C * RA + 4 * g), suf = *reinterpret_cast<const f32x4*>(M + C * RA + C + 4 * g);
+      const f32x4 rest = *reinterpret_cast<const f32x4*>(M + C * RA + 2 * C + 4 * g);
       const float total = M[C * RA + C - 1];
       f32x4 x, w;
 #pragma unroll
@@ -230,29 +272,28 @@ __global__ __launch_bounds__(512) void chunk_head_kernel(ChunkScanArgs a) {
       }
       const f32x4 before = st.times(q);
       f32x4 within = times_rows(A, m, g, w);
-      products_behind_reads<14, 20, 3, 12>();
+      if constexpr (KP == 128) products_behind_reads<8, 26, 3, 1>();
+      else products_behind_reads<10, 9, 3, 13>();
       if (some_not_finite(w)) {                            // (of x: then every row of w)
         if constexpr (DELTA) w = times_rows_in_order(M, m, g, x);
         within = times_rows_in_order(A, m, g, w);
       }
       f32x4 o;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = __builtin_fmaf(before[e], pre[e], within[e]);
+      for (int e = 0; e < 4; ++e) o[e] = __builtin_fmaf(before[e], pre[e], __builtin_fmaf(before[e], rest[e], within[e]));
       const int n = rows_of(c);
       const int64_t t0 = t_begin + (int64_t)c * C;
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if (4 * g + e < n && col < a.V) a.out[(t0 + 4 * g + e) * ((int64_t)a.heads * a.V) + (int64_t)head * a.V + col] = o[e];
+        if (4 * e + g < n && col < a.V) a.out[(t0 + 4 * e + g) * ((int64_t)a.heads * a.V) + (int64_t)head * a.V + col] = o[e];
 #pragma unroll
       for (int e = 0; e < 4; ++e) w[e] *= suf[e];
-      const float* kr = r + C * RS + 4 * g * RS + m;      // k of token 4 g + e, channel 16 kt + m
+      const float* kr = r + C * RS + 4 * g * RS + m;      // k of row 4 g + e, channel 16 kt + m
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt) {
-        f32x4 more = f32x4{0.f, 0.f, 0.f, 0.f};           // (summed apart: the state is rounded once a chunk)
+        st.S[kt] *= total;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) more = mma4(kr[e * RS + 16 * kt], w[e], more);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) st.S[kt][e] = __builtin_fmaf(st.S[kt][e], total, more[e]);
+        for (int e = 0; e < 4; ++e) st.S[kt] = mma4(kr[e * RS + 16 * kt], w[e], st.S[kt]);
       }
       products_behind_reads<16, 16, 2, 1>();
       lds_barrier();
@@ -263,62 +304,86 @@ __global__ __launch_bounds__(512) void chunk_head_kernel(ChunkScanArgs a) {
 
   // Producers: wave 0 A, prefixes and suffixes, wave 1 M, wave 2 brings q and the values, wave 3 k and the tokens' scalars.
   const int qk_head = head / (a.heads / a.qk_heads);
-  auto finish = [&](int chunk) __attribute__((always_inline)) {
-    if (chunk < 0 || chunk >= n_chunks || (wave == 1 && !DELTA)) return;
-    const float* r = raw(chunk);
-    const float *k = r + C * RS, *sc = r + 2 * C * RS + C * VS;
-    float* A = made(chunk) + wave * (C * RA);             // wave 1: T, then M
-    const float* rows_x = wave == 0 ? r : k;
-    // (x k^T)[i, j] with rows i = 4 g + e and column j = m
-    f32x4 p[4];
+  // (x k^T)[i, j] with rows i = 4 g + e and column j = m: tokens 4 e + g and t_m; N chains
+  const int t_m = row_of_token(m);
+  auto with_keys = [&](const float* rows_x, const float* k, auto chains) __attribute__((always_inline)) {
+    constexpr int N = decltype(chains)::value;
+    f32x4 p[N];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) p[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < N; ++i) p[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) {
       const f32x4 x = *reinterpret_cast<const f32x4*>(rows_x + m * RS + 16 * kt + 4 * g);
       const f32x4 y = *reinterpret_cast<const f32x4*>(k + m * RS + 16 * kt + 4 * g);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) p[e] = mma4(x[e], y[e], p[e]);
+      for (int e = 0; e < 4; ++e) p[(4 * kt + e) % N] = mma4(x[e], y[e], p[(4 * kt + e) % N]);
     }
-    const f32x4 xk = (p[0] + p[1]) + (p[2] + p[3]);
-    float d[C];
+#pragma unroll
+    for (int n = N / 2; n > 0; n >>= 1)
+#pragma unroll
+      for (int i = 0; i < n; ++i) p[i] += p[i + n];
+    return p[0];
+  };
+  auto decays = [&](const float* sc, float (&d)[C]) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < C / 4; ++i) {
       const f32x4 x = *reinterpret_cast<const f32x4*>(sc + 4 * i);
 #pragma unroll
       for (int e = 0; e < 4; ++e) d[4 * i + e] = x[e];
     }
-    // run = prod(m < r <= t) d_r, kept at the lane's four rows
-    float run = 1.f, prefix = 1.f, mine[4];
+  };
+  // A, prefixes and suffixes: with sixteen chains and products of decays rounded once, as A's rounding is the larger part of a
+  // result's error
+  auto finish_A = [&](int chunk) __attribute__((always_inline)) {
+    const float* r = raw(chunk);
+    float* A = made(chunk);
+    const f32x4 xk = with_keys(r, r + C * RS, std::integral_constant<int, 16>());
+    float d[C];
+    decays(r + 2 * C * RS + C * VS, d);
+    Product run, mine[4];                                 // run = prod(t_m < r <= t) d_r, kept at the lane's four rows
 #pragma unroll
     for (int t = 0; t < C; ++t) {
-      prefix *= t <= m ? d[t] : 1.f;                      // (up to token m)
-      run = t > m ? run * d[t] : 1.f;
-      if ((t & 3) == 0) mine[0] = t >> 2 == g ? run : mine[0];
-      if ((t & 3) == 1) mine[1] = t >> 2 == g ? run : mine[1];
-      if ((t & 3) == 2) mine[2] = t >> 2 == g ? run : mine[2];
-      if ((t & 3) == 3) mine[3] = t >> 2 == g ? run : mine[3];
+      run.by(t > t_m ? d[t] : 1.f);
+      const bool here = (t & 3) == 0 || (t & 3) == g;
+      mine[t >> 2].hi = here ? run.hi : mine[t >> 2].hi;
+      mine[t >> 2].lo = here ? run.lo : mine[t >> 2].lo;
     }
-    if (wave == 0) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) A[(4 * g + e) * RA + m] = m <= 4 * g + e ? xk[e] * mine[e] : 0.f;
-      if (g == 0) {
-        A[2 * C * RA + m] = prefix;
-        A[2 * C * RA + C + m] = run;                      // (behind token m)
+    for (int e = 0; e < 4; ++e) A[(4 * g + e) * RA + m] = t_m <= 4 * e + g ? mine[e].times(xk[e]) : 0.f;
+    if (g == 0) A[2 * C * RA + C + m] = run.value();      // behind token t_m
+    if (m == 0) {                                         // up to the rows' tokens: the first one's decay and all behind it
+      f32x4 prefix, rest;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        prefix[e] = mine[e].times(d[0]);
+        rest[e] = mine[e].rest(d[0], prefix[e]);
       }
-      return;
+      *reinterpret_cast<f32x4*>(A + 2 * C * RA + 4 * g) = prefix;
+      *reinterpret_cast<f32x4*>(A + 2 * C * RA + 2 * C + 4 * g) = rest;
+    }
+  };
+  auto finish_M = [&](int chunk) __attribute__((always_inline)) {
+    const float *k = raw(chunk) + C * RS, *sc = k + C * RS + C * VS;
+    float* A = made(chunk) + C * RA;                      // T (by tokens), then M
+    const f32x4 xk = with_keys(k, k, std::integral_constant<int, 4>());
+    float d[C], run = 1.f, mine[4];
+    decays(sc, d);
+#pragma unroll
+    for (int t = 0; t < C; ++t) {
+      run = t > t_m ? run * d[t] : 1.f;
+      mine[t >> 2] = (t & 3) == 0 || (t & 3) == g ? run : mine[t >> 2];
     }
     const f32x4 b = *reinterpret_cast<const f32x4*>(sc + 2 * C + 4 * g);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) A[(4 * g + e) * RA + m] = m < 4 * g + e ? b[e] * xk[e] * mine[e] : 0.f;
+    for (int e = 0; e < 4; ++e) A[(4 * e + g) * RA + t_m] = t_m < 4 * e + g ? b[e] * xk[e] * mine[e] : 0.f;      // (T: by tokens)
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // column m of (I + T)^-1: x_t = [t == m] - sum(s < t) T[t, s] x_s
+    // column t_m of (I + T)^-1: x_t = [t == t_m] - sum(s < t) T[t, s] x_s
     float x[C];
 #pragma unroll
     for (int t = 0; t < C; ++t) {
-      float s0 = t == m ? 1.f : 0.f, s1 = 0.f;
+      float s0 = t == t_m ? 1.f : 0.f, s1 = 0.f;
 #pragma unroll
       for (int s = 0; s < t; s += 4) {
         const f32x4 T = *reinterpret_cast<const f32x4*>(A + t * RA + s);
@@ -337,12 +402,15 @@ __global__ __launch_bounds__(512) void chunk_head_kernel(ChunkScanArgs a) {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     if (g == 0) {
 #pragma unroll
-      for (int t = 0; t < C; ++t) A[t * RA + m] = x[t];
+      for (int t = 0; t < C; ++t) A[row_of_token(t) * RA + m] = x[t];
     }
   };
   if (wave < 2) {
     for (int c = -2; c < n_chunks; ++c) {
-      finish(c + 1);
+      if (c + 1 >= 0 && c + 1 < n_chunks) {
+        if (wave == 0) finish_A(c + 1);
+        else if constexpr (DELTA) finish_M(c + 1);
+      }
       lds_barrier();
     }
     return;
@@ -374,10 +442,10 @@ __global__ __launch_bounds__(512) void chunk_head_kernel(ChunkScanArgs a) {
     s.rows.store(r + (wave == 2 ? 0 : C * RS), 0, a.K, n, 1.f, lane);
     s.values.store(r + 2 * C * RS, col0, a.V, n, 1.f, (int)threadIdx.x - 128);
     if (wave == 3 && g == 0) {             // (a row past the portion changes nothing)
-      float* sc = r + 2 * C * RS + C * VS + m;
-      sc[0] = m < n ? s.scalars[0] : 1.f;
-      sc[C] = m < n && a.vscale ? s.scalars[1] : 1.f;
-      sc[2 * C] = m < n && DELTA ? s.scalars[2] : 0.f;
+      float* sc = r + 2 * C * RS + C * VS;                 // (decays by token, the others by row)
+      sc[m] = m < n ? s.scalars[0] : 1.f;
+      sc[C + row_of_token(m)] = m < n && a.vscale ? s.scalars[1] : 1.f;
+      sc[2 * C + row_of_token(m)] = m < n && DELTA ? s.scalars[2] : 0.f;
     }
   };
 #pragma unroll
@@ -436,7 +504,9 @@ __global__ __launch_bounds__(768) void chunk_channel_kernel(ChunkScanArgs a) {
   constexpr int KT = KP / 16, RS = KP + 4, NP = KP / 64;  // NP key channels a lane of a producer wave
   constexpr bool GATED = FORM == hxm::kChunkGated, BONUS = FORM == hxm::kChunkBonus;
   constexpr int kGate = C * KP * (GATED ? 2 : 3);         // decays | q | k
-  constexpr int kMade = C * RS + KP * RA + C * RA + KP;   // q times prefix | (k times suffix)^T | A | total
+  // q times prefix | (k times suffix)^T | A | total | what the rounding of (k times suffix)^T left over, in bfloat16 (bonus form: its
+  // k v is often exact, and a rounded factor would be the larger part of the state's error)
+  constexpr int kMade = C * RS + KP * RA + C * RA + KP + (BONUS ? KP * RA / 2 : 0);
   extern __shared__ __attribute__((aligned(16))) float lds[];      // gates[2] | made[2] | values[3]
   const int seq = blockIdx.z, head = blockIdx.x, col0 = (int)blockIdx.y * VW;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -465,24 +535,31 @@ __global__ __launch_bounds__(768) void chunk_channel_kernel(ChunkScanArgs a) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) w[e] = vs[e * VS];
       const f32x4 before = st.times(p + m * RS + 4 * g);
-      f32x4 within = times_rows(A, m, g, w);
+      s16x4 w16;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w16[e] = (short)BF16::from_float(w[e]);
+      f32x4 o = BONUS ? times_rows_double(A, m, g, w, before) : times_rows(A, m, g, w, before);
       if constexpr (!GATED) products_behind_reads<10, 4, 4, 20>();
-      if (some_not_finite(w)) within = times_rows_in_order(A, m, g, w);
-      const f32x4 o = before + within;
+      if (some_not_finite(w)) o = before + times_rows_in_order(A, m, g, w);
       const int n = rows_of(c);
       const int64_t t0 = t_begin + (int64_t)c * C;
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if (4 * g + e < n && col < a.V) a.out[(t0 + 4 * g + e) * ((int64_t)a.heads * a.V) + (int64_t)head * a.V + col] = o[e];
+        if (4 * e + g < n && col < a.V) a.out[(t0 + 4 * e + g) * ((int64_t)a.heads * a.V) + (int64_t)head * a.V + col] = o[e];
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt) {
         const f32x4 d = *reinterpret_cast<const f32x4*>(total + 16 * kt + 4 * g);
         const f32x4 x = *reinterpret_cast<const f32x4*>(kt_ + (16 * kt + m) * RA + 4 * g);
-        f32x4 more = f32x4{0.f, 0.f, 0.f, 0.f};           // (summed apart: the state is rounded once a chunk)
+        if constexpr (BONUS) {
+          const s16x4 y = *reinterpret_cast<const s16x4*>(reinterpret_cast<const u16*>(total + KP) + (16 * kt + m) * RA + 4 * g);
+          const f32x4 rest = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(y, w16, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) more = mma4(x[e], w[e], more);
+          for (int e = 0; e < 4; ++e) st.S[kt][e] = __builtin_fmaf(st.S[kt][e], d[e], rest[e]);
+        } else {
+          st.S[kt] *= d;
+        }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) st.S[kt][e] = __builtin_fmaf(st.S[kt][e], d[e], more[e]);
+        for (int e = 0; e < 4; ++e) st.S[kt] = mma4(x[e], w[e], st.S[kt]);
       }
       if constexpr (!GATED) products_behind_reads<6, 10, 2, 12>();
       lds_barrier();
@@ -579,7 +656,7 @@ __global__ __launch_bounds__(768) void chunk_channel_kernel(ChunkScanArgs a) {
     else if (i < 25) s = 7 - W, t = 7 - W + i - (16 - W);
     else if (i < 33 - W) s = 8 + W, t = 8 + W + i - 25;
     else s = 15 - W, t = 15 - W + i - (33 - W);
-    to = t * RA + s;
+    to = row_of_token(t) * RA + row_of_token(s);
   }
   auto finish_wave = [&](int chunk, auto W_) __attribute__((always_inline)) {
     constexpr int W = decltype(W_)::value, S0 = 4 * W;
@@ -608,51 +685,51 @@ __global__ __launch_bounds__(768) void chunk_channel_kernel(ChunkScanArgs a) {
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
           if (t > column[j] && !BONUS) run[p] *= f[t][p];
-          s += q[t][p] * (BONUS && t == column[j] ? u[p] * run[p] : run[p]);
+          if (BONUS && t == column[j]) s = __builtin_fmaf(q[t][p] * run[p], u[p], s);
+          else s += q[t][p] * run[p];
           if (t > column[j] && BONUS) run[p] *= f[t][p];
         }
         x[at++] = s;
       }
     }
-    // prefixes up to this wave's tokens, suffixes behind them
-    float pre[NP], suf[NP];
+    // prefixes up to this wave's tokens, suffixes behind them (the gated form, whose decays are computed here, has no use for the
+    // rest of a product: its state is off by less than before)
+    typedef std::conditional_t<GATED, PlainProduct, Product> Decays;
+    Decays pre[NP], suf[NP];
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
-      pre[p] = 1.f;
 #pragma unroll
-      for (int t = 0; t < S0; ++t) pre[p] *= f[t][p];
-      suf[p] = 1.f;
+      for (int t = 0; t < S0; ++t) pre[p].by(f[t][p]);
 #pragma unroll
-      for (int t = C - 1; t >= S0 + 4; --t) suf[p] *= f[t][p];
+      for (int t = C - 1; t >= S0 + 4; --t) suf[p].by(f[t][p]);
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int p = 0; p < NP; ++p) {
-        if (!BONUS) pre[p] *= f[S0 + j][p];
-        P[(S0 + j) * RS + d0 + p] = q[S0 + j][p] * pre[p];
-        if (BONUS) pre[p] *= f[S0 + j][p];
+        if (!BONUS) pre[p].by(f[S0 + j][p]);
+        P[row_of_token(S0 + j) * RS + d0 + p] = pre[p].times(q[S0 + j][p]);
+        if (BONUS) pre[p].by(f[S0 + j][p]);
       }
     if (W == 3) {
 #pragma unroll
-      for (int p = 0; p < NP; ++p) A[C * RA + d0 + p] = pre[p];
+      for (int p = 0; p < NP; ++p) A[C * RA + d0 + p] = pre[p].value();
     }
-    f32x4 ks[NP];
 #pragma unroll
     for (int j = 3; j >= 0; --j)
 #pragma unroll
       for (int p = 0; p < NP; ++p) {
-        ks[p][j] = (GATED ? 1.0f - f[S0 + j][p] : G[2 * C * KP + (S0 + j) * KP + d0 + p]) * suf[p];
-        suf[p] *= f[S0 + j][p];
+        const float k = GATED ? 1.0f - f[S0 + j][p] : G[2 * C * KP + (S0 + j) * KP + d0 + p], ks = suf[p].times(k);
+        P[C * RS + (d0 + p) * RA + row_of_token(S0 + j)] = ks;
+        if constexpr (BONUS) reinterpret_cast<u16*>(A + C * RA + KP)[(d0 + p) * RA + row_of_token(S0 + j)] = BF16::from_float(suf[p].rest(k, ks));
+        if (j > 0) suf[p].by(f[S0 + j][p]);
       }
-#pragma unroll
-    for (int p = 0; p < NP; ++p) *reinterpret_cast<f32x4*>(P + C * RS + (d0 + p) * RA + S0) = ks[p];
     // the last two elements by themselves: token 15 of columns 8 + W (W = 0) or 15 - W, and the one before it
     float last[2] = {wave_total(x[32]), wave_total(x[33])};
     const float sum = transpose_sum32(x, lane);
     if ((lane & 1) == 0) A[to] = sum;
-    if (lane == 1) A[(W == 0 ? 15 : 14) * RA + (W == 0 ? 8 : 15 - W)] = last[0];
-    if (lane == 3) A[15 * RA + 15 - W] = last[1];
+    if (lane == 1) A[row_of_token(W == 0 ? 15 : 14) * RA + row_of_token(W == 0 ? 8 : 15 - W)] = last[0];
+    if (lane == 3) A[row_of_token(15) * RA + row_of_token(15 - W)] = last[1];
   };
   auto finish = [&](int chunk) __attribute__((always_inline)) {
     if (chunk < 0 || chunk >= n_chunks) return;
@@ -690,12 +767,12 @@ template <int KP, typename QK, typename VT, bool VEC>
 int launch_form(const ChunkScanArgs& a, hipStream_t s) {
   if (a.per_channel || a.form == hxm::kChunkGated) {
     const int kinds = a.form == hxm::kChunkGated ? 2 : 3;
-    const size_t lds = sizeof(float) * (2 * C * KP * kinds + 2 * (C * (KP + 4) + KP * RA + C * RA + KP) + 3 * C * VS);
+    const size_t lds = sizeof(float) * (2 * C * KP * kinds + 2 * (C * (KP + 4) + KP * RA + C * RA + KP + (a.form == hxm::kChunkBonus ? KP * RA / 2 : 0)) + 3 * C * VS);
     if (a.form == hxm::kChunkGated) return launch(chunk_channel_kernel<KP, hxm::kChunkGated, QK, VT, VEC>, 768, lds, a, s);
     if (a.form == hxm::kChunkBonus) return launch(chunk_channel_kernel<KP, hxm::kChunkBonus, QK, VT, VEC>, 768, lds, a, s);
     return launch(chunk_channel_kernel<KP, hxm::kChunkDecay, QK, VT, VEC>, 768, lds, a, s);
   }
-  const size_t lds = sizeof(float) * (3 * (2 * C * (KP + 4) + C * VS + 3 * C) + 2 * (2 * C * RA + 2 * C));
+  const size_t lds = sizeof(float) * (3 * (2 * C * (KP + 4) + C * VS + 3 * C) + 2 * (2 * C * RA + 3 * C));
   if (a.form == hxm::kChunkDelta) return launch(chunk_head_kernel<KP, true, QK, VT, VEC>, 512, lds, a, s);
   return launch(chunk_head_kernel<KP, false, QK, VT, VEC>, 512, lds, a, s);
 }

@@ -48,6 +48,37 @@ def test_portions_through_a_scan(lens, K, V, form, per_channel, types):
     _through_a_scan(lens, K, V, form, per_channel, types, 3)
 
 
+# out, state: what a token at a time loses in float over the same portions (2-norm, in 1e-7, measured with the form that walks the
+# tokens).  Chunks lose no more than that, give or take a twentieth.
+@pytest.mark.parametrize("form, K, out, state", [("delta", 128, 1.096, 0.780), ("delta", 64, 1.010, 0.838), ("decay", 128, 1.073, 0.825), ("decay", 64, 1.001, 0.808),
+                                                 ("bonus", 128, 0.908, 0.464), ("bonus", 64, 0.832, 0.464)])
+def test_chunks_round_no_more_than_single_tokens(form, K, out, state):
+    from hydrainfer_amd._C.kernel.seq_mix import state_scan
+    from hydrainfer_amd._C.kernel.stream_ops import SequenceState
+    g = torch.Generator().manual_seed(K)
+    lens, H, per_channel, bounds = [400, 250], 4, form == "bonus", (1.05e-7 * out, 1.05e-7 * state)
+    T, cu = sum(lens), [0, 400, 650]
+    f = lambda *s: torch.randn(s, generator=g)
+    unit = lambda x: torch.nn.functional.normalize(x, dim=-1).reshape(T, H * K)
+    if form == "delta":
+        q, k = unit(f(T, H, K)) * K ** -0.5, unit(f(T, H, K))
+    else:
+        q, k = ((f(T, H * K) * K ** -0.5).bfloat16() for _ in range(2))
+    v, step = f(T, H * K).bfloat16(), torch.nn.functional.softplus(f(T, H) - 2)
+    decay = torch.exp(-torch.exp(f(T, H * K) - 2)) if per_channel else torch.exp(-torch.exp(0.3 * f(H)) * step)
+    beta, bonus, state = torch.sigmoid(f(T, H)), f(H * K), 0.1 * f(2, 1, H * K * K)
+    h = lambda x: x.double().view(T, H, K)
+    want, S = _scan(form, h(q), h(k), h(v), decay.double().view(T, H, -1).expand(T, H, K), step.double() if form == "decay" else torch.ones((T, H), dtype=torch.float64),
+                    beta.double(), bonus.double().view(H, K), state.double().view(2, H, K, K), cu, [False, False])
+    c = lambda x: x.cuda()
+    st = c(state)
+    seq = SequenceState(st, torch.arange(2, dtype=torch.int32, device="cuda"), c(torch.tensor([0] * 400 + [1] * 250, dtype=torch.int32)))
+    got = state_scan(form, c(q), c(k), c(v), c(decay), seq, 0, c(torch.tensor(cu, dtype=torch.int32)), c(torch.arange(1, T + 1, dtype=torch.int32)), H, H, K, K,
+                     vscale=c(step) if form == "decay" else None, beta=c(beta) if form == "delta" else None, bonus=c(bonus) if form == "bonus" else None)
+    _check("out", got, want.reshape(T, H * K), bounds[0])
+    _check("state", st.view(2, H, K, K), S, bounds[1])
+
+
 # batches of as many tokens as sequences (csrc/state_scan.hip, the step form): columns and rows that fill no workgroup, a sequence that
 # brings two tokens and one that brings none, slots that start on a multiple of four floats and (the form with a column a lane) not
 @pytest.mark.parametrize("lens", [[1], [1, 1, 1, 1, 1], [2, 0, 1]])
