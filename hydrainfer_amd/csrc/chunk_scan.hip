@@ -20,7 +20,7 @@
 // What bounds it now: the chunks of a sequence follow each other (2.5 us each with states of 128 x 128; 1.8 us of float matrix
 // products on the SIMDs that hold a consumer and a maker of A or M).  Measured against one token at a time, 4 portions of 797 -
 // 1151 tokens: delta rule, 32 heads of 128 x 128, 479 -> 189 us; decayed sum, 64 heads of 128 x 64, 432 -> 143 us; bonus form, 32
-// heads of 64 x 64, 207 -> 105 us; gated form, 32 heads of 128 x 128, 720 -> 201 us with its norm.
+// heads of 64 x 64, 207 -> 105 us; gated form, 32 heads of 128 x 128, 720 -> 205 us with its norm.
 // What the rounding costs: a token at a time rounds a state's element once a token, and each rounding decays with the state.  Here
 // the products of decays, of keys with them and the chunk's sums are rounded besides, and four things keep that from showing: sums
 // over tokens run from the first token to the last and on top of the decayed state (row_of_token); products of decays carry what
@@ -28,7 +28,7 @@
 // k v is often exact, adds up within a chunk in double and keeps the rest of its suffixed keys.  Error against 64 bits (2-norm), a
 // token at a time and here, 3 portions of 200 - 600 tokens, 16 heads of 128 x 128 (64 x 64): results delta 1.07 1.07 (1.00 1.00),
 // decay 1.04 0.84 (0.97 0.77), bonus 0.90 0.82 (0.83 0.77) e-7; states delta 0.74 0.73 (0.75 0.74), decay 0.68 0.62 (0.72
-// 0.66), bonus 0.46 0.45 (0.47 0.45), gated 1.42 1.08 (1.41 1.07) e-7.
+// 0.66), bonus 0.46 0.45 (0.47 0.45), gated 1.42 1.09 (1.41 1.08) e-7.
 #include <type_traits>
 #include "chunk_scan.h"
 #include "mix_rows.h"
@@ -79,14 +79,13 @@ struct Piece {
   __device__ __forceinline__ float get(int j, bool in, int c, int n_ch) const { return in && c + j < n_ch ? A::to_float(r[j]) : 0.f; }
 };
 
-// 1 / (1 + e^-x) to about one unit in the last place in a third of the instructions that expf and a division take: the
-// hardware's exponential (the rounding of its argument moves the sum's place by less than that) and reciprocal with one
-// Newton step.  NaN stays NaN; the bound keeps the Newton step finite.
+// 1 / (1 + e^-x) to two or three units in the last place, however small it is, in a third of the instructions that expf and a division
+// take: the hardware's power of two and reciprocal, and what the rounding of the power's argument t left over, -x - t ln 2 (for x = -20
+// it would move the gate by 1e-6 of itself).  NaN stays NaN; where x or t is infinite there is no rest.
 __device__ __forceinline__ float sigmoid_gate(float x) {
-  float e = __expf(-x);
-  e = e > 1e37f ? 1e37f : e;
-  const float d = 1.0f + e, r = __builtin_amdgcn_rcpf(d);
-  return __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
+  const float t = x * -1.4426950408889634f;
+  const float rest = __builtin_fmaf(t, 1.9046543e-09f, __builtin_fmaf(t, -0.69314718246459961f, -x));
+  return __builtin_amdgcn_rcpf(__builtin_fmaf(__builtin_amdgcn_exp2f(t), 1.0f + (fabsf(rest) < 1.0f ? rest : 0.f), 1.0f));
 }
 
 // A product of decays with what its roundings left over: the value is rounded once, however many factors it has.

@@ -1,6 +1,8 @@
 """Portions of prompts through the recurrences with a matrix state (csrc/chunk_scan.hip) against a token at a time in 64 bits:
 portions around the sixteen tokens of a chunk, single tokens beside them, keys and values that fill no tile, every operand
 type, rows that cannot be read four elements at a time, decays that vanish."""
+import math
+
 import pytest
 import torch
 
@@ -235,3 +237,22 @@ def test_portions_through_the_gated_recurrence(lens, K, V, dtype):
     _check("state", st[:, 1].view(n, H, K, V), S, 2 * TOL)
     _check("out", got, want.reshape(T, H * V), 2 * TOL if dtype == torch.float32 else 2.0 ** -8)
     assert torch.equal(st[:, 0].cpu(), state[:, 0])
+
+
+def test_small_gates_are_as_exact_as_large_ones():
+    # without values a state is the product of its gates; two of them, each off by a few units in the last place (2^-23) of its exponential,
+    # sum and reciprocal
+    from hydrainfer_amd._C.kernel.recurrence import gated_recurrence
+    from hydrainfer_amd._C.kernel.stream_ops import SequenceState
+    H, K, V, T = 4, 128, 64, 2
+    proj = torch.zeros((T, H * (2 * K + V)))
+    proj[:, H * K:2 * H * K] = torch.linspace(-40.0, 100.0, T * H * K).view(T, H * K).flip(1)
+    proj[0, H * K], proj[1, H * K], proj[0, H * K + 1], proj[1, H * K + 1] = -80.0, 300.0, math.inf, math.inf
+    st = torch.ones((1, 1, H * K * V), device="cuda")
+    seq = SequenceState(st, torch.zeros(1, dtype=torch.int32, device="cuda"), torch.zeros(T, dtype=torch.int32, device="cuda"))
+    zero, p = torch.zeros(H * K, device="cuda"), proj.cuda()
+    gated_recurrence(p[:, :H * K], p[:, H * K:2 * H * K], p[:, 2 * H * K:], zero, zero, torch.ones(V, device="cuda"), 1e-5, seq, 0,
+                     torch.tensor([0, T], dtype=torch.int32).cuda(), torch.tensor([5, 6], dtype=torch.int32).cuda(), H, K, V, max_q_len=T)
+    want = torch.sigmoid(proj[:, H * K:2 * H * K].double()).prod(0).view(H, K, 1)
+    off = (st.double().cpu().view(H, K, V) - want).abs() / want
+    assert float(off.max()) <= 8 * 2.0 ** -23, float(off.max())
