@@ -600,14 +600,16 @@ __global__ __launch_bounds__(256) void biased_attn_group_kernel(hxm_biased_attn_
 //   * a tile's key and value rows go straight from the paged cache to LDS (1 KiB an instruction, whole rows), the next tile's
 //     while this one is worked on: two images, one barrier a tile.  Rows cannot be padded this way; their 16-byte chunks are
 //     swizzled by the lane that asks for them (keys: chunk ^ row, values: 64-byte quarter ^ row);
-//   * a row keeps the maximum it refers its weights to until a score exceeds it by 2^8: the accumulators are rarely rescaled.
+//   * a row's weights refer to its largest score so far, 32 keys at a time.  That costs a pass over the accumulators for nearly every
+//     half tile; left up to 2^8 behind, it took 52 us instead of 57 and results were off by 3 % more, as the largest weights were
+//     rounded to bfloat16 instead of being 1.
 // The order of the row tiles: the XCDs (workgroups are dealt round robin) take key heads of their own where there are enough of
 // them, and of every sequence the tiles with the most keys come first.
-// Measured, 4 portions of 797 - 1151 tokens, 32 heads of 128 on 8 key heads, sinks: 221 us in the group form, 51 us
-// here (630 TFLOP/s of the pairs that a mask leaves); window of 512 and soft cap 223 and 58 us; chunks of 512 and slopes 163 and
+// Measured, 4 portions of 797 - 1151 tokens, 32 heads of 128 on 8 key heads, sinks: 221 us in the group form, 57 us
+// here (570 TFLOP/s of the pairs that a mask leaves); window of 512 and soft cap 223 and 58 us; chunks of 512 and slopes 163 and
 // 45 us.  Down to 64 rows of a key head it is the faster one (16 tokens behind 500 keys: 30 and 21 us).
 // ---------------------------------------------------------------------------------------------------------------
-template <int D, int V, bool MODS>      // MODS: slopes or a soft cap
+template <int D, int V, bool MODS, bool FINE>      // MODS: slopes or a soft cap; FINE: every 32 keys' weights refer to their own largest score
 __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_attn_args a, int tile_slots) {
   constexpr int KT = 64, TQ = 128, KS = D / 16, NDB = V / 32;
   constexpr int RSK = 2 * D, RSV = 2 * V, LK = D / 8, LV = V / 8;        // bytes and 16-byte chunks of a row
@@ -774,13 +776,7 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
           for (int e = 0; e < 16; ++e) s[u][e] += __builtin_fmaf(slope2, (float)(32 * u + (e & 3) + 8 * (e >> 2)), base);
       }
     }
-    float mx = HX_NEG_BIG;
-    if (t * KT + KT - 1 <= wpos0 && t * KT >= wlo1) {      // every row of the wave sees the whole tile
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[u][e]);
-    } else {
+    if (!(t * KT + KT - 1 <= wpos0 && t * KT >= wlo1)) {      // (else every row of the wave sees the whole tile)
       const int last = pos - key_l, first = lo - key_l;
 #pragma unroll
       for (int u = 0; u < 2; ++u)
@@ -788,45 +784,72 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
         for (int e = 0; e < 16; ++e) {
           const int k = 32 * u + (e & 3) + 8 * (e >> 2);
           if (k > last || k < first) s[u][e] = -INFINITY;
-          mx = fmaxf(mx, s[u][e]);
         }
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float m_cand = fmaxf(m, mx * unit);
-    const bool grow = m_cand > m + 8.0f;
-    if (__builtin_amdgcn_ballot_w64(grow)) {
-      const float m_new = grow ? m_cand : m, alpha = fast_exp2(m - m_new);
-      l *= alpha;
+    // The weights refer to the largest score so far, half a tile at a time: its own is then 1, which no rounding to bfloat16 touches.  In
+    // launches of few rows (FINE) they refer to the largest of these 32 keys, and what they add is scaled behind the products: the tile
+    // form deals such a launch's keys to more waves, each with a largest score that weighs exactly 1.
+    float m_ref[2] = {HX_NEG_BIG, HX_NEG_BIG}, m_new[2];
 #pragma unroll
-      for (int i = 0; i < NDB; ++i)
+    for (int u = 0; u < 2; ++u) {
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[i][e] *= alpha;
-      m = m_new;
+      for (int e = 0; e < 16; ++e) m_ref[u] = fmaxf(m_ref[u], s[u][e]);
+      m_ref[u] = fmaxf(m_ref[u], __shfl_xor(m_ref[u], 32, 64)) * unit;
+      asm("" : "+v"(m_ref[u]));              // (rounded: left inside a difference below it would not be m_new's number)
+      m_new[u] = fmaxf(u ? m_new[0] : m, m_ref[u]);
+      if (!FINE) m_ref[u] = m_new[u];
     }
     u16x8 pf[2][2];
-    float pa = 0.f, pb = 0.f;
+    float ps[2];
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < 2; ++u) {
+      float pa = 0.f, pb = 0.f;
 #pragma unroll
       for (int e = 0; e < 16; e += 2) {
-        const float e0 = fast_exp2(__builtin_fmaf(s[u][e], unit, -m)), e1 = fast_exp2(__builtin_fmaf(s[u][e + 1], unit, -m));
+        const float e0 = fast_exp2(__builtin_fmaf(s[u][e], unit, -m_ref[u])), e1 = fast_exp2(__builtin_fmaf(s[u][e + 1], unit, -m_ref[u]));
         pa += e0;
         pb += e1;
         pf[u][e >> 3][e & 7] = BF16::from_float(e0);
         pf[u][e >> 3][(e & 7) + 1] = BF16::from_float(e1);
       }
-    l += pa + pb;
+      ps[u] = pa + pb;
+    }
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < 2; ++u) {
+      const float alpha = fast_exp2(m - m_new[u]), beta = fast_exp2(m_ref[u] - m_new[u]);
+      if (FINE || __builtin_amdgcn_ballot_w64(m_new[u] > m)) {
+        l *= alpha;
+        if constexpr (!FINE) {
 #pragma unroll
-      for (int k2 = 0; k2 < 2; ++k2) {
+          for (int i = 0; i < NDB; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][e] *= alpha;
+        }
+        m = m_new[u];
+      }
+      l = FINE ? __builtin_fmaf(ps[u], beta, l) : l + ps[u];
+      auto product = [&](int db, int k2, f32x16 c) __attribute__((always_inline)) {
         const char* vrd = vt + (32 * u + 16 * k2) * RSV + tr_off;
+        const u16x4 x0 = lds_tr_read(vrd + 64 * (db ^ tr_x)), x1 = lds_tr_read(vrd + 8 * RSV + 64 * (db ^ tr_x));
+        return mma32(u16x8{x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]}, pf[u][k2], c);
+      };
+      if constexpr (FINE) {
 #pragma unroll
         for (int db = 0; db < NDB; ++db) {
-          const u16x4 x0 = lds_tr_read(vrd + 64 * (db ^ tr_x)), x1 = lds_tr_read(vrd + 8 * RSV + 64 * (db ^ tr_x));
-          acc[db] = mma32(u16x8{x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]}, pf[u][k2], acc[db]);
+          f32x16 o;
+#pragma unroll
+          for (int e = 0; e < 16; ++e) o[e] = 0.f;
+          o = product(db, 1, product(db, 0, o));
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[db][e] = __builtin_fmaf(o[e], beta, acc[db][e] * alpha);
         }
+      } else {
+#pragma unroll
+        for (int k2 = 0; k2 < 2; ++k2)
+#pragma unroll
+          for (int db = 0; db < NDB; ++db) acc[db] = product(db, k2, acc[db]);
       }
+    }
   };
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
@@ -870,7 +893,10 @@ int launch_wide(const hxm_biased_attn_args& a, hipStream_t s) {
   const int64_t slots = ((int64_t)a.n_tokens * R + 127) / 128 + a.n_seq, grid = (slots * a.kv_heads + 7) / 8 * 8;
   if (grid > 0x7fffffff) return HX_ERR_SHAPE;
   const bool mods = a.slopes || a.softcap > 0.f;
-  auto kernel = mods ? biased_attn_wide_kernel<D, V, true> : biased_attn_wide_kernel<D, V, false>;
+  // few rows: fewer tiles of 16 than the waves that the tile form's keys are dealt to (see its callers)
+  const bool fine = (int64_t)a.n_seq * a.kv_heads * (((int64_t)a.max_q_len * R + 15) / 16) < 2048;
+  auto kernel = fine ? (mods ? biased_attn_wide_kernel<D, V, true, true> : biased_attn_wide_kernel<D, V, false, true>)
+                     : (mods ? biased_attn_wide_kernel<D, V, true, false> : biased_attn_wide_kernel<D, V, false, false>);
   constexpr size_t lds = 2 * 64 * (2 * D + 2 * V);
   if (lds > 48 * 1024) {
     const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -1054,29 +1080,29 @@ __global__ __launch_bounds__(64) void biased_attn_step_kernel(hxm_biased_attn_ar
         mx = fmaxf(mx, s[e >> 2][e & 3]);
       }
     }
-    mx = groups_max(mx);
-    // (the weights always refer to the largest score so far: its own is then 1, which no rounding to bfloat16 touches)
-    const float m_new = fmaxf(m, mx * unit);
-    if (__builtin_amdgcn_ballot_w64(m_new > m)) {
-      const float alpha = fast_exp2(m - m_new);
-      l *= alpha;
-#pragma unroll
-      for (int i = 0; i < NDB; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[i][e] *= alpha;
-      m = m_new;
-    }
+    // A tile's weights refer to the tile's own largest score, which is then 1 and which no rounding to bfloat16 touches; what the tile
+    // adds is scaled behind its products.  (Bound by memory, this costs nothing; with weights that refer to the largest score so far and
+    // half as many splits as the tile form took, 32 tokens of 1025 - 2047 keys were off by 2.17e-3 of the result, 2.13 in the tile form.)
+    float m_tile = groups_max(mx) * unit;
+    asm("" : "+v"(m_tile));                  // (rounded: left inside the difference below it would not be m_new's number)
+    const float m_new = fmaxf(m, m_tile);
+    const float alpha = fast_exp2(m - m_new), beta = fast_exp2(m_tile - m_new);
+    m = m_new;
     u16x8 pf;
+    float l_tile = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const float p = fast_exp2(__builtin_fmaf(s[e >> 2][e & 3], unit, -m));
-      l += p;
+      const float p = fast_exp2(__builtin_fmaf(s[e >> 2][e & 3], unit, -m_tile));
+      l_tile += p;
       pf[e] = BF16::from_float(p);
     }
+    l = __builtin_fmaf(l, alpha, l_tile * beta);
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
       const u16x4 x0 = tr_read(va ^ (32u * db)), x1 = tr_read((va ^ (32u * db)) + 16u * RSV);
-      acc[db] = Mfma<BF16>::mma(u16x8{x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]}, pf, acc[db]);
+      const f32x4 o = Mfma<BF16>::mma(u16x8{x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]}, pf, f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[db][e] = __builtin_fmaf(o[e], beta, acc[db][e] * alpha);
     }
     // (reads stay a few products ahead)
     constexpr int kAhead = NDB < 6 ? NDB : 6;

@@ -780,6 +780,8 @@ __global__ __launch_bounds__(256) void latent_attn_group_kernel(hxm_latent_attn_
   }
 }
 
+constexpr int64_t kTileWaves = 2048;      // what the tile form deals a launch of few rows to: 8 waves a CU
+
 // ---------------------------------------------------------------------------------------------------------------
 // Wide form (bfloat16, portions of prompts, latents of 64 KK columns, pages of whole 16-row groups): a workgroup of four waves takes
 // 128 rows, 32 a wave, and goes over the keys in tiles of 64 whose rows go straight from the paged cache to LDS, the next tile's
@@ -788,17 +790,20 @@ __global__ __launch_bounds__(256) void latent_attn_group_kernel(hxm_latent_attn_
 // chunk x of row r sits at x ^ swz(r), with the row's two low bits above its next two, so that the 16 rows of one pass of a
 // 16-byte read as well as the four rows of a transposing read fall into different banks.
 // The tile and group forms read a row from LDS (or memory) once per 16 x 16 x 32 product; here a byte feeds twice the products.  A
-// lane holds 24 KK registers of queries and accumulators: two waves a SIMD up to 256 columns, one at 320; wider latents take the
-// form below.  (No register may spill here: the waits for scratch would be waits for the tile on its way.)
-// Measured, 4 portions of 1000 tokens: 256 columns, 16 heads 282 us in the tile form, 62 us here; 64 columns, 32 heads 141 and
-// 35 us; 320 columns under a window of 512, 16 heads 315 (group form) and 92 us.
+// lane holds 48 KK registers of queries and accumulators: two waves a SIMD up to 192 columns; wider latents take the form below.
+// (No register may spill here: the waits for scratch would be waits for the tile on its way.)
+// A row's weights refer to its largest score so far, which costs a pass over the accumulators for nearly every tile.  (Left up to 2^8
+// behind it, 64 columns took 35 us instead of 39, and results were off by 3 % more: the largest weights were rounded to bfloat16
+// instead of being 1.)
+// Measured, 4 portions of 797 - 1151 tokens, 32 heads: 64 columns 134 us in the tile form, 39 here, 128 columns 209 and 60, 192
+// columns 393 and 84.  256 columns, 16 heads 70 us in this form, 65 in the one below; 320 columns 120 and 76.
 // ---------------------------------------------------------------------------------------------------------------
 __device__ __forceinline__ f32x16 mma32(u16x8 a, u16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
 template <int KK>
-__global__ __launch_bounds__(256, KK <= 4 ? 2 : 1) void latent_attn_wide_kernel(hxm_latent_attn_args a) {
+__global__ __launch_bounds__(256, 2) void latent_attn_wide_kernel(hxm_latent_attn_args a) {
   constexpr int R = 64 * KK, KT = 64, TQ = 128, KS = R / 16, NDB = R / 32, RS = 2 * R, L = R / 8, IMG = KT * RS;
   constexpr bool FULL = RS % 256 == 0;       // a row is whole bank rows (256 bytes): 16 rows need 16 places, else 8 of each parity
   extern __shared__ __attribute__((aligned(256))) char smem_w[];       // [2][64 rows]
@@ -927,11 +932,10 @@ __global__ __launch_bounds__(256, KK <= 4 ? 2 : 1) void latent_attn_wide_kernel(
       }
     }
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    // a row keeps the maximum its weights refer to until a score exceeds it by 2^8
-    const float m_cand = fmaxf(m, mx * scale2);
-    const bool grow = m_cand > m + 8.0f;
-    if (__builtin_amdgcn_ballot_w64(grow)) {
-      const float m_new = grow ? m_cand : m, alpha = fast_exp2(m - m_new);
+    // (the weights always refer to the largest score so far: its own is then 1, which no rounding to bfloat16 touches)
+    const float m_new = fmaxf(m, mx * scale2);
+    if (__builtin_amdgcn_ballot_w64(m_new > m)) {
+      const float alpha = fast_exp2(m - m_new);
       l *= alpha;
 #pragma unroll
       for (int i = 0; i < NDB; ++i)
@@ -1010,19 +1014,20 @@ __global__ __launch_bounds__(256, KK <= 4 ? 2 : 1) void latent_attn_wide_kernel(
   }
 }
 
-// The same for wider latents (64 KK columns, KK even): four waves of 16 rows, 16 x 16 x 32 products — a row's queries and
+// The same for wider latents (64 KK columns): four waves of 16 rows, 16 x 16 x 32 products — a row's queries and
 // accumulators are 192 registers a lane at 512 columns, two waves a SIMD.  A byte from LDS feeds half the products of the form
 // above; it is bound by the latency and number of its LDS reads (without those of the keys the same launch takes three quarters of
 // the time).  Tiles of 32 keys and 64 rows: two workgroups a CU, one working while the other brings queries in or results out.  Also
 // the form for few rows, decode steps first: the keys of a row tile are then dealt to several workgroups (wide_plan), each writes
 // its rows' sums, maximum and weight, and the kernel below merges them.
-// Measured, 4 portions of 797 - 1151 tokens, 32 heads, 512 columns: 861 us in the group form, 226 us here (560 TFLOP/s; 780
-// behind long contexts, where less of the time goes to queries and results).  32 tokens of 301 - 1747 keys, 32 heads, 512 columns
+// Measured, 4 portions of 797 - 1151 tokens, 32 heads, 512 columns: 861 us in the group form, 240 us here (530 TFLOP/s); 256
+// columns, 16 heads 268 and 65 us, 320 columns 396 and 76.  32 tokens of 301 - 1747 keys, 32 heads, 512 columns
 // under a window of 512: 31 us and 30 to merge in the tile form, 18 and 4.5 here, of which 6 pass before the first product and
-// about 5 are the splits' sums going out (8 MB); 1 token behind 1000 keys 70 us and 24, most of it the host's.  Row r of sixteen has its chunks at x ^ swz(r): rows r and 15 - r share a 32-byte place (their
+// about 5 are the splits' sums going out (8 MB); 1 token behind 1000 keys 70 us and 24, most of it the host's.
+// Row r of sixteen has its chunks at x ^ swz(r): rows r and 15 - r share a 32-byte place (their
 // chunks turned), so that a pass of a 16-byte read (rows 0-3 and 12-15 of one chunk, 4-11 of the next) and a transposing read
 // (eight rows, 32 bytes each) both reach every bank once.
-template <int KK>
+template <int KK, bool FINE>      // FINE: every tile's weights refer to their own largest score
 __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_attn_args a, int tiles_per_seq) {
   constexpr int R = 64 * KK, KT = 32, TQ = 64, KPW = 8, KS = R / 32, NDB = R / 16, RS = 2 * R, L = R / 8, IMG = KT * RS;
   constexpr bool FULL = RS % 256 == 0;       // rows of whole bank rows: 16 places of a chunk, else 8 for each parity of the row
@@ -1035,7 +1040,7 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
   typedef __attribute__((address_space(4))) const int32_t c_i32;       // (uniform indices: through the scalar cache)
   c_i32* q_cu = (c_i32*)a.q_cu;
   const int H = a.n_heads;
-  const int n_splits = a.n_splits > 1 ? a.n_splits : 1, split = n_splits > 1 ? (int)(blockIdx.x % n_splits) : 0;
+  const int n_splits = FINE && a.n_splits > 1 ? a.n_splits : 1, split = n_splits > 1 ? (int)(blockIdx.x % n_splits) : 0;
   int b, tile, q0, n_rows;
   if (!find_row_tile<TQ>(q_cu, a.n_seq, H, (int)(n_splits > 1 ? blockIdx.x / n_splits : blockIdx.x), b, tile, q0, n_rows)) return;      // spare slot (the grid is an upper bound)
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -1097,7 +1102,6 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
     for (int ks = 0; ks < KS; ++ks) qf[ks] ^= (u16)0x8000;
   }
   scale2 = fabsf(scale2) < 1e-30f ? 1e-30f : fabsf(scale2);      // (not fmaxf: what is not a number stays so)
-  const float lag = n_splits > 1 ? 0.f : 8.0f;
   f32x4 acc[NDB];
 #pragma unroll
   for (int i = 0; i < NDB; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1150,31 +1154,45 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
       }
     }
     mx = groups_max(mx);
-    // a row keeps the maximum its weights refer to until a score exceeds it by 2^8 (where the keys are dealt out, and few steps
-    // are taken, by nothing: the largest weight is then 1, which no rounding to bfloat16 touches)
-    const float m_cand = fmaxf(m, mx * scale2);
-    const bool grow = m_cand > m + lag;
-    if (__builtin_amdgcn_ballot_w64(grow)) {
-      const float m_new = grow ? m_cand : m, alpha = fast_exp2(m - m_new);
+    // The weights refer to the largest score so far, as above — or, in launches of few rows, to the largest of these 32 keys, and what
+    // they add is scaled behind the products: the tile form deals such a launch's keys to more waves, each with a largest score that
+    // weighs exactly 1 (32 tokens of 301 - 1747 keys, 2-norm of the error over the result: 1.909e-3 there, 1.933e-3 with its own splits' largest
+    // scores here, 1.900e-3 with every 32 keys').
+    float m_ref = mx * scale2;
+    asm("" : "+v"(m_ref));                   // (rounded: left inside a difference below it would not be m_new's number)
+    const float m_new = fmaxf(m, m_ref), alpha = fast_exp2(m - m_new), beta = fast_exp2(m_ref - m_new);
+    if constexpr (FINE) {
       l *= alpha;
+    } else {
+      m_ref = m_new;
+      if (__builtin_amdgcn_ballot_w64(m_new > m)) {
+        l *= alpha;
 #pragma unroll
-      for (int i = 0; i < NDB; ++i)
+        for (int i = 0; i < NDB; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[i][e] *= alpha;
-      m = m_new;
+          for (int e = 0; e < 4; ++e) acc[i][e] *= alpha;
+      }
     }
+    m = m_new;
     u16x8 pf;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const float p = fast_exp2(__builtin_fmaf(s[e >> 2][e & 3], scale2, -m));
-      l += p;
+      const float p = fast_exp2(__builtin_fmaf(s[e >> 2][e & 3], scale2, -m_ref));
+      l = FINE ? __builtin_fmaf(p, beta, l) : l + p;
       pf[e] = BF16::from_float(p);
     }
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
       const uint32_t at = (va ^ (32u * (db % (2 * NP)))) + 64u * NP * (db / (2 * NP));
       const u16x4 x0 = tr_read(at), x1 = tr_read(at + 16u * RS);
-      acc[db] = Mfma<BF16>::mma(u16x8{x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]}, pf, acc[db]);
+      const u16x8 x = u16x8{x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+      if constexpr (FINE) {
+        const f32x4 o = Mfma<BF16>::mma(x, pf, f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[db][e] = __builtin_fmaf(o[e], beta, acc[db][e] * alpha);
+      } else {
+        acc[db] = Mfma<BF16>::mma(x, pf, acc[db]);
+      }
     }
     constexpr int kAheadV = NDB < 6 ? NDB : 6;
     __builtin_amdgcn_sched_group_barrier(0x100, 2 * kAheadV, 0);
@@ -1309,7 +1327,7 @@ WidePlan wide_plan(const hxm_latent_attn_args& a) {
     return p;
   p.fits = true;
   const int64_t rows = (int64_t)a.max_q_len * a.n_heads;
-  p.rows32 = a.kv_rank <= 320 && a.n_seq * ((rows + 127) / 128) >= 256;
+  p.rows32 = a.kv_rank <= 192 && a.n_seq * ((rows + 127) / 128) >= 256;
   if (p.rows32) return p;
   int reach = a.max_kv_len;
   if (a.window > 0 && a.window + a.max_q_len < reach) reach = a.window + a.max_q_len;
@@ -1332,8 +1350,11 @@ int launch_wide16(const hxm_latent_attn_args& a, hipStream_t s) {
   const int64_t grid = (((int64_t)a.n_tokens * a.n_heads + 63) / 64 + a.n_seq) * n_splits;      // row tiles of all sequences, at most
   if (grid > 0x7fffffff) return HX_ERR_SHAPE;
   constexpr size_t lds = 2 * 32 * 2 * 64 * KK;
-  if (const int rc = prepare_lds((const void*)latent_attn_wide16_kernel<KK>, lds)) return rc;
-  latent_attn_wide16_kernel<KK><<<dim3((unsigned)grid), dim3(256), lds, s>>>(a, tiles16);
+  // (few rows: where the tile form would deal out the keys)
+  const bool fine = n_splits > 1 || (int64_t)a.n_seq * tiles16 < kTileWaves;
+  auto kernel = fine ? latent_attn_wide16_kernel<KK, true> : latent_attn_wide16_kernel<KK, false>;
+  if (const int rc = prepare_lds((const void*)kernel, lds)) return rc;
+  kernel<<<dim3((unsigned)grid), dim3(256), lds, s>>>(a, tiles16);
   if (n_splits > 1) {
     int lanes_log2 = 4;                      // a row to R / 4 lanes, at most a power of two of them
     while ((8 << lanes_log2) <= a.kv_rank && lanes_log2 < 7) ++lanes_log2;
@@ -1346,7 +1367,7 @@ int launch_wide16(const hxm_latent_attn_args& a, hipStream_t s) {
 template <int KK>
 int launch_wide(const hxm_latent_attn_args& a, const WidePlan& p, hipStream_t s) {
   if (a.n_splits > 1 && (a.n_splits > 64 || !a.ws_o || !a.ws_ml)) return HX_ERR_WORKSPACE;
-  if constexpr (KK <= 5) {
+  if constexpr (KK <= 3) {
     if (p.rows32) {
       const int64_t grid = ((int64_t)a.n_tokens * a.n_heads + 127) / 128 + a.n_seq;
       if (grid > 0x7fffffff) return HX_ERR_SHAPE;
@@ -1403,7 +1424,7 @@ static int tile_splits(const hxm_latent_attn_args& a) {
   int reach = a.max_kv_len > 0 ? a.max_kv_len : 1;
   if (a.window > 0 && a.window + a.max_q_len < reach) reach = a.window + a.max_q_len;
   const int chunks = (reach + 31) / 32;
-  int64_t want = (2048 + items - 1) / items;      // ~8 waves per CU
+  int64_t want = (kTileWaves + items - 1) / items;
   if (want > chunks / 2) want = chunks / 2;          // at least two chunks a split
   if (want > 64) want = 64;
   return want < 2 ? 1 : (int)want;

@@ -162,3 +162,33 @@ def test_a_sequence_without_keys(n, divided):
     alone = run(q[n:].contiguous(), own, [0, n], [0, 30], [0] * n)
     assert (got[:n] == 0).all()                                   # the sink takes all the weight
     assert float((got[n:].double() - alone.double()).norm() / alone.double().norm()) < 2.0 ** -7      # (keys may be dealt out otherwise)
+
+
+# (sequences, tokens brought, tokens held)
+@pytest.mark.parametrize("n, new, kv", [(2, 64, 64), (2, 250, 300), (1, 200, 700), (64, 1, 900)])
+@pytest.mark.parametrize("extra", ["plain", "slopes", "cap"])
+def test_weights_round_no_more_than_in_the_tile_form(n, new, kv, extra):
+    # The tile form's weights refer to the largest score so far, 32 keys at a time.  So do the wide form's, and round alike; the step
+    # form's refer to the largest of their own 32, and are compared over 2048 rows (two roundings of one row differ by a fifth or so).
+    from hydrainfer_amd._C.kernel.biased_attn import biased_attention
+    H, G, D = 32, 8, 128
+    g = torch.Generator().manual_seed(n + new + kv)
+    nb = (kv + BLOCK - 1) // BLOCK
+    r = lambda *s: torch.randn(s, generator=g).bfloat16()
+    i = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    q, kc, vc = r(n * new, H, D), r(n * nb, BLOCK, G, D), r(n * nb, BLOCK, G, D)
+    slopes, cap = torch.tensor([2.0 ** (-8.0 * (h + 1) / H) for h in range(H)]) if extra == "slopes" else None, 30.0 if extra == "cap" else 0.0
+    pos = list(range(kv - new, kv))
+    want = []
+    for s in range(n):
+        k, v = (x[s * nb:(s + 1) * nb].reshape(-1, G, D)[:kv].double().repeat_interleave(H // G, dim=1) for x in (kc, vc))
+        want.append(_reference(q[s * new:(s + 1) * new].double(), k, v, pos, torch.full((H,), D ** -0.5, dtype=torch.float64),
+                               None if slopes is None else slopes.double(), "causal", 0, cap, None)[0])
+    want = torch.cat(want)
+    off = {}
+    for form in ("auto", "tile"):
+        got = biased_attention(q.cuda(), kc.cuda(), vc.cuda(), D, i([s for s in range(n) for _ in pos]), i(pos * n), i([s * new for s in range(n + 1)]), i(list(range(n * nb))),
+                               i([s * nb for s in range(n + 1)]), D ** -0.5, None if slopes is None else slopes.cuda(), "causal", 0, max_q_len=new, max_kv_len=kv,
+                               softcap=cap, form=form).double().cpu()
+        off[form] = float((got - want).norm() / want.norm())
+    assert off["auto"] <= (1.0 if new == 1 else 1.005) * off["tile"], off

@@ -148,3 +148,35 @@ def test_rows_past_max_q_len_have_no_place_in_the_workspace():
     a.n_splits, a.ws_o, a.ws_ml = splits.value, ws_o.data_ptr(), ws_ml.data_ptr()
     _lib.mix_check(_lib.mix_lib().hxm_latent_attention(ctypes.byref(a), _lib.current_stream()), "latent_attention")
     assert (ws_o[n_o:] == 7.0).all() and (ws_ml[floats.value - n_o:] == 7.0).all()
+
+
+# (sequences, tokens brought, tokens held)
+@pytest.mark.parametrize("n, new, kv", [(2, 60, 60), (8, 140, 300), (64, 1, 900), (4, 16, 516)])
+@pytest.mark.parametrize("R", [64, 256, 512])
+def test_weights_round_no_more_than_in_the_tile_form(n, new, kv, R):
+    # The tile form's weights refer to the largest score so far, 32 keys at a time.  So do the wide forms', and round alike; where the keys
+    # are dealt out they refer to the largest of their own 32, and are compared over 2048 rows (two roundings of one row differ by a
+    # fifth or so).
+    from hydrainfer_amd import _lib
+    from hydrainfer_amd._C.kernel.latent_attn import latent_attention
+    H, nb = 32, (kv + BLOCK - 1) // BLOCK
+    g = torch.Generator().manual_seed(R + n + new + kv)
+    i = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    q, cache = torch.randn((n * new, H, R), generator=g).bfloat16(), torch.randn((n * nb, BLOCK, 1, R), generator=g).bfloat16()
+    pos = list(range(kv - new, kv))
+    seen = torch.tensor(pos)[:, None] >= torch.arange(kv)[None, :]
+    want = []
+    for s in range(n):
+        k = cache[s * nb:(s + 1) * nb].reshape(-1, R)[:kv].double()
+        z = torch.matmul(q[s * new:(s + 1) * new].double(), k.t()) * R ** -0.5
+        want.append(torch.matmul(torch.softmax(z.masked_fill(~seen[:, None], -math.inf), dim=2), k))
+    want, off = torch.cat(want), {}
+    try:
+        for form in (1, 2):
+            _lib.mix_lib().hxm_set_option(b"attn_tile_form", form)
+            got = latent_attention(q.cuda(), cache.cuda(), i([s for s in range(n) for _ in pos]), i(pos * n), i([s * new for s in range(n + 1)]), i(list(range(n * nb))),
+                                   i([s * nb for s in range(n + 1)]), R ** -0.5, None, new, max_kv_len=kv).double().cpu()
+            off[form] = float((got - want).norm() / want.norm())
+    finally:
+        _lib.mix_lib().hxm_set_option(b"attn_tile_form", 1)
+    assert off[1] <= (1.0 if new < 20 else 1.005) * off[2], off
