@@ -107,6 +107,37 @@ __device__ __forceinline__ void wave_lds_sync() {
 // a score under a soft cap: cap * tanh(s / cap); cap 0: the score itself
 __device__ __forceinline__ float capped(float s, float cap) { return cap > 0.f ? cap * tanhf(s / cap) : s; }
 
+// tanh(y) as exact near 0 as elsewhere, for y within kCapNear: an odd polynomial (its even part fitted to equal relative error, 5e-9); any y:
+// beyond it 1 - 2 / (1 + e^(2 |y|)) with y's sign.  (That form near 0 is off by a share of the cap and not of the score.)
+constexpr float kCapNear = 0.625f;
+__device__ __forceinline__ float tanh_near(float y) {
+  const float t = y * y;
+  const float p = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(__builtin_fmaf(-0.00570500642f, t, 0.0206391029f), t, -0.0537397191f), t, 0.133314416f), t, -0.333332807f);
+  return __builtin_fmaf(y * t, p, y);
+}
+__device__ __forceinline__ float tanh_any(float y) {
+  const float far = __builtin_fmaf(-2.f, __builtin_amdgcn_rcpf(1.f + fast_exp2(fabsf(y) * 2.8853900817779268f)), 1.f);
+  return fabsf(y) < kCapNear ? tanh_near(y) : copysignf(far, y);
+}
+// N scores times unit under a cap, times cap2.  Scores far below the cap are the rule: nothing but the polynomial then (4 portions of 797
+// - 1151 tokens, 32 / 8 heads of 128, window of 512: no cap 56 us, a cap of 30 68 us, a cap of 1, which takes both ways, 87).
+template <int N, typename S>
+__device__ __forceinline__ void cap_scores(S& s, float unit, float cap2) {
+  float top = 0.f;
+#pragma unroll
+  for (int e = 0; e < N; ++e) {
+    s[e] *= unit;
+    top = fmaxf(top, fabsf(s[e]));
+  }
+  if (__builtin_amdgcn_ballot_w64(top >= kCapNear)) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) s[e] = tanh_any(s[e]) * cap2;
+  } else {
+#pragma unroll
+    for (int e = 0; e < N; ++e) s[e] = tanh_near(s[e]) * cap2;
+  }
+}
+
 // D[32 x 32] += A[32 x 16] B[16 x 32]; lane (c = l % 32, h = l / 32): A[c][8 h + j], B[8 h + j][c], D[(e & 3) + 8 (e / 4) + 4 h][c]
 __device__ __forceinline__ f32x16 mma32(u16x8 a, u16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
@@ -606,8 +637,8 @@ __global__ __launch_bounds__(256) void biased_attn_group_kernel(hxm_biased_attn_
 // The order of the row tiles: the XCDs (workgroups are dealt round robin) take key heads of their own where there are enough of
 // them, and of every sequence the tiles with the most keys come first.
 // Measured, 4 portions of 797 - 1151 tokens, 32 heads of 128 on 8 key heads, sinks: 221 us in the group form, 57 us
-// here (570 TFLOP/s of the pairs that a mask leaves); window of 512 and soft cap 223 and 58 us; chunks of 512 and slopes 163 and
-// 45 us.  Down to 64 rows of a key head it is the faster one (16 tokens behind 500 keys: 30 and 21 us).
+// here (570 TFLOP/s of the pairs that a mask leaves); window of 512 and soft cap 223 and 68 us; chunks of 512 and slopes 163 and
+// 50 us.  Down to 64 rows of a key head it is the faster one (16 tokens behind 500 keys: 30 and 21 us).
 // ---------------------------------------------------------------------------------------------------------------
 template <int D, int V, bool MODS, bool FINE>      // MODS: slopes or a soft cap; FINE: every 32 keys' weights refer to their own largest score
 __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_attn_args a, int tile_slots) {
@@ -703,7 +734,7 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
   const float slope2 = MODS && a.slopes ? a.slopes[head] * kLog2e : 0.f;
   const bool cap = MODS && a.softcap > 0.f;
   const float cap2 = cap ? a.softcap * kLog2e : 0.f;
-  float scale2 = cap ? 2.f * kLog2e * hsc / a.softcap : hsc * kLog2e;
+  float scale2 = cap ? hsc / a.softcap : hsc * kLog2e;
   if (!MODS) {             // (a maximum of scores is one of scaled scores where the scale is positive; -inf times it stays -inf)
     if (scale2 < 0.f) {
 #pragma unroll
@@ -758,10 +789,7 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
       unit = 1.f;
       if (cap) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-          for (int e = 0; e < 16; ++e)       // cap2 tanh(y) = cap2 - 2 cap2 / (1 + e^(2 y))
-            s[u][e] = __builtin_fmaf(-2.f * cap2, __builtin_amdgcn_rcpf(1.f + fast_exp2(s[u][e] * scale2)), cap2);
+        for (int u = 0; u < 2; ++u) cap_scores<16>(s[u], scale2, cap2);
       } else {
 #pragma unroll
         for (int u = 0; u < 2; ++u)
@@ -1015,7 +1043,7 @@ __global__ __launch_bounds__(64) void biased_attn_step_kernel(hxm_biased_attn_ar
   // scores in units of log2: z = scale2 s - slope2 (pos - key), or under a cap cap2 tanh(s hsc / cap) in its place
   const bool cap = MODS && a.softcap > 0.f;
   const float cap2 = cap ? a.softcap * kLog2e : 0.f;
-  float scale2 = cap ? 2.f * kLog2e * hsc / a.softcap : hsc * kLog2e;
+  float scale2 = cap ? hsc / a.softcap : hsc * kLog2e;
   if (!MODS) {             // (a maximum of scores is one of scaled scores where the scale is positive; -inf times it stays -inf)
     if (scale2 < 0.f) {
 #pragma unroll
@@ -1059,12 +1087,13 @@ __global__ __launch_bounds__(64) void biased_attn_step_kernel(hxm_biased_attn_ar
     if (MODS) {
       unit = 1.f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        float z = s[e >> 2][e & 3];
-        // cap2 tanh(y) = cap2 - 2 cap2 / (1 + e^(2 y))
-        z = cap ? __builtin_fmaf(-2.f * cap2, __builtin_amdgcn_rcpf(1.f + fast_exp2(z * scale2)), cap2) : z * scale2;
-        if (a.slopes) z += slope2 * (float)(key_l + 16 * (e >> 2) + (e & 3) - pos);
-        s[e >> 2][e & 3] = z;
+      for (int u = 0; u < 2; ++u) {
+        if (cap) cap_scores<4>(s[u], scale2, cap2);
+        else s[u] *= scale2;
+      }
+      if (a.slopes) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[e >> 2][e & 3] += slope2 * (float)(key_l + 16 * (e >> 2) + (e & 3) - pos);
       }
     }
     float mx = HX_NEG_BIG;

@@ -96,7 +96,7 @@ def check(new, kv, H, G, D, V, mask, size, extra, divided=True, unseen=False):
     q = r(T, H, D)
     q[0] *= 20                    # a row whose weights sit on one key
     slopes = torch.tensor([2.0 ** (-8.0 * (h + 1) / H) for h in range(H)]) if extra == "slopes" else None
-    cap = 4.0 if extra == "cap" else 0.0
+    cap = 4.0 if extra == "cap" else 1e5 if extra == "a cap far above the scores" else 0.0
     temps = sinks = None
     if extra == "temperatures and sinks":
         temps, sinks = torch.randn(H, generator=g), 2 * torch.randn(H, generator=g)
@@ -124,6 +124,13 @@ def check(new, kv, H, G, D, V, mask, size, extra, divided=True, unseen=False):
                                  None if sinks is None else sinks.double())
         off = (got[lo:hi] - want).abs()
         assert bool((off <= bound).all()), (s, float((off - bound).max()))
+
+
+# a score is rounded as itself, not as a share of the cap (1e5 / 2^24 would move a weight by 1 %)
+@pytest.mark.parametrize("batch", [[(64, 65), (1, 200)], [(300, 1100)] * 8, [(1, 32), (1, 1025)]], ids=lambda b: f"{len(b)}x{max(b)}")
+@pytest.mark.parametrize("H, G, D, V", [(4, 1, 128, 128), (32, 8, 64, 64)])
+def test_a_cap_far_above_the_scores(batch, H, G, D, V):
+    check([a for a, _ in batch], [b for _, b in batch], H, G, D, V, "causal", 0, "a cap far above the scores")
 
 
 @pytest.mark.parametrize("new, kv", [([40, 16], [40, 300]), ([1, 1], [40, 300])])
