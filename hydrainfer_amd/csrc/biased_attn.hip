@@ -797,11 +797,11 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
           for (int e = 0; e < 16; ++e) s[u][e] *= scale2;
       }
       if (a.slopes) {
-        const float base = slope2 * (float)(key_l - pos);
+        const float near = (float)(key_l - pos);             // (the distance itself is exact: a key at distance 0 loses nothing)
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
-          for (int e = 0; e < 16; ++e) s[u][e] += __builtin_fmaf(slope2, (float)(32 * u + (e & 3) + 8 * (e >> 2)), base);
+          for (int e = 0; e < 16; ++e) s[u][e] = __builtin_fmaf(slope2, near + (float)(32 * u + (e & 3) + 8 * (e >> 2)), s[u][e]);
       }
     }
     if (!(t * KT + KT - 1 <= wpos0 && t * KT >= wlo1)) {      // (else every row of the wave sees the whole tile)

@@ -95,10 +95,12 @@ def check(new, kv, H, G, D, V, mask, size, extra, divided=True, unseen=False):
     T, kc, vc = sum(new), r(sum(nb) + 1, BLOCK, G, hs), r(sum(nb) + 1, BLOCK, G, hs)
     q = r(T, H, D)
     q[0] *= 20                    # a row whose weights sit on one key
-    slopes = torch.tensor([2.0 ** (-8.0 * (h + 1) / H) for h in range(H)]) if extra == "slopes" else None
-    cap = 4.0 if extra == "cap" else 1e5 if extra == "a cap far above the scores" else 0.0
+    slopes = torch.tensor([2.0 ** (-8.0 * (h + 1) / H) for h in range(H)]) if "slopes" in extra else None
+    if "steep" in extra:
+        slopes *= 1e5
+    cap = 1e5 if extra == "a cap far above the scores" else 4.0 if "cap" in extra else 0.0
     temps = sinks = None
-    if extra == "temperatures and sinks":
+    if "temperatures and sinks" in extra:
         temps, sinks = torch.randn(H, generator=g), 2 * torch.randn(H, generator=g)
         temps[0], sinks[1] = 0.0, -math.inf
     cu_b = torch.tensor([0] + nb).cumsum(0).int()
@@ -124,6 +126,16 @@ def check(new, kv, H, G, D, V, mask, size, extra, divided=True, unseen=False):
                                  None if sinks is None else sinks.double())
         off = (got[lo:hi] - want).abs()
         assert bool((off <= bound).all()), (s, float((off - bound).max()))
+
+
+# slopes, a cap, temperatures and sinks at once; and slopes so steep that the token's own key and the sink share the weights: that key is
+# at distance 0, where no slope adds a rounding
+@pytest.mark.parametrize("batch", [[(64, 65), (1, 200), (32, 32)], [(129, 129)], [(3, 70), (1, 16), (7, 2300)]], ids=lambda b: f"{len(b)}x{max(b)}")
+@pytest.mark.parametrize("H, G, D, V", [(4, 1, 128, 128), (32, 8, 64, 64), (6, 2, 128, 64)])
+@pytest.mark.parametrize("mask, size, extra", [("window", 63, "slopes and cap"), ("causal", 0, "slopes, cap, temperatures and sinks"),
+                                               ("causal", 0, "steep slopes, temperatures and sinks")])
+def test_slopes_with_the_other_extras(batch, H, G, D, V, mask, size, extra):
+    check([a for a, _ in batch], [b for _, b in batch], H, G, D, V, mask, size, extra)
 
 
 # a score is rounded as itself, not as a share of the cap (1e5 / 2^24 would move a weight by 1 %)
