@@ -732,9 +732,11 @@ extern "C" int hxm_router_topk(const float* x, int64_t x_stride, const float* w,
   if (x_stride < k_dim || x_stride % 4 || !aligned16(x) || !aligned16(w)) return HX_ERR_STRIDE;
   const dim3 grid((unsigned)((n_tokens + 15) / 16));
   hipStream_t s = (hipStream_t)stream;
-  // A workgroup a token while the CUs take them in one round, two where an expert's row is soon read (above / a workgroup a token:
-  // 16 experts of 4096, 256 tokens 17.4 / 7.3 us, 512 17.5 / 11.7, 1024 17.7 / 20.7; 128 of 1024, 256 21.4 / 20.2, 384 21.6 / 35.1).
-  if (n_tokens <= (n_experts <= 32 ? 512 : 256)) {
+  // A workgroup a token while the CUs take them in one round, two where the form above takes long (above / a workgroup a token:
+  // 16 experts of 4096, 256 tokens 17.4 / 7.3 us, 512 17.5 / 11.7, 1024 17.7 / 20.7; 32 of 2048, 512 13.9 / 12.0; 32 of 1024, 256 8.5 /
+  // 7.5, 384 8.5 / 11.3; 128 of 1024, 256 21.1 / 20.5, 384 21.6 / 35.1).  Every token reads all experts' rows then, and short rows are
+  // soon multiplied there: 128 of 512, 32 tokens 12.8 / 18.1, 32 of 512 5.7 / 6.6, 16 of 512 5.0 / 4.9.
+  if (k_dim >= 1024 && n_tokens <= (n_experts <= 32 && k_dim >= 2048 ? 512 : 256)) {
     router_few_kernel<<<dim3((unsigned)n_tokens), dim3(1024), 0, s>>>(x, x_stride, w, bias, k_dim, n_experts, top, weights, experts);
     return hxm::check_launch();
   }

@@ -6,8 +6,8 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("K", [4, 260, 2052])
-@pytest.mark.parametrize("E, T", [(16, 1), (16, 512), (16, 513), (33, 256), (33, 257), (128, 256), (128, 300)])
+@pytest.mark.parametrize("K", [4, 260, 1020, 1028, 2052])
+@pytest.mark.parametrize("E, T", [(16, 1), (16, 256), (16, 257), (16, 512), (16, 513), (33, 256), (33, 257), (128, 256), (128, 300)])
 @pytest.mark.parametrize("biased", [True, False])
 def test_router_forms(K, E, T, biased):
     from hydrainfer_amd._C.kernel.moe_mix import router_topk
