@@ -349,8 +349,13 @@ extern "C" int hxm_gated_recurrence(void* out, const void* q_pre, int64_t q_stri
   if (ws_floats < (int64_t)a.n_parts * n_tokens * heads * vdim) return HX_ERR_WORKSPACE;
   hipStream_t s = (hipStream_t)stream;
   if (dtype != HX_F32 && dtype != HX_BF16) return HX_ERR_DTYPE;
-  // (32 portions of two tokens, 32 heads of 128 x 128: 75 us token by token, 55 us in chunks)
-  if (max_q_len != 1) {
+  // Chunks from this longest portion on: a chunk costs its sixteen tokens and 64 or 128 by 64 channels however many there are (32 portions,
+  // token by token and in chunks, us: 32 heads of 128 x 128, which have a workgroup a CU and more, two tokens 75 and 55; 1 portion of
+  // 8 and 24 tokens 10 11, 14 13; 32 heads of 64 x 64, six and twelve 22 22, 27 22; 16 x 16, 24 and 64 18 26, 38 38; 32 x 32, 12 and
+  // 24 17 20, 26 27; 8 heads of 32 x 32, 256 workgroups, four and twelve 8 9, 10 9).
+  const int64_t groups = (int64_t)n_seq * heads * a.n_cw;
+  const int chunks_from = dim > 64 ? (groups >= 256 ? 2 : 16) : dim > 32 || groups < 512 ? 8 : dim > 16 ? 24 : 64;
+  if (max_q_len < 1 || max_q_len >= chunks_from) {
     hxm::ChunkScanArgs c{};
     c.out = ws; c.q = q_pre; c.k = f_pre; c.v = v;
     c.q_stride = q_stride; c.k_stride = f_stride; c.v_stride = v_stride;

@@ -206,6 +206,17 @@ def test_not_finite_numbers_in_the_gated_recurrence(what):
 @pytest.mark.parametrize("K, V", [(64, 64), (128, 128), (12, 20), (100, 130), (65, 7)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_portions_through_the_gated_recurrence(lens, K, V, dtype):
+    _through_the_gated_recurrence(lens, K, V, dtype)
+
+
+# the longest portion at which chunks begin: 8 and 16 tokens (24 and 64 where small states fill the chip, 2 where large ones do)
+@pytest.mark.parametrize("lens, K, V", [([7, 2], 64, 64), ([8, 2], 64, 64), ([15, 2], 128, 64), ([16, 2], 128, 64), ([23] + [2] * 180, 20, 12), ([24] + [2] * 180, 20, 12),
+                                        ([63] + [2] * 180, 16, 16), ([64] + [2] * 180, 16, 16), ([2] * 100, 65, 12)], ids=lambda v: f"{len(v)}x{v[0]}" if isinstance(v, list) else v)
+def test_portions_at_the_rule_of_the_gated_recurrence(lens, K, V):
+    _through_the_gated_recurrence(lens, K, V, torch.float32)
+
+
+def _through_the_gated_recurrence(lens, K, V, dtype):
     from hydrainfer_amd._C.kernel.recurrence import gated_recurrence
     from hydrainfer_amd._C.kernel.stream_ops import SequenceState
     g = torch.Generator().manual_seed(sum(lens) * 1000 + K + V)
@@ -239,7 +250,8 @@ def test_portions_through_the_gated_recurrence(lens, K, V, dtype):
     assert torch.equal(st[:, 0].cpu(), state[:, 0])
 
 
-def test_small_gates_are_as_exact_as_large_ones():
+@pytest.mark.parametrize("max_q_len", [0, 2])      # (in chunks, and a token at a time)
+def test_small_gates_are_as_exact_as_large_ones(max_q_len):
     # without values a state is the product of its gates; two of them, each off by a few units in the last place (2^-23) of its exponential,
     # sum and reciprocal
     from hydrainfer_amd._C.kernel.recurrence import gated_recurrence
@@ -252,7 +264,7 @@ def test_small_gates_are_as_exact_as_large_ones():
     seq = SequenceState(st, torch.zeros(1, dtype=torch.int32, device="cuda"), torch.zeros(T, dtype=torch.int32, device="cuda"))
     zero, p = torch.zeros(H * K, device="cuda"), proj.cuda()
     gated_recurrence(p[:, :H * K], p[:, H * K:2 * H * K], p[:, 2 * H * K:], zero, zero, torch.ones(V, device="cuda"), 1e-5, seq, 0,
-                     torch.tensor([0, T], dtype=torch.int32).cuda(), torch.tensor([5, 6], dtype=torch.int32).cuda(), H, K, V, max_q_len=T)
+                     torch.tensor([0, T], dtype=torch.int32).cuda(), torch.tensor([5, 6], dtype=torch.int32).cuda(), H, K, V, max_q_len=max_q_len)
     want = torch.sigmoid(proj[:, H * K:2 * H * K].double()).prod(0).view(H, K, 1)
     off = (st.double().cpu().view(H, K, V) - want).abs() / want
     assert float(off.max()) <= 8 * 2.0 ** -23, float(off.max())
