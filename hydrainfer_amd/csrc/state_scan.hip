@@ -495,8 +495,12 @@ extern "C" int hxm_state_scan(const hxm_state_scan_args* args, void* stream) {
   hipStream_t s = (hipStream_t)stream;
   // Portions of prompts go sixteen tokens at a time (chunk_scan.hip) where the sizes allow it, short ones one at a time here: a
   // chunk costs its sixteen however few tokens it holds.  Measured with 32 heads of 128 x 128 under the delta rule: 32 portions of
-  // two tokens 48 us here, 61 us in chunks; 16 of four 30 and 33; 8 of sixteen 26 and 22; 32 of 64 217 and 139.
-  if (a.n_tokens >= 6 * (int64_t)a.n_seq) {
+  // two tokens 48 us here, 61 us in chunks; 16 of four 30 and 33; 8 of sixteen 26 and 22; 32 of 64 217 and 139; one of six tokens 7 and 8.
+  // How the tokens are spread over the portions is not known here, and a long portion among single tokens is what chunks are for: 31
+  // single tokens and one portion of 200, 526 and 72 us, 32 heads of 16 x 16 50 and 34.  So chunks are also taken where equal portions
+  // would go faster here, small states that fill the chip: 32 portions of 64 tokens, 32 heads of 16 x 16 (padded to 64 x 64) 19 and
+  // 30 us, of six tokens 7 and 15; 64 x 64, 16 and 32 portions of six 9 and 11, 15 and 17.
+  if (a.n_tokens >= 6 * (int64_t)a.n_seq && a.n_tokens - a.n_seq >= 12) {      // (the longest portion may be of 13 tokens or more)
     hxm::ChunkScanArgs c{};
     c.out = a.out; c.q = a.q; c.k = a.k; c.v = a.v;
     c.q_stride = a.q_stride; c.k_stride = a.k_stride; c.v_stride = a.v_stride;

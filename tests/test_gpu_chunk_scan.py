@@ -91,6 +91,13 @@ def test_single_tokens_through_a_scan(lens, K, V, form, per_channel, types, pad)
     _through_a_scan(lens, K, V, form, per_channel, types, pad)
 
 
+# portions that may go either way: on both sides of the six tokens a sequence and of the thirteen that the longest may have
+@pytest.mark.parametrize("lens", [[12], [13], [5, 6], [6, 6], [1, 13], [7, 1, 10]])
+@pytest.mark.parametrize("form, per_channel", [("decay", False), ("decay", True), ("delta", False), ("bonus", True)])
+def test_portions_at_the_rule_between_the_forms(lens, form, per_channel):
+    _through_a_scan(lens, 40, 20, form, per_channel, "f32", 4)
+
+
 # portions that go a token at a time: short ones, and the forms and types that have no chunks; with few workgroups (more lanes a column)
 # and with many
 @pytest.mark.parametrize("lens", [[5], [3, 1, 2], [17, 33], [2] * 40], ids=lambda v: f"{len(v)}x{v[0]}")
