@@ -344,6 +344,7 @@ _MIX_SIGNATURES = {
                                       c_void_p, c_void_p, c_int64, c_int64, c_int32, c_int64, c_int, c_void_p]),
     "hxm_latent_attention": (c_int, [POINTER(hxm_latent_attn_args), c_void_p]),
     "hxm_latent_attention_plan": (c_int, [POINTER(hxm_latent_attn_args), POINTER(c_int32), POINTER(c_int64)]),
+    "hxm_latent_attention_form": (c_int, [POINTER(hxm_latent_attn_args)]),
     "hxm_embed_positions": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int64, c_int64, c_int64, c_int64,
                                     c_int, c_void_p]),
     "hxm_depth_norm": (c_int, [POINTER(hxm_depth_norm_args), c_void_p]),

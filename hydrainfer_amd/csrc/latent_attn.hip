@@ -1508,6 +1508,13 @@ extern "C" int hxm_latent_attention_plan(const hxm_latent_attn_args* args, int32
   return HX_OK;
 }
 
+extern "C" int hxm_latent_attention_form(const hxm_latent_attn_args* args) {
+  if (!args) return HX_ERR_NULL;
+  if (args->max_q_len < 1 || !tile_form_serves(*args)) return HXM_LATENT_ROW;
+  const WidePlan p = wide_plan(*args);
+  return !p.fits ? HXM_LATENT_TILE : p.rows32 ? HXM_LATENT_WIDE32 : HXM_LATENT_WIDE16;
+}
+
 extern "C" int hxm_latent_attention(const hxm_latent_attn_args* args, void* stream) {
   if (!args) return HX_ERR_NULL;
   const hxm_latent_attn_args& a = *args;

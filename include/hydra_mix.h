@@ -40,9 +40,10 @@ extern "C" {
 
 int hxm_abi_version(void);
 int hxm_last_hip_error(void);
-/* A/B measurements in one process: "attn_tile_form" = 0 keeps bfloat16 attention on the row form (one wave per token
- * and head) instead of the MFMA forms, 2 keeps portions of prompts on the tile form (one wave per 16 rows) instead of
- * the group form (four waves sharing every chunk of keys), 1 = the default.  Results agree within bfloat16 rounding. */
+/* A/B measurements in one process: "attn_tile_form" = 0 keeps bfloat16 attention over latents on the row form (one wave per
+ * token and head) instead of the MFMA forms, 2 keeps it on the tile form (one wave per 16 rows) instead of the wide forms (64 or
+ * 128 rows a workgroup, for single tokens too) and the group form (four waves sharing every chunk of keys), 1 = the default.
+ * Results agree within bfloat16 rounding. */
 int hxm_set_option(const char* name, int value);
 
 /* x[t, s, :] = table[ids[t], :] * scale for every stream s.  x: float [n_tokens, n_streams, width]; table: dtype
@@ -110,7 +111,7 @@ typedef struct hxm_latent_attn_args {
   float scale;
   int32_t dtype;
   int32_t max_kv_len;        /* the most keys a sequence of the batch holds (sizes the key splits) */
-  int32_t n_splits;          /* from hxm_latent_attention_plan; > 1: the key range of a row tile is dealt to n_splits waves */
+  int32_t n_splits;          /* from hxm_latent_attention_plan; > 1: the key range of a row tile is dealt to n_splits waves or workgroups */
   float* ws_o;               /* n_splits > 1: the plan's workspace, ws_floats floats; ws_ml = where its (max, sum) pairs go */
   float* ws_ml;
   const float* sinks;        /* [n_heads] or NULL: the softmax's denominator of head h holds one more term exp(sinks[h]), which
@@ -119,8 +120,15 @@ typedef struct hxm_latent_attn_args {
 
 /* How a launch with these arguments would be laid out: n_splits (1: no workspace) and the floats of workspace it needs
  * (ws_o = the first n_items * n_splits * 16 * ceil16(kv_rank) of them, ws_ml = the rest).  Pointers need not be set yet,
- * except q and cache (their alignment decides the form). */
+ * except q, cache and out (their alignment and strides decide the form). */
 int hxm_latent_attention_plan(const hxm_latent_attn_args* args, int32_t* n_splits, int64_t* ws_floats);
+
+#define HXM_LATENT_ROW 0       /* a wave a (token, head) */
+#define HXM_LATENT_TILE 1      /* tiles of 16 rows, or groups of four of them */
+#define HXM_LATENT_WIDE32 2    /* 128 rows a workgroup, 32 a wave */
+#define HXM_LATENT_WIDE16 3    /* 64 rows a workgroup, 16 a wave; with n_splits > 1 several workgroups a row tile */
+/* Which kernel hxm_latent_attention takes for these arguments (HX_ERR_NULL without any). */
+int hxm_latent_attention_form(const hxm_latent_attn_args* args);
 
 /* Softmax attention of every query over the latents of its own sequence in the paged cache (scores and weights in
  * float).  Queries of portions and single decoded tokens may share a batch. */
@@ -245,7 +253,8 @@ int hxm_moe_combine(void* out, const void* y, const int32_t* row_of, const float
  * last token.  q_cu: int32 [n_seq + 1]; positions: int32 [n_tokens]; slots: int32 [n_seq].  ws: float workspace of at least
  * hxm_gated_recurrence_workspace(n_tokens, heads, dim, vdim) floats (the partial results of the key channels' parts).
  * max_q_len: the longest portion of the batch if the caller knows it, else 0; 1 (every sequence brings one token) takes a
- * kernel without the chunk machinery. */
+ * kernel without the chunk machinery.  Longer portions of up to 128 key channels go sixteen tokens at a time through float matrix
+ * products, from a length on that depends on the sizes; what is said at hxm_state_scan holds for them. */
 int64_t hxm_gated_recurrence_workspace(int64_t n_tokens, int32_t heads, int32_t dim, int32_t vdim);
 int hxm_gated_recurrence(void* out, const void* q_pre, int64_t q_stride, const void* f_pre, int64_t f_stride, const void* v,
                          int64_t v_stride, const float* f_bias, const float* low, const float* norm_w, float eps,
@@ -289,8 +298,9 @@ typedef struct hxm_biased_attn_args {
   const int32_t* q_cu;       /* [n_seq + 1]: the tile form's portions */
   int32_t n_seq, max_q_len;  /* max_q_len: the longest portion of the batch (1: every sequence decodes) */
   int32_t form;              /* 0: the MFMA forms where they apply (bfloat16, sizes and strides multiples of 8), 1: the row form,
-                                2: the MFMA tile form also where the group form (four row tiles sharing each chunk) would run */
-  int32_t n_splits;          /* tile form, > 1: a tile's keys are dealt to n_splits waves (<= 64) and merged by a second kernel */
+                                2: the MFMA tile form also where the wide form (128 rows a workgroup), the step form (16 rows, whole
+                                key rows through LDS) or the group form (four row tiles sharing each chunk) would run */
+  int32_t n_splits;          /* tile and step form, > 1: a tile's keys are dealt to n_splits waves (<= 64) and merged by a second kernel */
   float* ws_o;               /* n_splits > 1: n_seq * kv_heads * ceil(max_q_len * heads / kv_heads / 16) * n_splits * 16 * ceil16(vdim) floats */
   float* ws_ml;              /* n_splits > 1: ... * n_splits * 32 floats */
   float softcap;             /* > 0: q . k * scale becomes softcap * tanh(q . k * scale / softcap) before the bias; 0: none */
@@ -495,8 +505,10 @@ typedef struct hxm_state_scan_args {
   int32_t n_seq, heads, qk_heads, dim, vdim, mode;
 } hxm_state_scan_args;
 
-/* The recurrence of one matrix state S [dim, vdim] per head and sequence, token by token in float, continued from and
- * left in the sequence's slot.  dim <= 256. */
+/* The recurrence of one matrix state S [dim, vdim] per head and sequence, continued from and left in the sequence's slot: token by
+ * token in float, or (portions of prompts, dim <= 128) sixteen tokens at a time as float matrix products, which round in other places
+ * and are no further from the exact result.  A value, scale or write strength that is not finite reaches later tokens of its own columns
+ * only, in either form; a key or decay that is not finite may leave NaN where a token at a time left an infinity.  dim <= 256. */
 int hxm_state_scan(const hxm_state_scan_args* args, void* stream);
 
 #define HXM_DECAY_CHUNK 32      /* tokens the chunked form of hxm_decay_attention takes at a time */

@@ -39,7 +39,8 @@ def _check(name, got, want, tol=TOL):
     assert float(off) <= tol, (name, float(off))
 
 
-LENS = [[17], [16, 1, 33], [1, 15, 31, 2], [48, 5]]
+# (rows are on their way three chunks ahead and pass through three images in LDS: both come round from the fourth chunk on)
+LENS = [[17], [16, 1, 33], [1, 15, 31, 2], [48, 5], [64, 113], [65, 300]]
 
 
 @pytest.mark.parametrize("lens", LENS)

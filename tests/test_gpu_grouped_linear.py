@@ -34,6 +34,15 @@ def test_grouped_linear_edges(rows, n, k, act):
     _check(rows, n, k, act, False)
 
 
+# more slices of 64 than a tile has slots for (three, or two with tiles of 256 rows), several turns of them, with a tail and without:
+# tiles of 32, 128 and 256 rows
+@pytest.mark.parametrize("rows", [[20, 0, 33], [128, 61], [300, 257]])
+@pytest.mark.parametrize("k", [256, 328, 1032])
+@pytest.mark.parametrize("act", ["none", "glu"])
+def test_grouped_linear_over_many_slices(rows, k, act):
+    _check(rows, 288, k, act, False)
+
+
 @pytest.mark.parametrize("rows", [[1, 30], [129, 0, 127], [256, 257]])
 def test_grouped_linear_of_rows_far_apart(rows):
     _check(rows, 160, 200, "none", True)

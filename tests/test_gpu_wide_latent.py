@@ -1,7 +1,8 @@
 """Latent attention over portions of prompts (csrc/latent_attn.hip, the wide forms: 64 to 320 columns, 384 and 512) at the edges of
 their tiles — 128 or 64 rows of token and head, 64 or 32 keys — with windows, sinks, gates, a negative scale, queries and results
-as views of other layouts; and over single tokens, whose keys are dealt to several workgroups."""
+as views of other layouts; and over single tokens, whose keys are dealt to several workgroups.  Every case says which form it is for."""
 import math
+from unittest import mock
 
 import pytest
 import torch
@@ -9,6 +10,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 BLOCK = 16
+WIDE32, WIDE16 = 2, 3           # 32 rows a wave, 16 rows a wave
 # (tokens brought, tokens held) of every sequence
 BATCHES = [[(2, 2)], [(33, 33), (2, 100)], [(5, 70), (1, 200), (32, 32)], [(129, 129)], [(40, 400), (5, 5), (16, 64), (31, 63), (17, 17)]]
 
@@ -20,7 +22,18 @@ def test_wide_forms(batch, R, H, window, extra):
     new, kv = [a for a, _ in batch], [b for _, b in batch]
     if max(new) * H < 64:
         new[0], kv[0] = 22, max(22, kv[0])
-    check(new, kv, R, H, window, extra)
+    check(new, kv, R, H, window, extra, WIDE16)
+
+
+# enough rows for 32 a wave (up to 192 columns), and for row tiles of 16 a wave that follow the largest score: several tiles a portion,
+# whole ones and partial ones, portions of one tile beside them
+MANY = [(130, 130), (1, 40), (129, 300), (128, 128), (131, 400), (97, 97), (133, 133), (64, 90)]
+
+
+@pytest.mark.parametrize("R", [64, 128, 192, 256, 320])
+@pytest.mark.parametrize("window, extra", [(0, "plain"), (1, "plain"), (64, "sinks and gate"), (31, "negative"), (0, "gate")])
+def test_wide_forms_of_many_rows(R, window, extra):
+    check([a for a, _ in MANY], [b for _, b in MANY], R, 32, window, extra, WIDE32 if R <= 192 else WIDE16)
 
 
 # single tokens: one tile and a split's edge, splits that get no tile (one sequence far shorter than another), more sequences than a
@@ -32,7 +45,7 @@ STEPS = [[64], [129, 1, 32, 33], [2000, 3], [700] * 5, [40] * 260 + [130]]
 @pytest.mark.parametrize("R", [64, 448, 512])
 @pytest.mark.parametrize("H, window, extra", [(1, 0, "plain"), (16, 0, "negative"), (16, 300, "sinks and gate"), (65, 300, "plain")])
 def test_single_tokens(kv, R, H, window, extra):
-    check([1] * len(kv), kv, R, H, window, extra)
+    check([1] * len(kv), kv, R, H, window, extra, WIDE32 if R <= 192 and len(kv) >= 256 else WIDE16)
 
 
 # Rows that no token of a portion sees are never read: pages left of a window may have been given back, and the rows of the last page
@@ -41,7 +54,7 @@ def test_single_tokens(kv, R, H, window, extra):
 @pytest.mark.parametrize("R", [64, 320, 512])
 @pytest.mark.parametrize("window", [300, 0])
 def test_rows_that_nobody_sees(new, kv, R, window):
-    check(new, kv, R, 32, window, "plain", unseen=True)
+    check(new, kv, R, 32, window, "plain", WIDE32 if R <= 192 and max(new) > 700 else WIDE16, unseen=True)
 
 
 def hide(cache, table, first, last):
@@ -55,7 +68,21 @@ def hide(cache, table, first, last):
             cache[page, (keys < first) | (keys > last)] = math.nan
 
 
-def check(new, kv, R, H, window, extra, unseen=False):
+class Spy:
+    """The library, noting which form every call takes."""
+    def __init__(self, lib):
+        self.lib, self.forms = lib, []
+
+    def __getattr__(self, name):
+        return getattr(self.lib, name)
+
+    def hxm_latent_attention(self, args, stream):
+        self.forms.append(self.lib.hxm_latent_attention_form(args))
+        return self.lib.hxm_latent_attention(args, stream)
+
+
+def check(new, kv, R, H, window, extra, form, unseen=False):
+    from hydrainfer_amd import _lib
     from hydrainfer_amd._C.kernel.latent_attn import latent_attention
     g = torch.Generator().manual_seed(R * 100 + H + window + sum(new) + sum(kv))
     nb = [(n + BLOCK - 1) // BLOCK for n in kv]
@@ -77,8 +104,11 @@ def check(new, kv, R, H, window, extra, unseen=False):
             rows = pos[int(cu_q[s]):int(cu_q[s + 1])]
             hide(shown, pages[int(cu_b[s]):int(cu_b[s + 1])], max(0, min(rows) - window + 1) if window else 0, max(rows))
     out = torch.full((H, T, R), 7.0, dtype=torch.bfloat16, device="cuda")
-    latent_attention(c(q).transpose(0, 1), c(shown), c(seq), c(torch.tensor(pos, dtype=torch.int32)), c(cu_q), c(pages), c(cu_b), scale, window or None,
-                     max(new), gate_pre=c(gate), out=out.transpose(0, 1), max_kv_len=max(kv), sinks=c(sinks))
+    spy = Spy(_lib.mix_lib())
+    with mock.patch.object(_lib, "mix_lib", lambda: spy):
+        latent_attention(c(q).transpose(0, 1), c(shown), c(seq), c(torch.tensor(pos, dtype=torch.int32)), c(cu_q), c(pages), c(cu_b), scale, window or None,
+                         max(new), gate_pre=c(gate), out=out.transpose(0, 1), max_kv_len=max(kv), sinks=c(sinks))
+    assert spy.forms == [form]
     got = out.double().cpu()
     for s in range(len(new)):
         lo, hi = int(cu_q[s]), int(cu_q[s + 1])
