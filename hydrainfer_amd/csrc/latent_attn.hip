@@ -1022,7 +1022,7 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide_kernel(hxm_latent_att
 // its rows' sums, maximum and weight, and the kernel below merges them.
 // Measured, 4 portions of 797 - 1151 tokens, 32 heads, 512 columns: 861 us in the group form, 240 us here (530 TFLOP/s); 256
 // columns, 16 heads 268 and 65 us, 320 columns 396 and 76.  32 tokens of 301 - 1747 keys, 32 heads, 512 columns
-// under a window of 512: 31 us and 30 to merge in the tile form, 18 and 4.5 here, of which 6 pass before the first product and
+// under a window of 512: 31 us and 30 to merge in the tile form, 20 and 4.5 here, of which 6 pass before the first product and
 // about 5 are the splits' sums going out (8 MB); 1 token behind 1000 keys 70 us and 24, most of it the host's.
 // Row r of sixteen has its chunks at x ^ swz(r): rows r and 15 - r share a 32-byte place (their
 // chunks turned), so that a pass of a 16-byte read (rows 0-3 and 12-15 of one chunk, 4-11 of the next) and a transposing read

@@ -387,8 +387,8 @@ __global__ __launch_bounds__(256) void grouped_linear_kernel(typename A::storage
 // column l % 16 of rows 4 (l / 16) .. + 3.  Half a slice is multiplied while the other half's operands are read from LDS, one
 // read between four products; the one workgroup barrier of a slice stands between its halves, so that a wave always has
 // products to issue behind it.
-// With many rows an expert it is bound by the matrix cores and LDS bandwidth (256 x 256: a byte read from LDS feeds 43
-// multiply-adds, 128 x 128 over four waves 32), with few by the weights: those of an expert with one row tile are read past
+// With many rows an expert it is bound by the matrix cores and LDS bandwidth (256 x 256: a byte read from LDS feeds 21
+// multiply-adds, 128 x 128 over four waves 16), with few by the weights: those of an expert with one row tile are read past
 // the caches.  Measured with 16 experts, 2 x 2752 outputs of 4096 and back: 15956 rows 866 + 444 us through registers in
 // tiles of 128 x 128 and padded LDS rows, 671 + 383 us here (1.07 and 0.94 PFLOP/s); 128 rows 162 + 75 us before, 123 + 61 us here (5.9 TB/s).
 // A slice's row is 128 bytes, unpadded (64 lanes land 16 bytes each one after the other): its 16-byte chunk c sits at position

@@ -507,8 +507,9 @@ typedef struct hxm_state_scan_args {
 
 /* The recurrence of one matrix state S [dim, vdim] per head and sequence, continued from and left in the sequence's slot: token by
  * token in float, or (portions of prompts, dim <= 128) sixteen tokens at a time as float matrix products, which round in other places
- * and are no further from the exact result.  A value, scale or write strength that is not finite reaches later tokens of its own columns
- * only, in either form; a key or decay that is not finite may leave NaN where a token at a time left an infinity.  dim <= 256. */
+ * and are no further from the exact result.  What is not finite in a token's operands shows from that token on, in either form, and a
+ * value, scale or write strength in its own columns only; sixteen tokens at a time it may come out as NaN where a token at a time left
+ * an infinity.  dim <= 256. */
 int hxm_state_scan(const hxm_state_scan_args* args, void* stream);
 
 #define HXM_DECAY_CHUNK 32      /* tokens the chunked form of hxm_decay_attention takes at a time */
