@@ -39,8 +39,9 @@ def _check(name, got, want, tol=TOL):
     assert float(off) <= tol, (name, float(off))
 
 
-# (rows are on their way three chunks ahead and pass through three images in LDS: both come round from the fourth chunk on)
-LENS = [[17], [16, 1, 33], [1, 15, 31, 2], [48, 5], [64, 113], [65, 300]]
+LENS = [[17], [16, 1, 33], [1, 15, 31, 2], [48, 5]]
+# rows are on their way three chunks ahead and pass through three images in LDS: both come round from the fourth chunk on
+LONG = [[64, 113], [65, 300]]
 
 
 @pytest.mark.parametrize("lens", LENS)
@@ -48,6 +49,13 @@ LENS = [[17], [16, 1, 33], [1, 15, 31, 2], [48, 5], [64, 113], [65, 300]]
 @pytest.mark.parametrize("form, per_channel", [("decay", False), ("decay", True), ("delta", False), ("bonus", True)])
 @pytest.mark.parametrize("types", ["bf16", "f32", "mixed"])
 def test_portions_through_a_scan(lens, K, V, form, per_channel, types):
+    _through_a_scan(lens, K, V, form, per_channel, types, 3)
+
+
+@pytest.mark.parametrize("lens", LONG)
+@pytest.mark.parametrize("K, V, types", [(64, 64, "bf16"), (100, 130, "f32"), (128, 128, "mixed")])
+@pytest.mark.parametrize("form, per_channel", [("decay", False), ("decay", True), ("delta", False), ("bonus", True)])
+def test_long_portions_through_a_scan(lens, K, V, form, per_channel, types):
     _through_a_scan(lens, K, V, form, per_channel, types, 3)
 
 
@@ -214,6 +222,12 @@ def test_not_finite_numbers_in_the_gated_recurrence(what):
 @pytest.mark.parametrize("K, V", [(64, 64), (128, 128), (12, 20), (100, 130), (65, 7)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_portions_through_the_gated_recurrence(lens, K, V, dtype):
+    _through_the_gated_recurrence(lens, K, V, dtype)
+
+
+@pytest.mark.parametrize("lens", LONG)
+@pytest.mark.parametrize("K, V, dtype", [(64, 64, torch.bfloat16), (100, 130, torch.float32)])
+def test_long_portions_through_the_gated_recurrence(lens, K, V, dtype):
     _through_the_gated_recurrence(lens, K, V, dtype)
 
 
