@@ -4,6 +4,7 @@
 // combine: the products are launched for the most rows there can be and find their expert from the plan's segments.
 #include <cfloat>
 #include "mix_rows.h"
+#include "tile_product.h"
 #include "../../include/hydra_mix.h"
 
 namespace hxm {
@@ -387,10 +388,9 @@ __global__ __launch_bounds__(256) void grouped_linear_kernel(typename A::storage
 // column l % 16 of rows 4 (l / 16) .. + 3.  Half a slice is multiplied while the other half's operands are read from LDS, one
 // read between four products; the one workgroup barrier of a slice stands between its halves, so that a wave always has
 // products to issue behind it.
-// With many rows an expert it is bound by the matrix cores and LDS bandwidth (256 x 256: a byte read from LDS feeds 21
-// multiply-adds, 128 x 128 over four waves 16), with few by the weights: those of an expert with one row tile are read past
-// the caches.  Measured with 16 experts, 2 x 2752 outputs of 4096 and back: 15956 rows 866 + 444 us through registers in
-// tiles of 128 x 128 and padded LDS rows, 671 + 383 us here (1.07 and 0.94 PFLOP/s); 128 rows 162 + 75 us before, 123 + 61 us here (5.9 TB/s).
+// With few rows an expert it is bound by the weights: those of an expert with one row tile are read past the caches (128 rows of 16
+// experts, 2 x 2752 outputs of 4096 and back: 162 + 75 us through registers in tiles of 128 x 128 and padded LDS rows, 123 + 61 us here,
+// 5.9 TB/s).  Many rows take grouped_linear_tile_kernel where they can; in tiles of 256 x 256 this form is bound by LDS bandwidth.
 // A slice's row is 128 bytes, unpadded (64 lanes land 16 bytes each one after the other): its 16-byte chunk c sits at position
 // c ^ (row / 2 % 8), so that the 16 lanes that one pass of a 16-byte LDS read serves — rows 0-3, 12-15 of one k group and
 // 4-11 of the next — fall into different banks.
@@ -622,6 +622,150 @@ int launch_grouped(u16* y, const u16* x, int64_t x_stride, const int32_t* src, c
   return hxm::check_launch();
 }
 
+// Many rows an expert: tiles of 256 rows and 256 columns (tile_product.h), one workgroup a CU that goes from tile to tile: the
+// first slices of the next one are on their way while the results of the last are stored.  Measured with 16 experts, 2 x 2752 outputs
+// of 4096 and back: 15956 rows 640 + 373 us in the form above, 585 + 318 us here (1.35 and 1.22 PFLOP/s with what is multiplied
+// for rows and columns past the end), where normal data takes all of the card's power.
+template <bool FAR>
+struct GroupedLoader {
+  const u16 *x, *w;               // (at the stream's k)
+  uint32_t ox[8], ow[8];          // bytes
+  const u16* px[8];
+  __device__ __forceinline__ void go(const u16* x_, int64_t x_stride, const int32_t* src, const u16* wt, int64_t K, int row0, int row1, int64_t cols) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    x = x_;
+    w = wt;
+    // (a row or column past the last one repeats it; never stored)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int r = min(row0 + tile_load_row(wave, j, lane), row1 - 1);
+      const int64_t at = (src ? (int64_t)src[r] : (int64_t)r) * x_stride + tile_load_k(j, lane);
+      if constexpr (FAR) px[j] = x_ + at;
+      else ox[j] = (uint32_t)(2 * at);
+      const int c = tile_load_row(wave, j, lane);
+      ow[j] = (uint32_t)(2 * ((c < cols ? c : cols - 1) * K + tile_load_k(j, lane)));
+    }
+  }
+  template <int J>
+  __device__ __forceinline__ void a(uint32_t lds) {
+    if constexpr (FAR) {
+      tile_load<J>(px[J], lds);
+      px[J] += kTileK;
+    } else {
+      tile_load<J>(x, ox[J], lds);
+      if constexpr (J == 7) x += kTileK;
+    }
+  }
+  template <int J>
+  __device__ __forceinline__ void b(uint32_t lds) {
+    tile_load<J>(w, ow[J], lds);
+    if constexpr (J == 7) w += kTileK;
+  }
+};
+
+// K is a multiple of 64 from 128 on, result rows come in whole 16-byte pieces.  GLU: act 2, else 0 or 1.
+template <bool FAR, bool GLU>
+__global__ __launch_bounds__(256, 1) void grouped_linear_tile_kernel(u16* __restrict__ y, const u16* __restrict__ x, int64_t x_stride,
+                                                                     const int32_t* __restrict__ src, const u16* __restrict__ w,
+                                                                     const int32_t* __restrict__ seg, int E, int64_t N, int64_t K, int act, Glu glu) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int n_col = (int)((N + kTileRows - 1) / kTileRows), n = (int)(K / kTileK);      // (n >= 2)
+  int at, end;
+  {
+    int m_tiles = 0;
+    for (int i = 0; i < E; ++i) m_tiles += (seg[i + 1] - seg[i] + kTileRows - 1) / kTileRows;
+    const int total = m_tiles * n_col, per = (total + 7) >> 3;
+    at = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    end = min(total, (int)(blockIdx.x & 7) * per + per);
+  }
+  if (at >= end) return;                                   // (the whole workgroup)
+  const int step = (int)(gridDim.x >> 3);
+  struct Tile {
+    int e, row0, row1;
+    int64_t col0;
+  } tile, next;
+  int e = 0, before = 0;                                   // the expert whose tiles are walked, tiles in front of it
+  auto find = [&](int i) __attribute__((always_inline)) {
+    for (;; ++e) {
+      const int r0 = seg[e], r1 = seg[e + 1], nt = (r1 - r0 + kTileRows - 1) / kTileRows, in = i - before;
+      if (in < nt * n_col) {
+        const int c = in / nt, row0 = r0 + (in - c * nt) * kTileRows;
+        return Tile{e, row0, min(r1, row0 + kTileRows), (int64_t)c * kTileRows};
+      }
+      before += nt * n_col;
+    }
+  };
+  GroupedLoader<FAR> loader;
+  auto go = [&](const Tile& t) __attribute__((always_inline)) {
+    loader.go(x, x_stride, src, w + ((int64_t)t.e * N + t.col0) * K, K, t.row0, t.row1, N - t.col0);
+  };
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int wm0 = (wave >> 1) * 128, wn0 = (wave & 1) * 128, l16 = lane & 15;
+  const int64_t out = GLU ? N >> 1 : N;
+  TileProduct<BF16, GroupedLoader<FAR>> p(smem, loader);
+  tile = find(at);
+  go(tile);
+  p.start();
+  for (;;) {
+    at += step;
+    for (int t = 0; t < n; ++t) {
+      if (t == n - 2) {                                    // from here on the next tile's slices are requested (behind the last: its own again)
+        next = at < end ? find(at) : tile;
+        go(next);
+      }
+      p.slice();
+    }
+    // a pair of results of 16 columns next to each other, the first at column c of this lane's row r
+    auto store = [&](int r, int64_t c, f32x4 first, f32x4 second) __attribute__((always_inline)) {
+      const u32x4 v = tile_pair(tile_round<BF16>(first), tile_round<BF16>(second));
+      c += tile_pair_column(lane);
+      if (r < tile.row1 && c < out) *reinterpret_cast<u32x4*>(y + (int64_t)r * out + c) = v;
+    };
+    const int64_t c0 = tile.col0 + wn0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = tile.row0 + wm0 + 16 * i + l16;
+#pragma unroll
+      for (int j = 0; j < 8; j += 4) {
+        f32x4 v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = p.take(i, j + q);
+        if constexpr (GLU) {      // columns in turns of 16 gates and 16 ups: a lane holds both numbers of a pair
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            v[0][q] = glu.of<BF16>(v[0][q], v[1][q]);
+            v[1][q] = glu.of<BF16>(v[2][q], v[3][q]);
+          }
+          store(r, (c0 >> 1) + 8 * j, v[0], v[1]);
+        } else {
+#pragma unroll
+          for (int q = 0; q < 16; ++q) v[q >> 2][q & 3] = act_apply(v[q >> 2][q & 3], act);
+          store(r, c0 + 16 * j, v[0], v[1]);
+          store(r, c0 + 16 * j + 32, v[2], v[3]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if (at >= end) break;
+    tile = next;
+    p.clear();
+  }
+  tile_wait<0>();                                          // (nothing lands in LDS that is no longer this workgroup's)
+}
+
+int launch_grouped_tiles(u16* y, const u16* x, int64_t x_stride, const int32_t* src, const u16* w, const int32_t* seg, int64_t max_rows, int E,
+                         int64_t N, int64_t K, int act, const Glu& glu, hipStream_t s) {
+  const int64_t tiles = ((max_rows + kTileRows - 1) / kTileRows + E) * ((N + kTileRows - 1) / kTileRows);      // every expert's rows start a tile
+  if (tiles > 0x7fffffff) return HX_ERR_SHAPE;
+  const int64_t grid = tiles < kTileGroups ? (tiles + 7) / 8 * 8 : kTileGroups;      // (the eight XCDs work on a run of tiles each)
+  const bool far = src || max_rows * x_stride > 0x3fffffff;
+  auto kernel = act == 2 ? (far ? grouped_linear_tile_kernel<true, true> : grouped_linear_tile_kernel<false, true>)
+                         : (far ? grouped_linear_tile_kernel<true, false> : grouped_linear_tile_kernel<false, false>);
+  (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTileLds);
+  kernel<<<dim3((unsigned)grid), dim3(256), kTileLds, s>>>(y, x, x_stride, src, w, seg, E, N, K, act, glu);
+  return hxm::check_launch();
+}
+
 // The same, four elements a lane: width, row strides and pointers are multiples of four elements.  Rows and weights of the
 // token's choices are read once into LDS; the choices' rows are requested four at a time.
 template <typename A>
@@ -772,12 +916,23 @@ extern "C" int hxm_grouped_linear(void* y, const void* x, int64_t x_stride, cons
     u16* yy = (u16*)y;
     const u16 *xx = (const u16*)x, *ww = (const u16*)w;
     // Rows an expert on average: up to 32 the weights are all there is to read (tiles of 32 rows: 123 us with 128 rows and 16
-    // experts of 5504 x 4096, like 128 x 128, at a quarter of its LDS).  A mean of 120 is where most experts need a second
-    // tile of 128 rows: 400 tokens of 4 choices and 16 experts take 181 + 82 us in tiles of 128, 206 + 94 us in tiles of 256;
-    // 512 tokens 252 + 105 and 223 + 96 us.
-    if (max_rows <= (int64_t)32 * n_experts) return launch_grouped<32, 128, 1, 4, 3>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
-    if (max_rows < (int64_t)120 * n_experts) return launch_grouped<128, 128, 2, 2, 3>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
-    return launch_grouped<256, 256, 2, 4, 2>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
+    // experts of 5504 x 4096, like 128 x 128, at a quarter of its LDS).  Up to 56 most experts' rows fit into 64, two workgroups a
+    // CU (tiles of 64 / 128 rows: 16 experts of 5504 x 4096 with 48 rows 121 / 143 us, 8 of 2816 x 2048 22 / 25, 32 of 1408 x 2048 40 /
+    // 51).  Up to 120 rows fit into 128, which reads long weight rows once (5504 x 4096, 100 rows: 177 / 157 us; short ones, 16 of
+    // 2816 x 2048: 38 / 56).
+    const int64_t E = n_experts;
+    if (max_rows <= 32 * E) return launch_grouped<32, 128, 1, 4, 3>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
+    if (max_rows > 56 * E && max_rows < 120 * E && k_dim >= 2560)
+      return launch_grouped<128, 128, 2, 2, 3>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
+    // More rows: a round of 256 tiles of 256 x 256, one a CU, takes as long as about 720 tiles of 64 x 128, two a CU, and a part of a
+    // round nearly as long as a whole one.  64 x 128 / 256 x 256: 8 experts of 2816 x 2048, 160 rows 34 / 43 us, 256 rows 42 / 45, 400
+    // rows 53 / 46; 32 of 1408 x 2048, 128 rows 49 / 51, 200 rows 63 / 52; 8 of 1408 x 1024, 200 rows 14 / 27.
+    auto tiles = [&](int64_t rows, int64_t cols) { return (n_dim + cols - 1) / cols * (max_rows / rows + E / 2 > E ? max_rows / rows + E / 2 : E); };
+    if (max_rows <= 56 * E || tiles(64, 128) <= 720 * ((tiles(256, 256) + kTileGroups - 1) / kTileGroups))
+      return launch_grouped<64, 128, 1, 4, 3>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
+    if (k_dim % kTileK || k_dim < 2 * kTileK || (act != 2 && n_dim % 8) || !aligned16(y))
+      return launch_grouped<256, 256, 2, 4, 2>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
+    return launch_grouped_tiles(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
   }
   const int64_t tiles = (max_rows + kGM - 1) / kGM + n_experts;
   if (tiles > 65535) return HX_ERR_SHAPE;

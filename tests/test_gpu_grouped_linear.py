@@ -43,6 +43,22 @@ def test_grouped_linear_over_many_slices(rows, k, act):
     _check(rows, 288, k, act, False)
 
 
+# long weight rows and about a hundred rows an expert: tiles of 128 rows
+@pytest.mark.parametrize("rows", [[70, 100], [129, 0, 150]])
+@pytest.mark.parametrize("k, act", [(2560, "glu"), (2568, "none")])
+def test_grouped_linear_of_long_weight_rows(rows, k, act):
+    _check(rows, 160, k, act, False)
+
+
+# enough tiles for those of 256 x 256: from tile to tile with two slices and with more, columns in 8s and whole turns, the last ones in
+# part; and k and n that take the form before it
+@pytest.mark.parametrize("rows", [[300, 257], [700, 0, 129], [1, 513]])
+@pytest.mark.parametrize("n, k, act", [(11040, 128, "glu"), (11048, 128, "none"), (11048, 192, "relu2"), (33088, 192, "glu"), (11040, 1088, "glu"),
+                                       (11044, 128, "none"), (11040, 200, "glu")])
+def test_grouped_linear_from_tile_to_tile(rows, n, k, act):
+    _check(rows, n, k, act, False)
+
+
 @pytest.mark.parametrize("rows", [[1, 30], [129, 0, 127], [256, 257]])
 def test_grouped_linear_of_rows_far_apart(rows):
     _check(rows, 160, 200, "none", True)
