@@ -36,6 +36,31 @@ def linear_decode(x: Tensor, weight: Tensor, out: Optional[Tensor] = None) -> Te
     return out
 
 
+def gate_up_rows_supported(x: Tensor, weight: Tensor) -> bool:
+    """True if gate_up_silu_rows takes these operands and is faster than a library product and silu_and_mul."""
+    M, K = x.shape
+    inter = weight.shape[0] // 2
+    return (x.is_cuda and weight.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and weight.dtype == x.dtype and weight.shape[1] == K
+            and weight.shape[0] == 2 * inter and x.stride(1) == 1 and weight.stride(1) == 1 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and max(M * x.stride(0), 2 * inter * weight.stride(0)) < 2 ** 31
+            and _lib.lib().hx_gate_up_silu_rows_supported(M, inter, K) == 1)
+
+
+def gate_up_silu_rows(x: Tensor, weight: Tensor) -> Tensor:
+    """act[M, inter] = silu(x @ gate.T) * (x @ up.T), weight [2 * inter, K] = gate rows, then up rows: one launch for batches of prompts,
+    rounded as a product of x's type and silu_and_mul round."""
+    _lib.require_gpu(x, weight)
+    if x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1] or x.dtype != weight.dtype or x.stride(1) != 1 or weight.stride(1) != 1 \
+            or weight.shape[0] % 2:
+        raise _lib.HydraHipError("gate_up_silu_rows: x [M, K], weight [2 * inter, K], same dtype, contiguous rows")
+    M, K = x.shape
+    inter = weight.shape[0] // 2
+    out = torch.empty((M, inter), dtype=x.dtype, device=x.device)
+    _lib.check(_lib.lib().hx_gate_up_silu_rows(out.data_ptr(), x.data_ptr(), weight.data_ptr(), M, inter, K, x.stride(0), weight.stride(0),
+                                               _lib.dtype_code(x), _lib.current_stream()), "gate_up_silu_rows")
+    return out
+
+
 def workspace_floats(M: int, N: int, K: int) -> int:
     return _lib.lib().hx_linear_decode_workspace_bytes(M, N, K) // 4
 

@@ -10,7 +10,8 @@ MI355X-first differences (all rounding-neutral with respect to the reference's u
     GEMMs instead of 7; `from_reference_state_dict` builds them from the reference's names.
   * residual-add + RMSNorm, RoPE (in place on the qkv buffer), set_kv_cache + attention and
     silu*mul each run as one HIP launch.
-GEMMs are plain library GEMMs (torch.matmul -> hipBLASLt); everything else is libhydra_hip."""
+GEMMs are plain library GEMMs (torch.matmul -> hipBLASLt) except those of decode batches and the gate|up product of large prompt
+batches; everything else is libhydra_hip."""
 import os
 from dataclasses import dataclass
 from typing import Dict, List, Optional
@@ -532,8 +533,11 @@ class LlamaForCausalLM:
                 # last layer of a prefill: only sampled tokens go through the MLP
                 h = h[model_params.selected_token_ids].contiguous()
                 x = x[model_params.selected_token_ids].contiguous()
-            gu = self.linear(x, st[f"l{l}.wgu"])
-            act = silu_and_mul(gu[:, :inter], gu[:, inter:])
+            if self.use_hip_gemm and hip_gemm.gate_up_rows_supported(x, st[f"l{l}.wgu"]):
+                act = hip_gemm.gate_up_silu_rows(x, st[f"l{l}.wgu"])      # one launch, the [n, 2 * inter] product is never stored
+            else:
+                gu = self.linear(x, st[f"l{l}.wgu"])
+                act = silu_and_mul(gu[:, :inter], gu[:, inter:])
             m = self.linear(act, st[f"l{l}.wdown"])
             nxt = st[f"l{l + 1}.norm1"] if l + 1 < L else st["norm"]
             if x.shape != h.shape:

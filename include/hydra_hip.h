@@ -227,6 +227,14 @@ int hx_embed_rms_norm(void* h_out, void* x_out, const void* ids, int ids_are_int
                       int dtype, hx_stream stream);
 int hx_argmax_rows(int64_t* out, const void* logits, int64_t rows, int64_t n, int64_t ld, int dtype,
                    hx_stream stream);
+/* act[M, inter] = silu(x Wg^T) * (x Wu^T) for batches of prompts in one launch (csrc/gemm_tile.hip): x [M, K] (row stride ldx), weight
+ * [2 inter, K] row-major, gate rows first (row stride ldw), out contiguous; fp16 / bf16, sums in float, rounded where a product of
+ * that type and hx_silu_and_mul round.  inter % 16 == 0, K % 64 == 0, K >= 128, 16-byte aligned rows, ldx * M and ldw * 2 inter below
+ * 2^31.  hx_gate_up_silu_rows_supported: 1 where it is also faster than a library product and hx_silu_and_mul.
+ * Replaces: gate_proj, up_proj and the activation of hydrainfer/model/model_forward.py:36 at prompt sizes. */
+int hx_gate_up_silu_rows_supported(int64_t M, int64_t inter, int64_t K);
+int hx_gate_up_silu_rows(void* out, const void* x, const void* weight, int64_t M, int64_t inter, int64_t K, int64_t ldx, int64_t ldw,
+                         int dtype, hx_stream stream);
 /* The same product for M <= 32 with the activations held in REGISTERS (csrc/gemm_xreg.hip): a
  * workgroup spans the whole K of its split, so K <= 4096 needs ONE slab (no K split) and K = 11008
  * three instead of eleven — the fp32 slab traffic of a decode layer drops from 25 MB to 6.5 MB.

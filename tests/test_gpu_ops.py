@@ -895,3 +895,37 @@ def test_wide_gate_up_with_silu_in_the_launch_is_bit_identical(dt):
             lib.hx_debug_set_option(b"xreg_no_producers", 0)
         assert torch.equal(h3, h1) and torch.equal(gemm.from_fragment_major(act2, M, inter), gemm.from_fragment_major(want, M, inter))
         assert int(sync[:, 1].abs().sum()) == 0
+
+
+# one row, a tile's edge and one row more, several row tiles; columns that end inside a turn's tile, more tiles than workgroups run at
+# a time; two slices of k and more
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M, inter, K", [(1, 16, 128), (255, 144, 192), (257, 128, 1088), (300, 2064, 128), (700, 11040, 192), (3100, 1536, 128)])
+def test_gate_up_silu_rows(M, inter, K, dt):
+    from hydrainfer_amd._C.kernel import gemm
+    g = torch.Generator().manual_seed(M + inter + K)
+    wide = torch.randn((M, K + 8), generator=g).to(dt).to(DEV)
+    x, w = wide[:, :K], (torch.randn((2 * inter, K), generator=g) * K ** -0.5).to(dt).to(DEV)
+    got = gemm.gate_up_silu_rows(x, w).double()
+    assert torch.equal(got.to(dt), gemm.gate_up_silu_rows(x.contiguous(), w))
+    xd, wd = x.double(), w.double()
+    z = torch.mm(xd, wd.t())
+    dz = K * 2.0 ** -24 * torch.mm(xd.abs(), wd.abs().t())
+    e = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11                        # half a unit in the last place
+    gt, up = z[:, :inter], z[:, inter:]
+    dg, du = dz[:, :inter] + e * gt.abs() + 2.0 ** -25, dz[:, inter:] + e * up.abs() + 2.0 ** -25      # (subnormal halves besides)
+    s = gt * torch.sigmoid(gt)
+    ds = 1.1 * dg + e * s.abs() + 2.0 ** -25                                     # |silu'| < 1.1
+    bound = ds * (up.abs() + du) + s.abs() * du + e * (s * up).abs() + 2.0 ** -25
+    off = (got - s * up).abs()
+    assert bool((off <= 1.02 * bound).all()), float((off / bound).max())
+
+
+def test_gate_up_silu_rows_refuses():
+    from hydrainfer_amd import _lib
+    from hydrainfer_amd._C.kernel import gemm
+    x, w = torch.zeros((300, 192), dtype=torch.bfloat16, device=DEV), torch.zeros((64, 192), dtype=torch.bfloat16, device=DEV)
+    for a, b in ((x[:, :160], w[:, :160]), (x[:, :64], w[:, :64]), (x, w[:40]), (x, w.half()), (x[:, 4:132], w[:, :128])):
+        with pytest.raises(_lib.HydraHipError):
+            gemm.gate_up_silu_rows(a, b)
+        assert not gemm.gate_up_rows_supported(a, b)
