@@ -843,14 +843,14 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide_kernel(hxm_latent_att
     const int page = bshift >= 0 ? key0 >> bshift : key0 / bs;
     const u16* base = cache + (int64_t)table[page] * a.cache_block_stride + (int64_t)(key0 - page * bs) * a.cache_row_stride;
     const uint32_t to = lds0 + (uint32_t)(img * IMG + 16 * wave * RS);
-    int ln = lane;
+    uint32_t ln = (uint32_t)lane;
     asm volatile("" : "+v"(ln));             // (worked out anew every time: kept, the addresses would push the queries out of registers)
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
     // (m0, the LDS address of the transfer, is a reserved register: nothing else in this kernel uses it)
 #pragma unroll
     for (int j = 0; j < NL; ++j) {
-      const int rr = (64 * j + ln) / L, ch = (64 * j + ln) % L;
+      const int rr = (int)((64u * j + ln) / L), ch = (int)((64u * j + ln) % L);
       const uint32_t off = (uint32_t)max(min(rr, r_max), r_min) * (uint32_t)(2 * a.cache_row_stride) + 16u * (uint32_t)(ch ^ swz(rr));
       asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(__builtin_amdgcn_readfirstlane(to + 1024u * j)) : "memory", "m0");
     }
@@ -1016,14 +1016,17 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide_kernel(hxm_latent_att
 
 // The same for wider latents (64 KK columns): four waves of 16 rows, 16 x 16 x 32 products — a row's queries and
 // accumulators are 192 registers a lane at 512 columns, two waves a SIMD.  A byte from LDS feeds half the products of the form
-// above; it is bound by the latency and number of its LDS reads (without those of the keys the same launch takes three quarters of
-// the time).  Tiles of 32 keys and 64 rows: two workgroups a CU, one working while the other brings queries in or results out.  Also
-// the form for few rows, decode steps first: the keys of a row tile are then dealt to several workgroups (wide_plan), each writes
-// its rows' sums, maximum and weight, and the kernel below merges them.
-// Measured, 4 portions of 797 - 1151 tokens, 32 heads, 512 columns: 861 us in the group form, 240 us here (530 TFLOP/s); 256
-// columns, 16 heads 268 and 65 us, 320 columns 396 and 76.  32 tokens of 301 - 1747 keys, 32 heads, 512 columns
-// under a window of 512: 31 us and 30 to merge in the tile form, 20 and 4.5 here, of which 6 pass before the first product and
-// about 5 are the splits' sums going out (8 MB); 1 token behind 1000 keys 70 us and 24, most of it the host's.
+// above, but nothing is full (matrix cores 32 % of the time, vector ALU 39, LDS 30): a wave goes through scores, softmax and values in
+// turn, waits for a quarter of its time, and there are two waves a SIMD.  Tiles of 32 keys and 64 rows: two workgroups a CU, one working while the other brings queries in or results
+// out.  Also the form for few rows, decode steps first: the keys of a row tile are then dealt to several workgroups (wide_plan),
+// each writes its rows' sums, maximum and weight, and the kernel below merges them.
+// Measured, 4 portions of 797 - 1151 tokens, 32 heads, 512 columns: 861 us in the group form, 191 us here (660 TFLOP/s; 240 while the
+// compiler had every read of a key waited for at once, 220 with addresses of the loads worked out lane by lane); 256 columns, 16
+// heads 268 and 64 us, 320 columns 396 and 68.  32 tokens of 301 - 1747 keys, 32 heads, 512 columns under a window of 512: 31 us and
+// 30 to merge in the tile form, 18 and 4.5 here, of which 6 pass before the first product and about 5 are the splits' sums going
+// out (8 MB); 1 token behind 1000 keys 70 us and 24, most of it the host's.
+// (Thirty-two rows a wave, one wave a SIMD, with weights as sums of two bfloat16 numbers instead of a pass over the 256 accumulators:
+// 245 us where this form took 253; the second set of products meets the card's power limit.)
 // Row r of sixteen has its chunks at x ^ swz(r): rows r and 15 - r share a 32-byte place (their
 // chunks turned), so that a pass of a 16-byte read (rows 0-3 and 12-15 of one chunk, 4-11 of the next) and a transposing read
 // (eight rows, 32 bytes each) both reach every bank once.
@@ -1067,20 +1070,27 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem_w;
   // Wave w brings keys 8 w .. of a tile (one page): 8 L chunks, 64 an instruction; none in front of the first or behind the last, as above.
   constexpr int NL = KPW * L / 64;
+  const uint32_t row_bytes = (uint32_t)(2 * a.cache_row_stride);
   auto bring = [&](int t, int img) __attribute__((always_inline)) {
     const int key0 = min(max(t * KT + KPW * wave, k_first & ~(KPW - 1)), k_last), r_min = k_first - key0, r_max = k_last - key0;
     const int page = bshift >= 0 ? key0 >> bshift : key0 / bs;
     const u16* base = cache + (int64_t)table[page] * a.cache_block_stride + (int64_t)(key0 - page * bs) * a.cache_row_stride;
     const uint32_t to = lds0 + (uint32_t)(img * IMG + KPW * wave * RS);
-    int ln = lane;
+    uint32_t ln = (uint32_t)lane;
     asm volatile("" : "+v"(ln));             // (worked out anew every time: kept, the addresses would push the queries out of registers)
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
     // (m0, the LDS address of the transfer, is a reserved register: nothing else in this kernel uses it)
 #pragma unroll
     for (int j = 0; j < NL; ++j) {
-      const int rr = (64 * j + ln) / L, ch = (64 * j + ln) % L;
-      const uint32_t off = (uint32_t)max(min(rr, r_max), r_min) * (uint32_t)(2 * a.cache_row_stride) + 16u * (uint32_t)(ch ^ swz(KPW * wave + rr));
+      uint32_t off;
+      if constexpr (L == 64) {               // a row a load: nothing of it differs from lane to lane but the column
+        off = (16u * ln ^ 16u * (uint32_t)swz(KPW * wave + j)) + (uint32_t)max(min(j, r_max), r_min) * row_bytes;
+      } else {
+        // (swz of row 8 wave + rr)
+        const uint32_t rr = (64u * j + ln) / L, ch = 64u * j + ln - rr * L, turned = wave & 1 ? (FULL ? 15u : 7u) : 0u;
+        off = (uint32_t)max(min((int)rr, r_max), r_min) * row_bytes + 16u * (ch ^ (FULL ? 2u * rr : rr & 6u) ^ turned);
+      }
       asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(__builtin_amdgcn_readfirstlane(to + 1024u * j)) : "memory", "m0");
     }
 #pragma clang diagnostic pop
@@ -1123,22 +1133,25 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
   auto step = [&](int key0, uint32_t kt) __attribute__((always_inline)) {
     uint32_t kp = kp0 + kt, va = vp0 + kt;
     asm volatile("" : "+v"(kp), "+v"(va));   // (their sums are made where they are read, not kept in registers)
+    // Rows of the keys, kAhead of them on their way.  The order is laid down product by product: left to the compiler, group barriers
+    // or not, every read was waited for where it stood (LDS answers after some 150 cycles, a product takes 16).
+    constexpr int kAhead = 2 * KS < 8 ? 2 * KS : 8;
     f32x4 s[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) s[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto key_read = [&](int i) __attribute__((always_inline)) {
+      return row_read((kp ^ (64u * (i / 2 % NP))) + 16u * (i & 1) * RS + 64u * NP * (i / 2 / NP));
+    };
+    u16x8 kf[kAhead];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
+    for (int i = 0; i < kAhead; ++i) kf[i] = key_read(i);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int u = 0; u < 2; ++u) s[u] = Mfma<BF16>::mma(row_read((kp ^ (64u * (ks % NP))) + 16u * u * RS + 64u * NP * (ks / NP)), qf[ks], s[u]);
-    // (reads stay a few products ahead)
-    constexpr int kAhead = 2 * KS < 8 ? 2 * KS : 8;
-    __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);
-#pragma unroll
-    for (int i = 0; i < 2 * KS - kAhead; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    for (int i = 0; i < 2 * KS; ++i) {
+      s[i & 1] = Mfma<BF16>::mma(kf[i % kAhead], qf[i / 2], s[i & 1]);
+      if (i + kAhead < 2 * KS) kf[i % kAhead] = key_read(i + kAhead);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, kAhead, 0);
     const int key_l = key0 + 4 * g;          // element e of half u: key key_l + 16 u + e
     float mx = HX_NEG_BIG;
     if (key0 + 31 <= wpos0 && key0 >= wlo1) {              // every row of the wave sees all of them
