@@ -318,6 +318,11 @@ def state_scan(mode: str, q: Tensor, k: Tensor, v: Tensor, decay: Tensor, seq: S
     a.decay_per_channel, a.decay, a.vscale, a.beta, a.bonus = int(per_channel), decay.data_ptr(), _ptr(vscale), _ptr(beta), _ptr(bonus)
     a.state, a.slot_stride, a.slots, a.q_cu, a.positions = base, stride, seq.slots.data_ptr(), q_cu.data_ptr(), positions.data_ptr()
     a.n_tokens, a.n_seq, a.heads, a.qk_heads, a.dim, a.vdim, a.mode = T, n_seq, int(heads), int(qk_heads), int(dim), int(vdim), SCAN_MODES[mode]
+    if T > n_seq:                         # portions of prompts: what their chunks need is made in a launch ahead
+        a.ws_floats = _lib.mix_lib().hxm_state_scan_workspace(ctypes.byref(a))
+        if a.ws_floats > 0:
+            ws = torch.empty(a.ws_floats, dtype=torch.float32, device=q.device)
+            a.ws = ws.data_ptr()
     _lib.mix_check(_lib.mix_lib().hxm_state_scan(ctypes.byref(a), _lib.current_stream()), "state_scan")
     return out
 

@@ -213,7 +213,7 @@ def lib() -> ctypes.CDLL:
 # a paged latent cache.  A library of its own, so that a model that needs only these builds only these (`make mix`).
 # ---------------------------------------------------------------------------------------------------------
 MIX_LIB_PATH = os.environ.get("HX_MIX_LIB_PATH") or os.path.join(_HERE, "lib", "libhydra_mix.so")
-HXM_ABI_VERSION = 6
+HXM_ABI_VERSION = 7
 HXM_MAX_STREAMS = 16
 HXM_MAX_LATENT = 1024
 
@@ -304,7 +304,7 @@ class hxm_state_scan_args(ctypes.Structure):
         ("decay", c_void_p), ("vscale", c_void_p), ("beta", c_void_p), ("bonus", c_void_p),
         ("state", c_void_p), ("slot_stride", c_int64), ("slots", c_void_p), ("q_cu", c_void_p), ("positions", c_void_p),
         ("n_tokens", c_int64), ("n_seq", c_int32), ("heads", c_int32), ("qk_heads", c_int32), ("dim", c_int32),
-        ("vdim", c_int32), ("mode", c_int32),
+        ("vdim", c_int32), ("mode", c_int32), ("ws", c_void_p), ("ws_floats", c_int64),
     ]
 
 
@@ -362,6 +362,7 @@ _MIX_SIGNATURES = {
     "hxm_moe_combine": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int64,
                                 c_int32, c_int64, c_int, c_void_p]),
     "hxm_gated_recurrence_workspace": (c_int64, [c_int64, c_int32, c_int32, c_int32]),
+    "hxm_gated_recurrence_batch_workspace": (c_int64, [c_int32, c_int64, c_int32, c_int32, c_int32, c_int32, c_int]),
     "hxm_gated_recurrence": (c_int, [c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_void_p,
                                      c_float, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int32, c_int64, c_int32, c_int32,
                                      c_int32, c_int32, c_void_p, c_int64, c_int, c_void_p]),
@@ -387,6 +388,7 @@ _MIX_SIGNATURES = {
     "hxm_decay_exp": (c_int, [c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int, c_void_p]),
     "hxm_unit_norm": (c_int, [c_void_p, c_void_p, c_int64, c_float, c_float, c_int64, c_int32, c_int32, c_int, c_void_p]),
     "hxm_head_norm_rope_cache": (c_int, [POINTER(hxm_head_rope_args), c_void_p]),
+    "hxm_state_scan_workspace": (c_int64, [POINTER(hxm_state_scan_args)]),
     "hxm_state_scan": (c_int, [POINTER(hxm_state_scan_args), c_void_p]),
     "hxm_decay_attention": (c_int, [POINTER(hxm_decay_attn_args), c_void_p]),
     "hxm_gated_group_norm": (c_int, [POINTER(hxm_group_norm_args), c_void_p]),

@@ -23,10 +23,16 @@ struct ChunkScanArgs {
   int64_t slot_stride;
   const int32_t *slots, *q_cu, *positions;
   int32_t n_seq, heads, qk_heads, K, V;
+  int64_t n_tokens;
+  int32_t longest;        // the longest portion, 0: not known
+  float* made;            // chunk_scan_workspace floats on a multiple of 16 bytes: what chunks need is made in a launch ahead; or NULL
 };
 
 // true if chunk_scan serves these sizes
 bool chunk_scan_fits(const ChunkScanArgs& a);
+// floats of workspace with which it goes faster; 0: none
+int64_t chunk_scan_workspace(const ChunkScanArgs& a);
 int chunk_scan(const ChunkScanArgs& a, hipStream_t s);
+int chunk_chain(const ChunkScanArgs& a, hipStream_t s);      // with a.made
 
 }  // namespace hxm

@@ -317,7 +317,31 @@ int launch_recurrence(const RecArgs& a, int n_seq, int dr, hipStream_t s) {
   return launch_norm<A>(a, s);
 }
 
+// Chunks from this longest portion on: a chunk costs its sixteen tokens and 64 or 128 by 64 channels however many there are (32 portions,
+// token by token and in chunks, us: 32 heads of 128 x 128, which have a workgroup a CU and more, two tokens 75 and 55; 1 portion of
+// 8 and 24 tokens 10 11, 14 13; 32 heads of 64 x 64, six and twelve 22 22, 27 22; 16 x 16, 24 and 64 18 26, 38 38; 32 x 32, 12 and
+// 24 17 20, 26 27; 8 heads of 32 x 32, 256 workgroups, four and twelve 8 9, 10 9).
+bool chunks_serve(int n_seq, int heads, int dim, int n_cw, int max_q_len) {
+  const int64_t groups = (int64_t)n_seq * heads * n_cw;
+  const int chunks_from = dim > 64 ? (groups >= 256 ? 2 : 16) : dim > 32 || groups < 512 ? 8 : dim > 16 ? 24 : 64;
+  return max_q_len < 1 || max_q_len >= chunks_from;
+}
+void chunk_sizes(hxm::ChunkScanArgs& c, int n_seq, int64_t n_tokens, int heads, int dim, int vdim, int max_q_len, int dtype) {
+  c.form = hxm::kChunkGated;
+  c.q_dtype = c.k_dtype = c.v_dtype = dtype;
+  c.n_seq = n_seq; c.heads = c.qk_heads = heads; c.K = dim; c.V = vdim; c.n_tokens = n_tokens; c.longest = max_q_len;
+}
+
 }  // namespace
+
+extern "C" int64_t hxm_gated_recurrence_batch_workspace(int32_t n_seq, int64_t n_tokens, int32_t heads, int32_t dim, int32_t vdim, int32_t max_q_len, int dtype) {
+  const int64_t least = hxm_gated_recurrence_workspace(n_tokens, heads, dim, vdim);
+  if (n_seq < 1 || least < 1 || !chunks_serve(n_seq, heads, dim, (vdim + 63) / 64, max_q_len)) return least;
+  hxm::ChunkScanArgs c{};
+  chunk_sizes(c, n_seq, n_tokens, heads, dim, vdim, max_q_len, dtype);
+  const int64_t floats = hxm::chunk_scan_workspace(c), whole = (n_tokens * heads * vdim + 3) / 4 * 4 + floats;
+  return floats > 0 && whole > least ? whole : least;
+}
 
 extern "C" int64_t hxm_gated_recurrence_workspace(int64_t n_tokens, int32_t heads, int32_t dim, int32_t vdim) {
   if (n_tokens < 0 || heads < 1 || dim < 1 || vdim < 1) return 0;
@@ -349,22 +373,16 @@ extern "C" int hxm_gated_recurrence(void* out, const void* q_pre, int64_t q_stri
   if (ws_floats < (int64_t)a.n_parts * n_tokens * heads * vdim) return HX_ERR_WORKSPACE;
   hipStream_t s = (hipStream_t)stream;
   if (dtype != HX_F32 && dtype != HX_BF16) return HX_ERR_DTYPE;
-  // Chunks from this longest portion on: a chunk costs its sixteen tokens and 64 or 128 by 64 channels however many there are (32 portions,
-  // token by token and in chunks, us: 32 heads of 128 x 128, which have a workgroup a CU and more, two tokens 75 and 55; 1 portion of
-  // 8 and 24 tokens 10 11, 14 13; 32 heads of 64 x 64, six and twelve 22 22, 27 22; 16 x 16, 24 and 64 18 26, 38 38; 32 x 32, 12 and
-  // 24 17 20, 26 27; 8 heads of 32 x 32, 256 workgroups, four and twelve 8 9, 10 9).
-  const int64_t groups = (int64_t)n_seq * heads * a.n_cw;
-  const int chunks_from = dim > 64 ? (groups >= 256 ? 2 : 16) : dim > 32 || groups < 512 ? 8 : dim > 16 ? 24 : 64;
-  if (max_q_len < 1 || max_q_len >= chunks_from) {
+  if (chunks_serve(n_seq, heads, dim, a.n_cw, max_q_len)) {
     hxm::ChunkScanArgs c{};
     c.out = ws; c.q = q_pre; c.k = f_pre; c.v = v;
     c.q_stride = q_stride; c.k_stride = f_stride; c.v_stride = v_stride;
-    c.q_dtype = c.k_dtype = c.v_dtype = dtype;
-    c.form = hxm::kChunkGated;
     c.f_bias = f_bias; c.low = low;
     c.state = state; c.slot_stride = slot_stride; c.slots = slots; c.q_cu = q_cu; c.positions = positions;
-    c.n_seq = n_seq; c.heads = c.qk_heads = heads; c.K = dim; c.V = vdim;
+    chunk_sizes(c, n_seq, n_tokens, heads, dim, vdim, max_q_len, dtype);
     if (hxm::chunk_scan_fits(c)) {
+      const int64_t floats = hxm::chunk_scan_workspace(c), first = (n_tokens * heads * vdim + 3) / 4 * 4;
+      if (floats > 0 && reinterpret_cast<uintptr_t>(ws) % 16 == 0 && ws_floats >= first + floats) c.made = ws + first;
       const int rc = hxm::chunk_scan(c, s);
       if (rc != HX_OK) return rc;
       a.n_parts = 1;

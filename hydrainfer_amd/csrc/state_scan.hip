@@ -477,7 +477,28 @@ bool step_serves(const hxm_state_scan_args& a) {
   return a.n_tokens == a.n_seq && a.vdim % 4 == 0 && a.slot_stride % 4 == 0 && al(a.state) && al(a.out);
 }
 
+bool chunks_serve(const hxm_state_scan_args& a) {
+  return a.n_tokens >= 6 * (int64_t)a.n_seq && a.n_tokens - a.n_seq >= 12;      // (the longest portion may be of 13 tokens or more)
+}
+hxm::ChunkScanArgs chunk_args(const hxm_state_scan_args& a) {
+  hxm::ChunkScanArgs c{};
+  c.out = a.out; c.q = a.q; c.k = a.k; c.v = a.v;
+  c.q_stride = a.q_stride; c.k_stride = a.k_stride; c.v_stride = a.v_stride;
+  c.q_dtype = a.q_dtype; c.k_dtype = a.k_dtype; c.v_dtype = a.v_dtype;
+  c.form = a.mode == HXM_SCAN_DECAY ? hxm::kChunkDecay : a.mode == HXM_SCAN_BONUS ? hxm::kChunkBonus : hxm::kChunkDelta;
+  c.per_channel = a.decay_per_channel;
+  c.decay = a.decay; c.vscale = a.vscale; c.beta = a.beta; c.bonus = a.bonus;
+  c.state = a.state; c.slot_stride = a.slot_stride; c.slots = a.slots; c.q_cu = a.q_cu; c.positions = a.positions;
+  c.n_seq = a.n_seq; c.heads = a.heads; c.qk_heads = a.qk_heads; c.K = a.dim; c.V = a.vdim; c.n_tokens = a.n_tokens;
+  return c;
+}
+
 }  // namespace
+
+extern "C" int64_t hxm_state_scan_workspace(const hxm_state_scan_args* args) {
+  if (!args || args->n_seq < 1 || args->heads < 1 || args->dim < 1 || args->vdim < 1 || !chunks_serve(*args)) return 0;
+  return hxm::chunk_scan_workspace(chunk_args(*args));
+}
 
 extern "C" int hxm_state_scan(const hxm_state_scan_args* args, void* stream) {
   if (!args) return HX_ERR_NULL;
@@ -500,17 +521,13 @@ extern "C" int hxm_state_scan(const hxm_state_scan_args* args, void* stream) {
   // single tokens and one portion of 200, 526 and 72 us, 32 heads of 16 x 16 50 and 34.  So chunks are also taken where equal portions
   // would go faster here, small states that fill the chip: 32 portions of 64 tokens, 32 heads of 16 x 16 (padded to 64 x 64) 19 and
   // 30 us, of six tokens 7 and 15; 64 x 64, 16 and 32 portions of six 9 and 11, 15 and 17.
-  if (a.n_tokens >= 6 * (int64_t)a.n_seq && a.n_tokens - a.n_seq >= 12) {      // (the longest portion may be of 13 tokens or more)
-    hxm::ChunkScanArgs c{};
-    c.out = a.out; c.q = a.q; c.k = a.k; c.v = a.v;
-    c.q_stride = a.q_stride; c.k_stride = a.k_stride; c.v_stride = a.v_stride;
-    c.q_dtype = a.q_dtype; c.k_dtype = a.k_dtype; c.v_dtype = a.v_dtype;
-    c.form = a.mode == HXM_SCAN_DECAY ? hxm::kChunkDecay : a.mode == HXM_SCAN_BONUS ? hxm::kChunkBonus : hxm::kChunkDelta;
-    c.per_channel = a.decay_per_channel;
-    c.decay = a.decay; c.vscale = a.vscale; c.beta = a.beta; c.bonus = a.bonus;
-    c.state = a.state; c.slot_stride = a.slot_stride; c.slots = a.slots; c.q_cu = a.q_cu; c.positions = a.positions;
-    c.n_seq = a.n_seq; c.heads = a.heads; c.qk_heads = a.qk_heads; c.K = a.dim; c.V = a.vdim;
-    if (hxm::chunk_scan_fits(c)) return hxm::chunk_scan(c, s);
+  if (chunks_serve(a)) {
+    hxm::ChunkScanArgs c = chunk_args(a);
+    if (hxm::chunk_scan_fits(c)) {
+      const int64_t floats = hxm::chunk_scan_workspace(c);
+      if (floats > 0 && a.ws && reinterpret_cast<uintptr_t>(a.ws) % 16 == 0 && a.ws_floats >= floats) c.made = a.ws;
+      return hxm::chunk_scan(c, s);
+    }
   }
   if (step_serves(a)) {
     if (a.dim <= 64) return launch_step<4>(a, s);

@@ -34,7 +34,7 @@
 extern "C" {
 #endif
 
-#define HXM_ABI_VERSION 6
+#define HXM_ABI_VERSION 7
 #define HXM_MAX_STREAMS 16
 #define HXM_MAX_LATENT 1024     /* widest latent row the attention kernels hold in registers (the MFMA tile form: 512) */
 
@@ -256,6 +256,8 @@ int hxm_moe_combine(void* out, const void* y, const int32_t* row_of, const float
  * kernel without the chunk machinery.  Longer portions of up to 128 key channels go sixteen tokens at a time through float matrix
  * products, from a length on that depends on the sizes; what is said at hxm_state_scan holds for them. */
 int64_t hxm_gated_recurrence_workspace(int64_t n_tokens, int32_t heads, int32_t dim, int32_t vdim);
+/* At least as many floats, and on a multiple of 16 bytes: with these the batch goes fastest. */
+int64_t hxm_gated_recurrence_batch_workspace(int32_t n_seq, int64_t n_tokens, int32_t heads, int32_t dim, int32_t vdim, int32_t max_q_len, int dtype);
 int hxm_gated_recurrence(void* out, const void* q_pre, int64_t q_stride, const void* f_pre, int64_t f_stride, const void* v,
                          int64_t v_stride, const float* f_bias, const float* low, const float* norm_w, float eps,
                          float* state, int64_t slot_stride, const int32_t* q_cu, const int32_t* positions,
@@ -503,6 +505,8 @@ typedef struct hxm_state_scan_args {
   const int32_t* positions;
   int64_t n_tokens;
   int32_t n_seq, heads, qk_heads, dim, vdim, mode;
+  float* ws;                 /* NULL, or hxm_state_scan_workspace(args) floats on a multiple of 16 bytes: long portions go faster */
+  int64_t ws_floats;
 } hxm_state_scan_args;
 
 /* The recurrence of one matrix state S [dim, vdim] per head and sequence, continued from and left in the sequence's slot: token by
@@ -510,6 +514,7 @@ typedef struct hxm_state_scan_args {
  * and are no further from the exact result.  What is not finite in a token's operands shows from that token on, in either form, and a
  * value, scale or write strength in its own columns only; sixteen tokens at a time it may come out as NaN where a token at a time left
  * an infinity.  dim <= 256. */
+int64_t hxm_state_scan_workspace(const hxm_state_scan_args* args);      /* by its sizes, types and mode; 0: none */
 int hxm_state_scan(const hxm_state_scan_args* args, void* stream);
 
 #define HXM_DECAY_CHUNK 32      /* tokens the chunked form of hxm_decay_attention takes at a time */

@@ -59,6 +59,62 @@ def test_long_portions_through_a_scan(lens, K, V, form, per_channel, types):
     _through_a_scan(lens, K, V, form, per_channel, types, 3)
 
 
+# portions whose chunks are made in a launch ahead (csrc/chunk_chain.hip): the same products and sums in the same order as in one launch,
+# so the same bits; tokens that fill no chunk, sequences without tokens, keys and values that fill no tile
+@pytest.mark.parametrize("lens", [[1151], [500, 0, 1, 417], [700, 333]], ids=str)
+@pytest.mark.parametrize("form, K, V, types", [("bonus", 64, 64, "bf16"), ("bonus", 128, 128, "f32"), ("bonus", 100, 130, "mixed"), ("decay", 128, 64, "bf16"),
+                                               ("decay", 65, 7, "f32"), ("decay", 64, 68, "mixed")])
+def test_chunks_made_ahead(lens, form, K, V, types, monkeypatch):
+    from hydrainfer_amd import _lib
+    lib, asked = _lib.mix_lib(), []
+
+    class Watch:
+        def __getattr__(self, name):
+            if name != "hxm_state_scan_workspace":
+                return getattr(lib, name)
+            return lambda a: asked.append(lib.hxm_state_scan_workspace(a)) or (asked[-1] if len(asked) == 1 else 0)
+
+    monkeypatch.setattr(_lib, "_mix", Watch())
+    ahead = _through_a_scan(lens, K, V, form, True, types, 3)
+    assert asked[0] > 0
+    for a, b in zip(ahead, _through_a_scan(lens, K, V, form, True, types, 3)):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("lens", [[1151], [0, 300, 0, 1, 417, 0]], ids=str)
+@pytest.mark.parametrize("K, V", [(64, 64), (128, 128), (100, 36), (48, 7)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_gates_made_ahead(lens, K, V, dt, monkeypatch):
+    from hydrainfer_amd import _lib
+    from hydrainfer_amd._C.kernel.recurrence import gated_recurrence
+    from hydrainfer_amd._C.kernel.stream_ops import SequenceState
+    lib, H, T, n = _lib.mix_lib(), 3, sum(lens), len(lens)
+    g = torch.Generator(device="cuda").manual_seed(K + V)
+    f = lambda *s: torch.randn(s, generator=g, device="cuda")
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    proj, bias, low, w, start = f(T, H * (2 * K + V)).to(dt), f(H * K), 0.9 * torch.rand(H * K, generator=g, device="cuda"), f(V), f(n, 1, H * K * V)
+    proj[T // 2, 2 * H * K + 1] = math.inf                        # (a chunk whose sums go in order)
+    cu = [sum(lens[:s]) for s in range(n + 1)]
+    pos = i32([p + 5 * (s % 2) for s, m in enumerate(lens) for p in range(m)])
+    seq_of = i32([s for s, m in enumerate(lens) for _ in range(m)])
+
+    def run():
+        st = start.clone()
+        return gated_recurrence(proj[:, :H * K], proj[:, H * K:2 * H * K], proj[:, 2 * H * K:], bias, low, w, 1e-5, SequenceState(st, i32(list(range(n))), seq_of), 0,
+                                i32(cu), pos, H, K, V, max_q_len=max(lens)), st
+
+    ahead = run()
+    assert lib.hxm_gated_recurrence_batch_workspace(n, T, H, K, V, max(lens), _lib._DTYPE[dt]) > lib.hxm_gated_recurrence_workspace(T, H, K, V)
+
+    class Least:
+        def __getattr__(self, name):
+            return (lambda n, T, H, K, V, m, dt: lib.hxm_gated_recurrence_workspace(T, H, K, V)) if name == "hxm_gated_recurrence_batch_workspace" else getattr(lib, name)
+
+    monkeypatch.setattr(_lib, "_mix", Least())
+    for a, b in zip(ahead, run()):
+        assert torch.equal(a.float().nan_to_num(nan=7.5), b.float().nan_to_num(nan=7.5)) and bool(torch.isfinite(a).any())
+
+
 # out, state: what a token at a time loses in float over the same portions (2-norm, in 1e-7, measured with the form that walks the
 # tokens).  Chunks lose no more than that, give or take a twentieth.
 @pytest.mark.parametrize("form, K, out, state", [("delta", 128, 1.096, 0.780), ("delta", 64, 1.010, 0.838), ("decay", 128, 1.073, 0.825), ("decay", 64, 1.001, 0.808),
@@ -155,6 +211,7 @@ def _through_a_scan(lens, K, V, form, per_channel, types, pad):
     _check("state", st[slots.long().cuda(), 0, pad:].view(n, H, K, V), S)
     other = [s for s in range(n + 1) if s not in slots.tolist()]
     assert torch.equal(st[other], before[other]) and torch.equal(st[:, 0, :pad], before[:, 0, :pad])
+    return got, st
 
 
 # What is not a finite number in a token's operands shows from that token on, in its columns, and nowhere before: the tokens are a chunk's
