@@ -24,6 +24,7 @@ from hydrainfer_amd._C.kernel.norm import (StepHead, add_rms_norm, add_rms_norm_
                                              embed_rms_norm, embed_rms_norm_supported, rms_norm)
 from hydrainfer_amd._C.kernel.position_embedding import rope_set_kv_cache
 from hydrainfer_amd.layer.causal_attention import AttentionParameters
+from hydrainfer_amd._C.kernel.decode_step import DecodeLayer, decode_layers
 from hydrainfer_amd._C.kernel.flash_attn import decode_attention_fused, mha_varlen_fwd
 from hydrainfer_amd._C.kernel import gemm as hip_gemm
 from hydrainfer_amd import _lib, launch_plan
@@ -109,6 +110,8 @@ class LlamaForCausalLM:
         self.use_wide = os.environ.get("HX_WIDE", "1") == "1"
         # ... with silu * mul inside the norm + gate|up launch (round 5: both K halves in one workgroup, no slabs)
         self.use_wide_silu = os.environ.get("HX_WIDE_SILU", "1") == "1"
+        # the layers of a step of <= 32 rows on these launches: issued by one native call (decode_step)
+        self.one_call = True
         self.sample_out: Optional[Tensor] = None   # int64 [rows]: forward() writes the sampled ids here (decode loops)
         self.xreg_sync: Optional[Tensor] = None   # [L, 2, XREG_SYNC_WORDS] of the last step (word 1 = wait gave up)
         self.packed_x: Dict[str, Tensor] = {}
@@ -388,6 +391,16 @@ class LlamaForCausalLM:
             x = x0          # the first layer's norm came with the embedding gather
         else:
             rms_norm(x, h, st["l0.norm1"], eps)
+        if self.one_call and fused and nf_gu and (L == 1 or "l1.wqkv" in self.dw) and all(f"l{l}.wo" in self.dw_lds for l in range(L)) and "l0.wqkv" in self.dw_lds:
+            layers = []
+            for l in range(L):
+                ap = model_params.attention_params[l]
+                layers.append(DecodeLayer(*ap.kv_cache.get_kv_cache(), ap.new_cache_slots, ap.q_cu_seq_lens, ap.kv_cu_seq_lens, ap.block_tables,
+                                          ap.cu_blocks_lens, ap.kv_max_seq_len, ap.decode_rank, self.dw[f"l{l}.wqkv"] if l else self.dw_lds["l0.wqkv"],
+                                          self.dw_lds[f"l{l}.wo"], self.dw[f"l{l}.wdown"], self.packed_x[f"l{l}.wgu"], st[f"l{l}.norm2"],
+                                          st[f"l{l + 1}.norm1"] if l + 1 < L else st["norm"]))
+            decode_layers(h, x, xf, actf, ws, ws_q, sync, inter, H, D, position_ids, self.cos_sin, D ** -0.5, eps, nf_qkv, layers)
+            return x
         s_qkv = None
         for l in range(L):
             ap = model_params.attention_params[l]

@@ -230,3 +230,33 @@ def test_decode_with_norm_fused_launches_equals_separate_launches(dt):
         outs.append((r.generated(), r.pool.clone()))
     assert torch.equal(outs[0][0], outs[1][0])
     assert torch.equal(outs[0][1], outs[1][1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hidden, inter, layers, batch", [(1024, 2816, 3, 1), (1024, 2816, 1, 32), (2048, 5632, 3, 5)])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_layers_in_one_call_equal_the_launches_one_by_one(hidden, inter, layers, batch, dt):
+    """The next layer's norm inside its qkv product (width 1024) and as a launch of its own (width 2048, two K splits): sampled
+    tokens and the KV pool bit-identical, eager steps and replayed graphs."""
+    from hydrainfer_amd.model import llama
+    from hydrainfer_amd.model.runner import DecodeRunner, RunnerConfig
+    sh = llama.LlamaShape(hidden, inter, layers, hidden // 128, hidden // 128, 128, 2048)
+    outs, calls = [], []
+    for one_call, graph in ((False, False), (True, False), (True, True)):
+        model = llama.LlamaForCausalLM.random_init(sh, dt, torch.device("cuda:0"), seed=3)
+        model.one_call = one_call
+        r = DecodeRunner(model, RunnerConfig(batch=batch, prompt_len=40, n_generate=16, use_graph=graph), seed=4)
+        g = torch.Generator().manual_seed(0)
+        r.prefill(torch.randint(5, 2000, (batch, 40), generator=g).cuda())
+        whole = llama.decode_layers
+        llama.decode_layers = lambda *a: calls.append(one_call) or whole(*a)
+        try:
+            for _ in range(12):
+                r.step()
+        finally:
+            llama.decode_layers = whole
+        torch.cuda.synchronize()
+        outs.append((r.generated(), r.pool.clone()))
+    assert calls and all(calls)
+    for tokens, pool in outs[1:]:
+        assert torch.equal(outs[0][0], tokens) and torch.equal(outs[0][1], pool)
