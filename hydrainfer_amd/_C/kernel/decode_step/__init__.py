@@ -1,8 +1,8 @@
-"""The layers of a decode step in one native call (csrc/decode_step.hip, hx_decode_layers): the launches that
+"""The layers of a decode step, each in one native call (csrc/decode_step.hip, hx_decode_layer_step): the launches that
 gemm.linear_decode_ex, flash_attn.decode_attention_fused, gemm.norm_gate_up_silu_xreg, gemm.norm_linear_decode_xreg and
 norm.add_rms_norm_slabs issue one by one, in the same order with the same arguments."""
 import ctypes
-from typing import List, NamedTuple, Optional
+from typing import Iterable, NamedTuple, Optional
 
 import torch
 from torch import Tensor
@@ -21,77 +21,85 @@ class DecodeLayer(NamedTuple):
     cu_block_lens: Tensor
     max_seqlen_k: int
     rank_desc: Optional[Tensor]
-    qkv: DecodeWeight               # the first layer's reads row-major activations, the others' are of the xreg layout
+    next_qkv: Optional[DecodeWeight]      # of the next layer, xreg layout as is down
     o: DecodeWeight
-    down: DecodeWeight              # xreg layout
+    down: DecodeWeight
     gate_up: Tensor                 # pack_weight_xreg(W [2 * inter, hidden], interleave_halves=True)
     norm_mlp: Tensor                # [hidden]
     norm_next: Tensor               # [hidden]: the next layer's first norm, or the final one
 
 
 def decode_layers(h: Tensor, x: Tensor, x_frag: Tensor, act: Tensor, ws: Tensor, ws_qkv: Tensor, sync: Tensor, inter: int, n_heads: int,
-                  head_dim: int, positions: Tensor, cos_sin: Tensor, softmax_scale: float, epsilon: float, norm_in_qkv: bool,
-                  layers: List[DecodeLayer]) -> None:
-    """h [rows <= 32, hidden] residual (updated); x [rows, hidden] the first layer's normed input, receives the final norm's output;
-    x_frag, act: fragment-major scratch of hidden and inter; ws, ws_qkv: float32 slabs (two buffers with norm_in_qkv, the qkv
-    product taking the norm of the layer before); sync: zeroed int32 [layers, 2, XREG_SYNC_WORDS]."""
+                  head_dim: int, positions: Tensor, cos_sin: Tensor, softmax_scale: float, epsilon: float, norm_in_qkv: bool, qkv_slabs: int,
+                  layers: Iterable[DecodeLayer]) -> None:
+    """h [rows <= 32, hidden] residual (updated); x [rows, hidden] receives the final norm's output; qkv_slabs of the first layer's qkv
+    product stand in ws_qkv; x_frag, act: fragment-major scratch of hidden and inter; ws, ws_qkv: float32 slabs (two buffers with norm_in_qkv, the qkv
+    product taking the norm of the layer before); sync: zeroed int32 [layers, 2, XREG_SYNC_WORDS].  layers may be a generator: the first
+    layer runs while the caller puts the next one together."""
     _lib.require_gpu(h, x, x_frag, act, ws, ws_qkv, sync, positions, cos_sin)
     rows, hidden = h.shape
-    dt, L = h.dtype, len(layers)
+    dt = h.dtype
     if dt not in (torch.float16, torch.bfloat16) or cos_sin.dtype != dt or any(t.dtype != dt or not t.is_contiguous() for t in (h, x, x_frag, act)) or x.shape != h.shape \
             or x_frag.numel() < fragment_major_elems(rows, hidden) or act.numel() < fragment_major_elems(rows, inter):
         raise _lib.HydraHipError("decode_layers: h, x [rows, hidden] and fragment-major scratch, contiguous and of one dtype (fp16 / bf16)")
     if any(t.dtype != torch.float32 or not t.is_contiguous() for t in (ws, ws_qkv)) or (norm_in_qkv and ws.data_ptr() == ws_qkv.data_ptr()):
         raise _lib.HydraHipError("decode_layers: slabs must be contiguous float32, of their own for the qkv product that takes the norm")
-    if sync.dtype != torch.int32 or not sync.is_contiguous() or sync.numel() < L * 2 * XREG_SYNC_WORDS:
+    if sync.dtype != torch.int32 or not sync.is_contiguous():
         raise _lib.HydraHipError("decode_layers: sync must be [layers, 2, XREG_SYNC_WORDS] contiguous int32 (zeroed)")
     if positions.dtype != torch.int32 or not positions.is_contiguous() or positions.numel() < rows:
         raise _lib.HydraHipError("decode_layers: positions must be contiguous int32 [rows]")
     q_size = n_heads * head_dim
     o = torch.empty((rows, q_size), dtype=dt, device=h.device)
-    attn, fused = _lib.hx_attn_args(), _lib.hx_fused_decode_args()
-    attn.out = attn.q = o.data_ptr()                              # (q, k_new and v_new are read from the slabs)
-    attn.batch, attn.n_heads, attn.head_dim, attn.max_seqlen_q, attn.total_q = rows, n_heads, head_dim, 1, rows
-    attn.q_row_stride = attn.o_row_stride = q_size
-    attn.softmax_scale, attn.causal, attn.dtype, attn.window_left, attn.window_right = float(softmax_scale), 1, _lib.dtype_code(h), -1, -1
-    fused.k_new = fused.v_new = attn.out
-    fused.k_new_row_stride = fused.v_new_row_stride = q_size
-    fused.positions, fused.cos_sin, fused.rotary_dim = positions.data_ptr(), cos_sin.data_ptr(), head_dim
-    array = (_lib.hx_decode_layer * L)()
-    for c, p in zip(array, layers):
+    lib, stream = _lib.lib(), _lib.current_stream()
+    c = _lib.hx_decode_layer()
+    a, f = c.attn, c.fused
+    a.out = a.q = o.data_ptr()                                    # (q, k_new and v_new are read from the slabs)
+    a.batch, a.n_heads, a.head_dim, a.max_seqlen_q, a.total_q = rows, n_heads, head_dim, 1, rows
+    a.q_row_stride = a.o_row_stride = q_size
+    a.softmax_scale, a.causal, a.dtype, a.window_left, a.window_right = float(softmax_scale), 1, _lib.dtype_code(h), -1, -1
+    f.k_new = f.v_new = a.out
+    f.k_new_row_stride = f.v_new_row_stride = q_size
+    f.positions, f.cos_sin, f.rotary_dim = positions.data_ptr(), cos_sin.data_ptr(), head_dim
+    c.h, c.x, c.x_frag, c.act, c.ws, c.ws_qkv = (t.data_ptr() for t in (h, x, x_frag, act, ws, ws_qkv))
+    c.ws_bytes, c.ws_qkv_bytes, c.rows, c.hidden, c.inter = 4 * ws.numel(), 4 * ws_qkv.numel(), rows, hidden, inter
+    c.epsilon, c.norm_in_qkv, c.dtype = float(epsilon), int(norm_in_qkv), a.dtype
+    slabs, attn_ws, first_sync, no_weight = int(qkv_slabs), None, sync.data_ptr(), _lib.hx_decode_weight()
+    for l, p in enumerate(layers):
         k, v, ints = p.key_cache, p.value_cache, p[2:7]
+        if sync.numel() < (l + 1) * 2 * XREG_SYNC_WORDS:
+            raise _lib.HydraHipError("decode_layers: sync has no words left for this layer")
         _lib.require_gpu(k, v, *ints, p.rank_desc, p.gate_up, p.norm_mlp, p.norm_next)
         if k.dtype != dt or v.dtype != dt or k.dim() != 4 or v.shape != k.shape:
             raise _lib.HydraHipError("decode_layers: caches [n_blocks, block_size, kv_heads, head_dim] of the activations' dtype")
         for t in ints:
             if t.dtype != torch.int32 or not t.is_contiguous():
                 raise _lib.HydraHipError("decode_layers: slots, lengths and block tables must be contiguous int32")
+        n_kv, nq = k.size(2), p.next_qkv
+        qkv_n = (n_heads + 2 * n_kv) * head_dim
+        if ws_qkv.numel() < slabs * rows * qkv_n:
+            raise _lib.HydraHipError("decode_layers: ws_qkv must hold the qkv product's slabs")
         if p.cu_seqlens_q.numel() != rows + 1:
             raise _lib.HydraHipError("decode_layers needs exactly one query token per sequence")
         if p.rank_desc is not None and (p.rank_desc.dtype != torch.int32 or not p.rank_desc.is_contiguous() or p.rank_desc.numel() < rows + 1):
             raise _lib.HydraHipError("decode_layers: rank_desc must be a contiguous int32 device tensor [1 + rows]")
-        if (p.qkv.K, p.o.N, p.o.K, p.down.N, p.down.K) != (hidden, hidden, q_size, hidden, inter) or p.qkv.N != (n_heads + 2 * k.size(2)) * head_dim \
-                or any(w.packed.dtype != dt for w in (p.qkv, p.o, p.down)) or p.gate_up.dtype != dt or p.gate_up.numel() != 2 * inter * hidden:
+        if (p.o.N, p.o.K, p.down.N, p.down.K) != (hidden, q_size, hidden, inter) or (nq is not None and ((nq.N, nq.K) != (qkv_n, hidden) or nq.packed.dtype != dt)) \
+                or p.o.packed.dtype != dt or p.down.packed.dtype != dt or p.gate_up.dtype != dt or p.gate_up.numel() != 2 * inter * hidden:
             raise _lib.HydraHipError("decode_layers: packed weights do not match the activations")
         for w in (p.norm_mlp, p.norm_next):
             if w.dtype != dt or w.numel() != hidden or not w.is_contiguous():
                 raise _lib.HydraHipError("decode_layers: norm weights [hidden] of the activations' dtype")
-        c.attn, c.fused, c.qkv, c.o, c.down = attn, fused, p.qkv.desc, p.o.desc, p.down.desc
+        c.o, c.down, c.next_qkv = p.o.desc, p.down.desc, no_weight if nq is None else nq.desc
         c.gate_up, c.norm_mlp, c.norm_next = p.gate_up.data_ptr(), p.norm_mlp.data_ptr(), p.norm_next.data_ptr()
-        a, f = c.attn, c.fused
-        a.k, a.v, a.n_kv_heads, a.block_size, a.max_seqlen_k = k.data_ptr(), v.data_ptr(), k.size(2), k.size(1), int(p.max_seqlen_k)
+        c.sync = first_sync + 4 * 2 * XREG_SYNC_WORDS * l
+        a.k, a.v, a.n_kv_heads, a.block_size, a.max_seqlen_k = k.data_ptr(), v.data_ptr(), n_kv, k.size(1), int(p.max_seqlen_k)
         a.k_block_stride, a.k_row_stride, a.k_head_stride = k.stride()[:3]
         a.v_block_stride, a.v_row_stride, a.v_head_stride = v.stride()[:3]
         f.new_cache_slots, a.cu_seqlens_q, a.cu_seqlens_k, a.block_table, a.cu_block_lens = (t.data_ptr() for t in ints)
         f.rank_desc = None if p.rank_desc is None else p.rank_desc.data_ptr()
-    lib = _lib.lib()
-    need = lib.hx_decode_layers_workspace_bytes(array, L)
-    if need > 0:
-        attn_ws = torch.empty(need, dtype=torch.uint8, device=h.device)
-        for c in array:
-            c.attn.workspace, c.attn.workspace_bytes = attn_ws.data_ptr(), need
-    g = _lib.hx_decode_layers_args()
-    g.h, g.x, g.x_frag, g.act, g.ws, g.ws_qkv, g.sync = (t.data_ptr() for t in (h, x, x_frag, act, ws, ws_qkv, sync))
-    g.ws_bytes, g.ws_qkv_bytes, g.rows, g.hidden, g.inter = 4 * ws.numel(), 4 * ws_qkv.numel(), rows, hidden, inter
-    g.epsilon, g.norm_in_qkv, g.dtype = float(epsilon), int(norm_in_qkv), _lib.dtype_code(h)
-    _lib.check(lib.hx_decode_layers(ctypes.byref(g), array, L, _lib.current_stream()), "decode_layers")
+        need = lib.hx_mha_varlen_fwd_workspace_bytes(ctypes.byref(a))
+        if need > (0 if attn_ws is None else attn_ws.numel()):
+            attn_ws = torch.empty(need, dtype=torch.uint8, device=h.device)
+            a.workspace, a.workspace_bytes = attn_ws.data_ptr(), need
+        slabs = lib.hx_decode_layer_step(ctypes.byref(c), slabs, stream)
+        if slabs < 0:
+            _lib.check(slabs, "decode_layers")

@@ -61,14 +61,11 @@ class hx_decode_weight(ctypes.Structure):
 
 
 class hx_decode_layer(ctypes.Structure):
-    _fields_ = [("attn", hx_attn_args), ("fused", hx_fused_decode_args), ("qkv", hx_decode_weight), ("o", hx_decode_weight),
-                ("down", hx_decode_weight), ("gate_up", c_void_p), ("norm_mlp", c_void_p), ("norm_next", c_void_p)]
-
-
-class hx_decode_layers_args(ctypes.Structure):
-    _fields_ = [("h", c_void_p), ("x", c_void_p), ("x_frag", c_void_p), ("act", c_void_p), ("ws", c_void_p), ("ws_qkv", c_void_p),
-                ("ws_bytes", c_int64), ("ws_qkv_bytes", c_int64), ("rows", c_int64), ("hidden", c_int64), ("inter", c_int64),
-                ("sync", c_void_p), ("epsilon", c_float), ("norm_in_qkv", c_int32), ("dtype", c_int32)]
+    _fields_ = [("attn", hx_attn_args), ("fused", hx_fused_decode_args), ("o", hx_decode_weight),
+                ("down", hx_decode_weight), ("next_qkv", hx_decode_weight), ("gate_up", c_void_p), ("norm_mlp", c_void_p),
+                ("norm_next", c_void_p), ("sync", c_void_p), ("h", c_void_p), ("x", c_void_p), ("x_frag", c_void_p), ("act", c_void_p),
+                ("ws", c_void_p), ("ws_qkv", c_void_p), ("ws_bytes", c_int64), ("ws_qkv_bytes", c_int64), ("rows", c_int64),
+                ("hidden", c_int64), ("inter", c_int64), ("epsilon", c_float), ("norm_in_qkv", c_int32), ("dtype", c_int32)]
 
 
 HX_DW_LDS_SLICE, HX_DW_XREG, HX_DW_GATE_UP = 0, 1, 1
@@ -173,8 +170,7 @@ _SIGNATURES = {
     "hx_gate_up_silu_wide_xreg_supported": (c_int, [c_int64, c_int64, c_int64]),
     "hx_norm_gate_up_silu_wide_xreg": (c_int, [c_void_p, c_void_p, c_void_p, c_int32, c_void_p, c_float, c_void_p, c_void_p,
                                                c_int64, c_int64, c_int64, c_void_p, c_int, c_void_p]),
-    "hx_decode_layers_workspace_bytes": (c_int64, [POINTER(hx_decode_layer), c_int32]),
-    "hx_decode_layers": (c_int, [POINTER(hx_decode_layers_args), POINTER(hx_decode_layer), c_int32, c_void_p]),
+    "hx_decode_layer_step": (c_int, [POINTER(hx_decode_layer), c_int32, c_void_p]),
     "hx_measure_read_stream": (c_int, [c_void_p, c_int64, c_void_p, c_void_p]),
     "hx_measure_read_grid": (c_int, [c_void_p, c_int64, c_int, c_void_p, c_void_p]),
     "hx_measure_paged_read": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int64, c_int64, c_int, c_void_p, c_void_p]),

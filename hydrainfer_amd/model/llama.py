@@ -110,7 +110,7 @@ class LlamaForCausalLM:
         self.use_wide = os.environ.get("HX_WIDE", "1") == "1"
         # ... with silu * mul inside the norm + gate|up launch (round 5: both K halves in one workgroup, no slabs)
         self.use_wide_silu = os.environ.get("HX_WIDE_SILU", "1") == "1"
-        # the layers of a step of <= 32 rows on these launches: issued by one native call (decode_step)
+        # the layers of a step of <= 32 rows on these launches: a native call each (decode_step)
         self.one_call = True
         self.sample_out: Optional[Tensor] = None   # int64 [rows]: forward() writes the sampled ids here (decode loops)
         self.xreg_sync: Optional[Tensor] = None   # [L, 2, XREG_SYNC_WORDS] of the last step (word 1 = wait gave up)
@@ -392,14 +392,15 @@ class LlamaForCausalLM:
         else:
             rms_norm(x, h, st["l0.norm1"], eps)
         if self.one_call and fused and nf_gu and (L == 1 or "l1.wqkv" in self.dw) and all(f"l{l}.wo" in self.dw_lds for l in range(L)) and "l0.wqkv" in self.dw_lds:
-            layers = []
-            for l in range(L):
-                ap = model_params.attention_params[l]
-                layers.append(DecodeLayer(*ap.kv_cache.get_kv_cache(), ap.new_cache_slots, ap.q_cu_seq_lens, ap.kv_cu_seq_lens, ap.block_tables,
-                                          ap.cu_blocks_lens, ap.kv_max_seq_len, ap.decode_rank, self.dw[f"l{l}.wqkv"] if l else self.dw_lds["l0.wqkv"],
-                                          self.dw_lds[f"l{l}.wo"], self.dw[f"l{l}.wdown"], self.packed_x[f"l{l}.wgu"], st[f"l{l}.norm2"],
-                                          st[f"l{l + 1}.norm1"] if l + 1 < L else st["norm"]))
-            decode_layers(h, x, xf, actf, ws, ws_q, sync, inter, H, D, position_ids, self.cos_sin, D ** -0.5, eps, nf_qkv, layers)
+            def layer(l: int) -> DecodeLayer:
+                ap, last = model_params.attention_params[l], l + 1 == L
+                return DecodeLayer(*ap.kv_cache.get_kv_cache(), ap.new_cache_slots, ap.q_cu_seq_lens, ap.kv_cu_seq_lens, ap.block_tables,
+                                   ap.cu_blocks_lens, ap.kv_max_seq_len, ap.decode_rank,
+                                   None if last else self.dw[f"l{l + 1}.wqkv"], self.dw_lds[f"l{l}.wo"], self.dw[f"l{l}.wdown"],
+                                   self.packed_x[f"l{l}.wgu"], st[f"l{l}.norm2"], st["norm"] if last else st[f"l{l + 1}.norm1"])
+            s_qkv = self._partial(x, "l0.wqkv", ws_q)
+            decode_layers(h, x, xf, actf, ws, ws_q, sync, inter, H, D, position_ids, self.cos_sin, D ** -0.5, eps, nf_qkv, s_qkv,
+                          map(layer, range(L)))
             return x
         s_qkv = None
         for l in range(L):

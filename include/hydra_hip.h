@@ -425,32 +425,31 @@ typedef struct hx_fused_decode_args {
 int hx_decode_attention_fused(const hx_attn_args* args, const hx_fused_decode_args* fused,
                               hx_stream stream);
 
-/* The layers of a decode step of <= 32 rows in one call: for every layer the qkv product, hx_decode_attention_fused, the o product,
- * hx_norm_gate_up_silu_xreg and the down product, with add + RMSNorm between a layer and the next (inside the next qkv product with
- * norm_in_qkv, hx_norm_linear_decode_xreg; else hx_add_rms_norm_slabs_ex) and behind the last.  The first layer's qkv product reads x
- * row-major, the others' (HX_DW_XREG) and the down products' activations are fragment-major. */
+/* A layer of a decode step of <= 32 rows in one call: with qkv_slabs slabs of its qkv product in ws_qkv,
+ * hx_decode_attention_fused, the o product, hx_norm_gate_up_silu_xreg, the down product, then add + RMSNorm and the next layer's qkv
+ * product — in one launch with norm_in_qkv (hx_norm_linear_decode_xreg, or hx_add_rms_norm_slabs_ex and hx_linear_decode_ex) — or, for
+ * the last layer (next_qkv.packed NULL), the final norm.  Returns the number of slabs left for the next layer (0 behind the last) or a
+ * negative hx_status. */
 typedef struct hx_decode_layer {
-  hx_attn_args attn;           /* out: [rows][n_heads * head_dim]; workspace: hx_decode_layers_workspace_bytes, layers may share both */
+  hx_attn_args attn;           /* out: [rows][n_heads * head_dim] scratch; its workspace as for hx_mha_varlen_fwd */
   hx_fused_decode_args fused;  /* qkv_partial / qkv_splits are set from the qkv product */
-  hx_decode_weight qkv, o, down;
+  hx_decode_weight o;          /* reads attn.out row-major */
+  hx_decode_weight down, next_qkv;      /* XREG layout: fragment-major activations */
   const void* gate_up;         /* packed with HX_DW_GATE_UP on the XREG layout */
   const void* norm_mlp;        /* weights of the norm before the feed-forward ... */
   const void* norm_next;       /* ... and of the next layer's first one (last layer: the final norm) */
-} hx_decode_layer;
-typedef struct hx_decode_layers_args {
+  int32_t* sync;               /* [2][HX_XREG_SYNC_WORDS], zero, this layer's own */
   void* h;                     /* [rows][hidden]: the residual, updated */
-  void* x;                     /* [rows][hidden]: normed input of the first layer; receives the final norm's output */
+  void* x;                     /* [rows][hidden]: receives the final norm's output (last layer) */
   void* x_frag;                /* hx_fragment_major_elems(rows, hidden) elements of scratch */
   void* act;                   /* hx_fragment_major_elems(rows, inter) elements of scratch */
   float* ws;                   /* slabs of the o and down products */
-  float* ws_qkv;               /* slabs of the qkv product; may be ws unless norm_in_qkv */
+  float* ws_qkv;               /* slabs of the qkv products; may be ws unless norm_in_qkv */
   int64_t ws_bytes, ws_qkv_bytes, rows, hidden, inter;
-  int32_t* sync;               /* [n_layers][2][HX_XREG_SYNC_WORDS], zero */
   float epsilon;
   int32_t norm_in_qkv, dtype;
-} hx_decode_layers_args;
-int64_t hx_decode_layers_workspace_bytes(const hx_decode_layer* layers, int32_t n_layers);
-int hx_decode_layers(const hx_decode_layers_args* args, const hx_decode_layer* layers, int32_t n_layers, hx_stream stream);
+} hx_decode_layer;
+int hx_decode_layer_step(const hx_decode_layer* layer, int32_t qkv_slabs, hx_stream stream);
 
 /* ------------------------------------------------------------------------
  * Cache-block migration between GPUs / processes.

@@ -235,7 +235,7 @@ def test_decode_with_norm_fused_launches_equals_separate_launches(dt):
 @pytest.mark.gpu
 @pytest.mark.parametrize("hidden, inter, layers, batch", [(1024, 2816, 3, 1), (1024, 2816, 1, 32), (2048, 5632, 3, 5)])
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
-def test_layers_in_one_call_equal_the_launches_one_by_one(hidden, inter, layers, batch, dt):
+def test_layers_in_one_call_each_equal_the_launches_one_by_one(hidden, inter, layers, batch, dt):
     """The next layer's norm inside its qkv product (width 1024) and as a launch of its own (width 2048, two K splits): sampled
     tokens and the KV pool bit-identical, eager steps and replayed graphs."""
     from hydrainfer_amd.model import llama
