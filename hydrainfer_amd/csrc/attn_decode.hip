@@ -665,7 +665,29 @@ int decode_pick_splits(int batch, int n_heads, int max_seqlen_k, int requested) 
   // mid-size batches, context <= 2048 keys: one 8-wave workgroup per (sequence, head) and no
   // combine launch.  Measured in the 7B decode graph (bench.py --batch N, whole step): batch 6 / 8 /
   // 12 / 16: -2.5 / -2.0 / -3.4 / -1.9 %; batch <= 4 or >= 20: the split (resp. 4-wave) form wins
-  if (base >= g_decode_small_lo && base <= g_decode_small_hi && n_tiles <= 128) return 1;
+  // — where their workgroups fill whole rounds of the 256 compute units: a compute unit streams at most 1.3 times its share of
+  // the memory's rate, and 320 workgroups leave three quarters of the chip one of two.  Then the smallest split whose
+  // workgroups fill nine tenths of their rounds, four only for longer contexts (contexts of 705 / 1100 / 2047 keys, us, one workgroup a pair and split:
+  // 160 pairs 17 / 23 / 39 and (3) 15.5 / 21 / 33; 320 30 / 43 / 74 and (3) 25 / 36 / 61; 384 31 / 43 / 75 and (2) 28 / 41 / 69;
+  // 192 17 / 24 / 39 and (4) 18.5 / 23 / 36; 256, whole as they are, 19 / 28 / 47 and (2) 21 / 29 / 48).
+  auto filled = [&](int64_t ns) { return (double)(base * ns) / (double)((base * ns + 255) / 256 * 256); };
+  if (base >= g_decode_small_lo && base <= g_decode_small_hi && n_tiles <= 128) {
+    if (n_tiles >= 40 && filled(1) < 0.8)
+      for (int ns = 2; ns <= (n_tiles >= 80 ? 4 : 3); ++ns)
+        if (filled(ns) >= 0.9) return ns;
+    return 1;
+  }
+  // Few pairs: a round of workgroups, two for contexts from 1024 keys on, at most eight a pair with four tiles or more each; contexts of up to
+  // 384 keys (more than 80 pairs: 512) whole, without a combine launch.  Contexts of 300 / 705 / 1100 / 2047 keys, us, one split for every 16 tiles as before and
+  // this: 16 pairs 7.9 / 11.5 / 11 / 11 and 7.9 / 9.3 / 10.1 / 11.2; 64 9.2 / 12.5 / 13.4 / 17.1 and 9.2 / 11.2 / 12.9 / 16.8; 80 9.6 / 13.3 /
+  // 16 / 22 and 9.6 / 12.1 / 14.5 / 20; 128 9.5 / 14.7 / 18.1 / 28.6 and 9.5 / 14.3 / 17.5 / 26.2.
+  if (base < g_decode_small_lo && n_tiles <= 128) {
+    if (n_tiles <= (base > 80 ? 32 : 24)) return 1;
+    int64_t ns = (n_tiles >= 64 ? 512 : 256) / base;
+    if (ns > 8) ns = 256 / base < 8 ? 256 / base : 8;
+    if (ns > n_tiles / 4) ns = n_tiles / 4;
+    return ns < 1 ? 1 : (int)ns;
+  }
   int64_t want = (1024 + base - 1) / base;       // ~4 workgroups per CU
   int64_t cap = n_tiles / 16;                    // >= 16 tiles (4 per wave) per split
   if (cap < 1) cap = 1;

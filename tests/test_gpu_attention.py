@@ -107,6 +107,21 @@ def test_decode_long_context_and_split_kv():
         assert_close_t(out, ref, 1e-3, 1e-3, what=f"splits={splits}")
 
 
+# the splits that the library chooses by itself: few pairs of a sequence and a head with contexts on both sides of 384, 512, 1024 and 1264 keys, pair
+# counts that fill a round of compute units (256) and that do not (144, 288, 384), one short sequence beside a long one
+@pytest.mark.parametrize("batch, H", [(1, 1), (1, 16), (1, 40), (4, 32), (9, 16), (16, 16), (9, 32), (12, 32)])
+@pytest.mark.parametrize("longest", [384, 385, 513, 640, 1024, 1280, 2048, 2049])
+def test_decode_splits_by_rule(batch, H, longest):
+    from oracle import ops
+    dt = torch.bfloat16
+    kv_lens = [longest] + [1 + (longest * s) // batch for s in range(1, batch)]
+    q, kc, vc, cu_q, cu_k, bt, cu_b = _random_paged(batch, H, H, 64, kv_lens, [1] * batch, dt, seed=longest + batch)
+    ref = ops.paged_attention(q, kc, vc, cu_q, cu_k, bt, cu_b)
+    out = _run(q, kc, vc, cu_q, cu_k, bt, cu_b, 1, longest)
+    atol, rtol = ATTN_TOL[dt]
+    assert_close_t(out, ref, atol, rtol, what=f"{batch} x {H} heads, {longest} keys")
+
+
 def test_mixed_prefill_decode_and_block_sizes():
     from oracle import ops
     for dt in (torch.float16, torch.bfloat16):
