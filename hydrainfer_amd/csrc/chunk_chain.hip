@@ -1,14 +1,21 @@
-// chunk_chain.hip — the recurrences with a decay per key channel over portions of prompts, sixteen tokens at a time (chunk_scan.hip says
-// how), in two launches: what does not depend on the state — A, the prefixed queries, the suffixed keys, all of it vector work — is
-// made for all chunks at once on the whole chip, and the chain of chunks is left with the products of the state.  One launch has these
-// made beside the chain, on the same SIMDs and once per 64 value channels: a chunk of the gated form with 128 x 128 took 2.6 us there and
-// takes 1.5 here, of which 0.95 are the products.  (Vector instructions of a consumer's own wave do not run beside its float products: a
-// multiplication behind each of them costs 7 cycles of 32; those of other waves cost nothing.  So results leave through LDS by the
-// waves that bring rows in.)  Measured, gated form, one launch and two with the norm: 4 portions of 797 - 1151 tokens, 32 heads of 128 x
-// 128 206 and 176 us; one of 1151, 4 heads 189 and 115, 64 x 64 117 and 72.  The first launch takes 53 us of the 176 (vector work: 560
-// instructions a wave of four tokens; 164 MB written), and so what it costs is weighed against the chain (chunk_scan_workspace).
-// Head-wise decays gain too little: with A and M made ahead the chain of the delta rule is bound by its own waves (2.5 -> 2.3 us a
-// chunk, 104 products of 32 cycles and 140 vector instructions of 7), and the launch ahead takes what it gives (204 and 199 us).
+// chunk_chain.hip — recurrences over portions of prompts, sixteen tokens at a time (chunk_scan.hip says how), in two launches: what
+// does not depend on the state — A, M, prefixed queries, suffixed keys, all of it vector work and a serial substitution — is made for all
+// chunks at once on the whole chip, and the chain of chunks is left with the products of the state.  One launch has these made beside
+// the chain, on the same SIMDs and once per 64 value channels.
+// What bounds the chain: a chunk is 104 float products a wave under the delta rule with 128 x 128 (68 without write strengths), 32 cycles
+// each, where a wave holds all keys of 16 value channels, and 140 (100) vector instructions that do not run beside the products of
+// their own wave (a multiplication behind a product costs 7 cycles; those of other waves cost it nothing).  So the keys of 16 value channels are
+// dealt to two waves, or to four where workgroups are few: a chunk then takes 1.1 to 1.7 us instead of 2.0 to 2.7 (reads from LDS
+// behind the barrier 0.3, products 0.25 a product with the state, sums and results 0.2, barrier 0.1).  Results and, under the delta rule, what the keys
+// read from the old state are shares of the parts; results leave by the waves that bring rows in, which add the shares up in
+// double.  A share comes in two numbers, what the state gave and what the chunk gave, so that it is rounded no more often than the
+// whole was: 2-norm of the error against 64 bits, one launch and two, 3 portions of 200 - 600 tokens, 16 heads of 128 x 128: delta 1.08
+// 1.02, decay 0.85 0.77, bonus 0.82 0.79 e-7 (added up in float and in one number 1.09, 0.85, 0.87).
+// Measured, one launch and two, us: 4 portions of 1000 tokens, 8 heads of 128 x 128: delta rule 166 and 131, decayed sum 127 and 83,
+// gated form (with its norm) 173 and 87, bonus form 160 and 101; one of 1151, 32 heads: 188 150, 144 95, 197 96, 182 113; 64 x 64: decayed sum 92 86, gated
+// form 121 81, bonus form 109 103; delta rule 122 128, which stays with one launch.  4 portions of 797 - 1151 tokens, 32 heads of 128 x 128, gated form 206 and 173 (54 of them the
+// first launch, 560 vector instructions a wave of four tokens and 164 MB written; delta rule 190 and 235, so the first launch is weighed
+// against the chain, chunk_scan_workspace).
 #include "chunk_parts.h"
 
 namespace {
@@ -49,23 +56,145 @@ struct MadeRows {
   }
 };
 
-// A chunk's results [16][VW] on their way from LDS, where they stand by row, to memory: 256 threads, four channels each.
-template <bool VEC>
-__device__ __forceinline__ void write_results(const ChunkScanArgs& a, const float* lds, int64_t t0, int n, int head, int col0, int tid) {
-  const int t = tid / (VW / 4), col = col0 + tid % (VW / 4) * 4;
-  const f32x4 o = *reinterpret_cast<const f32x4*>(lds + row_of_token(t) * VS + tid % (VW / 4) * 4);
-  float* to = a.out + (t0 + t) * ((int64_t)a.heads * a.V) + (int64_t)head * a.V + col;
-  if (t >= n) return;
-  if (VEC) {
-    if (col < a.V) *reinterpret_cast<f32x4*>(to) = o;
-  } else {
+// ---------------------------------------------------------------------------------------------------------------
+// What does not depend on the state, all chunks at once.
+// ---------------------------------------------------------------------------------------------------------------
+// What one chunk needs besides its rows: A | M (T while it is made; delta rule) | prefix, suffix, what the prefix's rounding left over
+template <bool DELTA>
+constexpr int kMadeHead = (DELTA ? 2 : 1) * C * RA + 3 * C;
+
+// A wave's (x k^T)[i, j] with rows i = 4 g + e and column j = m: tokens 4 e + g and t_m; N chains
+template <int KP, int N>
+__device__ __forceinline__ f32x4 with_keys(const float* rows_x, const float* k, int m, int g) {
+  constexpr int RS = KP + 4;
+  f32x4 p[N];
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (col + e < a.V) to[e] = o[e];
+  for (int i = 0; i < N; ++i) p[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int kt = 0; kt < KP / 16; ++kt) {
+    const f32x4 x = *reinterpret_cast<const f32x4*>(rows_x + m * RS + 16 * kt + 4 * g);
+    const f32x4 y = *reinterpret_cast<const f32x4*>(k + m * RS + 16 * kt + 4 * g);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) p[(4 * kt + e) % N] = mma4(x[e], y[e], p[(4 * kt + e) % N]);
+  }
+#pragma unroll
+  for (int n = N / 2; n > 0; n >>= 1)
+#pragma unroll
+    for (int i = 0; i < n; ++i) p[i] += p[i + n];
+  return p[0];
+}
+__device__ __forceinline__ void chunk_decays(const float* sc, float (&d)[C]) {
+#pragma unroll
+  for (int i = 0; i < C / 4; ++i) {
+    const f32x4 x = *reinterpret_cast<const f32x4*>(sc + 4 * i);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) d[4 * i + e] = x[e];
+  }
+}
+// A, prefixes and suffixes: with sixteen chains and products of decays rounded once, as A's rounding is the larger part of a
+// result's error.  scalars: the chunk's per head numbers besides.
+template <int KP>
+__device__ __forceinline__ void make_A(const float* q, const float* k, const float* sc, float* A, float* scalars, int m, int g, int t_m) {
+  const f32x4 xk = with_keys<KP, 16>(q, k, m, g);
+  float d[C];
+  chunk_decays(sc, d);
+  Product run, mine[4];                                   // run = prod(t_m < r <= t) d_r, kept at the lane's four rows
+#pragma unroll
+  for (int t = 0; t < C; ++t) {
+    run.by(t > t_m ? d[t] : 1.f);
+    const bool here = (t & 3) == 0 || (t & 3) == g;
+    mine[t >> 2].hi = here ? run.hi : mine[t >> 2].hi;
+    mine[t >> 2].lo = here ? run.lo : mine[t >> 2].lo;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) A[(4 * g + e) * RA + m] = t_m <= 4 * e + g ? mine[e].times(xk[e]) : 0.f;
+  if (g == 0) scalars[C + m] = run.value();               // behind token t_m
+  if (m == 0) {                                           // up to the rows' tokens: the first one's decay and all behind it
+    f32x4 prefix, rest;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      prefix[e] = mine[e].times(d[0]);
+      rest[e] = mine[e].rest(d[0], prefix[e]);
+    }
+    *reinterpret_cast<f32x4*>(scalars + 4 * g) = prefix;
+    *reinterpret_cast<f32x4*>(scalars + 2 * C + 4 * g) = rest;
+  }
+}
+template <int KP>
+__device__ __forceinline__ void make_M(const float* k, const float* sc, float* A, int m, int g, int t_m) {      // A: T (by tokens), then M
+  const f32x4 xk = with_keys<KP, 4>(k, k, m, g);
+  float d[C], run = 1.f, mine[4];
+  chunk_decays(sc, d);
+#pragma unroll
+  for (int t = 0; t < C; ++t) {
+    run = t > t_m ? run * d[t] : 1.f;
+    mine[t >> 2] = (t & 3) == 0 || (t & 3) == g ? run : mine[t >> 2];
+  }
+  const f32x4 b = *reinterpret_cast<const f32x4*>(sc + 2 * C + 4 * g);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) A[(4 * e + g) * RA + t_m] = t_m < 4 * e + g ? b[e] * xk[e] * mine[e] : 0.f;      // (T: by tokens)
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  // column t_m of (I + T)^-1: x_t = [t == t_m] - sum(s < t) T[t, s] x_s
+  float x[C];
+#pragma unroll
+  for (int t = 0; t < C; ++t) {
+    float s0 = t == t_m ? 1.f : 0.f, s1 = 0.f;
+#pragma unroll
+    for (int s = 0; s < t; s += 4) {
+      const f32x4 T = *reinterpret_cast<const f32x4*>(A + t * RA + s);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (s + e >= t) continue;
+        if (e & 1) s1 -= T[e] * x[s + e];
+        else s0 -= T[e] * x[s + e];
+      }
+    }
+    x[t] = s0 + s1;
+    if (t & 1) asm volatile("" ::: "memory");           // (two rows of T in registers at a time, not all of them)
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();                      // T has been read
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  if (g == 0) {
+#pragma unroll
+    for (int t = 0; t < C; ++t) A[row_of_token(t) * RA + m] = x[t];
   }
 }
 
-// What the chunks need besides their values, all chunks at once.
+// One decay per token and head: wave 0 A, prefixes and suffixes, wave 1 M.  (As chunk_head_kernel makes them; made by calls of these
+// functions there, its chunks take 6 % longer.)
+template <int KP, bool DELTA, typename QK, bool VEC>
+__global__ __launch_bounds__(128, 4) void chunk_head_make_kernel(ChunkScanArgs a) {
+  constexpr int RS = KP + 4, kMade = kMadeHead<DELTA>;
+  __shared__ __attribute__((aligned(16))) float rows[2 * C * RS + 3 * C + kMade];
+  const int head = blockIdx.x % (unsigned)a.heads;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int g = lane >> 4, m = lane & 15;
+  const ChunkAt at = chunk_at(a, blockIdx.x / (unsigned)a.heads);
+  if (at.n <= 0) return;                                  // (the whole workgroup)
+  const int qk_head = head / (a.heads / a.qk_heads);
+  float *sc = rows + 2 * C * RS, *A = sc + 3 * C;
+  Rows<QK, VEC, KP, 64> x;
+  const int64_t stride = wave == 0 ? a.q_stride : a.k_stride;
+  x.fetch((const typename QK::storage*)(wave == 0 ? a.q : a.k) + at.t0 * stride + (int64_t)qk_head * a.K, stride, 0, a.K, at.n, lane);
+  const int64_t th = (at.t0 + min(m, at.n - 1)) * a.heads + head;
+  const float decay = a.decay[th], beta = DELTA ? a.beta[th] : 0.f;
+  x.store(rows + wave * C * RS, 0, a.K, at.n, 1.f, lane);
+  if (threadIdx.x < C) {                                  // (decays by token, the others by row; a row past the portion changes nothing)
+    sc[m] = m < at.n ? decay : 1.f;
+    sc[2 * C + row_of_token(m)] = m < at.n ? beta : 0.f;
+  }
+  lds_barrier();
+  if (wave == 0) make_A<KP>(rows, rows + C * RS, sc, A, A + kMade - 3 * C, m, g, row_of_token(m));
+  else if constexpr (DELTA) make_M<KP>(rows + C * RS, sc, A + C * RA, m, g, row_of_token(m));
+  lds_barrier();
+  float* to = a.made + (int64_t)blockIdx.x * kMade;
+  for (int i = 4 * threadIdx.x; i < kMade; i += 4 * 128) *reinterpret_cast<f32x4*>(to + i) = *reinterpret_cast<const f32x4*>(A + i);
+}
+
+// One decay per token and key channel.
 template <int KP, int FORM, typename QK, bool VEC>
 __global__ __launch_bounds__(256, 4) void chunk_channel_make_kernel(ChunkScanArgs a) {
   constexpr int RS = KP + 4, NP = KP / 64, kGate = kGateFloats<KP, FORM>, kMade = kMadeChannel<KP, FORM>;
@@ -90,142 +219,314 @@ __global__ __launch_bounds__(256, 4) void chunk_channel_make_kernel(ChunkScanArg
   for (int i = 4 * threadIdx.x; i < kMade; i += 4 * 256) *reinterpret_cast<f32x4*>(to + i) = *reinterpret_cast<const f32x4*>(P + i);
 }
 
-template <int KP, int FORM, typename VT, bool VEC>
-__global__ __launch_bounds__(512, KP == 64 ? 4 : 2) void chunk_channel_chain_kernel(ChunkScanArgs a) {
-  constexpr int KT = KP / 16, RS = KP + 4;
-  constexpr bool BONUS = FORM == hxm::kChunkBonus;
-  constexpr int kMade = kMadeChannel<KP, FORM>;
-  extern __shared__ __attribute__((aligned(16))) float lds[];      // made[2] | values[2] | results[2]
-  const int seq = blockIdx.z, head = blockIdx.x, col0 = (int)blockIdx.y * VW;
+// ---------------------------------------------------------------------------------------------------------------
+// The chain.  Eight consumer waves hold the state, 32 key channels of 16 value channels each; four more bring in what a chunk takes,
+// kAhead chunks ahead of the interval that puts it in LDS, and take results out.
+// ---------------------------------------------------------------------------------------------------------------
+// delta rule: q | k | v | write strength, and A | M | scalars; decayed sum: the same with value scales and without M; a decay per
+// channel: v, and what chunk_channel_make_kernel makes
+template <int KP, int FORM, bool CHANNEL, int KS>
+struct Image {
+  static constexpr int W = 16 * 8 / KS, WS = W + 4;       // value channels a workgroup
+  static constexpr bool DELTA = FORM == hxm::kChunkDelta;
+  static constexpr int kMade = CHANNEL ? kMadeChannel<KP, CHANNEL ? FORM : hxm::kChunkDecay> : kMadeHead<DELTA>;
+  static constexpr int kRows = CHANNEL ? 0 : 2 * C * (KP + 4) + C;
+  static constexpr int kFloats = kMade + kRows + C * WS;
+  static constexpr int kImages = DELTA ? 3 : 2;
+  static constexpr int kShares = KS * C * WS;             // the key parts' shares of y, or of a chunk's results
+  // results whose rounding shows (the gated form's are rounded to an activation behind its norm) in two numbers
+  static constexpr int kResult = (FORM == hxm::kChunkGated ? 1 : 2) * kShares;
+  static constexpr int kLds = kImages * kFloats + 2 * kResult + (DELTA ? 2 * kShares : 0);
+};
+
+template <int KP, int FORM, bool CHANNEL, int KS, typename QK, typename VT, bool VEC>
+__global__ __launch_bounds__(768) void chunk_chain_kernel(ChunkScanArgs a) {
+  typedef Image<KP, FORM, CHANNEL, KS> I;
+  constexpr int RS = KP + 4, KT = KP / 16 / KS, W = I::W, WS = I::WS, kMade = I::kMade, kLead = I::kImages - 2;
+  constexpr bool DELTA = I::DELTA, BONUS = FORM == hxm::kChunkBonus;
+  extern __shared__ __attribute__((aligned(16))) float lds[];      // images | results[2] | y[2]
+  const int seq = blockIdx.z, head = blockIdx.x, col0 = (int)blockIdx.y * W;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int g = lane >> 4, m = lane & 15;
   const int64_t t_begin = a.q_cu[seq];
   const int n_tok = (int)(a.q_cu[seq + 1] - t_begin);
   if (n_tok <= 0) return;                                 // (the whole workgroup)
   const int n_chunks = (n_tok + C - 1) / C;
-  float* slot = a.state + (int64_t)a.slots[seq] * a.slot_stride + (int64_t)head * a.K * a.V;
-  auto made = [&](int chunk) { return lds + (chunk & 1) * kMade; };
-  auto vals = [&](int chunk) { return lds + 2 * kMade + (chunk & 1) * (C * VS); };
-  auto outs = [&](int chunk) { return lds + 2 * kMade + (2 + (chunk & 1)) * (C * VS); };
+  auto made = [&](int chunk) { return lds + chunk % I::kImages * I::kFloats; };
+  auto rows = [&](int chunk) { return made(chunk) + kMade; };
+  auto vals = [&](int chunk) { return made(chunk) + kMade + I::kRows; };
+  auto outs = [&](int chunk) { return lds + I::kImages * I::kFloats + (chunk & 1) * I::kResult; };
+  auto ys = [&](int chunk) { return lds + I::kImages * I::kFloats + 2 * I::kResult + (chunk & 1) * I::kShares; };      // (delta rule)
   auto rows_of = [&](int chunk) { return min(C, n_tok - chunk * C); };
 
   if (wave >= 4) {
-    const int cw = wave - 4, col = col0 + 16 * cw + m;
+    const int part = (wave - 4) % KS, cw = (wave - 4) / KS, col = col0 + 16 * cw + m, k0 = 16 * KT * part;
+    float* slot = a.state + (int64_t)a.slots[seq] * a.slot_stride + (int64_t)head * a.K * a.V + (int64_t)k0 * a.V;
     State<KT> st;
-    st.load(slot, a.K, a.V, col, g, a.positions[t_begin] == 0);
-    lds_barrier();
-    // What a chunk's first products take is read behind the barrier that ends the chunk before, whose products with its keys follow it.
-    f32x4 qx[KT];
-    read_row(qx, made(0) + m * RS + 4 * g);
-    for (int c = 0; c < n_chunks; ++c) {
-      const float* p = made(c);
-      const float *kt_ = p + C * RS, *A = kt_ + KP * RA, *total = A + C * RA;
-      const float* vs = vals(c) + 4 * g * VS + 16 * cw + m;
-      f32x4 w, kx[KT], d[KT];
-      s16x4 w16, ky[KT];
+    st.load(slot, a.K - k0, a.V, col, g, a.positions[t_begin] == 0);
+    const int share = part * C * WS + 4 * g * WS + 16 * cw + m;      // this lane's column of rows 4 g ..
+    // the keys' part of rows (token m) of x times the state; four chains of at most sixteen keys
+    auto times_state = [&](const float* row) __attribute__((always_inline)) {
+      f32x4 x[KT], o[4];
+      read_row(x, row + k0);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) w[e] = vs[e * VS];
-      const f32x4 A_row = *reinterpret_cast<const f32x4*>(A + (BONUS ? row_of_token(m) : m) * RA + 4 * g);
+      for (int e = 0; e < 4; ++e) o[e] = mma4(x[0][e], st.S[0][e], f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-      for (int kt = 0; kt < KT; ++kt) {
-        d[kt] = *reinterpret_cast<const f32x4*>(total + 16 * kt + 4 * g);
-        kx[kt] = *reinterpret_cast<const f32x4*>(kt_ + (16 * kt + m) * RA + 4 * g);
-        if constexpr (BONUS) ky[kt] = *reinterpret_cast<const s16x4*>(reinterpret_cast<const u16*>(total + KP) + (16 * kt + m) * RA + 4 * g);
-      }
-      const f32x4 before = st.times(qx);
-      __builtin_amdgcn_sched_group_barrier(0x100, 64, 0);
-      const bool odd = some_not_finite(w);
-      f32x4 in_order = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (odd) in_order = times_rows_in_order(A, m, g, w);
+      for (int kt = 1; kt < KT; ++kt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = mma4(x[kt][e], st.S[kt][e], o[e]);
+      return (o[0] + o[1]) + (o[2] + o[3]);
+    };
+    auto put = [&](float* to, f32x4 v) __attribute__((always_inline)) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) to[share + e * WS] = v[e];
+    };
+    if constexpr (DELTA) {
       lds_barrier();
-      read_row(qx, made(c + 1) + m * RS + 4 * g);         // (behind the last chunk: the one before it, unused)
+      put(ys(0), times_state(rows(0) + C * RS + m * RS + 4 * g));
+    }
+    for (int c = 0; c < n_chunks; ++c) {
+      lds_barrier();
+      const float *p = made(c), *A = CHANNEL ? p + C * RS + KP * RA : p, *r = rows(c), *vs = vals(c) + 4 * g * WS + 16 * cw + m;
+      f32x4 w, kx[KT], d[KT], pre, suf, rest;
+      s16x4 ky[KT];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = vs[e * WS];
+      const f32x4 A_row = *reinterpret_cast<const f32x4*>(A + (BONUS ? row_of_token(m) : m) * RA + 4 * g);
+      float total = 0.f;
+      if constexpr (CHANNEL) {
+        const float *kt_ = p + C * RS, *totals = A + C * RA;
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) {
+          kx[kt] = *reinterpret_cast<const f32x4*>(kt_ + (k0 + 16 * kt + m) * RA + 4 * g);
+          d[kt] = *reinterpret_cast<const f32x4*>(totals + k0 + 16 * kt + 4 * g);
+          if constexpr (BONUS) ky[kt] = *reinterpret_cast<const s16x4*>(reinterpret_cast<const u16*>(totals + KP) + (k0 + 16 * kt + m) * RA + 4 * g);
+        }
+      } else {
+        const float* scalars = p + kMade - 3 * C;
+        pre = *reinterpret_cast<const f32x4*>(scalars + 4 * g);
+        suf = *reinterpret_cast<const f32x4*>(scalars + C + 4 * g);
+        rest = *reinterpret_cast<const f32x4*>(scalars + 2 * C + 4 * g);
+        total = scalars[C - 1];
+        const f32x4 scale = *reinterpret_cast<const f32x4*>(r + 2 * C * RS + 4 * g);
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) kx[kt][e] = r[C * RS + (4 * g + e) * RS + k0 + 16 * kt + m];
+        if constexpr (DELTA) {
+          const float* y = ys(c) + 4 * g * WS + 16 * cw + m;
+          f32x4 s;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) s[e] = y[e * WS] + y[C * WS + e * WS];
+          if constexpr (KS == 4) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] += y[2 * C * WS + e * WS] + y[3 * C * WS + e * WS];
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) w[e] = scale[e] * (w[e] - pre[e] * s[e]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) w[e] *= scale[e];
+        }
+      }
+      const f32x4 x = w;
+      if constexpr (DELTA) w = times_rows(*reinterpret_cast<const f32x4*>(p + C * RA + m * RA + 4 * g), x);
+      const bool odd = some_not_finite(w);                // (delta rule: of x, then every row of w)
+      if constexpr (DELTA) {
+        if (odd) w = times_rows_in_order(p + C * RA, m, g, x);
+      }
+      // this part's share of the results: its keys' of what the state holds, its tokens' of the chunk's own
+      const f32x4 before = times_state((CHANNEL ? p : r) + m * RS + 4 * g);
+      f32x4 first = before, second = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (odd) {
+        if (part == 0) second = times_rows_in_order(A, m, g, w);
+        if (FORM == hxm::kChunkGated) second += before;
+      } else if constexpr (BONUS) {                       // (in double: what rounding leaves over goes to the smaller number)
+        f64x4 sum = f64x4{0., 0., 0., 0.};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (e / (4 / KS) == part) sum = __builtin_amdgcn_mfma_f64_16x16x4f64((double)A_row[e], (double)w[e], sum, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          second[e] = (float)sum[e];
+          first[e] += (float)(sum[e] - (double)second[e]);
+        }
+      } else {
+        if (FORM == hxm::kChunkGated) second = before;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (e / (4 / KS) == part) second = mma4(A_row[e], w[e], second);
+      }
+      if constexpr (!CHANNEL) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          first[e] = before[e] * pre[e];
+          second[e] += __builtin_fmaf(before[e], rest[e], __builtin_fmaf(before[e], pre[e], -first[e]));
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] *= suf[e];
+      }
+      s16x4 w16;
 #pragma unroll
       for (int e = 0; e < 4; ++e) w16[e] = (short)BF16::from_float(w[e]);
-      f32x4 o = BONUS ? times_rows_double(A_row, w, before) : times_rows(A_row, w, before);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = odd ? before[e] + in_order[e] : o[e];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) outs(c)[(4 * g + e) * VS + 16 * cw + m] = o[e];
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt) {
         if constexpr (BONUS) {
-          const f32x4 rest = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ky[kt], w16, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+          const f32x4 more = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ky[kt], w16, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) st.S[kt][e] = __builtin_fmaf(st.S[kt][e], d[kt][e], rest[e]);
-        } else {
+          for (int e = 0; e < 4; ++e) st.S[kt][e] = __builtin_fmaf(st.S[kt][e], d[kt][e], more[e]);
+        } else if constexpr (CHANNEL) {
           st.S[kt] *= d[kt];
+        } else {
+          st.S[kt] *= total;
         }
+      }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) st.S[kt] = mma4(kx[kt][e], w[e], st.S[kt]);
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) st.S[kt] = mma4(kx[kt][e], w[e], st.S[kt]);
+      put(outs(c), second);
+      if constexpr (FORM != hxm::kChunkGated) put(outs(c) + I::kShares, first);
+      if constexpr (DELTA) {
+        if (c + 1 < n_chunks) put(ys(c + 1), times_state(rows(c + 1) + C * RS + m * RS + 4 * g));
       }
     }
     lds_barrier();
-    st.store(slot, a.K, a.V, col, g);
+    st.store(slot, a.K - k0, a.V, col, g);
     return;
   }
 
-  const typename VT::storage* vp = (const typename VT::storage*)a.v + t_begin * a.v_stride + (int64_t)head * a.V;
-  const float* sp = FORM == hxm::kChunkDecay ? (a.vscale ? a.vscale : a.decay) + t_begin * a.heads + head : nullptr;
-  // Four waves that bring in the values and what was made of the keys and queries, kAhead chunks ahead of the interval that puts them in
-  // LDS: an interval is shorter than a load's way.  Behind the last chunk the last one comes again.
-  const int tid = (int)threadIdx.x;
+  const int tid = (int)threadIdx.x, qk_head = head / (a.heads / a.qk_heads);
+  const typename QK::storage* q = (const typename QK::storage*)a.q + t_begin * a.q_stride + (int64_t)qk_head * a.K;
+  const typename QK::storage* k = (const typename QK::storage*)a.k + t_begin * a.k_stride + (int64_t)qk_head * a.K;
+  const typename VT::storage* v = (const typename VT::storage*)a.v + t_begin * a.v_stride + (int64_t)head * a.V;
+  const bool scaled = !BONUS && FORM != hxm::kChunkGated && (DELTA || a.vscale);
+  const float* per_token = DELTA ? a.beta : a.vscale ? a.vscale : a.decay;
   const float* from = a.made + (chunk_number(t_begin, seq) * a.heads + head) * kMade;
+  const int v_row = tid / (W / 4), v_col = tid % (W / 4) * 4;      // (16 W / 4 threads)
+  const bool v_mine = 16 * W / 4 >= 256 || v_row < C;
   struct Set {
+    Rows<QK, VEC, KP, 256> q, k;           // (a decay per head)
+    Piece<VT, 4, VEC> v;
     MadeRows<kMade, 256> made;
-    Rows<VT, VEC, VW, 256> v;
     float scale;
   } sets[kAhead];
   auto fetch = [&](Set& s, int chunk) __attribute__((always_inline)) {
     chunk = min(chunk, n_chunks - 1);
     const int n = rows_of(chunk);
     const int64_t t0 = (int64_t)chunk * C;
+    if constexpr (!CHANNEL) {
+      s.q.fetch(q + t0 * a.q_stride, a.q_stride, 0, a.K, n, tid);
+      s.k.fetch(k + t0 * a.k_stride, a.k_stride, 0, a.K, n, tid);
+    }
     s.made.fetch(from + (int64_t)chunk * a.heads * kMade, tid);
-    s.v.fetch(vp + t0 * a.v_stride, a.v_stride, col0, a.V, n, tid);
-    if constexpr (FORM == hxm::kChunkDecay) s.scale = sp[(t0 + min(s.v.row_of(0, tid), n - 1)) * a.heads];
+    s.v.load(v + (t0 + min(v_row, n - 1)) * a.v_stride, col0 + v_col, a.V);
+    if constexpr (FORM == hxm::kChunkDecay || DELTA) s.scale = per_token[(t_begin + t0 + min(CHANNEL ? v_row : m, n - 1)) * a.heads + head];
   };
   auto store = [&](const Set& s, int chunk) __attribute__((always_inline)) {
     if (chunk >= n_chunks) return;
+    const int n = rows_of(chunk);
+    float* r = rows(chunk);
     s.made.store(made(chunk), tid);
-    s.v.store(vals(chunk), col0, a.V, rows_of(chunk), FORM == hxm::kChunkDecay && a.vscale ? s.scale : 1.f, tid);
+    if constexpr (!CHANNEL) {
+      s.q.store(r, 0, a.K, n, 1.f, tid);
+      s.k.store(r + C * RS, 0, a.K, n, 1.f, tid);
+      if (tid < C) r[2 * C * RS + row_of_token(m)] = m >= n ? (DELTA ? 0.f : 1.f) : scaled ? s.scale : 1.f;      // (a row past the portion changes nothing)
+    }
+    if (v_mine) {
+      f32x4 f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) f[j] = s.v.get(j, v_row < n, col0 + v_col, a.V) * (CHANNEL && scaled ? s.scale : 1.f);
+      *reinterpret_cast<f32x4*>(vals(chunk) + row_of_token(v_row) * WS + v_col) = f;
+    }
+  };
+  // results: the parts' shares added up in double, rounded once
+  auto write = [&](int chunk) __attribute__((always_inline)) {
+    const int col = col0 + v_col;
+    if (!v_mine || v_row >= rows_of(chunk)) return;
+    const float* o = outs(chunk) + row_of_token(v_row) * WS + v_col;
+    f32x4 f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      double sum = o[j];
+#pragma unroll
+      for (int share = 1; share < I::kResult / (C * WS); ++share) sum += (double)o[share * C * WS + j];
+      f[j] = (float)sum;
+    }
+    float* to = a.out + (t_begin + (int64_t)chunk * C + v_row) * ((int64_t)a.heads * a.V) + (int64_t)head * a.V + col;
+    if (VEC) {
+      if (col < a.V) *reinterpret_cast<f32x4*>(to) = f;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (col + j < a.V) to[j] = f[j];
+    }
   };
 #pragma unroll
   for (int i = 0; i < kAhead; ++i) fetch(sets[i], i);
-  for (int c0 = -1; c0 < n_chunks; c0 += kAhead) {
+  for (int c0 = -kLead; c0 < n_chunks; c0 += kAhead) {
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
       const int c = c0 + i;
       if (c >= n_chunks) break;
-      store(sets[i], c + 1);
-      fetch(sets[i], c + 1 + kAhead);
-      if (c >= 2) write_results<VEC>(a, outs(c - 2), t_begin + (int64_t)(c - 2) * C, C, head, col0, tid);      // (chunk c - 1's are being written)
+      store(sets[i], c + kLead);
+      fetch(sets[i], c + kLead + kAhead);
+      if (c >= 2) write(c - 2);                           // (chunk c - 1's are being made)
       lds_barrier();
     }
   }
-  if (n_chunks >= 2) write_results<VEC>(a, outs(n_chunks - 2), t_begin + (int64_t)(n_chunks - 2) * C, C, head, col0, tid);
+  if (n_chunks >= 2) write(n_chunks - 2);
   lds_barrier();
-  write_results<VEC>(a, outs(n_chunks - 1), t_begin + (int64_t)(n_chunks - 1) * C, rows_of(n_chunks - 1), head, col0, tid);
+  write(n_chunks - 1);
 }
 
 // numbers that chunks may have
 int64_t chunk_numbers(const ChunkScanArgs& a) { return a.n_tokens / C + a.n_seq; }
+// With 32 value channels a workgroup every one of them has a compute unit: the keys go to four waves.  (Else twice the rows would be
+// brought in for each channel: the gated form above 146 us in the chain, 115 with 64 channels.)
+bool few_chains(const ChunkScanArgs& a) { return (int64_t)a.n_seq * a.heads * ((a.V + 31) / 32) <= 256; }
 template <int KP>
 int64_t made_floats(const ChunkScanArgs& a) {
-  return a.form == hxm::kChunkGated ? kMadeChannel<KP, hxm::kChunkGated> : a.form == hxm::kChunkBonus ? kMadeChannel<KP, hxm::kChunkBonus> : kMadeChannel<KP, hxm::kChunkDecay>;
+  if (a.form == hxm::kChunkGated) return kMadeChannel<KP, hxm::kChunkGated>;
+  if (a.form == hxm::kChunkBonus) return kMadeChannel<KP, hxm::kChunkBonus>;
+  if (a.per_channel) return kMadeChannel<KP, hxm::kChunkDecay>;
+  return a.form == hxm::kChunkDelta ? kMadeHead<true> : kMadeHead<false>;
 }
 
+template <int KP, int FORM, bool CHANNEL, int KS, typename QK, typename VT, bool VEC>
+int launch_parts(const ChunkScanArgs& a, hipStream_t s) {
+  typedef Image<KP, FORM, CHANNEL, KS> I;
+  return launch_chunks(chunk_chain_kernel<KP, FORM, CHANNEL, KS, QK, VT, VEC>, dim3((unsigned)a.heads, (unsigned)((a.V + I::W - 1) / I::W), (unsigned)a.n_seq), 768,
+                       sizeof(float) * I::kLds, a, s);
+}
+template <int KP, int FORM, bool CHANNEL, typename QK, typename VT, bool VEC>
+int launch_chain(const ChunkScanArgs& a, hipStream_t s) {
+  if constexpr (KP == 128) {
+    if (few_chains(a)) return launch_parts<KP, FORM, CHANNEL, 4, QK, VT, VEC>(a, s);
+  }
+  return launch_parts<KP, FORM, CHANNEL, 2, QK, VT, VEC>(a, s);
+}
 template <int KP, int FORM, typename QK, typename VT, bool VEC>
 int launch_channel(const ChunkScanArgs& a, hipStream_t s) {
   const int rc = launch_chunks(chunk_channel_make_kernel<KP, FORM, QK, VEC>, dim3((unsigned)(chunk_numbers(a) * a.heads)), 256, 0, a, s);
-  if (rc != HX_OK) return rc;
-  return launch_chunks(chunk_channel_chain_kernel<KP, FORM, VT, VEC>, dim3((unsigned)a.heads, (unsigned)((a.V + VW - 1) / VW), (unsigned)a.n_seq), 512,
-                       sizeof(float) * (2 * kMadeChannel<KP, FORM> + 4 * C * VS), a, s);
+  return rc != HX_OK ? rc : launch_chain<KP, FORM, true, F32, VT, VEC>(a, s);
+}
+template <int KP, int FORM, typename QK, typename VT, bool VEC>
+int launch_head(const ChunkScanArgs& a, hipStream_t s) {
+  constexpr bool DELTA = FORM == hxm::kChunkDelta;
+  const int rc = launch_chunks(chunk_head_make_kernel<KP, DELTA, QK, VEC>, dim3((unsigned)(chunk_numbers(a) * a.heads)), 128, 0, a, s);
+  return rc != HX_OK ? rc : launch_chain<KP, FORM, false, QK, VT, VEC>(a, s);
 }
 
 template <int KP, typename QK, typename VT, bool VEC>
 int launch_form(const ChunkScanArgs& a, hipStream_t s) {
   if (a.form == hxm::kChunkGated) return launch_channel<KP, hxm::kChunkGated, QK, VT, VEC>(a, s);
   if (a.form == hxm::kChunkBonus) return launch_channel<KP, hxm::kChunkBonus, QK, VT, VEC>(a, s);
-  return launch_channel<KP, hxm::kChunkDecay, QK, VT, VEC>(a, s);
+  if (a.per_channel) return launch_channel<KP, hxm::kChunkDecay, QK, VT, VEC>(a, s);
+  if constexpr (KP == 128) {
+    if (a.form == hxm::kChunkDelta) return launch_head<KP, hxm::kChunkDelta, QK, VT, VEC>(a, s);
+  }
+  return launch_head<KP, hxm::kChunkDecay, QK, VT, VEC>(a, s);
 }
 
 template <typename QK, typename VT>
@@ -240,20 +541,28 @@ int launch_width(const ChunkScanArgs& a, hipStream_t s) {
 namespace hxm {
 
 int64_t chunk_scan_workspace(const ChunkScanArgs& a) {
-  if (!chunk_scan_fits(a) || !(a.per_channel || a.form == kChunkGated)) return 0;
+  if (!chunk_scan_fits(a) || (a.V + 31) / 32 > 65535 || (a.form == kChunkDelta && a.K <= 64)) return 0;
   const int64_t workgroups = chunk_numbers(a) * a.heads;
   const int64_t floats = workgroups * (a.K <= 64 ? made_floats<64>(a) : made_floats<128>(a));
   if (workgroups > INT32_MAX || floats > (int64_t)1 << 28) return 0;      // (1 GiB)
-  // Two launches save `gain` us for a chunk of the chain and take `cost` us for each chunk and head, and 2 us.  Fitted to batches of 1 to
-  // 64 portions of 32 to 1151 tokens and 4 to 32 heads, one launch and two, us: gated form, 128 x 128, 32 heads: 1 of 1151 197 131, 4 of
-  // 1000 189 175, 4 of 128 34 34, 4 of 64 21 24; 64 x 64: 1 of 1151 121 84, 4 of 128 22 24, 8 of 512 68 77; bonus form, 64 x 64, 32 heads: 1 of
-  // 1151 109 95, 4 of 1000 100 105, 8 heads: 4 of 256 29 28, of 64 11 14; 128 x 128, 32 heads: 4 of 256 50 56, 16 heads 48 47; a decay per
-  // channel, 128 x 64, 32 heads: 4 of 256 44 47, 16 heads 43 41, 8 of 512 85 124.
+  // Two launches save `few` or `many` us for a chunk of the chain and take `cost` us for each chunk and head, and 2 us.  Fitted to 12 batches
+  // of 1 to 16 portions of 64 to 1151 tokens, 8 to 32 heads and 12 forms and sizes; one launch and two, us, about the line: delta rule, 128 x 128, 32
+  // heads: 2 portions of 128 27 28, 2 of 600 104 91, 16 heads: 4 of 1000 167 143; decayed sum, 128 x 64, 32 heads: 4 of 256 40 33, 8 of 512 74 79;
+  // 64 x 64: one of 1151 92 86, 4 of 1000 83 86; gated form, 128 x 128, 32 heads: 4 of 64 21 23, 4 of 256 57 53; 64 x 64: 4 of 1000 115 97, 8 of 512 71
+  // 83; bonus form, 128 x 128, 16 heads: 4 of 1000 162 121, 8 of 512 95 98; 64 x 64, 8 heads: 8 of 512 52 55; a decay per channel, 128 x 64, 32 heads: 4 of 256 45
+  // 39, 8 of 512 89 123.
+  // (And one launch takes 20 us: shorter calls are bound by their caller, who would have to ask for a workspace: 19.2 and 21.7 us.)
+  struct Line { double few, many, cost, one; };           // few: keys dealt to four waves; one: us a chunk in one launch
   const bool wide = a.K > 64;
-  const double gain = a.form == kChunkGated ? (wide ? 1.0 : 0.6) : a.form == kChunkBonus ? (wide ? 0.6 : 0.28) : wide ? 0.7 : 0.28, cost = wide ? 0.0067 : 0.0025;
+  const Line line = a.form == kChunkGated   ? (wide ? Line{1.5, 1.05, 0.0067, 2.6} : Line{0.6, 0.6, 0.003, 1.6})
+                    : a.form == kChunkBonus ? (wide ? Line{1.1, 0.6, 0.008, 2.4} : Line{0.15, 0.15, 0.0027, 1.5})
+                    : a.form == kChunkDelta ? Line{0.65, 0.0, 0.0044, 2.7}
+                    : a.per_channel         ? (wide ? Line{1.15, 1.0, 0.0085, 2.3} : Line{0.2, 0.2, 0.003, 1.4})
+                                            : (wide ? Line{0.78, 0.3, 0.0025, 2.0} : Line{0.1, 0.1, 0.0009, 1.3});
   const double mean = (double)a.n_tokens / a.n_seq / C, longest = a.longest > 0 ? (double)a.longest / C : mean;
   const int64_t chains = (int64_t)a.n_seq * a.heads * ((a.V + VW - 1) / VW);      // a compute unit takes one at a time
-  return gain * (chains <= 256 ? longest : mean * ((chains + 255) / 256)) > cost * a.n_tokens / C * a.heads + 3.0 ? floats : 0;
+  const double chain = chains <= 256 ? longest : mean * ((chains + 255) / 256), saved = (few_chains(a) ? line.few : line.many) * chain;
+  return chain * line.one >= 20.0 && saved > line.cost * a.n_tokens / C * a.heads + 3.5 ? floats : 0;
 }
 
 int chunk_chain(const ChunkScanArgs& a, hipStream_t s) {
