@@ -562,12 +562,18 @@ class LlamaForCausalLM:
     def forward_logits(self, input_ids_or_embeds, position_ids, model_params) -> Tensor:
         x = self.forward_hidden(input_ids_or_embeds, position_ids, model_params)
         w = self.state["lm_head"]
+        # Up to 16 rows the weight-streaming product (its workgroups read whole rows, the library's tiles of 16 rows leave the memory half
+        # idle), where the weights come from memory: behind prompts, and from 256 MiB on, which the memory-side cache does not keep from
+        # step to step.  32064 outputs of 2048 / 4096 / 5120 from memory, library and this, us: 1 row 39 28, 61 52, 71 56; 16 rows 40
+        # 31, 60 56, 68 63; 17 rows 29 32, 62 57, 58 65.  Steps of one layer of width 4096, whose 263 MB stay: 132 and 140.
+        few = (self.use_hip_gemm and x.shape[0] <= 16 and hip_gemm.supported(x, w)
+               and (not model_params.all_sequences_decode or w.numel() * w.element_size() > 256 << 20))
         if launch_plan.current() is None:
-            return torch.matmul(x, w.t())
-        # a launch plan is being recorded: the library GEMM is a host-side step of the plan between two native
+            return hip_gemm.linear_decode(x, w) if few else torch.matmul(x, w.t())
+        # a launch plan is being recorded: the product is a host-side step of the plan between two native
         # launch segments, writing into a buffer of the plan's pool
         logits = torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype, device=x.device)
-        launch_plan.host_op(lambda: torch.matmul(x, w.t(), out=logits))
+        launch_plan.host_op((lambda: hip_gemm.linear_decode(x, w, logits)) if few else (lambda: torch.matmul(x, w.t(), out=logits)))
         return logits
 
     def forward(self, input_ids_or_embeds, position_ids, model_params) -> Tensor:

@@ -260,3 +260,20 @@ def test_layers_in_one_call_each_equal_the_launches_one_by_one(hidden, inter, la
     assert calls and all(calls)
     for tokens, pool in outs[1:]:
         assert torch.equal(outs[0][0], tokens) and torch.equal(outs[0][1], pool)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 16, 17])
+@pytest.mark.parametrize("vocab", [2048, 2050])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_logits_of_few_rows(rows, vocab, dt):
+    """On both sides of the 16 rows that the weight-streaming product takes, and with outputs that it does not take."""
+    from hydrainfer_amd.model.llama import LanguageModelParameters, LlamaForCausalLM, LlamaShape
+    model = LlamaForCausalLM.random_init(LlamaShape(1024, 2816, 1, 8, 8, 128, vocab), dt, torch.device("cuda:0"), seed=3)
+    x = torch.randn((rows, 1024), generator=torch.Generator().manual_seed(rows)).to(dt).cuda()
+    model.forward_hidden = lambda *a: x
+    got, want = model.forward_logits(None, None, LanguageModelParameters([], False)).float(), x.float() @ model.state["lm_head"].float().t()
+    # sums in float (1024 products, a unit of 2^-24 of the sum of their sizes each at worst), rounded once to dt
+    unit = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11
+    size = x.float().abs() @ model.state["lm_head"].float().abs().t()
+    assert got.shape == (rows, vocab) and bool(((got - want).abs() <= unit * want.abs() + 1024 * 2.0 ** -24 * size + 1e-7).all())
