@@ -380,6 +380,10 @@ int launch_gemm_mb(const GemmParams& p, hipStream_t stream) {
   // workgroups with 3 resp. 2 row groups per wave; qkv / o keep 4 waves x 1
   if (units > 4096) { nw = 8; rpw = 3; }
   else if (p.n_splits >= 8) { nw = 8; rpw = 2; }
+  // Up to 16 rows and 512 units (an o projection of width 2048: 256) four waves a workgroup leave half of the compute units without one, and
+  // one streams no more than 30 GB/s: two waves, us: 1 row, 2048 x 2048 4.6 -> 4.0, 2048 x 4096 5.6 -> 5.1, 1024 x 1024 4.2 -> 3.5
+  // (17 - 32 rows, whose x slice takes two waves longer to bring in, 5.5 -> 5.9)
+  if (units <= 512 && MB == 1 && p.packed) nw = 2;
   // 33..64 batch rows: the x slice alone is 133 KB of LDS, so one workgroup per CU whatever its
   // size — four waves cannot keep the CU streaming.  8 waves everywhere; cold-weight timing at
   // M = 48 / 64 (tools/bench_gemm_m.py): qkv 51 -> 31 us with two row groups per wave, o 21.5 -> 18.5
@@ -407,6 +411,9 @@ int launch_gemm_mb(const GemmParams& p, hipStream_t stream) {
     }
   }
   if (g_force_nw == 4 || g_force_nw == 8) nw = g_force_nw;
+  if constexpr (MB == 1) {
+    if (nw == 2 && rpw == 1) return launch_gemm_cfg<T, MB, 1, 2>(p, stream);
+  }
   if (g_force_r >= 1 && g_force_r <= 4) rpw = g_force_r;
   if (nw == 4) {
     switch (rpw) {

@@ -929,3 +929,17 @@ def test_gate_up_silu_rows_refuses():
         with pytest.raises(_lib.HydraHipError):
             gemm.gate_up_silu_rows(a, b)
         assert not gemm.gate_up_rows_supported(a, b)
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("N, K", [(16, 256), (48, 1024), (2048, 2048), (4096, 2048), (4112, 2048), (2048, 4352)])
+@pytest.mark.parametrize("M", [1, 16, 17])
+def test_packed_product_of_few_units_is_the_same(N, K, M, dt):
+    """Two waves a workgroup up to 16 rows and 512 (row group, split) pairs, four beside: bit-identical to the row-major product."""
+    from hydrainfer_amd._C.kernel import gemm
+    g = torch.Generator().manual_seed(N + K + M)
+    x, w = torch.randn((M, K), generator=g).to(dt).cuda(), torch.randn((N, K), generator=g).to(dt).cuda()
+    a, b = (torch.full((gemm.workspace_floats(M, N, K),), float("nan"), device="cuda") for _ in range(2))
+    s = gemm.linear_decode_partial(x, w, a)
+    assert gemm.linear_decode_partial_packed(x, gemm.pack_weight(w), N, b) == s
+    assert torch.equal(a[:s * M * N], b[:s * M * N]) and bool(torch.isfinite(a[:s * M * N]).all())
