@@ -13,7 +13,7 @@
 // 1.02, decay 0.85 0.77, bonus 0.82 0.79 e-7 (added up in float and in one number 1.09, 0.85, 0.87).
 // Measured, one launch and two, us: 4 portions of 1000 tokens, 8 heads of 128 x 128: delta rule 166 and 131, decayed sum 127 and 83,
 // gated form (with its norm) 173 and 87, bonus form 160 and 101; one of 1151, 32 heads: 188 150, 144 95, 197 96, 182 113; 64 x 64: decayed sum 92 86, gated
-// form 121 81, bonus form 109 103; delta rule 122 128, which stays with one launch.  4 portions of 797 - 1151 tokens, 32 heads of 128 x 128, gated form 206 and 173 (54 of them the
+// form 121 81, bonus form 109 103; delta rule 122 128, which stays with one launch.  4 portions of 797 - 1151 tokens, 32 heads of 128 x 128, gated form 206 and 171 (53 of them the
 // first launch, 560 vector instructions a wave of four tokens and 164 MB written; delta rule 190 and 235, so the first launch is weighed
 // against the chain, chunk_scan_workspace).
 #include "chunk_parts.h"

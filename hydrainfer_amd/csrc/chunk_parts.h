@@ -273,7 +273,9 @@ struct GateRows {
         const bool in = t < n && d0 + p < K;                // (a row past the portion, a channel past the key: nothing changes)
         const float qv = q[j].get(p, t < n, d0, K), kv = k[j].get(p, t < n, d0, K);
         if constexpr (GATED) {
-          G[t * KP + d0 + p] = in ? own.low[p] + (1.0f - own.low[p]) * sigmoid_gate(kv + own.bias[p]) : 1.f;
+          float f = own.low[p] + (1.0f - own.low[p]) * sigmoid_gate(kv + own.bias[p]);
+          asm("" : "+v"(f));                                // (no branch around it: it would stand between every two elements)
+          G[t * KP + d0 + p] = in ? f : 1.f;
           G[C * KP + t * KP + d0 + p] = qv * sigmoid_gate(qv);
         } else {
           G[t * KP + d0 + p] = in ? d[j].get(p, true, d0, K) : 1.f;

@@ -20,7 +20,7 @@
 // What bounds it now: the chunks of a sequence follow each other (2.5 us each with states of 128 x 128; 1.8 us of float matrix
 // products on the SIMDs that hold a consumer and a maker of A or M).  Measured against one token at a time, 4 portions of 797 -
 // 1151 tokens: delta rule, 32 heads of 128 x 128, 479 -> 189 us; decayed sum, 64 heads of 128 x 64, 432 -> 143 us; bonus form, 32
-// heads of 64 x 64, 207 -> 105 us; gated form, 32 heads of 128 x 128, 720 -> 205 us with its norm (173 in the two launches of chunk_chain.hip, which
+// heads of 64 x 64, 207 -> 105 us; gated form, 32 heads of 128 x 128, 720 -> 205 us with its norm (171 in the two launches of chunk_chain.hip, which
 // batches of few chains for their length take).
 // What the rounding costs: a token at a time rounds a state's element once a token, and each rounding decays with the state.  Here
 // the products of decays, of keys with them and the chunk's sums are rounded besides, and four things keep that from showing: sums
