@@ -766,9 +766,11 @@ int launch_grouped_tiles(u16* y, const u16* x, int64_t x_stride, const int32_t* 
   return hxm::check_launch();
 }
 
-// The same, four elements a lane: width, row strides and pointers are multiples of four elements.  Rows and weights of the
-// token's choices are read once into LDS; the choices' rows are requested four at a time.
-template <typename A>
+// The same, NE elements a lane: width, row strides and pointers are multiples of NE elements.  Rows and weights of the
+// token's choices are read once into LDS; the choices' rows are requested four at a time, with the shared expert's.  Bound by memory:
+// 4 of 16 experts of 4096 and a shared one, 3989 tokens 37.5 us (5.2 TB/s; 42.8 with four elements a lane and a token a workgroup), 2500 tokens of 2048
+// 11.8 (14.2).
+template <typename A, int NE>
 __global__ __launch_bounds__(256) void moe_combine_vec_kernel(typename A::storage* __restrict__ out, const typename A::storage* __restrict__ y,
                                                               const int32_t* __restrict__ row_of, const float* __restrict__ weights,
                                                               const typename A::storage* __restrict__ shared,
@@ -788,35 +790,40 @@ __global__ __launch_bounds__(256) void moe_combine_vec_kernel(typename A::storag
   if (identity)
     for (int k = 0; k < top; ++k)
       if (rows[k] < 0) idw += wts[k];
-  for (int64_t i = 4 * ((int64_t)blockIdx.y * 256 + threadIdx.x); i < W; i += 1024 * (int64_t)gridDim.y) {
-    f32x4 u = f32x4{0.f, 0.f, 0.f, 0.f};
+  typedef typename A::storage vec __attribute__((ext_vector_type(NE)));
+  auto load = [](const typename A::storage* p) { return *reinterpret_cast<const vec*>(p); };
+  for (int64_t i = NE * ((int64_t)blockIdx.y * 256 + threadIdx.x); i < W; i += NE * 256 * (int64_t)gridDim.y) {
+    float u[NE];
+#pragma unroll
+    for (int e = 0; e < NE; ++e) u[e] = 0.f;
+    vec sh;
+    if (shared) sh = load(shared + t * W + i);
     for (int k0 = 0; k0 < top; k0 += 4) {
-      f32x4 v[4];
+      vec v[4];
       float w[4];
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const bool there = k0 + k < top && rows[k0 + k < top ? k0 + k : 0] >= 0;
         const int at = there ? k0 + k : 0;
         w[k] = there ? wts[at] : 0.f;
-        v[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (there) v[k] = Row4<A>::load(y + (int64_t)rows[at] * W + i);
+#pragma unroll
+        for (int e = 0; e < NE; ++e) v[k][e] = 0;
+        if (there) v[k] = load(y + (int64_t)rows[at] * W + i);
       }
 #pragma unroll
       for (int k = 0; k < 4; ++k)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) u[e] += w[k] * v[k][e];
+        for (int e = 0; e < NE; ++e) u[e] += w[k] * A::to_float(v[k][e]);
     }
     if (idw != 0.f) {
-      const f32x4 v = Row4<A>::load(identity + t * identity_stride + i);
+      const vec v = load(identity + t * identity_stride + i);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) u[e] += idw * v[e];
+      for (int e = 0; e < NE; ++e) u[e] += idw * A::to_float(v[e]);
     }
-    if (shared) {
-      const f32x4 v = Row4<A>::load(shared + t * W + i);
+    vec o;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) u[e] += g * v[e];
-    }
-    Row4<A>::store(out + t * W + i, u);
+    for (int e = 0; e < NE; ++e) o[e] = A::from_float(shared ? u[e] + g * A::to_float(sh[e]) : u[e]);
+    *reinterpret_cast<vec*>(out + t * W + i) = o;
   }
 }
 
@@ -961,20 +968,24 @@ extern "C" int hxm_moe_combine(void* out, const void* y, const int32_t* row_of, 
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid((unsigned)n_tokens), block(256);
   const uintptr_t es = dtype == HX_F32 ? 4 : 2;
-  auto by4 = [&](const void* p) { return (uintptr_t)p % (4 * es) == 0; };
-  if (top <= 64 && width % 4 == 0 && identity_stride % 4 == 0 && by4(out) && by4(y) && by4(shared) && by4(identity)) {
-    const dim3 vgrid((unsigned)n_tokens, n_tokens <= 256 ? (unsigned)((width + 1023) / 1024 < 64 ? (width + 1023) / 1024 : 64) : 1u);
-    switch (dtype) {
-      case HX_F32:
-        moe_combine_vec_kernel<F32><<<vgrid, block, 0, s>>>((float*)out, (const float*)y, row_of, weights, (const float*)shared, shared_gate,
-                                                            gate_stride, top, width, (const float*)identity, identity_stride);
-        break;
-      case HX_BF16:
-        moe_combine_vec_kernel<BF16><<<vgrid, block, 0, s>>>((u16*)out, (const u16*)y, row_of, weights, (const u16*)shared, shared_gate,
-                                                             gate_stride, top, width, (const u16*)identity, identity_stride);
-        break;
-      default: return HX_ERR_DTYPE;
-    }
+  auto by = [&](int ne) {
+    auto aligned = [&](const void* p) { return (uintptr_t)p % (ne * es) == 0; };
+    return top <= 64 && width % ne == 0 && identity_stride % ne == 0 && aligned(out) && aligned(y) && aligned(shared) && aligned(identity);
+  };
+  auto vgrid = [&](int ne) {              // a piece of the row a workgroup
+    const int64_t pieces = (width + 256 * ne - 1) / (256 * ne);
+    return dim3((unsigned)n_tokens, (unsigned)(pieces < 64 ? pieces : 64));
+  };
+  if (dtype == HX_F32 && by(4)) {
+    moe_combine_vec_kernel<F32, 4><<<vgrid(4), block, 0, s>>>((float*)out, (const float*)y, row_of, weights, (const float*)shared, shared_gate, gate_stride, top,
+                                                              width, (const float*)identity, identity_stride);
+    return hxm::check_launch();
+  }
+  if (dtype == HX_BF16 && by(4)) {
+    const int ne = n_tokens > 256 && by(8) ? 8 : 4;      // (few tokens: more workgroups; 200 tokens of 2048 3.9 and 4.3 us)
+    auto kernel = ne == 8 ? moe_combine_vec_kernel<BF16, 8> : moe_combine_vec_kernel<BF16, 4>;
+    kernel<<<vgrid(ne), block, 0, s>>>((u16*)out, (const u16*)y, row_of, weights, (const u16*)shared, shared_gate, gate_stride, top, width,
+                                                  (const u16*)identity, identity_stride);
     return hxm::check_launch();
   }
   switch (dtype) {

@@ -26,3 +26,26 @@ def test_router_forms(K, E, T, biased):
     want = torch.softmax(chosen, dim=1)
     # a logit off by eps moves a weight by at most 2 eps of itself; 1e-6 for the exponentials and the quotient
     assert bool(((weights.double() - want).abs() <= want * (2 * torch.expm1(2 * eps) + 1e-6) + 1e-30).all())
+
+
+# the combine (csrc/moe_mix.hip): rows in pieces of eight, four and single elements, on both sides of the 256 tokens up to which pieces are of four
+@pytest.mark.parametrize("W", [8, 1028, 2048, 2056, 4099])
+@pytest.mark.parametrize("T", [1, 256, 257])
+@pytest.mark.parametrize("top, shared, missing", [(1, False, False), (3, True, False), (5, True, True)])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_combine_pieces(W, T, top, shared, missing, dt):
+    from hydrainfer_amd._C.kernel.moe_mix import moe_combine
+    g = torch.Generator().manual_seed(W + T + top)
+    y, sh, same = (torch.randn(n, W, generator=g).to(dt) for n in (T * top, T, T))
+    row_of = torch.randperm(T * top, generator=g).int().view(T, top)
+    if missing:
+        row_of[::3, 1] = -1
+    w = torch.rand(T, top, generator=g)
+    got = moe_combine(y.cuda(), row_of.cuda(), w.cuda(), sh.cuda() if shared else None, identity=same.cuda() if missing else None).cpu()
+    parts = [torch.where(row_of[:, k:k + 1] >= 0, y[row_of[:, k].clamp(min=0).long()].double(), same.double() if missing else torch.zeros(())) * w[:, k:k + 1].double()
+             for k in range(top)]
+    parts += [sh.double()] if shared else []
+    want, size = sum(parts), sum(p.abs() for p in parts)
+    # at most seven sums in float and one rounding to the result's type
+    unit = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -23
+    assert bool(((got.double() - want).abs() <= unit * want.abs() + 8 * 2.0 ** -24 * size + 1e-30).all())
