@@ -58,6 +58,11 @@ __device__ __forceinline__ int wave_min_int(int v) {
 }
 __device__ __forceinline__ int wave_max_int(int v) { return -wave_min_int(-v); }
 
+__device__ __forceinline__ float halves_max(float v) {      // with lane ^ 32, without the LDS crossbar
+  const auto a = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
+  const unsigned a0 = a[0], a1 = a[1];
+  return fmaxf(__builtin_bit_cast(float, a0), __builtin_bit_cast(float, a1));
+}
 __device__ __forceinline__ float groups_max(float v) {      // over the four lanes with the same lane % 16
   const auto a = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
   const unsigned a0 = a[0], a1 = a[1];

@@ -632,12 +632,12 @@ __global__ __launch_bounds__(256) void biased_attn_group_kernel(hxm_biased_attn_
 //     while this one is worked on: two images, one barrier a tile.  Rows cannot be padded this way; their 16-byte chunks are
 //     swizzled by the lane that asks for them (keys: chunk ^ row, values: 64-byte quarter ^ row);
 //   * a row's weights refer to its largest score so far, 32 keys at a time.  That costs a pass over the accumulators for nearly every
-//     half tile; left up to 2^8 behind, it took 52 us instead of 57 and results were off by 3 % more, as the largest weights were
+//     half tile; left up to 2^8 behind, it took 5 us less and results were off by 3 % more, as the largest weights were
 //     rounded to bfloat16 instead of being 1.
 // The order of the row tiles: the XCDs (workgroups are dealt round robin) take key heads of their own where there are enough of
 // them, and of every sequence the tiles with the most keys come first.
-// Measured, 4 portions of 797 - 1151 tokens, 32 heads of 128 on 8 key heads, sinks: 221 us in the group form, 57 us
-// here (570 TFLOP/s of the pairs that a mask leaves); window of 512 and soft cap 223 and 68 us; chunks of 512 and slopes 163 and
+// Measured, 4 portions of 797 - 1151 tokens, 32 heads of 128 on 8 key heads, sinks: 221 us in the group form, 55 us
+// here (590 TFLOP/s of the pairs that a mask leaves); window of 512 and soft cap 223 and 68 us; chunks of 512 and slopes 163 and
 // 50 us.  Down to 64 rows of a key head it is the faster one (16 tokens behind 500 keys: 30 and 21 us).
 // ---------------------------------------------------------------------------------------------------------------
 template <int D, int V, bool MODS, bool FINE>      // MODS: slopes or a soft cap; FINE: every 32 keys' weights refer to their own largest score
@@ -695,24 +695,43 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
   // first key that some row sees, or behind the last, is not touched (its page may be gone): rows there repeat that key, masked.
   constexpr int RPK = 64 / LK, RPV = 64 / LV;
   const int rk = lane / LK, ck = lane % LK, rv = lane / LV, cv = lane % LV;
+  uint32_t ko[16 / RPK], vo[16 / RPV];       // a lane's part of a group of sixteen whole rows, in bytes
+#pragma unroll
+  for (int j = 0; j < 16 / RPK; ++j) ko[j] = (uint32_t)(2 * ((RPK * j + rk) * (uint32_t)a.cache_row_stride + 8 * (ck ^ kswz(RPK * j + rk))));
+#pragma unroll
+  for (int j = 0; j < 16 / RPV; ++j) vo[j] = (uint32_t)(2 * ((RPV * j + rv) * (uint32_t)a.cache_row_stride + 8 * (cv ^ vswz(RPV * j + rv))));
+  // A group that lies between the first and the last key that are seen needs no address of its own per row and tile: offsets made once
+  // here, the page's address in scalars.  (With 64-bit products and clamps for each row of each tile, and the maxima exchanged through
+  // LDS, 57.0 us where 55.0 now.  What is clamped, or rows of which 16 reach past 32 bits, in bytes, still goes that way.)
+  const bool near_rows = a.cache_row_stride >= 0 && a.cache_row_stride < (1 << 26);
   auto bring = [&](int t, int img) __attribute__((always_inline)) {
     const int key0 = min(max(t * KT + 16 * wave, k_first & ~15), k_last), r_min = k_first - key0, r_max = k_last - key0;
     const int page = bshift >= 0 ? key0 >> bshift : key0 / bs;
     const int64_t off = (int64_t)table[page] * a.cache_block_stride + (int64_t)(key0 - page * bs) * a.cache_row_stride;
     const uint32_t kd = lds0 + (uint32_t)(img * IMG + 16 * wave * RSK), vd = lds0 + (uint32_t)(img * IMG + KTILE + 16 * wave * RSV);
+    const u16 *kb = kc + off, *vb = vc + off;
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
     // (m0, the LDS address of the transfer, is a reserved register: nothing else in this kernel uses it)
+    if (near_rows && r_min <= 0 && r_max >= 15) {      // nothing to clamp
+#pragma unroll
+      for (int j = 0; j < 16 / RPK; ++j)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(ko[j]), "s"(kb), "s"(__builtin_amdgcn_readfirstlane(kd + 1024u * j)) : "memory", "m0");
+#pragma unroll
+      for (int j = 0; j < 16 / RPV; ++j)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(vo[j]), "s"(vb), "s"(__builtin_amdgcn_readfirstlane(vd + 1024u * j)) : "memory", "m0");
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < 16 / RPK; ++j) {
       const int rr = RPK * j + rk;
-      const u16* from = kc + off + (int64_t)max(min(rr, r_max), r_min) * a.cache_row_stride + 8 * (ck ^ kswz(rr));
+      const u16* from = kb + (int64_t)max(min(rr, r_max), r_min) * a.cache_row_stride + 8 * (ck ^ kswz(rr));
       asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(__builtin_amdgcn_readfirstlane(kd + 1024u * j)) : "memory", "m0");
     }
 #pragma unroll
     for (int j = 0; j < 16 / RPV; ++j) {
       const int rr = RPV * j + rv;
-      const u16* from = vc + off + (int64_t)max(min(rr, r_max), r_min) * a.cache_row_stride + 8 * (cv ^ vswz(rr));
+      const u16* from = vb + (int64_t)max(min(rr, r_max), r_min) * a.cache_row_stride + 8 * (cv ^ vswz(rr));
       asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(__builtin_amdgcn_readfirstlane(vd + 1024u * j)) : "memory", "m0");
     }
 #pragma clang diagnostic pop
@@ -822,7 +841,7 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
     for (int u = 0; u < 2; ++u) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) m_ref[u] = fmaxf(m_ref[u], s[u][e]);
-      m_ref[u] = fmaxf(m_ref[u], __shfl_xor(m_ref[u], 32, 64)) * unit;
+      m_ref[u] = halves_max(m_ref[u]) * unit;
       asm("" : "+v"(m_ref[u]));              // (rounded: left inside a difference below it would not be m_new's number)
       m_new[u] = fmaxf(u ? m_new[0] : m, m_ref[u]);
       if (!FINE) m_ref[u] = m_new[u];

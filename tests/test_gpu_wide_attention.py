@@ -211,3 +211,24 @@ def test_weights_round_no_more_than_in_the_tile_form(n, new, kv, extra):
                                softcap=cap, form=form).double().cpu()
         off[form] = float((got - want).norm() / want.norm())
     assert off["auto"] <= (1.0 if new == 1 else 1.005) * off["tile"], off
+
+
+# Rows of a group of sixteen are addressed by offsets of 32 bits up to a stride of 2 ** 26 elements (16 rows, in bytes), by pointers past
+# it and in groups that reach past the keys that are seen: the same bytes, so the same result to the last bit.
+@pytest.mark.parametrize("stride", [2 ** 26 - 8, 2 ** 26], ids=["near", "far"])
+@pytest.mark.parametrize("D, V", [(64, 64), (128, 128), (64, 128)])
+def test_rows_far_apart(stride, D, V):
+    from hydrainfer_amd._C.kernel.biased_attn import biased_attention
+    g = torch.Generator().manual_seed(D + V)
+    new, nb, H, hs = [40, 30], [3, 2], 4, max(D, V)
+    kv = [16 * 3 - 5, 16 * 2]
+    r = lambda *s: torch.randn(s, generator=g).bfloat16().cuda()
+    i = lambda x: torch.tensor(x, dtype=torch.int32).cuda()
+    q, k, v = r(sum(new), H, D), r(sum(nb), BLOCK, 1, hs), r(sum(nb), BLOCK, 1, hs)
+    table, cu_b, cu_q = torch.randperm(sum(nb), generator=g).int().cuda(), i([0, 3, 5]), i([0, 40, 70])
+    pos, seq = i(list(range(kv[0] - 40, kv[0])) + list(range(kv[1] - 30, kv[1]))), i([0] * 40 + [1] * 30)
+    call = lambda k, v: biased_attention(q, k, v, V, seq, pos, cu_q, table, cu_b, D ** -0.5, None, "causal", 0, max_q_len=40, max_kv_len=max(kv))
+    want = call(k, v)
+    room = torch.empty(sum(nb) * BLOCK * stride, dtype=torch.bfloat16, device="cuda")      # (10 GB, of which the rows are touched)
+    apart = [room[n * hs:].as_strided(x.shape, (BLOCK * stride, stride, hs, 1)).copy_(x) for n, x in enumerate((k, v))]
+    assert torch.equal(call(*apart), want)
