@@ -13,7 +13,8 @@ def supported(x: Tensor, weight: Tensor) -> bool:
     M, K = x.shape
     N = weight.shape[0]
     return (x.dtype in (torch.float16, torch.bfloat16) and 1 <= M <= 64 and N % 16 == 0 and K % 256 == 0
-            and x.stride(1) == 1 and weight.stride(1) == 1 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0)
+            and x.stride(1) == 1 and weight.stride(1) == 1 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
 
 
 def linear_decode(x: Tensor, weight: Tensor, out: Optional[Tensor] = None) -> Tensor:
@@ -22,7 +23,7 @@ def linear_decode(x: Tensor, weight: Tensor, out: Optional[Tensor] = None) -> Te
     if x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1] or x.dtype != weight.dtype:
         raise _lib.HydraHipError("linear_decode: x [M, K], weight [N, K], same dtype")
     if not supported(x, weight):
-        raise _lib.HydraHipError("linear_decode: needs M <= 64, N % 16 == 0, K % 256 == 0, fp16/bf16, contiguous rows")
+        raise _lib.HydraHipError("linear_decode: needs M <= 64, N % 16 == 0, K % 256 == 0, fp16/bf16, contiguous rows that start on 16 bytes")
     M, K = x.shape
     N = weight.shape[0]
     if out is None:
@@ -70,7 +71,7 @@ def linear_decode_partial(x: Tensor, weight: Tensor, partial: Tensor) -> int:
     buffer of at least workspace_floats(M, N, K) elements) for a fused consumer.  Returns n_splits."""
     _lib.require_gpu(x, weight, partial)
     if not supported(x, weight) or x.dtype != weight.dtype:
-        raise _lib.HydraHipError("linear_decode_partial: needs M <= 64, N % 16 == 0, K % 256 == 0, fp16/bf16")
+        raise _lib.HydraHipError("linear_decode_partial: needs M <= 64, N % 16 == 0, K % 256 == 0, fp16/bf16, rows that start on 16 bytes")
     if partial.dtype != torch.float32 or not partial.is_contiguous():
         raise _lib.HydraHipError("linear_decode_partial: partial must be contiguous float32")
     M, K = x.shape

@@ -277,3 +277,29 @@ def test_logits_of_few_rows(rows, vocab, dt):
     unit = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11
     size = x.float().abs() @ model.state["lm_head"].float().abs().t()
     assert got.shape == (rows, vocab) and bool(((got - want).abs() <= unit * want.abs() + 1024 * 2.0 ** -24 * size + 1e-7).all())
+
+
+def test_products_of_few_rows_ask_for_addresses():
+    """Rows that do not start on 16 bytes are left to the library."""
+    from hydrainfer_amd._C.kernel import gemm
+    flat = torch.zeros(16 * 256 + 8, dtype=torch.bfloat16)
+    for off in range(9):
+        a, whole = flat[off:off + 16 * 256].view(16, 256), torch.zeros((16, 256), dtype=torch.bfloat16)
+        assert gemm.supported(a, whole) == gemm.supported(whole, a) == (off % 8 == 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 16])
+def test_logits_of_a_head_off_sixteen_bytes(rows):
+    """A head that is a view into a flat buffer: the same logits as from a head of its own, behind prompts as in steps."""
+    from hydrainfer_amd.model.llama import LanguageModelParameters, LlamaForCausalLM, LlamaShape
+    model = LlamaForCausalLM.random_init(LlamaShape(1024, 2816, 1, 8, 8, 128, 2048), torch.bfloat16, torch.device("cuda:0"), seed=3)
+    x, head = torch.randn((rows, 1024), generator=torch.Generator().manual_seed(rows)).bfloat16().cuda(), model.state["lm_head"]
+    model.forward_hidden = lambda *a: x
+    flat = torch.empty(head.numel() + 1, dtype=head.dtype, device=head.device)
+    model.state["lm_head"] = flat[1:].view_as(head).copy_(head)
+    for step in (False, True):
+        got, want = model.forward_logits(None, None, LanguageModelParameters([], step)).float(), x.float() @ head.float().t()
+        # sums in float (1024 products, a unit of 2^-24 of the sum of their sizes each at worst), rounded once
+        bound = 2.0 ** -8 * want.abs() + 1024 * 2.0 ** -24 * (x.float().abs() @ head.float().abs().t()) + 1e-7
+        assert bool(((got - want).abs() <= bound).all())
