@@ -681,9 +681,13 @@ int decode_pick_splits(int batch, int n_heads, int max_seqlen_k, int requested) 
   // 384 keys (more than 80 pairs: 512) whole, without a combine launch.  Contexts of 300 / 705 / 1100 / 2047 keys, us, one split for every 16 tiles as before and
   // this: 16 pairs 7.9 / 11.5 / 11 / 11 and 7.9 / 9.3 / 10.1 / 11.2; 64 9.2 / 12.5 / 13.4 / 17.1 and 9.2 / 11.2 / 12.9 / 16.8; 80 9.6 / 13.3 /
   // 16 / 22 and 9.6 / 12.1 / 14.5 / 20; 128 9.5 / 14.7 / 18.1 / 28.6 and 9.5 / 14.3 / 17.5 / 26.2.
+  // From 129 pairs on a round is one workgroup a pair, which leaves up to half of the chip without one: two rounds from 768 keys on, with an even number
+  // of heads (contexts of 705 / 760 / 900 / 1005 keys, us, one, two and three splits: 132 pairs of 4 heads - / 15.7 / 18.6 / 19.5, - / 18.1 / 20.8 / 22.0 and
+  // - / 15.5 / 17.6 / 18.9; 144 of 16 15.5 / 16.4 / 18.7 / 19.8, 17.7 / 18.5 / 20.9 / 22.3 and 15.0 / 15.9 / 17.6 / 19.0; 150 of 10 - / 16.4 / 18.9 / 19.8, - / 18.8 /
+  // 21.0 / 22.4 and - / 16.4 / 18.1 / 19.4; odd numbers, 155 of 5 - / 16.0 / 18.3 / 19.1, - / 18.6 / 20.7 / 22.1 and - / 16.5 / 18.2 / 19.7).
   if (base < g_decode_small_lo && n_tiles <= 128) {
     if (n_tiles <= (base > 80 ? 32 : 24)) return 1;
-    int64_t ns = (n_tiles >= 64 ? 512 : 256) / base;
+    int64_t ns = (n_tiles >= (base > 128 && n_heads % 2 == 0 ? 48 : 64) ? 512 : 256) / base;
     if (ns > 8) ns = 256 / base < 8 ? 256 / base : 8;
     if (ns > n_tiles / 4) ns = n_tiles / 4;
     return ns < 1 ? 1 : (int)ns;
