@@ -657,7 +657,7 @@ int launch_decode_combine(const AttnParams& p, int batch, int head_dim, int dtyp
   return check_launch();
 }
 
-int decode_pick_splits(int batch, int n_heads, int max_seqlen_k, int requested) {
+int decode_pick_splits(int batch, int n_heads, int head_dim, int max_seqlen_k, int requested) {
   if (requested >= 1) return requested > 128 ? 128 : requested;
   const int64_t base = (int64_t)batch * n_heads;
   if (base >= 768) return 1;
@@ -669,24 +669,27 @@ int decode_pick_splits(int batch, int n_heads, int max_seqlen_k, int requested) 
   // the memory's rate, and 320 workgroups leave three quarters of the chip one of two.  Then the smallest split whose
   // workgroups fill nine tenths of their rounds, four only for longer contexts (contexts of 705 / 1100 / 2047 keys, us, one workgroup a pair and split:
   // 160 pairs 17 / 23 / 39 and (3) 15.5 / 21 / 33; 320 30 / 43 / 74 and (3) 25 / 36 / 61; 384 31 / 43 / 75 and (2) 28 / 41 / 69;
-  // 192 17 / 24 / 39 and (4) 18.5 / 23 / 36; 256, whole as they are, 19 / 28 / 47 and (2) 21 / 29 / 48).
+  // 192 17 / 24 / 39 and (4) 18.5 / 23 / 36; 256, whole as they are, 19 / 28 / 47 and (2) 21 / 29 / 48).  Those are heads of 128.  Heads of 64 gain from four later
+  // (1300 / 1400 keys, 192 pairs 17.8 / 19.4 and 18.6 / 18.8); heads of 256, of which one workgroup streams twice as much, only where pairs are more than a
+  // round (1280 / 1600 keys, 160 pairs 41.6 / 50.6 and 42.0 / 50.8, 192 46.8 / 57.3 and 49.1 / 59.2; 320 89.7 / 109 and 75.1 / 93.0).
   auto filled = [&](int64_t ns) { return (double)(base * ns) / (double)((base * ns + 255) / 256 * 256); };
   if (base >= g_decode_small_lo && base <= g_decode_small_hi && n_tiles <= 128) {
-    if (n_tiles >= 40 && filled(1) < 0.8)
-      for (int ns = 2; ns <= (n_tiles >= 80 ? 4 : 3); ++ns)
+    if (n_tiles >= 40 && filled(1) < 0.8 && (head_dim <= 128 || base > 256))
+      for (int ns = 2; ns <= (n_tiles >= (head_dim <= 64 ? 88 : 80) ? 4 : 3); ++ns)
         if (filled(ns) >= 0.9) return ns;
     return 1;
   }
   // Few pairs: a round of workgroups, two for contexts from 1024 keys on, at most eight a pair with four tiles or more each; contexts of up to
   // 384 keys (more than 80 pairs: 512) whole, without a combine launch.  Contexts of 300 / 705 / 1100 / 2047 keys, us, one split for every 16 tiles as before and
   // this: 16 pairs 7.9 / 11.5 / 11 / 11 and 7.9 / 9.3 / 10.1 / 11.2; 64 9.2 / 12.5 / 13.4 / 17.1 and 9.2 / 11.2 / 12.9 / 16.8; 80 9.6 / 13.3 /
-  // 16 / 22 and 9.6 / 12.1 / 14.5 / 20; 128 9.5 / 14.7 / 18.1 / 28.6 and 9.5 / 14.3 / 17.5 / 26.2.
+  // 16 / 22 and 9.6 / 12.1 / 14.5 / 20; 128 9.5 / 14.7 / 18.1 / 28.6 and 9.5 / 14.3 / 17.5 / 26.2.  Heads of 64 stay whole up to 480 keys (one split and as above, 420 /
+  // 450 keys: 8 pairs 7.4 / 7.6 and 8.0 / 8.2, 32 8.2 / 8.4 and 8.6 / 8.7, 80 8.5 / 8.8 and 9.2 / 9.0; 500 keys, two and as above: 8.1 7.5, 8.9 8.1, 9.2 9.1).
   // From 129 pairs on a round is one workgroup a pair, which leaves up to half of the chip without one: two rounds from 768 keys on, with an even number
   // of heads (contexts of 705 / 760 / 900 / 1005 keys, us, one, two and three splits: 132 pairs of 4 heads - / 15.7 / 18.6 / 19.5, - / 18.1 / 20.8 / 22.0 and
   // - / 15.5 / 17.6 / 18.9; 144 of 16 15.5 / 16.4 / 18.7 / 19.8, 17.7 / 18.5 / 20.9 / 22.3 and 15.0 / 15.9 / 17.6 / 19.0; 150 of 10 - / 16.4 / 18.9 / 19.8, - / 18.8 /
   // 21.0 / 22.4 and - / 16.4 / 18.1 / 19.4; odd numbers, 155 of 5 - / 16.0 / 18.3 / 19.1, - / 18.6 / 20.7 / 22.1 and - / 16.5 / 18.2 / 19.7).
   if (base < g_decode_small_lo && n_tiles <= 128) {
-    if (n_tiles <= (base > 80 ? 32 : 24)) return 1;
+    if (n_tiles <= (base > 80 ? 32 : head_dim <= 64 ? 30 : 24)) return 1;
     int64_t ns = (n_tiles >= (base > 128 && n_heads % 2 == 0 ? 48 : 64) ? 512 : 256) / base;
     if (ns > 8) ns = 256 / base < 8 ? 256 / base : 8;
     if (ns > n_tiles / 4) ns = n_tiles / 4;

@@ -24,7 +24,7 @@ bool decode4_applies(const AttnParams& p, int batch, int head_dim, int n_cus);
 int launch_attn_decode4(const AttnParams& p, int batch, int dtype, hipStream_t stream);
 #endif
 bool fwd_supported(int head_dim);
-int decode_pick_splits(int batch, int n_heads, int max_seqlen_k, int requested);
+int decode_pick_splits(int batch, int n_heads, int head_dim, int max_seqlen_k, int requested);
 bool decode_gqa_supported(int head_dim, int group);
 int decode_gqa_pick_splits(int batch, int n_kv_heads, int max_seqlen_k, int requested);
 int launch_attn_decode_gqa(const AttnParams& p, int batch, int head_dim, int dtype, hipStream_t stream);
@@ -104,7 +104,7 @@ bool use_gqa(const hx_attn_args* a, bool fused) {
 
 int pick_splits(const hx_attn_args* a, bool fused) {
   return use_gqa(a, fused) ? decode_gqa_pick_splits(a->batch, a->n_kv_heads, a->max_seqlen_k, a->num_splits)
-                           : decode_pick_splits(a->batch, a->n_heads, a->max_seqlen_k, a->num_splits);
+                           : decode_pick_splits(a->batch, a->n_heads, a->head_dim, a->max_seqlen_k, a->num_splits);
 }
 
 int validate(const hx_attn_args* a) {

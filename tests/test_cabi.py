@@ -135,19 +135,29 @@ def test_xreg_split_plan_is_stable():
     assert l.hx_fragment_major_elems(5, 4096) == 16 * 4096 and l.hx_fragment_major_elems(32, 64) == 32 * 64
 
 
-def test_splits_of_a_decode_batch():
-    """Keys of a pair of a sequence and a head dealt to several workgroups, as the workspace shows it: about 144 pairs, where a round of compute
-    units is one workgroup a pair, on both sides of 768 keys, of 129 and 160 pairs, with even and odd numbers of heads."""
-    def splits(batch, heads, keys):
-        a = _lib.hx_attn_args()
-        a.out = a.q = a.k = a.v = a.cu_seqlens_q = a.cu_seqlens_k = a.block_table = a.cu_block_lens = 4096      # (not looked at)
-        a.batch, a.total_q, a.n_heads, a.n_kv_heads, a.head_dim, a.block_size, a.max_seqlen_q, a.max_seqlen_k = batch, batch, heads, heads, 128, 16, 1, keys
-        a.q_row_stride = a.o_row_stride = a.k_block_stride = a.k_row_stride = a.k_head_stride = a.v_block_stride = a.v_row_stride = a.v_head_stride = 128 * heads
-        a.causal, a.softmax_scale, a.dtype, a.window_left, a.window_right = 1, 1.0, _lib.HX_BF16, -1, -1
-        return max(1, _lib.lib().hx_mha_varlen_fwd_workspace_bytes(ctypes.byref(a)) // (batch * heads * (128 + 2) * 4))
+def _splits(batch, heads, keys, dim=128):
+    """Workgroups that share the keys of a pair of a sequence and a head, as the workspace shows them."""
+    a = _lib.hx_attn_args()
+    a.out = a.q = a.k = a.v = a.cu_seqlens_q = a.cu_seqlens_k = a.block_table = a.cu_block_lens = 4096      # (not looked at)
+    a.batch, a.total_q, a.n_heads, a.n_kv_heads, a.head_dim, a.block_size, a.max_seqlen_q, a.max_seqlen_k = batch, batch, heads, heads, dim, 16, 1, keys
+    a.q_row_stride = a.o_row_stride = a.k_block_stride = a.k_row_stride = a.k_head_stride = a.v_block_stride = a.v_row_stride = a.v_head_stride = dim * heads
+    a.causal, a.softmax_scale, a.dtype, a.window_left, a.window_right = 1, 1.0, _lib.HX_BF16, -1, -1
+    return max(1, _lib.lib().hx_mha_varlen_fwd_workspace_bytes(ctypes.byref(a)) // (batch * heads * (dim + 2) * 4))
 
+
+def test_splits_of_a_decode_batch():
+    """About 144 pairs, where a round of compute units is one workgroup a pair: on both sides of 768 keys, of 129 and 160 pairs, with even and odd
+    numbers of heads."""
     for batch, heads in ((65, 2), (33, 4), (9, 16), (15, 10), (79, 2)):
-        assert [splits(batch, heads, n) for n in (512, 752, 753, 900, 1008, 1009)] == [1, 1, 3, 3, 3, 3], (batch, heads)
-    assert [splits(31, 5, n) for n in (753, 1008, 1009)] == [1, 1, 3]
-    assert [splits(16, 8, n) for n in (753, 1008, 1009)] == [2, 2, 4]
-    assert [splits(10, 16, n) for n in (753, 1008)] == [3, 3]
+        assert [_splits(batch, heads, n) for n in (512, 752, 753, 900, 1008, 1009)] == [1, 1, 3, 3, 3, 3], (batch, heads)
+    assert [_splits(31, 5, n) for n in (753, 1008, 1009)] == [1, 1, 3]
+    assert [_splits(16, 8, n) for n in (753, 1008, 1009)] == [2, 2, 4]
+    assert [_splits(10, 16, n) for n in (753, 1008)] == [3, 3]
+
+
+def test_splits_by_the_size_of_heads():
+    for batch, heads in ((1, 8), (4, 8), (10, 8)):
+        assert [_splits(batch, heads, n, 64) == 1 for n in (385, 480, 481)] == [True, True, False], (batch, heads)
+        assert [_splits(batch, heads, n, d) == 1 for n in (384, 385) for d in (128, 256)] == [True, True, False, False], (batch, heads)
+    assert [_splits(24, 8, n, 64) for n in (1392, 1393)] == [1, 4] and [_splits(24, 8, n, 128) for n in (1264, 1265)] == [1, 4]
+    assert [_splits(pairs // 8, 8, 1600, 256) for pairs in (160, 192, 256, 320, 384)] == [1, 1, 1, 3, 2]
