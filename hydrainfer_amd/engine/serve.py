@@ -10,6 +10,7 @@ from typing import List, Optional, Tuple
 import numpy as np
 import torch
 
+from hydrainfer_amd._C.kernel import gemm as hip_gemm
 from hydrainfer_amd.engine.executor import BatchFillExecutor, BatchImageEmbedExecutor, InstructionExecutor
 from hydrainfer_amd.engine.node import EPDNode, LocalCluster, NodeType
 from hydrainfer_amd.engine.rcb import SamplingParameters
@@ -17,6 +18,7 @@ from hydrainfer_amd.engine.request_processor import InstructionCreator, TokenReq
 from hydrainfer_amd.engine.scheduler import BatchScheduler, BatchSchedulerConfig, BatchSchedulerContext
 from hydrainfer_amd.memory.token_cache_manger import (TokenCacheBlockManager, TokenCacheBlockManagerConfig,
                                                       TokenCacheBlockManagerContext)
+from hydrainfer_amd.model.llama import MEMORY_SIDE_CACHE
 
 _DTYPE_NAMES = {torch.float16: "fp16", torch.bfloat16: "bf16", torch.float32: "fp32"}
 
@@ -90,9 +92,12 @@ def warm_library_gemms(language_model, token_budget: int, max_decode_rows: int =
         x = torch.zeros((rows[-1], w.shape[1]), dtype=dt, device=dev)
         for m in rows:
             torch.matmul(x[:m], w.t())
-    x = torch.zeros((max_decode_rows, st["lm_head"].shape[1]), dtype=dt, device=dev)
+    head = st["lm_head"]
+    x = torch.zeros((max_decode_rows, head.shape[1]), dtype=dt, device=dev)
+    streams = head.numel() * head.element_size() > MEMORY_SIDE_CACHE and model.use_hip_gemm and hip_gemm.supported(x[:1], head)
     for m in (1, 2, 4, 8, 16, 32, max_decode_rows):      # (NOT every row count: warming 64 shapes was followed by 70-400 ms
-        torch.matmul(x[:m], st["lm_head"].t())           #  stalls in the first prefill chunks — the library re-loading kernels)
+        if m > 16 or not streams:                        #  stalls in the first prefill chunks — the library re-loading kernels)
+            torch.matmul(x[:m], head.t())
     if vision_model is not None and pixel_values is not None:      # the tower for 1 .. image_budget images
         px = pixel_values.to(device=dev, dtype=dt)
         for n in range(1, image_budget + 1):

@@ -72,6 +72,9 @@ def build_cos_sin(shape: LlamaShape, dtype: torch.dtype, device) -> Tensor:
     return cs.to(dtype).to(device)
 
 
+MEMORY_SIDE_CACHE = 256 << 20      # bytes
+
+
 class LlamaForCausalLM:
     """Weights live in fused device tensors; `state` maps fused names to tensors."""
 
@@ -81,6 +84,9 @@ class LlamaForCausalLM:
         self.cos_sin = build_cos_sin(shape, dtype, self.device)
         self.q_size = shape.num_attention_heads * shape.head_dim
         self.kv_size = shape.num_key_value_heads * shape.head_dim
+        # all products' weights, the head's with them
+        self.linear_bytes = dtype.itemsize * shape.hidden_size * (
+            shape.vocab_size + shape.num_hidden_layers * (2 * self.q_size + 2 * self.kv_size + 3 * shape.intermediate_size))
         # decode batches (<= 64 rows) stream the weights through the HIP kernel; larger
         # batches (prefill) use the library GEMM
         self.use_hip_gemm = True
@@ -563,11 +569,16 @@ class LlamaForCausalLM:
         x = self.forward_hidden(input_ids_or_embeds, position_ids, model_params)
         w = self.state["lm_head"]
         # Up to 16 rows the weight-streaming product (its workgroups read whole rows, the library's tiles of 16 rows leave the memory half
-        # idle), where the weights come from memory: behind prompts, and from 256 MiB on, which the memory-side cache does not keep from
-        # step to step.  32064 outputs of 2048 / 4096 / 5120 from memory, library and this, us: 1 row 39 28, 61 52, 71 56; 16 rows 40
-        # 31, 60 56, 68 63; 17 rows 29 32, 62 57, 58 65.  Steps of one layer of width 4096, whose 263 MB stay: 132 and 140.
+        # idle), where the head comes from memory.  32064 outputs of 2048 / 4096 / 5120 from memory, library and this, us: 1 row 39 28,
+        # 61 52, 71 56; 16 rows 40 31, 60 56, 68 63; 17 rows 29 32, 62 57, 58 65.
+        # What the memory-side cache keeps from call to call the library reads faster.  It keeps a head of 250 MiB through any number of layers, as
+        # products of up to 64 rows read their weights past it (replayed steps of width 4096, 16 rows, 1 / 8 / 32 layers: 165 / 959 / 3582 us with
+        # the library, 177 / 967 / 3590), and not one of 313 MiB (width 5120, 1 row, 1 / 3 layers 208 / 445 and 188 / 426).  The
+        # library's products of more tokens push the head out, unless all weights fit (5 rows of width 2048: 85 tokens, 321 MiB 179 and 161;
+        # 1000 tokens, 223 MiB 133 and 134; 17 tokens, 1 row, two layers of width 4096 276 and 279).
+        pushed_out = self.linear_bytes > MEMORY_SIDE_CACHE and not model_params.all_sequences_decode and input_ids_or_embeds.shape[0] > 64
         few = (self.use_hip_gemm and x.shape[0] <= 16 and hip_gemm.supported(x, w)
-               and (not model_params.all_sequences_decode or w.numel() * w.element_size() > 256 << 20))
+               and (pushed_out or w.numel() * w.element_size() > MEMORY_SIDE_CACHE))
         if launch_plan.current() is None:
             return hip_gemm.linear_decode(x, w) if few else torch.matmul(x, w.t())
         # a launch plan is being recorded: the product is a host-side step of the plan between two native

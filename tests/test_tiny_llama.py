@@ -266,13 +266,18 @@ def test_layers_in_one_call_each_equal_the_launches_one_by_one(hidden, inter, la
 @pytest.mark.parametrize("rows", [1, 16, 17])
 @pytest.mark.parametrize("vocab", [2048, 2050])
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
-def test_logits_of_few_rows(rows, vocab, dt):
+def test_logits_of_few_rows(rows, vocab, dt, monkeypatch):
     """On both sides of the 16 rows that the weight-streaming product takes, and with outputs that it does not take."""
+    from hydrainfer_amd.model import llama
     from hydrainfer_amd.model.llama import LanguageModelParameters, LlamaForCausalLM, LlamaShape
+    monkeypatch.setattr(llama, "MEMORY_SIDE_CACHE", 0)            # (a head of any size comes from memory)
+    streamed = []
+    monkeypatch.setattr(llama.hip_gemm, "linear_decode", lambda *a, whole=llama.hip_gemm.linear_decode: streamed.append(1) or whole(*a))
     model = LlamaForCausalLM.random_init(LlamaShape(1024, 2816, 1, 8, 8, 128, vocab), dt, torch.device("cuda:0"), seed=3)
     x = torch.randn((rows, 1024), generator=torch.Generator().manual_seed(rows)).to(dt).cuda()
     model.forward_hidden = lambda *a: x
-    got, want = model.forward_logits(None, None, LanguageModelParameters([], False)).float(), x.float() @ model.state["lm_head"].float().t()
+    got, want = model.forward_logits(x, None, LanguageModelParameters([], False)).float(), x.float() @ model.state["lm_head"].float().t()
+    assert len(streamed) == (rows <= 16 and vocab % 16 == 0)
     # sums in float (1024 products, a unit of 2^-24 of the sum of their sizes each at worst), rounded once to dt
     unit = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11
     size = x.float().abs() @ model.state["lm_head"].float().abs().t()
@@ -290,16 +295,37 @@ def test_products_of_few_rows_ask_for_addresses():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows", [1, 16])
-def test_logits_of_a_head_off_sixteen_bytes(rows):
+def test_logits_of_a_head_off_sixteen_bytes(rows, monkeypatch):
     """A head that is a view into a flat buffer: the same logits as from a head of its own, behind prompts as in steps."""
+    from hydrainfer_amd.model import llama
     from hydrainfer_amd.model.llama import LanguageModelParameters, LlamaForCausalLM, LlamaShape
+    monkeypatch.setattr(llama, "MEMORY_SIDE_CACHE", 0)            # (a head of any size comes from memory)
     model = LlamaForCausalLM.random_init(LlamaShape(1024, 2816, 1, 8, 8, 128, 2048), torch.bfloat16, torch.device("cuda:0"), seed=3)
     x, head = torch.randn((rows, 1024), generator=torch.Generator().manual_seed(rows)).bfloat16().cuda(), model.state["lm_head"]
     model.forward_hidden = lambda *a: x
     flat = torch.empty(head.numel() + 1, dtype=head.dtype, device=head.device)
     model.state["lm_head"] = flat[1:].view_as(head).copy_(head)
     for step in (False, True):
-        got, want = model.forward_logits(None, None, LanguageModelParameters([], step)).float(), x.float() @ head.float().t()
+        got, want = model.forward_logits(x, None, LanguageModelParameters([], step)).float(), x.float() @ head.float().t()
         # sums in float (1024 products, a unit of 2^-24 of the sum of their sizes each at worst), rounded once
         bound = 2.0 ** -8 * want.abs() + 1024 * 2.0 ** -24 * (x.float().abs() @ head.float().abs().t()) + 1e-7
         assert bool(((got - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("rows, tokens, step, head_fits, all_fit, streams", [
+    (16, 1000, False, True, False, True), (17, 1000, False, True, False, False), (5, 65, False, True, False, True), (5, 64, False, True, False, False),
+    (5, 1000, False, True, True, False), (1, 1, True, True, False, False), (16, 16, True, True, False, False), (16, 16, True, False, False, True),
+    (1, 17, False, False, False, True), (17, 17, True, False, False, False)])
+def test_which_product_makes_the_logits(rows, tokens, step, head_fits, all_fit, streams, monkeypatch):
+    """The streaming product where the head comes from memory: larger than the memory-side cache, or pushed out of it by the library's
+    products of more than 64 tokens."""
+    from hydrainfer_amd.model import llama
+    calls = []
+    model = llama.LlamaForCausalLM.random_init(llama.LlamaShape(256, 512, 2, 2, 2, 128, 160), torch.bfloat16, "cpu")
+    head, layer = model.state["lm_head"], sum(model.state[f"l0.{n}"].numel() for n in ("wqkv", "wo", "wgu", "wdown"))
+    assert model.linear_bytes == 2 * (head.numel() + 2 * layer)
+    monkeypatch.setattr(llama, "MEMORY_SIDE_CACHE", model.linear_bytes if all_fit else 2 * head.numel() - (not head_fits))
+    monkeypatch.setattr(llama.hip_gemm, "linear_decode", lambda x, w: calls.append(1) or torch.matmul(x, w.t()))
+    model.forward_hidden = lambda *a: torch.zeros((rows, 256), dtype=torch.bfloat16)
+    assert model.forward_logits(torch.zeros(tokens, dtype=torch.int64), None, llama.LanguageModelParameters([], step)).shape == (rows, 160)
+    assert bool(calls) == streams
