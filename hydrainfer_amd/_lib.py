@@ -366,6 +366,7 @@ _MIX_SIGNATURES = {
     "hxm_router_topk": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int64, c_int32, c_int32, c_void_p, c_void_p,
                                 c_void_p]),
     "hxm_moe_plan": (c_int, [c_void_p, c_int64, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "hxm_grouped_linear_tile_rows": (c_int, [c_int64, c_int32, c_int64, c_int64]),
     "hxm_grouped_linear": (c_int, [c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_int64, c_int64,
                                    c_int32, c_float, c_float, c_float, c_int, c_void_p]),
     "hxm_moe_combine": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int64,

@@ -3,6 +3,7 @@
 // and the weighted combine with an optional gated shared expert.  Nothing returns to the host between the router and the
 // combine: the products are launched for the most rows there can be and find their expert from the plan's segments.
 #include <cfloat>
+#include <cmath>
 #include "mix_rows.h"
 #include "tile_product.h"
 #include "../../include/hydra_mix.h"
@@ -766,6 +767,34 @@ int launch_grouped_tiles(u16* y, const u16* x, int64_t x_stride, const int32_t* 
   return hxm::check_launch();
 }
 
+// Rows of a tile (and with 256 as many columns, else 128).  Up to 32 rows an expert the weights are all there is to read: tiles of 32
+// rows (123 us with 128 rows and 16 experts of 5504 x 4096, like 128 x 128, at a quarter of its LDS).  More: the form that is expected to take the least
+// time, by the rounds of 256 tiles that a compute unit each is given, by the depth of a round and by the weights.  The numbers are fitted (us)
+// to 1552 launches with weights from memory and as many with weights that partly stay in the cache — 8 to 64 experts, 33 to 800 rows each, drawn evenly and
+// from 0.3 to 1.7 of the mean, depths of 704 to 4096, 704 to 5504 outputs: 1 and 3 % above the best form in the mean, 16 % below tiles of 128 up
+// to 120 rows an expert and of 256 from there on (by eight waves), slower than those by 4 % or more in 18 and 17 of them.  Rows an expert are taken
+// to spread over 0.8 to 1.2 of their mean.  64 / 128 / 256 rows, us: 8 experts of 2816 x 2048, 64 rows 23 26 48, 96 rows 35 27 47, 160 rows 43 46 47,
+// 256 rows 55 51 48; 32 of 2048 x 1408, 50 rows 46 47 48, 140 rows 74 86 51; 16 of 2816 x 4096, 110 rows 101 100 103, 290 rows 182 203 174.
+int grouped_tile_rows(int64_t max_rows, int E, int64_t N, int64_t K, bool walks) {
+  if (max_rows <= (int64_t)32 * E) return 32;
+  struct Form {
+    int rows, cols;
+    double once, round, depth, weights;      // us; a round; a round and 1024 of depth; a million bytes of weights
+  };
+  const Form forms[3] = {{64, 128, 3, 3, 4.4, 0.10}, {128, 128, 0, 9, 7.5, 0.06}, walks ? Form{256, 256, 3, 9, 17, 0.075} : Form{256, 256, 0, 15, 21, 0.045}};
+  const double mean = (double)max_rows / E;
+  int best = 0;
+  double least = 0;
+  for (const Form& f : forms) {
+    double tiles = 0;                         // an expert's
+    for (int i = 0; i < 4; ++i) tiles += ceil((0.85 + 0.1 * i) * mean / f.rows) / 4;
+    const double full = tiles * E * (double)((N + f.cols - 1) / f.cols) / kTileGroups, rounds = 0.75 * ceil(full) + 0.25 * full;      // (a part of a round takes nearly as long as a whole one)
+    const double time = f.once + rounds * (f.round + f.depth * (double)K / 1024) + f.weights * 2e-6 * E * (double)N * (double)K;
+    if (!best || time < least) best = f.rows, least = time;
+  }
+  return best;
+}
+
 // The same, NE elements a lane: width, row strides and pointers are multiples of NE elements.  Rows and weights of the
 // token's choices are read once into LDS; the choices' rows are requested four at a time, with the shared expert's.  Bound by memory:
 // 4 of 16 experts of 4096 and a shared one, 3989 tokens 37.5 us (5.2 TB/s; 42.8 with four elements a lane and a token a workgroup), 2500 tokens of 2048
@@ -909,6 +938,11 @@ extern "C" int hxm_moe_plan(const int32_t* experts, int64_t n_tokens, int32_t to
   return hxm::check_launch();
 }
 
+extern "C" int hxm_grouped_linear_tile_rows(int64_t max_rows, int32_t n_experts, int64_t n_dim, int64_t k_dim) {
+  if (max_rows < 1 || n_experts < 1 || n_dim < 1 || k_dim < 1) return 0;
+  return grouped_tile_rows(max_rows, n_experts, n_dim, k_dim, k_dim % kTileK == 0 && k_dim >= 2 * kTileK && n_dim % 8 == 0);
+}
+
 extern "C" int hxm_grouped_linear(void* y, const void* x, int64_t x_stride, const int32_t* src, const void* w,
                                   const int32_t* seg, int64_t max_rows, int32_t n_experts, int64_t n_dim, int64_t k_dim,
                                   int32_t act, float glu_limit, float glu_alpha, float glu_up_shift, int dtype, void* stream) {
@@ -922,24 +956,15 @@ extern "C" int hxm_grouped_linear(void* y, const void* x, int64_t x_stride, cons
   if (dtype == HX_BF16 && k_dim % 8 == 0 && k_dim < (1 << 22) && x_stride % 8 == 0 && aligned16(x) && aligned16(w)) {      // (offsets inside a weight tile: 32 bits)
     u16* yy = (u16*)y;
     const u16 *xx = (const u16*)x, *ww = (const u16*)w;
-    // Rows an expert on average: up to 32 the weights are all there is to read (tiles of 32 rows: 123 us with 128 rows and 16
-    // experts of 5504 x 4096, like 128 x 128, at a quarter of its LDS).  Up to 56 most experts' rows fit into 64, two workgroups a
-    // CU (tiles of 64 / 128 rows: 16 experts of 5504 x 4096 with 48 rows 121 / 143 us, 8 of 2816 x 2048 22 / 25, 32 of 1408 x 2048 40 /
-    // 51).  Up to 120 rows fit into 128, which reads long weight rows once (5504 x 4096, 100 rows: 177 / 157 us; short ones, 16 of
-    // 2816 x 2048: 38 / 56).
-    const int64_t E = n_experts;
-    if (max_rows <= 32 * E) return launch_grouped<32, 128, 1, 4, 3>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
-    if (max_rows > 56 * E && max_rows < 120 * E && k_dim >= 2560)
-      return launch_grouped<128, 128, 2, 2, 3>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
-    // More rows: a round of 256 tiles of 256 x 256, one a CU, takes as long as about 720 tiles of 64 x 128, two a CU, and a part of a
-    // round nearly as long as a whole one.  64 x 128 / 256 x 256: 8 experts of 2816 x 2048, 160 rows 34 / 43 us, 256 rows 42 / 45, 400
-    // rows 53 / 46; 32 of 1408 x 2048, 128 rows 49 / 51, 200 rows 63 / 52; 8 of 1408 x 1024, 200 rows 14 / 27.
-    auto tiles = [&](int64_t rows, int64_t cols) { return (n_dim + cols - 1) / cols * (max_rows / rows + E / 2 > E ? max_rows / rows + E / 2 : E); };
-    if (max_rows <= 56 * E || tiles(64, 128) <= 720 * ((tiles(256, 256) + kTileGroups - 1) / kTileGroups))
-      return launch_grouped<64, 128, 1, 4, 3>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
-    if (k_dim % kTileK || k_dim < 2 * kTileK || (act != 2 && n_dim % 8) || !aligned16(y))
-      return launch_grouped<256, 256, 2, 4, 2>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
-    return launch_grouped_tiles(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
+    const bool walks = k_dim % kTileK == 0 && k_dim >= 2 * kTileK && (act == 2 || n_dim % 8 == 0) && aligned16(y);
+    switch (grouped_tile_rows(max_rows, n_experts, n_dim, k_dim, walks)) {
+      case 32: return launch_grouped<32, 128, 1, 4, 3>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
+      case 64: return launch_grouped<64, 128, 1, 4, 3>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
+      case 128: return launch_grouped<128, 128, 2, 2, 3>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
+      default:
+        if (walks) return launch_grouped_tiles(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
+        return launch_grouped<256, 256, 2, 4, 2>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
+    }
   }
   const int64_t tiles = (max_rows + kGM - 1) / kGM + n_experts;
   if (tiles > 65535) return HX_ERR_SHAPE;

@@ -232,6 +232,8 @@ int hxm_moe_plan(const int32_t* experts, int64_t n_tokens, int32_t top, int32_t 
 int hxm_grouped_linear(void* y, const void* x, int64_t x_stride, const int32_t* src, const void* w, const int32_t* seg,
                        int64_t max_rows, int32_t n_experts, int64_t n_dim, int64_t k_dim, int32_t act, float glu_limit, float glu_alpha,
                        float glu_up_shift, int dtype, void* stream);
+/* Rows of the tiles (32, 64, 128 or 256) that hxm_grouped_linear takes for bfloat16 operands on 16 bytes, by their sizes; 0: sizes out of range. */
+int hxm_grouped_linear_tile_rows(int64_t max_rows, int32_t n_experts, int64_t n_dim, int64_t k_dim);
 
 /* out[t, :] = sum_k weights[t, k] * y[row_of[t * top + k], :] + (shared ? sigmoid(shared_gate[t * gate_stride]) * shared[t, :] : 0);
  * with shared_gate NULL the shared expert's result is added as it is.

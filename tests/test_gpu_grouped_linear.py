@@ -34,8 +34,7 @@ def test_grouped_linear_edges(rows, n, k, act):
     _check(rows, n, k, act, False)
 
 
-# more slices of 64 than a tile has slots for (three, or two with tiles of 256 rows), several turns of them, with a tail and without:
-# tiles of 32, 128 and 256 rows
+# more slices of 64 than a tile has slots for, several turns of them, with a tail and without: tiles of 32 and 64 rows
 @pytest.mark.parametrize("rows", [[20, 0, 33], [128, 61], [300, 257]])
 @pytest.mark.parametrize("k", [256, 328, 1032])
 @pytest.mark.parametrize("act", ["none", "glu"])
@@ -43,11 +42,22 @@ def test_grouped_linear_over_many_slices(rows, k, act):
     _check(rows, 288, k, act, False)
 
 
-# long weight rows and about a hundred rows an expert: tiles of 128 rows
+# long weight rows and about a hundred rows an expert
 @pytest.mark.parametrize("rows", [[70, 100], [129, 0, 150]])
 @pytest.mark.parametrize("k, act", [(2560, "glu"), (2568, "none")])
 def test_grouped_linear_of_long_weight_rows(rows, k, act):
     _check(rows, 160, k, act, False)
+
+
+# enough columns for tiles of 128 rows, and for tiles of 256 of which not every one starts where the walk from tile to tile needs it: up to a tile's
+# rows and one more, several turns of the slots, with a tail and without
+@pytest.mark.parametrize("rows, n, k, act, tile", [
+    ([128, 128], 8352, 1600, "glu", 128), ([129, 99], 8360, 1544, "none", 128), ([65, 127], 8352, 1544, "relu2", 128), ([128, 1, 128], 8352, 1600, "none", 128),
+    ([256, 257], 11040, 1096, "glu", 256), ([300, 212], 11044, 1088, "none", 256)])
+def test_grouped_linear_in_large_tiles(rows, n, k, act, tile):
+    from hydrainfer_amd import _lib
+    assert _lib.mix_lib().hxm_grouped_linear_tile_rows(sum(rows), len(rows), n, k) == tile
+    _check(rows, n, k, act, False)
 
 
 # enough tiles for those of 256 x 256: from tile to tile with two slices and with more, columns in 8s and whole turns, the last ones in
