@@ -504,7 +504,8 @@ int launch_chain(const ChunkScanArgs& a, hipStream_t s) {
   if constexpr (KP == 128) {
     if (few_chains(a)) return launch_parts<KP, FORM, CHANNEL, 4, QK, VT, VEC>(a, s);
   }
-  return launch_parts<KP, FORM, CHANNEL, 2, QK, VT, VEC>(a, s);
+  if constexpr (FORM == hxm::kChunkDelta) return HX_ERR_UNSUPPORTED;      // (many chains of the delta rule take one launch: two gain nothing, chunk_scan_workspace)
+  else return launch_parts<KP, FORM, CHANNEL, 2, QK, VT, VEC>(a, s);
 }
 template <int KP, int FORM, typename QK, typename VT, bool VEC>
 int launch_channel(const ChunkScanArgs& a, hipStream_t s) {
@@ -523,8 +524,9 @@ int launch_form(const ChunkScanArgs& a, hipStream_t s) {
   if (a.form == hxm::kChunkGated) return launch_channel<KP, hxm::kChunkGated, QK, VT, VEC>(a, s);
   if (a.form == hxm::kChunkBonus) return launch_channel<KP, hxm::kChunkBonus, QK, VT, VEC>(a, s);
   if (a.per_channel) return launch_channel<KP, hxm::kChunkDecay, QK, VT, VEC>(a, s);
-  if constexpr (KP == 128) {
-    if (a.form == hxm::kChunkDelta) return launch_head<KP, hxm::kChunkDelta, QK, VT, VEC>(a, s);
+  if (a.form == hxm::kChunkDelta) {
+    if constexpr (KP == 128) return launch_head<KP, hxm::kChunkDelta, QK, VT, VEC>(a, s);
+    else return HX_ERR_UNSUPPORTED;
   }
   return launch_head<KP, hxm::kChunkDecay, QK, VT, VEC>(a, s);
 }

@@ -26,3 +26,16 @@ def test_state_scan_refuses_an_unknown_recurrence(mode, n_tokens):
 def test_tiles_of_the_grouped_product(rows, experts, n, k, tile):
     from hydrainfer_amd import _lib
     assert _lib.mix_lib().hxm_grouped_linear_tile_rows(rows, experts, n, k) == tile
+
+
+@pytest.mark.parametrize("n_seq, tokens, heads, dim, vdim, ahead", [
+    (1, 1151, 32, 128, 128, True), (4, 4000, 8, 128, 128, True), (4, 4000, 16, 128, 128, True), (4, 4000, 17, 128, 128, False), (4, 4000, 32, 128, 128, False),
+    (64, 64000, 32, 128, 128, False), (4, 4000, 8, 65, 32, True), (4, 4000, 8, 64, 128, False), (1, 4000, 1, 64, 64, False), (1, 60, 8, 128, 128, False)])
+def test_delta_rule_in_two_launches(n_seq, tokens, heads, dim, vdim, ahead):
+    """Only where the keys of a value channel are dealt to four waves: there is no other form for the delta rule behind a launch ahead."""
+    from hydrainfer_amd import _lib
+    HX_F32 = 0
+    a = _lib.hxm_state_scan_args(q_dtype=HX_F32, k_dtype=HX_F32, v_dtype=HX_F32, n_tokens=tokens, n_seq=n_seq, heads=heads, qk_heads=heads, dim=dim, vdim=vdim,
+                                 mode=2)
+    assert (_lib.mix_lib().hxm_state_scan_workspace(ctypes.byref(a)) > 0) == ahead
+    assert not ahead or (dim > 64 and n_seq * heads * ((vdim + 31) // 32) <= 256)
