@@ -78,17 +78,102 @@ def test_chunks_made_ahead(lens, form, per_channel, K, V, types, monkeypatch):
 
     monkeypatch.setattr(_lib, "_mix", Watch())
     _through_a_scan(lens, K, V, form, per_channel, types, 3)
-    assert asked[0] > 0 or len(lens) > 3 or (K <= 64 and len(lens) > 1)
+    # by the rule: short portions of few key channels are left to one launch, and of many sequences those that have many chains for their length
+    ahead = {1: True, 4: K > 64, 22: (form, per_channel, K, V) in [("bonus", True, 100, 130), ("decay", True, 128, 64), ("decay", True, 65, 7), ("decay", False, 70, 130)]}
+    assert (asked[0] > 0) == ahead[len(lens)]
 
 
-@pytest.mark.parametrize("lens", [[1151], [0, 300, 0, 1, 417, 0]], ids=str)
+# the same with more than 256 chains of 32 value channels: the keys of 128 channels go to two waves
+MANY = [1003, 901, 930]
+
+
+@pytest.mark.parametrize("form, per_channel", [("bonus", True), ("decay", True), ("decay", False)])
+@pytest.mark.parametrize("K, V, types", [(128, 128, "bf16"), (100, 100, "f32"), (128, 126, "mixed")])
+def test_many_chunks_made_ahead(form, per_channel, K, V, types):
+    H, n, T = 22, len(MANY), sum(MANY)
+    assert n * H * ((V + 31) // 32) > 256
+    g = torch.Generator(device="cuda").manual_seed(K + V)
+    f = lambda *s: torch.randn(s, generator=g, device="cuda")
+    qk_t, v_t = (torch.bfloat16 if types == "bf16" else torch.float32), (torch.float32 if types == "f32" else torch.bfloat16)
+    unit = lambda: torch.nn.functional.normalize(f(T, H, K), dim=-1).reshape(T, H * K).to(qk_t)
+    x = dict(q=unit(), k=unit(), v=f(T, H * V).to(v_t), decay=torch.rand((T, H * K if per_channel else H), generator=g, device="cuda") ** 0.2,
+             vscale=torch.rand((T, H), generator=g, device="cuda") if form == "decay" else None, beta=None, bonus=f(H * K) if form == "bonus" else None,
+             state=f(n, 1, H * K * V))
+    got, want = _on_the_device(form, MANY, H, K, V, x)
+    for name, a, b in zip(("out", "state"), got, want):
+        _check(name, a, b)
+
+
+# numbers that are not finite behind a launch ahead: a chunk's last token, one in a chunk's middle, one in another portion; keys of a value channel in
+# two waves (64, and many chains of 128) and in four
+# (the delta rule only in four; the bonus form has no number a token and head)
+@pytest.mark.parametrize("lens, H, K, V, form, per_channel", [
+    (lens, H, K, V, form, per_channel) for lens, H, K, V in (([1151], 2, 64, 64), ([500, 0, 1, 417], 2, 128, 128), (MANY, 22, 128, 128))
+    for form, per_channel in (("decay", False), ("decay", True), ("delta", False), ("bonus", True)) if form != "delta" or (K == 128 and H == 2)])
+@pytest.mark.parametrize("what, value", [("v", float("inf")), ("v", float("nan")), ("k", float("nan")), ("scalar", float("nan"))])
+def test_not_finite_numbers_behind_a_launch_ahead(lens, H, K, V, form, per_channel, what, value):
+    if form == "bonus" and what == "scalar":
+        what = "v"
+    T, n = sum(lens), len(lens)
+    g = torch.Generator(device="cuda").manual_seed(K + V)
+    f, rand = (lambda *s: torch.randn(s, generator=g, device="cuda")), (lambda *s: torch.rand(s, generator=g, device="cuda"))
+    unit = lambda: torch.nn.functional.normalize(f(T, H, K), dim=-1).reshape(T, H * K)
+    x = dict(q=unit(), k=unit(), v=f(T, H * V), decay=0.5 + 0.5 * rand(T, H * K if per_channel else H), vscale=rand(T, H) if form == "decay" else None,
+             beta=rand(T, H) if form == "delta" else None, bonus=f(H * K) if form == "bonus" else None, state=f(n, 1, H * K * V))
+    for t in (271, 470, 700):
+        if what == "v":
+            x["v"][t, V + 3] = value
+        elif what == "k":
+            x["k"][t, K + 5] = value
+        else:
+            (x["beta"] if form == "delta" else x["vscale"])[t, 1] = value
+    for got, want in zip(*_on_the_device(form, lens, H, K, V, x)):
+        fine = torch.isfinite(want)
+        assert torch.equal(torch.isfinite(got).cpu(), fine) and not bool(fine.all()) and bool(fine.any())
+        _check("finite", got.cpu()[fine], want[fine])
+
+
+def _on_the_device(form, lens, H, K, V, x):
+    """(result, state) of state_scan, which has to go in two launches, and of a token at a time in 64 bits; every other sequence is continued."""
+    from hydrainfer_amd import _lib
+    from hydrainfer_amd._C.kernel.seq_mix import state_scan
+    from hydrainfer_amd._C.kernel.stream_ops import SequenceState
+    lib, n, T, asked = _lib.mix_lib(), len(lens), sum(lens), []
+
+    class Watch:
+        def __getattr__(self, name):
+            if name != "hxm_state_scan_workspace":
+                return getattr(lib, name)
+            return lambda a: asked.append(lib.hxm_state_scan_workspace(a)) or asked[-1]
+
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    cu = [sum(lens[:s]) for s in range(n + 1)]
+    starts = [0 if s % 2 == 0 else 9 for s in range(n)]
+    d = lambda t, *s: t.double().reshape(T, H, *s)
+    ones = torch.ones((T, H), dtype=torch.float64, device="cuda")
+    want, S = _scan(form, d(x["q"], K), d(x["k"], K), d(x["v"], V), d(x["decay"], -1).expand(T, H, K), ones if x["vscale"] is None else x["vscale"].double(),
+                    ones if x["beta"] is None else x["beta"].double(), None if x["bonus"] is None else x["bonus"].double().view(H, K),
+                    x["state"].double().view(n, H, K, V).clone(), cu, [p == 0 for p in starts])
+    st = x["state"].clone()
+    seq = SequenceState(st, i32(list(range(n))), i32([s for s in range(n) for _ in range(lens[s])]))
+    _lib._mix = Watch()
+    try:
+        got = state_scan(form, x["q"], x["k"], x["v"], x["decay"], seq, 0, i32(cu), i32([starts[s] + i for s in range(n) for i in range(lens[s])]), H, H, K, V,
+                         vscale=x["vscale"], beta=x["beta"], bonus=x["bonus"])
+    finally:
+        _lib._mix = lib
+    assert asked[0] > 0
+    return (got, st.view(n, H, K, V)), (want.reshape(T, H * V).cpu(), S.cpu())
+
+
+@pytest.mark.parametrize("lens, H", [([1151], 3), ([0, 300, 0, 1, 417, 0], 3), (MANY, 22)], ids=str)
 @pytest.mark.parametrize("K, V", [(64, 64), (128, 128), (100, 36), (48, 7)])
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
-def test_gates_made_ahead(lens, K, V, dt, monkeypatch):
+def test_gates_made_ahead(lens, H, K, V, dt, monkeypatch):
     from hydrainfer_amd import _lib
     from hydrainfer_amd._C.kernel.recurrence import gated_recurrence
     from hydrainfer_amd._C.kernel.stream_ops import SequenceState
-    lib, H, T, n = _lib.mix_lib(), 3, sum(lens), len(lens)
+    lib, T, n = _lib.mix_lib(), sum(lens), len(lens)
     g = torch.Generator(device="cuda").manual_seed(K + V)
     f = lambda *s: torch.randn(s, generator=g, device="cuda")
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
