@@ -98,8 +98,9 @@ using namespace hx;
 extern "C" int hx_gate_up_silu_rows_supported(int64_t M, int64_t inter, int64_t K) {
   if (M < 1 || inter < 16 || inter % 16 || K < 2 * kTileK || K % kTileK || M > (1 << 24) || inter > (1 << 24) || K > (1 << 24)) return 0;
   // Worth it where at least 0.6 of the rounds of tiles is rows and columns.  Library and silu / here, us: 2 x 11008 outputs of 4096,
-  // 600 rows (0.39) 128 / 150, 900 (0.59) 172 / 165, 1300 (0.64) 308 / 239, 2048 (0.90) 427 / 266, 4505 (0.86) 679 / 608; 2 x 5632 of
-  // 2048, 1300 (0.44) 74 / 83, 1800 (0.60) 90 / 87, 3300 (0.76) 163 / 137; 2 x 13824 of 5120, 768 (0.63) 207 / 209, 1024 (0.85) 282 / 216.
+  // 600 rows (0.39) 130 / 160, 900 (0.59) 168 / 168, 1300 (0.57) 303 / 247, 1400 (0.61) 301 / 248, 2048 (0.90) 424 / 269, 4505 (0.85) 680 / 600; 2 x 5632 of
+  // 2048, 1300 (0.44) 76 / 89, 1800 (0.60) 94 / 94, 3300 (0.74) 162 / 139; 2 x 13824 of 5120, 768 (0.63) 205 / 207, 1024 (0.85) 270 / 224.  The library's
+  // own steps lie elsewhere: at the line this loses up to 6 % (2 x 14336 of 4096, 384 rows (0.66) 93 / 99; 2 x 13824 of 5120, 1150 (0.63) 300 / 312) and gains 20.
   const int64_t tiles = (M + kTileRows - 1) / kTileRows * ((2 * inter + kTileRows - 1) / kTileRows);
   const int64_t rounds = (tiles + kTileGroups - 1) / kTileGroups;
   return (double)M * (double)(2 * inter) >= 0.6 * (double)rounds * kTileGroups * kTileRows * kTileRows;

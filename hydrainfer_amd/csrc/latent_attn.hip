@@ -1020,7 +1020,7 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide_kernel(hxm_latent_att
 // turn, waits for a quarter of its time, and there are two waves a SIMD.  Tiles of 32 keys and 64 rows: two workgroups a CU, one working while the other brings queries in or results
 // out.  Also the form for few rows, decode steps first: the keys of a row tile are then dealt to several workgroups (wide_plan),
 // each writes its rows' sums, maximum and weight, and the kernel below merges them.
-// Measured, 4 portions of 797 - 1151 tokens, 32 heads, 512 columns: 861 us in the group form, 191 us here (660 TFLOP/s; 240 while the
+// Measured, 4 portions of 797 - 1151 tokens, 32 heads, 512 columns: 861 us in the group form, 190 us here (670 TFLOP/s; 240 while the
 // compiler had every read of a key waited for at once, 220 with addresses of the loads worked out lane by lane); 256 columns, 16
 // heads 268 and 64 us, 320 columns 396 and 68.  32 tokens of 301 - 1747 keys, 32 heads, 512 columns under a window of 512: 31 us and
 // 30 to merge in the tile form, 18 and 4.5 here, of which 6 pass before the first product and about 5 are the splits' sums going

@@ -258,7 +258,9 @@ int hxm_moe_combine(void* out, const void* y, const int32_t* row_of, const float
  * kernel without the chunk machinery.  Longer portions of up to 128 key channels go sixteen tokens at a time through float matrix
  * products, from a length on that depends on the sizes; what is said at hxm_state_scan holds for them. */
 int64_t hxm_gated_recurrence_workspace(int64_t n_tokens, int32_t heads, int32_t dim, int32_t vdim);
-/* At least as many floats, and on a multiple of 16 bytes: with these the batch goes fastest. */
+/* At least as many floats, and on a multiple of 16 bytes: with these the batch goes fastest.  Besides n_tokens * heads * vdim for the results, for every
+ * sixteen tokens and head (and one more of each sequence) what hxm_state_scan_workspace says for the gated form: 3896 tokens of 32 heads
+ * of 128 x 128 64 MB and 162 MB; never more than 1 GiB besides the results. */
 int64_t hxm_gated_recurrence_batch_workspace(int32_t n_seq, int64_t n_tokens, int32_t heads, int32_t dim, int32_t vdim, int32_t max_q_len, int dtype);
 int hxm_gated_recurrence(void* out, const void* q_pre, int64_t q_stride, const void* f_pre, int64_t f_stride, const void* v,
                          int64_t v_stride, const float* f_bias, const float* low, const float* norm_w, float eps,
@@ -516,7 +518,10 @@ typedef struct hxm_state_scan_args {
  * and are no further from the exact result.  What is not finite in a token's operands shows from that token on, in either form, and a
  * value, scale or write strength in its own columns only; sixteen tokens at a time it may come out as NaN where a token at a time left
  * an infinity.  dim <= 256. */
-int64_t hxm_state_scan_workspace(const hxm_state_scan_args* args);      /* by its sizes, types and mode; 0: none */
+/* Floats by sizes, types and mode; 0: none.  For every sixteen tokens and head (and one more of each sequence), up to 64 key channels and up to 128: 2752 and
+ * 5120 with a decay per channel or gates, 3392 and 6400 in the bonus form, 368 with a decay per head, 688 for the delta rule (of more than 64);
+ * never more than 2^28 (1 GiB).  A call without it, or with less, takes one launch. */
+int64_t hxm_state_scan_workspace(const hxm_state_scan_args* args);
 int hxm_state_scan(const hxm_state_scan_args* args, void* stream);
 
 #define HXM_DECAY_CHUNK 32      /* tokens the chunked form of hxm_decay_attention takes at a time */
