@@ -7,7 +7,7 @@ import torch
 from torch import Tensor
 
 from hydrainfer_amd import _lib
-from hydrainfer_amd._C.kernel.stream_ops import SequenceState
+from hydrainfer_amd._C.kernel.stream_ops import SequenceState, long_chains
 
 
 def gated_recurrence(q_pre: Tensor, f_pre: Tensor, v: Tensor, f_bias: Tensor, low: Tensor, norm_w: Tensor, eps: float,
@@ -38,7 +38,10 @@ def gated_recurrence(q_pre: Tensor, f_pre: Tensor, v: Tensor, f_bias: Tensor, lo
             raise _lib.HydraHipError(f"gated_recurrence: {name} must be contiguous int32 [{n}]")
     out = torch.empty((T, heads * vdim), dtype=dt, device=q_pre.device)
     base = st.data_ptr() + 4 * state_row * st.stride(1)
-    n_ws = _lib.mix_lib().hxm_gated_recurrence_batch_workspace(n_seq, T, int(heads), int(dim), int(vdim), int(max_q_len), _lib._DTYPE[dt])
+    if long_chains(T, n_seq, heads, vdim, max_q_len):
+        n_ws = _lib.mix_lib().hxm_gated_recurrence_batch_workspace(n_seq, T, int(heads), int(dim), int(vdim), int(max_q_len), _lib._DTYPE[dt])
+    else:
+        n_ws = _lib.mix_lib().hxm_gated_recurrence_workspace(T, int(heads), int(dim), int(vdim))
     ws = torch.empty(max(n_ws, 1), dtype=torch.float32, device=q_pre.device)      # partial results of the key channels' parts, or results and what chunks need
     _lib.mix_check(_lib.mix_lib().hxm_gated_recurrence(
         out.data_ptr(), q_pre.data_ptr(), q_pre.stride(0), f_pre.data_ptr(), f_pre.stride(0), v.data_ptr(), v.stride(0),

@@ -14,7 +14,7 @@ import torch
 from torch import Tensor
 
 from hydrainfer_amd import _lib
-from hydrainfer_amd._C.kernel.stream_ops import SequenceState
+from hydrainfer_amd._C.kernel.stream_ops import SequenceState, long_chains
 
 ACT = {None: 0, "none": 0, "silu": 1, "sigmoid": 2, "tanh": 3}
 SCAN_MODES = {"decay": 0, "bonus": 1, "delta": 2}
@@ -318,7 +318,7 @@ def state_scan(mode: str, q: Tensor, k: Tensor, v: Tensor, decay: Tensor, seq: S
     a.decay_per_channel, a.decay, a.vscale, a.beta, a.bonus = int(per_channel), decay.data_ptr(), _ptr(vscale), _ptr(beta), _ptr(bonus)
     a.state, a.slot_stride, a.slots, a.q_cu, a.positions = base, stride, seq.slots.data_ptr(), q_cu.data_ptr(), positions.data_ptr()
     a.n_tokens, a.n_seq, a.heads, a.qk_heads, a.dim, a.vdim, a.mode = T, n_seq, int(heads), int(qk_heads), int(dim), int(vdim), SCAN_MODES[mode]
-    if T > n_seq:                         # portions of prompts: what their chunks need is made in a launch ahead
+    if T > n_seq and long_chains(T, n_seq, heads, vdim):      # portions of prompts: what their chunks need is made in a launch ahead
         a.ws_floats = _lib.mix_lib().hxm_state_scan_workspace(ctypes.byref(a))
         if a.ws_floats > 0:
             ws = torch.empty(a.ws_floats, dtype=torch.float32, device=q.device)

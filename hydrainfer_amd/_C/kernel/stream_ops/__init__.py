@@ -38,6 +38,14 @@ class SequenceState:
     tok_seq: Tensor
 
 
+def long_chains(n_tokens: int, n_seq: int, heads: int, vdim: int, longest: int = 0) -> bool:
+    """False where a recurrence over portions of prompts goes in one launch for certain: fewer than seven chunks of sixteen tokens follow each other
+    (a compute unit takes one chain of 64 value channels at a time; longest: of the portions, 0: not known).  Short calls are bound by their
+    caller, and asking the library for a workspace costs them 0.6 to 0.9 us of 15 to 18."""
+    rounds = (n_seq * heads * ((vdim + 63) // 64) + 255) // 256
+    return longest >= 112 if rounds <= 1 and longest > 0 else n_tokens * rounds > 112 * n_seq
+
+
 def stream_embed(ids: Tensor, table: Tensor, scale: float, n_streams: int) -> Tensor:
     """x[t, s, :] = table[ids[t]] * scale for every stream s (float32)."""
     _lib.require_gpu(ids, table)

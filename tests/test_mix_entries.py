@@ -39,3 +39,28 @@ def test_delta_rule_in_two_launches(n_seq, tokens, heads, dim, vdim, ahead):
                                  mode=2)
     assert (_lib.mix_lib().hxm_state_scan_workspace(ctypes.byref(a)) > 0) == ahead
     assert not ahead or (dim > 64 and n_seq * heads * ((vdim + 31) // 32) <= 256)
+
+
+def test_no_call_with_a_launch_ahead_is_taken_for_a_short_one():
+    """long_chains, which spares short calls the question, holds wherever the library would have asked for a workspace; and calls of short portions
+    and steps are spared it."""
+    import random
+    from hydrainfer_amd import _lib
+    from hydrainfer_amd._C.kernel.stream_ops import long_chains
+    lib, rng, HX_F32, asked = _lib.mix_lib(), random.Random(5), 0, 0
+    for _ in range(20000):
+        n_seq, heads, dim, vdim = rng.choice([1, 2, 3, 4, 7, 16, 40, 100]), rng.randint(1, 64), rng.choice([16, 64, 65, 128]), rng.choice([7, 64, 65, 128, 200])
+        longest = int(2 ** rng.uniform(0, 11))
+        tokens = rng.randint(longest, longest * n_seq)
+        for mode, per_channel in ((0, 0), (0, 1), (1, 1), (2, 0)):
+            a = _lib.hxm_state_scan_args(q_dtype=HX_F32, k_dtype=HX_F32, v_dtype=HX_F32, n_tokens=tokens, n_seq=n_seq, heads=heads, qk_heads=heads, dim=dim, vdim=vdim,
+                                         mode=mode, decay_per_channel=per_channel)
+            if tokens > n_seq and lib.hxm_state_scan_workspace(ctypes.byref(a)) > 0:
+                assert long_chains(tokens, n_seq, heads, vdim)
+                asked += 1
+        for known in (0, longest):
+            if lib.hxm_gated_recurrence_batch_workspace(n_seq, tokens, heads, dim, vdim, known, HX_F32) > lib.hxm_gated_recurrence_workspace(tokens, heads, dim, vdim):
+                assert long_chains(tokens, n_seq, heads, vdim, known)
+                asked += 1
+    assert asked > 1000
+    assert not long_chains(3, 3, 16, 64, 1) and not long_chains(300, 4, 32, 128) and not long_chains(100, 1, 64, 128, 100) and not long_chains(0, 0, 8, 64)
