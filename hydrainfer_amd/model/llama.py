@@ -362,7 +362,7 @@ class LlamaForCausalLM:
         eps, L = sh.rms_norm_eps, sh.num_hidden_layers
         ws_n = max(hip_gemm.workspace_floats(n, q_size + 2 * kv_size, hid), hip_gemm.workspace_floats(n, hid, q_size),
                    hip_gemm.workspace_floats(n, 2 * inter, hid), hip_gemm.workspace_floats(n, hid, inter),
-                   hip_gemm.xreg_workspace_floats(n, hid, inter))
+                   hip_gemm.xreg_workspace_floats(n, hid, inter), hip_gemm.xreg_workspace_floats(n, q_size + 2 * kv_size, hid))
         ws = torch.empty(ws_n, dtype=torch.float32, device=h.device)
         x = torch.empty_like(h)
         if n > self.decode_rows_prepared and not self.decode_only:

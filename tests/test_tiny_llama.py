@@ -263,6 +263,35 @@ def test_layers_in_one_call_each_equal_the_launches_one_by_one(hidden, inter, la
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows", [33, 40, 64])
+def test_wide_steps_of_a_narrow_model_equal_two_halves(rows):
+    """Width 2048, more than 32 rows: the qkv product of the second layer leaves two slabs, and its norm is a launch of its own."""
+    from hydrainfer_amd.layer.causal_attention import AttentionParametersBuilder
+    from hydrainfer_amd.memory.kv_cache import KVCache
+    from hydrainfer_amd.model.llama import LanguageModelParameters, LlamaForCausalLM, LlamaShape
+    dt, dev, L, H = torch.float16, torch.device("cuda:0"), 2, 16
+    model = LlamaForCausalLM.random_init(LlamaShape(2048, 5632, L, H, H, 128, 2048), dt, dev, seed=3)
+    model.prepare_decode(max_rows=rows)
+    g = torch.Generator().manual_seed(rows)
+    start, ids = torch.randn((L, 2, 4 * rows, 16, H, 128), generator=g).to(dt), torch.randint(0, 2048, (rows,), generator=g)
+    kv = [1 + (13 * r) % 60 for r in range(rows)]
+
+    def step(some):
+        pool, b = start.to(dev), AttentionParametersBuilder(H, H, 128, 16, dev)
+        for r in some:
+            b.add_request(1, kv[r], [64 * r + kv[r] - 1], [4 * r + i for i in range((kv[r] + 15) // 16)])
+        for l in range(L):
+            b.add_kv_cache(KVCache(pool[l, 0], pool[l, 1]))
+        return model.forward_logits(ids[list(some)].to(dev), torch.tensor([kv[r] - 1 for r in some], dtype=torch.int32, device=dev),
+                                    LanguageModelParameters(b.build_attention_parameters(), True)).float()
+
+    whole, halves = step(range(rows)), torch.cat([step(range(rows // 2)), step(range(rows // 2, rows))])
+    assert model._decode_plan(rows, dt)["wide"]
+    # (either is within 3e-2 of the oracle, as above)
+    assert bool(torch.isfinite(whole).all()) and float((whole - halves).abs().max()) <= 6e-2
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows", [1, 16, 17])
 @pytest.mark.parametrize("vocab", [2048, 2050])
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
