@@ -13,8 +13,7 @@ def supported(x: Tensor, weight: Tensor) -> bool:
     M, K = x.shape
     N = weight.shape[0]
     return (x.dtype in (torch.float16, torch.bfloat16) and 1 <= M <= 64 and N % 16 == 0 and K % 256 == 0
-            and x.stride(1) == 1 and weight.stride(1) == 1 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0
-            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+            and x.stride(1) == 1 and weight.stride(1) == 1 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0)
 
 
 def linear_decode(x: Tensor, weight: Tensor, out: Optional[Tensor] = None) -> Tensor:
@@ -23,7 +22,7 @@ def linear_decode(x: Tensor, weight: Tensor, out: Optional[Tensor] = None) -> Te
     if x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1] or x.dtype != weight.dtype:
         raise _lib.HydraHipError("linear_decode: x [M, K], weight [N, K], same dtype")
     if not supported(x, weight):
-        raise _lib.HydraHipError("linear_decode: needs M <= 64, N % 16 == 0, K % 256 == 0, fp16/bf16, contiguous rows that start on 16 bytes")
+        raise _lib.HydraHipError("linear_decode: needs M <= 64, N % 16 == 0, K % 256 == 0, fp16/bf16, contiguous rows")
     M, K = x.shape
     N = weight.shape[0]
     if out is None:
@@ -41,6 +40,8 @@ def gate_up_rows_supported(x: Tensor, weight: Tensor) -> bool:
     """True if gate_up_silu_rows takes these operands and is faster than a library product and silu_and_mul."""
     M, K = x.shape
     inter = weight.shape[0] // 2
+    if M <= 128:      # (no rounds of 256 rows are full enough: not asked, as short prompts are bound by their caller)
+        return False
     return (x.is_cuda and weight.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and weight.dtype == x.dtype and weight.shape[1] == K
             and weight.shape[0] == 2 * inter and x.stride(1) == 1 and weight.stride(1) == 1 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0
             and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and max(M * x.stride(0), 2 * inter * weight.stride(0)) < 2 ** 31
@@ -71,7 +72,7 @@ def linear_decode_partial(x: Tensor, weight: Tensor, partial: Tensor) -> int:
     buffer of at least workspace_floats(M, N, K) elements) for a fused consumer.  Returns n_splits."""
     _lib.require_gpu(x, weight, partial)
     if not supported(x, weight) or x.dtype != weight.dtype:
-        raise _lib.HydraHipError("linear_decode_partial: needs M <= 64, N % 16 == 0, K % 256 == 0, fp16/bf16, rows that start on 16 bytes")
+        raise _lib.HydraHipError("linear_decode_partial: needs M <= 64, N % 16 == 0, K % 256 == 0, fp16/bf16")
     if partial.dtype != torch.float32 or not partial.is_contiguous():
         raise _lib.HydraHipError("linear_decode_partial: partial must be contiguous float32")
     M, K = x.shape

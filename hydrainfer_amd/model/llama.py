@@ -577,7 +577,7 @@ class LlamaForCausalLM:
         # library's products of more tokens push the head out, unless all weights fit (5 rows of width 2048: 85 tokens, 321 MiB 179 and 161;
         # 1000 tokens, 223 MiB 133 and 134; 17 tokens, 1 row, two layers of width 4096 276 and 279).
         pushed_out = self.linear_bytes > MEMORY_SIDE_CACHE and not model_params.all_sequences_decode and input_ids_or_embeds.shape[0] > 64
-        few = (self.use_hip_gemm and x.shape[0] <= 16 and hip_gemm.supported(x, w)
+        few = (self.use_hip_gemm and x.shape[0] <= 16 and hip_gemm.supported(x, w) and w.data_ptr() % 16 == 0
                and (pushed_out or w.numel() * w.element_size() > MEMORY_SIDE_CACHE))
         if launch_plan.current() is None:
             return hip_gemm.linear_decode(x, w) if few else torch.matmul(x, w.t())

@@ -161,3 +161,10 @@ def test_splits_by_the_size_of_heads():
         assert [_splits(batch, heads, n, d) == 1 for n in (384, 385) for d in (128, 256)] == [True, True, False, False], (batch, heads)
     assert [_splits(24, 8, n, 64) for n in (1392, 1393)] == [1, 4] and [_splits(24, 8, n, 128) for n in (1264, 1265)] == [1, 4]
     assert [_splits(pairs // 8, 8, 1600, 256) for pairs in (160, 192, 256, 320, 384)] == [1, 1, 1, 3, 2]
+
+
+def test_few_rows_are_never_enough_for_the_gate_and_up_product():
+    """(what gate_up_rows_supported answers up to 128 rows without asking)"""
+    for inter in (16, 48, 2816, 5632, 8192, 11008, 13824, 14336, 32768, 1 << 20):
+        assert not any(_lib.lib().hx_gate_up_silu_rows_supported(m, inter, 4096) for m in range(1, 129)), inter
+    assert _lib.lib().hx_gate_up_silu_rows_supported(512, 11008, 4096)

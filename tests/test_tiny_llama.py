@@ -313,13 +313,17 @@ def test_logits_of_few_rows(rows, vocab, dt, monkeypatch):
     assert got.shape == (rows, vocab) and bool(((got - want).abs() <= unit * want.abs() + 1024 * 2.0 ** -24 * size + 1e-7).all())
 
 
-def test_products_of_few_rows_ask_for_addresses():
-    """Rows that do not start on 16 bytes are left to the library."""
-    from hydrainfer_amd._C.kernel import gemm
-    flat = torch.zeros(16 * 256 + 8, dtype=torch.bfloat16)
-    for off in range(9):
-        a, whole = flat[off:off + 16 * 256].view(16, 256), torch.zeros((16, 256), dtype=torch.bfloat16)
-        assert gemm.supported(a, whole) == gemm.supported(whole, a) == (off % 8 == 0)
+@pytest.mark.parametrize("off", range(9))
+def test_a_head_off_sixteen_bytes_is_left_to_the_library(off, monkeypatch):
+    from hydrainfer_amd.model import llama
+    calls = []
+    model = llama.LlamaForCausalLM.random_init(llama.LlamaShape(256, 512, 1, 2, 2, 128, 160), torch.bfloat16, "cpu")
+    model.state["lm_head"] = torch.zeros(160 * 256 + 8, dtype=torch.bfloat16)[off:off + 160 * 256].view(160, 256)
+    monkeypatch.setattr(llama, "MEMORY_SIDE_CACHE", 0)            # (a head of any size comes from memory)
+    monkeypatch.setattr(llama.hip_gemm, "linear_decode", lambda x, w: calls.append(1) or torch.matmul(x, w.t()))
+    model.forward_hidden = lambda *a: torch.zeros((3, 256), dtype=torch.bfloat16)
+    model.forward_logits(torch.zeros(3, dtype=torch.int64), None, llama.LanguageModelParameters([], False))
+    assert bool(calls) == (off % 8 == 0)
 
 
 @pytest.mark.gpu
