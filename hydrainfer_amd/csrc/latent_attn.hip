@@ -4,6 +4,7 @@
 // are the same rows: score = q~ . c_j * scale, out = sum_j softmax(score)_j c_j.  Scores, weights and sums are float.
 // Sliding window: a query at position i sees keys j with 0 <= i - j < window.
 #include "attn_common.h"
+#include "latent_step.h"
 #include "../../include/hydra_mix.h"
 
 namespace hxm {
@@ -1018,13 +1019,12 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide_kernel(hxm_latent_att
 // accumulators are 192 registers a lane at 512 columns, two waves a SIMD.  A byte from LDS feeds half the products of the form
 // above, but nothing is full (matrix cores 32 % of the time, vector ALU 39, LDS 30): a wave goes through scores, softmax and values in
 // turn, waits for a quarter of its time, and there are two waves a SIMD.  Tiles of 32 keys and 64 rows: two workgroups a CU, one working while the other brings queries in or results
-// out.  Also the form for few rows, decode steps first: the keys of a row tile are then dealt to several workgroups (wide_plan),
-// each writes its rows' sums, maximum and weight, and the kernel below merges them.
+// out.  Also the form for few rows (short portions; single tokens of more than 32 heads, those of fewer are latent_step.hip's): the keys of a row tile are then dealt to several
+// workgroups (wide_plan), each writes its rows' sums, maximum and weight, and the kernel below merges them.
 // Measured, 4 portions of 797 - 1151 tokens, 32 heads, 512 columns: 861 us in the group form, 190 us here (670 TFLOP/s; 240 while the
 // compiler had every read of a key waited for at once, 220 with addresses of the loads worked out lane by lane); 256 columns, 16
 // heads 268 and 64 us, 320 columns 396 and 68.  32 tokens of 301 - 1747 keys, 32 heads, 512 columns under a window of 512: 31 us and
-// 30 to merge in the tile form, 18 and 4.5 here, of which 6 pass before the first product and about 5 are the splits' sums going
-// out (8 MB); 1 token behind 1000 keys 70 us and 24, most of it the host's.
+// 30 to merge in the tile form, 18 and 4.5 here (15.6 in all in latent_step.hip).
 // (Thirty-two rows a wave, one wave a SIMD, with weights as sums of two bfloat16 numbers instead of a pass over the 256 accumulators:
 // 245 us where this form took 253; the second set of products meets the card's power limit.)
 // Row r of sixteen has its chunks at x ^ swz(r): rows r and 15 - r share a 32-byte place (their
@@ -1342,6 +1342,10 @@ WidePlan wide_plan(const hxm_latent_attn_args& a) {
   const int64_t rows = (int64_t)a.max_q_len * a.n_heads;
   p.rows32 = a.kv_rank <= 192 && a.n_seq * ((rows + 127) / 128) >= 256;
   if (p.rows32) return p;
+  if (hxm::latent_step_serves(a)) {
+    p.splits = hxm::latent_step_splits(a);
+    return p;
+  }
   int reach = a.max_kv_len;
   if (a.window > 0 && a.window + a.max_q_len < reach) reach = a.window + a.max_q_len;
   const int64_t tiles = a.n_seq * ((rows + 63) / 64);
@@ -1390,7 +1394,7 @@ int launch_wide(const hxm_latent_attn_args& a, const WidePlan& p, hipStream_t s)
       return hxm::check_launch();
     }
   }
-  return launch_wide16<KK>(a, s);
+  return hxm::latent_step_serves(a) ? hxm::launch_latent_step(a, s) : launch_wide16<KK>(a, s);
 }
 
 // the splits of a (sequence, row tile) merged: out = sum_s O_s e^(m_s - M) / sum_s l_s e^(m_s - M), times the head gate

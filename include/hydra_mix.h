@@ -126,7 +126,8 @@ int hxm_latent_attention_plan(const hxm_latent_attn_args* args, int32_t* n_split
 #define HXM_LATENT_ROW 0       /* a wave a (token, head) */
 #define HXM_LATENT_TILE 1      /* tiles of 16 rows, or groups of four of them */
 #define HXM_LATENT_WIDE32 2    /* 128 rows a workgroup, 32 a wave */
-#define HXM_LATENT_WIDE16 3    /* 64 rows a workgroup, 16 a wave; with n_splits > 1 several workgroups a row tile */
+#define HXM_LATENT_WIDE16 3    /* 64 rows a workgroup, 16 a wave; with n_splits > 1 several workgroups a row tile.  Batches of single
+                                * tokens of up to 32 heads: a token a workgroup, or several, whose waves share its keys */
 /* Which kernel hxm_latent_attention takes for these arguments (HX_ERR_NULL without any). */
 int hxm_latent_attention_form(const hxm_latent_attn_args* args);
 

@@ -57,6 +57,12 @@ def test_rows_that_nobody_sees(new, kv, R, window):
     check(new, kv, R, 32, window, "plain", WIDE32 if R <= 192 and max(new) > 700 else WIDE16, unseen=True)
 
 
+@pytest.mark.parametrize("R, H", [(64, 32), (320, 16), (512, 32)])
+@pytest.mark.parametrize("window", [300, 0])
+def test_rows_that_no_single_token_sees(R, H, window):
+    check([1] * 4, [700, 1101, 40, 1], R, H, window, "plain", WIDE16, unseen=True)
+
+
 def hide(cache, table, first, last):
     """What lies outside of keys first .. last of a sequence becomes NaN; its pages there the last block of the cache, all NaN."""
     cache[-1] = math.nan
@@ -210,3 +216,41 @@ def test_weights_round_no_more_than_in_the_tile_form(n, new, kv, R):
     finally:
         _lib.mix_lib().hxm_set_option(b"attn_tile_form", 1)
     assert off[1] <= (1.0 if new < 20 else 1.005) * off[2], off
+
+
+# Batches of single tokens of up to 32 heads: one group of heads and two, tiles in two, three and four places, keys up to a tile's and a group's edge and past it,
+# splits of one tile and of several, pages whose size is no power of two, sequences that bring no token, tokens in another order than their sequences.
+@pytest.mark.parametrize("kv", [[64, 0, 65, 1], [16, 17, 300, 513], [1040] + [90] * 20], ids=["edges", "few", "splits"])
+@pytest.mark.parametrize("R, H, block", [(64, 16, 16), (128, 17, 48), (192, 32, 16), (320, 32, 48), (384, 9, 16), (512, 32, 32)])
+@pytest.mark.parametrize("window, extra", [(0, "plain"), (63, "sinks and gate"), (500, "negative")])
+def test_steps_of_single_tokens(kv, R, H, block, window, extra):
+    from hydrainfer_amd._C.kernel.latent_attn import latent_attention
+    g = torch.Generator().manual_seed(R + H + window + sum(kv))
+    i = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    seqs = [s for s, n in enumerate(kv) if n]
+    if len(seqs) == len(kv):
+        seqs.reverse()                            # (q_cu says nothing to these launches but how many sequences there are)
+    nb = [(n + block - 1) // block for n in kv]
+    cu_b = [sum(nb[:s]) for s in range(len(kv) + 1)]
+    cache, q = torch.randn((sum(nb), block, 1, R), generator=g).bfloat16(), torch.randn((len(seqs), H, R), generator=g).bfloat16()
+    q[0, 0] *= 20
+    table = torch.randperm(sum(nb), generator=g)
+    scale = (-1.0 if extra == "negative" else 1.0) * R ** -0.5
+    sinks = 2 * torch.randn(H, generator=g) if "sinks" in extra else None
+    gate = torch.randn((len(seqs), H), generator=g).bfloat16() if "gate" in extra else None
+    q_cu = [sum(1 for s in seqs if s < x) for x in range(len(kv) + 1)]
+    c = lambda t: None if t is None else t.cuda()
+    got = latent_attention(c(q), c(cache), i(seqs), i([kv[s] - 1 for s in seqs]), i(q_cu), c(table.int()), i(cu_b), scale, window or None, 1, gate_pre=c(gate),
+                           max_kv_len=max(kv), sinks=c(sinks)).double().cpu()
+    for t, s in enumerate(seqs):
+        k = cache[table[cu_b[s]:cu_b[s + 1]]].reshape(-1, R)[:kv[s]].double()[-window if window else 0:]
+        z = torch.matmul(q[t].double(), k.t()) * scale
+        if sinks is not None:
+            z = torch.cat([z, sinks.double()[:, None]], dim=1)
+        p = torch.softmax(z, dim=1)[:, :k.shape[0]]
+        f = torch.sigmoid(gate[t].double())[:, None] if gate is not None else 1.0
+        want, size = torch.matmul(p, k) * f, torch.matmul(p, k.abs()) * f
+        # the result is rounded to bfloat16 once, the weights are sums of two bfloat16 numbers (2^-17); 1e-5 of what is summed for that and
+        # the float arithmetic
+        off = (got[t] - want).abs()
+        assert bool((off <= 2.0 ** -8 * want.abs() + 1e-5 * size + 1e-6).all()), (t, float((off - 2.0 ** -8 * want.abs() - 1e-5 * size).max()))
