@@ -74,6 +74,12 @@ def biased_attention(q: Tensor, key_cache: Tensor, value_cache: Tensor, vdim: in
     dtype and size).  head_scale [n_heads]: head h's scores are multiplied by head_scale[h] as well (a temperature per head);
     sinks [n_heads]: the softmax's denominator of head h holds one more term exp(sinks[h]) without a key or a value.
     Returns [n_tokens, n_heads, vdim]."""
+    front = _lib.front()
+    if front is not None:
+        got = front.biased_attention(q, key_cache, value_cache, vdim, tok_seq, positions, q_cu, block_table, cu_block_lens, scale, slopes, mask, mask_size,
+                                     max_q_len, kv_heads, max_kv_len, form, softcap, head_scale, sinks)
+        if got is not None:
+            return got
     _lib.require_gpu(q, key_cache, value_cache, tok_seq, positions, q_cu, block_table, cu_block_lens, slopes, head_scale, sinks)
     if q.dim() != 3 or not q.is_contiguous() or key_cache.dtype != q.dtype or value_cache.dtype != q.dtype:
         raise _lib.HydraHipError("biased_attention: q contiguous [n_tokens, n_heads, dim], caches of the same dtype")
@@ -109,25 +115,11 @@ def biased_attention(q: Tensor, key_cache: Tensor, value_cache: Tensor, vdim: in
     a.mask_kind, a.mask_size, a.scale, a.dtype = MASK_KINDS[mask], int(mask_size), float(scale), _code(q.dtype)
     a.n_seq, a.max_q_len, a.softcap = n_seq, int(max_q_len), float(softcap or 0.0)
     a.form, a.n_splits, a.ws_o, a.ws_ml = {"auto": 0, "rows": 1, "tile": 2}[form], 1, None, None
-    if form in ("auto", "tile") and q.dtype == torch.bfloat16 and max_q_len > 0 and max_kv_len > 0 and D % 8 == 0 and vdim % 8 == 0 \
-            and D <= 256 and vdim <= 256:
-        # key splits: enough waves to fill the chip when the launch has few row tiles, at least two 32-key chunks a split
-        rows = max_q_len * (H // G)
-        tiles = n_seq * G * ((rows + 15) // 16)
-        reach = max_kv_len
-        if mask != "causal":
-            reach = min(reach, mask_size + (max_q_len if mask == "window" else 0))
-        # heads of 64 and 128: five waves of the step form fill a CU (1024 and 2048 waves: 32 tokens of 1025 - 2047 keys 39.5 and
-        # 41.9 us, 128 of 500 - 1500 109 and 116); portions of 64 rows and more go undivided to the wide form unless they are few
-        # and their keys many (one portion behind keys, 32 heads on 8 key heads, wide and split: 32 tokens behind 2000 44.8 and
-        # 24.9 us, 100 behind 2000 46.4 and 36.4, 100 behind none 21 and 23.5, 8 times 16 behind 500 21.4 and 23.9)
-        whole = form == "auto" and D in (64, 128) and vdim in (64, 128) and bs % 16 == 0
-        ns = min(((1024 if whole else 2048) + tiles - 1) // tiles, ((reach + 31) // 32) // 2, 64)
-        if whole and rows >= 64 and (tiles > 256 or reach < 1024):
-            ns = 1
-        if ns > 1:
-            v16 = (vdim + 15) // 16 * 16
-            ws = torch.empty(tiles * ns * 16 * (v16 + 2), dtype=torch.float32, device=q.device)
-            a.n_splits, a.ws_o, a.ws_ml = ns, ws.data_ptr(), ws.data_ptr() + 4 * tiles * ns * 16 * v16
+    ns, need = ctypes.c_int32(1), ctypes.c_int64(0)
+    _lib.mix_check(_lib.mix_lib().hxm_biased_attention_plan(ctypes.byref(a), int(max_kv_len), ctypes.byref(ns), ctypes.byref(need)), "biased_attention_plan")
+    if ns.value > 1:
+        v16 = (vdim + 15) // 16 * 16
+        ws = torch.empty(need.value, dtype=torch.float32, device=q.device)
+        a.n_splits, a.ws_o, a.ws_ml = ns.value, ws.data_ptr(), ws.data_ptr() + 4 * (need.value // (v16 + 2) * v16)
     _lib.mix_check(_lib.mix_lib().hxm_biased_attention(ctypes.byref(a), _lib.current_stream()), "biased_attention")
     return out

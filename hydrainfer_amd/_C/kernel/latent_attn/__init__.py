@@ -55,6 +55,12 @@ def latent_attention(q: Tensor, cache: Tensor, tok_seq: Tensor, positions: Tenso
     of the batch holds — lets a launch with few rows (decode steps) deal every row tile's keys to several waves.  gate_pre [n_tokens, >= n_heads]:
     the result of head h is multiplied by sigmoid(gate_pre[t, h]).  sinks [n_heads] float32: the softmax's denominator of
     head h holds one more term exp(sinks[h]) without a key or a value.  Returns [n_tokens, n_heads, kv_rank]."""
+    front = _lib.front()
+    if front is not None:
+        got = front.latent_attention(q, cache, tok_seq, positions, q_cu, block_table, cu_block_lens, scale, window, max_q_len, gate_pre, out,
+                                     max_kv_len, sinks)
+        if got is not None:
+            return got
     _lib.require_gpu(q, cache, tok_seq, positions, q_cu, block_table, cu_block_lens, gate_pre, out, sinks)
     if q.dim() != 3 or q.stride(2) != 1 or cache.dtype != q.dtype:
         raise _lib.HydraHipError("latent_attention: q [n_tokens, n_heads, kv_rank] with contiguous rows, cache of the same dtype")

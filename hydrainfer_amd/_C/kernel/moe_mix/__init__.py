@@ -49,6 +49,11 @@ def router_topk(x: Tensor, w: Tensor, bias: Optional[Tensor], top: int) -> Tuple
     """The router in one kernel, in float: z = x @ w.T + bias; the `top` largest are chosen (ties: the lower expert), weighted by
     the softmax over the chosen alone.  x: float32 [n_tokens, width] rows (the residual itself); w: float32 [n_experts, width].
     Returns (weights float32 [n_tokens, top], experts int32 [n_tokens, top])."""
+    front = _lib.front()
+    if front is not None:
+        got = front.router_topk(x, w, bias, top)
+        if got is not None:
+            return got
     _lib.require_gpu(x, w, bias)
     E, K = w.shape
     if x.dtype != torch.float32 or x.dim() != 2 or x.shape[1] != K or x.stride(1) != 1 or w.dtype != torch.float32 or not w.is_contiguous():
@@ -67,6 +72,11 @@ def moe_plan(experts: Tensor, n_experts: int) -> Tuple[Tensor, Tensor, Tensor]:
     """experts: int32 [n_tokens, top].  Returns (seg int32 [n_experts + 1], row_of int32 [n_tokens, top], src int32
     [n_tokens * top]): rows seg[e] .. seg[e + 1] of the expert-major order belong to expert e, pair (t, k) is row
     row_of[t, k], and row r comes from token src[r]."""
+    front = _lib.front()
+    if front is not None:
+        got = front.moe_plan(experts, n_experts)
+        if got is not None:
+            return got
     _lib.require_gpu(experts)
     if experts.dtype != torch.int32 or experts.dim() != 2 or not experts.is_contiguous():
         raise _lib.HydraHipError("moe_plan: experts must be contiguous int32 [n_tokens, top]")
@@ -94,6 +104,11 @@ def grouped_linear(x: Tensor, w: Tensor, seg: Tensor, max_rows: int, src: Option
     n_out, k] contiguous; returns [max_rows, n_out] (rows beyond seg[-1] are not written).  act: "none" | "relu2" |
     "glu": w holds gates and ups in turns (gate_up_turns) and the result [max_rows, n_out / 2] is g sigmoid(alpha g) (u +
     up_shift) with g = min(gate, limit), u = clamp(up, -limit, limit) (limit 0: no clamp)."""
+    front = _lib.front()
+    if front is not None:
+        got = front.grouped_linear(x, w, seg, max_rows, src, act, limit, alpha, up_shift)
+        if got is not None:
+            return got
     _lib.require_gpu(x, w, seg, src)
     if x.dim() != 2 or x.stride(1) != 1 or w.dim() != 3 or not w.is_contiguous() or w.dtype != x.dtype or w.shape[2] != x.shape[1]:
         raise _lib.HydraHipError("grouped_linear: x [n, k] with contiguous rows, w [n_experts, n_out, k] contiguous, one dtype")
@@ -119,6 +134,11 @@ def moe_combine(y: Tensor, row_of: Tensor, weights: Tensor, shared: Optional[Ten
     number per token (any row stride: a column of a wider matrix will do); None: shared is added as it is.  identity [n_tokens, width] (the experts' input):
     a choice without a row (row_of < 0: an expert beyond those moe_plan was called with) is an identity expert and adds
     weights[t, k] * identity[t]; without it such a choice adds nothing."""
+    front = _lib.front()
+    if front is not None:
+        got = front.moe_combine(y, row_of, weights, shared, shared_gate, identity)
+        if got is not None:
+            return got
     _lib.require_gpu(y, row_of, weights, shared, shared_gate, identity)
     T, top = row_of.shape
     W = y.shape[1]

@@ -17,6 +17,11 @@ def gated_recurrence(q_pre: Tensor, f_pre: Tensor, v: Tensor, f_bias: Tensor, lo
     seq.state: float32 [n_slots, n_rows, >= heads * dim * vdim]; this layer's state is row `state_row` of a slot.
     max_q_len: the longest portion of the batch when known (1: every sequence brings one token — a decode step's kernel).
     Returns [n_tokens, heads * vdim] in the inputs' dtype."""
+    front = _lib.front()
+    if front is not None:
+        got = front.gated_recurrence(q_pre, f_pre, v, f_bias, low, norm_w, eps, seq, state_row, q_cu, positions, heads, dim, vdim, max_q_len)
+        if got is not None:
+            return got
     _lib.require_gpu(q_pre, f_pre, v, f_bias, low, norm_w, seq.state, seq.slots, q_cu, positions)
     T = q_pre.shape[0]
     dt = q_pre.dtype

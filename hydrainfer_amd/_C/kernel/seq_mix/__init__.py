@@ -299,6 +299,11 @@ def state_scan(mode: str, q: Tensor, k: Tensor, v: Tensor, decay: Tensor, seq: S
     q, k: [n_tokens, qk_heads * dim], v: [n_tokens, heads * vdim] (float32 or bfloat16, each its own; views will do);
     decay a: float32 [n_tokens, heads] or [n_tokens, heads * dim] (one per key channel); vscale s, beta b: float32
     [n_tokens, heads]; bonus u: float32 [heads * dim].  Returns o: float32 [n_tokens, heads * vdim]."""
+    front = _lib.front()
+    if front is not None:
+        got = front.state_scan(mode, q, k, v, decay, seq, offset, q_cu, positions, heads, qk_heads, dim, vdim, vscale, beta, bonus)
+        if got is not None:
+            return got
     _lib.require_gpu(q, k, v, decay, vscale, beta, bonus)
     _rows(q, qk_heads * dim, "state_scan: q")
     T = q.shape[0]

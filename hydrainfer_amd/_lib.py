@@ -6,6 +6,8 @@ wraps every `hydrainfer._C` import in try/except and silently drops to torch, e.
 hydrainfer/layer/causal_attention.py:13-17).
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 from ctypes import c_char_p, c_float, c_int, c_int32, c_int64, c_void_p, POINTER
 
@@ -380,6 +382,7 @@ _MIX_SIGNATURES = {
                                   c_float, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int32, c_int64, c_int,
                                   c_void_p]),
     "hxm_biased_attention": (c_int, [POINTER(hxm_biased_attn_args), c_void_p]),
+    "hxm_biased_attention_plan": (c_int, [POINTER(hxm_biased_attn_args), c_int32, POINTER(c_int32), POINTER(c_int64)]),
     "hxm_causal_conv": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int, c_void_p, c_int64, c_void_p,
                                 c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_int32, c_int32, c_int, c_void_p]),
     "hxm_causal_conv_pair": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p,
@@ -424,8 +427,30 @@ def mix_lib() -> ctypes.CDLL:
         if handle.hxm_abi_version() != HXM_ABI_VERSION:
             raise HydraHipError(f"libhydra_mix.so ABI version {handle.hxm_abi_version()} != {HXM_ABI_VERSION} of this binding: "
                                 "rebuild with `make -C hydrainfer_amd/csrc mix`")
+        _load_front(handle)
         _mix = handle
     return _mix
+
+
+FRONT_PATH = os.path.join(_HERE, "lib", "libhydra_front.so")
+_front = _front_of = None
+
+
+def _load_front(handle: ctypes.CDLL) -> None:
+    global _front, _front_of
+    if not os.path.exists(FRONT_PATH):
+        raise HydraHipError(f"{FRONT_PATH} is missing: build it with `make -C hydrainfer_amd/csrc mix`. There is no fallback path.")
+    loader = importlib.machinery.ExtensionFileLoader("_hydra_front", FRONT_PATH)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_hydra_front", FRONT_PATH, loader=loader))
+    loader.exec_module(module)
+    module.bind({name: ctypes.cast(getattr(handle, name), c_void_p).value for name in module.entries}, mix_check)
+    _front, _front_of = module, handle
+
+
+def front():
+    """The operators' native side (csrc/front.cpp: the calls of the mixers without the interpreter between their checks, allocations
+    and launch), bound to the library that mix_lib() opens.  None where something else stands in for that library."""
+    return _front if mix_lib() is _front_of else None
 
 
 def mix_check(status: int, what: str) -> None:

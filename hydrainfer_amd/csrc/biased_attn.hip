@@ -4,6 +4,8 @@
 // kernel in front of it: one RMS norm over a token's whole query projection and one over its whole key projection
 // (all heads at once), keys and values straight into the cache.
 #include <cfloat>
+#include <algorithm>
+
 #include "attn_common.h"
 #include "mix_rows.h"
 #include "../../include/hydra_mix.h"
@@ -1386,4 +1388,29 @@ extern "C" int hxm_biased_attention(const hxm_biased_attn_args* args, void* stre
     default: return HX_ERR_DTYPE;
   }
   return hxm::check_launch();
+}
+
+// Key splits: enough waves to fill the chip when the launch has few row tiles, at least two 32-key chunks a split.  Heads of 64 and 128:
+// five waves of the step form fill a CU (1024 and 2048 waves: 32 tokens of 1025 - 2047 keys 39.5 and 41.9 us, 128 of 500 - 1500 109
+// and 116); portions of 64 rows and more go undivided to the wide form unless they are few and their keys many (one portion behind
+// keys, 32 heads on 8 key heads, wide and split: 32 tokens behind 2000 44.8 and 24.9 us, 100 behind 2000 46.4 and 36.4, 100 behind
+// none 21 and 23.5, 8 times 16 behind 500 21.4 and 23.9).
+extern "C" int hxm_biased_attention_plan(const hxm_biased_attn_args* args, int32_t max_kv_len, int32_t* n_splits, int64_t* ws_floats) {
+  if (!args || !n_splits || !ws_floats) return HX_ERR_NULL;
+  const hxm_biased_attn_args& a = *args;
+  *n_splits = 1;
+  *ws_floats = 0;
+  if (a.form == 1 || a.dtype != HX_BF16 || a.max_q_len < 1 || max_kv_len < 1 || a.dim % 8 || a.vdim % 8 || a.dim > 256 || a.vdim > 256 || a.n_seq < 0) return HX_OK;
+  if (a.n_seq == 0 || a.kv_heads < 1) return HX_ERR_SHAPE;
+  const int64_t rows = (int64_t)a.max_q_len * (a.n_heads / a.kv_heads), tiles = (int64_t)a.n_seq * a.kv_heads * ((rows + 15) / 16);
+  if (tiles < 1) return HX_OK;
+  int64_t reach = max_kv_len;
+  if (a.mask_kind != HXM_MASK_CAUSAL) reach = std::min<int64_t>(reach, (int64_t)a.mask_size + (a.mask_kind == HXM_MASK_WINDOW ? a.max_q_len : 0));
+  const bool whole = a.form == 0 && (a.dim == 64 || a.dim == 128) && (a.vdim == 64 || a.vdim == 128) && a.block_size % 16 == 0;
+  int64_t ns = std::min({((whole ? 1024 : 2048) + tiles - 1) / tiles, (reach + 31) / 32 / 2, (int64_t)64});
+  if (whole && rows >= 64 && (tiles > 256 || reach < 1024)) ns = 1;
+  if (ns < 2) return HX_OK;
+  *n_splits = (int32_t)ns;
+  *ws_floats = tiles * ns * 16 * ((a.vdim + 15) / 16 * 16 + 2);
+  return HX_OK;
 }

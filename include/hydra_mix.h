@@ -320,6 +320,11 @@ typedef struct hxm_biased_attn_args {
  * float).  Queries of portions and single decoded tokens may share a batch. */
 int hxm_biased_attention(const hxm_biased_attn_args* args, void* stream);
 
+/* How the keys of a launch with these arguments are dealt out, max_kv_len: the most keys a sequence holds (0: unknown): n_splits (1: no
+ * workspace) and the floats of workspace (ws_o: the first ws_floats / (ceil16(vdim) + 2) * ceil16(vdim) of them, ws_ml the rest).
+ * No pointer is looked at. */
+int hxm_biased_attention_plan(const hxm_biased_attn_args* args, int32_t max_kv_len, int32_t* n_splits, int64_t* ws_floats);
+
 
 /* ------------------------------------------------------------------------------------------------------------------
  * Sequence mixers with per-sequence state beside the paged cache (csrc/seq_ops.hip, csrc/state_scan.hip): short causal
