@@ -434,3 +434,12 @@ def test_small_gates_are_as_exact_as_large_ones(max_q_len):
     want = torch.sigmoid(proj[:, H * K:2 * H * K].double()).prod(0).view(H, K, 1)
     off = (st.double().cpu().view(H, K, V) - want).abs() / want
     assert float(off.max()) <= 8 * 2.0 ** -23, float(off.max())
+
+
+# One decay a head in one launch (csrc/chunk_head.hip): portions at the edges of its chunks of 32 tokens and their tiles of 16, channels that fill no
+# tile and no vector, q and k in one part and in three
+@pytest.mark.parametrize("lens", [[13, 16, 17, 31, 32, 0, 33, 48, 49, 64, 65, 97] * 2, [47, 1, 15, 96]], ids=["edges", "few"])
+@pytest.mark.parametrize("form, K, V", [("delta", 128, 128), ("delta", 100, 34), ("delta", 65, 68), ("decay", 128, 64), ("decay", 64, 130), ("decay", 100, 7), ("decay", 17, 64)])
+@pytest.mark.parametrize("types, pad", [("bf16", 4), ("f32", 4), ("mixed", 3)])
+def test_chunks_of_two_tiles(lens, form, K, V, types, pad):
+    _through_a_scan(lens, K, V, form, False, types, pad)
