@@ -305,6 +305,21 @@ __device__ __forceinline__ bool find_tile(const int32_t* __restrict__ seg, int E
   return false;
 }
 
+// The same by the lanes of a wave, an expert each (one expert behind the other is a chain of loads: 1 us with 8 experts, 3 - 4 with 32, in
+// launches of 6 - 30): 64 experts from e0 on, their rows, their row tiles and those up to and with them.
+struct ExpertTiles {
+  int lo, hi, nt, run;
+  __device__ __forceinline__ ExpertTiles(const int32_t* __restrict__ seg, int E, int e0, int TM, int lane)
+      : lo(seg[min(e0 + lane, E)]), hi(seg[min(e0 + lane + 1, E)]), nt((hi - lo + TM - 1) / TM), run(nt) {
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int before = __shfl_up(run, d, 64);
+      run += lane >= d ? before : 0;
+    }
+  }
+  __device__ __forceinline__ int total() const { return __builtin_amdgcn_readlane(run, 63); }
+};
+
 __device__ __forceinline__ float act_apply(float v, int act) {
   if (act == 1) {
     v = fmaxf(v, 0.f);
@@ -390,8 +405,8 @@ __global__ __launch_bounds__(256) void grouped_linear_kernel(typename A::storage
 // read between four products; the one workgroup barrier of a slice stands between its halves, so that a wave always has
 // products to issue behind it.
 // With few rows an expert it is bound by the weights: those of an expert with one row tile are read past the caches (128 rows of 16
-// experts, 2 x 2752 outputs of 4096 and back: 162 + 75 us through registers in tiles of 128 x 128 and padded LDS rows, 123 + 61 us here,
-// 5.9 TB/s).  Many rows take grouped_linear_tile_kernel where they can; in tiles of 256 x 256 this form is bound by LDS bandwidth.
+// experts, 2 x 2752 outputs of 4096 and back: 162 + 75 us through registers in tiles of 128 x 128 and padded LDS rows, 115 + 58 us here,
+// 6.2 TB/s).  Many rows take grouped_linear_tile_kernel where they can; in tiles of 256 x 256 this form is bound by LDS bandwidth.
 // A slice's row is 128 bytes, unpadded (64 lanes land 16 bytes each one after the other): its 16-byte chunk c sits at position
 // c ^ (row / 2 % 8), so that the 16 lanes that one pass of a 16-byte LDS read serves — rows 0-3, 12-15 of one k group and
 // 4-11 of the next — fall into different banks.
@@ -416,26 +431,31 @@ __global__ __launch_bounds__(64 * WGM * WGN) void grouped_linear_mfma_kernel(u16
   int64_t col0 = 0;
   bool once = false;                                       // the expert has one row tile: nobody reads its weights again
   {
-    int m_tiles = 0;
-    for (int i = 0; i < E; ++i) m_tiles += (seg[i + 1] - seg[i] + TM - 1) / TM;
+    const int expert_lane = threadIdx.x & 63;
+    ExpertTiles some(seg, E, 0, TM, expert_lane);
+    int m_tiles = some.total();
+    for (int e0 = 64; e0 < E; e0 += 64) m_tiles += ExpertTiles(seg, E, e0, TM, expert_lane).total();
     const int total = m_tiles * n_col, per = (total + 7) >> 3;
     const int at = (int)(blockIdx.x >> 3);
     int tile = (int)(blockIdx.x & 7) * per + at;
     if (at >= per || tile >= total) return;                // (the whole workgroup: no barrier is left waiting)
-    for (; e < E; ++e) {
-      row0 = seg[e];
-      row1 = seg[e + 1];
-      const int nt = (row1 - row0 + TM - 1) / TM;
-      if (tile < nt * n_col) {
+    for (;;) {
+      const uint64_t behind = __builtin_amdgcn_ballot_w64(tile < some.run * n_col);
+      if (behind) {
+        const int l = __builtin_ctzll(behind), nt = __builtin_amdgcn_readlane(some.nt, l);
+        tile -= (__builtin_amdgcn_readlane(some.run, l) - nt) * n_col;
         const int c = tile / nt;
-        row0 += (tile - c * nt) * TM;
+        e += l;
+        row0 = __builtin_amdgcn_readlane(some.lo, l) + (tile - c * nt) * TM;
+        row1 = min(__builtin_amdgcn_readlane(some.hi, l), row0 + TM);
         col0 = (int64_t)c * TN;
         once = nt == 1;
         break;
       }
-      tile -= nt * n_col;
+      tile -= some.total() * n_col;
+      e += 64;
+      some = ExpertTiles(seg, E, e, TM, expert_lane);
     }
-    row1 = min(row1, row0 + TM);
   }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int wm0 = (wave / WGN) * (TM / WGM), wn0 = (wave % WGN) * (TN / WGN);
@@ -767,8 +787,12 @@ int launch_grouped_tiles(u16* y, const u16* x, int64_t x_stride, const int32_t* 
   return hxm::check_launch();
 }
 
-// Rows of a tile (and with 256 as many columns, else 128).  Up to 32 rows an expert the weights are all there is to read: tiles of 32
-// rows (123 us with 128 rows and 16 experts of 5504 x 4096, like 128 x 128, at a quarter of its LDS).  More: the form that is expected to take the least
+// Rows of a tile (and with 256 as many columns, else 128, with 32 half of that).  Up to 32 rows an expert the weights are all there is to read: tiles of 32
+// rows and 64 columns.  A slice takes what its bytes need to come from memory, divided by the slices on their way, so tiles are small — few experts
+// with rows still are a tile for most compute units — and six slots deep where rows are long; short ones take four, with three workgroups a compute
+// unit instead of two (us; 32 x 128 with three slots, 32 x 64 with four, with six: one row, 2 x 704 outputs of 4096 27.5 17.6 16.8 and back 7.5 5.7 5.5;
+// 30 rows of 32 such experts 50 45 43 and 24 22 24; 120 rows 68 62 60 and 31 31 34; 2 x 2752 of 4096, 120 rows of 16: 121 117 115 and 62 58 58;
+// in the mean of 196 launches of 1 to 256 rows, 8 to 32 experts and depths of 704 to 4096 3 and 2 % above the best of these and four more, 32 x 128 21 %).  More: the form that is expected to take the least
 // time, by the rounds of 256 tiles that a compute unit each is given, by the depth of a round and by the weights.  The numbers are fitted (us)
 // to 1552 launches with weights from memory and as many with weights that partly stay in the cache — 8 to 64 experts, 33 to 800 rows each, drawn evenly and
 // from 0.3 to 1.7 of the mean, depths of 704 to 4096, 704 to 5504 outputs: 1 and 3 % above the best form in the mean, 16 % below tiles of 128 up
@@ -958,7 +982,9 @@ extern "C" int hxm_grouped_linear(void* y, const void* x, int64_t x_stride, cons
     const u16 *xx = (const u16*)x, *ww = (const u16*)w;
     const bool walks = k_dim % kTileK == 0 && k_dim >= 2 * kTileK && (act == 2 || n_dim % 8 == 0) && aligned16(y);
     switch (grouped_tile_rows(max_rows, n_experts, n_dim, k_dim, walks)) {
-      case 32: return launch_grouped<32, 128, 1, 4, 3>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
+      case 32:
+        if (k_dim < 2048) return launch_grouped<32, 64, 2, 2, 4>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
+        return launch_grouped<32, 64, 2, 2, 6>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
       case 64: return launch_grouped<64, 128, 1, 4, 3>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
       case 128: return launch_grouped<128, 128, 2, 2, 3>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
       default:

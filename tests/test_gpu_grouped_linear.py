@@ -42,6 +42,21 @@ def test_grouped_linear_over_many_slices(rows, k, act):
     _check(rows, 288, k, act, False)
 
 
+# few rows an expert and short and long weight rows (four slots and six), with a tail and without, columns that no tile divides
+@pytest.mark.parametrize("rows", [[1], [0, 16, 17], [32, 0, 31], [33, 1, 0, 20]])
+@pytest.mark.parametrize("n, k", [(96, 2040), (160, 2048), (32, 2056), (224, 2432)])
+@pytest.mark.parametrize("act", ["none", "glu"])
+def test_grouped_linear_of_few_rows(rows, n, k, act):
+    _check(rows, n, k, act, False)
+
+
+# more experts than a wave has lanes, with rows on both sides of every 64th
+@pytest.mark.parametrize("experts", [63, 64, 65, 130])
+@pytest.mark.parametrize("every", [1, 21])
+def test_grouped_linear_of_many_experts(experts, every):
+    _check([1 + 40 * (e % 5 == 0) if e % every == 0 or e in (63, 64, 128) else 0 for e in range(experts)], 96, 136, "glu", False)
+
+
 # long weight rows and about a hundred rows an expert
 @pytest.mark.parametrize("rows", [[70, 100], [129, 0, 150]])
 @pytest.mark.parametrize("k, act", [(2560, "glu"), (2568, "none")])
