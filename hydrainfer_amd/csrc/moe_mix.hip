@@ -787,36 +787,39 @@ int launch_grouped_tiles(u16* y, const u16* x, int64_t x_stride, const int32_t* 
   return hxm::check_launch();
 }
 
-// Rows of a tile (and with 256 as many columns, else 128, with 32 half of that).  Up to 32 rows an expert the weights are all there is to read: tiles of 32
+// A tile's rows and columns.  Up to 32 rows an expert the weights are all there is to read: tiles of 32
 // rows and 64 columns.  A slice takes what its bytes need to come from memory, divided by the slices on their way, so tiles are small — few experts
 // with rows still are a tile for most compute units — and six slots deep where rows are long; short ones take four, with three workgroups a compute
 // unit instead of two (us; 32 x 128 with three slots, 32 x 64 with four, with six: one row, 2 x 704 outputs of 4096 27.5 17.6 16.8 and back 7.5 5.7 5.5;
 // 30 rows of 32 such experts 50 45 43 and 24 22 24; 120 rows 68 62 60 and 31 31 34; 2 x 2752 of 4096, 120 rows of 16: 121 117 115 and 62 58 58;
 // in the mean of 196 launches of 1 to 256 rows, 8 to 32 experts and depths of 704 to 4096 3 and 2 % above the best of these and four more, 32 x 128 21 %).  More: the form that is expected to take the least
 // time, by the rounds of 256 tiles that a compute unit each is given, by the depth of a round and by the weights.  The numbers are fitted (us)
-// to 1552 launches with weights from memory and as many with weights that partly stay in the cache — 8 to 64 experts, 33 to 800 rows each, drawn evenly and
-// from 0.3 to 1.7 of the mean, depths of 704 to 4096, 704 to 5504 outputs: 1 and 3 % above the best form in the mean, 16 % below tiles of 128 up
-// to 120 rows an expert and of 256 from there on (by eight waves), slower than those by 4 % or more in 18 and 17 of them.  Rows an expert are taken
-// to spread over 0.8 to 1.2 of their mean.  64 / 128 / 256 rows, us: 8 experts of 2816 x 2048, 64 rows 23 26 48, 96 rows 35 27 47, 160 rows 43 46 47,
-// 256 rows 55 51 48; 32 of 2048 x 1408, 50 rows 46 47 48, 140 rows 74 86 51; 16 of 2816 x 4096, 110 rows 101 100 103, 290 rows 182 203 174.
-int grouped_tile_rows(int64_t max_rows, int E, int64_t N, int64_t K, bool walks) {
-  if (max_rows <= (int64_t)32 * E) return 32;
-  struct Form {
-    int rows, cols;
-    double once, round, depth, weights;      // us; a round; a round and 1024 of depth; a million bytes of weights
-  };
-  const Form forms[3] = {{64, 128, 3, 3, 4.4, 0.10}, {128, 128, 0, 9, 7.5, 0.06}, walks ? Form{256, 256, 3, 9, 17, 0.075} : Form{256, 256, 0, 15, 21, 0.045}};
+// to 888 launches — 2 to 32 experts, 36 to 450 rows each, drawn evenly, depths of 704 to 5520, 704 to 11040 outputs — with the choices that older measurements over
+// 8 to 64 experts had settled kept: 3 % above the best of eleven forms in the mean.  Rows an expert are taken to spread over 0.8 to 1.2 of their mean.
+// Eight waves a tile, and tiles of 64 columns besides those of 128: the forms of four waves and 128 columns that stood here took 6 % longer in the mean
+// (us, 64 x 64, 64 x 128, 128 x 64, 128 x 128, 256 x 256; those of four waves 64 x 128 and 128 x 128: 8 experts of 2048 x 1408, 57 rows 17 16 14 17 35; 16 18; 16 of
+// 1408 x 1024, 100 rows 18 19 17 15 30; 19 16; 8 of 5504 x 4096, 100 rows 113 96 88 99 102; 96 97; 16 of 2048 x 1408, 160 rows 42 35 39 38 40; 38 41; 8 of 1408 x 4096, 256
+// rows 64 56 56 44 79; 57 46; 16 of 5504 x 4096, 320 rows 480 384 392 339 289; 386 380).
+struct GroupedForm {
+  int rows, cols;
+  double once, round, depth, weights;        // us; a round; a round and 1024 of depth; a million bytes of weights
+};
+GroupedForm grouped_form(int64_t max_rows, int E, int64_t N, int64_t K, bool walks) {
+  if (max_rows <= (int64_t)32 * E) return GroupedForm{32, 64, 0, 0, 0, 0};
+  const GroupedForm forms[5] = {{64, 64, 3.4, 0.86, 3.8, 0.061}, {64, 128, 4.7, 1.4, 5.3, 0.08}, {128, 64, 3.7, 1.5, 7.5, 0.02}, {128, 128, 1.6, 4.4, 10, 0.026},
+                                walks ? GroupedForm{256, 256, 4.1, 9.5, 15, 0.11} : GroupedForm{256, 256, 0, 9, 21, 0.08}};
   const double mean = (double)max_rows / E;
-  int best = 0;
+  int best = -1;
   double least = 0;
-  for (const Form& f : forms) {
+  for (int j = 0; j < 5; ++j) {
+    const GroupedForm& f = forms[j];
     double tiles = 0;                         // an expert's
     for (int i = 0; i < 4; ++i) tiles += ceil((0.85 + 0.1 * i) * mean / f.rows) / 4;
     const double full = tiles * E * (double)((N + f.cols - 1) / f.cols) / kTileGroups, rounds = 0.75 * ceil(full) + 0.25 * full;      // (a part of a round takes nearly as long as a whole one)
     const double time = f.once + rounds * (f.round + f.depth * (double)K / 1024) + f.weights * 2e-6 * E * (double)N * (double)K;
-    if (!best || time < least) best = f.rows, least = time;
+    if (best < 0 || time < least) best = j, least = time;
   }
-  return best;
+  return forms[best];
 }
 
 // The same, NE elements a lane: width, row strides and pointers are multiples of NE elements.  Rows and weights of the
@@ -964,7 +967,7 @@ extern "C" int hxm_moe_plan(const int32_t* experts, int64_t n_tokens, int32_t to
 
 extern "C" int hxm_grouped_linear_tile_rows(int64_t max_rows, int32_t n_experts, int64_t n_dim, int64_t k_dim) {
   if (max_rows < 1 || n_experts < 1 || n_dim < 1 || k_dim < 1) return 0;
-  return grouped_tile_rows(max_rows, n_experts, n_dim, k_dim, k_dim % kTileK == 0 && k_dim >= 2 * kTileK && n_dim % 8 == 0);
+  return grouped_form(max_rows, n_experts, n_dim, k_dim, k_dim % kTileK == 0 && k_dim >= 2 * kTileK && n_dim % 8 == 0).rows;
 }
 
 extern "C" int hxm_grouped_linear(void* y, const void* x, int64_t x_stride, const int32_t* src, const void* w,
@@ -981,16 +984,12 @@ extern "C" int hxm_grouped_linear(void* y, const void* x, int64_t x_stride, cons
     u16* yy = (u16*)y;
     const u16 *xx = (const u16*)x, *ww = (const u16*)w;
     const bool walks = k_dim % kTileK == 0 && k_dim >= 2 * kTileK && (act == 2 || n_dim % 8 == 0) && aligned16(y);
-    switch (grouped_tile_rows(max_rows, n_experts, n_dim, k_dim, walks)) {
-      case 32:
-        if (k_dim < 2048) return launch_grouped<32, 64, 2, 2, 4>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
-        return launch_grouped<32, 64, 2, 2, 6>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
-      case 64: return launch_grouped<64, 128, 1, 4, 3>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
-      case 128: return launch_grouped<128, 128, 2, 2, 3>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
-      default:
-        if (walks) return launch_grouped_tiles(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
-        return launch_grouped<256, 256, 2, 4, 2>(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s);
-    }
+    const GroupedForm f = grouped_form(max_rows, n_experts, n_dim, k_dim, walks);
+    auto go = [&](auto launch) { return launch(yy, xx, x_stride, src, ww, seg, max_rows, n_experts, n_dim, k_dim, act, glu, s); };
+    if (f.rows == 32) return k_dim < 2048 ? go(launch_grouped<32, 64, 2, 2, 4>) : go(launch_grouped<32, 64, 2, 2, 6>);
+    if (f.rows == 64) return f.cols == 64 ? go(launch_grouped<64, 64, 4, 2, 3>) : go(launch_grouped<64, 128, 2, 4, 3>);
+    if (f.rows == 128) return f.cols == 64 ? go(launch_grouped<128, 64, 4, 2, 3>) : go(launch_grouped<128, 128, 2, 4, 3>);
+    return walks ? go(launch_grouped_tiles) : go(launch_grouped<256, 256, 2, 4, 2>);
   }
   const int64_t tiles = (max_rows + kGM - 1) / kGM + n_experts;
   if (tiles > 65535) return HX_ERR_SHAPE;

@@ -75,6 +75,17 @@ def test_grouped_linear_in_large_tiles(rows, n, k, act, tile):
     _check(rows, n, k, act, False)
 
 
+# tiles of 64 and of 128 rows by eight waves, 64 columns wide and 128: up to a tile's rows and one more, columns that no tile divides, with a
+# tail and without
+@pytest.mark.parametrize("rows, n, k, act, tile", [
+    ([129, 71], 4136, 264, "none", 128), ([1, 130, 128, 141], 2080, 520, "glu", 128), ([128, 72], 4128, 320, "relu2", 128), ([129, 171], 6184, 136, "none", 128),
+    ([172, 128], 6176, 520, "glu", 128), ([65, 1, 127, 87], 8256, 264, "glu", 64), ([63, 337], 8264, 520, "none", 64), ([65, 64, 1, 150], 8256, 320, "none", 64)])
+def test_grouped_linear_by_eight_waves(rows, n, k, act, tile):
+    from hydrainfer_amd import _lib
+    assert _lib.mix_lib().hxm_grouped_linear_tile_rows(sum(rows), len(rows), n, k) == tile
+    _check(rows, n, k, act, False)
+
+
 # enough tiles for those of 256 x 256: from tile to tile with two slices and with more, columns in 8s and whole turns, the last ones in
 # part; and k and n that take the form before it
 @pytest.mark.parametrize("rows", [[300, 257], [700, 0, 129], [1, 513]])
