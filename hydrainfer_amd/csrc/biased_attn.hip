@@ -640,18 +640,21 @@ __global__ __launch_bounds__(256) void biased_attn_group_kernel(hxm_biased_attn_
 // Measured, the two last points: 55.4 us before, 54.3 now, 2-norm of the error against 64 bits 2.057e-3 and 2.043e-3 (all tiles whole 54.2, but
 // portions of 64 keys off by 1 % more; half tiles as before, sums of the weights as they were before rounding: 53.7 with whole tiles
 // behind the first two, off by 0.05 % more).
+//   * where workgroups are few, two groups of four waves take every other tile of keys each, with images of their own, and add up what they have at
+//     the end: each hands the other half of its columns through LDS, scaled like the splits of a row (a wave alone on its SIMD goes from products
+//     to softmax to products, 2 - 3 us a tile).
 // The order of the row tiles: the XCDs (workgroups are dealt round robin) take key heads of their own where there are enough of
 // them, and of every sequence the tiles with the most keys come first.
 // Measured, 4 portions of 797 - 1151 tokens, 32 heads of 128 on 8 key heads, sinks: 221 us in the group form, 54 us
 // here (600 TFLOP/s of the pairs that a mask leaves); window of 512 and soft cap 223 and 68 us; chunks of 512 and slopes 163 and
 // 50 us.  Down to 64 rows of a key head it is the faster one (16 tokens behind 500 keys: 30 and 21 us).
 // ---------------------------------------------------------------------------------------------------------------
-template <int D, int V, bool MODS, bool FINE>      // MODS: slopes or a soft cap; FINE: every 32 keys' weights refer to their own largest score
-__global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_attn_args a, int tile_slots) {
+template <int D, int V, bool MODS, bool FINE, int KG>      // MODS: slopes or a soft cap; FINE: every 32 keys' weights refer to their own largest score; KG: groups of four waves
+__global__ __launch_bounds__(256 * KG, 2) void biased_attn_wide_kernel(hxm_biased_attn_args a, int tile_slots) {
   constexpr int KT = 64, TQ = 128, KS = D / 16, NDB = V / 32;
   constexpr int RSK = 2 * D, RSV = 2 * V, LK = D / 8, LV = V / 8;        // bytes and 16-byte chunks of a row
   constexpr int KTILE = KT * RSK, IMG = KTILE + KT * RSV;
-  extern __shared__ __attribute__((aligned(16))) char smem_w[];        // [2][K tile | V tile]
+  extern __shared__ __attribute__((aligned(16))) char smem_w[];        // [KG][2][K tile | V tile]
   auto kswz = [](int row) { return LK == 16 ? (row & 15) : ((row >> 1) & 7); };
   auto vswz = [](int row) { return LV == 16 ? ((row & 3) << 2) : (((row >> 1) & 1) << 2); };
   typedef __attribute__((address_space(4))) const int32_t c_i32;       // (uniform indices: through the scalar cache)
@@ -674,7 +677,8 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
   }
   int b, tile, q0, n_rows;
   if (!find_row_tile<TQ>(q_cu, a.n_seq, R, slot, b, tile, q0, n_rows)) return;      // spare slot (the grid is an upper bound)
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3), lane = threadIdx.x & 63;
+  const int group = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;      // takes every KG-th tile of keys
   const int c = lane & 31, hi = lane >> 5;
   // row tiles end with the portion: a partial one is the first, with the fewest keys.  Rows below 0 do not exist.
   const int row0_wg = n_rows - ((n_rows + TQ - 1) / TQ - tile) * TQ, row0 = row0_wg + 32 * wave;
@@ -696,7 +700,7 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
   const u16* vc = (const u16*)a.value_cache + (int64_t)kvh * a.head_stride;
   c_i32* table = (c_i32*)(a.block_table + ((c_i32*)a.cu_block_lens)[b]);
   const int bs = a.block_size, bshift = (bs & (bs - 1)) == 0 ? __ffs(bs) - 1 : -1;
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem_w;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem_w + (uint32_t)(group * 2 * IMG);
   // Wave w brings keys 16 w .. of a tile (one page): RPK / RPV rows an instruction, LK / LV lanes a row.  What lies in front of the
   // first key that some row sees, or behind the last, is not touched (its page may be gone): rows there repeat that key, masked.
   constexpr int RPK = 64 / LK, RPV = 64 / LV;
@@ -742,7 +746,7 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
     }
 #pragma clang diagnostic pop
   };
-  if (t_first <= t_last) bring(t_first, 0);
+  if (t_first + group <= t_last) bring(t_first + group, 0);
   // the queries (B operand): row c, columns 16 ks + 8 hi ..
   u16x8 qf[KS];
   {
@@ -778,7 +782,7 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
   const int tr_q = (lane & 15) >> 2, tr_x = vswz(tr_q) >> 2;
   const int tr_off = (4 * hi + tr_q) * RSV + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
   auto tile_step = [&](int t, int img) __attribute__((always_inline)) {
-    const char* kt = smem_w + img * IMG;
+    const char* kt = smem_w + (2 * group + img) * IMG;
     const char* vt = kt + KTILE;
     f32x16 s[2];
 #pragma unroll
@@ -910,21 +914,62 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
   };
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  for (int t = t_first; t <= t_last; ++t) {
-    const int img = (t - t_first) & 1;
-    if (t < t_last) bring(t + 1, img ^ 1);
-    if (live && t * KT <= wpos1 && t * KT + KT - 1 >= wlo0) tile_step(t, img);
+  for (int t0 = t_first; t0 <= t_last; t0 += KG) {
+    const int t = t0 + group, img = (t0 - t_first) / KG & 1;
+    if (t + KG <= t_last) bring(t + KG, img ^ 1);
+    if (live && t <= t_last && t * KT <= wpos1 && t * KT + KT - 1 >= wlo0) tile_step(t, img);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this wave's part of the next tile is there
     __syncthreads();                                       // everybody's is, and this one has been read
   }
-  if (!live) return;
+  // Two groups: each hands the other half of its columns and finishes the rest.  (One tile: the first group has it all.)
+  const bool two = KG > 1 && t_last > t_first;
+  if constexpr (KG > 1) {
+    if (two) {
+      f32x4* part = reinterpret_cast<f32x4*>(smem_w + 2 * IMG) + wave * (4 * NDB + 1) * 64 + lane;
+      auto hand = [&](auto first) __attribute__((always_inline)) {      // (first: the first column block that the other group finishes)
+#pragma unroll
+        for (int i = 0; i < NDB / 2; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const f32x16& x = acc[first + i];
+            part[(4 * (first + i) + e) * 64] = f32x4{x[4 * e], x[4 * e + 1], x[4 * e + 2], x[4 * e + 3]};
+          }
+      };
+      float2* ml = reinterpret_cast<float2*>(part - lane + 4 * NDB * 64) + lane;
+      if (group) hand(std::integral_constant<int, 0>());
+      else hand(std::integral_constant<int, NDB / 2>());
+      ml[64 * group] = float2{m, l};
+      __syncthreads();
+      const float2 o = ml[64 * (1 - group)];
+      const float top = fmaxf(m, o.x), mine = fast_exp2(m - top), theirs = fast_exp2(o.x - top);
+      l = __builtin_fmaf(l, mine, o.y * theirs);
+      m = top;
+      auto take = [&](auto first) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NDB / 2; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            f32x16& x = acc[first + i];
+            const f32x4 y = part[(4 * (first + i) + e) * 64];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) x[4 * e + k] = __builtin_fmaf(x[4 * e + k], mine, y[k] * theirs);
+          }
+      };
+      if (group) take(std::integral_constant<int, NDB / 2>());
+      else take(std::integral_constant<int, 0>());
+    } else if (group) {
+      return;
+    }
+  }
+  if (!live && !two) return;
   // out, through LDS (the images are free): whole rows a store.  O[row c][column 32 db + 8 (e >> 2) + 4 hi + (e & 3)]
   float total = l + __shfl_xor(l, 32, 64);
   if (a.sinks) total += fast_exp2(a.sinks[head] * kLog2e - m);      // the sink: one more term, without a value
   const float inv = 1.0f / total;
   char* ob = smem_w + wave * 32 * RSV;
 #pragma unroll
-  for (int db = 0; db < NDB; ++db)
+  for (int db = 0; db < NDB; ++db) {
+    if (two && (db < NDB / 2) == (group != 0)) continue;
 #pragma unroll
     for (int e4 = 0; e4 < 4; ++e4) {
       u16x4 o;
@@ -932,9 +977,12 @@ __global__ __launch_bounds__(256, 2) void biased_attn_wide_kernel(hxm_biased_att
       for (int i = 0; i < 4; ++i) o[i] = BF16::from_float(acc[db][4 * e4 + i] * inv);
       *reinterpret_cast<u16x4*>(ob + c * RSV + (((8 * db + 2 * e4 + hi) ^ (c & (LV - 1))) << 3)) = o;
     }
-  wave_lds_sync();
+  }
+  if (two) __syncthreads();
+  else wave_lds_sync();
 #pragma unroll
   for (int j = 0; j < 32 / RPV; ++j) {
+    if (two && (j & 1) != group) continue;
     const int rl = RPV * j + rv, ro = row0 + rl;
     // 8-byte slots 2 ch, 2 ch + 1 of row rl sit in chunk ch ^ (rl' >> 1), in turned order when rl' is odd (rl' = rl mod V / 8)
     u16x8 v = *reinterpret_cast<const u16x8*>(ob + rl * RSV + 16 * (cv ^ ((rl & (LV - 1)) >> 1)));
@@ -952,9 +1000,15 @@ int launch_wide(const hxm_biased_attn_args& a, hipStream_t s) {
   const bool mods = a.slopes || a.softcap > 0.f;
   // few rows: fewer tiles of 16 than the waves that the tile form's keys are dealt to (see its callers)
   const bool fine = (int64_t)a.n_seq * a.kv_heads * (((int64_t)a.max_q_len * R + 15) / 16) < 2048;
-  auto kernel = fine ? (mods ? biased_attn_wide_kernel<D, V, true, true> : biased_attn_wide_kernel<D, V, false, true>)
-                     : (mods ? biased_attn_wide_kernel<D, V, true, false> : biased_attn_wide_kernel<D, V, false, false>);
-  constexpr size_t lds = 2 * 64 * (2 * D + 2 * V);
+  // Such a launch gives a compute unit one workgroup: two groups of waves share its keys, so that a SIMD has two waves.  Portions of up to a
+  // tile's keys have nothing to share (us, one group and two: 4 of 20 - 52 tokens, cap and slopes 10.6 11.6; one of 128 - 152, 10.4 10.6; 2 of 81 - 217
+  // 18.1 16.2, 1082 behind 463 41.8 33.4, 110 behind 495 25.5 19.7; 40 launches drawn from these ranges 1 and 0.94).
+  const int groups = fine && a.max_q_len > 64 ? 2 : 1;
+  auto kernel = groups == 2 ? (mods ? biased_attn_wide_kernel<D, V, true, true, 2> : biased_attn_wide_kernel<D, V, false, true, 2>)
+                : fine      ? (mods ? biased_attn_wide_kernel<D, V, true, true, 1> : biased_attn_wide_kernel<D, V, false, true, 1>)
+                            : (mods ? biased_attn_wide_kernel<D, V, true, false, 1> : biased_attn_wide_kernel<D, V, false, false, 1>);
+  constexpr size_t images = 2 * 64 * (2 * D + 2 * V), part = 4 * (V / 2 + 4) * 256;      // (of a group of waves; what the groups hand over, in the place of the second one's images)
+  const size_t lds = groups == 2 ? images + std::max(images, part) : images;
   if (lds > 48 * 1024) {
     const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) {
@@ -962,7 +1016,7 @@ int launch_wide(const hxm_biased_attn_args& a, hipStream_t s) {
       return HX_ERR_HIP;
     }
   }
-  kernel<<<dim3((unsigned)grid), dim3(256), lds, s>>>(a, (int)slots);
+  kernel<<<dim3((unsigned)grid), dim3(256 * groups), lds, s>>>(a, (int)slots);
   return hxm::check_launch();
 }
 

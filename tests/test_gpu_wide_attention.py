@@ -51,6 +51,14 @@ def test_wide_form(batch, H, G, D, V, mask, size, extra):
     check(new, kv, H, G, D, V, mask, size, extra)
 
 
+# keys shared by two groups of waves: one tile, two, three, an odd and an even number of them, tiles that only one group's rows or neither's see
+@pytest.mark.parametrize("batch", [[(65, 65)], [(66, 128)], [(100, 129)], [(70, 257), (200, 200), (1, 64)], [(129, 705)]], ids=lambda b: f"{len(b)}x{max(b)}")
+@pytest.mark.parametrize("H, G, D, V", [(4, 1, 128, 128), (8, 8, 64, 64), (6, 2, 128, 64), (4, 4, 64, 128)])
+@pytest.mark.parametrize("mask, size, extra", [("causal", 0, "plain"), ("window", 70, "slopes"), ("chunk", 128, "cap"), ("window", 3, "temperatures and sinks")])
+def test_two_groups_of_waves(batch, H, G, D, V, mask, size, extra):
+    check([a for a, _ in batch], [b for _, b in batch], H, G, D, V, mask, size, extra)
+
+
 # single tokens at the edges of tiles and splits, sequences far shorter than others, two row tiles, more keys in one run than a wave
 # holds pages of (1024), sixteen tokens behind many keys
 STEPS = [[(1, 1)], [(1, 32), (1, 33), (1, 200), (1, 1025)], [(3, 70), (1, 16), (7, 2300)], [(1, 100)] * 40, [(16, 1500), (2, 40)]]
