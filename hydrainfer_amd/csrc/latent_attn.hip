@@ -1030,11 +1030,11 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide_kernel(hxm_latent_att
 // Row r of sixteen has its chunks at x ^ swz(r): rows r and 15 - r share a 32-byte place (their
 // chunks turned), so that a pass of a 16-byte read (rows 0-3 and 12-15 of one chunk, 4-11 of the next) and a transposing read
 // (eight rows, 32 bytes each) both reach every bank once.
-template <int KK, bool FINE>      // FINE: every tile's weights refer to their own largest score
-__global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_attn_args a, int tiles_per_seq) {
+template <int KK, bool FINE, int KG>      // FINE: every tile's weights refer to their own largest score; KG: groups of four waves, which share the keys
+__global__ __launch_bounds__(256 * KG, 2) void latent_attn_wide16_kernel(hxm_latent_attn_args a, int tiles_per_seq) {
   constexpr int R = 64 * KK, KT = 32, TQ = 64, KPW = 8, KS = R / 32, NDB = R / 16, RS = 2 * R, L = R / 8, IMG = KT * RS;
   constexpr bool FULL = RS % 256 == 0;       // rows of whole bank rows: 16 places of a chunk, else 8 for each parity of the row
-  extern __shared__ __attribute__((aligned(256))) char smem_w[];       // [2][32 rows]
+  extern __shared__ __attribute__((aligned(256))) char smem_w[];       // [KG][2][32 rows]
   auto swz = [](int row) {
     if (FULL) return (row & 15) < 8 ? 2 * (row & 7) : 31 - 2 * (row & 15);
     const int h = (row & 15) >> 1;
@@ -1046,7 +1046,8 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
   const int n_splits = FINE && a.n_splits > 1 ? a.n_splits : 1, split = n_splits > 1 ? (int)(blockIdx.x % n_splits) : 0;
   int b, tile, q0, n_rows;
   if (!find_row_tile<TQ>(q_cu, a.n_seq, H, (int)(n_splits > 1 ? blockIdx.x / n_splits : blockIdx.x), b, tile, q0, n_rows)) return;      // spare slot (the grid is an upper bound)
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3), lane = threadIdx.x & 63;
+  const int group = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;      // takes every KG-th tile of keys
   const int c = lane & 15, g = lane >> 4;
   const int row0_wg = n_rows - ((n_rows + TQ - 1) / TQ - tile) * TQ, row0 = row0_wg + 16 * wave;
   const int r = max(row0 + c, 0), tok = r / H, head = r % H;
@@ -1067,7 +1068,7 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
   const u16* cache = (const u16*)a.cache;
   c_i32* table = (c_i32*)(a.block_table + ((c_i32*)a.cu_block_lens)[b]);
   const int bs = a.block_size, bshift = (bs & (bs - 1)) == 0 ? __ffs(bs) - 1 : -1;
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem_w;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem_w + (uint32_t)(group * 2 * IMG);
   // Wave w brings keys 8 w .. of a tile (one page): 8 L chunks, 64 an instruction; none in front of the first or behind the last, as above.
   constexpr int NL = KPW * L / 64;
   const uint32_t row_bytes = (uint32_t)(2 * a.cache_row_stride);
@@ -1095,7 +1096,7 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
     }
 #pragma clang diagnostic pop
   };
-  if (t_first <= t_last) bring(t_first, 0);
+  if (t_first + group <= t_last) bring(t_first + group, 0);
   u16x8 qf[KS];                              // the queries (B operand): row c, columns 32 ks + 8 g ..
   {
     const u16* qg = (const u16*)a.q + (int64_t)(q0 + tok) * a.q_token_stride + (int64_t)head * a.q_head_stride + 8 * g;
@@ -1218,14 +1219,48 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
   };
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  for (int t = t_first; t <= t_last; ++t) {
-    const int img = (t - t_first) & 1;
-    if (t < t_last) bring(t + 1, img ^ 1);
-    if (live && t * KT <= wpos1 && t * KT + KT - 1 >= wlo0) step(t * KT, (uint32_t)(img * IMG));
+  for (int t0 = t_first; t0 <= t_last; t0 += KG) {
+    const int t = t0 + group, img = (t0 - t_first) / KG & 1;
+    if (t + KG <= t_last) bring(t + KG, img ^ 1);
+    if (live && t <= t_last && t * KT <= wpos1 && t * KT + KT - 1 >= wlo0) step(t * KT, (uint32_t)(img * IMG));
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this wave's part of the next tile is there
     __syncthreads();                                       // everybody's is, and this one has been read
   }
-  if (!live) return;
+  // Two groups: each hands the other half of its columns and finishes the rest.  (One tile: the first group has it all.)
+  const bool two = KG > 1 && t_last > t_first;
+  if constexpr (KG > 1) {
+    if (two) {
+      f32x4* part = reinterpret_cast<f32x4*>(smem_w) + wave * NDB * 64 + lane;
+      float2* ml = reinterpret_cast<float2*>(smem_w + 4 * NDB * 1024) + wave * 128 + lane;
+      auto hand = [&](auto first) __attribute__((always_inline)) {      // (first: the first column block that the other group finishes)
+#pragma unroll
+        for (int i = first; i < first + NDB / 2; ++i) part[i * 64] = acc[i];
+      };
+      if (group) hand(std::integral_constant<int, 0>());
+      else hand(std::integral_constant<int, NDB / 2>());
+      ml[64 * group] = float2{m, l};
+      __syncthreads();
+      const float2 o = ml[64 * (1 - group)];
+      const float top = fmaxf(m, o.x), mine = fast_exp2(m - top), theirs = fast_exp2(o.x - top);
+      l = __builtin_fmaf(l, mine, o.y * theirs);
+      m = top;
+      auto take = [&](auto first) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = first; i < first + NDB / 2; ++i) {
+          const f32x4 x = part[i * 64];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i][e] = __builtin_fmaf(acc[i][e], mine, x[e] * theirs);
+        }
+      };
+      if (group) take(std::integral_constant<int, NDB / 2>());
+      else take(std::integral_constant<int, 0>());
+      __syncthreads();                                     // (results go where these came from)
+    } else if (group) {
+      return;
+    }
+  }
+  auto finishes = [&](int db) { return !two || (db >= NDB / 2) == (group != 0); };
+  if (!live && !two) return;
   // out, through LDS (the images are free): whole rows a store.  O[row c][column 16 db + 4 g + e]
   float total = l + __shfl_xor(l, 16, 64);
   total += __shfl_xor(total, 32, 64);
@@ -1235,8 +1270,9 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
       const size_t at = ((size_t)b * tiles_per_seq * 16 + (row0 + c)) * n_splits + split;
       float* wo = a.ws_o + at * R + 4 * g;
 #pragma unroll
-      for (int db = 0; db < NDB; ++db) *reinterpret_cast<f32x4*>(wo + 16 * db) = acc[db];
-      if (g == 0) {
+      for (int db = 0; db < NDB; ++db)
+        if (finishes(db)) *reinterpret_cast<f32x4*>(wo + 16 * db) = acc[db];
+      if (g == 0 && group == 0) {
         a.ws_ml[2 * at] = m;
         a.ws_ml[2 * at + 1] = total;
       }
@@ -1252,16 +1288,19 @@ __global__ __launch_bounds__(256, 2) void latent_attn_wide16_kernel(hxm_latent_a
   char* ob = smem_w + wave * 16 * RS;
 #pragma unroll
   for (int db = 0; db < NDB; ++db) {         // 8-byte slot 4 db + g of row c, turned by the row within its 128 bytes
+    if (!finishes(db)) continue;
     u16x4 o;
 #pragma unroll
     for (int i = 0; i < 4; ++i) o[i] = BF16::from_float(acc[db][i] * gsc);
     *reinterpret_cast<u16x4*>(ob + c * RS + (((4 * db + g) ^ c) << 3)) = o;
   }
+  if (two) __syncthreads();
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
   for (int j = 0; j < 16 * L / 64; ++j) {
+    if (two && (j & 1) != group) continue;
     const int rl = (64 * j + lane) / L, ch = (64 * j + lane) % L, ro = row0 + rl;
     // slots 2 ch, 2 ch + 1 of row rl sit in chunk ch ^ (rl >> 1), in turned order when rl is odd
     u16x8 v = *reinterpret_cast<const u16x8*>(ob + rl * RS + 16 * (ch ^ (rl >> 1)));
@@ -1333,6 +1372,10 @@ struct WidePlan {
   bool fits, rows32;
   int splits;
 };
+// keys that a portion looks at, at most
+int key_reach(const hxm_latent_attn_args& a) {
+  return a.window > 0 && a.window + a.max_q_len < a.max_kv_len ? a.window + a.max_q_len : a.max_kv_len;
+}
 WidePlan wide_plan(const hxm_latent_attn_args& a) {
   WidePlan p{false, false, 1};
   if (a.kv_rank % 64 || a.block_size % 16 || a.out_token_stride % 8 || a.out_head_stride % 8 || !aligned16(a.out) || !aligned16(a.ws_o) ||
@@ -1346,8 +1389,7 @@ WidePlan wide_plan(const hxm_latent_attn_args& a) {
     p.splits = hxm::latent_step_splits(a);
     return p;
   }
-  int reach = a.max_kv_len;
-  if (a.window > 0 && a.window + a.max_q_len < reach) reach = a.window + a.max_q_len;
+  const int reach = key_reach(a);
   const int64_t tiles = a.n_seq * ((rows + 63) / 64);
   int64_t want = (512 + tiles - 1) / tiles;
   // (a split more shortens the walk over the keys and lengthens the writing and merging of what the splits hold, 8 bytes a row and
@@ -1366,12 +1408,21 @@ int launch_wide16(const hxm_latent_attn_args& a, hipStream_t s) {
   const int n_splits = a.n_splits > 1 ? a.n_splits : 1, tiles16 = (int)(((int64_t)a.max_q_len * a.n_heads + 15) / 16);
   const int64_t grid = (((int64_t)a.n_tokens * a.n_heads + 63) / 64 + a.n_seq) * n_splits;      // row tiles of all sequences, at most
   if (grid > 0x7fffffff) return HX_ERR_SHAPE;
-  constexpr size_t lds = 2 * 32 * 2 * 64 * KK;
+  constexpr size_t images = 2 * 32 * 2 * 64 * KK;          // (of a group of waves)
   // (few rows: where the tile form would deal out the keys)
   const bool fine = n_splits > 1 || (int64_t)a.n_seq * tiles16 < kTileWaves;
-  auto kernel = fine ? latent_attn_wide16_kernel<KK, true> : latent_attn_wide16_kernel<KK, false>;
+  // One workgroup a compute unit leaves a SIMD one wave: two groups of waves share the keys, from seven tiles of them on (us, one group and two, 32 heads
+  // on portions of 100 - 200 tokens: 50 keys of 256 columns 9.7 10.7, 195 of 320 17.5 17.4, 283 of 128 12.9 11.9, 450 of 256 25.2 21.9, 554 of 256 28.4 23.5; up to
+  // 128 columns a compute unit takes two such workgroups: 16 heads on 198 and 845 tokens of 128 columns, 271 workgroups, 26.1 21.1).  More
+  // than 320 columns are more than a second group's sums leave registers for, and what is dealt to workgroups already gains nothing.
+  const bool two = KK <= 5 && n_splits == 1 && fine && grid - a.n_seq <= (KK <= 2 ? 512 : 256) && key_reach(a) >= 224;
+  const size_t lds = two ? 2 * images + 4096 : images;
+  auto kernel = fine ? latent_attn_wide16_kernel<KK, true, 1> : latent_attn_wide16_kernel<KK, false, 1>;
+  if constexpr (KK <= 5) {
+    if (two) kernel = latent_attn_wide16_kernel<KK, true, 2>;
+  }
   if (const int rc = prepare_lds((const void*)kernel, lds)) return rc;
-  kernel<<<dim3((unsigned)grid), dim3(256), lds, s>>>(a, tiles16);
+  kernel<<<dim3((unsigned)grid), dim3(two ? 512 : 256), lds, s>>>(a, tiles16);
   if (n_splits > 1) {
     int lanes_log2 = 4;                      // a row to R / 4 lanes, at most a power of two of them
     while ((8 << lanes_log2) <= a.kv_rank && lanes_log2 < 7) ++lanes_log2;

@@ -36,6 +36,15 @@ def test_wide_forms_of_many_rows(R, window, extra):
     check([a for a, _ in MANY], [b for _, b in MANY], R, 32, window, extra, WIDE32 if R <= 192 else WIDE16)
 
 
+# keys shared by two groups of waves (up to 320 columns, few row tiles): an odd and an even number of tiles, portions of one tile beside
+# others, tiles that only one group's rows or neither's see
+@pytest.mark.parametrize("batch", [[(150, 257)], [(160, 224), (70, 300), (1, 20)], [(400, 700)]], ids=lambda b: f"{len(b)}x{max(b)}")
+@pytest.mark.parametrize("R", [64, 128, 192, 256, 320, 384])
+@pytest.mark.parametrize("window, extra", [(0, "plain"), (0, "sinks and gate"), (200, "negative"), (160, "sinks")])
+def test_two_groups_of_waves(batch, R, window, extra):
+    check([a for a, _ in batch], [b for _, b in batch], R, 32, window, extra, WIDE16)
+
+
 # single tokens: one tile and a split's edge, splits that get no tile (one sequence far shorter than another), more sequences than a
 # round of the row tiles' search holds
 STEPS = [[64], [129, 1, 32, 33], [2000, 3], [700] * 5, [40] * 260 + [130]]
