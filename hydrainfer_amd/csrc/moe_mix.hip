@@ -691,21 +691,34 @@ __global__ __launch_bounds__(256, 1) void grouped_linear_tile_kernel(u16* __rest
                                                                      const int32_t* __restrict__ seg, int E, int64_t N, int64_t K, int act, Glu glu) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int n_col = (int)((N + kTileRows - 1) / kTileRows), n = (int)(K / kTileK);      // (n >= 2)
-  int at, end;
+  int at, end, e = 0, before = 0;                          // the expert whose tiles are walked, tiles in front of it
   {
-    int m_tiles = 0;
-    for (int i = 0; i < E; ++i) m_tiles += (seg[i + 1] - seg[i] + kTileRows - 1) / kTileRows;
+    const int expert_lane = threadIdx.x & 63;
+    ExpertTiles some(seg, E, 0, kTileRows, expert_lane);
+    int m_tiles = some.total();
+    for (int e0 = 64; e0 < E; e0 += 64) m_tiles += ExpertTiles(seg, E, e0, kTileRows, expert_lane).total();
     const int total = m_tiles * n_col, per = (total + 7) >> 3;
     at = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
     end = min(total, (int)(blockIdx.x & 7) * per + per);
+    if (at >= end) return;                                 // (the whole workgroup)
+    for (;;) {                                             // the first tile's expert
+      const uint64_t behind = __builtin_amdgcn_ballot_w64(at - before < some.run * n_col);
+      if (behind) {
+        const int l = __builtin_ctzll(behind);
+        e += l;
+        before += (__builtin_amdgcn_readlane(some.run, l) - __builtin_amdgcn_readlane(some.nt, l)) * n_col;
+        break;
+      }
+      before += some.total() * n_col;
+      e += 64;
+      some = ExpertTiles(seg, E, e, kTileRows, expert_lane);
+    }
   }
-  if (at >= end) return;                                   // (the whole workgroup)
   const int step = (int)(gridDim.x >> 3);
   struct Tile {
     int e, row0, row1;
     int64_t col0;
   } tile, next;
-  int e = 0, before = 0;                                   // the expert whose tiles are walked, tiles in front of it
   auto find = [&](int i) __attribute__((always_inline)) {
     for (;; ++e) {
       const int r0 = seg[e], r1 = seg[e + 1], nt = (r1 - r0 + kTileRows - 1) / kTileRows, in = i - before;

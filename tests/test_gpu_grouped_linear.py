@@ -95,6 +95,14 @@ def test_grouped_linear_from_tile_to_tile(rows, n, k, act):
     _check(rows, n, k, act, False)
 
 
+# the same with more experts than a wave has lanes, some of them without rows
+def test_grouped_linear_from_tile_to_tile_of_many_experts():
+    from hydrainfer_amd import _lib
+    rows = [0 if e in (0, 5, 64) else 257 if e % 2 else 240 for e in range(67)]
+    assert _lib.mix_lib().hxm_grouped_linear_tile_rows(sum(rows), len(rows), 512, 256) == 256
+    _check(rows, 512, 256, "none", False)
+
+
 @pytest.mark.parametrize("rows", [[1, 30], [129, 0, 127], [256, 257]])
 def test_grouped_linear_of_rows_far_apart(rows):
     _check(rows, 160, 200, "none", True)
