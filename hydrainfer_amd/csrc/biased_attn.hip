@@ -1029,15 +1029,18 @@ int launch_wide(const hxm_biased_attn_args& a, hipStream_t s) {
 // O^T += V^T P^T: a row of the softmax is one lane, its weights stay in their registers.  16-byte chunk x of row r sits at
 // x ^ swz(r): rows r and 15 - r share a 32-byte place (their chunks turned), so that a pass of a 16-byte read and a transposing
 // read (eight rows, 32 bytes each) both reach every bank once.
+// Two or four runs of a row tile's keys are a workgroup's, a wave each, merged through LDS where the images were; only more of them go through memory
+// and a second launch.  32 tokens of 1025 - 2047 keys 46.7 us with it, 43 without, 20 of 55 - 253 9.6 and 6.7, 224 row tiles of 1500 45.9 and 35.3 (with five
+// splits); 15 % in the mean of 50 batches.
 // Measured, 32 heads of 128 on 8 key heads, kernel and merge: 32 tokens of 1025 - 2047 keys 48 + 8 us in the tile form, 36 + 4 here
 // (5.5 TB/s); 128 tokens of 500 - 1500 keys 163 us and 109; 32 tokens, 2 key heads 57 us and 24; 16 tokens behind 4000 keys
 // 93 us (tile), 79 (wide) and 29.
 // ---------------------------------------------------------------------------------------------------------------
-template <int D, int V, bool MODS>      // MODS: slopes or a soft cap
-__global__ __launch_bounds__(64) void biased_attn_step_kernel(hxm_biased_attn_args a, int tiles_per_seq) {
+template <int D, int V, bool MODS, int W>      // MODS: slopes or a soft cap; W: waves, a split each
+__global__ __launch_bounds__(64 * W) void biased_attn_step_kernel(hxm_biased_attn_args a, int tiles_per_seq) {
   constexpr int KT = 32, KS = D / 32, NDB = V / 16, RSK = 2 * D, RSV = 2 * V, LK = D / 8, LV = V / 8;
   constexpr int KTILE = KT * RSK, IMG = KTILE + KT * RSV, NLK = 16 * LK / 64, NLV = 16 * LV / 64;      // transfers of 16 rows
-  extern __shared__ __attribute__((aligned(256))) char smem_s[];       // [2][K rows | V rows]
+  extern __shared__ __attribute__((aligned(256))) char smem_s[];       // [W][2][K rows | V rows]
   auto swz = [](int row, bool full) {        // full: rows of whole bank rows, 16 places of a chunk, else 8 for each parity of the row
     if (full) return (row & 15) < 8 ? 2 * (row & 7) : 31 - 2 * (row & 15);
     const int h = (row & 15) >> 1;
@@ -1049,12 +1052,13 @@ __global__ __launch_bounds__(64) void biased_attn_step_kernel(hxm_biased_attn_ar
   int at = blockIdx.x;
   const int kvh = at % G;
   at /= G;
-  const int split = at % n_splits;
-  at /= n_splits;
+  const int wave = W > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0, n_groups = n_splits / W, group = at % n_groups;
+  const int split = group * W + wave;
+  at /= n_groups;
   const int tile = at % tiles_per_seq, b = at / tiles_per_seq;
   const int q0 = ((c_i32*)a.q_cu)[b], n_rows = (((c_i32*)a.q_cu)[b + 1] - q0) * R, n_tiles = (n_rows + 15) / 16;
   if (tile >= n_tiles) return;
-  const int lane = threadIdx.x, c = lane & 15, g = lane >> 4;
+  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   const int row0 = n_rows - (n_tiles - tile) * 16;      // (row tiles end with the portion; rows below 0 do not exist)
   const int r = max(row0 + c, 0), tok = r / R, head = kvh * R + r % R;
   const int pos = a.positions[q0 + tok], lo = first_visible(pos, a.mask_kind, a.mask_size);
@@ -1089,7 +1093,7 @@ __global__ __launch_bounds__(64) void biased_attn_step_kernel(hxm_biased_attn_ar
   asm volatile("" : "+v"(pages), "+v"(hsc), "+v"(slope2), "+v"(sink2));      // (all there before the transfers start: a wait for them would be one for those)
   const u16* kc = (const u16*)a.key_cache + (int64_t)kvh * a.head_stride;
   const u16* vc = (const u16*)a.value_cache + (int64_t)kvh * a.head_stride;
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem_s;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem_s + (uint32_t)(wave * 2 * IMG);
   const uint32_t row_bytes = (uint32_t)(2 * a.cache_row_stride);
   auto bring = [&](int t, int img) __attribute__((always_inline)) {
     if (2 * t + 1 - pages0 > 63) {
@@ -1226,34 +1230,67 @@ __global__ __launch_bounds__(64) void biased_attn_step_kernel(hxm_biased_attn_ar
     }
     __builtin_amdgcn_sched_group_barrier(0x008, kAhead, 0);
   }
-  if (row0 + c < 0) return;
-  float total = l + __shfl_xor(l, 16, 64);      // (rows below 0 are whole columns of lanes)
+  float total = l + __shfl_xor(l, 16, 64);
   total += __shfl_xor(total, 32, 64);
-  if (n_splits > 1) {
-    // what this split adds to a row, not normalised: ws_o [sequence, key head, tile][row][split][V], ws_ml [..][split][maximum (log2), sum]
-    const size_t slot = ((((size_t)b * G + kvh) * tiles_per_seq + tile) * 16 + c) * n_splits + split;
-    float* wo = a.ws_o + slot * V + 4 * g;
+  constexpr int NW = NDB / W;                // column blocks that a wave finishes
+  if constexpr (W > 1) {                     // the waves' splits merged, each wave's part where its images were
+    f32x4* part = reinterpret_cast<f32x4*>(smem_s);
+    auto part_of = [&](int w) { return part + w * (2 * IMG / 16); };
 #pragma unroll
-    for (int db = 0; db < NDB; ++db) *reinterpret_cast<f32x4*>(wo + 16 * db) = acc[db];
-    if (g == 0) {
+    for (int db = 0; db < NDB; ++db) part_of(wave)[64 * db + lane] = acc[db];
+    reinterpret_cast<float2*>(part_of(wave) + 64 * NDB)[lane] = float2{m, total};
+    __syncthreads();
+    float2 ml[W];
+    f32x4 v[W][NW];
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      ml[w] = reinterpret_cast<const float2*>(part_of(w) + 64 * NDB)[lane];
+#pragma unroll
+      for (int i = 0; i < NW; ++i) v[w][i] = part_of(w)[64 * (NW * wave + i) + lane];
+    }
+    m = ml[0].x;
+#pragma unroll
+    for (int w = 1; w < W; ++w) m = fmaxf(m, ml[w].x);
+    total = 0.f;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const float weight = fast_exp2(ml[w].x - m);
+      total += weight * ml[w].y;
+#pragma unroll
+      for (int i = 0; i < NW; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][e] += weight * v[w][i][e];
+    }
+  }
+  if (row0 + c < 0) return;                  // (rows below 0 are whole columns of lanes)
+  const int col0 = 16 * NW * wave;
+  if (n_groups > 1) {
+    // what this split adds to a row, not normalised: ws_o [sequence, key head, tile][row][split][V], ws_ml [..][split][maximum (log2), sum]
+    const size_t slot = ((((size_t)b * G + kvh) * tiles_per_seq + tile) * 16 + c) * n_groups + group;
+    float* wo = a.ws_o + slot * V + col0 + 4 * g;
+#pragma unroll
+    for (int db = 0; db < NW; ++db) *reinterpret_cast<f32x4*>(wo + 16 * db) = acc[db];
+    if (g == 0 && wave == 0) {
       a.ws_ml[2 * slot] = m;
       a.ws_ml[2 * slot + 1] = total;
     }
     return;
   }
   const float inv = 1.0f / (total + fast_exp2(sink2 - m));      // the sink: one more term, without a value
-  u16* og = (u16*)a.out + ((int64_t)(q0 + tok) * a.n_heads + head) * V + 4 * g;
+  u16* og = (u16*)a.out + ((int64_t)(q0 + tok) * a.n_heads + head) * V + col0 + 4 * g;
 #pragma unroll
-  for (int db = 0; db < NDB; ++db)
+  for (int db = 0; db < NW; ++db)
     *reinterpret_cast<u16x4*>(og + 16 * db) = u16x4{BF16::from_float(acc[db][0] * inv), BF16::from_float(acc[db][1] * inv), BF16::from_float(acc[db][2] * inv), BF16::from_float(acc[db][3] * inv)};
 }
 
 // The splits of a row merged: out = sum_s O_s 2^(m_s - M) / sum_s l_s 2^(m_s - M).  A row to V / 4 lanes; one pass over the splits,
 // four at a time, their loads all in flight together.
 template <int V>
-__global__ __launch_bounds__(256) void biased_attn_merge_kernel(hxm_biased_attn_args a, int tiles_per_seq) {
+__global__ __launch_bounds__(256) void biased_attn_merge_kernel(hxm_biased_attn_args a, int n_parts, int tiles_per_seq) {
   const int64_t at = (int64_t)blockIdx.x * 256 + threadIdx.x, slot = at / (V / 4);      // slot: row c of (sequence, key head, tile)
-  const int G = a.kv_heads, R = a.n_heads / a.kv_heads, NS = a.n_splits, col = 4 * (int)(at % (V / 4));
+  const int G = a.kv_heads, R = a.n_heads / a.kv_heads, NS = n_parts, col = 4 * (int)(at % (V / 4));
   const int64_t item = slot / 16;
   const int tile = (int)(item % tiles_per_seq), kvh = (int)(item / tiles_per_seq % G), b = (int)(item / tiles_per_seq / G);
   if (b >= a.n_seq) return;
@@ -1295,16 +1332,35 @@ __global__ __launch_bounds__(256) void biased_attn_merge_kernel(hxm_biased_attn_
   *reinterpret_cast<u16x4*>(og) = u16x4{BF16::from_float(o[0] * inv), BF16::from_float(o[1] * inv), BF16::from_float(o[2] * inv), BF16::from_float(o[3] * inv)};
 }
 
+template <int D, int V, int W>
+int launch_step_waves(const hxm_biased_attn_args& a, hipStream_t s) {
+  const int R = a.n_heads / a.kv_heads, tiles_per_seq = (int)(((int64_t)a.max_q_len * R + 15) / 16), n_groups = (a.n_splits > 1 ? a.n_splits : 1) / W;
+  const int64_t items = (int64_t)a.n_seq * a.kv_heads * tiles_per_seq;
+  if (items * n_groups > 0x7fffffff) return HX_ERR_SHAPE;
+  const bool mods = a.slopes || a.softcap > 0.f;
+  auto kernel = mods ? biased_attn_step_kernel<D, V, true, W> : biased_attn_step_kernel<D, V, false, W>;
+  constexpr size_t lds = (size_t)W * 2 * 32 * (2 * D + 2 * V);
+  if (lds > 48 * 1024) {
+    const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) {
+      hxm::last_hip_error() = (int)e;
+      return HX_ERR_HIP;
+    }
+  }
+  kernel<<<dim3((unsigned)(items * n_groups)), dim3(64 * W), lds, s>>>(a, tiles_per_seq);
+  if (n_groups > 1) biased_attn_merge_kernel<V><<<dim3((unsigned)((items * 16 * (V / 4) + 255) / 256)), dim3(256), 0, s>>>(a, n_groups, tiles_per_seq);
+  return hxm::check_launch();
+}
+// A few workgroups of four waves more than compute units take as long as twice as many: waves by themselves then (288 row tiles of 700 - 2100 keys 52.6 us,
+// by fours 55.8)
+bool between_rounds(int64_t tiles) { return tiles > 256 && tiles < 384; }
 template <int D, int V>
 int launch_step(const hxm_biased_attn_args& a, hipStream_t s) {
-  const int R = a.n_heads / a.kv_heads, tiles_per_seq = (int)(((int64_t)a.max_q_len * R + 15) / 16), n_splits = a.n_splits > 1 ? a.n_splits : 1;
-  const int64_t items = (int64_t)a.n_seq * a.kv_heads * tiles_per_seq;
-  if (items * n_splits > 0x7fffffff) return HX_ERR_SHAPE;
-  const bool mods = a.slopes || a.softcap > 0.f;
-  auto kernel = mods ? biased_attn_step_kernel<D, V, true> : biased_attn_step_kernel<D, V, false>;
-  kernel<<<dim3((unsigned)(items * n_splits)), dim3(64), 2 * 32 * (2 * D + 2 * V), s>>>(a, tiles_per_seq);
-  if (n_splits > 1) biased_attn_merge_kernel<V><<<dim3((unsigned)((items * 16 * (V / 4) + 255) / 256)), dim3(256), 0, s>>>(a, tiles_per_seq);
-  return hxm::check_launch();
+  const int64_t tiles = (int64_t)a.n_seq * a.kv_heads * (((int64_t)a.max_q_len * (a.n_heads / a.kv_heads) + 15) / 16);
+  if (a.n_splits == 4 && between_rounds(tiles)) return launch_step_waves<D, V, 1>(a, s);
+  if (a.n_splits > 1 && a.n_splits % 4 == 0) return launch_step_waves<D, V, 4>(a, s);
+  if (a.n_splits > 1 && a.n_splits % 2 == 0) return launch_step_waves<D, V, 2>(a, s);
+  return launch_step_waves<D, V, 1>(a, s);
 }
 
 // the splits of a (sequence, kv head, row tile) merged: out = sum_s O_s e^(m_s - M) / sum_s l_s e^(m_s - M)
@@ -1456,7 +1512,11 @@ extern "C" int hxm_biased_attention(const hxm_biased_attn_args* args, void* stre
 // five waves of the step form fill a CU (1024 and 2048 waves: 32 tokens of 1025 - 2047 keys 39.5 and 41.9 us, 128 of 500 - 1500 109
 // and 116); portions of 64 rows and more go undivided to the wide form unless they are few and their keys many (one portion behind
 // keys, 32 heads on 8 key heads, wide and split: 32 tokens behind 2000 44.8 and 24.9 us, 100 behind 2000 46.4 and 36.4, 100 behind
-// none 21 and 23.5, 8 times 16 behind 500 21.4 and 23.9).
+// none 21 and 23.5, 8 times 16 behind 500 21.4 and 23.9).  Four splits are merged where they are made and take one launch: that many where
+// there would be up to seven, or up to eleven on 64 row tiles and more with 2000 keys and fewer (the other launch is 4 us); multiples of four else, no more than four
+// a compute unit (us; splits as they were, four, eight: 32 heads of 128 on 8 key heads, tokens of 700 keys: one 9.4 10.6 9.2, eight 13.0 12.1 12.4, 13 15.2 12.5
+// 14.4, 16 15.9 13.1 15.5, 24 22.9 16.1 22.5; of 1500 16 24.4 23.5 23.8; of 3000 13 47 44 37, 16 42.9 46.2 42.0, 24 71 58 67; nine of 2100, 15 splits, 16: 24.1 26.9;
+// 18 of 1333 - 4000 48 57).
 extern "C" int hxm_biased_attention_plan(const hxm_biased_attn_args* args, int32_t max_kv_len, int32_t* n_splits, int64_t* ws_floats) {
   if (!args || !n_splits || !ws_floats) return HX_ERR_NULL;
   const hxm_biased_attn_args& a = *args;
@@ -1471,6 +1531,11 @@ extern "C" int hxm_biased_attention_plan(const hxm_biased_attn_args* args, int32
   const bool whole = a.form == 0 && (a.dim == 64 || a.dim == 128) && (a.vdim == 64 || a.vdim == 128) && a.block_size % 16 == 0;
   int64_t ns = std::min({((whole ? 1024 : 2048) + tiles - 1) / tiles, (reach + 31) / 32 / 2, (int64_t)64});
   if (whole && rows >= 64 && (tiles > 256 || reach < 1024)) ns = 1;
+  if (whole && ns > 2 && !between_rounds(tiles)) {
+    if (ns < 8 || (reach <= 2000 && ns < 12 && tiles >= 64) || (reach <= 512 && ns == 8)) ns = 4;
+    else if (tiles > 128) ns = 7;            // (longer keys and just too many row tiles for eight: waves by themselves)
+    else ns = std::min((ns + 3) / 4 * 4, 1024 / tiles / 4 * 4);
+  }
   if (ns < 2) return HX_OK;
   *n_splits = (int32_t)ns;
   *ws_floats = tiles * ns * 16 * ((a.vdim + 15) / 16 * 16 + 2);

@@ -72,6 +72,14 @@ def test_step_form(batch, H, G, D, V, mask, size, extra, divided):
     check([a for a, _ in batch], [b for _, b in batch], H, G, D, V, mask, size, extra, divided)
 
 
+# two and four runs of keys a workgroup, and two workgroups of four: runs without keys, rows that some of them do not see, partial row tiles
+@pytest.mark.parametrize("batch", [[(1, 140), (1, 1), (5, 64)], [(1, 250), (1, 3), (2, 33)], [(1, 511), (3, 40), (1, 129)], [(2, 600), (1, 65), (1, 1)]], ids=lambda b: f"{len(b)}x{max(b)}")
+@pytest.mark.parametrize("H, G, D, V", [(4, 1, 128, 128), (32, 8, 64, 64), (6, 2, 128, 64), (16, 16, 64, 128)])
+@pytest.mark.parametrize("mask, size, extra", [("causal", 0, "plain"), ("window", 300, "slopes"), ("chunk", 257, "cap"), ("causal", 0, "temperatures and sinks")])
+def test_step_form_merged_in_place(batch, H, G, D, V, mask, size, extra):
+    check([a for a, _ in batch], [b for _, b in batch], H, G, D, V, mask, size, extra)
+
+
 # Rows that no token of a portion sees are never read: pages left of a window or chunk may have been given back, and the rows of the last
 # page behind the last token hold anything.
 @pytest.mark.parametrize("batch", [[(64, 700), (33, 1100)], [(129, 333)], [(1, 700), (3, 1101), (1, 40)], [(16, 2005)]], ids=lambda b: f"{len(b)}x{max(b)}")
