@@ -1370,14 +1370,14 @@ int prepare_lds(const void* kernel, size_t lds) {
 // and the keys of a row tile dealt to `splits` workgroups where there are few of them.
 struct WidePlan {
   bool fits, rows32;
-  int splits;
+  int splits, groups;
 };
 // keys that a portion looks at, at most
 int key_reach(const hxm_latent_attn_args& a) {
   return a.window > 0 && a.window + a.max_q_len < a.max_kv_len ? a.window + a.max_q_len : a.max_kv_len;
 }
 WidePlan wide_plan(const hxm_latent_attn_args& a) {
-  WidePlan p{false, false, 1};
+  WidePlan p{false, false, 1, 1};
   if (a.kv_rank % 64 || a.block_size % 16 || a.out_token_stride % 8 || a.out_head_stride % 8 || !aligned16(a.out) || !aligned16(a.ws_o) ||
       a.cache_row_stride >= (1 << 26) || hxm::tile_form() != 1)
     return p;
@@ -1399,23 +1399,30 @@ WidePlan wide_plan(const hxm_latent_attn_args& a) {
   while (want > 1 && want * want * a.n_seq * rows > (int64_t)72 * reach) --want;
   if (want > reach / 64) want = reach / 64;      // (two tiles of 32 keys a split at least)
   if (want > 64) want = 64;
-  if (want > 1) p.splits = (int)want;
+  // One workgroup a compute unit leaves a SIMD one wave: two groups of waves share the keys, from seven tiles of them on (us, one group and two, 32 heads
+  // on portions of 100 - 200 tokens: 50 keys of 256 columns 9.7 10.7, 195 of 320 17.5 17.4, 283 of 128 12.9 11.9, 450 of 256 25.2 21.9, 554 of 256 28.4 23.5; up to
+  // 128 columns a compute unit takes two such workgroups: 16 heads on 198 and 845 tokens of 128 columns, 271 workgroups, 26.1 21.1), and in the place of two
+  // or three splits, whose merge is a launch (one portion, 16 heads: 302 tokens of 320 columns 25.3 18.9, 922 of 128 29.3 22.2; eight heads on 948 of 320 32.9
+  // 25.7; on 36 and 277 behind 334 of 256 22.5 23.4; as half of more splits no gain: 33 tokens behind 323 of 128, 32 heads, 11.6 13.0).  More than 320 columns
+  // are more than a second group's sums leave registers for.
+  const bool narrow = a.kv_rank <= 320;
+  if (want > 3 || !narrow) {
+    p.splits = (int)want;
+  } else if (want > 1 || (reach >= 224 && (int64_t)a.n_tokens * a.n_heads <= 64 * (a.kv_rank <= 128 ? 512 : 256))) {
+    p.groups = 2;
+  }
   return p;
 }
 
 template <int KK>
-int launch_wide16(const hxm_latent_attn_args& a, hipStream_t s) {
+int launch_wide16(const hxm_latent_attn_args& a, int groups, hipStream_t s) {
   const int n_splits = a.n_splits > 1 ? a.n_splits : 1, tiles16 = (int)(((int64_t)a.max_q_len * a.n_heads + 15) / 16);
   const int64_t grid = (((int64_t)a.n_tokens * a.n_heads + 63) / 64 + a.n_seq) * n_splits;      // row tiles of all sequences, at most
   if (grid > 0x7fffffff) return HX_ERR_SHAPE;
   constexpr size_t images = 2 * 32 * 2 * 64 * KK;          // (of a group of waves)
   // (few rows: where the tile form would deal out the keys)
   const bool fine = n_splits > 1 || (int64_t)a.n_seq * tiles16 < kTileWaves;
-  // One workgroup a compute unit leaves a SIMD one wave: two groups of waves share the keys, from seven tiles of them on (us, one group and two, 32 heads
-  // on portions of 100 - 200 tokens: 50 keys of 256 columns 9.7 10.7, 195 of 320 17.5 17.4, 283 of 128 12.9 11.9, 450 of 256 25.2 21.9, 554 of 256 28.4 23.5; up to
-  // 128 columns a compute unit takes two such workgroups: 16 heads on 198 and 845 tokens of 128 columns, 271 workgroups, 26.1 21.1).  More
-  // than 320 columns are more than a second group's sums leave registers for, and what is dealt to workgroups already gains nothing.
-  const bool two = KK <= 5 && n_splits == 1 && fine && grid - a.n_seq <= (KK <= 2 ? 512 : 256) && key_reach(a) >= 224;
+  const bool two = KK <= 5 && fine && groups == 2;
   const size_t lds = two ? 2 * images + 4096 : images;
   auto kernel = fine ? latent_attn_wide16_kernel<KK, true, 1> : latent_attn_wide16_kernel<KK, false, 1>;
   if constexpr (KK <= 5) {
@@ -1445,7 +1452,7 @@ int launch_wide(const hxm_latent_attn_args& a, const WidePlan& p, hipStream_t s)
       return hxm::check_launch();
     }
   }
-  return hxm::latent_step_serves(a) ? hxm::launch_latent_step(a, s) : launch_wide16<KK>(a, s);
+  return hxm::latent_step_serves(a) ? hxm::launch_latent_step(a, s) : launch_wide16<KK>(a, p.groups, s);
 }
 
 // the splits of a (sequence, row tile) merged: out = sum_s O_s e^(m_s - M) / sum_s l_s e^(m_s - M), times the head gate
