@@ -1000,15 +1000,17 @@ int launch_wide(const hxm_biased_attn_args& a, hipStream_t s) {
   const bool mods = a.slopes || a.softcap > 0.f;
   // few rows: fewer tiles of 16 than the waves that the tile form's keys are dealt to (see its callers)
   const bool fine = (int64_t)a.n_seq * a.kv_heads * (((int64_t)a.max_q_len * R + 15) / 16) < 2048;
-  // Such a launch gives a compute unit one workgroup: two groups of waves share its keys, so that a SIMD has two waves.  Portions of up to a
-  // tile's keys have nothing to share (us, one group and two: 4 of 20 - 52 tokens, cap and slopes 10.6 11.6; one of 128 - 152, 10.4 10.6; 2 of 81 - 217
-  // 18.1 16.2, 1082 behind 463 41.8 33.4, 110 behind 495 25.5 19.7; 40 launches drawn from these ranges 1 and 0.94).
-  const int groups = fine && a.max_q_len > 64 ? 2 : 1;
-  auto kernel = groups == 2 ? (mods ? biased_attn_wide_kernel<D, V, true, true, 2> : biased_attn_wide_kernel<D, V, false, true, 2>)
-                : fine      ? (mods ? biased_attn_wide_kernel<D, V, true, true, 1> : biased_attn_wide_kernel<D, V, false, true, 1>)
-                            : (mods ? biased_attn_wide_kernel<D, V, true, false, 1> : biased_attn_wide_kernel<D, V, false, false, 1>);
+  // A workgroup a compute unit: two groups of waves share its keys, so that a SIMD has two waves.  Portions of up to a tile's keys have nothing to
+  // share (us, one group and two: 4 of 20 - 52 tokens, cap and slopes 10.6 11.6; one of 128 - 152, 10.4 10.6; 2 of 81 - 217 18.1 16.2, 1082 behind 463 41.8
+  // 33.4, 110 behind 495 25.5 19.7; by the number of workgroups 140 - 256 3 - 25 % faster, 272 20.5 28.4 under a short window, 280 37.1 28.9, 320 18.8 28.1 and 28.4
+  // 28.6, 600 - 1000 12 - 25 % slower).
+  const bool two = a.max_q_len > 64 && (fine || ((int64_t)a.n_tokens * R / 64 + a.n_seq) * a.kv_heads / 2 <= 256);
+  auto kernel = two ? (fine ? (mods ? biased_attn_wide_kernel<D, V, true, true, 2> : biased_attn_wide_kernel<D, V, false, true, 2>)
+                            : (mods ? biased_attn_wide_kernel<D, V, true, false, 2> : biased_attn_wide_kernel<D, V, false, false, 2>))
+                    : (fine ? (mods ? biased_attn_wide_kernel<D, V, true, true, 1> : biased_attn_wide_kernel<D, V, false, true, 1>)
+                            : (mods ? biased_attn_wide_kernel<D, V, true, false, 1> : biased_attn_wide_kernel<D, V, false, false, 1>));
   constexpr size_t images = 2 * 64 * (2 * D + 2 * V), part = 4 * (V / 2 + 4) * 256;      // (of a group of waves; what the groups hand over, in the place of the second one's images)
-  const size_t lds = groups == 2 ? images + std::max(images, part) : images;
+  const size_t lds = two ? images + std::max(images, part) : images;
   if (lds > 48 * 1024) {
     const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) {
@@ -1016,7 +1018,7 @@ int launch_wide(const hxm_biased_attn_args& a, hipStream_t s) {
       return HX_ERR_HIP;
     }
   }
-  kernel<<<dim3((unsigned)grid), dim3(256 * groups), lds, s>>>(a, (int)slots);
+  kernel<<<dim3((unsigned)grid), dim3(two ? 512 : 256), lds, s>>>(a, (int)slots);
   return hxm::check_launch();
 }
 

@@ -51,6 +51,13 @@ def test_wide_form(batch, H, G, D, V, mask, size, extra):
     check(new, kv, H, G, D, V, mask, size, extra)
 
 
+# the same among portions so uneven that the longest one speaks for more row tiles than there are
+@pytest.mark.parametrize("H, G, D, V", [(32, 8, 64, 64), (32, 32, 128, 128), (32, 16, 64, 128)])
+@pytest.mark.parametrize("mask, size, extra", [("causal", 0, "plain"), ("window", 200, "slopes"), ("chunk", 130, "temperatures and sinks")])
+def test_two_groups_of_waves_among_uneven_portions(H, G, D, V, mask, size, extra):
+    check([601, 20, 33, 7], [601, 90, 33, 300], H, G, D, V, mask, size, extra)
+
+
 # keys shared by two groups of waves: one tile, two, three, an odd and an even number of them, tiles that only one group's rows or neither's see
 @pytest.mark.parametrize("batch", [[(65, 65)], [(66, 128)], [(100, 129)], [(70, 257), (200, 200), (1, 64)], [(129, 705)]], ids=lambda b: f"{len(b)}x{max(b)}")
 @pytest.mark.parametrize("H, G, D, V", [(4, 1, 128, 128), (8, 8, 64, 64), (6, 2, 128, 64), (4, 4, 64, 128)])
