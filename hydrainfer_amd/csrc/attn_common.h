@@ -21,13 +21,6 @@ template <> struct Mfma<BF16> {
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// sum + both numbers of pair i of eight weights in bfloat16: the sum of what the products take, one instruction for two of them
-__device__ __forceinline__ float add_weights(float sum, u16x8 w, int i) {
-  typedef __bf16 pair_t __attribute__((ext_vector_type(2)));
-  typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(pair_t, (unsigned)__builtin_bit_cast(u32x4_t, w)[i]), __builtin_bit_cast(pair_t, 0x3f803f80u), sum, false);
-}
-
 // ds_read_b64_tr_b16: lane (g = l>>4, c = l&15) of a [16 rows][16 cols] 2-byte tile whose rows
 // start at lds_ptr(row-group base) receives column-major data suitable as an MFMA A operand of
 // the transposed tile (see attn_fwd.hip for the addressing used with it).

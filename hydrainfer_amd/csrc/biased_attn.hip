@@ -633,20 +633,17 @@ __global__ __launch_bounds__(256) void biased_attn_group_kernel(hxm_biased_attn_
 //   * a tile's key and value rows go straight from the paged cache to LDS (1 KiB an instruction, whole rows), the next tile's
 //     while this one is worked on: two images, one barrier a tile.  Rows cannot be padded this way; their 16-byte chunks are
 //     swizzled by the lane that asks for them (keys: chunk ^ row, values: 64-byte quarter ^ row);
-//   * a row's weights refer to its largest score so far, which costs a pass over the accumulators for nearly every new one: 32 keys at a
-//     time through the first two tiles, 64 behind them.  Left up to 2^8 behind, results were off by 3 % more, as the largest weights
-//     were rounded to bfloat16 instead of being 1;
-//   * the weights' sum is that of the rounded ones, which the values meet: results are off by less for it, and an instruction adds two.
-// Measured, the two last points: 55.4 us before, 54.3 now, 2-norm of the error against 64 bits 2.057e-3 and 2.043e-3 (all tiles whole 54.2, but
-// portions of 64 keys off by 1 % more; half tiles as before, sums of the weights as they were before rounding: 53.7 with whole tiles
-// behind the first two, off by 0.05 % more).
+//   * a row's weights refer to its largest score so far, 32 keys at a time, and their sum is that of the floats.  That costs a pass over the
+//     accumulators for nearly every half tile; left up to 2^8 behind, it took 5 us less and results were off by 3 % more, as the largest
+//     weights were rounded to bfloat16 instead of being 1.  (64 keys at a time behind a workgroup's first two tiles, and sums of the rounded
+//     weights: 1 us less, and off by more where all of a row's keys lie in such tiles, as behind the edge of a chunk.)
 //   * where workgroups are few, two groups of four waves take every other tile of keys each, with images of their own, and add up what they have at
 //     the end: each hands the other half of its columns through LDS, scaled like the splits of a row (a wave alone on its SIMD goes from products
 //     to softmax to products, 2 - 3 us a tile).
 // The order of the row tiles: the XCDs (workgroups are dealt round robin) take key heads of their own where there are enough of
 // them, and of every sequence the tiles with the most keys come first.
-// Measured, 4 portions of 797 - 1151 tokens, 32 heads of 128 on 8 key heads, sinks: 221 us in the group form, 54 us
-// here (600 TFLOP/s of the pairs that a mask leaves); window of 512 and soft cap 223 and 68 us; chunks of 512 and slopes 163 and
+// Measured, 4 portions of 797 - 1151 tokens, 32 heads of 128 on 8 key heads, sinks: 221 us in the group form, 55 us
+// here (580 TFLOP/s of the pairs that a mask leaves); window of 512 and soft cap 223 and 68 us; chunks of 512 and slopes 163 and
 // 50 us.  Down to 64 rows of a key head it is the faster one (16 tokens behind 500 keys: 30 and 21 us).
 // ---------------------------------------------------------------------------------------------------------------
 template <int D, int V, bool MODS, bool FINE, int KG>      // MODS: slopes or a soft cap; FINE: every 32 keys' weights refer to their own largest score; KG: groups of four waves
@@ -843,8 +840,7 @@ __global__ __launch_bounds__(256 * KG, 2) void biased_attn_wide_kernel(hxm_biase
           if (k > last || k < first) s[u][e] = -INFINITY;
         }
     }
-    // The weights refer to the largest score so far: its own is then 1, which no rounding to bfloat16 touches.  Half a tile at a time in the first
-    // two tiles, where most largest scores are met, a whole tile at a time behind them: one pass over the accumulators less.  In
+    // The weights refer to the largest score so far, half a tile at a time: its own is then 1, which no rounding to bfloat16 touches.  In
     // launches of few rows (FINE) they refer to the largest of these 32 keys, and what they add is scaled behind the products: the tile
     // form deals such a launch's keys to more waves, each with a largest score that weighs exactly 1.
     float m_ref[2] = {HX_NEG_BIG, HX_NEG_BIG}, m_new[2];
@@ -855,23 +851,20 @@ __global__ __launch_bounds__(256 * KG, 2) void biased_attn_wide_kernel(hxm_biase
       m_ref[u] = halves_max(m_ref[u]) * unit;
       asm("" : "+v"(m_ref[u]));              // (rounded: left inside a difference below it would not be m_new's number)
       m_new[u] = fmaxf(u ? m_new[0] : m, m_ref[u]);
-    }
-    if constexpr (!FINE) {
-      if (t >= t_first + 2) m_new[0] = m_new[1];
-      m_ref[0] = m_new[0];
-      m_ref[1] = m_new[1];
+      if (!FINE) m_ref[u] = m_new[u];
     }
     u16x8 pf[2][2];
     float ps[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) pf[u][e >> 3][e & 7] = BF16::from_float(fast_exp2(__builtin_fmaf(s[u][e], unit, -m_ref[u])));
       float pa = 0.f, pb = 0.f;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        pa = add_weights(pa, pf[u][0], i);
-        pb = add_weights(pb, pf[u][1], i);
+      for (int e = 0; e < 16; e += 2) {
+        const float e0 = fast_exp2(__builtin_fmaf(s[u][e], unit, -m_ref[u])), e1 = fast_exp2(__builtin_fmaf(s[u][e + 1], unit, -m_ref[u]));
+        pa += e0;
+        pb += e1;
+        pf[u][e >> 3][e & 7] = BF16::from_float(e0);
+        pf[u][e >> 3][(e & 7) + 1] = BF16::from_float(e1);
       }
       ps[u] = pa + pb;
     }

@@ -236,6 +236,37 @@ def test_weights_round_no_more_than_in_the_tile_form(n, new, kv, extra):
     assert off["auto"] <= (1.0 if new == 1 else 1.005) * off["tile"], off
 
 
+# What a row adds up: a key weighs 1 and others w, halfway between two bfloat16 numbers, and everything else nothing.  "sum": 31 of them in the
+# 32 keys of the one with a value, whose share 1 / (1 + 31 w) shows a denominator of rounded weights (off by up to 2^-8); "share": one of them, with the
+# value, in the 32 keys in front, where it is the largest score so far: w / (1 + w), and no rounding of w.  So the result's rounding is all there is.
+@pytest.mark.parametrize("what", ["sum", "share"])
+@pytest.mark.parametrize("n", [1, 16], ids=["few", "many"])
+@pytest.mark.parametrize("D, V", [(64, 64), (128, 128)])
+def test_weights_that_no_bfloat16_holds(what, n, D, V):
+    from hydrainfer_amd._C.kernel.biased_attn import biased_attention
+    H, kv = 8, 256
+    i = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    w = torch.tensor([(0.5 if what == "sum" else 2.0 ** -4) * (1 + (2 * h + 1) * 2.0 ** -8) for h in range(H)], dtype=torch.float64)
+    temps = -torch.log(w).float()
+    k, v, q = torch.zeros((kv, D)), torch.zeros((kv, V)), torch.zeros((n * kv, H, D))
+    q[:, :, 0] = 1
+    k[:, 0] = -1000
+    if what == "sum":
+        k[192:224, 0], k[200, 0], v[200] = -1, 0, 1
+        want = 1 / (1 + 31 * w)
+    else:
+        k[197, 0], k[229, 0], v[197] = -1, 0, 1
+        want = w / (1 + w)
+    pages = lambda x: x.bfloat16()[:, None].expand(-1, H, -1).contiguous().view(kv // BLOCK, BLOCK, H, -1).repeat(n, 1, 1, 1).cuda()
+    out = biased_attention(q.bfloat16().cuda(), pages(k), pages(v), V, i([s for s in range(n) for _ in range(kv)]), i(list(range(kv)) * n), i([kv * s for s in range(n + 1)]),
+                           i(list(range(n * kv // BLOCK))), i([kv // BLOCK * s for s in range(n + 1)]), 1.0, None, "causal", 0, max_q_len=kv, max_kv_len=kv,
+                           head_scale=temps.cuda()).view(n, kv, H, V)[:, 230:].double().cpu()
+    # half of a last place of bfloat16, and 1e-5 for the float arithmetic (an exponential of scores up to 3)
+    bound = 2.0 ** (torch.floor(torch.log2(want)) - 8) + 1e-5 * want
+    off = (out - want[:, None]).abs().amax(dim=(0, 1, 3))
+    assert bool((off <= bound).all()), (off / bound).tolist()
+
+
 # Rows of a group of sixteen are addressed by offsets of 32 bits up to a stride of 2 ** 26 elements (16 rows, in bytes), by pointers past
 # it and in groups that reach past the keys that are seen: the same bytes, so the same result to the last bit.
 @pytest.mark.parametrize("stride", [2 ** 26 - 8, 2 ** 26], ids=["near", "far"])
