@@ -1400,16 +1400,22 @@ WidePlan wide_plan(const hxm_latent_attn_args& a) {
   if (want > reach / 64) want = reach / 64;      // (two tiles of 32 keys a split at least)
   if (want > 64) want = 64;
   // One workgroup a compute unit leaves a SIMD one wave: two groups of waves share the keys, from seven tiles of them on (us, one group and two, 32 heads
-  // on portions of 100 - 200 tokens: 50 keys of 256 columns 9.7 10.7, 195 of 320 17.5 17.4, 283 of 128 12.9 11.9, 450 of 256 25.2 21.9, 554 of 256 28.4 23.5; up to
-  // 128 columns a compute unit takes two such workgroups: 16 heads on 198 and 845 tokens of 128 columns, 271 workgroups, 26.1 21.1), and in the place of two
-  // or three splits, whose merge is a launch (one portion, 16 heads: 302 tokens of 320 columns 25.3 18.9, 922 of 128 29.3 22.2; eight heads on 948 of 320 32.9
-  // 25.7; on 36 and 277 behind 334 of 256 22.5 23.4; as half of more splits no gain: 33 tokens behind 323 of 128, 32 heads, 11.6 13.0).  More than 320 columns
-  // are more than a second group's sums leave registers for.
-  const bool narrow = a.kv_rank <= 320;
-  if (want > 3 || !narrow) {
-    p.splits = (int)want;
-  } else if (want > 1 || (reach >= 224 && (int64_t)a.n_tokens * a.n_heads <= 64 * (a.kv_rank <= 128 ? 512 : 256))) {
+  // on portions of 100 - 200 tokens: 50 keys of 256 columns 9.7 10.7, 195 of 320 17.5 17.4, 283 of 128 12.9 11.9, 450 of 256 25.2 21.9, 554 of 256 28.4 23.5) and in
+  // the place of two splits, whose merge is a launch (one portion, 16 heads: 302 tokens of 320 columns 25.3 18.9, 922 of 128 29.3 22.2).  Three splits walk a third
+  // of the keys each: two groups are faster only where the keys that a row sees, in the mean, are few: up to 500 in portions that bring a tenth of them and more
+  // (eight heads on 948 tokens of 320 columns 32.9 25.7), 300 in shorter ones, where narrow rows are all that a split has to hand on (of 548 batches 5 %
+  // in the mean, 26 slower by 2 - 8 %; behind the line, six portions of 28 tokens behind 1200, 256 columns, 27.7 35.7).  A compute unit takes one such
+  // workgroup, so all of them have to be there at once: 320 portions of two tokens behind 520 keys, 256 columns, 24.7 33.1.  Up to 128 columns it takes two, and
+  // from 400 keys on that is faster than one group each (16 heads on 198 and 845 tokens of 128 columns, 271 workgroups, 26.1 21.1; 250 keys 2 % slower).
+  // More than 320 columns are more than a second group's sums leave registers for.
+  const int64_t row_tiles = (int64_t)a.n_tokens * a.n_heads / 64 + a.n_seq;      // at most
+  const bool narrow = a.kv_rank <= 320, at_once = row_tiles <= 256 || (a.kv_rank <= 128 && row_tiles <= 512 && reach >= 400);
+  const int seen = reach - a.max_q_len / 2;      // in the mean
+  const bool as_three = 10 * (int64_t)a.max_q_len >= reach ? seen <= 500 : a.kv_rank <= 192 && seen <= 300;
+  if (narrow && at_once && (want < 2 ? reach >= 224 : want == 2 || (want == 3 && as_three))) {
     p.groups = 2;
+  } else if (want > 1) {
+    p.splits = (int)want;
   }
   return p;
 }

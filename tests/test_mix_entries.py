@@ -64,3 +64,26 @@ def test_no_call_with_a_launch_ahead_is_taken_for_a_short_one():
                 asked += 1
     assert asked > 1000
     assert not long_chains(3, 3, 16, 64, 1) and not long_chains(300, 4, 32, 128) and not long_chains(100, 1, 64, 128, 100) and not long_chains(0, 0, 8, 64)
+
+
+def _latent_splits(lens, kv, heads, rank, window=0):
+    from hydrainfer_amd import _lib
+    HX_BF16 = _lib._DTYPE[__import__("torch").bfloat16]
+    a = _lib.hxm_latent_attn_args(q_token_stride=heads * rank, q_head_stride=rank, out_token_stride=heads * rank, out_head_stride=rank, cache_block_stride=16 * rank,
+                                  cache_row_stride=rank, n_tokens=sum(lens), n_seq=len(lens), n_heads=heads, kv_rank=rank, block_size=16, window=window,
+                                  max_q_len=max(lens), scale=1.0, dtype=HX_BF16, max_kv_len=kv)
+    n, floats = ctypes.c_int32(), ctypes.c_int64()
+    assert _lib.mix_lib().hxm_latent_attention_plan(ctypes.byref(a), ctypes.byref(n), ctypes.byref(floats)) == 0
+    assert floats.value == (0 if n.value == 1 else len(lens) * ((max(lens) * heads + 15) // 16) * n.value * 16 * (rank + 2))
+    return n.value
+
+
+@pytest.mark.parametrize("lens, kv, heads, rank, splits", [
+    # two groups of waves in the place of two splits, and of three where the keys that a row sees are few: no workspace
+    ([302], 302, 16, 320, 1), ([922], 922, 16, 128, 1), ([948], 948, 8, 320, 1), ([100, 64], 500, 16, 256, 1), ([5] * 8, 250, 32, 64, 1),
+    # three splits of more keys or wider rows (us in three and by two groups, the second and third: 46.6 58, 31.6 40.7)
+    ([28] * 6, 1128, 32, 256, 3), ([3] * 96, 1771, 32, 320, 3), ([1] * 192, 2047, 33, 128, 3), ([25, 9, 11, 20], 694, 40, 64, 3), ([5] * 8, 250, 32, 256, 3),
+    # more row tiles than can be there at once (24.7 33.1, 68.2 90, 82 103)
+    ([2] * 320, 522, 8, 256, 2), ([1] * 320, 1500, 33, 256, 2), ([116] * 24, 2172, 8, 192, 2)])
+def test_splits_of_latent_portions(lens, kv, heads, rank, splits):
+    assert _latent_splits(lens, kv, heads, rank) == splits
