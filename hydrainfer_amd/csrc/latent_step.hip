@@ -336,7 +336,16 @@ int launch_heads(const hxm_latent_attn_args& a, hipStream_t s) {
 
 namespace hxm {
 
-bool latent_step_serves(const hxm_latent_attn_args& a) { return a.max_q_len == 1 && a.n_tokens <= a.n_seq && a.n_heads <= 32 && a.n_tokens < (1 << 24); }
+// Up to 2048 tiles of keys in all, 1365 for more than 16 heads and 64 tokens: behind that the compute units are full, and what counts is not the way to
+// the first tile but how many rows a byte from LDS feeds, which are more in the row tiles' form (us there and here, 32 heads: 192 tokens of 200 - 2047 keys, 128
+// columns 29.6 43.2, 320 columns 53 69; 512 under a window of 512, 320 columns 47 56; 64 of 1000 - 8000, 128 columns 37 46; in front of the line, 512 columns, 128 of
+// 26 - 300 27.7 19.7, 64 of 200 - 2047 41 35).  Of 2337 batches of 1 - 768 tokens behind 17 - 16000 keys 1370 lie in front of it: 0.78 of that form's time in the mean, 8 of them
+// 2 - 9 % more.
+bool latent_step_serves(const hxm_latent_attn_args& a) {
+  if (a.max_q_len != 1 || a.n_tokens > a.n_seq || a.n_heads > 32) return false;
+  const int reach = a.window > 0 && a.window < a.max_kv_len ? a.window + 1 : a.max_kv_len;
+  return (int64_t)a.n_tokens * ((std::max(reach, 1) + kTile - 1) / kTile) <= (a.n_heads <= 16 || a.n_tokens <= 64 ? 2048 : 1365);
+}
 
 // Splits of a token's keys: a launch lasts as long as its rounds of workgroups (256 of more than 256 columns at a time, 512 of fewer), a round
 // about 6 us and its tiles, the merge 3 us and what the splits hold.  Only splits of whole tiles are looked at: half a tile costs a whole one.

@@ -57,6 +57,13 @@ def test_single_tokens(kv, R, H, window, extra):
     check([1] * len(kv), kv, R, H, window, extra, WIDE32 if R <= 192 and len(kv) >= 256 else WIDE16)
 
 
+# more keys in all than the form of single tokens takes: row tiles again, in three splits and in two
+@pytest.mark.parametrize("kv", [[700] * 189 + [3], [450] * 299 + [64]], ids=lambda v: f"{len(v)}x{max(v)}")
+@pytest.mark.parametrize("R, H, window, extra", [(256, 17, 0, "plain"), (320, 8, 0, "sinks and gate"), (512, 32, 400, "plain")])
+def test_many_single_tokens(kv, R, H, window, extra):
+    check([1] * len(kv), kv, R, H, window, extra, WIDE16)
+
+
 # Rows that no token of a portion sees are never read: pages left of a window may have been given back, and the rows of the last page
 # behind the last token hold anything.
 @pytest.mark.parametrize("new, kv", [([1, 3, 1], [700, 1101, 40]), ([33, 20], [700, 90]), ([300, 41, 761], [700, 2005, 800])])

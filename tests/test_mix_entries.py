@@ -87,3 +87,10 @@ def _latent_splits(lens, kv, heads, rank, window=0):
     ([2] * 320, 522, 8, 256, 2), ([1] * 320, 1500, 33, 256, 2), ([116] * 24, 2172, 8, 192, 2)])
 def test_splits_of_latent_portions(lens, kv, heads, rank, splits):
     assert _latent_splits(lens, kv, heads, rank) == splits
+@pytest.mark.parametrize("tokens, kv, heads, rank, window, splits", [
+    # a token's keys shared by the waves of a workgroup: up to 2048 tiles of 64 keys in all, 1365 for more than 16 heads and 64 tokens
+    (1, 149, 32, 512, 0, 3), (32, 1747, 32, 512, 512, 5), (64, 2047, 32, 512, 0, 4), (64, 2047, 32, 128, 0, 8), (128, 300, 32, 512, 0, 1), (300, 300, 16, 512, 0, 1),
+    # row tiles of 64 rows, as many splits as before there was the other form (us there and in it: 29.6 43.2, 53 69, 44 59, 33.8 37.3, 61 66)
+    (192, 2047, 32, 128, 0, 3), (192, 2047, 32, 320, 0, 3), (192, 2047, 8, 320, 0, 3), (128, 2047, 8, 320, 0, 4), (160, 2047, 32, 320, 0, 4), (64, 8000, 32, 128, 0, 8)])
+def test_splits_of_single_latent_tokens(tokens, kv, heads, rank, window, splits):
+    assert _latent_splits([1] * tokens, kv, heads, rank, window) == splits
