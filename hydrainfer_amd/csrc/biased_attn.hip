@@ -995,9 +995,12 @@ int launch_wide(const hxm_biased_attn_args& a, hipStream_t s) {
   const bool fine = (int64_t)a.n_seq * a.kv_heads * (((int64_t)a.max_q_len * R + 15) / 16) < 2048;
   // A workgroup a compute unit: two groups of waves share its keys, so that a SIMD has two waves.  Portions of up to a tile's keys have nothing to
   // share (us, one group and two: 4 of 20 - 52 tokens, cap and slopes 10.6 11.6; one of 128 - 152, 10.4 10.6; 2 of 81 - 217 18.1 16.2, 1082 behind 463 41.8
-  // 33.4, 110 behind 495 25.5 19.7; by the number of workgroups 140 - 256 3 - 25 % faster, 272 20.5 28.4 under a short window, 280 37.1 28.9, 320 18.8 28.1 and 28.4
-  // 28.6, 600 - 1000 12 - 25 % slower).
-  const bool two = a.max_q_len > 64 && (fine || ((int64_t)a.n_tokens * R / 64 + a.n_seq) * a.kv_heads / 2 <= 256);
+  // 33.4, 110 behind 495 25.5 19.7; by the number of workgroups 140 - 256 3 - 25 % faster, 272 20.5 28.4 under a short window, 280 37.1 28.9, 288, of 24 portions
+  // of 78, 16.6 22.5, 320 18.8 28.1 and 28.4 28.6, 600 - 1000 12 - 25 % slower).  The portions' last row tiles are half full in the mean; equal portions are
+  // counted as they are (12 of 67 tokens in 288 workgroups 10.3 12.9).
+  int64_t workgroups = ((int64_t)a.n_tokens * R / 64 + a.n_seq) * a.kv_heads / 2;
+  if (a.n_tokens == (int64_t)a.n_seq * a.max_q_len) workgroups = std::max(workgroups, a.n_seq * (((int64_t)a.max_q_len * R + 127) / 128) * a.kv_heads);
+  const bool two = a.max_q_len > 64 && workgroups <= 256;
   auto kernel = two ? (fine ? (mods ? biased_attn_wide_kernel<D, V, true, true, 2> : biased_attn_wide_kernel<D, V, false, true, 2>)
                             : (mods ? biased_attn_wide_kernel<D, V, true, false, 2> : biased_attn_wide_kernel<D, V, false, false, 2>))
                     : (fine ? (mods ? biased_attn_wide_kernel<D, V, true, true, 1> : biased_attn_wide_kernel<D, V, false, true, 1>)

@@ -58,6 +58,13 @@ def test_two_groups_of_waves_among_uneven_portions(H, G, D, V, mask, size, extra
     check([601, 20, 33, 7], [601, 90, 33, 300], H, G, D, V, mask, size, extra)
 
 
+# equal portions in as many workgroups as there are compute units, and in a few more, which one group of waves each takes
+@pytest.mark.parametrize("batch", [[(65, 70)] * 16, [(65, 70)] * 17], ids=lambda b: f"{len(b)}x{max(b)}")
+@pytest.mark.parametrize("H, G, D, V, mask, size", [(16, 16, 64, 64, "causal", 0), (32, 16, 128, 128, "window", 66)])
+def test_groups_of_waves_by_the_number_of_workgroups(batch, H, G, D, V, mask, size):
+    check([a for a, _ in batch], [b for _, b in batch], H, G, D, V, mask, size, "plain")
+
+
 # keys shared by two groups of waves: one tile, two, three, an odd and an even number of them, tiles that only one group's rows or neither's see
 @pytest.mark.parametrize("batch", [[(65, 65)], [(66, 128)], [(100, 129)], [(70, 257), (200, 200), (1, 64)], [(129, 705)]], ids=lambda b: f"{len(b)}x{max(b)}")
 @pytest.mark.parametrize("H, G, D, V", [(4, 1, 128, 128), (8, 8, 64, 64), (6, 2, 128, 64), (4, 4, 64, 128)])
