@@ -254,7 +254,7 @@ __global__ __launch_bounds__(512) void chunk_head32_kernel(ChunkScanArgs a) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float in = within[u][e], more = u ? across[e] : 0.f;
-          if constexpr (DELTA && NP == 3) {
+          if constexpr (NP == 3) {                        // (the delta rule)
             const float before = sum[u][0][e] + sum[u][1][e];
             result[u][e] = __builtin_fmaf(before, pre[u][e], __builtin_fmaf(before, rest[u][e], in + more));
           } else {                                        // (in double: the operands' products are exact, and a rounding here shows.  3 % of the time)
@@ -575,14 +575,15 @@ int launch(const ChunkScanArgs& a, hipStream_t s) {
   return launch_chunks(chunk_head32_kernel<KP, DELTA, QK, VT, VEC>, dim3((unsigned)a.heads, (unsigned)((a.V + VW - 1) / VW), (unsigned)a.n_seq), 512,
                        HeadImage<KP, QK, DELTA>::kLds, a, s);
 }
+// (what chunk_scan.hip sends here: the delta rule with more than 64 key channels, and the decayed sum of bfloat16 q and k)
 template <int KP, typename QK, typename VT, bool VEC>
 int launch_form(const ChunkScanArgs& a, hipStream_t s) {
-  if constexpr (KP == 128) {
-    if (a.form == hxm::kChunkDelta) return launch<KP, true, QK, VT, VEC>(a, s);
+  if (a.form == hxm::kChunkDelta) {
+    if constexpr (KP == 128) return launch<KP, true, QK, VT, VEC>(a, s);
   } else {
-    if (a.form == hxm::kChunkDelta) return HX_ERR_UNSUPPORTED;
+    if constexpr (QK::kDtype == HX_BF16) return launch<KP, false, QK, VT, VEC>(a, s);
   }
-  return launch<KP, false, QK, VT, VEC>(a, s);
+  return HX_ERR_UNSUPPORTED;
 }
 template <typename QK, typename VT>
 int launch_width(const ChunkScanArgs& a, hipStream_t s) {

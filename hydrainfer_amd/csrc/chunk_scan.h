@@ -34,6 +34,6 @@ bool chunk_scan_fits(const ChunkScanArgs& a);
 int64_t chunk_scan_workspace(const ChunkScanArgs& a);
 int chunk_scan(const ChunkScanArgs& a, hipStream_t s);
 int chunk_chain(const ChunkScanArgs& a, hipStream_t s);      // with a.made
-int chunk_head(const ChunkScanArgs& a, hipStream_t s);       // one decay per token and head, without it; delta rule: more than 64 key channels
+int chunk_head(const ChunkScanArgs& a, hipStream_t s);       // one decay per token and head, without it: the delta rule with more than 64 key channels, the decayed sum of bfloat16 q and k
 
 }  // namespace hxm

@@ -14,26 +14,32 @@
 // its registers.  Producer waves work one chunk ahead (A, M, prefixes, suffixes) and bring rows in two chunks ahead, requested
 // three chunks before that from clamped addresses; one workgroup barrier a chunk.  The workgroups of a sequence stand next to
 // each other: a long portion among short ones is spread over all XCDs (dealt round robin).
-//   per head:    chunk_head.hip, thirty-two tokens at a time; here (chunk_delta_kernel) the delta rule with up to 64 key channels — Q K^T and K K^T
-//                on the matrix cores, decays as factors of the accumulators' rows.
+//   per head:    chunk_head_kernel — Q K^T and K K^T on the matrix cores, decays as factors of the accumulators' rows.  (Thirty-two tokens at
+//                a time, in bfloat16 parts, where that is faster: chunk_head.hip.)
 //   per channel: chunk_channel_kernel — A by running products over the tokens on the vector ALU, a lane one or two key channels,
 //                summed over the wave by a transposing butterfly that leaves one element of A in every second lane.
-// What bounds it now: the chunks of a sequence follow each other.  Measured against one token at a time, 4 portions of 797 -
-// 1151 tokens: bonus form, 32 heads of 64 x 64, 207 -> 105 us; gated form, 32 heads of 128 x 128, 720 -> 205 us with its norm (171 in the two launches of chunk_chain.hip, which
+// What bounds it now: the chunks of a sequence follow each other (2.5 us each with states of 128 x 128; 1.8 us of float matrix
+// products on the SIMDs that hold a consumer and a maker of A or M).  Measured against one token at a time, 4 portions of 797 -
+// 1151 tokens: delta rule, 32 heads of 128 x 128, 479 -> 189 us; bonus form, 32 heads of 64 x 64, 207 -> 105 us; gated form, 32 heads of 128 x 128, 720 -> 205 us with its norm (171 in the two launches of chunk_chain.hip, which
 // batches of few chains for their length take).
 // What the rounding costs: a token at a time rounds a state's element once a token, and each rounding decays with the state.  Here
 // the products of decays, of keys with them and the chunk's sums are rounded besides, and four things keep that from showing: sums
 // over tokens run from the first token to the last and on top of the decayed state (row_of_token); products of decays carry what
 // their roundings leave over (Product); sums over key channels are cut in eight or sixteen chains; and the bonus form, whose
 // k v is often exact, adds up within a chunk in double and keeps the rest of its suffixed keys.  Error against 64 bits (2-norm), a
-// token at a time and here, 3 portions of 200 - 600 tokens, 16 heads of 128 x 128 (64 x 64): results delta 64 x 64 1.00 1.00, bonus 0.90 0.82 (0.83 0.77) e-7; states delta 64 x 64 0.75 0.74, bonus 0.46 0.45 (0.47 0.45), gated 1.42 1.09 (1.41 1.08) e-7.
+// token at a time and here, 3 portions of 200 - 600 tokens, 16 heads of 128 x 128 (64 x 64): results delta 1.07 1.07 (1.00 1.00),
+// decay 1.04 0.84 (0.97 0.77), bonus 0.90 0.82 (0.83 0.77) e-7; states delta 0.74 0.73 (0.75 0.74), decay 0.68 0.62 (0.72
+// 0.66), bonus 0.46 0.45 (0.47 0.45), gated 1.42 1.09 (1.41 1.08) e-7.
+#include <cmath>
+
 #include "chunk_parts.h"
 
 namespace {
 
 // (for the scheduler) FIRST reads from LDS, then a read behind every PER products, N times, then REST products: left alone it
 // asks for two rows and waits for them after every eight products.  Tuned by measuring, 4 portions of 797 - 1151 tokens and 32 heads:
-// delta rule 64 x 64 126 us without, 122 here; bonus form 64 x 64 115 and 105.  The gated form, bound by its producers, gains nothing.
+// delta rule 128 x 128 207 us without, 189 here (<6, 28, 2, 12> 200, <12, 22, 3, 3> 214), 64 x 64 126 and 122; bonus form 64 x 64
+// 115 and 105.  The gated form, bound by its producers, gains nothing.
 template <int FIRST, int N, int PER, int REST>
 __device__ __forceinline__ void products_behind_reads() {
   __builtin_amdgcn_sched_group_barrier(0x100, FIRST, 0);
@@ -46,13 +52,12 @@ __device__ __forceinline__ void products_behind_reads() {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// The delta rule with up to 64 key channels.  (Thirty-two tokens at a time, as chunk_head.hip does it with more: 16 portions of 60 tokens, 32 heads
-// of 64 x 64 22.1 us here and 24.1, 4 of 797 - 1151 124 and 122, 12 of 300 - 900 124 and 130.  There two workgroups do not share a compute unit.)
+// One decay per token and head.
 // ---------------------------------------------------------------------------------------------------------------
-template <typename QK, typename VT, bool VEC>
-__global__ __launch_bounds__(512) void chunk_delta_kernel(ChunkScanArgs a) {
-  constexpr int KP = 64, KT = KP / 16, RS = KP + 4;
-  constexpr int kRaw = 2 * C * RS + C * VS + 2 * C;       // q | k | v | decay, write strength
+template <int KP, bool DELTA, typename QK, typename VT, bool VEC>
+__global__ __launch_bounds__(512) void chunk_head_kernel(ChunkScanArgs a) {
+  constexpr int KT = KP / 16, RS = KP + 4;
+  constexpr int kRaw = 2 * C * RS + C * VS + 3 * C;       // q | k | v | decay, value scale, write strength
   constexpr int kMade = 2 * C * RA + 3 * C;               // A | M (T while it is made) | prefix, suffix, what the prefix's rounding left over
   extern __shared__ __attribute__((aligned(16))) float lds[];      // raw[3] | made[2]
   const int seq = blockIdx.z, head = blockIdx.x, col0 = (int)blockIdx.y * VW;
@@ -81,18 +86,25 @@ __global__ __launch_bounds__(512) void chunk_delta_kernel(ChunkScanArgs a) {
       const f32x4 pre = *reinterpret_cast<const f32x4*>(M + C * RA + 4 * g), suf = *reinterpret_cast<const f32x4*>(M + C * RA + C + 4 * g);
       const f32x4 rest = *reinterpret_cast<const f32x4*>(M + C * RA + 2 * C + 4 * g);
       const float total = M[C * RA + C - 1];
-      f32x4 x;
+      f32x4 x, w;
 #pragma unroll
       for (int e = 0; e < 4; ++e) x[e] = vs[(4 * g + e) * VS + 16 * cw + m];
-      const f32x4 y = st.times(k), b = *reinterpret_cast<const f32x4*>(sc + C + 4 * g);
+      if constexpr (DELTA) {
+        const f32x4 y = st.times(k), b = *reinterpret_cast<const f32x4*>(sc + 2 * C + 4 * g);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) x[e] = b[e] * (x[e] - pre[e] * y[e]);
-      f32x4 w = times_rows(*reinterpret_cast<const f32x4*>(M + m * RA + 4 * g), x);
+        for (int e = 0; e < 4; ++e) x[e] = b[e] * (x[e] - pre[e] * y[e]);
+        w = times_rows(*reinterpret_cast<const f32x4*>(M + m * RA + 4 * g), x);
+      } else {
+        const f32x4 s = *reinterpret_cast<const f32x4*>(sc + C + 4 * g);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = x[e] * s[e];
+      }
       const f32x4 before = st.times(q);
       f32x4 within = times_rows(*reinterpret_cast<const f32x4*>(A + m * RA + 4 * g), w);
-      products_behind_reads<10, 9, 3, 13>();
+      if constexpr (KP == 128) products_behind_reads<8, 26, 3, 1>();
+      else products_behind_reads<10, 9, 3, 13>();
       if (some_not_finite(w)) {                            // (of x: then every row of w)
-        w = times_rows_in_order(M, m, g, x);
+        if constexpr (DELTA) w = times_rows_in_order(M, m, g, x);
         within = times_rows_in_order(A, m, g, w);
       }
       f32x4 o;
@@ -190,7 +202,7 @@ __global__ __launch_bounds__(512) void chunk_delta_kernel(ChunkScanArgs a) {
       run = t > t_m ? run * d[t] : 1.f;
       mine[t >> 2] = (t & 3) == 0 || (t & 3) == g ? run : mine[t >> 2];
     }
-    const f32x4 b = *reinterpret_cast<const f32x4*>(sc + C + 4 * g);
+    const f32x4 b = *reinterpret_cast<const f32x4*>(sc + 2 * C + 4 * g);
 #pragma unroll
     for (int e = 0; e < 4; ++e) A[(4 * e + g) * RA + t_m] = t_m < 4 * e + g ? b[e] * xk[e] * mine[e] : 0.f;      // (T: by tokens)
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -226,7 +238,7 @@ __global__ __launch_bounds__(512) void chunk_delta_kernel(ChunkScanArgs a) {
     for (int c = -2; c < n_chunks; ++c) {
       if (c + 1 >= 0 && c + 1 < n_chunks) {
         if (wave == 0) finish_A(c + 1);
-        else finish_M(c + 1);
+        else if constexpr (DELTA) finish_M(c + 1);
       }
       lds_barrier();
     }
@@ -237,10 +249,11 @@ __global__ __launch_bounds__(512) void chunk_delta_kernel(ChunkScanArgs a) {
   const typename QK::storage* x = (const typename QK::storage*)(wave == 2 ? a.q : a.k) + t_begin * (wave == 2 ? a.q_stride : a.k_stride) + (int64_t)qk_head * a.K;
   const int64_t x_stride = wave == 2 ? a.q_stride : a.k_stride;
   const typename VT::storage* v = (const typename VT::storage*)a.v + t_begin * a.v_stride + (int64_t)head * a.V;
+  const float* per_token[3] = {a.decay, a.vscale ? a.vscale : a.decay, DELTA ? a.beta : a.decay};
   struct Set {
     Rows<QK, VEC, KP, 64> rows;
     Rows<VT, VEC, VW, 128> values;         // (waves 2 and 3 half of them each)
-    float decay, beta;
+    float scalars[3];
   } sets[kAhead];
   auto fetch = [&](Set& s, int chunk) __attribute__((always_inline)) {
     chunk = min(chunk, n_chunks - 1);
@@ -248,8 +261,8 @@ __global__ __launch_bounds__(512) void chunk_delta_kernel(ChunkScanArgs a) {
     s.rows.fetch(x + (int64_t)chunk * C * x_stride, x_stride, 0, a.K, n, lane);
     s.values.fetch(v + (int64_t)chunk * C * a.v_stride, a.v_stride, col0, a.V, n, (int)threadIdx.x - 128);
     const int64_t th = (t_begin + chunk * C + min(m, n - 1)) * a.heads + head;
-    s.decay = a.decay[th];
-    s.beta = a.beta[th];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) s.scalars[i] = per_token[i][th];
   };
   auto store = [&](const Set& s, int chunk) __attribute__((always_inline)) {
     if (chunk >= n_chunks) return;
@@ -259,8 +272,9 @@ __global__ __launch_bounds__(512) void chunk_delta_kernel(ChunkScanArgs a) {
     s.values.store(r + 2 * C * RS, col0, a.V, n, 1.f, (int)threadIdx.x - 128);
     if (wave == 3 && g == 0) {             // (a row past the portion changes nothing)
       float* sc = r + 2 * C * RS + C * VS;                 // (decays by token, the others by row)
-      sc[m] = m < n ? s.decay : 1.f;
-      sc[C + row_of_token(m)] = m < n ? s.beta : 0.f;
+      sc[m] = m < n ? s.scalars[0] : 1.f;
+      sc[C + row_of_token(m)] = m < n && a.vscale ? s.scalars[1] : 1.f;
+      sc[2 * C + row_of_token(m)] = m < n && DELTA ? s.scalars[2] : 0.f;
     }
   };
 #pragma unroll
@@ -426,11 +440,10 @@ template <int KP, typename QK, typename VT, bool VEC>
 int launch_form(const ChunkScanArgs& a, hipStream_t s) {
   if (a.form == hxm::kChunkGated) return launch_channel<KP, hxm::kChunkGated, QK, VT, VEC>(a, s);
   if (a.form == hxm::kChunkBonus) return launch_channel<KP, hxm::kChunkBonus, QK, VT, VEC>(a, s);
-  if constexpr (KP == 64) {
-    if (a.form == hxm::kChunkDelta)
-      return launch(chunk_delta_kernel<QK, VT, VEC>, 512, sizeof(float) * (3 * (2 * C * (KP + 4) + C * VS + 2 * C) + 2 * (2 * C * RA + 3 * C)), a, s);
-  }
-  return launch_channel<KP, hxm::kChunkDecay, QK, VT, VEC>(a, s);
+  if (a.per_channel) return launch_channel<KP, hxm::kChunkDecay, QK, VT, VEC>(a, s);
+  const size_t lds = sizeof(float) * (3 * (2 * C * (KP + 4) + C * VS + 3 * C) + 2 * (2 * C * RA + 3 * C));
+  if (a.form == hxm::kChunkDelta) return launch(chunk_head_kernel<KP, true, QK, VT, VEC>, 512, lds, a, s);
+  return launch(chunk_head_kernel<KP, false, QK, VT, VEC>, 512, lds, a, s);
 }
 
 template <typename QK, typename VT>
@@ -454,9 +467,24 @@ bool chunk_scan_fits(const ChunkScanArgs& a) {
          !(a.form == kChunkBonus && !a.per_channel);
 }
 
+// One decay a head: thirty-two tokens at a time (chunk_head.hip)?  Of the time here:
+//   delta rule, up to 64 key channels: no (16 portions of 60 tokens, 32 heads of 64 x 64 22.1 us here and 24.1, 4 of 797 - 1151 124 and 122, 12 of 300 - 900 124
+//     and 130; there two workgroups do not share a compute unit);
+//   decayed sum of float q and k, which are split in three parts: no (up to 64 key channels 1.05 - 1.5 in all of 150 batches; more, 0.95 in long portions, 1.1 -
+//     1.28 in short ones);
+//   bfloat16 q and k, one part each, more than 64 key channels: yes (0.67 - 1.03);
+//   the rest where the tokens that a portion has in the mean fill chunks of thirty-two well enough, which take 1.7 of one of sixteen (delta rule, float: 6 - 16
+//     tokens 1.17, 17 - 32 0.94, 33 - 48 1.07, 49 - 64 0.9, long ones 0.87 - 0.94) or 1.85 (decayed sum, bfloat16, up to 64 channels: up to 1.06, 0.9, 1, 0.97, 0.92).
+bool by_thirty_two(const ChunkScanArgs& a) {
+  const bool wide = a.K > 64, delta = a.form == kChunkDelta, parts = a.q_dtype == HX_F32;
+  if (a.per_channel || a.form == kChunkGated || !(delta ? wide : !parts)) return false;
+  const double mean = (double)a.n_tokens / a.n_seq;
+  return (wide && !parts) || (parts ? 1.7 : 1.85) * ceil(mean / (2 * C)) < ceil(mean / C);
+}
+
 int chunk_scan(const ChunkScanArgs& a, hipStream_t s) {
   if (a.made) return chunk_chain(a, s);
-  if (!a.per_channel && a.form != kChunkGated && !(a.form == kChunkDelta && a.K <= 64)) return chunk_head(a, s);
+  if (by_thirty_two(a)) return chunk_head(a, s);
   if (a.q_dtype == HX_BF16) return launch_width<BF16, BF16>(a, s);
   return a.v_dtype == HX_F32 ? launch_width<F32, F32>(a, s) : launch_width<F32, BF16>(a, s);
 }
