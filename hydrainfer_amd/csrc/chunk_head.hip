@@ -332,7 +332,7 @@ __global__ __launch_bounds__(512) void chunk_head32_kernel(ChunkScanArgs a) {
     Piece<VT, 4, VEC> v[NV];
     float scale;
   } next;                                                 // the chunk's whose rows are on their way
-  // (strides below 2^28: chunk_scan_fits)
+  // (strides below 2^28: what chunk_scan.hip sends here)
   auto at_row = [&](auto* base, int r, int64_t stride) __attribute__((always_inline)) {
     typedef std::remove_pointer_t<decltype(base)> E;
     return reinterpret_cast<E*>(reinterpret_cast<uintptr_t>(base) + (uint64_t)(uint32_t)r * (uint32_t)(stride * sizeof(E)));

@@ -461,9 +461,7 @@ bool chunk_scan_fits(const ChunkScanArgs& a) {
   // the delta rule with a decay per channel and the bonus form with one per head have no chunk form; q and k of one type, and
   // bfloat16 q and k come with bfloat16 v
   const bool types = a.q_dtype == a.k_dtype && (a.q_dtype == HX_F32 || a.v_dtype == HX_BF16);
-  // (rows of a chunk are addressed by 32-bit offsets)
-  const bool near_rows = a.q_stride < (1 << 28) && a.k_stride < (1 << 28) && a.v_stride < (1 << 28);
-  return types && near_rows && a.K <= 128 && a.n_seq <= 65535 && (a.V + VW - 1) / VW <= 65535 && !(a.form == kChunkDelta && a.per_channel) &&
+  return types && a.K <= 128 && a.n_seq <= 65535 && (a.V + VW - 1) / VW <= 65535 && !(a.form == kChunkDelta && a.per_channel) &&
          !(a.form == kChunkBonus && !a.per_channel);
 }
 
@@ -475,9 +473,11 @@ bool chunk_scan_fits(const ChunkScanArgs& a) {
 //   bfloat16 q and k, one part each, more than 64 key channels: yes (0.67 - 1.03);
 //   the rest where the tokens that a portion has in the mean fill chunks of thirty-two well enough, which take 1.7 of one of sixteen (delta rule, float: 6 - 16
 //     tokens 1.17, 17 - 32 0.94, 33 - 48 1.07, 49 - 64 0.9, long ones 0.87 - 0.94) or 1.85 (decayed sum, bfloat16, up to 64 channels: up to 1.06, 0.9, 1, 0.97, 0.92).
+// Rows of a chunk are addressed by 32-bit offsets there: strides of 2^28 elements and more come here.
 bool by_thirty_two(const ChunkScanArgs& a) {
   const bool wide = a.K > 64, delta = a.form == kChunkDelta, parts = a.q_dtype == HX_F32;
-  if (a.per_channel || a.form == kChunkGated || !(delta ? wide : !parts)) return false;
+  const bool near_rows = a.q_stride < (1 << 28) && a.k_stride < (1 << 28) && a.v_stride < (1 << 28);
+  if (a.per_channel || a.form == kChunkGated || !(delta ? wide : !parts) || !near_rows) return false;
   const double mean = (double)a.n_tokens / a.n_seq;
   return (wide && !parts) || (parts ? 1.7 : 1.85) * ceil(mean / (2 * C)) < ceil(mean / C);
 }

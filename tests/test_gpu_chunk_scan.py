@@ -443,3 +443,26 @@ def test_small_gates_are_as_exact_as_large_ones(max_q_len):
 @pytest.mark.parametrize("types, pad", [("bf16", 4), ("f32", 4), ("mixed", 3)])
 def test_chunks_of_two_tiles(lens, form, K, V, types, pad):
     _through_a_scan(lens, K, V, form, False, types, pad)
+
+
+# rows so far apart that chunks of thirty-two tokens do not address them: in chunks of sixteen all the same
+@pytest.mark.parametrize("form", ["decay", "delta"])
+def test_rows_far_apart(form):
+    from hydrainfer_amd._C.kernel.seq_mix import state_scan
+    from hydrainfer_amd._C.kernel.stream_ops import SequenceState
+    T, H, K, V, stride = 17, 2, 128, 64, 2 ** 28
+    g = torch.Generator(device="cuda").manual_seed(5)
+    f = lambda *s: torch.randn(s, generator=g, device="cuda")
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    unit = lambda: torch.nn.functional.normalize(f(T, H, K), dim=-1).reshape(T, H * K).bfloat16()
+    near, state, decay, beta = (unit(), unit(), f(T, H * V).bfloat16()), f(1, 1, H * K * V), torch.rand((T, H), generator=g, device="cuda"), torch.rand((T, H), generator=g, device="cuda")
+    room = torch.empty((T - 1) * stride + 2048, dtype=torch.bfloat16, device="cuda")      # (9 GB, of which the rows are touched)
+    far = [room[512 * n:].as_strided(x.shape, (stride, 1)).copy_(x) for n, x in enumerate(near)]
+    got = []
+    for q, k, v in (near, far):
+        st = state.clone()
+        seq = SequenceState(st, i32([0]), i32([0] * T))
+        got.append((state_scan(form, q, k, v, decay, seq, 0, i32([0, T]), i32(list(range(9, 9 + T))), H, H, K, V, beta=beta if form == "delta" else None).double(), st.double()))
+    # thirty-two tokens in parts and sixteen in float: either is within 2e-7 of 64 bits (2-norm)
+    for a, b in zip(*got):
+        assert float((a - b).norm() / a.norm()) < 1e-6

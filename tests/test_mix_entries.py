@@ -94,3 +94,14 @@ def test_splits_of_latent_portions(lens, kv, heads, rank, splits):
     (192, 2047, 32, 128, 0, 3), (192, 2047, 32, 320, 0, 3), (192, 2047, 8, 320, 0, 3), (128, 2047, 8, 320, 0, 4), (160, 2047, 32, 320, 0, 4), (64, 8000, 32, 128, 0, 8)])
 def test_splits_of_single_latent_tokens(tokens, kv, heads, rank, window, splits):
     assert _latent_splits([1] * tokens, kv, heads, rank, window) == splits
+
+
+@pytest.mark.parametrize("stride", [128 * 128, 2 ** 28 - 1, 2 ** 28, 2 ** 40])
+@pytest.mark.parametrize("mode, per_channel", [(0, 0), (0, 1), (1, 1), (2, 0)])
+def test_rows_far_apart_still_go_in_chunks(stride, mode, per_channel):
+    """The launch ahead is asked for wherever chunks serve; how far apart rows are is no reason not to."""
+    from hydrainfer_amd import _lib
+    HX_F32 = 0
+    a = _lib.hxm_state_scan_args(q_dtype=HX_F32, k_dtype=HX_F32, v_dtype=HX_F32, n_tokens=1151, n_seq=1, heads=32, qk_heads=32, dim=128, vdim=128, mode=mode,
+                                 decay_per_channel=per_channel, q_stride=stride, k_stride=stride, v_stride=stride)
+    assert _lib.mix_lib().hxm_state_scan_workspace(ctypes.byref(a)) > 0
