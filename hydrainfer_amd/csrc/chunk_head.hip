@@ -2,23 +2,26 @@
 // decayed sum), in one launch, thirty-two tokens at a time.  A chunk is two tiles of sixteen tokens:
 //     W_0 = M_00 b (V - R)_0,  W_1 = M_11 b (V - R - T_10 W_0)_1      R = prefix (K S), M_uu = (I + b T_uu)^-1      (decayed sum: W = s V)
 //     O_u = prefix (Q S) + sum(v <= u) A_uv W_v,  S <- total S + (K * suffix)^T W
-// The products with the state and q k^T, k k^T are bfloat16 products of operands that are split in three: x = hi + mid + lo, each rounded to
-// bfloat16, holds all of a float's 24 bits, and of the nine products of two such numbers the three that are left out are below
-// 2^-24 of the whole.  Six products of 16 x 16 x 32 take 96 cycles where float products of the same size take 256, and round less: hi hi is
+// The products with the state and q k^T, k k^T are bfloat16 products of operands that are split in three (Henry, Tang and Heinecke, Leveraging the
+// bfloat16 artificial intelligence datatype for higher-precision computations, 2019): x = hi + mid + lo, each rounded to bfloat16, holds all of a
+// float's 24 bits, and of the nine products of two such numbers the three that are left out are below 2^-24 of the whole.  Six products of 16 x 16 x 32 take 96 cycles where float products of the same size take 256, and round less: hi hi is
 // summed by itself and the other five beside it (2-norm of the error over 128 channels, operands normal: 8.8e-8 in float with eight
 // chains, 6.5e-8 here; all six in one sum 1.5e-7).  bfloat16 q and k are one part and take three products, all of them exact.
-// W, M, A and T stay float, and so do the state and everything that is added up.
+// W, M, A and T stay float, and so do the state and everything that is added up.  Limits: lo is below bfloat16's smallest numbers where x is below
+// 2^-110 (its parts are then off by up to 2^-134: subnormal ones are kept), and a finite x above 3.39e38 rounds to an infinite hi and counts as infinite.
 // A workgroup owns 64 value channels of one (sequence, head): four consumer waves hold the state, 16 channels of values and all keys
 // each, as accumulators, and split it anew for each chunk; the parts are the operand of the products with S as they lie in the registers
 // (a lane group's eight keys: rows 4 g + e of two tiles of 16).  Four producer waves bring rows in (requested a chunk ahead), split
 // them into planes in LDS and make A, M and T of the next chunk while the consumers work on this one; two barriers a chunk.
 // What bounds it: the vector ALU of a SIMD, which a consumer (430 instructions a chunk under the delta rule: parts, sums, results) and a producer (850:
-// parts of rows, products of decays, the substitution) share, and which does not run beside the products of its own wave.  Of a chunk's 4.4 us
+// parts of rows, products of decays, the substitution) share, and which does not run beside the products of its own wave.  Of a chunk's 4.6 us
 // 1.3 are matrix products.
 // Measured, one launch of sixteen tokens at a time in float and this one, us: delta rule, 128 x 128, 32 heads, 4 portions of 797 - 1151 tokens 191 and
 // 169, 12 of 300 - 900 348 and 309, 16 of 60 55.6 and 55.6; decayed sum, 128 x 128, 32 heads, 4 of 797 - 1151 145 and 103, 12 of 300 - 900 263 and 190,
 // one of 100 19.8 and 17.1, 64 x 64 93 and 83.  Results' error against 64 bits (2-norm, 400 and 250 tokens, 1e-7): delta rule 1.08 and 1.00,
 // decayed sum 128 x 128 0.867 and 0.863, 64 x 64 0.79 and 0.76; states 0.77 and 0.72, 0.73 and 0.62, 0.72 and 0.64.
+#include <cfloat>
+
 #include "attn_common.h"
 #include "chunk_parts.h"
 
@@ -48,6 +51,16 @@ __device__ __forceinline__ void split(f32x4 x, u16x4 (&part)[3]) {
       part[p][e] = BF16::from_float(x[e]);
       if (p < 2) x[e] -= BF16::to_float(part[p][e]);
     }
+}
+
+// What is infinite has no lower parts (inf - inf), and an infinity times another's lower part of zero is no number: where the sum of hi hi is not finite it
+// says by itself what a product is, and the other sum, whatever it came to, is only to be finite.  (v_med3 with an operand that is no number gives the least of
+// the others.)
+__device__ __forceinline__ f32x4 total_of(const f32x4 (&sum)[2]) {
+  f32x4 t;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) t[e] = sum[0][e] + __builtin_amdgcn_fmed3f(sum[1][e], -FLT_MAX, FLT_MAX);
+  return t;
 }
 
 // Products of N operands in parts with one in parts (SECOND: the other way round): hi hi to sum[0], the others, smallest first, to sum[1].  A product
@@ -158,10 +171,10 @@ __global__ __launch_bounds__(512) void chunk_head32_kernel(ChunkScanArgs a) {
       const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
       f32x4 w[2], scale[2], pre[2], rest[2], suffix[2], m00, m11, t10, a00, a10, a11;
       float total;
+      auto token = [&](int what, int u) __attribute__((always_inline)) { return *reinterpret_cast<const f32x4*>(tk + what + 4 * (16 * u + 4 * g)); };
+      auto row = [&](const float* of, int u, int v) __attribute__((always_inline)) { return *reinterpret_cast<const f32x4*>(of + (16 * u + m) * RM + 16 * v + 4 * g); };
+      const float* vs = reinterpret_cast<const float*>(im + I::kV) + 4 * g * VS + 16 * cw + m;
       auto rest_at = [&]() __attribute__((always_inline)) {
-        auto token = [&](int what, int u) __attribute__((always_inline)) { return *reinterpret_cast<const f32x4*>(tk + what + 4 * (16 * u + 4 * g)); };
-        auto row = [&](const float* of, int u, int v) __attribute__((always_inline)) { return *reinterpret_cast<const f32x4*>(of + (16 * u + m) * RM + 16 * v + 4 * g); };
-        const float* vs = reinterpret_cast<const float*>(im + I::kV) + 4 * g * VS + 16 * cw + m;
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           scale[u] = token(I::kScale, u);
@@ -204,7 +217,6 @@ __global__ __launch_bounds__(512) void chunk_head32_kernel(ChunkScanArgs a) {
       __builtin_amdgcn_sched_barrier(0);
       lds_barrier();                                      // (the next chunk's rows are there)
       const int n = rows_of(c);
-      const f32x4 again[2] = {w[0], w[1]};
       f32x4 x[2], within[2], across;                      // x (delta rule): what M is multiplied with; across: what the second tile has of the first
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
@@ -236,61 +248,61 @@ __global__ __launch_bounds__(512) void chunk_head32_kernel(ChunkScanArgs a) {
         }
       }
       within[1] = times_rows(a11, w[1]);
-      if (some_not_finite(w[0]) || some_not_finite(w[1])) {      // (of x, then every row of w) again, so that nothing reaches earlier tokens
+      auto results = [&](const f32x4 (&before)[2], const f32x4 (&low)[2], const f32x4 (&pre)[2], const f32x4 (&rest)[2], const f32x4 (&within)[2], f32x4 across, f32x4 (&result)[2]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          f32x4 earlier = zero;
-          if constexpr (DELTA) {
-            if (u == 1) x[1] = scale[1] * (again[1] - ((sum[3][0] + sum[3][1]) * pre[1] + times_rows(t10, w[0])));
-            w[u] = rows_in_order(M + 16 * u * RM + 16 * u, m, g, x[u], zero);
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float in = within[u][e], more = u ? across[e] : 0.f;
+            if constexpr (NP == 3) {                      // (the delta rule)
+              const float read = before[u][e] + low[u][e];
+              result[u][e] = __builtin_fmaf(read, pre[u][e], __builtin_fmaf(read, rest[u][e], in + more));
+            } else {                                      // (in double: the operands' products are exact, and a rounding here shows.  3 % of the time)
+              const double p = (double)pre[u][e] + (double)rest[u][e];
+              result[u][e] = (float)__builtin_fma((double)before[u][e], p, __builtin_fma((double)low[u][e], p, (double)in + (double)more));
+            }
           }
-          if (u == 1) across = times_rows(a10, w[0]);
-          within[u] = rows_in_order(A + 16 * u * RM + 16 * u, m, g, w[u], earlier);
+      };
+      auto write = [&](const f32x4 (&result)[2]) __attribute__((always_inline)) {
+        if (col < a.V) {
+          if (n == CW) {                                  // (no question for every row: they took longer than the products)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) out[4 * i * out_row] = result[i >> 2][i & 3];
+          } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+              if (4 * i + g < n) out[4 * i * out_row] = result[i >> 2][i & 3];
+          }
         }
-      }
+      };
       f32x4 result[2];
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float in = within[u][e], more = u ? across[e] : 0.f;
-          if constexpr (NP == 3) {                        // (the delta rule)
-            const float before = sum[u][0][e] + sum[u][1][e];
-            result[u][e] = __builtin_fmaf(before, pre[u][e], __builtin_fmaf(before, rest[u][e], in + more));
-          } else {                                        // (in double: the operands' products are exact, and a rounding here shows.  3 % of the time)
-            const double p = (double)pre[u][e] + (double)rest[u][e];
-            result[u][e] = (float)__builtin_fma((double)sum[u][0][e], p, __builtin_fma((double)sum[u][1][e], p, (double)in + (double)more));
-          }
-        }
-      if (col < a.V) {
-        if (n == CW) {                                    // (no question for every row: they took longer than the products)
-#pragma unroll
-          for (int i = 0; i < 8; ++i) out[4 * i * out_row] = result[i >> 2][i & 3];
-        } else {
-#pragma unroll
-          for (int i = 0; i < 8; ++i)
-            if (4 * i + g < n) out[4 * i * out_row] = result[i >> 2][i & 3];
-        }
-      }
-      out += CW * out_row;
-      u16x8 wp[3];
-      {
+      results({sum[0][0], sum[1][0]}, {sum[0][1], sum[1][1]}, pre, rest, within, across, result);
+      write(result);
+      auto parts_of = [&](const f32x4 (&w)[2], const f32x4 (&suffix)[2], u16x8 (&wp)[3]) __attribute__((always_inline)) {
         u16x4 w0[3], w1[3];
         split(w[0] * suffix[0], w0);
         split(w[1] * suffix[1], w1);
 #pragma unroll
         for (int p = 0; p < 3; ++p) wp[p] = both(w0[p], w1[p]);
-      }
+      };
+      // Numbers that are not finite: in the state (a row of q times it is none then), in w or in a token's keys (q k of a token with itself, so its row of A w).
+      // The chunk is gone through again below, from the state as it is here, which its slot keeps.  (Behind the results: the branch would wait for them.)
+      const bool wild = some_not_finite(within[0]) || some_not_finite(within[1]) || (!DELTA && __builtin_amdgcn_ballot_w64(!__builtin_isfinite(sum[0][0][0])));
+      if (wild) st.store(slot, a.K, a.V, col, g);
+      u16x8 wp[3];
+      parts_of(w, suffix, wp);
       // the transposing reads: lane 4 q + p of a group of 16 brings row 4 g + q (and the row 16 below it), keys 16 kt + 4 p ..
+      auto keys_of = [&](int kt, u16x8 (&x)[NP]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+          const char* at = im + I::kK + p * I::kPlane + place_of(4 * g + (m >> 2)) * I::kRow + 32 * kt + 8 * (m & 3);
+          x[p] = both(lds_tr_read(at), lds_tr_read(at + 16 * I::kRow));
+        }
+      };
       u16x8 kx[2][4][NP];
       auto keys_at = [&](int k2) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int p = 0; p < NP; ++p) {
-            const char* at = im + I::kK + p * I::kPlane + place_of(4 * g + (m >> 2)) * I::kRow + 32 * (4 * k2 + i) + 8 * (m & 3);
-            kx[k2 & 1][i][p] = both(lds_tr_read(at), lds_tr_read(at + 16 * I::kRow));
-          }
+        for (int i = 0; i < 4; ++i) keys_of(4 * k2 + i, kx[k2 & 1][i]);
       };
       keys_at(0);
 #pragma unroll
@@ -310,6 +322,63 @@ __global__ __launch_bounds__(512) void chunk_head32_kernel(ChunkScanArgs a) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) st.S[4 * k2 + i][e] = __builtin_fmaf(st.S[4 * k2 + i][e], total, more[i][0][e] + more[i][1][e]);
       }
+      if (wild) {                                         // token by token where nothing may reach earlier ones, infinities as what they are
+        __builtin_amdgcn_sched_barrier(0);
+        st.load(slot, a.K, a.V, col, g, false);
+        f32x4 s[NX][2], total_s[NX], w[2], pre[2], rest[2], suffix[2], within[2], across = zero;
+#pragma unroll
+        for (int i = 0; i < NX; ++i) s[i][0] = s[i][1] = zero;
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+          __builtin_amdgcn_sched_barrier(0);
+          u16x8 x[NX][NP];
+#pragma unroll
+          for (int i = 0; i < NX; ++i) parts_at(im + (i < 2 ? I::kQ : I::kK), i & 1, kb, x[i]);
+          state_at(kb);
+          add_products(x, sp[kb & 1], s);
+        }
+#pragma unroll
+        for (int i = 0; i < NX; ++i) total_s[i] = total_of(s[i]);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          pre[u] = token(I::kPrefix, u);
+          rest[u] = token(I::kRest, u);
+          suffix[u] = token(I::kSuffix, u);
+          const f32x4 scale = token(I::kScale, u);
+          f32x4 v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = vs[(16 * u + e) * VS];
+          if constexpr (DELTA) {
+            f32x4 read = total_s[2 + u] * pre[u];
+            if (u == 1) read += times_rows(row(M, 1, 0), w[0]);
+            w[u] = rows_in_order(M + 16 * u * RM + 16 * u, m, g, scale * (v - read), zero);
+          } else {
+            w[u] = v * scale;
+          }
+          if (u == 1) across = times_rows(row(A, 1, 0), w[0]);
+          within[u] = rows_in_order(A + 16 * u * RM + 16 * u, m, g, w[u], zero);
+        }
+        f32x4 result[2];
+        results({total_s[0], total_s[1]}, {zero, zero}, pre, rest, within, across, result);
+        write(result);
+        parts_of(w, suffix, wp);
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) {
+          __builtin_amdgcn_sched_barrier(0);
+          u16x8 x[1][NP];
+          keys_of(kt, x[0]);
+#pragma unroll
+          for (int p = 0; p < NP; ++p)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[0][p][e] = 4 * e + g < n ? x[0][p][e] : u16(0);      // (rows past the portion: no zeros of theirs meet its last key)
+          f32x4 more[1][2] = {{zero, zero}};
+          add_products(x, wp, more);
+          const f32x4 t = total_of(more[0]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) st.S[kt][e] = __builtin_fmaf(st.S[kt][e], total, t[e]);
+        }
+      }
+      out += CW * out_row;
     }
     st.store(slot, a.K, a.V, col, g);
     return;

@@ -341,6 +341,48 @@ def test_not_finite_numbers_reach_later_tokens_only(K, V, form, per_channel, wha
         _check("finite", got[fine], want[fine])
 
 
+# Infinities stay infinities of their sign where the arithmetic has one answer: values of a portion's last token (its state is then k times them), keys of
+# it, and what the state held before (a decayed sum's stays).  Under the delta rule the last token is a chunk's last: rows past a portion read it.
+@pytest.mark.parametrize("form, K, V, types", [("decay", 128, 64, "bf16"), ("decay", 64, 34, "bf16"), ("decay", 128, 128, "f32"), ("decay", 64, 64, "mixed"),
+                                               ("delta", 128, 64, "bf16"), ("delta", 100, 130, "f32"), ("delta", 128, 128, "mixed"), ("delta", 64, 64, "mixed")])
+@pytest.mark.parametrize("what", ["v", "k", "state"])
+def test_infinities_stay_infinities(form, K, V, types, what):
+    if form == "delta" and what != "v":
+        pytest.skip("the portion's tokens read what is infinite, in sums of both signs")
+    from hydrainfer_amd._C.kernel.seq_mix import state_scan
+    from hydrainfer_amd._C.kernel.stream_ops import SequenceState
+    g = torch.Generator().manual_seed(K + V)
+    lens, H, inf = [60, 17, 55, 96] if form == "decay" else [64, 32, 32, 96], 2, float("inf")
+    n, T, cu = len(lens), sum(lens), [sum(lens[:s]) for s in range(len(lens) + 1)]
+    qk_t, v_t = (torch.bfloat16 if types == "bf16" else torch.float32), (torch.float32 if types == "f32" else torch.bfloat16)
+    unit = lambda: torch.nn.functional.normalize(torch.randn((T, H, K), generator=g), dim=-1).reshape(T, H * K).to(qk_t)
+    q, k, v = unit(), unit(), torch.randn((T, H * V), generator=g).to(v_t)
+    decay, beta, state = 0.5 + 0.5 * torch.rand((T, H), generator=g), torch.rand((T, H), generator=g), torch.randn((n, 1, H * K * V), generator=g)
+    for s in range(n):
+        last = cu[s + 1] - 1
+        if what == "v":
+            v[last, V + 3], v[last, 7] = inf, -inf
+        elif what == "k":
+            k[last, 5], k[last, K + 9] = inf, -inf
+        else:
+            state.view(n, H, K, V)[s, 1, 5, 3], state.view(n, H, K, V)[s, 0, 9, 7] = inf, -inf
+    h = lambda x, m: x.double().view(T, H, m)
+    want, S = _scan(form, h(q, K), h(k, K), h(v, V), decay.double().view(T, H, 1).expand(T, H, K), torch.ones((T, H), dtype=torch.float64), beta.double(), None,
+                    state.double().view(n, H, K, V), cu, [False] * n)
+    d = lambda x: x.cuda()
+    st = d(state)
+    seq = SequenceState(st, torch.arange(n, dtype=torch.int32, device="cuda"), d(torch.tensor([s for s in range(n) for _ in range(lens[s])], dtype=torch.int32)))
+    got = state_scan(form, d(q), d(k), d(v), d(decay), seq, 0, d(torch.tensor(cu, dtype=torch.int32)), d(torch.tensor([9 + i for m in lens for i in range(m)], dtype=torch.int32)),
+                     H, H, K, V, beta=d(beta) if form == "delta" else None)
+    for name, got, want in (("out", got.double().cpu(), want.reshape(T, H * V)), ("state", st.double().cpu().view(n, H, K, V), S)):
+        fine = torch.isfinite(want)
+        assert torch.equal(torch.isfinite(got), fine)
+        if name == "state":                   # (results are sums over infinities of both signs)
+            assert bool(torch.isinf(want).any()) and not bool(torch.isnan(want).any())
+            assert torch.equal(got[~fine], want[~fine])
+        _check("finite", got[fine], want[fine])
+
+
 @pytest.mark.parametrize("what", ["v", "k"])
 def test_not_finite_numbers_in_the_gated_recurrence(what):
     from hydrainfer_amd._C.kernel.recurrence import gated_recurrence
