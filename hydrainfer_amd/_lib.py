@@ -224,7 +224,7 @@ def lib() -> ctypes.CDLL:
 # a paged latent cache.  A library of its own, so that a model that needs only these builds only these (`make mix`).
 # ---------------------------------------------------------------------------------------------------------
 MIX_LIB_PATH = os.environ.get("HX_MIX_LIB_PATH") or os.path.join(_HERE, "lib", "libhydra_mix.so")
-HXM_ABI_VERSION = 7
+HXM_ABI_VERSION = 8
 HXM_MAX_STREAMS = 16
 HXM_MAX_LATENT = 1024
 
@@ -420,13 +420,14 @@ def mix_lib() -> ctypes.CDLL:
             raise HydraHipError(f"{MIX_LIB_PATH} is missing: build it with `make -C hydrainfer_amd/csrc mix`. "
                                 "There is no fallback path.")
         handle = ctypes.CDLL(MIX_LIB_PATH)
+        version = handle.hxm_abi_version()      # (before the entry points: a library of another version need not have them all)
+        if version != HXM_ABI_VERSION:
+            raise HydraHipError(f"libhydra_mix.so ABI version {version} != {HXM_ABI_VERSION} of this binding: "
+                                "rebuild with `make -C hydrainfer_amd/csrc mix`")
         for name, (restype, argtypes) in _MIX_SIGNATURES.items():
             fn = getattr(handle, name)
             fn.restype = restype
             fn.argtypes = argtypes
-        if handle.hxm_abi_version() != HXM_ABI_VERSION:
-            raise HydraHipError(f"libhydra_mix.so ABI version {handle.hxm_abi_version()} != {HXM_ABI_VERSION} of this binding: "
-                                "rebuild with `make -C hydrainfer_amd/csrc mix`")
         _load_front(handle)
         _mix = handle
     return _mix

@@ -34,7 +34,7 @@
 extern "C" {
 #endif
 
-#define HXM_ABI_VERSION 7
+#define HXM_ABI_VERSION 8
 #define HXM_MAX_STREAMS 16
 #define HXM_MAX_LATENT 1024     /* widest latent row the attention kernels hold in registers (the MFMA tile form: 512) */
 
