@@ -3,12 +3,16 @@
 This is the only place the shared library is opened.  Loading fails loudly: there is
 no CPU or eager-PyTorch fallback anywhere in the product path (the reference instead
 wraps every `hydrainfer._C` import in try/except and silently drops to torch, e.g.
-hydrainfer/layer/causal_attention.py:13-17).
+hydrainfer/layer/causal_attention.py:13-17).  libhydra_front.so, host code in front of some
+of its calls, is the one that may be missing: they launch the same kernels without it.
 """
 import ctypes
 import importlib.machinery
 import importlib.util
 import os
+import sys
+import threading
+import warnings
 from ctypes import c_char_p, c_float, c_int, c_int32, c_int64, c_void_p, POINTER
 
 import torch
@@ -414,8 +418,17 @@ _STATUS_TEXT = {-1: "dtype not supported", -2: "size / divisibility constraint v
 
 def mix_lib() -> ctypes.CDLL:
     """Open libhydra_mix.so once and type every entry point.  No fallback: a missing library raises."""
+    return _mix if _mix is not None else _open_mix()
+
+
+_mix_lock = threading.Lock()
+
+
+def _open_mix() -> ctypes.CDLL:
     global _mix
-    if _mix is None:
+    with _mix_lock:
+        if _mix is not None:
+            return _mix
         if not os.path.exists(MIX_LIB_PATH):
             raise HydraHipError(f"{MIX_LIB_PATH} is missing: build it with `make -C hydrainfer_amd/csrc mix`. "
                                 "There is no fallback path.")
@@ -430,7 +443,7 @@ def mix_lib() -> ctypes.CDLL:
             fn.argtypes = argtypes
         _load_front(handle)
         _mix = handle
-    return _mix
+        return handle
 
 
 FRONT_PATH = os.path.join(_HERE, "lib", "libhydra_front.so")
@@ -438,19 +451,28 @@ _front = _front_of = None
 
 
 def _load_front(handle: ctypes.CDLL) -> None:
+    """The module is built against one torch and one version of the argument blocks; what it was not built for it does not serve, and its
+    calls go on in Python, which launches the same kernels."""
     global _front, _front_of
-    if not os.path.exists(FRONT_PATH):
-        raise HydraHipError(f"{FRONT_PATH} is missing: build it with `make -C hydrainfer_amd/csrc mix`. There is no fallback path.")
-    loader = importlib.machinery.ExtensionFileLoader("_hydra_front", FRONT_PATH)
-    module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_hydra_front", FRONT_PATH, loader=loader))
-    loader.exec_module(module)
+    here = f"ABI {HXM_ABI_VERSION}, torch {torch.__version__}, Python {sys.version_info[0]}.{sys.version_info[1]}"
+    try:
+        built_for = ctypes.CDLL(FRONT_PATH).hydra_front_built_for
+        built_for.restype = c_char_p
+        if built_for().decode() != here:
+            raise ImportError(f"built for {built_for().decode()}, this is {here}")
+        loader = importlib.machinery.ExtensionFileLoader("_hydra_front", FRONT_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_hydra_front", FRONT_PATH, loader=loader))
+        loader.exec_module(module)
+    except (ImportError, OSError, AttributeError) as e:
+        warnings.warn(f"{FRONT_PATH} is not used ({e}): the mixers' calls take longer on the host.  Build it with `make -C hydrainfer_amd/csrc front`.")
+        return
     module.bind({name: ctypes.cast(getattr(handle, name), c_void_p).value for name in module.entries}, mix_check)
     _front, _front_of = module, handle
 
 
 def front():
     """The operators' native side (csrc/front.cpp: the calls of the mixers without the interpreter between their checks, allocations
-    and launch), bound to the library that mix_lib() opens.  None where something else stands in for that library."""
+    and launch), bound to the library that mix_lib() opens.  None where something else stands in for that library, or the module is not there."""
     return _front if mix_lib() is _front_of else None
 
 

@@ -539,6 +539,13 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_hydra_front", nullptr, -1, method
 
 }  // namespace
 
+// What this was compiled for: the binding asks before it takes this for a module.
+#define TEXT(x) #x
+#define TEXT_OF(x) TEXT(x)
+extern "C" __attribute__((visibility("default"))) const char* hydra_front_built_for() {
+  return "ABI " TEXT_OF(HXM_ABI_VERSION) ", torch " HYDRA_TORCH_VERSION ", Python " TEXT_OF(PY_MAJOR_VERSION) "." TEXT_OF(PY_MINOR_VERSION);
+}
+
 PyMODINIT_FUNC PyInit__hydra_front() {
   PyObject* m = PyModule_Create(&module);
   if (!m) return nullptr;
