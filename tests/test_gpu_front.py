@@ -112,6 +112,24 @@ def test_experts(T, act):
     both(lambda: moe_combine(y, row_of, weights, shared=shared, shared_gate=gate[:, 1], identity=h if act == "glu" else None))
 
 
+def refused(call):
+    """call() is refused, and by way of the native side in the words that Python has by itself."""
+    from hydrainfer_amd import _lib
+    lib = _lib.mix_lib()
+    assert _lib.front() is not None
+
+    class StandIn:
+        def __getattr__(self, name):
+            return getattr(lib, name)
+
+    said = []
+    for stand_in in (lib, StandIn()):
+        with mock.patch.object(_lib, "_mix", stand_in), pytest.raises(Exception) as e:
+            call()
+        said.append((e.type, str(e.value)))
+    assert said[0] == said[1] and issubclass(said[0][0], (_lib.HydraHipError, KeyError)), said
+
+
 def test_what_is_refused_stays_refused():
     from hydrainfer_amd import _lib
     from hydrainfer_amd._C.kernel.latent_attn import latent_attention
@@ -125,8 +143,77 @@ def test_what_is_refused_stays_refused():
                   dict(cache=cache[..., :32]), dict(sinks=rand(4)), dict(gate_pre=rand(2, 3)), dict(out=rand(2, 4, 32)), dict(q=q.cpu()), dict(max_q_len=0)):
         with pytest.raises(_lib.HydraHipError):
             latent_attention(**{**args, **wrong})
+        refused(lambda: latent_attention(**{**args, **wrong}))
     x, w = rand(2, 64, dtype=torch.float32), rand(4, 64, dtype=torch.float32)
     for call in (lambda: router_topk(x.bfloat16(), w, None, 2), lambda: router_topk(x, w, None, 9), lambda: moe_plan(b["seq"], 4), lambda: moe_plan(b["seq"][:, None].long(), 4),
                  lambda: grouped_linear(q[0], rand(1, 32, 64), b["q_cu"][:2], 9), lambda: moe_combine(q[0], b["seq"][:, None], x)):
         with pytest.raises(_lib.HydraHipError):
             call()
+        refused(call)
+
+
+def test_attention_refuses_in_the_same_words():
+    from hydrainfer_amd._C.kernel.biased_attn import biased_attention
+    b = batch([1, 1], [20, 3])
+    q, k, v = rand(2, 8, 64), rand(b["n_blocks"], BLOCK, 4, 64), rand(b["n_blocks"], BLOCK, 4, 64)
+    args = dict(q=q, key_cache=k, value_cache=v, vdim=64, tok_seq=b["seq"], positions=b["pos"], q_cu=b["q_cu"], block_table=b["table"], cu_block_lens=b["blocks"],
+                scale=0.125, max_q_len=1, max_kv_len=20)
+    biased_attention(**args)
+    for wrong in (dict(q=q.float()), dict(q=q[:, :, :32]), dict(value_cache=v.float()), dict(value_cache=v.transpose(1, 2)), dict(kv_heads=3), dict(kv_heads=16), dict(vdim=65),
+                  dict(vdim=0), dict(tok_seq=b["seq"][:1]), dict(positions=b["pos"].long()), dict(q_cu=b["q_cu"].float()), dict(block_table=b["table"].long()),
+                  dict(cu_block_lens=b["blocks"][:2]), dict(slopes=rand(8)), dict(slopes=rand(7, dtype=torch.float32)), dict(head_scale=rand(8)),
+                  dict(sinks=rand(16, dtype=torch.float32)[::2]), dict(mask="window"), dict(mask="none"), dict(mask="chunk", mask_size=-1), dict(form="other"), dict(q=q.cpu()),
+                  dict(key_cache=k[:, :8], value_cache=v[:, :8]), dict(q=q.half(), key_cache=k.half(), value_cache=v.half())):
+        refused(lambda: biased_attention(**{**args, **wrong}))
+
+
+def test_recurrences_refuse_in_the_same_words():
+    from hydrainfer_amd._C.kernel.recurrence import gated_recurrence
+    from hydrainfer_amd._C.kernel.seq_mix import state_scan
+    from hydrainfer_amd._C.kernel.stream_ops import SequenceState
+    b, T, H, G, K, V, f32 = batch([4, 3], [4, 3]), 7, 4, 2, 16, 8, torch.float32
+    state, slots = rand(3, 2, H * K * V + 4, dtype=f32), torch.tensor([2, 0], dtype=torch.int32, device="cuda")
+    seq = SequenceState(state, slots, b["seq"])
+    other = lambda **x: SequenceState(**{**dict(state=state, slots=slots, tok_seq=b["seq"]), **x})
+    q, k, v, decay, beta = rand(T, G * K), rand(T, G * K), rand(T, H * V), torch.rand((T, H), device="cuda"), torch.rand((T, H), device="cuda")
+    args = dict(mode="delta", q=q, k=k, v=v, decay=decay, seq=seq, offset=4, q_cu=b["q_cu"], positions=b["pos"], heads=H, qk_heads=G, dim=K, vdim=V, beta=beta)
+    state_scan(**args)
+    for wrong in (dict(mode="other"), dict(beta=None), dict(mode="bonus"), dict(q=q.half()), dict(q=q[:, 1:]), dict(q=q.t().contiguous().t()), dict(k=k[:3]), dict(v=v[:, ::2]),
+                  dict(decay=decay.bfloat16()), dict(decay=decay[:, :2]), dict(beta=beta[:2]), dict(vscale=rand(T, H)), dict(bonus=rand(H, dtype=f32)),
+                  dict(offset=-1), dict(offset=2 * state.shape[2]), dict(q_cu=b["q_cu"].long()), dict(positions=b["pos"][:3]), dict(seq=other(slots=slots[:1])),
+                  dict(seq=other(slots=slots.long())), dict(seq=other(tok_seq=b["seq"][:2])), dict(seq=other(state=state.bfloat16())), dict(seq=other(state=state[:, :, 1:])),
+                  dict(seq=other(state=state.cpu())), dict(v=v.cpu()), dict(heads=3), dict(qk_heads=3), dict(dim=300)):
+        refused(lambda: state_scan(**{**args, **wrong}))
+    p, bias, low, norm = rand(T, H * (2 * K + V)), rand(H * K, dtype=f32), torch.rand(H * K, device="cuda"), rand(V, dtype=f32)
+    args = dict(q_pre=p[:, :H * K], f_pre=p[:, H * K:2 * H * K], v=p[:, 2 * H * K:], f_bias=bias, low=low, norm_w=norm, eps=1e-5, seq=seq, state_row=1, q_cu=b["q_cu"],
+                positions=b["pos"], heads=H, dim=K, vdim=V, max_q_len=4)
+    gated_recurrence(**args)
+    for wrong in (dict(q_pre=args["q_pre"].half()), dict(q_pre=args["q_pre"].float()), dict(f_pre=args["f_pre"][:, 1:]), dict(v=args["v"][:2]), dict(f_bias=bias.bfloat16()),
+                  dict(low=low[1:]), dict(norm_w=norm[:3]), dict(state_row=2), dict(state_row=-1), dict(seq=other(state=state[:, :, :64].contiguous())),
+                  dict(seq=other(state=state.double())), dict(seq=other(slots=slots[:1])), dict(q_cu=b["q_cu"].long()), dict(positions=b["pos"].long()), dict(positions=b["pos"][:2]),
+                  dict(low=low.cpu()), dict(dim=17), dict(vdim=9)):
+        refused(lambda: gated_recurrence(**{**args, **wrong}))
+
+
+def test_experts_refuse_in_the_same_words():
+    from hydrainfer_amd._C.kernel.moe_mix import grouped_linear, moe_combine, moe_plan, router_topk
+    T, E, W, top, f32 = 5, 4, 64, 2, torch.float32
+    x, w = rand(T, W, dtype=f32), rand(E, W, dtype=f32)
+    weights, experts = router_topk(x, w, None, top)
+    seg, row_of, src = moe_plan(experts, E)
+    h, up, y = rand(T, W), rand(E, 96, W), rand(T * top, W)
+    refused(lambda: router_topk(x[:, 1:], w, None, top))
+    refused(lambda: router_topk(x, w.t(), None, top))
+    refused(lambda: router_topk(x, w, rand(E), top))
+    refused(lambda: router_topk(x, w, rand(E + 1, dtype=f32), top))
+    refused(lambda: router_topk(x, w, None, E + 1))
+    refused(lambda: moe_plan(experts.t(), E))
+    refused(lambda: moe_plan(experts.long(), E))
+    refused(lambda: moe_plan(experts.cpu(), E))
+    for wrong in (dict(x=h.float()), dict(x=h[:, 1:]), dict(w=up.transpose(1, 2)), dict(seg=seg[1:]), dict(seg=seg.long()), dict(src=src[1:]), dict(src=src.long()), dict(src=None),
+                  dict(act="other"), dict(act="glu", w=rand(E, 80, W)), dict(x=h.half(), w=up.half()), dict(x=h.cpu())):
+        refused(lambda: grouped_linear(**{**dict(x=h, w=up, seg=seg, max_rows=T * top, src=src), **wrong}))
+    for wrong in (dict(y=y.t()), dict(y=y.half()), dict(row_of=row_of.long()), dict(weights=weights.bfloat16()), dict(weights=weights[:, :1]), dict(shared=h[:3]), dict(shared=h.float()),
+                  dict(shared=h, shared_gate=rand(T)), dict(shared=h, shared_gate=rand(T + 1, dtype=f32)), dict(identity=h[:3]), dict(identity=h[:, 1:]), dict(identity=h.float()),
+                  dict(shared=h.cpu())):
+        refused(lambda: moe_combine(**{**dict(y=y, row_of=row_of, weights=weights), **wrong}))

@@ -86,12 +86,28 @@ def test_step_form(batch, H, G, D, V, mask, size, extra, divided):
     check([a for a, _ in batch], [b for _, b in batch], H, G, D, V, mask, size, extra, divided)
 
 
-# two and four runs of keys a workgroup, and two workgroups of four: runs without keys, rows that some of them do not see, partial row tiles
+# two and four runs of keys a workgroup, and three workgroups of four: runs without keys, rows that some of them do not see, partial row tiles
 @pytest.mark.parametrize("batch", [[(1, 140), (1, 1), (5, 64)], [(1, 250), (1, 3), (2, 33)], [(1, 511), (3, 40), (1, 129)], [(2, 600), (1, 65), (1, 1)]], ids=lambda b: f"{len(b)}x{max(b)}")
 @pytest.mark.parametrize("H, G, D, V", [(4, 1, 128, 128), (32, 8, 64, 64), (6, 2, 128, 64), (16, 16, 64, 128)])
 @pytest.mark.parametrize("mask, size, extra", [("causal", 0, "plain"), ("window", 300, "slopes"), ("chunk", 257, "cap"), ("causal", 0, "temperatures and sinks")])
 def test_step_form_merged_in_place(batch, H, G, D, V, mask, size, extra):
     check([a for a, _ in batch], [b for _, b in batch], H, G, D, V, mask, size, extra)
+
+
+# every way that a row tile's splits are dealt out: by twos and fours in one workgroup, two workgroups of four, and single waves with a launch that merges
+# (three and four splits of 257 - 383 row tiles, seven of just more than 128)
+@pytest.mark.parametrize("kv, H, G, D, V, splits", [
+    ([200] * 15 + [1], 32, 8, 128, 128, 4), ([127, 100, 3], 32, 8, 64, 64, 2), ([160, 128], 8, 8, 128, 64, 2), ([700, 512, 33] * 2, 32, 8, 64, 128, 12),
+    ([2048] * 3 + [1, 40, 1999] + [500] * 10, 32, 8, 128, 128, 8), ([700] * 39 + [1], 32, 8, 128, 128, 4), ([700] * 46 + [2], 32, 8, 64, 128, 3),
+    ([2101] + [700] * 15 + [64], 32, 8, 128, 64, 7), ([2600, 1, 300] + [90] * 15, 16, 8, 64, 64, 7)], ids=lambda v: f"{len(v)}x{max(v)}" if isinstance(v, list) else str(v))
+@pytest.mark.parametrize("extra", ["plain", "slopes", "temperatures and sinks"])
+def test_step_form_by_its_splits(kv, H, G, D, V, splits, extra):
+    import ctypes
+    from hydrainfer_amd import _lib
+    a = _lib.hxm_biased_attn_args(n_tokens=len(kv), n_seq=len(kv), n_heads=H, kv_heads=G, dim=D, vdim=V, block_size=BLOCK, max_q_len=1, dtype=_lib._DTYPE[torch.bfloat16])
+    n, floats = ctypes.c_int32(), ctypes.c_int64()
+    assert _lib.mix_lib().hxm_biased_attention_plan(ctypes.byref(a), max(kv), ctypes.byref(n), ctypes.byref(floats)) == 0 and n.value == splits
+    check([1] * len(kv), kv, H, G, D, V, "causal", 0, extra)
 
 
 # Rows that no token of a portion sees are never read: pages left of a window or chunk may have been given back, and the rows of the last

@@ -105,3 +105,36 @@ def test_rows_far_apart_still_go_in_chunks(stride, mode, per_channel):
     a = _lib.hxm_state_scan_args(q_dtype=HX_F32, k_dtype=HX_F32, v_dtype=HX_F32, n_tokens=1151, n_seq=1, heads=32, qk_heads=32, dim=128, vdim=128, mode=mode,
                                  decay_per_channel=per_channel, q_stride=stride, k_stride=stride, v_stride=stride)
     assert _lib.mix_lib().hxm_state_scan_workspace(ctypes.byref(a)) > 0
+
+
+@pytest.mark.parametrize("n_seq, q, heads, kv_heads, dim, vdim, kv, mask, size, splits", [
+    # one row tile a key head: two splits from four tiles of 32 keys on, four from six on, more where they take rounds of four
+    (1, 1, 32, 8, 128, 128, 64, 0, 0, 1), (1, 1, 32, 8, 128, 128, 127, 0, 0, 2), (1, 1, 32, 8, 128, 128, 160, 0, 0, 2), (1, 1, 32, 8, 128, 128, 161, 0, 0, 4),
+    (1, 1, 32, 8, 128, 128, 512, 0, 0, 4), (1, 1, 32, 8, 128, 128, 513, 0, 0, 8), (1, 1, 32, 8, 128, 128, 576, 0, 0, 12), (1, 1, 32, 8, 128, 128, 20000, 0, 0, 64),
+    (7, 1, 32, 8, 128, 128, 700, 0, 0, 12), (2, 16, 32, 8, 128, 128, 1500, 0, 0, 16), (1, 1, 8, 1, 64, 128, 700, 1, 300, 4), (1, 1, 8, 1, 64, 128, 700, 2, 60, 1),
+    # 64 row tiles and more of up to 2000 keys: four in the place of up to eleven
+    (8, 1, 32, 8, 128, 128, 704, 0, 0, 4), (8, 1, 32, 8, 128, 128, 768, 0, 0, 12), (16, 1, 32, 8, 128, 128, 2000, 0, 0, 4), (16, 1, 32, 8, 128, 128, 2001, 0, 0, 8),
+    # more than 128 row tiles behind longer keys: seven, and four where there would be seven
+    (17, 1, 32, 8, 128, 128, 2000, 0, 0, 4), (17, 1, 32, 8, 128, 128, 2001, 0, 0, 7), (18, 1, 32, 8, 128, 128, 2100, 0, 0, 7), (19, 1, 32, 8, 128, 128, 2100, 0, 0, 4),
+    # 257 - 383 row tiles: as many as there are waves for
+    (32, 1, 32, 8, 128, 128, 700, 0, 0, 4), (33, 1, 32, 8, 128, 128, 700, 0, 0, 4), (42, 1, 32, 8, 128, 128, 700, 0, 0, 4), (43, 1, 32, 8, 128, 128, 700, 0, 0, 3),
+    (47, 1, 32, 8, 128, 128, 700, 0, 0, 3), (48, 1, 32, 8, 128, 128, 700, 0, 0, 4), (64, 1, 32, 8, 128, 128, 700, 0, 0, 2), (127, 1, 32, 8, 128, 128, 700, 0, 0, 2),
+    (128, 1, 32, 8, 128, 128, 700, 0, 0, 1),
+    # portions of 64 rows and more: only few of them behind many keys; heads of other sizes: 2048 waves
+    (1, 100, 32, 8, 128, 128, 2000, 0, 0, 4), (1, 100, 32, 8, 128, 128, 1000, 0, 0, 1), (1, 1, 32, 8, 96, 96, 2000, 0, 0, 31)])
+def test_splits_of_attention(n_seq, q, heads, kv_heads, dim, vdim, kv, mask, size, splits):
+    import torch
+    from hydrainfer_amd import _lib
+    a = _lib.hxm_biased_attn_args(n_tokens=n_seq * q, n_seq=n_seq, n_heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim, block_size=16, mask_kind=mask, mask_size=size,
+                                  max_q_len=q, dtype=_lib._DTYPE[torch.bfloat16])
+    n, floats = ctypes.c_int32(), ctypes.c_int64()
+    plan = lambda: _lib.mix_lib().hxm_biased_attention_plan(ctypes.byref(a), kv, ctypes.byref(n), ctypes.byref(floats))
+    tiles = n_seq * kv_heads * ((q * (heads // kv_heads) + 15) // 16)
+    assert plan() == 0 and n.value == splits
+    assert floats.value == (0 if splits == 1 else tiles * splits * 16 * ((vdim + 15) // 16 * 16 + 2))
+    # no splits for what the forms with splits do not serve
+    for name, value in (("form", 1), ("dtype", 0), ("max_q_len", 0), ("dim", 260), ("vdim", 36)):
+        before = getattr(a, name)
+        setattr(a, name, value)
+        assert plan() == 0 and (n.value, floats.value) == (1, 0)
+        setattr(a, name, before)
