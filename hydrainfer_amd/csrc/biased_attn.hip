@@ -1020,18 +1020,18 @@ int launch_wide(const hxm_biased_attn_args& a, hipStream_t s) {
 
 // ---------------------------------------------------------------------------------------------------------------
 // Step form (bfloat16, fewer than 64 rows of a key head or few row tiles behind many keys, key and value heads of 64 or 128,
-// pages of whole 16-row groups): a workgroup is one wave with 16 rows of ONE (sequence, key head) and one run of its keys, in tiles of 32.  Bound by memory: the
+// pages of whole 16-row groups): a wave takes 16 rows of ONE (sequence, key head) and one run of its keys, in tiles of 32.  Bound by memory: the
 // tile form asks for a key's row in 64-byte pieces, sixteen rows an instruction, and has one chunk in flight; here rows go whole
 // from the paged cache to LDS, the next tile's while this one's are awaited — no register holds them and no barrier is needed.
-// 32 KB of LDS at heads of 128: five waves a CU, 80 to 160 KB in flight.  Products are 16 x 16 x 32 and swapped, S^T = K Q^T,
+// A wave's two images are 32 KB of LDS at heads of 128 (64: 16): five waves a compute unit by themselves, one workgroup of four.  Products are 16 x 16 x 32 and swapped, S^T = K Q^T,
 // O^T += V^T P^T: a row of the softmax is one lane, its weights stay in their registers.  16-byte chunk x of row r sits at
 // x ^ swz(r): rows r and 15 - r share a 32-byte place (their chunks turned), so that a pass of a 16-byte read and a transposing
 // read (eight rows, 32 bytes each) both reach every bank once.
-// Two or four runs of a row tile's keys are a workgroup's, a wave each, merged through LDS where the images were; only more of them go through memory
-// and a second launch.  32 tokens of 1025 - 2047 keys 46.7 us with it, 43 without, 20 of 55 - 253 9.6 and 6.7, 224 row tiles of 1500 45.9 and 35.3 (with five
-// splits); 15 % in the mean of 50 batches.
-// Measured, 32 heads of 128 on 8 key heads, kernel and merge: 32 tokens of 1025 - 2047 keys 48 + 8 us in the tile form, 36 + 4 here
-// (5.5 TB/s); 128 tokens of 500 - 1500 keys 163 us and 109; 32 tokens, 2 key heads 57 us and 24; 16 tokens behind 4000 keys
+// Two or four runs of a row tile's keys are a workgroup's, a wave each, merged through LDS where the images were; only more of them, and three or seven, go
+// through memory and a second launch.  32 tokens of 1025 - 2047 keys 46.7 us with that launch, 43 in workgroups of four, 20 of 55 - 253 9.6 and 6.7, 224 row tiles of
+// 1500 45.9 (five splits) and 35.3; 15 % in the mean of 50 batches.
+// Measured, 32 heads of 128 on 8 key heads: 32 tokens of 1025 - 2047 keys 56 us in the tile form and its merge, 43 here (4.7 TB/s, with the way to the first
+// keys); by single waves and the launch that merges: 128 tokens of 500 - 1500 keys 163 us and 109; 32 tokens, 2 key heads 57 us and 24; 16 tokens behind 4000 keys
 // 93 us (tile), 79 (wide) and 29.
 // ---------------------------------------------------------------------------------------------------------------
 template <int D, int V, bool MODS, int W>      // MODS: slopes or a soft cap; W: waves, a split each
@@ -1506,7 +1506,8 @@ extern "C" int hxm_biased_attention(const hxm_biased_attn_args* args, void* stre
   return hxm::check_launch();
 }
 
-// Key splits: enough waves to fill the chip when the launch has few row tiles, at least two 32-key chunks a split.  Heads of 64 and 128:
+// Key splits: enough waves to fill the chip when the launch has few row tiles, two 32-key chunks a split and more (before the number is rounded up to fours:
+// of 576 keys' twelve splits three stay without keys).  Heads of 64 and 128:
 // five waves of the step form fill a CU (1024 and 2048 waves: 32 tokens of 1025 - 2047 keys 39.5 and 41.9 us, 128 of 500 - 1500 109
 // and 116); portions of 64 rows and more go undivided to the wide form unless they are few and their keys many (one portion behind
 // keys, 32 heads on 8 key heads, wide and split: 32 tokens behind 2000 44.8 and 24.9 us, 100 behind 2000 46.4 and 36.4, 100 behind

@@ -553,9 +553,10 @@ int64_t chunk_scan_workspace(const ChunkScanArgs& a) {
   // 64 x 64: one of 1151 92 86, 4 of 1000 83 86; gated form, 128 x 128, 32 heads: 4 of 64 21 23, 4 of 256 57 53; 64 x 64: 4 of 1000 115 97, 8 of 512 71
   // 83; bonus form, 128 x 128, 16 heads: 4 of 1000 162 121, 8 of 512 95 98; 64 x 64, 8 heads: 8 of 512 52 55; a decay per channel, 128 x 64, 32 heads: 4 of 256 45
   // 39, 8 of 512 89 123.
-  // (One decay a head and more than 64 key channels: fitted against one launch of sixteen tokens at a time.  Against that of chunk_head.hip two are as fast or
-  // faster up to 128 workgroups — one of 1100, 16 heads of 128 x 128: delta rule 138 and 157, decayed sum 87 and 98 — and behind it about 256: 4 of 1000, 32
-  // heads of 128 x 64: 177 and 165, 108 and 101.  The line stays: the decayed sum's results are less off in two, 0.78 and 0.86 e-7.)
+  // (One decay a head: fitted against one launch of sixteen tokens at a time, which float q and k of a decayed sum still take.  Against chunk_head.hip, thirty-two
+  // at a time, two launches are as fast or faster up to 128 workgroups — one of 1100, 16 heads of 128 x 128: delta rule 138 and 157, decayed sum of bfloat16 q
+  // and k 87 and 98 — and up to 7 % behind at 256: 4 of 1000, 32 heads of 128 x 64: 177 and 165, 108 and 101.  Not fitted anew for those; the decayed sum's
+  // results are less off in two, 0.78 and 0.86 e-7.)
   // (And one launch takes 20 us: shorter calls are bound by their caller, who would have to ask for a workspace: 19.2 and 21.7 us.)
   struct Line { double few, many, cost, one; };           // few: keys dealt to four waves; one: us a chunk in one launch
   const bool wide = a.K > 64;

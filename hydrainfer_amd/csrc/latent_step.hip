@@ -3,7 +3,7 @@
 // a wave 16 rows of token and head for all of a tile's keys: with 8 to 32 rows a token two or three of its four waves stand idle, the others go
 // through keys, softmax and values alone, and what they wait for in front of the first product are five loads behind each other.
 // Here a tile is 64 keys, in the scores wave w takes 16 of them (for 16 heads), in the values a quarter of the columns; scores
-// pass between the two through LDS as floats, so that every wave makes the weights it needs itself and a tile costs two barriers.
+// pass between the two through LDS as floats, so that every wave makes the weights it needs itself and a tile costs two barriers, and one more where another tile comes into its place.
 // A weight enters the second product as the sum of two bfloat16 numbers (p = hi + lo, relative 2^-17): it costs matrix time that is idle here and the
 // results' own rounding is all that is left.
 // Latency bounds it: the way to the first tile, then for each tile keys, softmax and values in turn, and the launch that merges.  Measured, 32 tokens

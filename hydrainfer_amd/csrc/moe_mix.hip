@@ -401,8 +401,8 @@ __global__ __launch_bounds__(256) void grouped_linear_kernel(typename A::storage
 // and TN output columns.  The rows' inputs (gathered through src) and the expert's weight rows go straight from memory to LDS
 // (no registers, no writes by the waves) in slices of 64 k and NS slots; every wave multiplies its (TM / WGM) x (TN / WGN)
 // part with 16x16x32 MFMAs: lane l holds k 8 (l / 16) .. + 7 of row (A) or column (B) l % 16, the accumulator's lane l
-// column l % 16 of rows 4 (l / 16) .. + 3.  Half a slice is multiplied while the other half's operands are read from LDS, one
-// read between four products; the one workgroup barrier of a slice stands between its halves, so that a wave always has
+// column l % 16 of rows 4 (l / 16) .. + 3.  Half a slice is multiplied while the other half's operands are read from LDS, a
+// read between two products in tiles of 256 rows, one in those of 128 and of 64 x 128 (narrower tiles have fewer products than reads, in the compiler's order); the one workgroup barrier of a slice stands between its halves, so that a wave always has
 // products to issue behind it.
 // With few rows an expert it is bound by the weights: those of an expert with one row tile are read past the caches (128 rows of 16
 // experts, 2 x 2752 outputs of 4096 and back: 162 + 75 us through registers in tiles of 128 x 128 and padded LDS rows, 115 + 58 us here,
