@@ -479,12 +479,22 @@ def test_small_gates_are_as_exact_as_large_ones(max_q_len):
 
 
 # One decay a head in one launch (csrc/chunk_head.hip): portions at the edges of its chunks of 32 tokens and their tiles of 16, channels that fill no
-# tile and no vector, q and k in one part and in three
+# tile and no vector, q and k in one part (float ones: the test below; here they go sixteen tokens at a time)
 @pytest.mark.parametrize("lens", [[13, 16, 17, 31, 32, 0, 33, 48, 49, 64, 65, 97] * 2, [47, 1, 15, 96]], ids=["edges", "few"])
 @pytest.mark.parametrize("form, K, V", [("delta", 128, 128), ("delta", 100, 34), ("delta", 65, 68), ("decay", 128, 64), ("decay", 64, 130), ("decay", 100, 7), ("decay", 17, 64)])
 @pytest.mark.parametrize("types, pad", [("bf16", 4), ("f32", 4), ("mixed", 3)])
 def test_chunks_of_two_tiles(lens, form, K, V, types, pad):
     _through_a_scan(lens, K, V, form, False, types, pad)
+
+
+# The same of float q and k under the delta rule, which take chunks of 32 where portions fill them in the mean (17 - 32 tokens, 49 - 64, and more than 80)
+@pytest.mark.parametrize("lens", [[13, 16, 17, 31, 32, 33, 48, 5], [49, 64, 65, 97, 33, 48, 1], [81, 96, 97]], ids=["short", "two", "three"])
+@pytest.mark.parametrize("K, V", [(128, 128), (100, 34), (65, 68)])
+@pytest.mark.parametrize("types, pad", [("f32", 4), ("mixed", 3)])
+def test_chunks_of_two_tiles_in_three_parts(lens, K, V, types, pad):
+    mean = sum(lens) / len(lens)
+    assert 1.7 * -(-mean // 32) < -(-mean // 16)
+    _through_a_scan(lens, K, V, "delta", False, types, pad)
 
 
 # rows so far apart that chunks of thirty-two tokens do not address them: in chunks of sixteen all the same

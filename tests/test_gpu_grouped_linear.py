@@ -95,6 +95,15 @@ def test_grouped_linear_from_tile_to_tile(rows, n, k, act):
     _check(rows, n, k, act, False)
 
 
+# the same with rows enough that tiles of 256 are chosen for two slices too: the walk starts and ends in the first turn of its slots
+@pytest.mark.parametrize("rows", [[500, 520], [1000, 20], [1, 1023]])
+@pytest.mark.parametrize("n, k, act", [(11040, 128, "glu"), (11048, 128, "none"), (11048, 192, "relu2"), (33088, 192, "glu")])
+def test_grouped_linear_from_tile_to_tile_with_few_slices(rows, n, k, act):
+    from hydrainfer_amd import _lib
+    assert _lib.mix_lib().hxm_grouped_linear_tile_rows(sum(rows), len(rows), n, k) == 256
+    _check(rows, n, k, act, False)
+
+
 # the same with more experts than a wave has lanes, some of them without rows
 def test_grouped_linear_from_tile_to_tile_of_many_experts():
     from hydrainfer_amd import _lib
