@@ -520,10 +520,10 @@ typedef struct hxm_state_scan_args {
 } hxm_state_scan_args;
 
 /* The recurrence of one matrix state S [dim, vdim] per head and sequence, continued from and left in the sequence's slot: token by
- * token in float, or (portions of prompts, dim <= 128) sixteen tokens at a time as float matrix products, which round in other places
- * and are no further from the exact result.  What is not finite in a token's operands shows from that token on, in either form, and a
- * value, scale or write strength in its own columns only; sixteen tokens at a time it may come out as NaN where a token at a time left
- * an infinity.  dim <= 256. */
+ * token in float, or (portions of prompts, dim <= 128) sixteen or 32 tokens at a time as matrix products of floats or of their bfloat16
+ * parts, which round in other places and are no further from the exact result.  What is not finite in a token's operands shows from that
+ * token on, in any form, and a value, scale or write strength in its own columns only; sixteen or 32 tokens at a time it may come out as
+ * NaN where a token at a time left an infinity.  dim <= 256. */
 /* Floats by sizes, types and mode; 0: none.  For every sixteen tokens and head (and one more of each sequence), up to 64 key channels and up to 128: 2752 and
  * 5120 with a decay per channel or gates, 3392 and 6400 in the bonus form, 368 with a decay per head, 688 for the delta rule (of more than 64);
  * never more than 2^28 (1 GiB).  A call without it, or with less, takes one launch. */
