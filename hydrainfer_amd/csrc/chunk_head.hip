@@ -16,7 +16,9 @@
 // What bounds it: the vector ALU of a SIMD, which a consumer (430 instructions a chunk under the delta rule: parts, sums, results) and a producer (850:
 // parts of rows, products of decays, the substitution) share, and which does not run beside the products of its own wave.  Of a chunk's 4.6 us
 // 1.3 are matrix products.
-// Measured, one launch of sixteen tokens at a time in float and this one, us: delta rule, 128 x 128, 32 heads, 4 portions of 797 - 1151 tokens 191 and
+// Rows are read eight bytes at a time (two reads made one by the compiler bring a quarter of their bytes a cycle) and parts made by v_dot2_f32_bf16: delta rule, 128 x 128, 32
+// heads, 4 portions of 797 - 1151 tokens 166.5 -> 163.0 us, decayed sum of bfloat16 q and k, 3 of 168 - 723, 128 x 64 65.3 -> 63.7, 2 of 28 - 130 18.4 -> 17.6.
+// Measured before that, one launch of sixteen tokens at a time in float and this one, us: delta rule, 128 x 128, 32 heads, 4 portions of 797 - 1151 tokens 191 and
 // 169, 12 of 300 - 900 348 and 309, 16 of 60 55.6 and 55.6; decayed sum, 128 x 128, 32 heads, 4 of 797 - 1151 145 and 103, 12 of 300 - 900 263 and 190,
 // one of 100 19.8 and 17.1, 64 x 64 93 and 83.  Results' error against 64 bits (2-norm, 400 and 250 tokens, 1e-7): delta rule 1.08 and 1.00,
 // decayed sum 128 x 128 0.867 and 0.863, 64 x 64 0.79 and 0.76; states 0.77 and 0.72, 0.73 and 0.62, 0.72 and 0.64.
@@ -42,14 +44,31 @@ __device__ __forceinline__ f32x4 mma_parts(u16x8 a, u16x8 b, f32x4 c) {
 }
 __device__ __forceinline__ u16x8 both(u16x4 a, u16x4 b) { return u16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}; }
 
-// Four floats in three parts
+// Four floats in three parts, two at a time: one conversion makes both numbers' parts, and v_dot2_f32_bf16 takes a part from its float (1 and 0 times the two parts, exact,
+// subnormal numbers kept): 7 instructions a pair, 11 with shifts and subtractions.  Beside an infinite part the neighbour's lower ones are no numbers then, which is
+// nothing where neighbours are summed over (channels of a query, keys and tokens of a value channel: that sum holds the infinity as well, and total_of is made for
+// it); keys, whose channels are rows of the state, are kept APART.
+template <bool APART = false>
 __device__ __forceinline__ void split(f32x4 x, u16x4 (&part)[3]) {
+  typedef __bf16 pair_t __attribute__((ext_vector_type(2)));
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  uint32_t first = 0x0000bf80u, second = 0xbf800000u;     // (-1, 0) and (0, -1); in registers: as an inline constant the second would be another number
+  asm("" : "+s"(first), "+s"(second));
 #pragma unroll
   for (int p = 0; p < 3; ++p)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      part[p][e] = BF16::from_float(x[e]);
-      if (p < 2) x[e] -= BF16::to_float(part[p][e]);
+    for (int e = 0; e < 4; e += 2) {
+      const pair_t two = __builtin_convertvector((f32x2{x[e], x[e + 1]}), pair_t);
+      const uint32_t bits = __builtin_bit_cast(uint32_t, two);
+      part[p][e] = (u16)bits;
+      part[p][e + 1] = (u16)(bits >> 16);
+      if (p < 2 && APART) {
+        x[e] -= __builtin_bit_cast(float, bits << 16);
+        x[e + 1] -= __builtin_bit_cast(float, bits & 0xffff0000u);
+      } else if (p < 2) {
+        x[e] = __builtin_amdgcn_fdot2_f32_bf16(two, __builtin_bit_cast(pair_t, first), x[e], false);
+        x[e + 1] = __builtin_amdgcn_fdot2_f32_bf16(two, __builtin_bit_cast(pair_t, second), x[e + 1], false);
+      }
     }
 }
 
@@ -127,11 +146,15 @@ __global__ __launch_bounds__(512) void chunk_head32_kernel(ChunkScanArgs a) {
   auto tokens = [&](int chunk) { return smem + 2 * I::kBytes + chunk % 3 * I::kTokens; };
   auto rows_of = [&](int chunk) { return min(CW, n_tok - chunk * CW); };
   // 16 rows (row m of tile u) times 32 channels of an operand in parts; as A and as B operand alike
+  // (two reads of eight bytes from addresses that the compiler does not know to be near each other: it would make one ds_read2_b64 of them, which
+  // brings 64 bytes a cycle where the two bring 230)
+  int half_at[2] = {place_of(m) * I::kRow + 8 * g, place_of(m) * I::kRow + 8 * g + 32};
+  asm volatile("" : "+v"(half_at[1]));
   auto parts_at = [&](const char* planes, int u, int kb, u16x8 (&x)[NP]) __attribute__((always_inline)) {
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
-      const char* at = planes + p * I::kPlane + (16 * u + place_of(m)) * I::kRow + 64 * kb + 8 * g;
-      x[p] = both(*reinterpret_cast<const u16x4*>(at), *reinterpret_cast<const u16x4*>(at + 32));
+      const int at = p * I::kPlane + 16 * u * I::kRow + 64 * kb;
+      x[p] = both(*reinterpret_cast<const u16x4*>(planes + half_at[0] + at), *reinterpret_cast<const u16x4*>(planes + half_at[1] + at));
     }
   };
 
@@ -206,7 +229,7 @@ __global__ __launch_bounds__(512) void chunk_head32_kernel(ChunkScanArgs a) {
           rest_at();
         }
         add_products(rows[kb & 1], sp[kb & 1], sum);
-        constexpr int products = NX * (NP == 1 ? 3 : 6), reads = NX * NP;
+        constexpr int products = NX * (NP == 1 ? 3 : 6), reads = 2 * NX * NP;
 #pragma unroll
         for (int i = 0; i < products; ++i) {
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -404,7 +427,7 @@ __global__ __launch_bounds__(512) void chunk_head32_kernel(ChunkScanArgs a) {
   // (strides below 2^28: what chunk_scan.hip sends here)
   auto at_row = [&](auto* base, int r, int64_t stride) __attribute__((always_inline)) {
     typedef std::remove_pointer_t<decltype(base)> E;
-    return reinterpret_cast<E*>(reinterpret_cast<uintptr_t>(base) + (uint64_t)(uint32_t)r * (uint32_t)(stride * sizeof(E)));
+    return reinterpret_cast<E*>(reinterpret_cast<const char*>(base) + (uint64_t)(uint32_t)r * (uint32_t)(stride * sizeof(E)));
   };
   auto fetch = [&](Set& s, int chunk) __attribute__((always_inline)) {
     if (chunk >= n_chunks) return;                        // (what is there stays, and nobody looks at it)
@@ -426,7 +449,7 @@ __global__ __launch_bounds__(512) void chunk_head32_kernel(ChunkScanArgs a) {
   };
   // (rows past the portion repeat its last one: the values and write strengths there are none)
   const bool whole = a.K == KP;
-  auto planes = [&](char* to, const Piece<QK, 4, VEC>& p, int at) __attribute__((always_inline)) {
+  auto planes = [&](char* to, const Piece<QK, 4, VEC>& p, int at, auto apart) __attribute__((always_inline)) {
     const int col = qk_col(at);
     f32x4 x;
 #pragma unroll
@@ -440,7 +463,7 @@ __global__ __launch_bounds__(512) void chunk_head32_kernel(ChunkScanArgs a) {
       *reinterpret_cast<u16x4*>(dst) = u16x4{BF16::from_float(x[0]), BF16::from_float(x[1]), BF16::from_float(x[2]), BF16::from_float(x[3])};
     } else {
       u16x4 part[3];
-      split(x, part);
+      split<decltype(apart)::value>(x, part);
 #pragma unroll
       for (int i = 0; i < 3; ++i) *reinterpret_cast<u16x4*>(dst + i * I::kPlane) = part[i];
     }
@@ -450,8 +473,8 @@ __global__ __launch_bounds__(512) void chunk_head32_kernel(ChunkScanArgs a) {
     char* im = image(chunk);
 #pragma unroll
     for (int i = 0; i < NQ; ++i) {
-      planes(im + I::kQ, s.q[i], i);
-      planes(im + I::kK, s.k[i], i);
+      planes(im + I::kQ, s.q[i], i, std::false_type());
+      planes(im + I::kK, s.k[i], i, std::true_type());
     }
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
