@@ -86,6 +86,40 @@ __device__ __forceinline__ float row16_max(float v) {
   return v;
 }
 
+// x[0 .. 31] of every lane: lane l ends with the sum over the wave of x[l / 2].  Every step keeps half of the values and adds
+// the partner's share of them: 32 values in 75 instructions instead of 32 x 6.
+template <int CTRL>
+__device__ __forceinline__ float pair_sum(float keep, float give) { return keep + dpp_move<CTRL>(give); }
+__device__ __forceinline__ float swap32_sum(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+  const unsigned lo = r[0], hi = r[1];                    // (a bit cast of r[1] itself is taken from r[0] by this compiler)
+  return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+}
+__device__ __forceinline__ float swap16_sum(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+  const unsigned lo = r[0], hi = r[1];
+  return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+}
+__device__ __forceinline__ float transpose_sum32(const float* x, int lane) {
+  float y[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) y[i] = swap32_sum(x[i], x[i + 16]);      // (lanes 32 .. hold the second of the two)
+#pragma unroll
+  for (int i = 0; i < 8; ++i) y[i] = swap16_sum(y[i], y[i + 8]);
+  const bool b8 = lane & 8, b4 = lane & 4, b2 = lane & 2;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) y[i] = pair_sum<kDppMirror>(b8 ? y[i + 4] : y[i], b8 ? y[i] : y[i + 4]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) y[i] = pair_sum<kDppHalfMirror>(b4 ? y[i + 2] : y[i], b4 ? y[i] : y[i + 2]);
+  y[0] = pair_sum<kDppXor2>(b2 ? y[1] : y[0], b2 ? y[0] : y[1]);
+  return pair_sum<kDppXor1>(y[0], y[0]);
+}
+__device__ __forceinline__ float wave_total(float v) {
+  v = row16_sum(v);
+  v = swap16_sum(v, v);
+  return swap32_sum(v, v);
+}
+
 // A workgroup barrier that orders LDS traffic only: global loads and stores that are in flight (a prefetch for the next
 // step, results on their way out) are not waited for, as __syncthreads() would.  For exchanges through LDS alone.
 __device__ __forceinline__ void lds_barrier() {

@@ -252,6 +252,67 @@ __global__ __launch_bounds__(1024) void router_few_kernel(const float* __restric
   choose_top<2>(z, lane, E, top, weights + t * top, experts + t * top);
 }
 
+// Four tokens a workgroup, products on the vector ALU: a wave takes 256 neighbouring k (1 KB of every row) of all four tokens and of NG groups of eight experts, a lane
+// sums its k of 32 pairs of a token and an expert, and a transposing sum over the wave leaves one of them in every second lane.
+// What bounds the form with sixteen tokens a workgroup is what one CU gets from memory (about 25 bytes a ns: 256 KB of tokens are 10 us), with most CUs idle up to a few
+// thousand tokens; here every CU has rows, and the experts' come from its L2 a quarter as often as with a workgroup a token.  Above (or a workgroup a token, *) and
+// here, us: 16 experts of 4096, 32 tokens 6.6* 6.2, 400 11.7* 7.0, 1000 17.5 8.3, 2500 18.9 15.5, 4000 23.9 25.2; of 2048, 1000 10.6 6.4; 8 experts of 4096, 4000 22.5
+// 18.7; 32 of 4096, 400 18.9* 13.3, 1000 24.8 14.5, 1500 25.0 25.4.
+template <int NG, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void router_four_kernel(const float* __restrict__ x, int64_t x_stride, const float* __restrict__ w, const float* __restrict__ bias,
+                                                                int64_t n_tokens, int64_t K, int E, int top, float* __restrict__ weights, int32_t* __restrict__ experts) {
+  __shared__ float sums[WAVES][4][8 * NG];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int64_t t0 = (int64_t)blockIdx.x * 4;
+  float acc[NG][32];
+#pragma unroll
+  for (int n = 0; n < NG; ++n)
+#pragma unroll
+    for (int i = 0; i < 32; ++i) acc[n][i] = 0.f;
+  for (int64_t k0 = 256 * wave; k0 < K; k0 += 256 * WAVES) {
+    const bool in = k0 + 4 * lane < K;
+    const int64_t k = in ? k0 + 4 * lane : 0;             // (past the end: the row's start, and not used)
+    f32x4 xv[4], wv[NG][8];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) xv[t] = *reinterpret_cast<const f32x4*>(x + (t0 + t < n_tokens ? t0 + t : n_tokens - 1) * x_stride + k);
+#pragma unroll
+    for (int n = 0; n < NG; ++n)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) wv[n][e] = *reinterpret_cast<const f32x4*>(w + (int64_t)(8 * n + e < E ? 8 * n + e : E - 1) * K + k);
+    if (!in) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) xv[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int n = 0; n < NG; ++n)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) wv[n][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int n = 0; n < NG; ++n)
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) acc[n][8 * t + e] = __builtin_fmaf(xv[t][i], wv[n][e][i], acc[n][8 * t + e]);
+  }
+#pragma unroll
+  for (int n = 0; n < NG; ++n) {
+    const float sum = transpose_sum32(acc[n], lane);
+    if ((lane & 1) == 0) sums[wave][lane >> 4][8 * n + (lane >> 1 & 7)] = sum;
+  }
+  __syncthreads();
+  if (wave >= 4 || t0 + wave >= n_tokens) return;
+  float z[1] = {-INFINITY};
+  if (lane < E) {
+    float s = 0.f;
+#pragma unroll
+    for (int v = 0; v < WAVES; ++v) s += sums[v][wave][lane];
+    z[0] = s + (bias ? bias[lane] : 0.f);
+  }
+  choose_top<1>(z, lane, E, top, weights + (t0 + wave) * top, experts + (t0 + wave) * top);
+}
+
 // one workgroup of 1024 threads: histogram, exclusive scan, scatter, all through LDS counters
 __global__ __launch_bounds__(1024) void moe_plan_kernel(const int32_t* __restrict__ experts, int64_t n, int top, int E,
                                                         int32_t* __restrict__ seg, int32_t* __restrict__ row_of,
@@ -952,6 +1013,28 @@ extern "C" int hxm_router_topk(const float* x, int64_t x_stride, const float* w,
   if (x_stride < k_dim || x_stride % 4 || !aligned16(x) || !aligned16(w)) return HX_ERR_STRIDE;
   const dim3 grid((unsigned)((n_tokens + 15) / 16));
   hipStream_t s = (hipStream_t)stream;
+  // Four tokens a workgroup: up to 8 experts always, up to 16 and 32 while that reads the experts' rows from L2 less than about 750 and 256 times and the rows are long
+  // enough to fill its waves; but a workgroup a token where it is the faster one by a little (us, here and there: 16 experts of 2048, 32 tokens 5.1 4.8, 400 5.4 7.7; 32 of
+  // 2048, 128 8.2 7.1, of 1024 6.3 7.1).  Short rows: 16 of 256, 8 tokens 4.0 here and 3.8 below, 2500 5.2 and 4.7; of 512, 1000 4.5 and 5.3; 32 of 512, 8 5.6 and 5.1.
+  // Four waves of up to 512 registers are fewer rows in flight than eight, and more workgroups a CU: 16 of 4096, 400 tokens 8.0 and 7.0, 2500 15.5 and 17.8.
+  const bool four = n_experts <= 8    ? true
+                    : n_experts <= 16 ? (n_tokens <= 1024 ? k_dim >= 512 && (k_dim < 2048 || k_dim >= 4096 || n_tokens > 128) : n_tokens <= 3072 && k_dim >= 1024)
+                                      : n_experts <= 32 && n_tokens <= 1024 && k_dim >= 1024 && (k_dim < 2048 || n_tokens > 256);
+  if (four) {
+    const dim3 fours((unsigned)((n_tokens + 3) / 4));
+#define HXM_FOUR(NG_, W_) router_four_kernel<NG_, W_><<<fours, dim3(64 * W_), 0, s>>>(x, x_stride, w, bias, n_tokens, k_dim, n_experts, top, weights, experts)
+    if (n_experts <= 8) {
+      if (n_tokens <= 1024) HXM_FOUR(1, 8);
+      else HXM_FOUR(1, 4);
+    } else if (n_experts <= 16) {
+      if (n_tokens <= 1024) HXM_FOUR(2, 8);
+      else HXM_FOUR(2, 4);
+    } else {
+      HXM_FOUR(4, 4);
+    }
+#undef HXM_FOUR
+    return hxm::check_launch();
+  }
   // A workgroup a token while the CUs take them in one round, two where the form above takes long (above / a workgroup a token:
   // 16 experts of 4096, 256 tokens 17.4 / 7.3 us, 512 17.5 / 11.7, 1024 17.7 / 20.7; 32 of 2048, 512 13.9 / 12.0; 32 of 1024, 256 8.5 /
   // 7.5, 384 8.5 / 11.3; 128 of 1024, 256 21.1 / 20.5, 384 21.6 / 35.1).  Every token reads all experts' rows then, and short rows are

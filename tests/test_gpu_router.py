@@ -28,6 +28,13 @@ def test_router_forms(K, E, T, biased):
     assert bool(((weights.double() - want).abs() <= want * (2 * torch.expm1(2 * eps) + 1e-6) + 1e-30).all())
 
 
+# four tokens a workgroup: its groups of experts, ends of rows inside a wave's piece and inside a round of waves, and the lines at 128, 256, 1024 and 3072 tokens
+@pytest.mark.parametrize("K", [4, 516, 1028, 2052, 4100])
+@pytest.mark.parametrize("E, T", [(5, 1), (8, 1024), (8, 1027), (9, 130), (16, 1025), (16, 3071), (16, 3073), (17, 258), (32, 1024), (32, 1025)])
+def test_four_tokens_a_workgroup(K, E, T):
+    test_router_forms(K, E, T, True)
+
+
 # the combine (csrc/moe_mix.hip): rows in pieces of eight, four and single elements, on both sides of the 256 tokens up to which pieces are of four
 @pytest.mark.parametrize("W", [8, 1028, 2048, 2056, 4099])
 @pytest.mark.parametrize("T", [1, 256, 257])
