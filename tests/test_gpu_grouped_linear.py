@@ -86,6 +86,17 @@ def test_grouped_linear_by_eight_waves(rows, n, k, act, tile):
     _check(rows, n, k, act, False)
 
 
+# tiles of 128 x 192, 192 x 192 and 128 x 256 (the last three): up to a tile's rows and one more, columns that no tile divides, with a tail and without
+@pytest.mark.parametrize("rows, n, k, act, tile", [
+    ([129, 1, 128, 142], 8264, 520, "none", 128), ([100, 127, 173, 0], 8256, 520, "glu", 128), ([64, 192, 0, 144], 8264, 1096, "relu2", 128),
+    ([192, 193, 1, 126], 8264, 264, "none", 192), ([191, 321, 0, 0], 8256, 1096, "glu", 192), ([128, 129, 1, 127, 115], 11040, 520, "glu", 128),
+    ([255, 257, 128, 360], 6184, 520, "none", 128), ([385, 127, 0, 488], 6184, 320, "relu2", 128)])
+def test_grouped_linear_in_tiles_for_full_rounds(rows, n, k, act, tile):
+    from hydrainfer_amd import _lib
+    assert _lib.mix_lib().hxm_grouped_linear_tile_rows(sum(rows), len(rows), n, k) == tile
+    _check(rows, n, k, act, False)
+
+
 # enough tiles for those of 256 x 256: from tile to tile with two slices and with more, columns in 8s and whole turns, the last ones in
 # part; and k and n that take the form before it
 @pytest.mark.parametrize("rows", [[300, 257], [700, 0, 129], [1, 513]])
