@@ -40,12 +40,35 @@ def gate_up_rows_supported(x: Tensor, weight: Tensor) -> bool:
     """True if gate_up_silu_rows takes these operands and is faster than a library product and silu_and_mul."""
     M, K = x.shape
     inter = weight.shape[0] // 2
-    if M <= 128:      # (no rounds of 256 rows are full enough: not asked, as short prompts are bound by their caller)
+    if M <= 64:
         return False
-    return (x.is_cuda and weight.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and weight.dtype == x.dtype and weight.shape[1] == K
+    if not (x.is_cuda and weight.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and weight.dtype == x.dtype and weight.shape[1] == K
             and weight.shape[0] == 2 * inter and x.stride(1) == 1 and weight.stride(1) == 1 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0
-            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and max(M * x.stride(0), 2 * inter * weight.stride(0)) < 2 ** 31
-            and _lib.lib().hx_gate_up_silu_rows_supported(M, inter, K) == 1)
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and max(M * x.stride(0), 2 * inter * weight.stride(0)) < 2 ** 31):
+        return False
+    l = _lib.lib()
+    return K >= 128 and (l.hx_gate_up_silu_few_rows_supported(M, inter, K) == 1 or (M > 128 and l.hx_gate_up_silu_rows_supported(M, inter, K) == 1))
+
+
+def linear_rows(x: Tensor, weight: Tensor) -> Optional[Tensor]:
+    """x [M, K] @ weight [N, K]^T for batches of prompts, for an add and norm behind it: [M, N] of x's type, or float slabs [splits, M, N]
+    (add_rms_norm_slabs sums them); None where a library product is expected to be as fast."""
+    M, K = x.shape
+    N = weight.shape[0]
+    if M <= 64 or not (x.is_cuda and weight.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and weight.dtype == x.dtype and weight.shape[1] == K
+                       and x.stride(1) == 1 and weight.stride(1) == 1 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0
+                       and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and max(M * x.stride(0), N * weight.stride(0)) < 2 ** 31):
+        return None
+    l = _lib.lib()
+    splits = l.hx_linear_rows_splits(M, N, K)
+    if splits == 0:
+        return None
+    _lib.require_gpu(x, weight)
+    out = torch.empty((splits, M, N), dtype=torch.float32, device=x.device) if splits > 1 else torch.empty((M, N), dtype=x.dtype, device=x.device)
+    at = out.data_ptr()
+    _lib.check(l.hx_linear_rows(None if splits > 1 else at, at if splits > 1 else None, splits, x.data_ptr(), weight.data_ptr(), M, N, K, x.stride(0),
+                                weight.stride(0), _lib.dtype_code(x), _lib.current_stream()), "linear_rows")
+    return out
 
 
 def gate_up_silu_rows(x: Tensor, weight: Tensor) -> Tensor:

@@ -93,7 +93,14 @@ __global__ __launch_bounds__(256, 1) void gate_up_silu_rows_kernel(u16* __restri
 }  // namespace
 }  // namespace hx
 
+namespace hx {
+bool gate_up_in_small_tiles(int64_t M, int64_t inter, int64_t K);      // gemm_rows.hip
+int gate_up_small_tiles(void* out, const void* x, const void* weight, int64_t M, int64_t inter, int64_t K, int64_t ldx, int64_t ldw, int dtype, hipStream_t s);
+}  // namespace hx
+
 using namespace hx;
+
+extern "C" int hx_gate_up_silu_few_rows_supported(int64_t M, int64_t inter, int64_t K) { return gate_up_in_small_tiles(M, inter, K) ? 1 : 0; }
 
 extern "C" int hx_gate_up_silu_rows_supported(int64_t M, int64_t inter, int64_t K) {
   if (M < 1 || inter < 16 || inter % 16 || K < 2 * kTileK || K % kTileK || M > (1 << 24) || inter > (1 << 24) || K > (1 << 24)) return 0;
@@ -115,6 +122,7 @@ extern "C" int hx_gate_up_silu_rows(void* out, const void* x, const void* weight
   if (ldx < K || ldw < K || ldx % 8 || ldw % 8 || !aligned16(out) || !aligned16(x) || !aligned16(weight)) return HX_ERR_STRIDE;
   // (32-bit byte offsets of rows and weight rows)
   if (ldx > 0x7fffffff / M || ldw > 0x7fffffff / (2 * inter)) return HX_ERR_STRIDE;
+  if (gate_up_in_small_tiles(M, inter, K)) return gate_up_small_tiles(out, x, weight, M, inter, K, ldx, ldw, dtype, (hipStream_t)stream);
   const int64_t n_row = (M + kTileRows - 1) / kTileRows, n_col = (inter + kTileRows / 2 - 1) / (kTileRows / 2), tiles = n_row * n_col;
   if (tiles > 0x7fffffff) return HX_ERR_SHAPE;
   const int64_t panels = (n_row + 10) / 11;

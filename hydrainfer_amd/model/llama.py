@@ -257,6 +257,16 @@ class LlamaForCausalLM:
             return hip_gemm.linear_decode(x, w)
         return torch.matmul(x, w.t())
 
+    def _linear_add_norm(self, out: Tensor, h: Tensor, x: Tensor, w: Tensor, norm: Tensor) -> None:
+        """h += x w^T; out = rms_norm(h)"""
+        part = hip_gemm.linear_rows(x, w) if self.use_hip_gemm and x.shape[0] > 64 and w.device.type != "meta" else None
+        if part is None:
+            part = self.linear(x, w)
+        if part.dim() == 3:
+            add_rms_norm_slabs(out, h, part, part.shape[0], norm, self.shape.rms_norm_eps)
+        else:
+            add_rms_norm(out, h, part, norm, self.shape.rms_norm_eps)
+
     # ------------------------------------------------------------------ construction
     @classmethod
     def random_init(cls, shape: LlamaShape, dtype: torch.dtype, device, seed: int = 0,
@@ -545,9 +555,8 @@ class LlamaForCausalLM:
                 mha_varlen_fwd(o, q, kc, vc, ap.q_cu_seq_lens, ap.kv_cu_seq_lens, ap.block_tables,
                                ap.cu_blocks_lens, None, ap.q_max_seq_len, ap.kv_max_seq_len,
                                D ** -0.5, 0, -1, 0, 0)
-            a = self.linear(o.view(n, q_size), st[f"l{l}.wo"])
-            # h += a ; x = norm2(h)
-            add_rms_norm(x, h, a, st[f"l{l}.norm2"], eps)
+            # h += o wo^T ; x = norm2(h)
+            self._linear_add_norm(x, h, o.view(n, q_size), st[f"l{l}.wo"], st[f"l{l}.norm2"])
             if (not model_params.all_sequences_decode) and l == L - 1 \
                     and model_params.selected_token_ids is not None:
                 # last layer of a prefill: only sampled tokens go through the MLP
@@ -558,11 +567,10 @@ class LlamaForCausalLM:
             else:
                 gu = self.linear(x, st[f"l{l}.wgu"])
                 act = silu_and_mul(gu[:, :inter], gu[:, inter:])
-            m = self.linear(act, st[f"l{l}.wdown"])
             nxt = st[f"l{l + 1}.norm1"] if l + 1 < L else st["norm"]
             if x.shape != h.shape:
                 x = torch.empty_like(h)
-            add_rms_norm(x, h, m, nxt, eps)   # h += m ; x = next norm (final norm after last layer)
+            self._linear_add_norm(x, h, act, st[f"l{l}.wdown"], nxt)   # h += act wdown^T ; x = next norm (final norm after last layer)
         return x
 
     def forward_logits(self, input_ids_or_embeds, position_ids, model_params) -> Tensor:

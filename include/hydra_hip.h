@@ -233,8 +233,16 @@ int hx_argmax_rows(int64_t* out, const void* logits, int64_t rows, int64_t n, in
  * 2^31.  hx_gate_up_silu_rows_supported: 1 where it is also faster than a library product and hx_silu_and_mul.
  * Replaces: gate_proj, up_proj and the activation of hydrainfer/model/model_forward.py:36 at prompt sizes. */
 int hx_gate_up_silu_rows_supported(int64_t M, int64_t inter, int64_t K);
+int hx_gate_up_silu_few_rows_supported(int64_t M, int64_t inter, int64_t K);      /* the same for 65 to about 1000 rows (csrc/gemm_rows.hip) */
 int hx_gate_up_silu_rows(void* out, const void* x, const void* weight, int64_t M, int64_t inter, int64_t K, int64_t ldx, int64_t ldw,
                          int dtype, hx_stream stream);
+/* out[M, N] = x[M, K] W[N, K]^T for batches of prompts (csrc/gemm_rows.hip), fp16 / bf16, sums in float.  hx_linear_rows_splits: 0 where a library product is
+ * expected to be as fast, else how many slabs [splits, M, N] of float the call writes (1: out and no slabs), to be summed by hx_add_rms_norm_slabs.
+ * N % 32 == 0, K % 64 == 0, 16-byte aligned rows, ldx * M and ldw * N below 2^31.
+ * Replaces: o_proj of hydrainfer/model/model_forward.py and down_proj of its feed-forward at prompt sizes. */
+int hx_linear_rows_splits(int64_t M, int64_t N, int64_t K);
+int hx_linear_rows(void* out, float* slabs, int32_t n_splits, const void* x, const void* weight, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
+                   int dtype, hx_stream stream);
 /* The same product for M <= 32 with the activations held in REGISTERS (csrc/gemm_xreg.hip): a
  * workgroup spans the whole K of its split, so K <= 4096 needs ONE slab (no K split) and K = 11008
  * three instead of eleven — the fp32 slab traffic of a decode layer drops from 25 MB to 6.5 MB.
