@@ -124,6 +124,7 @@ _SIGNATURES = {
     "hx_norm_gate_up_silu_xreg": (c_int, [c_void_p] * 3 + [c_int32, c_void_p, c_float, c_void_p, c_void_p] + [c_int64] * 3 + [c_void_p, c_int, c_void_p]),
     "hx_gate_up_silu_rows_supported": (c_int, [c_int64] * 3),
     "hx_gate_up_silu_few_rows_supported": (c_int, [c_int64] * 3),
+    "hx_prompt_rows": (c_int, [c_void_p, c_int32] + [c_int64] * 3 + [c_void_p] * 8 + [c_int64, c_void_p, c_void_p]),
     "hx_linear_rows_splits": (c_int, [c_int64] * 3),
     "hx_linear_rows": (c_int, [c_void_p, c_void_p, c_int32, c_void_p, c_void_p] + [c_int64] * 5 + [c_int, c_void_p]),
     "hx_gate_up_silu_rows": (c_int, [c_void_p] * 3 + [c_int64] * 5 + [c_int, c_void_p]),

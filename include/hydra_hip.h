@@ -243,6 +243,12 @@ int hx_gate_up_silu_rows(void* out, const void* x, const void* weight, int64_t M
 int hx_linear_rows_splits(int64_t M, int64_t N, int64_t K);
 int hx_linear_rows(void* out, float* slabs, int32_t n_splits, const void* x, const void* weight, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
                    int dtype, hx_stream stream);
+/* The sampled rows of a batch of prompts (csrc/prompt_rows.hip): rows [n] (int32 or int64, negative ones from the end) of x and h
+ * [n_tokens, row_bytes] into x_out, h_out; tables (4 n + 3 int32): q_cu | kv_cu | cu_blocks [n + 1 each] of a batch in which each row is a sequence of one query
+ * that sees the keys the row sees (a causal row of its own sequence), and the rows' positions [n].  cu_blocks has no other use than its starts. */
+int hx_prompt_rows(const void* rows, int32_t rows_are_int64, int64_t n, int64_t n_tokens, int64_t n_seq, const int32_t* q_cu, const int32_t* kv_cu,
+                   const int32_t* cu_blocks, const int32_t* positions, const void* x, const void* h, void* x_out, void* h_out, int64_t row_bytes,
+                   int32_t* tables, hx_stream stream);
 /* The same product for M <= 32 with the activations held in REGISTERS (csrc/gemm_xreg.hip): a
  * workgroup spans the whole K of its split, so K <= 4096 needs ONE slab (no K split) and K = 11008
  * three instead of eleven — the fp32 slab traffic of a decode layer drops from 25 MB to 6.5 MB.

@@ -1,0 +1,80 @@
+"""The last layer of a batch of prompts, whose queries are made of the sampled rows only (csrc/prompt_rows.hip, model/llama.py), against all rows
+through it and the sampled ones taken out behind its attention."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+BLOCK = 16
+
+
+def _batch(new, kv, seed):
+    n_blocks = [(k + BLOCK - 1) // BLOCK for k in kv]
+    perm = torch.randperm(sum(n_blocks), generator=torch.Generator().manual_seed(seed)).tolist()
+    cu_b, cu_q, cu_k = [0], [0], [0]
+    for b, q, k in zip(n_blocks, new, kv):
+        cu_b.append(cu_b[-1] + b)
+        cu_q.append(cu_q[-1] + q)
+        cu_k.append(cu_k[-1] + k)
+    pos = [p for q, k in zip(new, kv) for p in range(k - q, k)]
+    seq = [s for s, q in enumerate(new) for _ in range(q)]
+    slots = [perm[cu_b[s] + p // BLOCK] * BLOCK + p % BLOCK for s, p in zip(seq, pos)]
+    i = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    return dict(n=sum(n_blocks), table=i(perm), cu_blocks=i(cu_b), q_cu=i(cu_q), k_cu=i(cu_k), pos=i(pos), seq=seq, slots=i(slots))
+
+
+@pytest.mark.parametrize("new, kv", [([100], [100]), ([3, 0, 70, 1], [40, 9, 70, 33]), ([65] * 3, [65, 300, 129])])
+@pytest.mark.parametrize("rows", [[0], [-1, 5, 5, 64], list(range(0, 64))], ids=lambda r: f"{len(r)} rows")
+@pytest.mark.parametrize("wide", [True, False])
+def test_prompt_rows(new, kv, rows, wide):
+    from hydrainfer_amd._C.kernel.position_embedding import prompt_rows
+    b, T = _batch(new, kv, 1), sum(new)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x, h = (torch.randn(T, 264, generator=g, device="cuda").bfloat16() for _ in range(2))
+    at = torch.tensor(rows, dtype=torch.int64 if wide else torch.int32, device="cuda")
+    xs, hs, q_cu, kv_cu, cu_blocks, pos = prompt_rows(at, b["q_cu"], b["k_cu"], b["cu_blocks"], b["pos"], x, h)
+    want = [r % T for r in rows]
+    assert torch.equal(xs, x[want]) and torch.equal(hs, h[want]) and torch.equal(pos, b["pos"][want])
+    assert q_cu.tolist() == list(range(len(rows) + 1))
+    keys = [int(b["pos"][r]) + 1 for r in want]
+    assert kv_cu.tolist() == [sum(keys[:i]) for i in range(len(keys) + 1)]
+    assert cu_blocks.tolist()[:-1] == [int(b["cu_blocks"][b["seq"][r]]) for r in want]
+
+
+# sequences that begin and that continue, one of them without a sampled row, one sampled in its middle too; as many key heads as heads and fewer
+@pytest.mark.parametrize("new, kv, rows", [([70], [70], [69]), ([40, 3, 30, 1], [40, 90, 333, 17], [39, 42, 73]), ([65, 66], [65, 200], [130, 64, 10])])
+@pytest.mark.parametrize("heads, kv_heads", [(4, 4), (8, 2)])
+@pytest.mark.parametrize("layers, dt", [(1, torch.bfloat16), (2, torch.float16)])
+def test_sampled_rows_of_the_last_layer(new, kv, rows, heads, kv_heads, layers, dt):
+    from hydrainfer_amd.layer.causal_attention import AttentionParameters
+    from hydrainfer_amd.memory.kv_cache import KVCache
+    from hydrainfer_amd.model.llama import LanguageModelParameters, LlamaForCausalLM, LlamaShape
+    W, inner, D, vocab = 512, 1024, 128, 320
+    g = torch.Generator(device="cuda").manual_seed(sum(new) + heads)
+    w = lambda *s: torch.randn(s, generator=g, device="cuda").mul_(s[-1] ** -0.5).to(dt)
+    state = {"embed": w(vocab, W), "lm_head": w(vocab, W), "norm": torch.ones(W, device="cuda", dtype=dt)}
+    for l in range(layers):
+        state.update({f"l{l}.wqkv": w((heads + 2 * kv_heads) * D, W), f"l{l}.wo": w(W, heads * D), f"l{l}.wgu": w(2 * inner, W), f"l{l}.wdown": w(W, inner),
+                      f"l{l}.norm1": torch.ones(W, device="cuda", dtype=dt), f"l{l}.norm2": torch.ones(W, device="cuda", dtype=dt)})
+    model = LlamaForCausalLM(LlamaShape(W, inner, layers, heads, kv_heads, D, vocab), dt, "cuda", state)
+    b = _batch(new, kv, 3)
+    ids = torch.randint(0, vocab, (sum(new),), generator=g, device="cuda")
+    pool = torch.randn(layers, 2, b["n"], BLOCK, kv_heads, D, generator=g, device="cuda").to(dt)
+
+    def through(sampled_only, rows):
+        caches = pool.clone()
+        model._sampled_rows_only = (lambda *a: took.append(LlamaForCausalLM._sampled_rows_only(model, *a)) or took[-1]) if sampled_only else lambda *a: False
+        params = [AttentionParameters(kv_cache=KVCache(c[0], c[1]), q_cu_seq_lens=b["q_cu"], kv_cu_seq_lens=b["k_cu"], new_cache_slots=b["slots"], block_tables=b["table"],
+                                      cu_blocks_lens=b["cu_blocks"], num_sequences=len(new), all_sequences_decode=False, q_max_seq_len=max(new), kv_max_seq_len=max(kv)) for c in caches]
+        with torch.inference_mode():
+            return model.forward_logits(ids, b["pos"], LanguageModelParameters(params, False, torch.tensor(rows, device="cuda"))), caches
+
+    took = []
+    got, got_caches = through(True, rows)
+    assert took == [True]
+    want, want_caches = through(False, rows)
+    # the keys and values of every token: the same sums in another product's order, rounded
+    half = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11
+    assert float((got_caches.float() - want_caches.float()).norm() / want_caches.float().norm()) < half
+    # attention and three products behind it, rounded each: 8 times half a unit in the last place
+    assert float((got.float() - want.float()).norm() / want.float().norm()) < 8 * half
