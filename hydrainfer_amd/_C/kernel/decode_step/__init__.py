@@ -1,6 +1,6 @@
 """The layers of a decode step, each in one native call (csrc/decode_step.hip, hx_decode_layer_step): the launches that
 gemm.linear_decode_ex, flash_attn.decode_attention_fused, gemm.norm_gate_up_silu_xreg, gemm.norm_linear_decode_xreg and
-norm.add_rms_norm_slabs issue one by one, in the same order with the same arguments."""
+norm.add_rms_norm_slabs issue one by one, in the same order with the same arguments.  And the last layer of a batch of prompts (csrc/prompt_rows.hip)."""
 import ctypes
 from typing import Iterable, NamedTuple, Optional
 
@@ -103,3 +103,48 @@ def decode_layers(h: Tensor, x: Tensor, x_frag: Tensor, act: Tensor, ws: Tensor,
         slabs = lib.hx_decode_layer_step(ctypes.byref(c), slabs, stream)
         if slabs < 0:
             _lib.check(slabs, "decode_layers")
+
+
+def prompt_last_layer(x: Tensor, h: Tensor, rows: Tensor, kv: Tensor, positions: Tensor, cos_sin: Tensor, key_cache: Tensor, value_cache: Tensor, new_cache_slots: Tensor,
+                      cu_seqlens_q: Tensor, cu_seqlens_k: Tensor, block_table: Tensor, cu_block_lens: Tensor, max_seqlen_k: int, wq: Tensor, wo: Tensor,
+                      w_gate_up: Tensor, w_down: Tensor, norm_mlp: Tensor, norm_next: Tensor, softmax_scale: float, epsilon: float) -> Tensor:
+    """The last layer of a batch of prompts for the rows of x that are sampled (csrc/prompt_rows.hip): kv [n_tokens, keys | values] of x = norm1(h), unrotated,
+    goes to the cache (kv's keys are rotated in place).  rms_norm(h[rows] + attention + feed-forward) * norm_next."""
+    tensors = (x, h, rows, kv, positions, cos_sin, key_cache, value_cache, new_cache_slots, cu_seqlens_q, cu_seqlens_k, block_table, cu_block_lens, wq, wo, w_gate_up,
+               w_down, norm_mlp, norm_next)
+    _lib.require_gpu(*tensors)
+    (n_tokens, hidden), n, n_kv, D, width, inter, dt = x.shape, rows.shape[0], key_cache.shape[2], key_cache.shape[3], wq.shape[0], w_down.shape[1], x.dtype
+    if dt not in (torch.float16, torch.bfloat16) or any(t.dtype != dt for t in (h, kv, cos_sin, key_cache, value_cache, wq, wo, w_gate_up, w_down, norm_mlp, norm_next)):
+        raise _lib.HydraHipError("prompt_last_layer: one dtype (fp16 / bf16)")
+    if any(t.dtype != torch.int32 or not t.is_contiguous() for t in (positions, new_cache_slots, cu_seqlens_q, cu_seqlens_k, block_table, cu_block_lens)):
+        raise _lib.HydraHipError("prompt_last_layer: positions, slots, lengths and block table must be contiguous int32")
+    if rows.dim() != 1 or not 1 <= n <= 64 or rows.dtype not in (torch.int32, torch.int64) or any(not t.is_contiguous() for t in (rows, x, h, kv, cos_sin, norm_mlp, norm_next)):
+        raise _lib.HydraHipError("prompt_last_layer: 1 to 64 rows, int32 or int64; rows, x, h, kv, cos_sin and norms contiguous")
+    if h.shape != x.shape or kv.shape != (n_tokens, 2 * n_kv * D) or positions.numel() != n_tokens or new_cache_slots.numel() != n_tokens or value_cache.shape != key_cache.shape \
+            or width % D or wq.shape[1] != hidden or wo.shape != (hidden, width) or w_gate_up.shape != (2 * inter, hidden) or w_down.shape != (hidden, inter) \
+            or norm_mlp.numel() != hidden or norm_next.numel() != hidden or cu_seqlens_k.numel() != cu_seqlens_q.numel() or cu_block_lens.numel() < cu_seqlens_q.numel():
+        raise _lib.HydraHipError("prompt_last_layer: shape mismatch")
+    if any(t.stride(-1) != 1 for t in (wq, wo, w_gate_up, w_down)) or any(c.stride(3) != 1 or c.stride(2) != D or c.stride(1) != n_kv * D for c in (key_cache, value_cache)):
+        raise _lib.HydraHipError("prompt_last_layer: rows of weights and of a cache block must be contiguous")
+    out = torch.empty((n, hidden), dtype=dt, device=x.device)
+    c = _lib.hx_prompt_last()
+    a = c.attn
+    a.k, a.v, a.block_size = key_cache.data_ptr(), value_cache.data_ptr(), key_cache.shape[1]
+    a.k_block_stride, a.k_row_stride, a.k_head_stride = key_cache.stride()[:3]
+    a.v_block_stride, a.v_row_stride, a.v_head_stride = value_cache.stride()[:3]
+    a.cu_seqlens_q, a.cu_seqlens_k, a.block_table, a.cu_block_lens = (t.data_ptr() for t in (cu_seqlens_q, cu_seqlens_k, block_table, cu_block_lens))
+    a.n_heads, a.n_kv_heads, a.head_dim, a.max_seqlen_k = width // D, n_kv, D, int(max_seqlen_k)
+    a.softmax_scale, a.causal, a.dtype, a.window_left, a.window_right = float(softmax_scale), 1, _lib.dtype_code(x), -1, -1
+    c.x, c.h, c.rows, c.kv, c.positions, c.cos_sin, c.new_cache_slots = (t.data_ptr() for t in (x, h, rows, kv, positions, cos_sin, new_cache_slots))
+    c.wq, c.wo, c.w_gate_up, c.w_down, c.norm_mlp, c.norm_next, c.out = (t.data_ptr() for t in (wq, wo, w_gate_up, w_down, norm_mlp, norm_next, out))
+    c.ld_wq, c.ld_wo, c.ld_gate_up, c.ld_down = wq.stride(0), wo.stride(0), w_gate_up.stride(0), w_down.stride(0)
+    c.n, c.n_tokens, c.n_seq, c.hidden, c.inter = n, n_tokens, cu_seqlens_q.numel() - 1, hidden, inter
+    c.epsilon, c.rows_are_int64 = float(epsilon), rows.dtype == torch.int64
+    lib = _lib.lib()
+    need = lib.hx_prompt_last_scratch_bytes(ctypes.byref(c))
+    if need < 0:
+        _lib.check(int(need), "prompt_last_layer")
+    scratch = torch.empty(need, dtype=torch.uint8, device=x.device)
+    c.scratch, c.scratch_bytes = scratch.data_ptr(), need
+    _lib.check(lib.hx_prompt_last_layer(ctypes.byref(c), _lib.current_stream()), "prompt_last_layer")
+    return out

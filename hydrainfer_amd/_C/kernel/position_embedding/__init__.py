@@ -1,8 +1,6 @@
 """hydrainfer._C.kernel.position_embedding — drop-in surface
 (reference stub: hydrainfer/_C/kernel/position_embedding/__init__.pyi:5-11;
 CUDA original: csrc/kernel/position_embedding/rope.cu:82-117)."""
-from typing import Tuple
-
 import torch
 from torch import Tensor
 
@@ -56,44 +54,3 @@ def rope_set_kv_cache(query: Tensor, key: Tensor, value: Tensor, positions: Tens
         query.size(0), query.size(1), key.size(1), query.size(2), int(rotary_dim), query.stride(0),
         key.stride(0), value.stride(0), key_cache.size(1), key_cache.stride(0), value_cache.stride(0),
         _lib.dtype_code(query), _lib.current_stream()), "rope_set_kv_cache")
-
-
-def rope_queries(query: Tensor, positions: Tensor, cos_sin: Tensor, rotary_dim: int) -> None:
-    """apply_rotary_pos_emb(query, ..., interleaved=False) without keys."""
-    _lib.check(_lib.lib().hx_apply_rotary_pos_emb(
-        query.data_ptr(), query.data_ptr(), positions.data_ptr(), cos_sin.data_ptr(), query.size(0), query.size(1), 0, query.size(2), int(rotary_dim),
-        query.stride(0), query.stride(0), 0, _lib.dtype_code(query), _lib.current_stream()), "rope_queries")
-
-
-def rope_keys_set_kv_cache(key: Tensor, value: Tensor, positions: Tensor, cos_sin: Tensor, rotary_dim: int, slot_ids: Tensor,
-                           key_cache: Tensor, value_cache: Tensor) -> None:
-    """rope_set_kv_cache of a batch whose queries are made elsewhere."""
-    _lib.require_gpu(key, value, positions, cos_sin, slot_ids, key_cache, value_cache)
-    for t in (key, value):
-        if t.dim() != 3 or t.stride(-1) != 1 or t.stride(-2) != t.size(-1):
-            raise _lib.HydraHipError("rope_keys_set_kv_cache: k/v must be [n, heads, head_dim], last two dims contiguous")
-    for c in (key_cache, value_cache):
-        if c.dim() != 4 or c.stride(-1) != 1 or c.stride(-2) != c.size(-1) or c.stride(-3) != c.size(-1) * c.size(-2):
-            raise _lib.HydraHipError("rope_keys_set_kv_cache: cache rows inside a block must be contiguous")
-    if positions.dtype.itemsize != 4 or slot_ids.dtype.itemsize != 4:
-        raise _lib.HydraHipError("rope_keys_set_kv_cache: positions / slot_ids must be int32")
-    if not (key.dtype == value.dtype == cos_sin.dtype == key_cache.dtype == value_cache.dtype):
-        raise _lib.HydraHipError("rope_keys_set_kv_cache: dtype mismatch")
-    _lib.check(_lib.lib().hx_rope_set_kv_cache(
-        key.data_ptr(), key.data_ptr(), value.data_ptr(), positions.contiguous().data_ptr(), cos_sin.data_ptr(), slot_ids.contiguous().data_ptr(),
-        key_cache.data_ptr(), value_cache.data_ptr(), key.size(0), 0, key.size(1), key.size(2), int(rotary_dim), key.stride(0), key.stride(0),
-        value.stride(0), key_cache.size(1), key_cache.stride(0), value_cache.stride(0), _lib.dtype_code(key), _lib.current_stream()), "rope_keys_set_kv_cache")
-
-
-def prompt_rows(rows: Tensor, q_cu: Tensor, kv_cu: Tensor, cu_blocks: Tensor, positions: Tensor, x: Tensor,
-                h: Tensor) -> Tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
-    """(x[rows], h[rows], q_cu, kv_cu, cu_blocks, positions[rows]): each of these rows as a sequence of one query that sees the keys it sees in the
-    batch (q_cu, kv_cu, cu_blocks), one launch."""
-    n, width = rows.shape[0], x.shape[1]
-    x_out, h_out = torch.empty((n, width), dtype=x.dtype, device=x.device), torch.empty((n, width), dtype=x.dtype, device=x.device)
-    tables = torch.empty(4 * n + 3, dtype=torch.int32, device=x.device)
-    _lib.check(_lib.lib().hx_prompt_rows(rows.data_ptr(), 1 if rows.dtype == torch.int64 else 0, n, x.shape[0], q_cu.shape[0] - 1, q_cu.data_ptr(), kv_cu.data_ptr(),
-                                         cu_blocks.data_ptr(), positions.data_ptr(), x.data_ptr(), h.data_ptr(), x_out.data_ptr(), h_out.data_ptr(),
-                                         width * x.element_size(), tables.data_ptr(), _lib.current_stream()), "prompt_rows")
-    m = n + 1
-    return x_out, h_out, tables[:m], tables[m:2 * m], tables[2 * m:3 * m], tables[3 * m:]

@@ -74,6 +74,13 @@ class hx_decode_layer(ctypes.Structure):
                 ("hidden", c_int64), ("inter", c_int64), ("epsilon", c_float), ("norm_in_qkv", c_int32), ("dtype", c_int32)]
 
 
+class hx_prompt_last(ctypes.Structure):
+    _fields_ = [("attn", hx_attn_args)] + [(p, c_void_p) for p in (
+        "rows", "positions", "new_cache_slots", "x", "h", "kv", "cos_sin", "wq", "wo", "w_gate_up", "w_down", "norm_mlp", "norm_next", "out", "scratch")] + [
+        (i, c_int64) for i in ("scratch_bytes", "n", "n_tokens", "n_seq", "hidden", "inter", "ld_wq", "ld_wo", "ld_gate_up", "ld_down")] + [
+        ("epsilon", c_float), ("rows_are_int64", c_int32)]
+
+
 HX_DW_LDS_SLICE, HX_DW_XREG, HX_DW_GATE_UP = 0, 1, 1
 HX_DW_FORCE_LDS_SLICE = 2
 
@@ -125,6 +132,8 @@ _SIGNATURES = {
     "hx_gate_up_silu_rows_supported": (c_int, [c_int64] * 3),
     "hx_gate_up_silu_few_rows_supported": (c_int, [c_int64] * 3),
     "hx_prompt_rows": (c_int, [c_void_p, c_int32] + [c_int64] * 3 + [c_void_p] * 8 + [c_int64, c_void_p, c_void_p]),
+    "hx_prompt_last_scratch_bytes": (c_int64, [POINTER(hx_prompt_last)]),
+    "hx_prompt_last_layer": (c_int, [POINTER(hx_prompt_last), c_void_p]),
     "hx_linear_rows_splits": (c_int, [c_int64] * 3),
     "hx_linear_rows": (c_int, [c_void_p, c_void_p, c_int32, c_void_p, c_void_p] + [c_int64] * 5 + [c_int, c_void_p]),
     "hx_gate_up_silu_rows": (c_int, [c_void_p] * 3 + [c_int64] * 5 + [c_int, c_void_p]),

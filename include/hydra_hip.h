@@ -407,6 +407,27 @@ typedef struct hx_attn_args {
 int64_t hx_mha_varlen_fwd_workspace_bytes(const hx_attn_args* args);
 int hx_mha_varlen_fwd(const hx_attn_args* args, hx_stream stream);
 
+/* The last layer of a batch of prompts behind its keys' and values' product, by one call (csrc/prompt_rows.hip): kv [n_tokens, 2 * n_kv_heads * head_dim] (keys,
+ * rotated here, then values) goes to the cache; the queries, the attention and the feed-forward are made of the n <= 64 sampled rows alone.  out [n, hidden] =
+ * rms_norm(h + ...) * norm_next of those rows.  attn: the cache, its block table and the batch's cu_seqlens_q, cu_seqlens_k, cu_block_lens [n_seq + 1];
+ * its queries, output, batch and workspace are set by the call.  hidden, inter, n_heads * head_dim: multiples of 256; weights row-major, strides in elements.
+ * Replaces: the last layer of hydrainfer/model/model_forward.py:39-105, whose other rows nothing uses. */
+typedef struct hx_prompt_last {
+  hx_attn_args attn;
+  const void* rows;            /* [n], as for hx_prompt_rows */
+  const int32_t* positions;    /* [n_tokens], as new_cache_slots */
+  const int32_t* new_cache_slots;
+  const void *x, *h;           /* [n_tokens, hidden]: norm1 of the layer's input, and the input */
+  void* kv;                    /* its keys are rotated in place */
+  const void *cos_sin, *wq, *wo, *w_gate_up, *w_down, *norm_mlp, *norm_next;
+  void *out, *scratch;
+  int64_t scratch_bytes, n, n_tokens, n_seq, hidden, inter, ld_wq, ld_wo, ld_gate_up, ld_down;
+  float epsilon;
+  int32_t rows_are_int64;
+} hx_prompt_last;
+int64_t hx_prompt_last_scratch_bytes(const hx_prompt_last* layer);
+int hx_prompt_last_layer(const hx_prompt_last* layer, hx_stream stream);
+
 /* Extension (SURVEY §8f-2 taken to the end): one launch for the three consecutive steps of a
  * decode layer — apply_rotary_pos_emb(q, k) (NeoX, rotary_dim == head_dim), set_kv_cache(slots,
  * k, v) and the paged attention itself (hydrainfer/model/model_forward.py:78-84 +

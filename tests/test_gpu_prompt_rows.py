@@ -27,12 +27,16 @@ def _batch(new, kv, seed):
 @pytest.mark.parametrize("rows", [[0], [-1, 5, 5, 64], list(range(0, 64))], ids=lambda r: f"{len(r)} rows")
 @pytest.mark.parametrize("wide", [True, False])
 def test_prompt_rows(new, kv, rows, wide):
-    from hydrainfer_amd._C.kernel.position_embedding import prompt_rows
+    from hydrainfer_amd import _lib
     b, T = _batch(new, kv, 1), sum(new)
     g = torch.Generator(device="cuda").manual_seed(T)
     x, h = (torch.randn(T, 264, generator=g, device="cuda").bfloat16() for _ in range(2))
     at = torch.tensor(rows, dtype=torch.int64 if wide else torch.int32, device="cuda")
-    xs, hs, q_cu, kv_cu, cu_blocks, pos = prompt_rows(at, b["q_cu"], b["k_cu"], b["cu_blocks"], b["pos"], x, h)
+    m = len(rows) + 1
+    xs, hs, tables = torch.empty(len(rows), 264, dtype=x.dtype, device="cuda"), torch.empty(len(rows), 264, dtype=x.dtype, device="cuda"), torch.empty(4 * m - 1, dtype=torch.int32, device="cuda")
+    _lib.check(_lib.lib().hx_prompt_rows(at.data_ptr(), int(wide), len(rows), T, len(new), b["q_cu"].data_ptr(), b["k_cu"].data_ptr(), b["cu_blocks"].data_ptr(), b["pos"].data_ptr(),
+                                         x.data_ptr(), h.data_ptr(), xs.data_ptr(), hs.data_ptr(), 2 * 264, tables.data_ptr(), _lib.current_stream()), "prompt_rows")
+    q_cu, kv_cu, cu_blocks, pos = tables[:m], tables[m:2 * m], tables[2 * m:3 * m], tables[3 * m:]
     want = [r % T for r in rows]
     assert torch.equal(xs, x[want]) and torch.equal(hs, h[want]) and torch.equal(pos, b["pos"][want])
     assert q_cu.tolist() == list(range(len(rows) + 1))
