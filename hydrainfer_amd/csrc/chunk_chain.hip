@@ -1,7 +1,7 @@
 // chunk_chain.hip — recurrences over portions of prompts, sixteen tokens at a time (chunk_scan.hip says how), in two launches: what
 // does not depend on the state — A, M, prefixed queries, suffixed keys, all of it vector work and a serial substitution — is made for all
 // chunks at once on the whole chip, and the chain of chunks is left with the products of the state.  One launch has these made beside
-// the chain, on the same SIMDs and once per 64 value channels.
+// the chain, on the same SIMDs and once per 64 value channels.  Few long chains go in segments, in a launch more (segment_chunks).
 // What bounds the chain: a chunk is 104 float products a wave under the delta rule with 128 x 128 (68 without write strengths), 32 cycles
 // each, where a wave holds all keys of 16 value channels, and 140 (100) vector instructions that do not run beside the products of
 // their own wave (a multiplication behind a product costs 7 cycles; those of other waves cost it nothing).  So the keys of 16 value channels are
@@ -17,6 +17,8 @@
 // first launch, 560 vector instructions a wave of four tokens and 164 MB written; delta rule 190 and 235, so the first launch is weighed
 // against the chain, chunk_scan_workspace).
 #include "chunk_parts.h"
+#include <algorithm>
+#include <cmath>
 
 namespace {
 
@@ -239,18 +241,66 @@ struct Image {
   static constexpr int kLds = kImages * kFloats + 2 * kResult + (DELTA ? 2 * kShares : 0);
 };
 
-template <int KP, int FORM, bool CHANNEL, int KS, typename QK, typename VT, bool VEC>
+// Few chains leave most compute units idle, and a chain is as long as its portion.  The state behind a segment of a portion is what its
+// own tokens give from an empty state and what its decays leave of the state ahead of it, so the segments' states are made all at
+// once by a launch ahead (kSegmentStates: the chain without queries and results), and the segments of every portion are then chains of
+// their own (kSegmentResults), which put the state that they start from together out of those.
+// Segment p of sequence s, `segment` chunks each, has number q_cu[s] / (16 segment) + s + p and, for every head, K V + 2 K floats in
+// `segments`: the state behind the segment ahead of it (the first one's from the portion's true start, the others' from nothing; of
+// segment 0 the start itself: the last segment may store the final state before the first one begins), and its product of decays, in
+// double for the range.
+enum { kWhole, kSegmentStates, kSegmentResults };
+__host__ __device__ inline int64_t segment_state(const ChunkScanArgs& a) { return ((int64_t)a.K * a.V + 1) / 2 * 2; }      // (doubles behind it)
+__device__ __forceinline__ float* segment_at(const ChunkScanArgs& a, int64_t number, int head) {
+  return a.segments + (number * a.heads + head) * (int64_t)(segment_state(a) + 2 * a.K);
+}
+struct SegmentAt {
+  int seq, p;               // seq < 0: nobody's
+};
+__device__ __forceinline__ SegmentAt segment_of(const ChunkScanArgs& a, int64_t number) {
+  const int lane = threadIdx.x & 63, tokens = C * a.segment;
+  int seq = -1;
+  for (int s0 = 0; s0 < a.n_seq; s0 += 64) {              // the last sequence that starts at or before this number
+    const int s = s0 + lane;
+    const int here = __popcll(__builtin_amdgcn_ballot_w64(s < a.n_seq && a.q_cu[min(s, a.n_seq - 1)] / tokens + s <= number));
+    seq += here;
+    if (here < 64) break;
+  }
+  return seq < 0 ? SegmentAt{-1, 0} : SegmentAt{seq, (int)(number - (a.q_cu[seq] / tokens + seq))};
+}
+// what a product of decays becomes with one more: it does not leave the range while its factors are in theirs (what it leaves of an infinity is one)
+__device__ __forceinline__ double decayed(double product, float d) {
+  const double x = product * (double)d;
+  return d != 0.f && fabs(x) < 1e-300 ? copysign(1e-300, x) : x;
+}
+
+template <int KP, int FORM, bool CHANNEL, int KS, typename QK, typename VT, bool VEC, int PASS>
 __global__ __launch_bounds__(768) void chunk_chain_kernel(ChunkScanArgs a) {
   typedef Image<KP, FORM, CHANNEL, KS> I;
   constexpr int RS = KP + 4, KT = KP / 16 / KS, W = I::W, WS = I::WS, kMade = I::kMade, kLead = I::kImages - 2;
   constexpr bool DELTA = I::DELTA, BONUS = FORM == hxm::kChunkBonus;
   extern __shared__ __attribute__((aligned(16))) float lds[];      // images | results[2] | y[2]
-  const int seq = blockIdx.z, head = blockIdx.x, col0 = (int)blockIdx.y * W;
+  constexpr bool kResults = PASS != kSegmentStates;
+  constexpr int kSkip = CHANNEL && !kResults ? C * RS : 0;      // (the queries)
+  const int head = blockIdx.x, col0 = (int)blockIdx.y * W;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int g = lane >> 4, m = lane & 15;
-  const int64_t t_begin = a.q_cu[seq];
-  const int n_tok = (int)(a.q_cu[seq + 1] - t_begin);
+  int seq = blockIdx.z, part_at = 0;                      // part_at: the segment
+  if constexpr (PASS != kWhole) {
+    const SegmentAt at = segment_of(a, blockIdx.z);
+    if (at.seq < 0) return;                               // (the whole workgroup, as below)
+    seq = __builtin_amdgcn_readfirstlane(at.seq);
+    part_at = __builtin_amdgcn_readfirstlane(at.p);
+  }
+  const int64_t t_seq = a.q_cu[seq], t_begin = PASS == kWhole ? t_seq : t_seq + (int64_t)part_at * a.segment * C;
+  int n_tok = (int)(a.q_cu[seq + 1] - t_begin);
   if (n_tok <= 0) return;                                 // (the whole workgroup)
+  bool last = true;
+  if constexpr (PASS != kWhole) {
+    last = n_tok <= a.segment * C;
+    if (PASS == kSegmentStates && last) return;
+    n_tok = min(n_tok, a.segment * C);
+  }
   const int n_chunks = (n_tok + C - 1) / C;
   auto made = [&](int chunk) { return lds + chunk % I::kImages * I::kFloats; };
   auto rows = [&](int chunk) { return made(chunk) + kMade; };
@@ -263,7 +313,37 @@ __global__ __launch_bounds__(768) void chunk_chain_kernel(ChunkScanArgs a) {
     const int part = (wave - 4) % KS, cw = (wave - 4) / KS, col = col0 + 16 * cw + m, k0 = 16 * KT * part;
     float* slot = a.state + (int64_t)a.slots[seq] * a.slot_stride + (int64_t)head * a.K * a.V + (int64_t)k0 * a.V;
     State<KT> st;
-    st.load(slot, a.K - k0, a.V, col, g, a.positions[t_begin] == 0);
+    const bool fresh = a.positions[t_seq] == 0;
+    double left[CHANNEL ? KT : 1][4];                     // (kSegmentStates: this segment's product of decays)
+    if constexpr (PASS == kWhole) {
+      st.load(slot, a.K - k0, a.V, col, g, fresh);
+    } else if constexpr (PASS == kSegmentStates) {
+      st.load(slot, a.K - k0, a.V, col, g, fresh || part_at > 0);
+      if (part_at == 0) st.store(segment_at(a, blockIdx.z, head) + (int64_t)k0 * a.V, a.K - k0, a.V, col, g);
+#pragma unroll
+      for (int kt = 0; kt < (CHANNEL ? KT : 1); ++kt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) left[kt][e] = 1.0;
+    } else if (part_at == 0) {
+      const bool alone = last;                            // (nobody else reads or writes the slot's columns)
+      st.load(alone ? slot : segment_at(a, blockIdx.z, head) + (int64_t)k0 * a.V, a.K - k0, a.V, col, g, alone && fresh);
+    } else {
+      const int64_t first = (int64_t)blockIdx.z - part_at;
+      st.load(segment_at(a, first + 1, head) + (int64_t)k0 * a.V, a.K - k0, a.V, col, g, false);
+#pragma unroll 1
+      for (int p = 1; p < part_at; ++p) {                 // what segment p makes of the state behind the one ahead of it
+        State<KT> own;
+        own.load(segment_at(a, first + p + 1, head) + (int64_t)k0 * a.V, a.K - k0, a.V, col, g, false);
+        const double* decays = reinterpret_cast<const double*>(segment_at(a, first + p, head) + segment_state(a));
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int kk = k0 + 16 * kt + 4 * g + e;
+            st.S[kt][e] = (float)__builtin_fma(decays[min(kk, a.K - 1)], (double)st.S[kt][e], (double)own.S[kt][e]);
+          }
+      }
+    }
     const int share = part * C * WS + 4 * g * WS + 16 * cw + m;      // this lane's column of rows 4 g ..
     // the keys' part of rows (token m) of x times the state; four chains of at most sixteen keys
     auto times_state = [&](const float* row) __attribute__((always_inline)) {
@@ -336,33 +416,38 @@ __global__ __launch_bounds__(768) void chunk_chain_kernel(ChunkScanArgs a) {
         if (odd) w = times_rows_in_order(p + C * RA, m, g, x);
       }
       // this part's share of the results: its keys' of what the state holds, its tokens' of the chunk's own
-      const f32x4 before = times_state((CHANNEL ? p : r) + m * RS + 4 * g);
-      f32x4 first = before, second = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (odd) {
-        if (part == 0) second = times_rows_in_order(A, m, g, w);
-        if (FORM == hxm::kChunkGated) second += before;
-      } else if constexpr (BONUS) {                       // (in double: what rounding leaves over goes to the smaller number)
-        f64x4 sum = f64x4{0., 0., 0., 0.};
+      f32x4 first, second = f32x4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (kResults) {
+        const f32x4 before = times_state((CHANNEL ? p : r) + m * RS + 4 * g);
+        first = before;
+        if (odd) {
+          if (part == 0) second = times_rows_in_order(A, m, g, w);
+          if (FORM == hxm::kChunkGated) second += before;
+        } else if constexpr (BONUS) {                       // (in double: what rounding leaves over goes to the smaller number)
+          f64x4 sum = f64x4{0., 0., 0., 0.};
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (e / (4 / KS) == part) sum = __builtin_amdgcn_mfma_f64_16x16x4f64((double)A_row[e], (double)w[e], sum, 0, 0, 0);
+          for (int e = 0; e < 4; ++e)
+            if (e / (4 / KS) == part) sum = __builtin_amdgcn_mfma_f64_16x16x4f64((double)A_row[e], (double)w[e], sum, 0, 0, 0);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          second[e] = (float)sum[e];
-          first[e] += (float)(sum[e] - (double)second[e]);
+          for (int e = 0; e < 4; ++e) {
+            second[e] = (float)sum[e];
+            first[e] += (float)(sum[e] - (double)second[e]);
+          }
+        } else {
+          if (FORM == hxm::kChunkGated) second = before;
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (e / (4 / KS) == part) second = mma4(A_row[e], w[e], second);
         }
-      } else {
-        if (FORM == hxm::kChunkGated) second = before;
+        if constexpr (!CHANNEL) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (e / (4 / KS) == part) second = mma4(A_row[e], w[e], second);
+          for (int e = 0; e < 4; ++e) {
+            first[e] = before[e] * pre[e];
+            second[e] += __builtin_fmaf(before[e], rest[e], __builtin_fmaf(before[e], pre[e], -first[e]));
+          }
+        }
       }
       if constexpr (!CHANNEL) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          first[e] = before[e] * pre[e];
-          second[e] += __builtin_fmaf(before[e], rest[e], __builtin_fmaf(before[e], pre[e], -first[e]));
-        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) w[e] *= suf[e];
       }
@@ -385,14 +470,35 @@ __global__ __launch_bounds__(768) void chunk_chain_kernel(ChunkScanArgs a) {
       for (int e = 0; e < 4; ++e)
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt) st.S[kt] = mma4(kx[kt][e], w[e], st.S[kt]);
-      put(outs(c), second);
-      if constexpr (FORM != hxm::kChunkGated) put(outs(c) + I::kShares, first);
+      if constexpr (!kResults) {
+#pragma unroll
+        for (int kt = 0; kt < (CHANNEL ? KT : 1); ++kt)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) left[kt][e] = decayed(left[kt][e], CHANNEL ? d[kt][e] : total);
+      } else {
+        put(outs(c), second);
+        if constexpr (FORM != hxm::kChunkGated) put(outs(c) + I::kShares, first);
+      }
       if constexpr (DELTA) {
         if (c + 1 < n_chunks) put(ys(c + 1), times_state(rows(c + 1) + C * RS + m * RS + 4 * g));
       }
     }
     lds_barrier();
-    st.store(slot, a.K - k0, a.V, col, g);
+    if constexpr (PASS == kSegmentStates) {
+      st.store(segment_at(a, (int64_t)blockIdx.z + 1, head) + (int64_t)k0 * a.V, a.K - k0, a.V, col, g);
+      if (blockIdx.y == 0 && cw == 0 && m == 0) {
+        double* decays = reinterpret_cast<double*>(segment_at(a, blockIdx.z, head) + segment_state(a));
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int kk = k0 + 16 * kt + 4 * g + e;
+            if (kk < a.K) decays[kk] = left[CHANNEL ? kt : 0][e];
+          }
+      }
+    } else if (last) {
+      st.store(slot, a.K - k0, a.V, col, g);
+    }
     return;
   }
 
@@ -402,13 +508,13 @@ __global__ __launch_bounds__(768) void chunk_chain_kernel(ChunkScanArgs a) {
   const typename VT::storage* v = (const typename VT::storage*)a.v + t_begin * a.v_stride + (int64_t)head * a.V;
   const bool scaled = !BONUS && FORM != hxm::kChunkGated && (DELTA || a.vscale);
   const float* per_token = DELTA ? a.beta : a.vscale ? a.vscale : a.decay;
-  const float* from = a.made + (chunk_number(t_begin, seq) * a.heads + head) * kMade;
+  const float* from = a.made + ((chunk_number(t_seq, seq) + (PASS == kWhole ? 0 : (int64_t)part_at * a.segment)) * a.heads + head) * kMade + kSkip;
   const int v_row = tid / (W / 4), v_col = tid % (W / 4) * 4;      // (16 W / 4 threads)
   const bool v_mine = 16 * W / 4 >= 256 || v_row < C;
   struct Set {
     Rows<QK, VEC, KP, 256> q, k;           // (a decay per head)
     Piece<VT, 4, VEC> v;
-    MadeRows<kMade, 256> made;
+    MadeRows<kMade - kSkip, 256> made;
     float scale;
   } sets[kAhead];
   auto fetch = [&](Set& s, int chunk) __attribute__((always_inline)) {
@@ -416,7 +522,7 @@ __global__ __launch_bounds__(768) void chunk_chain_kernel(ChunkScanArgs a) {
     const int n = rows_of(chunk);
     const int64_t t0 = (int64_t)chunk * C;
     if constexpr (!CHANNEL) {
-      s.q.fetch(q + t0 * a.q_stride, a.q_stride, 0, a.K, n, tid);
+      if constexpr (kResults) s.q.fetch(q + t0 * a.q_stride, a.q_stride, 0, a.K, n, tid);
       s.k.fetch(k + t0 * a.k_stride, a.k_stride, 0, a.K, n, tid);
     }
     s.made.fetch(from + (int64_t)chunk * a.heads * kMade, tid);
@@ -427,9 +533,9 @@ __global__ __launch_bounds__(768) void chunk_chain_kernel(ChunkScanArgs a) {
     if (chunk >= n_chunks) return;
     const int n = rows_of(chunk);
     float* r = rows(chunk);
-    s.made.store(made(chunk), tid);
+    s.made.store(made(chunk) + kSkip, tid);
     if constexpr (!CHANNEL) {
-      s.q.store(r, 0, a.K, n, 1.f, tid);
+      if constexpr (kResults) s.q.store(r, 0, a.K, n, 1.f, tid);
       s.k.store(r + C * RS, 0, a.K, n, 1.f, tid);
       if (tid < C) r[2 * C * RS + row_of_token(m)] = m >= n ? (DELTA ? 0.f : 1.f) : scaled ? s.scale : 1.f;      // (a row past the portion changes nothing)
     }
@@ -442,6 +548,7 @@ __global__ __launch_bounds__(768) void chunk_chain_kernel(ChunkScanArgs a) {
   };
   // results: the parts' shares added up in double, rounded once
   auto write = [&](int chunk) __attribute__((always_inline)) {
+    if constexpr (!kResults) return;
     const int col = col0 + v_col;
     if (!v_mine || v_row >= rows_of(chunk)) return;
     const float* o = outs(chunk) + row_of_token(v_row) * WS + v_col;
@@ -482,6 +589,7 @@ __global__ __launch_bounds__(768) void chunk_chain_kernel(ChunkScanArgs a) {
 
 // numbers that chunks may have
 int64_t chunk_numbers(const ChunkScanArgs& a) { return a.n_tokens / C + a.n_seq; }
+int64_t segment_numbers(const ChunkScanArgs& a, int segment) { return a.n_tokens / (C * segment) + a.n_seq; }
 // With 32 value channels a workgroup every one of them has a compute unit: the keys go to four waves.  (Else twice the rows would be
 // brought in for each channel: the gated form above 146 us in the chain, 115 with 64 channels.)
 bool few_chains(const ChunkScanArgs& a) { return (int64_t)a.n_seq * a.heads * ((a.V + 31) / 32) <= 256; }
@@ -493,19 +601,27 @@ int64_t made_floats(const ChunkScanArgs& a) {
   return a.form == hxm::kChunkDelta ? kMadeHead<true> : kMadeHead<false>;
 }
 
-template <int KP, int FORM, bool CHANNEL, int KS, typename QK, typename VT, bool VEC>
+template <int KP, int FORM, bool CHANNEL, int KS, typename QK, typename VT, bool VEC, int PASS>
 int launch_parts(const ChunkScanArgs& a, hipStream_t s) {
   typedef Image<KP, FORM, CHANNEL, KS> I;
-  return launch_chunks(chunk_chain_kernel<KP, FORM, CHANNEL, KS, QK, VT, VEC>, dim3((unsigned)a.heads, (unsigned)((a.V + I::W - 1) / I::W), (unsigned)a.n_seq), 768,
+  const int64_t z = PASS == kWhole ? a.n_seq : segment_numbers(a, a.segment);
+  return launch_chunks(chunk_chain_kernel<KP, FORM, CHANNEL, KS, QK, VT, VEC, PASS>, dim3((unsigned)a.heads, (unsigned)((a.V + I::W - 1) / I::W), (unsigned)z), 768,
                        sizeof(float) * I::kLds, a, s);
 }
 template <int KP, int FORM, bool CHANNEL, typename QK, typename VT, bool VEC>
 int launch_chain(const ChunkScanArgs& a, hipStream_t s) {
+  constexpr int KS = KP == 128 ? 4 : 2;                   // of few chains
+  if constexpr (FORM != hxm::kChunkDelta) {
+    if (a.segment > 0) {
+      const int rc = launch_parts<KP, FORM, CHANNEL, KS, QK, VT, VEC, kSegmentStates>(a, s);
+      return rc != HX_OK ? rc : launch_parts<KP, FORM, CHANNEL, KS, QK, VT, VEC, kSegmentResults>(a, s);
+    }
+  }
   if constexpr (KP == 128) {
-    if (few_chains(a)) return launch_parts<KP, FORM, CHANNEL, 4, QK, VT, VEC>(a, s);
+    if (few_chains(a)) return launch_parts<KP, FORM, CHANNEL, KS, QK, VT, VEC, kWhole>(a, s);
   }
   if constexpr (FORM == hxm::kChunkDelta) return HX_ERR_UNSUPPORTED;      // (many chains of the delta rule take one launch: two gain nothing, chunk_scan_workspace)
-  else return launch_parts<KP, FORM, CHANNEL, 2, QK, VT, VEC>(a, s);
+  else return launch_parts<KP, FORM, CHANNEL, 2, QK, VT, VEC, kWhole>(a, s);
 }
 template <int KP, int FORM, typename QK, typename VT, bool VEC>
 int launch_channel(const ChunkScanArgs& a, hipStream_t s) {
@@ -542,11 +658,31 @@ int launch_width(const ChunkScanArgs& a, hipStream_t s) {
 
 namespace hxm {
 
-int64_t chunk_scan_workspace(const ChunkScanArgs& a) {
-  if (!chunk_scan_fits(a) || (a.V + 31) / 32 > 65535 || (a.form == kChunkDelta && a.K <= 64)) return 0;
-  const int64_t workgroups = chunk_numbers(a) * a.heads;
-  const int64_t floats = workgroups * (a.K <= 64 ? made_floats<64>(a) : made_floats<128>(a));
-  if (workgroups > INT32_MAX || floats > (int64_t)1 << 28) return 0;      // (1 GiB)
+static int64_t plan_made(const ChunkScanArgs& a) { return chunk_numbers(a) * a.heads * (a.K <= 64 ? made_floats<64>(a) : made_floats<128>(a)); }
+static int64_t plan_floats(const ChunkScanArgs& a, int segment) {
+  return plan_made(a) + (segment > 0 ? segment_numbers(a, segment) * a.heads * (segment_state(a) + 2 * a.K) : 0);
+}
+// Chunks a segment, 0: portions stay whole.  longest: chunks of the longest portion, or of the mean one where that is all that is known.
+// Segments take a launch more and every chunk's keys twice (a chunk of the states' launch costs about 0.6 of one with results), and pay where the compute
+// units have room for all of them at once: a second round costs more than longer segments (2 portions of 500 - 684 tokens, 32 heads of 128 x 128,
+// gated: whole 74 us, segments of 8, 12, 16 chunks 115, 110, 103).  So a segment is as short as that room allows, at least 6 chunks (96 tokens; at 4
+// the launches around them cost as much) and a seventh of the portion, as the last segment's start is put together out of all before it (8 heads of 128 x 128, 1151
+// tokens in segments of 4, 8, 12, 16 chunks 81, 53, 47, 50 us, whole 83).
+// Whole and in segments, us: gated, 3 of 54 - 839 tokens, 8 heads of 64 x 64 57 36; bonus form, one of 1002, 16 heads of 64 x 64 87 44; decayed
+// sum, 2 of 57 - 1100, 8 heads of 64 x 128 75 35, one of 1100, 8 of 128 x 128 84 40.  In 110 batches of 1 to 10 portions 0.89 of the time in the mean (the best
+// length of each would be 0.87), none slower.  Errors against 64 bits are the same to the third digit (a chain rounds as often as its segments do).
+static int segment_chunks(const ChunkScanArgs& a, double longest) {
+  if (a.form == kChunkDelta) return 0;                    // (what a chunk leaves of a state is a matrix there)
+  const int64_t columns = a.heads * (int64_t)((a.V + (a.K <= 64 ? 63 : 31)) / (a.K <= 64 ? 64 : 32)), room = 256 / columns - a.n_seq;
+  if (room < 1) return 0;
+  const int64_t fits = a.n_tokens / (C * (room + 1)) + 1;      // the least with n_tokens / (16 segment) <= room
+  const int64_t segment = std::max<int64_t>({6, fits, (int64_t)std::ceil(longest / 7)});
+  return longest >= 1.6 * segment + 6 ? (int)segment : 0;
+}
+// Whether a call takes the launches of this file: the chunks of a segment (0: whole portions), -1: it does not
+static int chain_plan(const ChunkScanArgs& a) {
+  if (!chunk_scan_fits(a) || (a.V + 31) / 32 > 65535 || (a.form == kChunkDelta && a.K <= 64)) return -1;
+  if (chunk_numbers(a) * a.heads > INT32_MAX || plan_floats(a, 0) > (int64_t)1 << 28) return -1;      // (1 GiB)
   // Two launches save `few` or `many` us for a chunk of the chain and take `cost` us for each chunk and head, and 2 us.  Fitted to 12 batches
   // of 1 to 16 portions of 64 to 1151 tokens, 8 to 32 heads and 12 forms and sizes; one launch and two, us, about the line: delta rule, 128 x 128, 32
   // heads: 2 portions of 128 27 28, 2 of 600 104 91, 16 heads: 4 of 1000 167 143; decayed sum, 128 x 64, 32 heads: 4 of 256 40 33, 8 of 512 74 79;
@@ -568,10 +704,22 @@ int64_t chunk_scan_workspace(const ChunkScanArgs& a) {
   const double mean = (double)a.n_tokens / a.n_seq / C, longest = a.longest > 0 ? (double)a.longest / C : mean;
   const int64_t chains = (int64_t)a.n_seq * a.heads * ((a.V + VW - 1) / VW);      // a compute unit takes one at a time
   const double chain = chains <= 256 ? longest : mean * ((chains + 255) / 256), saved = (few_chains(a) ? line.few : line.many) * chain;
-  return chain * line.one >= 20.0 && saved > line.cost * a.n_tokens / C * a.heads + 3.5 ? floats : 0;
+  const bool whole = chain * line.one >= 20.0 && saved > line.cost * a.n_tokens / C * a.heads + 3.5;
+  const int segment = segment_chunks(a, longest);
+  if (segment > 0 && plan_floats(a, segment) <= (int64_t)1 << 28) return segment;
+  return whole ? 0 : -1;
 }
 
-int chunk_chain(const ChunkScanArgs& a, hipStream_t s) {
+int64_t chunk_scan_workspace(const ChunkScanArgs& a) {
+  const int segment = chain_plan(a);
+  return segment < 0 ? 0 : plan_floats(a, segment);
+}
+
+int chunk_chain(const ChunkScanArgs& args, hipStream_t s) {
+  ChunkScanArgs a = args;
+  const int segment = chain_plan(a);
+  a.segment = segment > 0 ? segment : 0;
+  a.segments = a.made + plan_made(a);
   if (a.q_dtype == HX_BF16) return launch_width<BF16, BF16>(a, s);
   return a.v_dtype == HX_F32 ? launch_width<F32, F32>(a, s) : launch_width<F32, BF16>(a, s);
 }

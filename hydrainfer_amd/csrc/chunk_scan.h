@@ -26,6 +26,8 @@ struct ChunkScanArgs {
   int64_t n_tokens;
   int32_t longest;        // the longest portion, 0: not known
   float* made;            // chunk_scan_workspace floats on a multiple of 16 bytes: what chunks need is made in a launch ahead; or NULL
+  int32_t segment;        // chunk_chain.hip's own: chunks a segment of a portion (0: a portion is one chain), and what the segments leave for each other
+  float* segments;
 };
 
 // true if chunk_scan serves these sizes

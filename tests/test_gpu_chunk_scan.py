@@ -166,6 +166,46 @@ def _on_the_device(form, lens, H, K, V, x):
     return (got, st.view(n, H, K, V)), (want.reshape(T, H * V).cpu(), S.cpu())
 
 
+# few chains of long portions: segments of six chunks (96 tokens), whose states a launch ahead makes.  Whole segments, a token more and one less,
+# portions of one segment, of one token and of none beside them, a state of an odd number of floats, more columns than a workgroup takes
+SEGMENTS = [[288], [289], [383], [700, 0, 96, 480, 1, 97, 1000]]
+
+
+@pytest.mark.parametrize("lens", SEGMENTS, ids=lambda v: f"{len(v)}x{v[0]}")
+@pytest.mark.parametrize("K, V", [(64, 64), (128, 128), (65, 7), (20, 70)])
+@pytest.mark.parametrize("form, per_channel, types", [("decay", False, "bf16"), ("decay", True, "f32"), ("bonus", True, "mixed")])
+def test_portions_in_segments(lens, K, V, form, per_channel, types, monkeypatch):
+    from hydrainfer_amd import _lib
+    lib, H, n, T, asked = _lib.mix_lib(), 2, len(lens), sum(lens), []
+
+    class Watch:
+        def __getattr__(self, name):
+            if name != "hxm_state_scan_workspace":
+                return getattr(lib, name)
+            return lambda a: asked.append(lib.hxm_state_scan_workspace(a)) or asked[-1]
+
+    monkeypatch.setattr(_lib, "_mix", Watch())
+    g = torch.Generator(device="cuda").manual_seed(K + V)
+    f, rand = (lambda *s: torch.randn(s, generator=g, device="cuda")), (lambda *s: torch.rand(s, generator=g, device="cuda"))
+    qk_t, v_t = (torch.bfloat16 if types == "bf16" else torch.float32), (torch.float32 if types == "f32" else torch.bfloat16)
+    unit = lambda: torch.nn.functional.normalize(f(T, H, K), dim=-1).reshape(T, H * K).to(qk_t)
+    decay = rand(T, H * K if per_channel else H) ** 0.2
+    decay[150:160, 0] = 0.0                                # (nothing is left behind these; what stands there has to vanish, not to turn into NaN)
+    x = dict(q=unit(), k=unit(), v=f(T, H * V).to(v_t), decay=decay, vscale=rand(T, H) if form == "decay" else None, beta=None,
+             bonus=f(H * K) if form == "bonus" else None, state=f(n, 1, H * K * V))
+    got, want = _on_the_device(form, lens, H, K, V, x)
+    rest = asked[0] - H * (T // 96 + n) * ((K * V + 1) // 2 * 2 + 2 * K)      # floats of the segments, and those of the chunks
+    assert rest > 0 and rest % (H * (T // 16 + n)) == 0
+    for name, a, b in zip(("out", "state"), got, want):
+        _check(name, a, b)
+
+
+@pytest.mark.parametrize("lens", SEGMENTS[1:], ids=lambda v: f"{len(v)}x{v[0]}")
+@pytest.mark.parametrize("K, V, dtype", [(64, 64, torch.bfloat16), (100, 130, torch.float32), (65, 7, torch.float32)])
+def test_gated_portions_in_segments(lens, K, V, dtype):
+    _through_the_gated_recurrence(lens, K, V, dtype)
+
+
 @pytest.mark.parametrize("lens, H", [([1151], 3), ([0, 300, 0, 1, 417, 0], 3), (MANY, 22)], ids=str)
 @pytest.mark.parametrize("K, V", [(64, 64), (128, 128), (100, 36), (48, 7)])
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
