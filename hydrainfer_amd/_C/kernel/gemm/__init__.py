@@ -50,14 +50,33 @@ def gate_up_rows_supported(x: Tensor, weight: Tensor) -> bool:
     return K >= 128 and (l.hx_gate_up_silu_few_rows_supported(M, inter, K) == 1 or (M > 128 and l.hx_gate_up_silu_rows_supported(M, inter, K) == 1))
 
 
+def _rows_take(x: Tensor, weight: Tensor) -> bool:
+    """Operands as csrc/gemm_rows.hip reads them, of more than 64 rows"""
+    M, K = x.shape
+    return (M > 64 and x.is_cuda and weight.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and weight.dtype == x.dtype and weight.shape[1] == K
+            and x.stride(1) == 1 and weight.stride(1) == 1 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and max(M * x.stride(0), weight.shape[0] * weight.stride(0)) < 2 ** 31)
+
+
+def linear_rows_whole(x: Tensor, weight: Tensor) -> Optional[Tensor]:
+    """x [M, K] @ weight [N, K]^T for batches of prompts, in one launch and rounded once; None where a library product is expected to be as fast."""
+    M, K = x.shape
+    N = weight.shape[0]
+    if not _rows_take(x, weight) or _lib.lib().hx_linear_rows_whole_supported(M, N, K) != 1:
+        return None
+    _lib.require_gpu(x, weight)
+    out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    _lib.check(_lib.lib().hx_linear_rows_whole(out.data_ptr(), x.data_ptr(), weight.data_ptr(), M, N, K, x.stride(0), weight.stride(0), _lib.dtype_code(x),
+                                               _lib.current_stream()), "linear_rows_whole")
+    return out
+
+
 def linear_rows(x: Tensor, weight: Tensor) -> Optional[Tensor]:
     """x [M, K] @ weight [N, K]^T for batches of prompts, for an add and norm behind it: [M, N] of x's type, or float slabs [splits, M, N]
     (add_rms_norm_slabs sums them); None where a library product is expected to be as fast."""
     M, K = x.shape
     N = weight.shape[0]
-    if M <= 64 or not (x.is_cuda and weight.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and weight.dtype == x.dtype and weight.shape[1] == K
-                       and x.stride(1) == 1 and weight.stride(1) == 1 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0
-                       and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and max(M * x.stride(0), N * weight.stride(0)) < 2 ** 31):
+    if not _rows_take(x, weight):
         return None
     l = _lib.lib()
     splits = l.hx_linear_rows_splits(M, N, K)

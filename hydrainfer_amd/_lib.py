@@ -136,6 +136,8 @@ _SIGNATURES = {
     "hx_prompt_last_layer": (c_int, [POINTER(hx_prompt_last), c_void_p]),
     "hx_linear_rows_splits": (c_int, [c_int64] * 3),
     "hx_linear_rows": (c_int, [c_void_p, c_void_p, c_int32, c_void_p, c_void_p] + [c_int64] * 5 + [c_int, c_void_p]),
+    "hx_linear_rows_whole_supported": (c_int, [c_int64] * 3),
+    "hx_linear_rows_whole": (c_int, [c_void_p] * 3 + [c_int64] * 5 + [c_int, c_void_p]),
     "hx_gate_up_silu_rows": (c_int, [c_void_p] * 3 + [c_int64] * 5 + [c_int, c_void_p]),
     "hx_gate_up_silu_xreg_supported": (c_int, [c_int64] * 3),
     "hx_gate_up_silu_xreg": (c_int, [c_void_p] * 3 + [c_int64] * 4 + [c_int, c_int, c_void_p]),

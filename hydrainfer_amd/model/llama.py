@@ -255,7 +255,8 @@ class LlamaForCausalLM:
                                "are not available on this node")
         if self.use_hip_gemm and x.shape[0] <= 64 and hip_gemm.supported(x, w):
             return hip_gemm.linear_decode(x, w)
-        return torch.matmul(x, w.t())
+        out = hip_gemm.linear_rows_whole(x, w) if self.use_hip_gemm and x.dim() == 2 else None
+        return torch.matmul(x, w.t()) if out is None else out
 
     def _feed_forward(self, x: Tensor, h: Tensor, l: int) -> None:
         """h += the layer's feed-forward of x = norm2(h); x = the next layer's norm (the final norm after the last)"""

@@ -243,6 +243,10 @@ int hx_gate_up_silu_rows(void* out, const void* x, const void* weight, int64_t M
 int hx_linear_rows_splits(int64_t M, int64_t N, int64_t K);
 int hx_linear_rows(void* out, float* slabs, int32_t n_splits, const void* x, const void* weight, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
                    int dtype, hx_stream stream);
+/* The same without splits, for products that no add and norm stands behind: out [M, N].  hx_linear_rows_whole_supported: 1 where it serves and a library
+ * product is not expected to be faster. */
+int hx_linear_rows_whole_supported(int64_t M, int64_t N, int64_t K);
+int hx_linear_rows_whole(void* out, const void* x, const void* weight, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int dtype, hx_stream stream);
 /* The sampled rows of a batch of prompts (csrc/prompt_rows.hip): rows [n] (int32 or int64, negative ones from the end) of x and h
  * [n_tokens, row_bytes] into x_out, h_out; tables (4 n + 3 int32): q_cu | kv_cu | cu_blocks [n + 1 each] of a batch in which each row is a sequence of one query
  * that sees the keys the row sees (a causal row of its own sequence), and the rows' positions [n].  cu_blocks has no other use than its starts. */

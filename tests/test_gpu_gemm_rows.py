@@ -36,6 +36,23 @@ def test_linear_rows(M, N, K, dt):
     assert bool(((got.double() - z).abs() <= eps).all())
 
 
+@pytest.mark.parametrize("M, N, K", [(65, 32, 64), (127, 96, 128), (129, 2080, 192), (104, 6144, 2048), (257, 4128, 512), (300, 6144, 2048), (1024, 4096, 2048), (1000, 32, 2048)])
+@pytest.mark.parametrize("dt", DTYPES)
+def test_linear_rows_whole(M, N, K, dt):
+    from hydrainfer_amd._C.kernel.gemm import linear_rows_whole
+    x, w, z, eps = _operands(M, N, K, dt, M + N + K)
+    got = linear_rows_whole(x, w)
+    assert got is not None and got.shape == (M, N) and got.dtype == dt
+    assert bool(((got.double() - z).abs() <= eps + DTYPES[dt] * z.abs() + (2.0 ** -25 if dt == torch.float16 else 0)).all())
+
+
+@pytest.mark.parametrize("M, N, K", [(64, 4096, 2048), (1025, 4096, 2048), (128, 2064, 2048), (128, 4096, 2080), (128, 6176, 2048), (128, 64, 4096)])
+def test_linear_rows_whole_is_left_to_the_library(M, N, K):
+    from hydrainfer_amd._C.kernel.gemm import linear_rows_whole
+    x, w, _, _ = _operands(M, N, K, torch.bfloat16, 1)
+    assert linear_rows_whole(x, w) is None
+
+
 @pytest.mark.parametrize("M, N, K", [(64, 2048, 2048), (513, 2048, 2048), (1025, 2048, 5632), (128, 2064, 2048), (128, 2048, 2080)])
 def test_linear_rows_is_left_to_the_library(M, N, K):
     from hydrainfer_amd._C.kernel.gemm import linear_rows
