@@ -16,8 +16,8 @@
 // What bounds it: the vector ALU of a SIMD, which a consumer (430 instructions a chunk under the delta rule: parts, sums, results) and a producer (850:
 // parts of rows, products of decays, the substitution) share, and which does not run beside the products of its own wave.  Of a chunk's 4.6 us
 // 1.3 are matrix products.
-// Rows are read eight bytes at a time (two reads made one by the compiler bring a quarter of their bytes a cycle) and parts made by v_dot2_f32_bf16: delta rule, 128 x 128, 32
-// heads, 4 portions of 797 - 1151 tokens 166.5 -> 163.0 us, decayed sum of bfloat16 q and k, 3 of 168 - 723, 128 x 64 65.3 -> 63.7, 2 of 28 - 130 18.4 -> 17.6.
+// Rows are read eight bytes at a time (two reads made one by the compiler bring a quarter of their bytes a cycle) and straight from global memory (through flat
+// addresses every barrier waited for them): delta rule, 128 x 128, 32 heads, 4 portions of 797 - 1151 tokens 167.2 -> 159.2 us, the same bits.
 // Measured before that, one launch of sixteen tokens at a time in float and this one, us: delta rule, 128 x 128, 32 heads, 4 portions of 797 - 1151 tokens 191 and
 // 169, 12 of 300 - 900 348 and 309, 16 of 60 55.6 and 55.6; decayed sum, 128 x 128, 32 heads, 4 of 797 - 1151 145 and 103, 12 of 300 - 900 263 and 190,
 // one of 100 19.8 and 17.1, 64 x 64 93 and 83.  Results' error against 64 bits (2-norm, 400 and 250 tokens, 1e-7): delta rule 1.08 and 1.00,
@@ -44,30 +44,21 @@ __device__ __forceinline__ f32x4 mma_parts(u16x8 a, u16x8 b, f32x4 c) {
 }
 __device__ __forceinline__ u16x8 both(u16x4 a, u16x4 b) { return u16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}; }
 
-// Four floats in three parts, two at a time: one conversion makes both numbers' parts, and v_dot2_f32_bf16 takes a part from its float (1 and 0 times the two parts, exact,
-// subnormal numbers kept): 7 instructions a pair, 11 with shifts and subtractions.  Beside an infinite part the neighbour's lower ones are no numbers then, which is
-// nothing where neighbours are summed over (channels of a query, keys and tokens of a value channel: that sum holds the infinity as well, and total_of is made for
-// it); keys, whose channels are rows of the state, are kept APART.
-template <bool APART = false>
+// Four floats in three parts, two at a time: one conversion makes both numbers' parts.  (v_dot2_f32_bf16 would take a part from its float in one instruction and not in
+// two: the delta rule on 4 portions of 797 - 1151 tokens, 32 heads of 128 x 128, 164 us and not 159, and states off by 5 % more, 7.12 and 7.44e-8.)
 __device__ __forceinline__ void split(f32x4 x, u16x4 (&part)[3]) {
   typedef __bf16 pair_t __attribute__((ext_vector_type(2)));
   typedef float f32x2 __attribute__((ext_vector_type(2)));
-  uint32_t first = 0x0000bf80u, second = 0xbf800000u;     // (-1, 0) and (0, -1); in registers: as an inline constant the second would be another number
-  asm("" : "+s"(first), "+s"(second));
 #pragma unroll
   for (int p = 0; p < 3; ++p)
 #pragma unroll
     for (int e = 0; e < 4; e += 2) {
-      const pair_t two = __builtin_convertvector((f32x2{x[e], x[e + 1]}), pair_t);
-      const uint32_t bits = __builtin_bit_cast(uint32_t, two);
+      const uint32_t bits = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x[e], x[e + 1]}), pair_t));
       part[p][e] = (u16)bits;
       part[p][e + 1] = (u16)(bits >> 16);
-      if (p < 2 && APART) {
+      if (p < 2) {
         x[e] -= __builtin_bit_cast(float, bits << 16);
         x[e + 1] -= __builtin_bit_cast(float, bits & 0xffff0000u);
-      } else if (p < 2) {
-        x[e] = __builtin_amdgcn_fdot2_f32_bf16(two, __builtin_bit_cast(pair_t, first), x[e], false);
-        x[e + 1] = __builtin_amdgcn_fdot2_f32_bf16(two, __builtin_bit_cast(pair_t, second), x[e + 1], false);
       }
     }
 }
@@ -449,7 +440,7 @@ __global__ __launch_bounds__(512) void chunk_head32_kernel(ChunkScanArgs a) {
   };
   // (rows past the portion repeat its last one: the values and write strengths there are none)
   const bool whole = a.K == KP;
-  auto planes = [&](char* to, const Piece<QK, 4, VEC>& p, int at, auto apart) __attribute__((always_inline)) {
+  auto planes = [&](char* to, const Piece<QK, 4, VEC>& p, int at) __attribute__((always_inline)) {
     const int col = qk_col(at);
     f32x4 x;
 #pragma unroll
@@ -463,7 +454,7 @@ __global__ __launch_bounds__(512) void chunk_head32_kernel(ChunkScanArgs a) {
       *reinterpret_cast<u16x4*>(dst) = u16x4{BF16::from_float(x[0]), BF16::from_float(x[1]), BF16::from_float(x[2]), BF16::from_float(x[3])};
     } else {
       u16x4 part[3];
-      split<decltype(apart)::value>(x, part);
+      split(x, part);
 #pragma unroll
       for (int i = 0; i < 3; ++i) *reinterpret_cast<u16x4*>(dst + i * I::kPlane) = part[i];
     }
@@ -473,8 +464,8 @@ __global__ __launch_bounds__(512) void chunk_head32_kernel(ChunkScanArgs a) {
     char* im = image(chunk);
 #pragma unroll
     for (int i = 0; i < NQ; ++i) {
-      planes(im + I::kQ, s.q[i], i, std::false_type());
-      planes(im + I::kK, s.k[i], i, std::true_type());
+      planes(im + I::kQ, s.q[i], i);
+      planes(im + I::kK, s.k[i], i);
     }
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
