@@ -305,10 +305,11 @@ __global__ __launch_bounds__(64 * WAVES) void router_four_kernel(const float* __
   if (wave >= 4 || t0 + wave >= n_tokens) return;
   float z[1] = {-INFINITY};
   if (lane < E) {
-    float s = 0.f;
+    // (in double: weights' error against 64 bits for 16 experts of 4096 is 1.01e-7 with these added up in float, 0.80 so, 0.97 with a workgroup a token)
+    double s = bias ? bias[lane] : 0.f;
 #pragma unroll
     for (int v = 0; v < WAVES; ++v) s += sums[v][wave][lane];
-    z[0] = s + (bias ? bias[lane] : 0.f);
+    z[0] = (float)s;
   }
   choose_top<1>(z, lane, E, top, weights + (t0 + wave) * top, experts + (t0 + wave) * top);
 }
