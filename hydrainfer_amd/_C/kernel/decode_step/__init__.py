@@ -1,6 +1,6 @@
 """The layers of a decode step, each in one native call (csrc/decode_step.hip, hx_decode_layer_step): the launches that
 gemm.linear_decode_ex, flash_attn.decode_attention_fused, gemm.norm_gate_up_silu_xreg, gemm.norm_linear_decode_xreg and
-norm.add_rms_norm_slabs issue one by one, in the same order with the same arguments.  And the last layer of a batch of prompts (csrc/prompt_rows.hip)."""
+norm.add_rms_norm_slabs issue one by one, in the same order with the same arguments.  And layers of a batch of prompts (csrc/prompt_rows.hip)."""
 import ctypes
 from typing import Iterable, NamedTuple, Optional
 
@@ -148,3 +148,46 @@ def prompt_last_layer(x: Tensor, h: Tensor, rows: Tensor, kv: Tensor, positions:
     c.scratch, c.scratch_bytes = scratch.data_ptr(), need
     _lib.check(lib.hx_prompt_last_layer(ctypes.byref(c), _lib.current_stream()), "prompt_last_layer")
     return out
+
+
+def prompt_layer(x: Tensor, h: Tensor, qkv: Tensor, positions: Tensor, cos_sin: Tensor, key_cache: Tensor, value_cache: Tensor, new_cache_slots: Tensor, cu_seqlens_q: Tensor,
+                 cu_seqlens_k: Tensor, block_table: Tensor, cu_block_lens: Tensor, max_seqlen_q: int, max_seqlen_k: int, n_heads: int, wo: Tensor, w_gate_up: Tensor, w_down: Tensor,
+                 norm_mlp: Tensor, norm_next: Tensor, softmax_scale: float, epsilon: float) -> bool:
+    """A layer of a batch of prompts behind its qkv product (csrc/prompt_rows.hip), in place: qkv [n_tokens, q | k | v] of x = norm1(h) is rotated, its keys and values go
+    to the cache, h += attention and feed-forward, x = rms_norm(h) * norm_next.  False, and nothing done, where a product of it is left to a library."""
+    _lib.require_gpu(x, h, qkv, positions, cos_sin, key_cache, value_cache, new_cache_slots, cu_seqlens_q, cu_seqlens_k, block_table, cu_block_lens, wo, w_gate_up, w_down, norm_mlp,
+                     norm_next)
+    (n, hidden), n_kv, D, inter, dt = x.shape, key_cache.shape[2], key_cache.shape[3], w_down.shape[1], x.dtype
+    width = n_heads * D
+    if dt not in (torch.float16, torch.bfloat16) or any(t.dtype != dt or not t.is_contiguous() for t in (x, h, qkv, cos_sin, norm_mlp, norm_next)) \
+            or any(t.dtype != dt or t.stride(-1) != 1 for t in (key_cache, value_cache, wo, w_gate_up, w_down)):
+        raise _lib.HydraHipError("prompt_layer: one dtype (fp16 / bf16); x, h, qkv, cos_sin, norms and rows of weights and caches contiguous")
+    if any(t.dtype != torch.int32 or not t.is_contiguous() for t in (positions, new_cache_slots, cu_seqlens_q, cu_seqlens_k, block_table, cu_block_lens)):
+        raise _lib.HydraHipError("prompt_layer: positions, slots, lengths and block table must be contiguous int32")
+    if h.shape != x.shape or qkv.shape != (n, width + 2 * n_kv * D) or positions.numel() != n or new_cache_slots.numel() != n or value_cache.shape != key_cache.shape \
+            or wo.shape != (hidden, width) or w_gate_up.shape != (2 * inter, hidden) or w_down.shape != (hidden, inter) or norm_mlp.numel() != hidden or norm_next.numel() != hidden \
+            or cu_seqlens_q.numel() < 2 or cu_seqlens_k.numel() != cu_seqlens_q.numel() or cu_block_lens.numel() < cu_seqlens_q.numel() or D % 8 or D > 256 or key_cache.shape[1] % 16 \
+            or any(c.stride(2) != D or c.stride(1) != n_kv * D for c in (key_cache, value_cache)):
+        raise _lib.HydraHipError("prompt_layer: shape mismatch")
+    c = _lib.hx_prompt_layer()
+    a = c.attn
+    a.k, a.v, a.block_size = key_cache.data_ptr(), value_cache.data_ptr(), key_cache.shape[1]
+    a.k_block_stride, a.k_row_stride, a.k_head_stride = key_cache.stride()[:3]
+    a.v_block_stride, a.v_row_stride, a.v_head_stride = value_cache.stride()[:3]
+    a.cu_seqlens_q, a.cu_seqlens_k, a.block_table, a.cu_block_lens = cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(), block_table.data_ptr(), cu_block_lens.data_ptr()
+    a.batch, a.n_heads, a.n_kv_heads, a.head_dim, a.max_seqlen_q, a.max_seqlen_k = cu_seqlens_q.numel() - 1, n_heads, n_kv, D, int(max_seqlen_q), int(max_seqlen_k)
+    a.softmax_scale, a.causal, a.dtype, a.window_left, a.window_right = float(softmax_scale), 1, _lib.dtype_code(x), -1, -1
+    c.positions, c.new_cache_slots, c.qkv, c.x, c.h, c.cos_sin = (t.data_ptr() for t in (positions, new_cache_slots, qkv, x, h, cos_sin))
+    c.wo, c.w_gate_up, c.w_down, c.norm_mlp, c.norm_next = (t.data_ptr() for t in (wo, w_gate_up, w_down, norm_mlp, norm_next))
+    c.n_tokens, c.hidden, c.inter, c.ld_wo, c.ld_gate_up, c.ld_down = n, hidden, inter, wo.stride(0), w_gate_up.stride(0), w_down.stride(0)
+    c.epsilon = float(epsilon)
+    lib = _lib.lib()
+    need = lib.hx_prompt_layer_scratch_bytes(ctypes.byref(c))
+    if need == _lib.HX_ERR_UNSUPPORTED:
+        return False
+    if need < 0:
+        _lib.check(int(need), "prompt_layer")
+    scratch = torch.empty(need, dtype=torch.uint8, device=x.device)
+    c.scratch, c.scratch_bytes = scratch.data_ptr(), need
+    _lib.check(lib.hx_prompt_layer_step(ctypes.byref(c), _lib.current_stream()), "prompt_layer")
+    return True

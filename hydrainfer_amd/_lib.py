@@ -81,6 +81,13 @@ class hx_prompt_last(ctypes.Structure):
         ("epsilon", c_float), ("rows_are_int64", c_int32)]
 
 
+class hx_prompt_layer(ctypes.Structure):
+    _fields_ = [("attn", hx_attn_args)] + [(p, c_void_p) for p in (
+        "positions", "new_cache_slots", "qkv", "x", "h", "cos_sin", "wo", "w_gate_up", "w_down", "norm_mlp", "norm_next", "scratch")] + [
+        (i, c_int64) for i in ("scratch_bytes", "n_tokens", "hidden", "inter", "ld_wo", "ld_gate_up", "ld_down")] + [("epsilon", c_float)]
+
+
+HX_ERR_UNSUPPORTED = -5
 HX_DW_LDS_SLICE, HX_DW_XREG, HX_DW_GATE_UP = 0, 1, 1
 HX_DW_FORCE_LDS_SLICE = 2
 
@@ -134,6 +141,8 @@ _SIGNATURES = {
     "hx_prompt_rows": (c_int, [c_void_p, c_int32] + [c_int64] * 3 + [c_void_p] * 8 + [c_int64, c_void_p, c_void_p]),
     "hx_prompt_last_scratch_bytes": (c_int64, [POINTER(hx_prompt_last)]),
     "hx_prompt_last_layer": (c_int, [POINTER(hx_prompt_last), c_void_p]),
+    "hx_prompt_layer_scratch_bytes": (c_int64, [POINTER(hx_prompt_layer)]),
+    "hx_prompt_layer_step": (c_int, [POINTER(hx_prompt_layer), c_void_p]),
     "hx_linear_rows_splits": (c_int, [c_int64] * 3),
     "hx_linear_rows": (c_int, [c_void_p, c_void_p, c_int32, c_void_p, c_void_p] + [c_int64] * 5 + [c_int, c_void_p]),
     "hx_linear_rows_whole_supported": (c_int, [c_int64] * 3),

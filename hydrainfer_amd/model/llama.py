@@ -24,7 +24,7 @@ from hydrainfer_amd._C.kernel.norm import (StepHead, add_rms_norm, add_rms_norm_
                                              embed_rms_norm, embed_rms_norm_supported, rms_norm)
 from hydrainfer_amd._C.kernel.position_embedding import rope_set_kv_cache
 from hydrainfer_amd.layer.causal_attention import AttentionParameters
-from hydrainfer_amd._C.kernel.decode_step import DecodeLayer, decode_layers, prompt_last_layer
+from hydrainfer_amd._C.kernel.decode_step import DecodeLayer, decode_layers, prompt_last_layer, prompt_layer
 from hydrainfer_amd._C.kernel.flash_attn import decode_attention_fused, mha_varlen_fwd
 from hydrainfer_amd._C.kernel import gemm as hip_gemm
 from hydrainfer_amd import _lib, launch_plan
@@ -295,6 +295,24 @@ class LlamaForCausalLM:
         return prompt_last_layer(x, h, rows, kv, position_ids, self.cos_sin, *ap.kv_cache.get_kv_cache(), ap.new_cache_slots, ap.q_cu_seq_lens, ap.kv_cu_seq_lens,
                                  ap.block_tables, ap.cu_blocks_lens, ap.kv_max_seq_len, w[:self.q_size], st[f"l{l}.wo"], st[f"l{l}.wgu"], st[f"l{l}.wdown"],
                                  st[f"l{l}.norm2"], st["norm"], D ** -0.5, self.shape.rms_norm_eps)
+
+    def _layer_of_few_prompts(self, x: Tensor, h: Tensor, qkv: Tensor, position_ids: Tensor, ap, l: int) -> bool:
+        """The rest of a layer behind its qkv product by one call, where all its products are made in tiles of 64 to 192 (65 to some 500 tokens) and the launches take the
+        operands; False, and nothing done, elsewhere.  The launches are those that the general path issues one by one."""
+        st, n, D = self.state, x.shape[0], self.shape.head_dim
+        if not (self.use_hip_gemm and 64 < n <= 512 and h.is_cuda and h.dtype in (torch.float16, torch.bfloat16)):
+            return False
+        kc, vc = ap.kv_cache.get_kv_cache()
+        weights = [st[f"l{l}.{k}"] for k in ("wo", "wgu", "wdown")]
+        tables = (position_ids, ap.new_cache_slots, ap.q_cu_seq_lens, ap.kv_cu_seq_lens, ap.block_tables, ap.cu_blocks_lens)
+        if not (all(w.device == h.device and w.dtype == h.dtype and w.is_contiguous() and w.data_ptr() % 16 == 0 for w in weights) and h.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0
+                and qkv.is_contiguous() and all(t is not None and t.dtype == torch.int32 and t.device == h.device and t.is_contiguous() for t in tables)
+                and position_ids.shape == ap.new_cache_slots.shape == (n,) and ap.q_cu_seq_lens.shape == ap.kv_cu_seq_lens.shape
+                and ap.cu_blocks_lens.numel() >= ap.q_cu_seq_lens.numel() >= 2 and self.cos_sin.is_contiguous() and self.cos_sin.dtype == h.dtype and D % 8 == 0 and D <= 256
+                and kc.shape[1] % 16 == 0 and all(c.dtype == h.dtype and c.stride()[1:] == (c.shape[2] * D, D, 1) for c in (kc, vc))):
+            return False
+        return prompt_layer(x, h, qkv, position_ids, self.cos_sin, kc, vc, *tables[1:], ap.q_max_seq_len, ap.kv_max_seq_len, self.shape.num_attention_heads, *weights,
+                            st[f"l{l}.norm2"], st[f"l{l + 1}.norm1"], D ** -0.5, self.shape.rms_norm_eps)
 
     def _linear_add_norm(self, out: Tensor, h: Tensor, x: Tensor, w: Tensor, norm: Tensor) -> None:
         """h += x w^T; out = rms_norm(h)"""
@@ -579,6 +597,8 @@ class LlamaForCausalLM:
             if l == L - 1 and self._sampled_rows_only(h, position_ids, ap, model_params):
                 return self._last_layer_of_sampled_rows(x, h, position_ids, ap, model_params.selected_token_ids)
             qkv = self.linear(x, st[f"l{l}.wqkv"])
+            if l < L - 1 and not model_params.all_sequences_decode and self._layer_of_few_prompts(x, h, qkv, position_ids, ap, l):
+                continue
             q = qkv[:, :q_size].view(n, H, D)
             k = qkv[:, q_size:q_size + kv_size].view(n, HK, D)
             v = qkv[:, q_size + kv_size:].view(n, HK, D)

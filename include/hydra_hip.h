@@ -432,6 +432,22 @@ typedef struct hx_prompt_last {
 int64_t hx_prompt_last_scratch_bytes(const hx_prompt_last* layer);
 int hx_prompt_last_layer(const hx_prompt_last* layer, hx_stream stream);
 
+/* A layer of a batch of prompts of a few hundred tokens behind its qkv product, by one call: RoPE and cache append, attention, x = norm_mlp(h += o wo^T), feed-forward, x =
+ * norm_next(h += ...).  qkv [n_tokens, (n_heads + 2 n_kv_heads) * head_dim] is rotated in place; attn: the cache, its block table, the batch's lengths, batch, max_seqlen_q and
+ * max_seqlen_k (queries, output, total_q and workspace are set by the call).  The same launches, in the same order and with the same results, as hx_rope_set_kv_cache, hx_mha_varlen_fwd, hx_linear_rows,
+ * hx_add_rms_norm(_slabs) and hx_gate_up_silu_rows; HX_ERR_UNSUPPORTED where hx_linear_rows_splits or hx_gate_up_silu_few_rows_supported leave a product to a library. */
+typedef struct hx_prompt_layer {
+  hx_attn_args attn;
+  const int32_t *positions, *new_cache_slots;      /* [n_tokens] */
+  void *qkv, *x, *h;
+  const void *cos_sin, *wo, *w_gate_up, *w_down, *norm_mlp, *norm_next;
+  void* scratch;
+  int64_t scratch_bytes, n_tokens, hidden, inter, ld_wo, ld_gate_up, ld_down;
+  float epsilon;
+} hx_prompt_layer;
+int64_t hx_prompt_layer_scratch_bytes(const hx_prompt_layer* layer);
+int hx_prompt_layer_step(const hx_prompt_layer* layer, hx_stream stream);
+
 /* Extension (SURVEY §8f-2 taken to the end): one launch for the three consecutive steps of a
  * decode layer — apply_rotary_pos_emb(q, k) (NeoX, rotary_dim == head_dim), set_kv_cache(slots,
  * k, v) and the paged attention itself (hydrainfer/model/model_forward.py:78-84 +

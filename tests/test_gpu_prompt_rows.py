@@ -82,3 +82,49 @@ def test_sampled_rows_of_the_last_layer(new, kv, rows, heads, kv_heads, layers, 
     assert float((got_caches.float() - want_caches.float()).norm() / want_caches.float().norm()) < half
     # attention and three products behind it, rounded each: 8 times half a unit in the last place
     assert float((got.float() - want.float()).norm() / want.float().norm()) < 8 * half
+
+
+# the smallest and largest number of tokens that go this way, ragged portions with an empty one, as many key heads as heads and fewer, slabs of several splits and of none
+@pytest.mark.parametrize("new, kv", [([65], [65]), ([40, 3, 0, 61], [40, 90, 17, 333]), ([300, 212], [300, 500])])
+@pytest.mark.parametrize("heads, kv_heads, W, inner", [(4, 4, 512, 1024), (8, 2, 512, 640), (16, 16, 2048, 5632)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_layer_by_one_call(new, kv, heads, kv_heads, W, inner, dt):
+    from hydrainfer_amd.layer.causal_attention import AttentionParameters
+    from hydrainfer_amd.memory.kv_cache import KVCache
+    from hydrainfer_amd.model.llama import LanguageModelParameters, LlamaForCausalLM, LlamaShape
+    D, vocab, layers = 128, 320, 3
+    g = torch.Generator(device="cuda").manual_seed(sum(new) + heads)
+    w = lambda *s: torch.randn(s, generator=g, device="cuda").mul_(s[-1] ** -0.5).to(dt)
+    norm = lambda: (1 + 0.1 * torch.randn(W, generator=g, device="cuda")).to(dt)
+    state = {"embed": w(vocab, W), "lm_head": w(vocab, W), "norm": norm()}
+    for l in range(layers):
+        state.update({f"l{l}.wqkv": w((heads + 2 * kv_heads) * D, W), f"l{l}.wo": w(W, heads * D), f"l{l}.wgu": w(2 * inner, W), f"l{l}.wdown": w(W, inner), f"l{l}.norm1": norm(), f"l{l}.norm2": norm()})
+    model = LlamaForCausalLM(LlamaShape(W, inner, layers, heads, kv_heads, D, vocab), dt, "cuda", state)
+    b = _batch(new, kv, 3)
+    ids = torch.randint(0, vocab, (sum(new),), generator=g, device="cuda")
+    pool = torch.randn(layers, 2, b["n"], BLOCK, kv_heads, D, generator=g, device="cuda").to(dt)
+
+    def through(one_call):
+        caches = pool.clone()
+        model._layer_of_few_prompts = (lambda *a: took.append(LlamaForCausalLM._layer_of_few_prompts(model, *a)) or took[-1]) if one_call else lambda *a: False
+        params = [AttentionParameters(kv_cache=KVCache(c[0], c[1]), q_cu_seq_lens=b["q_cu"], kv_cu_seq_lens=b["k_cu"], new_cache_slots=b["slots"], block_tables=b["table"],
+                                      cu_blocks_lens=b["cu_blocks"], num_sequences=len(new), all_sequences_decode=False, q_max_seq_len=max(new), kv_max_seq_len=max(kv)) for c in caches]
+        with torch.inference_mode():
+            return model.forward_logits(ids, b["pos"], LanguageModelParameters(params, False, torch.tensor([0, sum(new) - 1], device="cuda"))), caches
+
+    took = []
+    got, got_caches = through(True)
+    assert took == [True] * (layers - 1)
+    want, want_caches = through(False)
+    assert torch.equal(got, want) and torch.equal(got_caches, want_caches)      # (the same launches)
+
+
+def test_layer_that_the_call_does_not_take():
+    from hydrainfer_amd._C.kernel.decode_step import prompt_layer
+    n, W, inner, D, H = 600, 512, 1024, 128, 4                   # (more tokens than o is made of in these tiles)
+    b = _batch([n], [n], 1)
+    t = lambda *s: torch.randn(s, device="cuda").bfloat16()
+    x, h, qkv, kc, vc = t(n, W), t(n, W), t(n, 3 * H * D), t(b["n"], BLOCK, H, D), t(b["n"], BLOCK, H, D)
+    held = [y.clone() for y in (x, h, qkv, kc)]
+    assert not prompt_layer(x, h, qkv, b["pos"], t(1024, 2, D // 2), kc, vc, b["slots"], b["q_cu"], b["k_cu"], b["table"], b["cu_blocks"], n, n, H, t(W, H * D), t(2 * inner, W), t(W, inner), t(W), t(W), D ** -0.5, 1e-5)
+    assert all(torch.equal(y, z) for y, z in zip(held, (x, h, qkv, kc)))
