@@ -669,7 +669,7 @@ static int64_t plan_floats(const ChunkScanArgs& a, int segment) {
 // the launches around them cost as much) and a seventh of the portion, as the last segment's start is put together out of all before it (8 heads of 128 x 128, 1151
 // tokens in segments of 4, 8, 12, 16 chunks 81, 53, 47, 50 us, whole 83).
 // Whole and in segments, us: gated, 3 of 54 - 839 tokens, 8 heads of 64 x 64 57 36; bonus form, one of 1002, 16 heads of 64 x 64 87 44; decayed
-// sum, 2 of 57 - 1100, 8 heads of 64 x 128 75 35, one of 1100, 8 of 128 x 128 84 40.  In 110 batches of 1 to 10 portions 0.89 of the time in the mean (the best
+// sum, one of 1100, 8 of 128 x 128 84 40.  In 110 batches of 1 to 10 portions 0.89 of the time in the mean (the best
 // length of each would be 0.87), none slower.  Errors against 64 bits are the same to the third digit (a chain rounds as often as its segments do).
 static int segment_chunks(const ChunkScanArgs& a, double longest) {
   if (a.form == kChunkDelta) return 0;                    // (what a chunk leaves of a state is a matrix there)
@@ -705,7 +705,10 @@ static int chain_plan(const ChunkScanArgs& a) {
   const int64_t chains = (int64_t)a.n_seq * a.heads * ((a.V + VW - 1) / VW);      // a compute unit takes one at a time
   const double chain = chains <= 256 ? longest : mean * ((chains + 255) / 256), saved = (few_chains(a) ? line.few : line.many) * chain;
   const bool whole = chain * line.one >= 20.0 && saved > line.cost * a.n_tokens / C * a.heads + 3.5;
-  const int segment = segment_chunks(a, longest);
+  // (Decayed sums of bfloat16 q and k with one decay a head that one launch of chunk_head.hip would serve stay there: segments of sixteen tokens at a time are up to twice as fast, but leave
+  // states off by up to a tenth more where the last chunk is short: one portion of 483, 8 heads of 64 x 64, 37 and 28 us, 6.1 and 6.7e-8.)
+  const bool by_parts = a.form == kChunkDecay && !a.per_channel && a.q_dtype == HX_BF16 && a.k_dtype == HX_BF16;
+  const int segment = by_parts && !whole ? 0 : segment_chunks(a, longest);
   if (segment > 0 && plan_floats(a, segment) <= (int64_t)1 << 28) return segment;
   return whole ? 0 : -1;
 }

@@ -173,7 +173,7 @@ SEGMENTS = [[288], [289], [383], [700, 0, 96, 480, 1, 97, 1000]]
 
 @pytest.mark.parametrize("lens", SEGMENTS, ids=lambda v: f"{len(v)}x{v[0]}")
 @pytest.mark.parametrize("K, V", [(64, 64), (128, 128), (65, 7), (20, 70)])
-@pytest.mark.parametrize("form, per_channel, types", [("decay", False, "bf16"), ("decay", True, "f32"), ("bonus", True, "mixed")])
+@pytest.mark.parametrize("form, per_channel, types", [("decay", False, "f32"), ("decay", True, "bf16"), ("bonus", True, "mixed")])
 def test_portions_in_segments(lens, K, V, form, per_channel, types, monkeypatch):
     from hydrainfer_amd import _lib
     lib, H, n, T, asked = _lib.mix_lib(), 2, len(lens), sum(lens), []
